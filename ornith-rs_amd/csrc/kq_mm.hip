@@ -25,6 +25,7 @@
 #include <type_traits>
 
 #include "dmath.h"
+#include "mm_narrow_host.h"
 #include "rt.h"
 
 namespace {
@@ -1040,8 +1041,22 @@ __device__ __forceinline__ void order_tiles(uint32_t total_tiles, int bm, const 
 }
 
 
+// The tiles of the shared expert, which every token goes through: number E, "pairs" pairs + t. They
+// follow the routed ones in the list. Returns how many there are.
+__device__ __forceinline__ uint32_t shared_tiles(int shared_rows, int pairs, int E, int bm, uint32_t at, uint32_t* t_expert,
+                                                 uint32_t* t_start, uint32_t* t_count, uint32_t* pair) {
+  const uint32_t n = (uint32_t)(shared_rows + bm - 1) / bm;
+  for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) {
+    t_expert[at + i] = E;
+    t_start[at + i] = pairs + i * bm;
+    t_count[at + i] = min((uint32_t)bm, (uint32_t)shared_rows - i * bm);
+  }
+  for (int i = threadIdx.x; i < shared_rows; i += blockDim.x) pair[pairs + i] = pairs + i;
+  return n;
+}
+
 __global__ __launch_bounds__(1024) void moe_sort_pairs_kernel(const uint32_t* inds, int pairs, int E,
-                                                              int bm, uint32_t* pair, uint32_t* tile_expert,
+                                                              int bm, int shared_rows, uint32_t* pair, uint32_t* tile_expert,
                                                               uint32_t* tile_start, uint32_t* tile_count,
                                                               uint32_t* n_tiles) {
   __shared__ uint32_t cnt[1024], fill[1024];
@@ -1077,7 +1092,8 @@ __global__ __launch_bounds__(1024) void moe_sort_pairs_kernel(const uint32_t* in
   const uint32_t my_tiles = (mine + bm - 1) / bm;
   const uint32_t start = (uint32_t)(incl & ((1ull << 40) - 1)) - mine;
   const uint32_t tiles_before = (uint32_t)(incl >> 40) - my_tiles;
-  const uint32_t total_tiles = (uint32_t)(scan[cur][1023] >> 40);
+  const uint32_t routed_tiles = (uint32_t)(scan[cur][1023] >> 40);
+  const uint32_t total_tiles = routed_tiles + (uint32_t)(shared_rows + bm - 1) / bm;
   if (tid == 0) *n_tiles = total_tiles;
   __syncthreads();
   scan[0][tid] = start;  // (reused: where an expert's run of pairs begins)
@@ -1107,6 +1123,8 @@ __global__ __launch_bounds__(1024) void moe_sort_pairs_kernel(const uint32_t* in
         tile_count[i] = c;
       }
     }
+  if (ordered) shared_tiles(shared_rows, pairs, E, bm, routed_tiles, t_expert, t_start, t_count, pair);
+  else shared_tiles(shared_rows, pairs, E, bm, routed_tiles, tile_expert, tile_start, tile_count, pair);
   __syncthreads();
   if (!ordered) return;
   order_tiles(total_tiles, bm, t_expert, t_start, t_count, tile_expert, tile_start, tile_count);
@@ -1131,7 +1149,8 @@ __global__ __launch_bounds__(256) void moe_sort_count_kernel(const uint32_t* ind
 }
 
 // part_cnt [parts, E] in: pairs of expert e in slice b; out: where slice b's pairs of expert e begin
-__global__ __launch_bounds__(1024) void moe_sort_plan_kernel(int E, int bm, uint32_t* part_cnt, uint32_t* tile_expert,
+__global__ __launch_bounds__(1024) void moe_sort_plan_kernel(int pairs, int E, int bm, int shared_rows, uint32_t* part_cnt,
+                                                             uint32_t* pair, uint32_t* tile_expert,
                                                              uint32_t* tile_start, uint32_t* tile_count,
                                                              uint32_t* n_tiles) {
   __shared__ unsigned long long scan[2][1024];
@@ -1153,7 +1172,8 @@ __global__ __launch_bounds__(1024) void moe_sort_plan_kernel(int E, int bm, uint
   const unsigned long long incl = scan[cur][tid];
   const uint32_t start = (uint32_t)(incl & ((1ull << 40) - 1)) - mine;
   const uint32_t tiles_before = (uint32_t)(incl >> 40) - my_tiles;
-  const uint32_t total_tiles = (uint32_t)(scan[cur][1023] >> 40);
+  const uint32_t routed_tiles = (uint32_t)(scan[cur][1023] >> 40);
+  const uint32_t total_tiles = routed_tiles + (uint32_t)(shared_rows + bm - 1) / bm;
   if (tid == 0) *n_tiles = total_tiles;
   if (tid < E) {
     uint32_t at = start;
@@ -1177,6 +1197,8 @@ __global__ __launch_bounds__(1024) void moe_sort_plan_kernel(int E, int bm, uint
         tile_count[i] = c;
       }
     }
+  if (ordered) shared_tiles(shared_rows, pairs, E, bm, routed_tiles, t_expert, t_start, t_count, pair);
+  else shared_tiles(shared_rows, pairs, E, bm, routed_tiles, tile_expert, tile_start, tile_count, pair);
   __syncthreads();
   if (!ordered) return;
   order_tiles(total_tiles, bm, t_expert, t_start, t_count, tile_expert, tile_start, tile_count);
@@ -1200,6 +1222,40 @@ int check(const ornith_kmatrix* w, const char* who) {
 }
 
 }  // namespace
+
+// What a plan takes: pairs and tile list of the routed experts and, if shared_rows > 0, of the shared one.
+size_t moe_plan_bytes(int pairs, int E, int rows, int shared_rows) {
+  const size_t tiles = (size_t)pairs / rows + (size_t)E + 1 + (size_t)(shared_rows + rows - 1) / rows;
+  return ((size_t)pairs + shared_rows + tiles * 3 + 1 + (size_t)kSortParts * E) * 4 + 6 * 256;
+}
+
+// Lays the plan out in d_plan; with `build` it is made from the pairs' experts first.
+int moe_plan(ornith_ctx* ctx, const uint32_t* d_inds, int pairs, int E, int rows, int shared_rows, void* d_plan, bool build,
+             nmm::Plan* out) {
+  nmm::Plan p{};
+  p.rows = rows;
+  p.tiles_max = (size_t)pairs / rows + (size_t)E + 1 + (size_t)(shared_rows + rows - 1) / rows;
+  ScratchCursor pc(d_plan);
+  p.pair = pc.take<uint32_t>((size_t)pairs + shared_rows);
+  p.tile_expert = pc.take<uint32_t>(p.tiles_max);
+  p.tile_start = pc.take<uint32_t>(p.tiles_max);
+  p.tile_count = pc.take<uint32_t>(p.tiles_max);
+  p.n_tiles = pc.take<uint32_t>(1);
+  uint32_t* parts = pc.take<uint32_t>((size_t)kSortParts * E);
+  if (build && pairs >= 8192) {
+    hipLaunchKernelGGL(moe_sort_count_kernel, dim3(kSortParts), dim3(256), 0, ctx->stream, d_inds, pairs, E, parts);
+    hipLaunchKernelGGL(moe_sort_plan_kernel, dim3(1), dim3(1024), 0, ctx->stream, pairs, E, rows, shared_rows, parts, p.pair,
+                       p.tile_expert, p.tile_start, p.tile_count, p.n_tiles);
+    hipLaunchKernelGGL(moe_sort_scatter_kernel, dim3(kSortParts), dim3(256), 0, ctx->stream, d_inds, pairs, E, parts, p.pair);
+    ORN_LAUNCH_CHECK("moe_sort_*_kernel");
+  } else if (build) {
+    hipLaunchKernelGGL(moe_sort_pairs_kernel, dim3(1), dim3(1024), 0, ctx->stream, d_inds, pairs, E, rows, shared_rows,
+                       p.pair, p.tile_expert, p.tile_start, p.tile_count, p.n_tiles);
+    ORN_LAUNCH_CHECK("moe_sort_pairs_kernel");
+  }
+  *out = p;
+  return ORNITH_OK;
+}
 
 extern "C" {
 
@@ -1279,10 +1335,7 @@ int ornith_kq_matmul(ornith_ctx* ctx, const ornith_kmatrix* w, const void* d_x, 
 
 // gather plan: expert-sorted pairs and the tile list, in caller-provided device memory
 // (ornith_kq_gather_plan_bytes(pairs, E) bytes)
-size_t ornith_kq_gather_plan_bytes(int pairs, int E) {
-  const size_t tiles = (size_t)pairs / 64 + (size_t)E + 1;
-  return ((size_t)pairs + tiles * 3 + 1 + (size_t)kSortParts * E) * 4 + 6 * 256;
-}
+size_t ornith_kq_gather_plan_bytes(int pairs, int E) { return moe_plan_bytes(pairs, E, 16, 0); }
 
 int ornith_kq_gather_matmul(ornith_ctx* ctx, const ornith_kmatrix* w, const void* d_x,
                             const uint32_t* d_inds, int pairs, int top_k, int is_up, void* d_plan,
@@ -1292,47 +1345,37 @@ int ornith_kq_gather_matmul(ornith_ctx* ctx, const ornith_kmatrix* w, const void
   if (rc) return rc;
   ORN_REQUIRE(pairs >= 1 && top_k >= 1 && pairs % top_k == 0 && w->E <= 1024,
               "kq_gather_matmul: pairs=%d top_k=%d E=%d", pairs, top_k, w->E);
-  const size_t tiles_max = (size_t)pairs / 64 + (size_t)w->E + 1;
-  ScratchCursor pc(d_plan);
-  uint32_t* pair = pc.take<uint32_t>(pairs);
-  uint32_t* te = pc.take<uint32_t>(tiles_max);
-  uint32_t* ts = pc.take<uint32_t>(tiles_max);
-  uint32_t* tc = pc.take<uint32_t>(tiles_max);
-  uint32_t* nt = pc.take<uint32_t>(1);
-  uint32_t* parts = pc.take<uint32_t>((size_t)kSortParts * w->E);
   // Rows per plan tile: the choice depends only on pairs and E (and the option), so the calls
   // sharing a plan agree on it. With 48 rows an expert or more: the smallest of 96 / 128 / 160 /
   // 192 rows that holds an expert's share of the pairs with 2.5 standard deviations to spare, so
   // that nearly every expert is one tile (the register form dequantizes its weights once).
-  // Otherwise 128-row tiles from 96 rows an expert on average, else 64.
+  // Otherwise the same rule over the few-row kernels' 16 / 32 / 64 rows.
   const int avg = pairs / w->E;
   int spare = 0;
   while (4 * spare * spare < 25 * avg) ++spare;
   const int need = avg + spare;
-  const bool tall = ornith_option_gemm_reg() && avg >= 48;
-  const int tile_rows = tall ? (need <= 96 ? 96 : need <= 128 ? 128 : need <= 160 ? 160 : 192) : avg >= 96 ? 128 : 64;
-  // The kernel for this matrix. Tall plans take the register form when its 32-bit offsets reach:
+  const bool narrow = pairs < nmm::kNarrowPairs * w->E;
+  const bool tall = ornith_option_gemm_reg() && !narrow;
+  const int tile_rows = narrow ? nmm::tile_rows(pairs, w->E)
+                        : tall ? (need <= 96 ? 96 : need <= 128 ? 128 : need <= 160 ? 160 : 192)
+                               : avg >= 96 ? 128 : 64;
+  // The kernel for this matrix. Few rows an expert: the few-row kernels (mm_narrow.h). Tall plans
+  // take the register form when its 32-bit offsets reach:
   // for K >= 1024 a workgroup a plan tile (one a compute unit), for fewer K slabs 64-row
   // workgroups, two a compute unit (a workgroup's way in and out, which weighs more the fewer
   // slabs there are, then runs beside the other's main loop; the weights still bypass LDS, which
   // is what bounds the LDS form at 64 rows). Otherwise the LDS form: 128 rows a workgroup from 96
   // rows an expert on and K >= 1024, else 64. A plan tile taller than its kernel's workgroups is
   // split over several of them.
-  const size_t x_bytes = (size_t)(is_up ? pairs / top_k : pairs) * w->K * 2;
+  const size_t x_rows = (size_t)(is_up ? pairs / top_k : pairs), x_bytes = x_rows * w->K * 2;
   const size_t q_bytes = (size_t)w->E * w->O * (w->K / 256) * (w->kind == ORNITH_Q4K ? 128 : 192);
   const bool reg = tall && w->K >= 1024 && x_bytes < (size_t(1) << 32) && q_bytes < (size_t(1) << 32);
   const int lds_rows = (avg >= 96 && w->K >= 1024) ? 128 : 64;
-  if (rebuild_plan && pairs >= 8192) {
-    hipLaunchKernelGGL(moe_sort_count_kernel, dim3(kSortParts), dim3(256), 0, ctx->stream, d_inds, pairs, w->E, parts);
-    hipLaunchKernelGGL(moe_sort_plan_kernel, dim3(1), dim3(1024), 0, ctx->stream, w->E, tile_rows, parts, te, ts, tc, nt);
-    hipLaunchKernelGGL(moe_sort_scatter_kernel, dim3(kSortParts), dim3(256), 0, ctx->stream, d_inds, pairs, w->E,
-                       parts, pair);
-    ORN_LAUNCH_CHECK("moe_sort_*_kernel");
-  } else if (rebuild_plan) {
-    hipLaunchKernelGGL(moe_sort_pairs_kernel, dim3(1), dim3(1024), 0, ctx->stream, d_inds, pairs, w->E,
-                       tile_rows, pair, te, ts, tc, nt);
-    ORN_LAUNCH_CHECK("moe_sort_pairs_kernel");
-  }
+  nmm::Plan pl;
+  rc = moe_plan(ctx, d_inds, pairs, w->E, tile_rows, 0, d_plan, rebuild_plan != 0, &pl);
+  if (rc) return rc;
+  if (narrow && nmm::experts_ok(w, d_x, x_rows, d_y)) return nmm::gathered(ctx, w, nullptr, d_x, pairs, is_up ? top_k : 1, pl, d_y);
+  const size_t tiles_max = pl.tiles_max;
   MmArgs a{};
   a.qs = (const uint8_t*)w->d_qs;
   a.scales = (const uint8_t*)w->d_scales;
@@ -1343,12 +1386,12 @@ int ornith_kq_gather_matmul(ornith_ctx* ctx, const ornith_kmatrix* w, const void
   a.O = w->O;
   a.K = w->K;
   a.vec = w->O % 8 == 0 && ((uintptr_t)d_y & 15) == 0;
-  a.pair = pair;
+  a.pair = pl.pair;
   a.up_div = is_up ? top_k : 1;
-  a.tile_expert = te;
-  a.tile_start = ts;
-  a.tile_count = tc;
-  a.n_tiles = nt;
+  a.tile_expert = pl.tile_expert;
+  a.tile_start = pl.tile_start;
+  a.tile_count = pl.tile_count;
+  a.n_tiles = pl.n_tiles;
   if (reg) {
     a.sub = 1;
     const dim3 rgrid((w->O + RN - 1) / RN, (unsigned)tiles_max);

@@ -12,6 +12,7 @@
 // head), so the layout favours a fixed summation order over tuning.
 #include "dmath.h"
 #include "linear_device.h"
+#include "mm_narrow_host.h"
 #include "rt.h"
 
 // kquant.hip
@@ -30,26 +31,7 @@ __global__ __launch_bounds__(64) void affine8_qmv_kernel(const uint8_t* w, const
   const bf16_t* sr = scales + (size_t)o * (K / 64);
   const bf16_t* br = biases + (size_t)o * (K / 64);
   const bf16_t* xr = x + (size_t)m * K;
-  float acc_lane = 0.f;
-  for (int j = lane; j < K / 8; j += 64) {
-    const uint2 q = *reinterpret_cast<const uint2*>(wr + 8 * j);
-    const uint4 xv = *reinterpret_cast<const uint4*>(xr + 8 * j);
-    const float xs[8] = {dm_bf2f_lo(xv.x), dm_bf2f_hi(xv.x), dm_bf2f_lo(xv.y), dm_bf2f_hi(xv.y),
-                         dm_bf2f_lo(xv.z), dm_bf2f_hi(xv.z), dm_bf2f_lo(xv.w), dm_bf2f_hi(xv.w)};
-    const uint32_t qw[2] = {q.x, q.y};
-    float acc = 0.f, sum = 0.f;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const float qf = (float)((qw[i >> 2] >> (8 * (i & 3))) & 0xffu);
-      acc = dm_fma(xs[i], qf, acc);
-      sum = sum + xs[i];
-    }
-    const float s = dm_bf2f(sr[j >> 3]), b = dm_bf2f(br[j >> 3]);
-    float p = s * acc;
-    p = dm_fma(sum, b, p);
-    acc_lane = acc_lane + p;
-  }
-  const float v = dm_wave_sum<64>(acc_lane);
+  const float v = affine8_row_dot(wr, sr, br, xr, K, lane);
   if (lane == 0) y[(size_t)m * O + o] = dm_f2bf(v);
 }
 
@@ -74,29 +56,7 @@ __global__ __launch_bounds__(256) void affine4_qmv_kernel(const uint8_t* w, cons
   const bf16_t* sr = scales + row * (K / 32);
   const bf16_t* br = biases + row * (K / 32);
   const bf16_t* xr = x + xi * K;
-  float acc_lane = 0.f;
-  for (int j = lane; j < K / 16; j += 64) {
-    const uint2 q = *reinterpret_cast<const uint2*>(wr + 8 * j);
-    const uint4 xa = *reinterpret_cast<const uint4*>(xr + 16 * j);
-    const uint4 xb = *reinterpret_cast<const uint4*>(xr + 16 * j + 8);
-    const float xs[16] = {dm_bf2f_lo(xa.x), dm_bf2f_hi(xa.x), dm_bf2f_lo(xa.y), dm_bf2f_hi(xa.y),
-                          dm_bf2f_lo(xa.z), dm_bf2f_hi(xa.z), dm_bf2f_lo(xa.w), dm_bf2f_hi(xa.w),
-                          dm_bf2f_lo(xb.x), dm_bf2f_hi(xb.x), dm_bf2f_lo(xb.y), dm_bf2f_hi(xb.y),
-                          dm_bf2f_lo(xb.z), dm_bf2f_hi(xb.z), dm_bf2f_lo(xb.w), dm_bf2f_hi(xb.w)};
-    const uint32_t qw[2] = {q.x, q.y};
-    float acc = 0.f, sum = 0.f;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const float qf = (float)((qw[i >> 3] >> (4 * (i & 7))) & 0xfu);
-      acc = dm_fma(xs[i], qf, acc);
-      sum = sum + xs[i];
-    }
-    const float s = dm_bf2f(sr[j >> 1]), b = dm_bf2f(br[j >> 1]);
-    float p = s * acc;
-    p = dm_fma(sum, b, p);
-    acc_lane = acc_lane + p;
-  }
-  const float v = dm_wave_sum<64>(acc_lane);
+  const float v = affine4_row_dot(wr, sr, br, xr, K, lane);
   if (lane == 0) y[(size_t)r * O + o] = dm_f2bf(v);
 }
 
@@ -315,13 +275,15 @@ int ornith_linear_matmul(ornith_ctx* ctx, const ornith_linear* w, const void* d_
     case ORNITH_LIN_KQUANT:
       ORN_REQUIRE(w->km.O == w->O && w->km.K == w->K, "linear_matmul: k-quant dims disagree");
       // kquant::matmul (src/ops/kquant.rs:783-800): rows within the exact window go through
-      // the mat-vec (each row as if alone), prefill widths through the tiled GEMM
+      // the mat-vec (each row as if alone), prefill widths through the matrix cores
+      if (nmm::plain_ok(&w, 1, d_x, M, &d_y)) return nmm::plain(ctx, &w, 1, d_x, M, &d_y);
       if (M >= kPrefillRows) return ornith_kq_matmul(ctx, &w->km, d_x, M, d_y);
       return ornith_kq_qmv(ctx, &w->km, d_x, ORNITH_BF16, M, d_y, ORNITH_BF16);
     case ORNITH_LIN_AFFINE8:
       ORN_REQUIRE(w->d_w && w->d_scales && w->d_biases, "linear_matmul: affine tensor missing");
       ORN_REQUIRE(w->K % 64 == 0 && w->O >= 1 && M <= 65535, "linear_matmul: affine O=%d K=%d",
                   w->O, w->K);
+      if (nmm::plain_ok(&w, 1, d_x, M, &d_y)) return nmm::plain(ctx, &w, 1, d_x, M, &d_y);
       hipLaunchKernelGGL(affine8_qmv_kernel, dim3(w->O, M), dim3(64), 0, ctx->stream,
                          (const uint8_t*)w->d_w, (const bf16_t*)w->d_scales,
                          (const bf16_t*)w->d_biases, (const bf16_t*)d_x, (bf16_t*)d_y, w->O, w->K);
@@ -330,6 +292,7 @@ int ornith_linear_matmul(ornith_ctx* ctx, const ornith_linear* w, const void* d_
     case ORNITH_LIN_AFFINE4:
       ORN_REQUIRE(w->d_w && w->d_scales && w->d_biases, "linear_matmul: affine tensor missing");
       ORN_REQUIRE(w->K % 32 == 0 && w->O >= 1 && M <= 65535, "linear_matmul: 4-bit affine O=%d K=%d", w->O, w->K);
+      if (nmm::plain_ok(&w, 1, d_x, M, &d_y)) return nmm::plain(ctx, &w, 1, d_x, M, &d_y);
       hipLaunchKernelGGL(affine4_qmv_kernel<false>, dim3((w->O + 3) / 4, M), dim3(256), 0, ctx->stream,
                          (const uint8_t*)w->d_w, (const bf16_t*)w->d_scales, (const bf16_t*)w->d_biases,
                          (const bf16_t*)d_x, (bf16_t*)d_y, 1, w->O, w->K, M, (const uint32_t*)nullptr,
@@ -383,7 +346,23 @@ int ornith_linear_matmul_multi(ornith_ctx* ctx, const ornith_linear* const* ws, 
     }
     return launch_dense<false>(ctx, s, d_x, ws[0]->K, 1, M, nullptr, nullptr, M);
   }
-  // prefill widths: dense matrices of one K share a launch
+  // Prefill widths: the matrices that take the few-row GEMM share a launch of it (all of them, or the
+  // ones with few columns of a wider call), the others go on below.
+  if (M >= kPrefillRows && ornith_option_fuse_proj() && n >= 2 && n <= 4) {
+    const ornith_linear *few[4], *rest[4];
+    void *yf[4], *yr[4];
+    int nf = 0, nr = 0;
+    for (int i = 0; i < n; ++i) {
+      const bool ok = nmm::plain_ok(&ws[i], 1, d_x, M, &d_ys[i]);
+      (ok ? few[nf] : rest[nr]) = ws[i];
+      (ok ? yf[nf++] : yr[nr++]) = d_ys[i];
+    }
+    if (nf >= 2 && nmm::plain_ok(few, nf, d_x, M, yf)) {
+      const int rc = nmm::plain(ctx, few, nf, d_x, M, yf);
+      return rc || nr == 0 ? rc : ornith_linear_matmul_multi(ctx, rest, nr, d_x, M, yr);
+    }
+  }
+  // ... dense matrices of one K likewise
   if (M >= kPrefillRows && ornith_option_fuse_proj() && n >= 2 && launch_dense_mm(ctx, ws, n, d_x, M, d_ys)) {
     ORN_LAUNCH_CHECK("dense_mm_kernel");
     return ORNITH_OK;

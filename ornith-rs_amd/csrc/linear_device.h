@@ -59,3 +59,58 @@ __device__ __forceinline__ float dense_row_dot(const bf16_t* wr, const bf16_t* x
   dense_rows_dot<1, NU>(rows, xr, K, lane, v);
   return v[0];
 }
+
+// One row of the affine mat-vecs by one wavefront: lane l owns the chunks l + 64c in ascending c
+// (8 codes of the 8-bit group-64 format, 16 of the 4-bit group-32 one), one fma chain a chunk in
+// code order beside the plain sum of its activations, scale * chain + bias * sum per chunk added
+// to the lane's running value, then the butterfly. wr / sr / br: the row's codes, scales, biases.
+__device__ __forceinline__ float affine8_row_dot(const uint8_t* wr, const bf16_t* sr, const bf16_t* br, const bf16_t* xr,
+                                                 int K, int lane) {
+  float acc_lane = 0.f;
+  for (int j = lane; j < K / 8; j += 64) {
+    const uint2 q = *reinterpret_cast<const uint2*>(wr + 8 * j);
+    const uint4 xv = *reinterpret_cast<const uint4*>(xr + 8 * j);
+    const float xs[8] = {dm_bf2f_lo(xv.x), dm_bf2f_hi(xv.x), dm_bf2f_lo(xv.y), dm_bf2f_hi(xv.y),
+                         dm_bf2f_lo(xv.z), dm_bf2f_hi(xv.z), dm_bf2f_lo(xv.w), dm_bf2f_hi(xv.w)};
+    const uint32_t qw[2] = {q.x, q.y};
+    float acc = 0.f, sum = 0.f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const float qf = (float)((qw[i >> 2] >> (8 * (i & 3))) & 0xffu);
+      acc = dm_fma(xs[i], qf, acc);
+      sum = sum + xs[i];
+    }
+    const float s = dm_bf2f(sr[j >> 3]), b = dm_bf2f(br[j >> 3]);
+    float p = s * acc;
+    p = dm_fma(sum, b, p);
+    acc_lane = acc_lane + p;
+  }
+  return dm_wave_sum<64>(acc_lane);
+}
+
+__device__ __forceinline__ float affine4_row_dot(const uint8_t* wr, const bf16_t* sr, const bf16_t* br, const bf16_t* xr,
+                                                 int K, int lane) {
+  float acc_lane = 0.f;
+  for (int j = lane; j < K / 16; j += 64) {
+    const uint2 q = *reinterpret_cast<const uint2*>(wr + 8 * j);
+    const uint4 xa = *reinterpret_cast<const uint4*>(xr + 16 * j);
+    const uint4 xb = *reinterpret_cast<const uint4*>(xr + 16 * j + 8);
+    const float xs[16] = {dm_bf2f_lo(xa.x), dm_bf2f_hi(xa.x), dm_bf2f_lo(xa.y), dm_bf2f_hi(xa.y),
+                          dm_bf2f_lo(xa.z), dm_bf2f_hi(xa.z), dm_bf2f_lo(xa.w), dm_bf2f_hi(xa.w),
+                          dm_bf2f_lo(xb.x), dm_bf2f_hi(xb.x), dm_bf2f_lo(xb.y), dm_bf2f_hi(xb.y),
+                          dm_bf2f_lo(xb.z), dm_bf2f_hi(xb.z), dm_bf2f_lo(xb.w), dm_bf2f_hi(xb.w)};
+    const uint32_t qw[2] = {q.x, q.y};
+    float acc = 0.f, sum = 0.f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const float qf = (float)((qw[i >> 3] >> (4 * (i & 7))) & 0xfu);
+      acc = dm_fma(xs[i], qf, acc);
+      sum = sum + xs[i];
+    }
+    const float s = dm_bf2f(sr[j >> 1]), b = dm_bf2f(br[j >> 1]);
+    float p = s * acc;
+    p = dm_fma(sum, b, p);
+    acc_lane = acc_lane + p;
+  }
+  return dm_wave_sum<64>(acc_lane);
+}

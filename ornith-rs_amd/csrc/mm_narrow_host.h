@@ -1,0 +1,73 @@
+// Host side of the few-row GEMM: what the dispatches of linear.hip, kq_mm.hip and moe.hip ask and
+// call, and the kernels of one weight family.
+#pragma once
+
+#include "mm_narrow.h"
+
+namespace nmm {
+
+// Rows up to which a k-quant projection takes these kernels: the wide kernels' 256 x 128 tiles fill
+// the device from about 200 rows of 4096 columns and more on (12288 x 2048, us: 64 rows 15.8 here against
+// 29.5 there, 128 rows 21 / 29, 256 rows 33 / 31, 700 rows 79 / 68), for up to 2048 columns not before a
+// thousand rows (2048 x 4096: 64 rows 11.8 / 52, 256 rows 17 / 53, 700 rows 35 / 54, 1024 rows 38 / 55;
+// 256 x 2048: 7 / 29, 1024 rows 9 / 29). The rule looks at one matrix at a time, never at what shares
+// its launch: a matrix gives the same bits alone and in company.
+constexpr int kNarrowRows = 192, kNarrowRowsSlim = 1024;
+// pairs an expert below which the routed experts take them
+constexpr int kNarrowPairs = 48;
+
+// an expert-sorted pair list in device memory, tiles of up to `rows` pairs
+struct Plan {
+  uint32_t *pair, *tile_expert, *tile_start, *tile_count, *n_tiles;
+  size_t tiles_max;
+  int rows;
+};
+
+// up to four matrices of one K over the same activations
+bool plain_ok(const ornith_linear* const* ws, int n, const void* d_x, int M, void* const* d_ys);
+int plain(ornith_ctx* ctx, const ornith_linear* const* ws, int n, const void* d_x, int M, void* const* d_ys);
+// rows of a plan tile
+int tile_rows(int pairs, int E);
+bool experts_ok(const ornith_kmatrix* w, const void* d_x, size_t x_rows, const void* d_y);
+// y[p] = x[row of pair p] . w[expert of p]; with `shared`, pairs + t is token t through that matrix
+int gathered(ornith_ctx* ctx, const ornith_kmatrix* w, const ornith_linear* shared, const void* d_x, int pairs, int up_div,
+             const Plan& p, void* d_y);
+// act[p] = swiglu of the gate and up rows, routed and shared
+int gate_up(ornith_ctx* ctx, const ornith_moe_weights* w, const void* d_x, int pairs, const Plan& p, void* d_act);
+bool moe_ok(const ornith_moe_weights* w, const void* d_x, int T, const void* d_act, const void* d_y);
+
+// the launches of a family; the first one on a context's device raises the kernels' LDS limits
+int launch_kq(ornith_ctx* ctx, const Args& a, int mode, int ct, int rows, dim3 grid, int lds);
+int launch_affine(ornith_ctx* ctx, const Args& a, int mode, int ct, int rows, dim3 grid, int lds);
+
+}  // namespace nmm
+
+// The kernels of a family. A plain workgroup is eight wavefronts, two a SIMD; a gathered one four,
+// and as many workgroups a compute unit as accumulators, codes and activation chunks leave room for
+// without spilling (W16, W32: wavefronts a SIMD at 16 and 32 rows).
+#define NMM_KERNELS(NAME, AFF, W16, W32, LDS_BIT)                                                                   \
+  template <int CT>                                                                                                 \
+  __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void NAME##_plain_kernel(Args a) {   \
+    body<AFF, CT, kPlain, 64, 4>(a);                                                                                \
+  }                                                                                                                 \
+  template <int MODE, int ROWS>                                                                                     \
+  __global__ __launch_bounds__(256)                                                                                 \
+      __attribute__((amdgpu_waves_per_eu(ROWS == 16 ? W16 : ROWS == 32 ? W32 : 2))) void NAME##_gather_kernel(Args a) { \
+    body<AFF, 4, MODE, ROWS, 4>(a);                                                                                 \
+  }                                                                                                                 \
+  int launch_##NAME(ornith_ctx* ctx, const Args& a, int mode, int ct, int rows, dim3 grid, int lds) {               \
+    typedef void (*Kernel)(Args);                                                                                   \
+    static const Kernel kernels[9] = {                                                                              \
+        NAME##_plain_kernel<1>,           NAME##_plain_kernel<2>,           NAME##_plain_kernel<4>,                 \
+        NAME##_gather_kernel<kGather, 16>, NAME##_gather_kernel<kGather, 32>, NAME##_gather_kernel<kGather, 64>,    \
+        NAME##_gather_kernel<kGateUp, 16>, NAME##_gather_kernel<kGateUp, 32>, NAME##_gather_kernel<kGateUp, 64>};   \
+    if (!(ctx->lds_attr_set & LDS_BIT)) {                                                                           \
+      for (const Kernel k : kernels)                                                                                \
+        ORN_HIP(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes));        \
+      ctx->lds_attr_set |= LDS_BIT;                                                                                 \
+    }                                                                                                               \
+    const int i = mode == kPlain ? ct / 2 : (mode == kGather ? 3 : 6) + (rows == 16 ? 0 : rows == 32 ? 1 : 2);      \
+    hipLaunchKernelGGL(kernels[i], grid, dim3(256), lds, ctx->stream, a);                    \
+    ORN_LAUNCH_CHECK("nmm::" #NAME);                                                                                \
+    return ORNITH_OK;                                                                                               \
+  }

@@ -1,0 +1,179 @@
+// The few-row GEMM (mm_narrow.h) over Q4_K / Q6_K weights, and the launch rules of both families.
+#include <algorithm>
+
+#include "mm_narrow_host.h"
+
+namespace nmm {
+NMM_KERNELS(kq, false, 4, 3, 4u)
+
+namespace {
+
+int kind_of(const ornith_linear& w) {
+  switch (w.mode) {
+    case ORNITH_LIN_KQUANT: return w.km.kind == ORNITH_Q4K ? kQ4K : w.km.kind == ORNITH_Q6K ? kQ6K : -1;
+    case ORNITH_LIN_AFFINE4: return kA4;
+    case ORNITH_LIN_AFFINE8: return kA8;
+    default: return -1;
+  }
+}
+int kind_of(const ornith_kmatrix& w) {
+  return w.kind == ORNITH_Q4K ? kQ4K : w.kind == ORNITH_Q6K ? kQ6K : w.kind == ORNITH_AFFINE4_G32 ? kA4 : -1;
+}
+bool affine(int kind) { return kind >= kA4; }
+
+Mat mat_of(const ornith_linear& w, void* y) {
+  if (w.mode == ORNITH_LIN_KQUANT)
+    return {(const uint8_t*)w.km.d_qs, (const uint8_t*)w.km.d_scales, (const uint8_t*)w.km.d_dm, (bf16_t*)y, w.O, kind_of(w), 0};
+  return {(const uint8_t*)w.d_w, (const uint8_t*)w.d_scales, (const uint8_t*)w.d_biases, (bf16_t*)y, w.O, kind_of(w), 0};
+}
+Mat mat_of(const ornith_kmatrix& w, void* y) {
+  return {(const uint8_t*)w.d_qs, (const uint8_t*)w.d_scales, (const uint8_t*)w.d_dm, (bf16_t*)y, w.O, kind_of(w), 0};
+}
+// the kernels' 16-byte loads (the scales of 16 rows, or of what is left of the matrix, are whole
+// 16-byte pieces) and 32-bit offsets inside one matrix
+bool reachable(const Mat& m, int K) {
+  return m.kind >= 0 && m.O >= 1 && m.q && m.s && m.d && (size_t)m.O * K < (size_t(1) << 32) && m.O * (size_t)(K / 256) % 8 == 0 &&
+         (((uintptr_t)m.q | (uintptr_t)m.s | (uintptr_t)m.d) & 15) == 0 && ((uintptr_t)m.y & 7) == 0;
+}
+// LDS of a launch: activations and scales (of the widest format), or the partial tiles
+int lds_bytes(const Args& a, int mats, int halves, int cols, int rows, int ct, int nw) {
+  int per_block = 0;
+  for (int i = 0; i < mats; ++i)
+    if (a.m[i].q) per_block = std::max(per_block, s_bytes(a.m[i].kind) + d_bytes(a.m[i].kind));
+  return std::max(x_bytes(rows, nw) + halves * cols * (a.K / 256) * per_block, red_bytes(rows, ct, nw));
+}
+// wavefronts of NW that split K: as many as there are 256-wide blocks, a power of two
+int k_split(int K, int nw) {
+  int ks = 1;
+  while (2 * ks <= nw && 2 * ks <= K / 256) ks *= 2;
+  return ks;
+}
+
+}  // namespace
+
+bool plain_ok(const ornith_linear* const* ws, int n, const void* d_x, int M, void* const* d_ys) {
+  if (n < 1 || n > 4 || M < kPrefillRows || ((uintptr_t)d_x & 15) != 0) return false;
+  const int K = ws[0]->K;
+  if (K < 512 || K % 256 != 0 || (size_t)M * K * 2 >= (size_t(1) << 32)) return false;
+  for (int i = 0; i < n; ++i) {
+    const Mat m = mat_of(*ws[i], d_ys[i]);
+    if (!reachable(m, K) || ws[i]->K != K || affine(m.kind) != affine(kind_of(*ws[0]))) return false;
+    if (ws[i]->mode == ORNITH_LIN_KQUANT && (ws[i]->km.E != 1 || ws[i]->km.O != ws[i]->O || ws[i]->km.K != K)) return false;
+  }
+  if (K > 4096) return false;  // (the scales of a workgroup's rows would not fit beside the activations)
+  // The k-quants have wide kernels of their own; the affine formats do not.
+  if (affine(kind_of(*ws[0]))) return true;
+  for (int i = 0; i < n; ++i)
+    if (M > (ws[i]->O > 2048 ? kNarrowRows : kNarrowRowsSlim)) return false;
+  return true;
+}
+
+int plain(ornith_ctx* ctx, const ornith_linear* const* ws, int n, const void* d_x, int M, void* const* d_ys) {
+  Args a{};
+  a.n = n;
+  a.x = (const bf16_t*)d_x;
+  a.M = M;
+  a.K = ws[0]->K;
+  a.ks = k_split(a.K, 4);
+  const int row_tiles = (M + 63) / 64;
+  // Columns a workgroup: 64 (four tiles a wavefront, each activation fragment used four times)
+  // once that gives most compute units a workgroup, else 32 or 16.
+  int ct = 4, blocks = 0;
+  for (;; ct /= 2) {
+    const int cols = (4 / a.ks) * ct * 16;
+    blocks = 0;
+    for (int i = 0; i < n; ++i) blocks += (ws[i]->O + cols - 1) / cols;
+    if (ct == 1 || blocks * row_tiles >= 3 * ctx->compute_units / 4) break;
+  }
+  const int cols = (4 / a.ks) * ct * 16;
+  blocks = 0;
+  for (int i = 0; i < n; ++i) {
+    a.m[i] = mat_of(*ws[i], d_ys[i]);
+    a.m[i].cb0 = blocks;
+    blocks += (ws[i]->O + cols - 1) / cols;
+  }
+  const dim3 grid(blocks, row_tiles);
+  const int lds = lds_bytes(a, n, 1, cols, 64, ct, 4);
+  return affine(a.m[0].kind) ? launch_affine(ctx, a, kPlain, ct, 64, grid, lds) : launch_kq(ctx, a, kPlain, ct, 64, grid, lds);
+}
+
+int tile_rows(int pairs, int E) {
+  // The smallest tile that most experts' shares of the pairs fit (an expert over it takes a second
+  // tile and has its weights unpacked twice): one standard deviation to spare. Smaller tiles keep
+  // more wavefronts on a compute unit, which pays for the few that spill over (5600 pairs of 256
+  // experts, gate and up / down: 64-row tiles 134 / 88 us, 32-row ones 113 / 77).
+  const int avg = (pairs + E - 1) / E;
+  int spare = 0;
+  while (spare * spare < avg) ++spare;
+  return avg + spare <= 16 ? 16 : avg + spare <= 32 ? 32 : 64;
+}
+
+bool experts_ok(const ornith_kmatrix* w, const void* d_x, size_t x_rows, const void* d_y) {
+  return w->K >= 512 && w->K <= 4096 && w->K % 256 == 0 && w->E <= 1024 && ((uintptr_t)d_x & 15) == 0 &&
+         x_rows * w->K * 2 < (size_t(1) << 32) && reachable(mat_of(*w, const_cast<void*>(d_y)), w->K);
+}
+
+namespace {
+int launch_gathered(ornith_ctx* ctx, Args& a, int mode, const Plan& p, int O) {
+  a.ks = k_split(a.K, 4);
+  a.pair = p.pair;
+  a.tile_expert = p.tile_expert;
+  a.tile_start = p.tile_start;
+  a.tile_count = p.tile_count;
+  a.n_tiles = p.n_tiles;
+  const int cols = (4 / a.ks) * (mode == kGateUp ? 2 : 4) * 16;
+  const dim3 grid((O + cols - 1) / cols, (unsigned)p.tiles_max);
+  const int lds = lds_bytes(a, 4, mode == kGateUp ? 2 : 1, cols, p.rows, 4, 4);
+  return affine(a.m[0].kind) ? launch_affine(ctx, a, mode, 4, p.rows, grid, lds) : launch_kq(ctx, a, mode, 4, p.rows, grid, lds);
+}
+}  // namespace
+
+int gathered(ornith_ctx* ctx, const ornith_kmatrix* w, const ornith_linear* shared, const void* d_x, int pairs, int up_div,
+             const Plan& p, void* d_y) {
+  Args a{};
+  a.m[0] = mat_of(*w, d_y);
+  if (shared) a.m[2] = mat_of(*shared, d_y);
+  a.x = (const bf16_t*)d_x;
+  a.M = pairs;
+  a.K = w->K;
+  a.up_div = up_div;
+  a.pairs = pairs;
+  a.E = w->E;
+  return launch_gathered(ctx, a, kGather, p, w->O);
+}
+
+int gate_up(ornith_ctx* ctx, const ornith_moe_weights* w, const void* d_x, int pairs, const Plan& p, void* d_act) {
+  Args a{};
+  a.m[0] = mat_of(w->ex_gate, d_act);
+  a.m[1] = mat_of(w->ex_up, d_act);
+  a.m[2] = mat_of(w->sh_gate, d_act);
+  a.m[3] = mat_of(w->sh_up, d_act);
+  a.x = (const bf16_t*)d_x;
+  a.M = pairs;
+  a.K = w->ex_gate.K;
+  a.up_div = w->top_k;
+  a.pairs = pairs;
+  a.E = w->ex_gate.E;
+  return launch_gathered(ctx, a, kGateUp, p, w->ex_gate.O);
+}
+
+bool moe_ok(const ornith_moe_weights* w, const void* d_x, int T, const void* d_act, const void* d_y) {
+  if (w->ex_dense) return false;
+  const int pairs = T * w->top_k, E = w->ex_gate.E, H = w->router.K;
+  const int kg = kind_of(w->ex_gate), sg = kind_of(w->sh_gate);
+  if (kg < 0 || sg < 0 || kind_of(w->ex_up) != kg || kind_of(w->sh_up) != sg || w->sh_gate.O != w->ex_gate.O) return false;
+  if (affine(kg) != affine(sg) || affine(kind_of(w->ex_down)) != affine(kg) || affine(kind_of(w->sh_down)) != affine(kg)) return false;
+  if (!experts_ok(&w->ex_gate, d_x, T, d_act) || !experts_ok(&w->ex_up, d_x, T, d_act) ||
+      !experts_ok(&w->ex_down, d_act, (size_t)pairs + T, d_y))
+    return false;
+  const ornith_linear* sh[3] = {&w->sh_gate, &w->sh_up, &w->sh_down};
+  for (int i = 0; i < 3; ++i) {
+    if (!reachable(mat_of(*sh[i], const_cast<void*>(i < 2 ? d_act : d_y)), sh[i]->K)) return false;
+    if (sh[i]->mode == ORNITH_LIN_KQUANT && (sh[i]->km.O != sh[i]->O || sh[i]->km.K != sh[i]->K || sh[i]->km.E != 1)) return false;
+  }
+  if (w->ex_gate.O % 4 != 0 || H % 4 != 0) return false;
+  // experts with many rows belong to the tall tiles of kq_mm.hip; the affine format has none
+  return affine(kg) || pairs < kNarrowPairs * E;
+}
+
+}  // namespace nmm

@@ -9,6 +9,10 @@
 //
 // Rounding points are the reference's: gates, probabilities, every expert output
 // and every step of the tail are bf16; sums inside a kernel are fp32.
+#include <algorithm>
+
+#include "linear_device.h"
+#include "mm_narrow_host.h"
 #include "moe_device.h"
 #include "norm_device.h"
 #include "rt.h"
@@ -32,6 +36,10 @@ int moe_affine4_experts(ornith_ctx* ctx, const ornith_moe_weights* w, const void
 bool moe_dense_supported(const ornith_moe_weights* w);
 int moe_dense_experts(ornith_ctx* ctx, const ornith_moe_weights* w, const void* d_x, int T, const uint32_t* d_inds,
                       const void* d_scores, const void* d_egate, void* d_act, void* d_out, const void* d_gates);
+// kq_mm.hip
+size_t moe_plan_bytes(int pairs, int E, int rows, int shared_rows);
+int moe_plan(ornith_ctx* ctx, const uint32_t* d_inds, int pairs, int E, int rows, int shared_rows, void* d_plan, bool build,
+             nmm::Plan* out);
 int moe_fused_experts(ornith_ctx* ctx, const ornith_moe_weights* w, const void* d_x, int T,
                       const uint32_t* d_inds, const void* d_scores, const void* d_egate, void* d_act,
                       void* d_out, int phases, const void* d_gates);
@@ -56,6 +64,26 @@ __global__ __launch_bounds__(64) void router_topk_kernel(const bf16_t* gates, in
     if (lhs_tok) lhs_tok[t * k + lane] = t;
     if (lhs_row) lhs_row[t * k + lane] = t * k + lane;
   }
+}
+
+// The router's tail at prefill widths, one wavefront a token: the shared expert's gate (one affine
+// row dot, its loads ahead of the softmax's arithmetic) and softmax + top-k.
+struct EgateArgs {
+  const uint8_t* w;
+  const bf16_t *s, *b, *x;
+  bf16_t* y;
+  int K, bits;  // bits 0: not made here
+};
+template <int PER>
+__global__ __launch_bounds__(64) void router_egate_kernel(const bf16_t* gates, int E, int k, uint32_t* inds,
+                                                          bf16_t* scores, EgateArgs g) {
+  const int t = blockIdx.x, lane = threadIdx.x;
+  if (g.bits) {
+    const bf16_t* xr = g.x + (size_t)t * g.K;
+    const float v = g.bits == 8 ? affine8_row_dot(g.w, g.s, g.b, xr, g.K, lane) : affine4_row_dot(g.w, g.s, g.b, xr, g.K, lane);
+    if (lane == 0) g.y[t] = dm_f2bf(v);
+  }
+  router_topk_wave<PER>(gates + (size_t)t * E, k, inds + (size_t)t * k, scores + (size_t)t * k, nullptr, lane);
 }
 
 // V consecutive elements a thread (V = 8: 16-byte loads and stores; V = 1 for odd sizes)
@@ -157,6 +185,76 @@ int launch_router(ornith_ctx* ctx, const bf16_t* gates, int T, int E, int k, uin
 #undef ROUTER_CASE
   ORN_LAUNCH_CHECK("router_topk_kernel");
   return ORNITH_OK;
+}
+
+int launch_router_egate(ornith_ctx* ctx, const bf16_t* gates, int T, int E, int k, uint32_t* inds, bf16_t* scores,
+                        const ornith_linear& w, const bf16_t* x, bf16_t* egate) {
+  EgateArgs g{};
+  if (w.mode == ORNITH_LIN_AFFINE8 || w.mode == ORNITH_LIN_AFFINE4) {
+    ORN_REQUIRE(w.d_w && w.d_scales && w.d_biases && w.K % 64 == 0, "moe_block: shared expert gate K=%d", w.K);
+    g = {(const uint8_t*)w.d_w, (const bf16_t*)w.d_scales, (const bf16_t*)w.d_biases, x, egate, w.K, w.mode == ORNITH_LIN_AFFINE8 ? 8 : 4};
+  } else {
+    const int rc = ornith_linear_matmul(ctx, &w, x, T, egate);
+    if (rc) return rc;
+  }
+#define ROUTER_CASE(P)                                                                                         \
+  case P:                                                                                                      \
+    hipLaunchKernelGGL(router_egate_kernel<P>, dim3(T), dim3(64), 0, ctx->stream, gates, E, k, inds, scores, g); \
+    break;
+  switch (E / 64) {
+    ROUTER_CASE(1)
+    ROUTER_CASE(2)
+    ROUTER_CASE(4)
+    ROUTER_CASE(8)
+    ROUTER_CASE(16)
+    default:
+      return ornith_fail(ORNITH_ERR_UNSUPPORTED, "router_topk: E=%d (need 64,128,256,512,1024)", E);
+  }
+#undef ROUTER_CASE
+  ORN_LAUNCH_CHECK("router_egate_kernel");
+  return ORNITH_OK;
+}
+
+// Prompts of few rows an expert (and any prompt over affine experts, which have no wide form): the
+// shared expert is one more expert of the pair list, so the block is six launches: router, its
+// tail (shared gate, softmax + top-k), plan, gate + up + swiglu, down, combine.
+// false: the shapes are not covered.
+bool moe_block_narrow(ornith_ctx* ctx, const ornith_moe_weights* w, const void* d_x, int T, void* d_out, int* rc_out) {
+  const int E = w->router.O, H = w->router.K, I = w->ex_gate.O, k = w->top_k, pairs = T * k;
+  if (E % 64 != 0 || E > 1024) return false;
+  const int rows = nmm::tile_rows(pairs, E);
+  const size_t plan_bytes = moe_plan_bytes(pairs, E, rows, T);
+  const size_t need = 2 * ((size_t)T * E + T + (size_t)(pairs + T) * (I + H) + (size_t)pairs) + 4 * (size_t)pairs + plan_bytes + 16 * 256;
+  void* base = nullptr;
+  int rc = *rc_out = ornith_scratch(ctx, need, &base);
+  if (rc) return true;
+  ScratchCursor sc(base);
+  bf16_t* gates = sc.take<bf16_t>((size_t)T * E);
+  uint32_t* inds = sc.take<uint32_t>(pairs);
+  bf16_t* scores = sc.take<bf16_t>(pairs);
+  bf16_t* eg = sc.take<bf16_t>(T);
+  bf16_t* act = sc.take<bf16_t>((size_t)(pairs + T) * I);
+  bf16_t* y = sc.take<bf16_t>((size_t)(pairs + T) * H);
+  void* plan = sc.take<char>(plan_bytes);
+  if (!nmm::moe_ok(w, d_x, T, act, y)) return false;
+  nmm::Plan pl;
+  auto go = [&]() -> int {
+#define TRY(e)          \
+  do {                  \
+    rc = (e);           \
+    if (rc) return rc;  \
+  } while (0)
+    TRY(ornith_linear_matmul(ctx, &w->router, d_x, T, gates));
+    TRY(launch_router_egate(ctx, gates, T, E, k, inds, scores, w->sh_egate, (const bf16_t*)d_x, eg));
+    TRY(moe_plan(ctx, inds, pairs, E, rows, T, plan, true, &pl));
+    TRY(nmm::gate_up(ctx, w, d_x, pairs, pl, act));
+    TRY(nmm::gathered(ctx, &w->ex_down, &w->sh_down, act, pairs, 1, pl, y));
+    TRY(ornith_moe_combine(ctx, scores, y, eg, y + (size_t)pairs * H, T, k, H, w->norm_topk_prob, d_out));
+#undef TRY
+    return ORNITH_OK;
+  };
+  *rc_out = go();
+  return true;
 }
 
 // Prefill widths: the same block with every projection as a matrix-core GEMM and the routed
@@ -308,15 +406,21 @@ static int moe_block_impl(ornith_ctx* ctx, const ornith_moe_weights* w, const vo
   if (ex_affine4)
     ORN_REQUIRE(w->ex_up.kind == ORNITH_AFFINE4_G32 && w->ex_down.kind == ORNITH_AFFINE4_G32,
                 "moe_block: the three expert stacks must share the 4-bit affine format");
+  if (T >= kPrefillRows && !w->ex_dense && !d_inds_out && !d_scores_out) {
+    int rcn = ORNITH_OK;
+    if (moe_block_narrow(ctx, w, d_x, T, d_out, &rcn)) return rcn;
+  }
   if (T >= kPrefillRows && !w->ex_dense && !ex_affine4) {
     ORN_REQUIRE(!d_inds_out && !d_scores_out, "moe_block: index outputs are a decode-width feature");
     return moe_block_prefill(ctx, w, d_x, T, d_out);
   }
-  if (T > 64) {
-    // dense and 4-bit affine experts have no prefill-width form: the operator path takes the
-    // rows in blocks of 64 (rows are independent of each other, so the result is the same)
-    for (int t0 = 0; t0 < T; t0 += 64) {
-      const int n = T - t0 < 64 ? T - t0 : 64;
+  // dense experts have no prefill-width form, and the ids and scores are made by the exact path:
+  // the rows go in blocks (they are independent of each other, so the result is the same) of 64,
+  // of affine experts in blocks inside the exact window, so that every projection stays exact
+  const int block = ex_affine4 ? std::min(64, kPrefillRows - 1) : 64;
+  if (T > block) {
+    for (int t0 = 0; t0 < T; t0 += block) {
+      const int n = std::min(block, T - t0);
       const int rcb = moe_block_impl(ctx, w, static_cast<const bf16_t*>(d_x) + (size_t)t0 * H, n,
                                      static_cast<bf16_t*>(d_out) + (size_t)t0 * H,
                                      d_inds_out ? d_inds_out + (size_t)t0 * k : nullptr,

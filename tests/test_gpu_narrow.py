@@ -1,0 +1,71 @@
+"""GPU: the few-row GEMM over quantized weights (csrc/mm_narrow.h) at the edges of its row tiles and
+column blocks, against a float64 product: of the weights rounded to bf16 for the k-quants (what
+the kernel feeds the matrix cores), of the true weights for the affine formats (which it does not
+round), and the MoE block built on it against the oracle's exact block."""
+import numpy as np
+import pytest
+
+import util
+from util import Q4K, Q6K
+
+pytestmark = pytest.mark.gpu
+
+
+def _weights(lin):
+    if lin.mode == "kq":
+        w = util.orc_dequant(lin.km.kind, lin.km.qs, lin.km.scales, lin.km.dm, lin.O * lin.K // 256)
+        return util.bf16_to_f32(util.f32_to_bf16(w)).astype(np.float64).reshape(lin.O, lin.K)
+    if lin.mode == "affine4":
+        q = np.stack([lin.w & 15, lin.w >> 4], -1).reshape(lin.O, lin.K).astype(np.float64)
+        g = 32
+    else:
+        q, g = lin.w.astype(np.float64), 64
+    s, b = (np.repeat(util.bf16_to_f32(t).astype(np.float64), g, axis=1) for t in (lin.scales, lin.biases))
+    return q * s + b
+
+
+@pytest.mark.parametrize("fmt", ["q4k", "q6k", "affine4", "affine8"])
+@pytest.mark.parametrize("O,K,M", [(512, 2048, 32), (200, 512, 33), (264, 768, 48), (2048, 4096, 65), (40, 1024, 130),
+                                    (4096, 2048, 64), (64, 4096, 17 + 64), (8, 2048, 200)])
+def test_few_row_matmul_vs_float64(orn, ctx, fmt, O, K, M):
+    rng = np.random.default_rng(O + K + M)
+    lin = (util.HostLinear.kq(rng, Q4K if fmt == "q4k" else Q6K, O, K) if fmt[0] == "q" else
+           getattr(util.HostLinear, fmt)(rng, O, K))
+    dl = lin.dev(orn, ctx)
+    xb = util.bf16_normal(rng, (M, K))
+    dx, dy = ctx.to_device(xb), ctx.alloc(M * O * 2)
+    ctx.memset(dy, 0xFF, M * O * 2)
+    ctx.linear_matmul(dl, dx, M, dy)
+    got = util.bf16_to_f32(dy.download(np.uint16, (M, O))).astype(np.float64)
+    want = util.bf16_to_f32(xb).astype(np.float64) @ _weights(lin).T
+    scale = np.sqrt(np.mean(want ** 2))
+    # one rounding of the output, and fp32 sums in another order
+    assert np.all(np.abs(got - want) <= 2.0 ** -8 * np.abs(want) + 2e-5 * scale), float(np.abs(got - want).max() / scale)
+    for b in (dx, dy): b.free()
+    dl.free()
+
+
+@pytest.mark.parametrize("fmt", ["kq", "affine4"])
+@pytest.mark.parametrize("T", [32, 100, 150, 300])
+def test_few_row_moe_block_vs_exact(orn, ctx, fmt, T):
+    """16-, 32- and 64-row expert tiles (4 to 38 rows an expert on average), the shared expert among
+    them. A router tie may fall the other way than in the oracle's exact block: such a row differs by an
+    expert, so the bound is on the rows' median and 93 % of them."""
+    rng = np.random.default_rng(T)
+    moe = util.HostMoe(rng, H=1024, E=64, I=512, top_k=8, gate_kind=util.AFFINE4 if fmt == "affine4" else Q4K)
+    xb = util.bf16_normal(rng, (T, 1024))
+    want = util.bf16_to_f32(util.orc_moe_block(moe, xb, T)[0]).astype(np.float64)
+    w = moe.dev(orn, ctx)
+    dx, out = ctx.to_device(xb), ctx.alloc(T * 1024 * 2)
+    outs = []
+    for fill in (0xFF, 0x00):
+        ctx.memset(out, fill, T * 1024 * 2)
+        ctx.moe_block(w, dx, T, out)
+        outs.append(out.download(np.uint16, (T, 1024)))
+    assert np.array_equal(outs[0], outs[1])
+    got = util.bf16_to_f32(outs[0]).astype(np.float64)
+    rel = np.linalg.norm(got - want, axis=1) / np.linalg.norm(want, axis=1)
+    bound = 0.004 if fmt == "affine4" else 0.01
+    assert np.median(rel) < bound and (rel < 0.03).mean() >= 0.93, (float(np.median(rel)), float(np.sort(rel)[-5]))
+    for b in (dx, out): b.free()
+    moe.free()
