@@ -151,6 +151,9 @@ struct ornith_caches {
   int capacity = 0, max_window = 0, conv_rows = 0;
   bool growable = true;  // a forward past the capacity grows the KV tensors (else it is refused)
   std::vector<LayerCache> layers;
+  ornith_zero_range* d_zero = nullptr;  // what a reset clears: the first window rows and state slot of every gated-delta layer
+  int n_zero = 0;
+  size_t zero_max = 0;
   // one set of cursors serves every layer: they all advance together
   int offset = 0;     // tokens held
   int conv_cur = 0;   // which conv buffer holds the live window

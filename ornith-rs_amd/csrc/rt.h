@@ -49,6 +49,14 @@ int ornith_scratch(ornith_ctx* ctx, size_t bytes, void** out);
 int ornith_gather_rows(ornith_ctx* ctx, const void* d_src, size_t row_bytes, const uint32_t* d_ids,
                        int n, void* d_dst);
 
+// n ranges of device memory (16-byte aligned, a multiple of 16 bytes each) set to zero in one launch;
+// the list itself is in device memory, max_bytes is its longest range
+struct ornith_zero_range {
+  void* p;
+  size_t bytes;
+};
+int ornith_zero_ranges(ornith_ctx* ctx, const ornith_zero_range* d_ranges, int n, size_t max_bytes);
+
 // bump allocator over a scratch block
 struct ScratchCursor {
   char* base;

@@ -112,6 +112,23 @@ int ornith_gather_rows(ornith_ctx* ctx, const void* d_src, size_t row_bytes, con
   return ORNITH_OK;
 }
 
+// Ranges of 16-byte pieces set to zero, range blockIdx.y, 16 KB a workgroup.
+__global__ __launch_bounds__(256) void zero_ranges_kernel(const ornith_zero_range* r) {
+  const ornith_zero_range z = r[blockIdx.y];
+  uint4* p = static_cast<uint4*>(z.p);
+  size_t i = (size_t)blockIdx.x * 1024 + threadIdx.x;
+#pragma unroll
+  for (int n = 0; n < 4; ++n, i += 256)
+    if (i < z.bytes / 16) p[i] = make_uint4(0, 0, 0, 0);
+}
+
+int ornith_zero_ranges(ornith_ctx* ctx, const ornith_zero_range* d_ranges, int n, size_t max_bytes) {
+  ORN_REQUIRE(ctx && d_ranges && n >= 1 && n <= 65535, "zero_ranges: bad argument");
+  hipLaunchKernelGGL(zero_ranges_kernel, dim3((unsigned)((max_bytes + 16383) / 16384), n), dim3(256), 0, ctx->stream, d_ranges);
+  ORN_LAUNCH_CHECK("zero_ranges_kernel");
+  return ORNITH_OK;
+}
+
 extern "C" {
 
 int ornith_set_option(const char* name, int value) {
