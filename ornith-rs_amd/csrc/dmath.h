@@ -127,12 +127,27 @@ __device__ __forceinline__ float dm_log1p(float u) {
 
 __device__ __forceinline__ float dm_rsqrt(float x) { return 1.0f / __builtin_sqrtf(x); }
 
-// sigmoid with every intermediate held in bf16
+// sigmoid of a bf16 number with every intermediate held in bf16
 // (/root/reference/kernels/ornith_sigmoid.h:27-31 at T = bfloat16).
+//
+// The exponential and the reciprocal are the hardware's: what is kept of each is a bf16, and no
+// input brings them within their own error of a rounding boundary. For the reciprocal that follows
+// from the numbers: s = a / 2^j with a in [128, 256), and 128 / a is either a power of two or at
+// least 2^-18 away from every odd multiple of a half bf16 step. For the exponential, whose argument
+// x * log2(e) enters with its rounding error as a second term, it is a matter of the 2^15 inputs
+// there are, all of which are compared with the form that dm_exp and a division give
+// (tests/test_gpu_kquant.py). 16 vector instructions instead of 50: in the gated-delta front end
+// and swiglu at prompt widths the two functions were most of what a channel cost.
 __device__ __forceinline__ float dm_sigmoid_bf16(float x) {
-  float e = dm_rb(dm_exp(__builtin_fabsf(x)));
-  float s = dm_rb(1.0f + e);
-  float y = dm_rb(1.0f / s);
+  const float a = __builtin_fabsf(x);
+  const float t = a * 1.44269504088896341f;
+  const float lo = dm_fma(a, 1.925963033e-8f, dm_fma(a, 1.44269504088896341f, -t));
+  float e = __builtin_amdgcn_exp2f(t);
+  e = dm_fma(e * 0.693147180559945309f, lo, e);
+  e = dm_rb(a > 88.0f ? DM_INF : e);
+  const float s = dm_rb(1.0f + e);
+  // (scaled: the instruction flushes results below the normal range, and 1 / exp(88) is there)
+  const float y = dm_rb(__builtin_amdgcn_rcpf(s * 0x1p-32f) * 0x1p-32f);
   return (x < 0.0f) ? y : dm_rb(1.0f - y);
 }
 __device__ __forceinline__ float dm_sigmoid_f32(float x) {

@@ -104,22 +104,36 @@ __global__ __launch_bounds__(64) void gdn_front_kernel(FrontArgs p) {
   }
 }
 
-// The same for a run of tokens per workgroup (kernel size 4, prefill widths): the taps are
+// The same for a run of tokens per wavefront (kernel size 4, prefill widths): the taps are
 // loaded once and each token's inputs are read once and kept as the sliding window, instead of
 // one 64-thread workgroup per token and 128 channels. Per token the arithmetic and its order
-// are those of gdn_front_kernel. grid (D / 128, ceil(T / kFrontRun)), 64 threads.
-constexpr int kFrontRun = 16;
+// are those of gdn_front_kernel; the decays and betas have grid column D / 128 to themselves (in
+// the wavefront of a conv column they were a second run of exponentials and logarithms behind its
+// own). What bounds it: vector instructions at long prompts (two exponentials, two reciprocals
+// and half a norm a channel pair), the run's serial chain at short ones. So the run is 16 tokens
+// where that still fills the chip and 4 below.
+// grid (D / 128 + 1, ceil(T / RUN)), 64 threads.
+template <int RUN>
 __global__ __launch_bounds__(64) void gdn_front_run_kernel(FrontArgs p) {
   constexpr int K = 4, S = K - 1;
-  const int slot = blockIdx.x, t0 = blockIdx.y * kFrontRun, lane = threadIdx.x;
+  const int slot = blockIdx.x, t0 = blockIdx.y * RUN, lane = threadIdx.x;
   const int D = p.D, c0 = slot * 128 + 2 * lane, key_dim = p.Hk * 128;
-  const int t1 = min(t0 + kFrontRun, p.T);
+  const int t1 = min(t0 + RUN, p.T);
+  if (c0 >= D) {
+    for (int i = t0 * p.Hv + lane; i < t1 * p.Hv; i += 64) {
+      const int h = i % p.Hv;
+      const float sp = softplus_bf16(dm_rb(dm_bf2f(p.a_in[i]) + dm_bf2f(p.dt_bias[h])));
+      const float decay = dm_exp(dm_bf2f(p.a_log[h]));
+      p.g[i] = dm_exp(-decay * sp);
+      p.beta[i] = dm_f2bf(dm_sigmoid_bf16(dm_bf2f(p.b_in[i])));
+    }
+    return;
+  }
   float w0[K], w1[K];
   {
-    const uint2 a = *reinterpret_cast<const uint2*>(p.cw + (size_t)c0 * K);
-    const uint2 b = *reinterpret_cast<const uint2*>(p.cw + (size_t)(c0 + 1) * K);
+    const uint4 a = *reinterpret_cast<const uint4*>(p.cw + (size_t)c0 * K);
     w0[0] = dm_bf2f_lo(a.x); w0[1] = dm_bf2f_hi(a.x); w0[2] = dm_bf2f_lo(a.y); w0[3] = dm_bf2f_hi(a.y);
-    w1[0] = dm_bf2f_lo(b.x); w1[1] = dm_bf2f_hi(b.x); w1[2] = dm_bf2f_lo(b.y); w1[3] = dm_bf2f_hi(b.y);
+    w1[0] = dm_bf2f_lo(a.z); w1[1] = dm_bf2f_hi(a.z); w1[2] = dm_bf2f_lo(a.w); w1[3] = dm_bf2f_hi(a.w);
   }
   // window position j holds conv_state[j] for j < S, qkv[j - S] from there on
   auto input = [&](int j) {
@@ -137,11 +151,11 @@ __global__ __launch_bounds__(64) void gdn_front_run_kernel(FrontArgs p) {
   const float sc = is_q ? p.q_scale : p.k_scale;
   // the run's inputs are asked for together (one after the other, every token would wait out a
   // memory latency of its own); rows past the end of the call read the last row, unused
-  uint32_t in[kFrontRun];
+  uint32_t in[RUN];
 #pragma unroll
-  for (int u = 0; u < kFrontRun; ++u) in[u] = input(min(t0 + u, p.T - 1) + S);
+  for (int u = 0; u < RUN; ++u) in[u] = input(min(t0 + u, p.T - 1) + S);
 #pragma unroll
-  for (int u = 0; u < kFrontRun; ++u) {
+  for (int u = 0; u < RUN; ++u) {
     const int t = t0 + u;
     if (t >= t1) break;
     win[S] = in[u];  // = qkv[t]
@@ -161,20 +175,11 @@ __global__ __launch_bounds__(64) void gdn_front_run_kernel(FrontArgs p) {
       ss = dm_fma(y1, y1, ss);
       const float inv = dm_rsqrt(dm_wave_sum<64>(ss) / 128.0f + p.eps);
       bf16_t* dst = (is_q ? p.q : p.k) + (size_t)t * key_dim + (is_q ? c0 : c0 - key_dim);
-      const uint32_t lo = dm_f2bf(sc * dm_rb(y0 * inv)), hi = dm_f2bf(sc * dm_rb(y1 * inv));
-      *reinterpret_cast<uint32_t*>(dst) = lo | (hi << 16);
+      const uint32_t n = dm_f2bf2(y0 * inv, y1 * inv);
+      *reinterpret_cast<uint32_t*>(dst) = dm_f2bf2(sc * dm_bf2f_lo(n), sc * dm_bf2f_hi(n));
     } else {
       bf16_t* dst = p.v + (size_t)t * (D - 2 * key_dim) + (c0 - 2 * key_dim);
-      *reinterpret_cast<uint32_t*>(dst) = (uint32_t)dm_f2bf(y0) | ((uint32_t)dm_f2bf(y1) << 16);
-    }
-  }
-  if (slot == 0) {
-    for (int i = t0 * p.Hv + lane; i < t1 * p.Hv; i += 64) {
-      const int h = i % p.Hv;
-      const float sp = softplus_bf16(dm_rb(dm_bf2f(p.a_in[i]) + dm_bf2f(p.dt_bias[h])));
-      const float decay = dm_exp(dm_bf2f(p.a_log[h]));
-      p.g[i] = dm_exp(-decay * sp);
-      p.beta[i] = dm_f2bf(dm_sigmoid_bf16(dm_bf2f(p.b_in[i])));
+      *reinterpret_cast<uint32_t*>(dst) = dm_f2bf2(y0, y1);
     }
   }
 }
@@ -884,9 +889,13 @@ int ornith_gdn_front(ornith_ctx* ctx, const void* d_conv_state, const void* d_qk
   u = (u + 0x7fffu + ((u >> 16) & 1u)) & 0xffff0000u;
   memcpy(&p.k_scale, &u, 4);
   p.eps = eps;
-  if (p.K == 4 && T >= 2 * kFrontRun)
-    hipLaunchKernelGGL(gdn_front_run_kernel, dim3(p.D / 128, (T + kFrontRun - 1) / kFrontRun), dim3(64), 0,
-                       ctx->stream, p);
+  // 16 tokens a wavefront from 16 wavefronts a compute unit on (at 700 rows, two thirds of that,
+  // 4 are faster)
+  const bool wide = (long)(p.D / 128) * ((T + 15) / 16) >= 16L * ctx->compute_units;
+  if (p.K == 4 && T >= 32 && ((uintptr_t)d_cw & 15) == 0 && wide)
+    hipLaunchKernelGGL(gdn_front_run_kernel<16>, dim3(p.D / 128 + 1, (T + 15) / 16), dim3(64), 0, ctx->stream, p);
+  else if (p.K == 4 && T >= 32 && ((uintptr_t)d_cw & 15) == 0)
+    hipLaunchKernelGGL(gdn_front_run_kernel<4>, dim3(p.D / 128 + 1, (T + 3) / 4), dim3(64), 0, ctx->stream, p);
   else
     hipLaunchKernelGGL(gdn_front_kernel, dim3(p.D / 128, T), dim3(64), 0, ctx->stream, p);
   ORN_LAUNCH_CHECK("gdn_front_kernel");
