@@ -137,9 +137,13 @@ __global__ void embedding4_kernel(const uint8_t* w, const bf16_t* scales, const 
 // ---- dense bf16 at prefill widths: a small GEMM on the matrix cores -------------------
 // y[M, O] = x[M, K] . W[O, K]^T for the narrow dense projections (the gated-delta a / b heads,
 // the shared expert's gate: O of 1 .. 64): as mat-vecs every activation row is read by O / 4
-// workgroups. One workgroup = 16 rows; its four wavefronts split K and add up through LDS; a
+// workgroups. One workgroup = 16 rows; its wavefronts split K and add up through LDS; a
 // wavefront feeds v_mfma_f32_16x16x32_bf16 straight from global memory (A: 16 rows x 32
 // channels, B: 16 outputs x 32 channels, 16 bytes a lane each). grid.y covers O in 64s.
+// A launch is one latency chain of some workgroups, so K goes over as many wavefronts as it
+// divides into 128-channel pieces (up to 16) and a wavefront asks for a piece's operands at once:
+// 2 x 32 outputs of K = 2048, 51 / 700 / 6621 rows, with four wavefronts 24.4 / 24.5 / 25.5 us, with
+// sixteen 12.7 / 13.5 / 24.1.
 typedef __bf16 dmm_bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float dmm_f32x4_t __attribute__((ext_vector_type(4)));
 
@@ -150,11 +154,12 @@ struct DenseMmSegs {
   int n;
 };
 
-__global__ __launch_bounds__(256) void dense_mm_kernel(DenseMmSegs s, const bf16_t* x, int M, int K) {
-  __shared__ float red[3][4][64][4];
+template <int NW>
+__global__ __launch_bounds__(64 * NW) void dense_mm_kernel(DenseMmSegs s, const bf16_t* x, int M, int K) {
+  __shared__ __attribute__((aligned(16))) dmm_f32x4_t red[NW][4][64];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l16 = lane & 15, lg = lane >> 4;
   const int row0 = blockIdx.x * 16;
-  const int kw = K / 4, k0 = wave * kw;  // K is a multiple of 128
+  const int kw = K / NW, k0 = wave * kw;  // a multiple of 32
   const bf16_t* xp = x + (size_t)min(row0 + l16, M - 1) * K + k0 + 8 * lg;
   // the four 16-output tiles of this workgroup: tile 4 * blockIdx.y + nt of the segments' tiles
   // laid end to end (a segment's last tile may be ragged)
@@ -190,23 +195,28 @@ __global__ __launch_bounds__(256) void dense_mm_kernel(DenseMmSegs s, const bf16
         acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[nt], 0, 0, 0);
       }
   }
-  if (wave > 0) {
 #pragma unroll
-    for (int nt = 0; nt < 4; ++nt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) red[wave - 1][nt][lane][r] = acc[nt][r];
-  }
+  for (int nt = 0; nt < 4; ++nt) red[wave][nt][lane] = acc[nt];
   __syncthreads();
-  if (wave > 0) return;
-  // D[m = 4 * lg + r][n = l16]
+  if (wave >= 4) return;
+  // output tile nt = wave: D[m = 4 * lg + r][n = l16]
+  dmm_f32x4_t v = red[0][wave][lane];
 #pragma unroll
-  for (int nt = 0; nt < 4; ++nt) {
+  for (int w = 1; w < NW; ++w) v += red[w][wave][lane];
+  int col = 0, end = 0, stride = 0;
+  bf16_t* y = nullptr;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int row = row0 + 4 * lg + r;
-      const float v = ((acc[nt][r] + red[0][nt][lane][r]) + red[1][nt][lane][r]) + red[2][nt][lane][r];
-      if (ocol[nt] < oend[nt] && row < M) yp[nt][(size_t)row * ostride[nt] + ocol[nt]] = dm_f2bf(v);
+  for (int nt = 0; nt < 4; ++nt)
+    if (nt == wave) {
+      col = ocol[nt];
+      end = oend[nt];
+      stride = ostride[nt];
+      y = yp[nt];
     }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int row = row0 + 4 * lg + r;
+    if (col < end && row < M) y[(size_t)row * stride + col] = dm_f2bf(v[r]);
   }
 }
 
@@ -227,8 +237,14 @@ static bool launch_dense_mm(ornith_ctx* ctx, const ornith_linear* const* ws, int
     s.O[i] = ws[i]->O;
     tiles += (ws[i]->O + 15) / 16;
   }
-  hipLaunchKernelGGL(dense_mm_kernel, dim3((M + 15) / 16, (tiles + 3) / 4), dim3(256), 0, ctx->stream, s,
-                     (const bf16_t*)d_x, M, ws[0]->K);
+  const dim3 grid((M + 15) / 16, (tiles + 3) / 4);
+  const int K = ws[0]->K;
+  if (K % 2048 == 0)
+    hipLaunchKernelGGL(dense_mm_kernel<16>, grid, dim3(1024), 0, ctx->stream, s, (const bf16_t*)d_x, M, K);
+  else if (K % 1024 == 0)
+    hipLaunchKernelGGL(dense_mm_kernel<8>, grid, dim3(512), 0, ctx->stream, s, (const bf16_t*)d_x, M, K);
+  else
+    hipLaunchKernelGGL(dense_mm_kernel<4>, grid, dim3(256), 0, ctx->stream, s, (const bf16_t*)d_x, M, K);
   return true;
 }
 
