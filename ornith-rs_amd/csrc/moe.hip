@@ -143,20 +143,28 @@ __global__ void moe_combine_kernel(const bf16_t* scores, const bf16_t* y, const 
   float denom = 0.f;
   if (normalize)
     for (int j = 0; j < k; ++j) denom = dm_rb(dm_bf2f(s[j]) + denom);
+  // eight experts' rows are asked for at once (in a loop over the experts every row waited for the
+  // arithmetic of the one before); past k the last row again, unused
+  const P sh = *reinterpret_cast<const P*>(shared + (size_t)t * dim + c);
   float acc[V];
 #pragma unroll
   for (int e = 0; e < V; ++e) acc[e] = 0.f;
-  for (int j = 0; j < k; ++j) {
-    const float w = normalize ? dm_rb(dm_bf2f(s[j]) / denom) : dm_bf2f(s[j]);
-    const P yj = *reinterpret_cast<const P*>(y + ((size_t)t * k + j) * dim + c);
+  for (int j0 = 0; j0 < k; j0 += 8) {
+    P yj[8];
 #pragma unroll
-    for (int e = 0; e < V; ++e) {
-      const float weighted = dm_rb(bf_get<V>(yj, e) * w);
-      acc[e] = dm_rb(weighted + acc[e]);
+    for (int j = 0; j < 8; ++j) yj[j] = *reinterpret_cast<const P*>(y + ((size_t)t * k + min(j0 + j, k - 1)) * dim + c);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      if (j0 + j >= k) break;
+      const float w = normalize ? dm_rb(dm_bf2f(s[j0 + j]) / denom) : dm_bf2f(s[j0 + j]);
+#pragma unroll
+      for (int e = 0; e < V; ++e) {
+        const float weighted = dm_rb(bf_get<V>(yj[j], e) * w);
+        acc[e] = dm_rb(weighted + acc[e]);
+      }
     }
   }
   const float g = dm_sigmoid_bf16(dm_bf2f(gate[t]));
-  const P sh = *reinterpret_cast<const P*>(shared + (size_t)t * dim + c);
   P o;
 #pragma unroll
   for (int e = 0; e < V; ++e) {
