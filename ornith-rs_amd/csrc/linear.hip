@@ -13,12 +13,17 @@
 #include "dmath.h"
 #include "linear_device.h"
 #include "mm_narrow_host.h"
+#include "norm_device.h"
 #include "rt.h"
 
 // kquant.hip
 extern "C" int kq_qmv_multi_prenorm(ornith_ctx* ctx, const ornith_kmatrix* const* ws, int n,
                                     const void* d_res, const void* d_y, const void* d_wnorm, float eps,
                                     int M, void* d_h_out, void* d_normed_out, void* const* d_ys);
+
+// affine_mv.hip
+int affine_mv_multi(ornith_ctx* ctx, const ornith_linear* const* ws, int n, const void* d_x, int M, void* const* d_ys,
+                    const PreNorm* pre);
 
 namespace {
 
@@ -300,6 +305,7 @@ int ornith_linear_matmul(ornith_ctx* ctx, const ornith_linear* w, const void* d_
       ORN_REQUIRE(w->K % 64 == 0 && w->O >= 1 && M <= 65535, "linear_matmul: affine O=%d K=%d",
                   w->O, w->K);
       if (nmm::plain_ok(&w, 1, d_x, M, &d_y)) return nmm::plain(ctx, &w, 1, d_x, M, &d_y);
+      if (const int rc = affine_mv_multi(ctx, &w, 1, d_x, M, &d_y, nullptr); rc >= 0) return rc;
       hipLaunchKernelGGL(affine8_qmv_kernel, dim3(w->O, M), dim3(64), 0, ctx->stream,
                          (const uint8_t*)w->d_w, (const bf16_t*)w->d_scales,
                          (const bf16_t*)w->d_biases, (const bf16_t*)d_x, (bf16_t*)d_y, w->O, w->K);
@@ -309,6 +315,7 @@ int ornith_linear_matmul(ornith_ctx* ctx, const ornith_linear* w, const void* d_
       ORN_REQUIRE(w->d_w && w->d_scales && w->d_biases, "linear_matmul: affine tensor missing");
       ORN_REQUIRE(w->K % 32 == 0 && w->O >= 1 && M <= 65535, "linear_matmul: 4-bit affine O=%d K=%d", w->O, w->K);
       if (nmm::plain_ok(&w, 1, d_x, M, &d_y)) return nmm::plain(ctx, &w, 1, d_x, M, &d_y);
+      if (const int rc = affine_mv_multi(ctx, &w, 1, d_x, M, &d_y, nullptr); rc >= 0) return rc;
       hipLaunchKernelGGL(affine4_qmv_kernel<false>, dim3((w->O + 3) / 4, M), dim3(256), 0, ctx->stream,
                          (const uint8_t*)w->d_w, (const bf16_t*)w->d_scales, (const bf16_t*)w->d_biases,
                          (const bf16_t*)d_x, (bf16_t*)d_y, 1, w->O, w->K, M, (const uint32_t*)nullptr,
@@ -346,6 +353,9 @@ int ornith_linear_matmul_multi(ornith_ctx* ctx, const ornith_linear* const* ws, 
     fuse = fuse && ws[i]->mode == ws[0]->mode && ws[i]->K == ws[0]->K;
     if (ws[i]->mode == ORNITH_LIN_KQUANT) fuse = fuse && ws[i]->km.kind == ws[0]->km.kind;
   }
+  // affine matrices share a launch whatever their width in bits
+  if (ornith_option_fuse_proj() && n >= 2 && M < kPrefillRows)
+    if (const int rc = affine_mv_multi(ctx, ws, n, d_x, M, d_ys, nullptr); rc >= 0) return rc;
   if (fuse && ws[0]->mode == ORNITH_LIN_KQUANT) {
     const ornith_kmatrix* kms[4];
     for (int i = 0; i < n; ++i) kms[i] = &ws[i]->km;
@@ -429,6 +439,13 @@ int ornith_add_rms_linear_multi(ornith_ctx* ctx, const ornith_linear* const* ws,
   }
   if (fuse) {
     const int rc = kq_qmv_multi_prenorm(ctx, kms, n, d_res, d_y, d_wnorm, eps, M, d_h_out, d_normed_out, d_ys);
+    if (rc >= 0) return rc;
+  }
+  if (ornith_option_fuse_norm() && n <= 4 && M <= 4 && M < kPrefillRows) {
+    const PreNorm pre{(const bf16_t*)d_res, (const bf16_t*)d_y, (const bf16_t*)d_wnorm, (bf16_t*)d_h_out, (bf16_t*)d_normed_out, eps};
+    bool all = true;
+    for (int i = 0; i < n; ++i) all = all && ws[i];
+    const int rc = all ? affine_mv_multi(ctx, ws, n, nullptr, M, d_ys, &pre) : -1;
     if (rc >= 0) return rc;
   }
   int rc = ornith_add_rms_norm(ctx, d_res, d_y, d_wnorm, M, ws[0]->K, eps, d_h_out, d_normed_out);

@@ -405,12 +405,15 @@ static int moe_block_impl(ornith_ctx* ctx, const ornith_moe_weights* w, const vo
   const bool pre_in_kernel = pre && T <= 4 && H == kPreN && ornith_option_fuse_norm() &&
                              ornith_option_fuse_moe() && moe_fused_supported(w) &&
                              w->router.mode == ORNITH_LIN_KQUANT;
-  if (pre && !pre_in_kernel) {
+  // (an affine block's router and shared-expert gate take it in the head of their launch, below)
+  const bool ex_affine4 = !w->ex_dense && w->ex_gate.kind == ORNITH_AFFINE4_G32;
+  const bool pair_a4 = ex_affine4 && moe_affine4_supported(w);
+  const bool pre_in_a4 = pre && T <= 4 && T < kPrefillRows && ornith_option_fuse_moe() && pair_a4;
+  if (pre && !pre_in_kernel && !pre_in_a4) {
     int rcn = ornith_add_rms_norm(ctx, pre->res, pre->y, pre->w, T, H, pre->eps, pre->h_out, pre->normed_out);
     if (rcn) return rcn;
     pre = nullptr;
   }
-  const bool ex_affine4 = !w->ex_dense && w->ex_gate.kind == ORNITH_AFFINE4_G32;
   if (ex_affine4)
     ORN_REQUIRE(w->ex_up.kind == ORNITH_AFFINE4_G32 && w->ex_down.kind == ORNITH_AFFINE4_G32,
                 "moe_block: the three expert stacks must share the 4-bit affine format");
@@ -497,14 +500,17 @@ static int moe_block_impl(ornith_ctx* ctx, const ornith_moe_weights* w, const vo
                              ctx->stream));
     return ORNITH_OK;
   }
-  const bool pair_a4 = ex_affine4 && moe_affine4_supported(w), pair_dense = w->ex_dense && moe_dense_supported(w);
+  const bool pair_dense = w->ex_dense && moe_dense_supported(w);
   if (ornith_option_fuse_moe() && (pair_a4 || pair_dense)) {
     // the published artifact's block, and the MTP head's dense one, in three launches: router +
     // shared-expert gate (one launch when their formats match), then the two expert launches of
     // moe_affine4.hip, the softmax + top-k in the head of the first where the expert count allows
     const ornith_linear* in2[2] = {&w->router, &w->sh_egate};
     void* out2[2] = {gates, eg};
-    TRY(ornith_linear_matmul_multi(ctx, in2, 2, d_x, T, out2));
+    if (pre)  // (falls back to the separate norm where the launch does not cover the shapes)
+      TRY(ornith_add_rms_linear_multi(ctx, in2, 2, pre->res, pre->y, pre->w, pre->eps, T, pre->h_out, pre->normed_out, out2));
+    else
+      TRY(ornith_linear_matmul_multi(ctx, in2, 2, d_x, T, out2));
     const bool topk_in_up = E % 64 == 0 && E <= 1024 && ((E / 64) & (E / 64 - 1)) == 0 && k <= 16;
     if (!topk_in_up) TRY(launch_router(ctx, gates, T, E, k, inds, scores, nullptr, nullptr, nullptr));
     if (pair_a4)

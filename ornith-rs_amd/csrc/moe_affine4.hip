@@ -20,6 +20,7 @@
 // value, then the 64-lane butterfly; a dense one is dense_row_dot (linear_device.h), the
 // function the operator path's kernels call. So the two launches give the bits of the operator
 // path and of the oracle (oracle/orc_moe.c).
+#include "affine_device.h"
 #include "linear_device.h"
 #include "moe_device.h"
 #include "rt.h"
@@ -143,22 +144,26 @@ struct A4UpArgs {
   bf16_t* scores_out;    // [T*k]
 };
 
-// grid (ceil(I / 4), T*k + T), 256 threads: a wavefront an output row
-template <class F, bool ROUTE>
-__global__ __launch_bounds__(256) void moe_up_affine4_kernel(A4UpArgs<F> a) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int r = blockIdx.y, routed = a.T * a.k;
+// What row blockIdx.y of an up launch works on: its token, the first weight row of its expert and
+// the two matrices. With ROUTE softmax + top-k of the row's token are made here.
+template <class F>
+struct A4UpRow {
   int token;
   size_t row0;
   typename F::Mat wg, wu;
+};
+template <class F, bool ROUTE>
+__device__ __forceinline__ A4UpRow<F> a4_up_row(const A4UpArgs<F>& a, int lane, int wave) {
+  const int r = blockIdx.y, routed = a.T * a.k;
+  A4UpRow<F> u;
   if (r < routed) {
-    token = r / a.k;
+    u.token = r / a.k;
     uint32_t e;
     if constexpr (ROUTE) {
       __shared__ uint32_t s_inds[16];
       __shared__ bf16_t s_scores[16];
       if (wave == 0) {
-        const bf16_t* g = a.gates + (size_t)token * a.E;
+        const bf16_t* g = a.gates + (size_t)u.token * a.E;
         switch (a.E / 64) {
           case 1: router_topk_wave<1>(g, a.k, s_inds, s_scores, nullptr, lane); break;
           case 2: router_topk_wave<2>(g, a.k, s_inds, s_scores, nullptr, lane); break;
@@ -168,29 +173,72 @@ __global__ __launch_bounds__(256) void moe_up_affine4_kernel(A4UpArgs<F> a) {
         }
       }
       __syncthreads();
-      e = s_inds[r - token * a.k];
-      if (blockIdx.x == 0 && r == token * a.k && (int)threadIdx.x < a.k) {
+      e = s_inds[r - u.token * a.k];
+      if (blockIdx.x == 0 && r == u.token * a.k && (int)threadIdx.x < a.k) {
         a.inds_out[r + threadIdx.x] = s_inds[threadIdx.x];
         a.scores_out[r + threadIdx.x] = s_scores[threadIdx.x];
       }
     } else {
       e = a.inds[r];
     }
-    row0 = (size_t)min(e, (uint32_t)(a.E - 1)) * a.I;
-    wg = a.gate;
-    wu = a.up;
+    u.row0 = (size_t)min(e, (uint32_t)(a.E - 1)) * a.I;
+    u.wg = a.gate;
+    u.wu = a.up;
   } else {
-    token = r - routed;
-    row0 = 0;
-    wg = a.sgate;
-    wu = a.sup;
+    u.token = r - routed;
+    u.row0 = 0;
+    u.wg = a.sgate;
+    u.wu = a.sup;
   }
+  return u;
+}
+
+// grid (ceil(I / 4), T*k + T), 256 threads: a wavefront an output row
+template <class F, bool ROUTE>
+__global__ __launch_bounds__(256) void moe_up_affine4_kernel(A4UpArgs<F> a) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = blockIdx.y;
+  const A4UpRow<F> u = a4_up_row<F, ROUTE>(a, lane, wave);
   const int o = blockIdx.x * 4 + wave;
   if (o >= a.I) return;
-  const bf16_t* xr = a.x + (size_t)token * a.K;
-  float g, u;
-  F::dot2(wg, wu, row0 + o, a.K, xr, lane, g, u);
-  if (lane == 0) a.act[(size_t)r * a.I + o] = swiglu_bf16(g, u);
+  const bf16_t* xr = a.x + (size_t)u.token * a.K;
+  float gs, us;
+  F::dot2(u.wg, u.wu, u.row0 + o, a.K, xr, lane, gs, us);
+  if (lane == 0) a.act[(size_t)r * a.I + o] = swiglu_bf16(gs, us);
+}
+
+// The same for 4-bit rows of K = 1024 NC: two intermediate rows a wavefront, the codes and scales of
+// their gate and up rows asked for together and the four sums folded as one. What bounds it is the
+// chain gates -> top-k -> rows -> sums; the kernel above, which every other width takes, adds a trip
+// to memory for every 1024 columns of a row and unpacks with three instructions a code where this
+// one needs one and a half. us at T = 1 / 2, K = 2048, I = 512: 11.3 / 16.6 -> 7.3 / 10.2
+// grid (ceil(I / 8), T*k + T), 256 threads
+template <int NC, bool ROUTE>
+__global__ __launch_bounds__(256) void moe_up_a4_kernel(A4UpArgs<FmtA4> a) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = blockIdx.y;
+  const A4UpRow<FmtA4> u = a4_up_row<FmtA4, ROUTE>(a, lane, wave);
+  const int base = (blockIdx.x * 4 + wave) * 2;
+  AffRow<4, 64, NC> rg[2], ru[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const size_t row = u.row0 + min(base + i, a.I - 1);
+    rg[i].load(u.wg.w, u.wg.scales, u.wg.biases, row, lane);
+    ru[i].load(u.wu.w, u.wu.scales, u.wu.biases, row, lane);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  AffLane<4, 64, NC, 1> L;
+  const bf16_t* xr[1] = {a.x + (size_t)u.token * a.K};
+  L.load(xr, lane);
+  float g0[1] = {0.f}, u0[1] = {0.f}, g1[1] = {0.f}, u1[1] = {0.f};
+  rg[0].accumulate(L, g0);
+  ru[0].accumulate(L, u0);
+  rg[1].accumulate(L, g1);
+  ru[1].accumulate(L, u1);
+  // lanes [0,16): gate row 0, [32,48): up row 0, [16,32): gate row 1, [48,64): up row 1
+  const float red = dm_wave_sum4(g0[0], u0[0], g1[0], u1[0], lane);
+  float gs, us;
+  dm_row_swap<32>(red, gs, us);
+  const int o = base + ((lane >> 4) & 1);
+  if ((lane & 47) == 0 && o < a.I) a.act[(size_t)r * a.I + o] = swiglu_bf16(gs, us);
 }
 
 template <class F>
@@ -204,6 +252,29 @@ struct A4DownArgs {
   bf16_t* out;           // [T, H]
   int T, k, E, H, I, normalize;
 };
+
+// the router weights of a token, from its scores (one a lane): denom = ((0+s0)+s1)..., w_j = bf16(s_j / denom)
+__device__ __forceinline__ void a4_combine_weights(uint16_t score_bits, uint16_t egate_bits, int k, int normalize, int lane,
+                                                   float* wj, float* gsig) {
+  float denom = 0.f;
+  if (normalize) {
+#pragma unroll
+    for (int i = 0; i < kA4MaxK; ++i)
+      if (i < k) denom = dm_rb(dm_bf2f((bf16_t)__builtin_amdgcn_readlane((int)score_bits, i)) + denom);
+  }
+  if (lane < k) wj[lane] = normalize ? dm_rb(dm_bf2f(score_bits) / denom) : dm_bf2f(score_bits);
+  if (lane == 0) *gsig = dm_sigmoid_bf16(dm_bf2f(egate_bits));
+}
+// one output column of a token: y[i * ld] the experts' sums in slot order, the shared one last
+__device__ __forceinline__ bf16_t a4_combine(const float* y, int ld, const float* wj, float gsig, int k) {
+  float s = 0.f;
+  for (int i = 0; i < k; ++i) {
+    const float weighted = dm_rb(y[i * ld] * wj[i]);
+    s = dm_rb(weighted + s);
+  }
+  const float gated = dm_rb(gsig * y[k * ld]);
+  return dm_f2bf(s + gated);
+}
 
 constexpr int kA4Cols = 8;
 
@@ -227,31 +298,59 @@ __global__ __launch_bounds__(64 * (kA4MaxK + 1)) void moe_down_affine4_kernel(A4
   const bf16_t* xr = a.act + (size_t)arow * a.I;
   float v[kA4Cols];
   F::template dotn<kA4Cols>(w, row0, c0, a.H, a.I, xr, lane, v);
-  if (j == 0) {
-    // the router weights of this token: denom = ((0+s0)+s1)..., w_j = bf16(s_j / denom)
-    float denom = 0.f;
-    if (a.normalize) {
-#pragma unroll
-      for (int i = 0; i < kA4MaxK; ++i)
-        if (i < k) denom = dm_rb(dm_bf2f((bf16_t)__builtin_amdgcn_readlane((int)score_bits, i)) + denom);
-    }
-    if (lane < k) wj[lane] = a.normalize ? dm_rb(dm_bf2f(score_bits) / denom) : dm_bf2f(score_bits);
-    if (lane == 0) gsig = dm_sigmoid_bf16(dm_bf2f(egate_bits));
-  }
+  if (j == 0) a4_combine_weights(score_bits, egate_bits, k, a.normalize, lane, wj, &gsig);
 #pragma unroll
   for (int c = 0; c < kA4Cols; ++c)
     if (lane == 0) yl[j][c] = dm_rb(v[c]);  // expert outputs are bf16 in the operator path
   __syncthreads();
   const int col = threadIdx.x;
-  if (col < kA4Cols && c0 + col < a.H) {
-    float s = 0.f;
-    for (int i = 0; i < k; ++i) {
-      const float weighted = dm_rb(yl[i][col] * wj[i]);
-      s = dm_rb(weighted + s);
-    }
-    const float gated = dm_rb(gsig * yl[k][col]);
-    a.out[(size_t)t * a.H + c0 + col] = dm_f2bf(s + gated);
+  if (col < kA4Cols && c0 + col < a.H) a.out[(size_t)t * a.H + c0 + col] = a4_combine(&yl[0][col], kA4Cols, wj, gsig, k);
+}
+
+// The same for 4-bit rows of I = 16 LPR columns: 64 / LPR output columns a wavefront pass (32 lanes
+// are a row of 512: the kernel above left the other half of its wavefronts idle and asked for a row
+// after it had worked off the one before), ITERS passes asked for at once. At 32 columns a workgroup
+// the shared expert's passes go over four wavefronts, so that the four SIMDs carry the same number.
+// us at T = 1 / 2, I = 512, H = 2048: 14.0 / 25.5 -> 4.3 / 5.8
+// grid (ceil(H / COLS), T), 64 * (k + 1) threads, 64 * (k + 4) at 32 columns
+constexpr int a4_shared_waves(int cols) { return cols >= 32 ? 4 : 1; }
+template <int LPR, int ITERS>
+__global__ __launch_bounds__(64 * (kA4MaxK + a4_shared_waves(64 / LPR * ITERS))) void moe_down_a4_kernel(A4DownArgs<FmtA4> a) {
+  constexpr int RPW = 64 / LPR, COLS = RPW * ITERS, SW = a4_shared_waves(COLS), SHARE = ITERS / SW;
+  const int lane = threadIdx.x & 63, j = threadIdx.x >> 6;  // j < k: expert slot, else the shared expert
+  const int slot = lane / LPR, c = lane % LPR;
+  const int t = blockIdx.y, k = a.k, c0 = blockIdx.x * COLS;
+  __shared__ float yl[kA4MaxK + 1][COLS];
+  __shared__ float wj[kA4MaxK];
+  __shared__ float gsig;
+  const bool shared = j >= k;
+  const int it0 = shared ? (j - k) * SHARE : 0, its = shared ? SHARE : ITERS;
+  const FmtA4::Mat w = shared ? a.sdown : a.down;
+  const size_t row0 = shared ? 0 : (size_t)min(a.inds[t * k + j], (uint32_t)(a.E - 1)) * a.H;
+  // what is small and cached first: loads return in issue order
+  AffLane<4, LPR, 1, 1> L;
+  const bf16_t* xr[1] = {a.act + (size_t)(shared ? a.T * k + t : t * k + j) * a.I};
+  L.load(xr, c);
+  const uint16_t score_bits = a.scores[(size_t)t * k + (lane < k ? lane : 0)];
+  const uint16_t egate_bits = a.egate[t];
+  __builtin_amdgcn_sched_barrier(0);
+  AffRow<4, LPR, 1> rr[ITERS];
+#pragma unroll
+  for (int i = 0; i < ITERS; ++i)
+    if (SW == 1 || i < its) rr[i].load(w.w, w.scales, w.biases, row0 + min(c0 + (it0 + i) * RPW + slot, a.H - 1), c);
+  __builtin_amdgcn_sched_barrier(0);
+  if (j == 0) a4_combine_weights(score_bits, egate_bits, k, a.normalize, lane, wj, &gsig);
+#pragma unroll
+  for (int i = 0; i < ITERS; ++i) {
+    if (SW > 1 && i >= its) continue;
+    float acc[1] = {0.f};
+    rr[i].accumulate(L, acc);
+    const float v = dm_wave_sum<LPR>(acc[0]);
+    if (c == 0) yl[shared ? k : j][(it0 + i) * RPW + slot] = dm_rb(v);  // expert outputs are bf16 in the operator path
   }
+  __syncthreads();
+  const int col = threadIdx.x;
+  if (col < COLS && c0 + col < a.H) a.out[(size_t)t * a.H + c0 + col] = a4_combine(&yl[0][col], COLS, wj, gsig, k);
 }
 
 A4Mat mat_of(const ornith_kmatrix& m) {
@@ -280,6 +379,49 @@ bool moe_affine4_supported(const ornith_moe_weights* w) {
 
 namespace {
 
+// the 4-bit kernels of fixed width; false: another format or width
+template <class F>
+bool launch_up_a4(ornith_ctx*, const A4UpArgs<F>&, bool) { return false; }
+bool launch_up_a4(ornith_ctx* ctx, const A4UpArgs<FmtA4>& u, bool route) {
+  const dim3 grid((u.I + 7) / 8, u.T * u.k + u.T);
+  const int nc = u.K % 1024 == 0 ? u.K / 1024 : 0;
+#define UP_NC(NC)                                                                                       \
+  if (route)                                                                                            \
+    hipLaunchKernelGGL((moe_up_a4_kernel<NC, true>), grid, dim3(256), 0, ctx->stream, u);               \
+  else                                                                                                  \
+    hipLaunchKernelGGL((moe_up_a4_kernel<NC, false>), grid, dim3(256), 0, ctx->stream, u);              \
+  return true;
+  switch (nc) {
+    case 1: UP_NC(1)
+    case 2: UP_NC(2)
+    case 4: UP_NC(4)
+    default: return false;
+  }
+#undef UP_NC
+}
+template <class F>
+bool launch_down_a4(ornith_ctx*, const A4DownArgs<F>&) { return false; }
+bool launch_down_a4(ornith_ctx* ctx, const A4DownArgs<FmtA4>& d) {
+  // columns a workgroup: 8 while that is no more than two workgroups a compute unit, then 16, then 32
+  const int g8 = (d.H + 7) / 8 * d.T, cu = ctx->compute_units;
+  const int cols = g8 >= 3 * cu ? 32 : g8 >= 2 * cu ? 16 : 8;
+  const dim3 grid((d.H + cols - 1) / cols, d.T), block(64 * (d.k + a4_shared_waves(cols)));
+#define DOWN_LPR(LPR)                                                                                              \
+  if (cols == 8)                                                                                                   \
+    hipLaunchKernelGGL((moe_down_a4_kernel<LPR, 8 * LPR / 64>), grid, block, 0, ctx->stream, d);                   \
+  else if (cols == 16)                                                                                             \
+    hipLaunchKernelGGL((moe_down_a4_kernel<LPR, 16 * LPR / 64>), grid, block, 0, ctx->stream, d);                  \
+  else                                                                                                             \
+    hipLaunchKernelGGL((moe_down_a4_kernel<LPR, 32 * LPR / 64>), grid, block, 0, ctx->stream, d);                  \
+  return true;
+  switch (d.I) {
+    case 256: DOWN_LPR(16)
+    case 512: DOWN_LPR(32)
+    default: return false;
+  }
+#undef DOWN_LPR
+}
+
 template <class F>
 int launch_pair(ornith_ctx* ctx, const ornith_moe_weights* w, const typename F::Mat (&m)[6], const void* d_x, int T,
                 const uint32_t* d_inds, const void* d_scores, const void* d_egate, void* d_act, void* d_out,
@@ -302,7 +444,8 @@ int launch_pair(ornith_ctx* ctx, const ornith_moe_weights* w, const typename F::
   u.inds_out = const_cast<uint32_t*>(d_inds);
   u.scores_out = (bf16_t*)const_cast<void*>(d_scores);
   const dim3 ugrid((I + 3) / 4, T * k + T);
-  if (d_gates)
+  if (launch_up_a4(ctx, u, d_gates != nullptr)) {
+  } else if (d_gates)
     hipLaunchKernelGGL((moe_up_affine4_kernel<F, true>), ugrid, dim3(256), 0, ctx->stream, u);
   else
     hipLaunchKernelGGL((moe_up_affine4_kernel<F, false>), ugrid, dim3(256), 0, ctx->stream, u);
@@ -321,7 +464,7 @@ int launch_pair(ornith_ctx* ctx, const ornith_moe_weights* w, const typename F::
   d.H = H;
   d.I = I;
   d.normalize = w->norm_topk_prob;
-  hipLaunchKernelGGL(moe_down_affine4_kernel<F>, dim3((H + kA4Cols - 1) / kA4Cols, T), dim3(64 * (k + 1)), 0,
+  if (!launch_down_a4(ctx, d)) hipLaunchKernelGGL(moe_down_affine4_kernel<F>, dim3((H + kA4Cols - 1) / kA4Cols, T), dim3(64 * (k + 1)), 0,
                      ctx->stream, d);
   ORN_LAUNCH_CHECK("moe_down_affine4_kernel");
   return ORNITH_OK;
