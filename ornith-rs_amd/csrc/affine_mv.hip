@@ -80,7 +80,7 @@ __device__ __forceinline__ void aff_rows(const AffSeg& sg, int block, int iters,
       // all loads in flight)
       if constexpr (!ONE) fetch(min(it + PF, iters - 1), pf[i]);
       __builtin_amdgcn_sched_barrier(0);
-      const float r = dm_wave_sum4(v[0], v[1], v[2], v[3], lane);
+      const float r = dm_wave_sum4(v[0], v[1], v[2], v[3]);
       // lane 0 holds sum 0, lane 16 sum 2, lane 32 sum 1, lane 48 sum 3
       const int k = ((lane >> 5) & 1) | ((lane >> 3) & 2), g = k / M, t = m0 + k - g * M, o = base + it * G + g;
       if ((lane & 15) == 0 && g < G && t < Mt && o < sg.O) sg.y[(size_t)t * sg.O + o] = dm_f2bf(r);

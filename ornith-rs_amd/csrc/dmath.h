@@ -227,21 +227,78 @@ __device__ __forceinline__ float dm_wave_max(float v) {
   return v;
 }
 
-// Four 64-lane butterfly sums for the price of one and a bit: at the 32 and 16 steps
-// each lane sends the value its partner is going to keep, so two sums share a permute.
-// Every addition pairs the same two operands as the plain butterfly, so the bits are
-// those of dm_wave_sum<64>. On return lanes [0,16) hold sum(a), [16,32) sum(c),
-// [32,48) sum(b), [48,64) sum(d).
-__device__ __forceinline__ float dm_wave_sum4(float a, float b, float c, float d, int lane) {
-  const bool h32 = lane & 32, h16 = lane & 16;
-  const float r1 = (h32 ? b : a) + dm_xor_lane<32>(h32 ? a : b);
-  const float r2 = (h32 ? d : c) + dm_xor_lane<32>(h32 ? c : d);
-  float r = (h16 ? r2 : r1) + dm_xor_lane<16>(h16 ? r1 : r2);
-  r = r + dm_xor_lane<8>(r);
-  r = r + dm_xor_lane<4>(r);
-  r = r + dm_xor_lane<2>(r);
-  r = r + dm_xor_lane<1>(r);
-  return r;
+// Several butterfly sums for the price of one and a bit. A swap of rows between TWO values leaves in
+// their sum the first one's pair in the even rows and the second one's in the odd rows, so the 32 and
+// 16 steps (and, with a select, the 8 step) halve the number of values instead of repeating them.
+// Every addition pairs the same two operands as the plain butterfly, so the bits are those of
+// dm_wave_sum.
+template <int ROWS>
+__device__ __forceinline__ float dm_fold_rows(float a, float b) {
+  if constexpr (ROWS == 32)
+    asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
+  else
+    asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
+  return a + b;
+}
+// two pairs, the waits shared
+template <int ROWS>
+__device__ __forceinline__ void dm_fold_rows2(float a, float b, float c, float d, float& ab, float& cd) {
+  if constexpr (ROWS == 32)
+    asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\tv_permlane32_swap_b32 %2, %3\n\ts_nop 1" : "+v"(a), "+v"(b), "+v"(c), "+v"(d));
+  else
+    asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\tv_permlane16_swap_b32 %2, %3\n\ts_nop 1" : "+v"(a), "+v"(b), "+v"(c), "+v"(d));
+  ab = a + b;
+  cd = c + d;
+}
+// the steps 8 .. 1 of a butterfly: lane l ends with the sum over its row of 16
+__device__ __forceinline__ float dm_row_sum(float v) {
+  v = v + dm_xor_lane<8>(v);
+  v = v + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x124, 0xF, 0xF, false));
+  v = v + dm_xor_lane<2>(v);
+  return v + dm_xor_lane<1>(v);
+}
+// Four 64-lane sums: on return lanes [0,16) hold sum(a), [16,32) sum(c), [32,48) sum(b), [48,64) sum(d).
+__device__ __forceinline__ float dm_wave_sum4(float a, float b, float c, float d) {
+  float ab, cd;
+  dm_fold_rows2<32>(a, b, c, d, ab, cd);
+  return dm_row_sum(dm_fold_rows<16>(ab, cd));
+}
+// M sums over groups of W lanes, one of them in each of the lanes for which dm_multi_leads holds:
+// lane c of the group has sum dm_multi_of(c) of them (>= M: none).
+template <int W, int M>
+__device__ __forceinline__ float dm_multi_sum(const float (&v)[M]) {
+  if constexpr (M == 1 || W < 32) {
+    static_assert(M == 1, "groups of 32 or 64 lanes");
+    return dm_wave_sum<W>(v[0]);
+  } else if constexpr (W == 64) {
+    if constexpr (M == 2) {
+      float a, b, r = dm_fold_rows<32>(v[0], v[1]);
+      dm_row_swap<16>(r, a, b);
+      return dm_row_sum(a + b);
+    } else {
+      return dm_wave_sum4(v[0], v[1], v[2], M > 3 ? v[M - 1] : 0.f);
+    }
+  } else {
+    if constexpr (M == 2) {
+      return dm_row_sum(dm_fold_rows<16>(v[0], v[1]));
+    } else {
+      float ab, cd;
+      dm_fold_rows2<16>(v[0], v[1], v[2], M > 3 ? v[M - 1] : 0.f, ab, cd);
+      const bool h8 = __lane_id() & 8;
+      float r = (h8 ? cd : ab) + dm_xor_lane<8>(h8 ? ab : cd);
+      r = r + dm_xor_lane<4>(r);
+      r = r + dm_xor_lane<2>(r);
+      return r + dm_xor_lane<1>(r);
+    }
+  }
+}
+template <int W, int M>
+__device__ __forceinline__ bool dm_multi_leads(int c) {
+  return (c & ((M == 1 ? W : M == 2 ? W / 2 : W / 4) - 1)) == 0;
+}
+template <int W, int M>
+__device__ __forceinline__ int dm_multi_of(int c) {
+  return M == 1 ? 0 : M == 2 ? c / (W / 2) : (c / (W / 2)) | (c / (W / 4) & 1) << 1;
 }
 __device__ __forceinline__ float dm_lane_value(float v, int lane) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane));

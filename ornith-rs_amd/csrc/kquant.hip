@@ -47,7 +47,7 @@ struct KqArgs {
   const uint32_t* lhs;  // gather only
   const uint32_t* rhs;  // gather only
   int K;
-  int E, x_rows;  // gather only: bounds for rhs / lhs (out-of-range ids are clamped)
+  int E, x_rows;  // gather: bounds for rhs / lhs (out-of-range ids are clamped); x_rows: activation rows
   int iters;      // row iterations per wavefront
   int y_bf16;     // 1: round outputs to bf16, 0: fp32
   PreNorm pre;    // PRE kernels: the activations are rms_norm(res + y) computed by every workgroup
@@ -67,7 +67,9 @@ extern "C" __attribute__((visibility("default"))) int ornith_debug_marks(long lo
 // One kernel for plain and gathered mat-vecs.
 //   KIND  format; LPR lanes per row (4,8,16,32,64); KS wavefronts per row (1,2)
 //   M     activation rows sharing each weight read (1..4); gather uses M == 1
-//   grid.x covers output rows (of all segments), grid.y is the gather row
+//   grid.x covers output rows (of all segments); grid.y is the gather row, else the group of M
+//   activation rows (a call of more than four goes in equal groups: one launch, and the groups find
+//   each other's weight rows in L2, where a launch a group read them again from memory)
 //   PRE   the activation rows are not read but made: every workgroup computes
 //         h = res + y, x = rms_norm(h) of the M rows (K == 2048) into LDS while its weight
 //         loads are in flight; workgroup 0 also stores h and x for later consumers
@@ -148,7 +150,9 @@ __global__ __launch_bounds__(256) void kq_qmv_kernel(KqArgs a) {
     yrow0 = (int64_t)r * O;
   } else {
 #pragma unroll
-    for (int t = 0; t < M; ++t) xrow[t] = static_cast<const char*>(a.x) + (size_t)t * a.K * xsz;
+    for (int t = 0; t < M; ++t)
+      xrow[t] = static_cast<const char*>(a.x) + (size_t)min((int)blockIdx.y * M + t, a.x_rows - 1) * a.K * xsz;
+    yrow0 = (int64_t)blockIdx.y * M * O;
   }
 
   // Rows kept in flight per wavefront. Cold weights come from HBM with a latency many
@@ -156,10 +160,13 @@ __global__ __launch_bounds__(256) void kq_qmv_kernel(KqArgs a) {
   // rows at once (they depend on nothing), behind only the few cached operands named
   // below, and refills a slot as soon as that row's registers are consumed.
   constexpr int PF = (KIND == ORNITH_Q4K) ? (M <= 2 ? 4 : 2) : (M <= 2 ? 2 : 1);
+  // rows whose sums are folded together: those that make four (dm_multi_sum); one for Q6_K, whose
+  // kernels would lose a wavefront a SIMD to the registers of a second row in work
+  constexpr int FR = LPR < 32 || KIND == ORNITH_Q6K ? 1 : PF < 4 / M ? PF : M > 2 ? 1 : 4 / M;
   typename KL::Lane L;
   L.set_chunk(c + 64 * ks);
 
-  __shared__ float part[(KS == 2) ? 2 * M * 64 : 1];
+  __shared__ float part[(KS == 2) ? 2 * FR * M * 64 : 1];
 
   const int rows_per_wave = RPW * a.iters;
   const int base = (((int)blockIdx.x - sg.first_block) * WPB + rw) * rows_per_wave;
@@ -198,44 +205,60 @@ __global__ __launch_bounds__(256) void kq_qmv_kernel(KqArgs a) {
 
   for (int it0 = 0; it0 < a.iters; it0 += PF) {
 #pragma unroll
-   for (int i = 0; i < PF; ++i) {
-    const int it = it0 + i;
-    if (it >= a.iters) break;
-    const int o = base + it * RPW + slot;
-    const bool valid = o < O;
-    float acc[M];
+    for (int i = 0; i < PF; i += FR) {
+      const int it = it0 + i;
+      if (it >= a.iters) break;
+      float acc[FR * M];  // row it + u, activation t at u * M + t
 #pragma unroll
-    for (int t = 0; t < M; ++t) acc[t] = 0.f;
-    const typename KL::Row r = pf[i];
-    if (it + PF < a.iters) pf[i] = KL::load(sg.qs, sg.scales, sg.dm, row_of(it + PF), nb, L);
-    KL::accumulate(r, L, acc);
-    if (it == 0) ORN_MARK(4);
-    if constexpr (KS == 2) {
-      // lane partial = (chunk l) + (chunk l + 64), in that order
-      float* mine = part + rw * M * 64;
-      __syncthreads();
-      if (ks == 1) {
+      for (int u = 0; u < FR; ++u) {
+        float one[M];
 #pragma unroll
-        for (int t = 0; t < M; ++t) mine[t * 64 + lane] = acc[t];
+        for (int t = 0; t < M; ++t) one[t] = 0.f;
+        if (u == 0 || it + u < a.iters) {
+          const typename KL::Row r = pf[i + u];
+          if (it + u + PF < a.iters) pf[i + u] = KL::load(sg.qs, sg.scales, sg.dm, row_of(it + u + PF), nb, L);
+          KL::accumulate(r, L, one);
+        }
+#pragma unroll
+        for (int t = 0; t < M; ++t) acc[u * M + t] = one[t];
       }
-      __syncthreads();
-      if (ks == 0) {
+      if (it == 0) ORN_MARK(4);
+      if constexpr (KS == 2) {
+        // lane partial = (chunk l) + (chunk l + 64), in that order
+        float* mine = part + rw * FR * M * 64;
+        __syncthreads();
+        if (ks == 1) {
 #pragma unroll
-        for (int t = 0; t < M; ++t) acc[t] = acc[t] + mine[t * 64 + lane];
+          for (int t = 0; t < FR * M; ++t) mine[t * 64 + lane] = acc[t];
+        }
+        __syncthreads();
+        if (ks == 0) {
+#pragma unroll
+          for (int t = 0; t < FR * M; ++t) acc[t] = acc[t] + mine[t * 64 + lane];
+        }
       }
-    }
-#pragma unroll
-    for (int t = 0; t < M; ++t) {
-      const float v = dm_wave_sum<LPR>(acc[t]);
-      if (c == 0 && ks == 0 && valid) {
-        const int64_t yi = (GATHER ? yrow0 : (int64_t)t * O) + o;
+      auto put = [&](int n, float v) {
+        const int u = n / M, t = n - u * M, o = base + (it + u) * RPW + slot;
+        if (o >= O || it + u >= a.iters || (!GATHER && !PRE && (int)blockIdx.y * M + t >= a.x_rows)) return;
+        const int64_t yi = yrow0 + (GATHER ? 0 : (int64_t)t * O) + o;
         if (a.y_bf16)
           static_cast<bf16_t*>(sg.y)[yi] = dm_f2bf(v);
         else
           static_cast<float*>(sg.y)[yi] = v;
+      };
+      if constexpr (LPR >= 32) {
+        // the sums fold together, each into the lane that stores it
+        const float v = dm_multi_sum<LPR, FR * M>(acc);
+        const int n = dm_multi_of<LPR, FR * M>(c);
+        if (dm_multi_leads<LPR, FR * M>(c) && n < FR * M && ks == 0) put(n, v);
+      } else {
+#pragma unroll
+        for (int n = 0; n < FR * M; ++n) {
+          const float v = dm_wave_sum<LPR>(acc[n]);
+          if (c == 0 && ks == 0) put(n, v);
+        }
       }
     }
-   }
   }
   ORN_MARK(5);
 }
@@ -331,24 +354,28 @@ int resident_workgroups(Kernel kernel) {
 // costs the same second round: 8192 + 4096 Q4_K rows of four activation rows take 19.0 us as
 // 342 + 171 workgroups where 512 fit, 15.8 us as 384), while rows beyond that only lengthen the
 // one round; and beyond three workgroups a compute unit the activations' conversion (and a norm
-// made in the head) is repeated for nothing.
-template <int LPR, int KS>
+// made in the head) is repeated for nothing. A grid that does not fit with 8 rows a wavefront goes on
+// to 32 where several activation rows make the arithmetic the larger part (248320 rows of four
+// activation rows 181 -> 165 us, 12288 rows of two groups of four 20.5 -> 18.3), but not for one,
+// which is a stream of weights that more workgroups keep fuller (60 us against 67).
+template <int LPR, int KS, int M>
 int auto_iters(const ornith_ctx* ctx, const KqArgs& a, int grid_y, int resident, int most = 3) {
+  constexpr int cap = M > 1 ? 32 : 8;
   constexpr int rows_per_pass = (64 / LPR) * (4 / KS);
   const long room = (long)ctx->compute_units * (resident < most ? resident : most);
-  for (int iters = 1; iters < 8; ++iters) {
+  for (int iters = 1; iters < cap; ++iters) {
     long blocks = 0;
     for (int s = 0; s < a.nseg; ++s) blocks += (a.seg[s].O + rows_per_pass * iters - 1) / (rows_per_pass * iters);
     if (blocks * grid_y <= room) return iters;
   }
-  return 8;
+  return cap;
 }
 
 template <int KIND, int LPR, int KS, int M, bool XF32, bool GATHER>
 int launch_one(ornith_ctx* ctx, KqArgs& a, int grid_y) {
   static const int resident = resident_workgroups(kq_qmv_kernel<KIND, LPR, KS, M, XF32, GATHER>);
   const int asked = a.iters;
-  if (!asked) a.iters = auto_iters<LPR, KS>(ctx, a, grid_y, resident);
+  if (!asked) a.iters = auto_iters<LPR, KS, M>(ctx, a, grid_y, resident);
   dim3 grid(layout_segments<LPR, KS>(a), grid_y, 1);
   hipLaunchKernelGGL((kq_qmv_kernel<KIND, LPR, KS, M, XF32, GATHER>), grid, dim3(256), 0,
                      ctx->stream, a);
@@ -380,7 +407,7 @@ int launch_pre(ornith_ctx* ctx, KqArgs& a) {
   static const int resident = resident_workgroups(kq_qmv_kernel<KIND, LPR, 1, M, false, false, true>);
   // (with the norm in its head a Q6_K launch, whose lanes take 64 weights a pass, measures best
   // at no more than two workgroups a compute unit: 9216 rows of one activation row 8.0 -> 7.4 us)
-  if (!a.iters) a.iters = auto_iters<LPR, 1>(ctx, a, 1, resident, KIND == ORNITH_Q6K ? 2 : 3);
+  if (!a.iters) a.iters = auto_iters<LPR, 1, M>(ctx, a, 1, resident, KIND == ORNITH_Q6K ? 2 : 3);
   dim3 grid(layout_segments<LPR, 1>(a), 1, 1);
   hipLaunchKernelGGL((kq_qmv_kernel<KIND, LPR, 1, M, false, false, true>), grid, dim3(256), 0, ctx->stream, a);
   ORN_LAUNCH_CHECK("kq_qmv_kernel<pre-norm>");
@@ -396,13 +423,18 @@ int launch_pre_m(ornith_ctx* ctx, KqArgs& a, int M) {
   }
 }
 
+// M activation rows in equal groups of up to four; more than four Q6_K rows in groups of two, whose
+// kernel keeps twice the wavefronts on a compute unit (9216 x 2048, us: 6 rows 23.7 in threes, 14.6 in
+// twos, 13 rows 41.8 in fours, 25.6 in twos)
 template <int KIND, bool XF32>
 int launch_m(ornith_ctx* ctx, KqArgs& a, int M) {
-  switch (M) {
-    case 1: return launch_shape<KIND, 1, XF32, false>(ctx, a, 1);
-    case 2: return launch_shape<KIND, 2, XF32, false>(ctx, a, 1);
-    case 3: return launch_shape<KIND, 3, XF32, false>(ctx, a, 1);
-    default: return launch_shape<KIND, 4, XF32, false>(ctx, a, 1);
+  const int most = KIND == ORNITH_Q6K && M > 4 ? 2 : 4, groups = (M + most - 1) / most;
+  a.x_rows = M;
+  switch ((M + groups - 1) / groups) {
+    case 1: return launch_shape<KIND, 1, XF32, false>(ctx, a, groups);
+    case 2: return launch_shape<KIND, 2, XF32, false>(ctx, a, groups);
+    case 3: return launch_shape<KIND, 3, XF32, false>(ctx, a, groups);
+    default: return launch_shape<KIND, 4, XF32, false>(ctx, a, groups);
   }
 }
 
@@ -509,7 +541,7 @@ int ornith_kq_qmv_multi(ornith_ctx* ctx, const ornith_kmatrix* const* ws, int n,
                         int x_dtype, int M, void* const* d_ys, int y_dtype) {
   ORN_REQUIRE(ctx && ws && d_x && d_ys, "kq_qmv: null argument");
   ORN_REQUIRE(n >= 1 && n <= kMaxSeg, "kq_qmv: %d matrices in one launch (1..%d)", n, kMaxSeg);
-  ORN_REQUIRE(M >= 1, "kq_qmv: M=%d", M);
+  ORN_REQUIRE(M >= 1 && M <= 4 * 65535, "kq_qmv: M=%d", M);
   ORN_REQUIRE(((uintptr_t)d_x & 15) == 0, "kq_qmv: x must be 16-byte aligned");
   for (int s = 0; s < n; ++s) {
     int rc = check_matrix(ws[s], "kq_qmv");
@@ -520,32 +552,22 @@ int ornith_kq_qmv_multi(ornith_ctx* ctx, const ornith_kmatrix* const* ws, int n,
     ORN_REQUIRE(d_ys[s], "kq_qmv: null output");
   }
   const int kind = ws[0]->kind, K = ws[0]->K;
-  const size_t xs = ornith_dtype_size(x_dtype), ys = ornith_dtype_size(y_dtype);
   KqArgs a{};
   a.nseg = n;
   a.K = K;
   a.y_bf16 = y_dtype == ORNITH_BF16;
   a.iters = pick_iters();
-  for (int m0 = 0; m0 < M; m0 += 4) {
-    const int mw = M - m0 < 4 ? M - m0 : 4;
-    a.x = (const char*)d_x + (size_t)m0 * K * xs;
-    for (int s = 0; s < n; ++s) {
-      a.seg[s].qs = (const uint8_t*)ws[s]->d_qs;
-      a.seg[s].scales = (const uint8_t*)ws[s]->d_scales;
-      a.seg[s].dm = (const uint16_t*)ws[s]->d_dm;
-      a.seg[s].O = ws[s]->O;
-      a.seg[s].y = (char*)d_ys[s] + (size_t)m0 * ws[s]->O * ys;
-    }
-    int rc;
-    if (kind == ORNITH_Q4K)
-      rc = x_dtype == ORNITH_F32 ? launch_m<ORNITH_Q4K, true>(ctx, a, mw)
-                                 : launch_m<ORNITH_Q4K, false>(ctx, a, mw);
-    else
-      rc = x_dtype == ORNITH_F32 ? launch_m<ORNITH_Q6K, true>(ctx, a, mw)
-                                 : launch_m<ORNITH_Q6K, false>(ctx, a, mw);
-    if (rc) return rc;
+  a.x = d_x;
+  for (int s = 0; s < n; ++s) {
+    a.seg[s].qs = (const uint8_t*)ws[s]->d_qs;
+    a.seg[s].scales = (const uint8_t*)ws[s]->d_scales;
+    a.seg[s].dm = (const uint16_t*)ws[s]->d_dm;
+    a.seg[s].O = ws[s]->O;
+    a.seg[s].y = d_ys[s];
   }
-  return ORNITH_OK;
+  if (kind == ORNITH_Q4K)
+    return x_dtype == ORNITH_F32 ? launch_m<ORNITH_Q4K, true>(ctx, a, M) : launch_m<ORNITH_Q4K, false>(ctx, a, M);
+  return x_dtype == ORNITH_F32 ? launch_m<ORNITH_Q6K, true>(ctx, a, M) : launch_m<ORNITH_Q6K, false>(ctx, a, M);
 }
 
 int ornith_kq_qmv(ornith_ctx* ctx, const ornith_kmatrix* w, const void* d_x, int x_dtype, int M,

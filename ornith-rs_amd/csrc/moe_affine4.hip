@@ -234,7 +234,7 @@ __global__ __launch_bounds__(256) void moe_up_a4_kernel(A4UpArgs<FmtA4> a) {
   rg[1].accumulate(L, g1);
   ru[1].accumulate(L, u1);
   // lanes [0,16): gate row 0, [32,48): up row 0, [16,32): gate row 1, [48,64): up row 1
-  const float red = dm_wave_sum4(g0[0], u0[0], g1[0], u1[0], lane);
+  const float red = dm_wave_sum4(g0[0], u0[0], g1[0], u1[0]);
   float gs, us;
   dm_row_swap<32>(red, gs, us);
   const int o = base + ((lane >> 4) & 1);

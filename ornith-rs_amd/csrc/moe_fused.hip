@@ -175,7 +175,7 @@ __global__ __launch_bounds__(256) void moe_up_kernel(const bf16_t* h_gates, cons
       ORN_KL_ACC(ru[it], L, u0);
       ORN_KL_ACC(rg[it + 1], L, g1);
       ORN_KL_ACC(ru[it + 1], L, u1);
-      const float red = dm_wave_sum4(g0[0], u0[0], g1[0], u1[0], lane);
+      const float red = dm_wave_sum4(g0[0], u0[0], g1[0], u1[0]);
       // lanes [0,16): gate row it, [32,48): up row it, [16,32): gate row it+1, [48,64): up row it+1;
       // after the halves trade places every lane holds a row's gate and up sums, and lanes 0
       // and 16 finish the two rows in one pass over the swiglu code
@@ -667,7 +667,7 @@ __device__ __forceinline__ void one_up(const OneArgs& o, int u, char* lds) {
       KL::accumulate(ru[it], L, u0);
       KL::accumulate(rg[it + 1], L, g1);
       KL::accumulate(ru[it + 1], L, u1);
-      const float red = dm_wave_sum4(g0[0], u0[0], g1[0], u1[0], lane);
+      const float red = dm_wave_sum4(g0[0], u0[0], g1[0], u1[0]);
       float gsum, usum;
       dm_row_swap<32>(red, gsum, usum);
       const int oo = base + it + ((lane >> 4) & 1);
