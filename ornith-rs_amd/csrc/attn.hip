@@ -323,17 +323,17 @@ __global__ __launch_bounds__(SDPA_NT) __attribute__((amdgpu_waves_per_eu(4, 4)))
 #pragma unroll
     for (int i = 0; i < KC / 8; ++i)
       kws[i] = *reinterpret_cast<const u32x4*>(stage + grp * (ATT_KB * KROW) + key * KROW + 16 * i);
-    // the panel's 64 query values: one per lane, handed out through scalar registers
-    const int qv = __float_as_int(qs[grp * KC + lane]);
-    float acc = 0.f;
+    // the panel's 64 query values: channel 16 g + l in lane l of every 16-lane row
+    float qv[4], acc = 0.f;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) qv[g] = qs[grp * KC + 16 * g + (lane & 15)];
 #pragma unroll
     for (int i = 0; i < KC / 8; ++i) {
       const u32x4 kw = kws[i];
       const float kf[8] = {dm_bf2f_lo(kw.x), dm_bf2f_hi(kw.x), dm_bf2f_lo(kw.y), dm_bf2f_hi(kw.y),
                            dm_bf2f_lo(kw.z), dm_bf2f_hi(kw.z), dm_bf2f_lo(kw.w), dm_bf2f_hi(kw.w)};
-#pragma unroll
-      for (int e = 0; e < 8; ++e)
-        acc = dm_fma(__int_as_float(__builtin_amdgcn_readlane(qv, 8 * i + e)), kf[e], acc);
+      if (i & 1) dm_dot8<8>(acc, qv[i >> 1], kf);
+      else dm_dot8<0>(acc, qv[i >> 1], kf);
     }
     part[grp * ATT_KB + key] = acc;
   }
@@ -360,24 +360,46 @@ __global__ __launch_bounds__(SDPA_NT) __attribute__((amdgpu_waves_per_eu(4, 4)))
   }
   // values: thread (channel, group of 64 keys) runs the chain over the group's valid keys
   bf16_t (*vst)[HD] = reinterpret_cast<bf16_t (*)[HD]>(stage);
+  // (up to the end of the last chain that runs, zeros past the last key: its probabilities are 0)
+  const int nstage = (nvalid + VB - 1) / VB * VB;
 #pragma unroll
-  for (int u = 0; u < NLD; ++u)
-    if (row0 + RPU * u < nvalid) *reinterpret_cast<u32x4*>(&vst[row0 + RPU * u][8 * piece]) = vreg[u];
+  for (int u = 0; u < NLD; ++u) {
+    const int r = row0 + RPU * u;
+    if (r < nstage) *reinterpret_cast<u32x4*>(&vst[r][8 * piece]) = r < nvalid ? vreg[u] : u32x4{0, 0, 0, 0};
+  }
   __syncthreads();  // probabilities and value rows in place (the key panels were last read two barriers ago)
-  const int ch = tid % HD, vg = tid / HD;
-  if (vg < NVB && VB * vg >= nvalid) part[vg * HD + ch] = 0.f;  // a chain with no valid key
+  // two channels a thread
+  const int ch = 2 * (tid % (HD / 2)), vg = tid / (HD / 2);
+  if (vg < NVB && VB * vg >= nvalid) part[vg * HD + ch] = part[vg * HD + ch + 1] = 0.f;  // a chain with no valid key
   if (vg < NVB && VB * vg < nvalid) {
-    const int prv = __float_as_int(pr[VB * vg + lane]);
-    bf16_t vv[VB];
+    float o[2] = {0.f, 0.f};
+    auto sixteen = [&](auto gc) {
+      constexpr int G = decltype(gc)::value;
+      const float w = pr[VB * vg + 16 * G + (lane & 15)];
+      uint32_t raw[16];
 #pragma unroll
-    for (int j = 0; j < VB; ++j) vv[j] = vst[VB * vg + j][ch];
-    float o = 0.f;
+      for (int u = 0; u < 16; ++u) raw[u] = *reinterpret_cast<const uint32_t*>(&vst[VB * vg + 16 * G + u][ch]);
+      auto four = [&](auto bc) {
+        constexpr int B = decltype(bc)::value;
+        float v[4][2];
 #pragma unroll
-    for (int j = 0; j < VB; ++j) {
-      const float next = dm_fma(__int_as_float(__builtin_amdgcn_readlane(prv, j)), dm_bf2f(vv[j]), o);
-      o = VB * vg + j < nvalid ? next : o;
-    }
-    part[vg * HD + ch] = o;
+        for (int u = 0; u < 4; ++u) {
+          v[u][0] = dm_bf2f_lo(raw[B + u]);
+          v[u][1] = dm_bf2f_hi(raw[B + u]);
+        }
+        dm_axpy4<B>(o, w, v);
+      };
+      four(std::integral_constant<int, 0>{});
+      four(std::integral_constant<int, 4>{});
+      four(std::integral_constant<int, 8>{});
+      four(std::integral_constant<int, 12>{});
+    };
+    sixteen(std::integral_constant<int, 0>{});
+    sixteen(std::integral_constant<int, 1>{});
+    sixteen(std::integral_constant<int, 2>{});
+    sixteen(std::integral_constant<int, 3>{});
+    part[vg * HD + ch] = o[0];
+    part[vg * HD + ch + 1] = o[1];
   }
   __syncthreads();
   const size_t pi = ((size_t)t * p.Hq + hq) * p.nblk + b;
@@ -403,188 +425,222 @@ __global__ __launch_bounds__(SDPA_NT) __attribute__((amdgpu_waves_per_eu(4, 4)))
   }
 }
 
-// The same partial sums when there are many blocks to work through (long contexts): 256
-// threads a block, several blocks resident per compute unit. A workgroup takes NH query heads
-// of one KV group (four when the group allows it): the key and value block is then read once
-// for the four instead of once a head (with one head a workgroup the L2 delivered every block
-// 32 times for 8 heads a group and 4 rows, 440 MB a call at a 6.6 k context, and that, not
-// HBM or the arithmetic, set the time). Thread `tid` owns key `tid` for the scores and runs
-// the chains of 64 channels one after the other; the key block reaches it through LDS, 64
-// channels at a time, so that the global loads are whole 128-byte pieces of a row. For the
-// values a thread owns four channels of one 64-key chain (8-byte loads, a wavefront reads 512
-// contiguous bytes a key); the four chains of a channel meet in LDS. Every sum of every head
-// keeps its order. grid (nblk, Hq / NH, T), 256 threads.
-template <int HD, int NH>
-__global__ __launch_bounds__(256) void sdpa_partial_many_kernel(SdpaArgs p) {
-  const int b = blockIdx.x, hq0 = blockIdx.y * NH, t = blockIdx.z, tid = threadIdx.x;
-  const int lane = tid & 63, wave = tid >> 6;
+// Which (key block, first of four heads, row) a workgroup of a linear grid works on.
+// Workgroups go round the eight dies in order, and every die has an L2 of its own: with the block
+// index running fastest the heads and rows that read one key / value block sit on different dies, each
+// of which fetches it (nine rows at a 16 k context: 97 us against 82). So everything that reads one (block, KV head) is given to one die, next
+// to each other in its order. false: past the end (the last round of dies is padded).
+constexpr int kDies = 8, kManyHeads = 4;
+__host__ __device__ __forceinline__ int sdpa_head_groups(const SdpaArgs& p) { return (p.Hq / p.Hkv + kManyHeads - 1) / kManyHeads; }
+// the (KV head, first head, how many of the four exist, row) of this workgroup
+__device__ __forceinline__ bool sdpa_place(const SdpaArgs& p, int& b, int& hk, int& hq0, int& nh, int& t) {
+  const int group = p.Hq / p.Hkv, per = sdpa_head_groups(p), sharers = per * p.T;
+  const int die = blockIdx.x % kDies, n = blockIdx.x / kDies, round = n / sharers, s = n - round * sharers;
+  const int pair = round * kDies + die;  // KV head fastest: the pairs of a short context on different dies
+  if (pair >= p.nblk * p.Hkv) return false;
+  b = pair / p.Hkv;
+  hk = pair - b * p.Hkv;
+  t = s / per;
+  const int h = (s - t * per) * kManyHeads;
+  hq0 = hk * group + h;
+  nh = min(kManyHeads, group - h);
+  return true;
+}
+unsigned sdpa_many_grid(const SdpaArgs& p) {
+  return (unsigned)((p.nblk * p.Hkv + kDies - 1) / kDies * kDies * sdpa_head_groups(p) * p.T);
+}
+
+// The same partial sums when there are many blocks to work through (long contexts): several
+// workgroups resident per compute unit, and four query heads of a KV group in each, so that the key
+// and value block is read once for the four.
+//
+// The arithmetic, fp32 chains of 64 whose order is fixed, is what bounds a block, and it runs on the
+// matrix cores all the same: v_mfma_f32_4x4x1_16b_f32 adds one product to every element with one
+// rounding (K = 1: the fused multiply-add of the chain's next step, bit for bit), 64 keys or channels
+// by four heads an instruction. The heads' side (queries, later probabilities) is broadcast inside the
+// instruction (cbsz = 4: every block takes the four values of block abid), so a register holds 16 steps
+// of it. Eight clocks for 256 multiply-adds where vector instructions take 11 to 20 (two to four
+// wavefronts a SIMD; a wavefront alone on its SIMD issues one every eight clocks).
+//
+// Scores: lane = key; wavefronts 0 - 3 run the lower half of the 64-channel chains, 4 - 7 the upper
+// half, the key block reaching them through LDS a chain of each at a time (global loads of whole
+// 128-byte pieces). Values: a wavefront has one 64-key chain of half the channels, two a lane; the
+// four chains of a channel meet in LDS. Every sum of every head keeps its order.
+// us before (256 threads, vector fmas, queries read from LDS) -> now, two KV groups of eight heads of 256:
+// 4 rows at 6621 keys 23.7 -> 17.4, 2 at 9000 23.2 -> 17.0, 6 at 1445 19.3 -> 12.3, 9 at 16000 117 -> 62.
+// (A KV group that is no multiple of four heads repeats its last one; what that makes is not stored.)
+// grid sdpa_many_grid, 512 threads
+template <int HD>
+__global__ __launch_bounds__(512, 4) void sdpa_partial_many_kernel(SdpaArgs p) {
+  constexpr int NH = kManyHeads, NT = 512;
+  int b, hk, hq0, nh, t;
+  if (!sdpa_place(p, b, hk, hq0, nh, t)) return;
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int offset = p.d_offset ? *p.d_offset : p.offset;
   const int last = min(offset + t, p.cap - 1);
   if (b * ATT_KB > last) return;
-  const int hk = hq0 / (p.Hq / p.Hkv);  // the NH heads share it
-  constexpr int NKC = HD / 64, NVB = ATT_KB / 64, KLD = 64 + 8;
-  static_assert(ATT_KB == 256, "one key per thread");
+  constexpr int NKC = HD / 64, NVB = ATT_KB / 64, KLD = 64 + 8, STEPS = NKC / 2;
+  static_assert(ATT_KB == 256, "four wavefronts of keys");
   static_assert(NKC == 2 || NKC == 4, "head widths of 128 and 256");
+  typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-  __shared__ __align__(16) bf16_t ks[ATT_KB][KLD];
-  __shared__ __align__(16) float qs[NH][HD];
+  // the key panels; before them the queries, after them the halves' score sums and the value chains
+  __shared__ __align__(16) bf16_t ks[2][ATT_KB][KLD];
   __shared__ float pr[NH][ATT_KB];
   __shared__ float red[NH][4];
-  __shared__ float part[NH][NVB * HD];
+  float* const part = reinterpret_cast<float*>(ks);  // [NH][NVB * HD]
+  static_assert(sizeof(ks) >= NH * NVB * HD * 4, "the value chains fit where the keys were");
 
-  const int key = b * ATT_KB + tid;
-  const bool valid = key <= last;
+  const int half = wave >> 2, row = (wave & 3) * 64 + lane;  // of the scores: chains of this half, this key
+  const int j0 = 2 * half;                                   // of the softmax: heads j0, j0 + 1
+  const bool valid = b * ATT_KB + row <= last;
   const int nvalid = min(ATT_KB, last - b * ATT_KB + 1);
-  const bf16_t* kblk = p.k_cache + ((size_t)hk * p.cap + (size_t)b * ATT_KB) * HD;
+  // (rows past the last key read as zeros: their scores are masked, their probabilities 0)
+  const size_t blk0 = ((size_t)hk * p.cap + (size_t)b * ATT_KB) * HD;
+  const __amdgpu_buffer_rsrc_t kbuf = dm_buffer(p.k_cache + blk0, nvalid * HD * 2), vbuf = dm_buffer(p.v_cache + blk0, nvalid * HD * 2);
 
-  // 64-channel panel c of the key block: 2048 16-byte pieces, eight a thread (rows past the
-  // last key read the last key's: their scores are masked). Two panels travel in registers
-  // ahead of their use, and so do the first 32 keys of this thread's value chain: a block is a
-  // chain of memory latencies otherwise.
-  u32x4 kreg[2][8];
-  auto fetch_panel = [&](auto set, int c) {
-    constexpr int S = decltype(set)::value;
+  // step s: panels s and s + STEPS, 4096 16-byte pieces. All of a step travels in registers ahead of
+  // its use, and so do the first 32 keys of this thread's value chain: a block is a chain of memory
+  // latencies otherwise.
+  u32x4 kreg[8];
+  auto fetch_keys = [&](int s) {
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
-      const int idx = tid + 256 * u, r = min(idx >> 3, nvalid - 1), part8 = idx & 7;
-      kreg[S][u] = *reinterpret_cast<const u32x4*>(kblk + (size_t)r * HD + 64 * c + 8 * part8);
+      const int idx = tid + NT * (u & 3);
+      kreg[u] = __builtin_amdgcn_raw_buffer_load_b128(kbuf, (idx >> 3) * (HD * 2) + 16 * (idx & 7) + 128 * (s + STEPS * (u >> 2)), 0, 0);
+    }
+  };
+  fetch_keys(0);
+  constexpr int TPC = HD / 2;  // threads a value chain
+  const int vg = tid / TPC, vcg = tid % TPC;
+  const bool holds = vg < NVB;  // (whole wavefronts)
+  uint32_t vreg[2][16];
+  auto fetch_values = [&](auto set, int i0) {
+    constexpr int S = decltype(set)::value;
+    if (holds) {
+#pragma unroll
+      for (int u = 0; u < 16; ++u)
+        vreg[S][u] = __builtin_amdgcn_raw_buffer_load_b32(vbuf, (64 * vg + i0 + u) * (HD * 2) + 4 * vcg, 0, 0);
     }
   };
   using S0 = std::integral_constant<int, 0>;
   using S1 = std::integral_constant<int, 1>;
-  fetch_panel(S0{}, 0);
-  fetch_panel(S1{}, 1);
-  constexpr int TPC = HD / 4;  // threads a value chain
-  const int vg = tid / TPC, vcg = tid % TPC;
-  const bf16_t* vcol = p.v_cache + ((size_t)hk * p.cap + (size_t)b * ATT_KB + 64 * vg) * HD + 4 * vcg;
-  const int vn = min(64, nvalid - 64 * vg);  // keys of this thread's chain that exist (may be <= 0)
-  uint2 vreg[2][16];
-  auto fetch_values = [&](auto set, int i0) {
-    constexpr int S = decltype(set)::value;
-    if (tid < HD) {
-#pragma unroll
-      for (int u = 0; u < 16; ++u)
-        vreg[S][u] = *reinterpret_cast<const uint2*>(vcol + (size_t)min(i0 + u, max(vn - 1, 0)) * HD);
-    }
-  };
   fetch_values(S0{}, 0);
   fetch_values(S1{}, 16);
-  for (int i = tid; i < NH * HD; i += 256)
-    qs[i / HD][i % HD] = p.scale * dm_bf2f(p.q_rot[((size_t)t * p.Hq + hq0 + i / HD) * HD + i % HD]);
-  float cpart[NH][NKC];
-  auto panel = [&](auto set, auto cc) {
-    constexpr int S = decltype(set)::value, c = decltype(cc)::value;
+  // this half's query channels: 16 g + a of head i in lane 4 a + i
+  constexpr int QG = HD / 32;
+  float q[QG];
+  {
+    const bf16_t* qrow = p.q_rot + ((size_t)t * p.Hq + hq0 + min(lane & 3, nh - 1)) * HD + half * (HD / 2) + (lane >> 2);
+#pragma unroll
+    for (int g = 0; g < QG; ++g) q[g] = p.scale * dm_bf2f(qrow[16 * g]);
+  }
+  auto step16 = [&](f32x4 acc, float qv, const float (&k)[16]) {
+#define ORN_STEP(A) acc = __builtin_amdgcn_mfma_f32_4x4x1f32(qv, k[A], acc, 4, A, 0);
+    ORN_STEP(0) ORN_STEP(1) ORN_STEP(2) ORN_STEP(3) ORN_STEP(4) ORN_STEP(5) ORN_STEP(6) ORN_STEP(7)
+    ORN_STEP(8) ORN_STEP(9) ORN_STEP(10) ORN_STEP(11) ORN_STEP(12) ORN_STEP(13) ORN_STEP(14) ORN_STEP(15)
+#undef ORN_STEP
+    return acc;
+  };
+  f32x4 chain[STEPS];
+  auto scores = [&](auto sc) {
+    constexpr int s = decltype(sc)::value;
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
-      const int idx = tid + 256 * u;
-      *reinterpret_cast<u32x4*>(&ks[idx >> 3][8 * (idx & 7)]) = kreg[S][u];
+      const int idx = tid + NT * (u & 3);
+      *reinterpret_cast<u32x4*>(&ks[u >> 2][idx >> 3][8 * (idx & 7)]) = kreg[u];
     }
     __syncthreads();
-    if constexpr (c + 2 < NKC) fetch_panel(set, c + 2);
-    float a[NH];
+    if constexpr (s + 1 < STEPS) fetch_keys(s + 1);
+    chain[s] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int j = 0; j < NH; ++j) a[j] = 0.f;
+    for (int g = 0; g < 4; ++g) {
+      float k[16];
 #pragma unroll
-    for (int dc = 0; dc < 8; ++dc) {
-      const uint4 kw = *reinterpret_cast<const uint4*>(&ks[tid][8 * dc]);
-      const float k0 = dm_bf2f_lo(kw.x), k1 = dm_bf2f_hi(kw.x), k2 = dm_bf2f_lo(kw.y), k3 = dm_bf2f_hi(kw.y);
-      const float k4 = dm_bf2f_lo(kw.z), k5 = dm_bf2f_hi(kw.z), k6 = dm_bf2f_lo(kw.w), k7 = dm_bf2f_hi(kw.w);
+      for (int h = 0; h < 2; ++h) {
+        const uint4 kw = *reinterpret_cast<const uint4*>(&ks[half][row][16 * g + 8 * h]);
+        const uint32_t w[4] = {kw.x, kw.y, kw.z, kw.w};
 #pragma unroll
-      for (int j = 0; j < NH; ++j) {
-        const float4 q0 = *reinterpret_cast<const float4*>(&qs[j][64 * c + 8 * dc]);
-        const float4 q1 = *reinterpret_cast<const float4*>(&qs[j][64 * c + 8 * dc + 4]);
-        a[j] = dm_fma(q0.x, k0, a[j]);
-        a[j] = dm_fma(q0.y, k1, a[j]);
-        a[j] = dm_fma(q0.z, k2, a[j]);
-        a[j] = dm_fma(q0.w, k3, a[j]);
-        a[j] = dm_fma(q1.x, k4, a[j]);
-        a[j] = dm_fma(q1.y, k5, a[j]);
-        a[j] = dm_fma(q1.z, k6, a[j]);
-        a[j] = dm_fma(q1.w, k7, a[j]);
+        for (int e = 0; e < 4; ++e) {
+          k[8 * h + 2 * e] = dm_bf2f_lo(w[e]);
+          k[8 * h + 2 * e + 1] = dm_bf2f_hi(w[e]);
+        }
       }
+      chain[s] = step16(chain[s], q[4 * s + g], k);
     }
-#pragma unroll
-    for (int j = 0; j < NH; ++j) cpart[j][c] = a[j];
     __syncthreads();
   };
-  panel(S0{}, std::integral_constant<int, 0>{});
-  panel(S1{}, std::integral_constant<int, 1>{});
-  if constexpr (NKC > 2) {
-    panel(S0{}, std::integral_constant<int, 2>{});
-    panel(S1{}, std::integral_constant<int, 3>{});
-  }
-  float sc[NH], mg[NH];
+  scores(S0{});
+  if constexpr (STEPS == 2) scores(S1{});
+  // (c0 + c1) + (c2 + c3): each half hands the other the two heads it does not go on with
+  f32x4 sum = chain[0];
+  if constexpr (STEPS == 2) sum = chain[0] + chain[1];
+  float* const other = part + row;
 #pragma unroll
-  for (int j = 0; j < NH; ++j) {
-    sc[j] = sdpa_pair_tree<NKC>(cpart[j], 1);
+  for (int j = 0; j < 2; ++j) other[((half ^ 1) * 2 + j) * ATT_KB] = half ? sum[j] : sum[2 + j];
+  __syncthreads();
+  float sc[2], mg[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const float mine = half ? sum[2 + j] : sum[j], theirs = other[(j0 + j) * ATT_KB];
+    sc[j] = mine + theirs;
     const float m = dm_wave_max<64>(valid ? sc[j] : -DM_INF);  // block max
-    if (lane == 0) red[j][wave] = m;
+    if (lane == 0) red[j0 + j][wave & 3] = m;
   }
   __syncthreads();
 #pragma unroll
-  for (int j = 0; j < NH; ++j) {
-    float m = red[j][0];
-    m = red[j][1] > m ? red[j][1] : m;
-    m = red[j][2] > m ? red[j][2] : m;
-    m = red[j][3] > m ? red[j][3] : m;
+  for (int j = 0; j < 2; ++j) {
+    const float* r = red[j0 + j];
+    float m = r[0];
+    m = r[1] > m ? r[1] : m;
+    m = r[2] > m ? r[2] : m;
+    m = r[3] > m ? r[3] : m;
     mg[j] = m;
   }
   __syncthreads();
 #pragma unroll
-  for (int j = 0; j < NH; ++j) {
+  for (int j = 0; j < 2; ++j) {
     const float pv = valid ? dm_exp(sc[j] - mg[j]) : 0.f;
-    pr[j][tid] = pv;
+    pr[j0 + j][row] = pv;
     const float ws = dm_wave_sum<64>(pv);
-    if (lane == 0) red[j][wave] = ws;
+    if (lane == 0) red[j0 + j][wave & 3] = ws;
+    if (row == 0 && j0 + j < nh) p.part_m[((size_t)t * p.Hq + hq0 + j0 + j) * p.nblk + b] = mg[j];
   }
   __syncthreads();
-  // values: chain vg = keys 64 * vg .. + 64, channels 4 * vcg .. + 4, for every head
-  if (tid < HD) {
-    float o[NH][4];
-#pragma unroll
-    for (int j = 0; j < NH; ++j)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) o[j][e] = 0.f;
-    auto batch = [&](auto set, int i0) {
+  // values: chain vg = keys 64 * vg .. + 64, channels 2 vcg, 2 vcg + 1 of the four heads
+  if (holds) {
+    f32x4 o0 = {0.f, 0.f, 0.f, 0.f}, o1 = o0;
+    auto batch = [&](auto set, int g) {
       constexpr int S = decltype(set)::value;
-#pragma unroll
-      for (int u = 0; u < 16; ++u)
-        if (i0 + u < vn) {
-          const float v0 = dm_bf2f_lo(vreg[S][u].x), v1 = dm_bf2f_hi(vreg[S][u].x);
-          const float v2 = dm_bf2f_lo(vreg[S][u].y), v3 = dm_bf2f_hi(vreg[S][u].y);
-#pragma unroll
-          for (int j = 0; j < NH; ++j) {
-            const float pw = pr[j][64 * vg + i0 + u];
-            o[j][0] = dm_fma(pw, v0, o[j][0]);
-            o[j][1] = dm_fma(pw, v1, o[j][1]);
-            o[j][2] = dm_fma(pw, v2, o[j][2]);
-            o[j][3] = dm_fma(pw, v3, o[j][3]);
-          }
-        }
+      const float w = pr[lane & 3][64 * vg + 16 * g + (lane >> 2)];  // key a of head i in lane 4 a + i
+#define ORN_KEY(A)                                                                                  \
+  o0 = __builtin_amdgcn_mfma_f32_4x4x1f32(w, dm_bf2f_lo(vreg[S][A]), o0, 4, A, 0);                  \
+  o1 = __builtin_amdgcn_mfma_f32_4x4x1f32(w, dm_bf2f_hi(vreg[S][A]), o1, 4, A, 0);
+      ORN_KEY(0) ORN_KEY(1) ORN_KEY(2) ORN_KEY(3) ORN_KEY(4) ORN_KEY(5) ORN_KEY(6) ORN_KEY(7)
+      ORN_KEY(8) ORN_KEY(9) ORN_KEY(10) ORN_KEY(11) ORN_KEY(12) ORN_KEY(13) ORN_KEY(14) ORN_KEY(15)
+#undef ORN_KEY
     };
     batch(S0{}, 0);
     fetch_values(S0{}, 32);
-    batch(S1{}, 16);
+    batch(S1{}, 1);
     fetch_values(S1{}, 48);
-    batch(S0{}, 32);
-    batch(S1{}, 48);
+    batch(S0{}, 2);
+    batch(S1{}, 3);
 #pragma unroll
     for (int j = 0; j < NH; ++j)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) part[j][vg * HD + 4 * vcg + e] = o[j][e];
+      *reinterpret_cast<float2*>(&part[j * (NVB * HD) + vg * HD + 2 * vcg]) = make_float2(o0[j], o1[j]);
   }
   __syncthreads();
-#pragma unroll
-  for (int j = 0; j < NH; ++j) {
-    const size_t pi = ((size_t)t * p.Hq + hq0 + j) * p.nblk + b;
-    if (tid < HD) p.part_o[pi * HD + tid] = sdpa_pair_tree<NVB>(part[j] + tid, HD);
-    if (tid == 0) {
-      float l = red[j][0] + red[j][1];
-      l = l + red[j][2];
-      l = l + red[j][3];
-      p.part_m[pi] = mg[j];
-      p.part_l[pi] = l;
-    }
+  for (int i = tid; i < nh * HD; i += NT) {
+    const int j = i / HD, d = i - j * HD;
+    p.part_o[(((size_t)t * p.Hq + hq0 + j) * p.nblk + b) * HD + d] = sdpa_pair_tree<NVB>(part + j * (NVB * HD) + d, HD);
+  }
+  if (tid < nh) {
+    float l = red[tid][0] + red[tid][1];
+    l = l + red[tid][2];
+    l = l + red[tid][3];
+    p.part_l[((size_t)t * p.Hq + hq0 + tid) * p.nblk + b] = l;
   }
 }
 
@@ -780,7 +836,7 @@ static int sdpa_decode(ornith_ctx* ctx, const void* d_q_rot, const void* d_k_cac
   p.scale = scale;
   // one query head per workgroup: the arithmetic (256 keys x head_dim fmas per head) is what
   // bounds a block, so spreading heads over workgroups beats sharing the key loads
-  dim3 grid(nblk, Hq, T);
+  const dim3 grid(nblk, Hq, T);
   // few live blocks (short contexts): one 1024-thread block per (key block, head) finishes
   // soonest; many: the 256-thread form keeps more blocks in flight. Same sums either way.
   const int last_max = (d_offset ? cap - 1 : (offset + T - 1 < cap - 1 ? offset + T - 1 : cap - 1));
@@ -803,14 +859,10 @@ static int sdpa_decode(ornith_ctx* ctx, const void* d_q_rot, const void* d_k_cac
     }
   }
   if (many) {
-    const dim3 g4(nblk, Hq / 4, T);
-    if (hd == 256) {
-      if (four) hipLaunchKernelGGL((sdpa_partial_many_kernel<256, 4>), g4, dim3(256), 0, ctx->stream, p);
-      else hipLaunchKernelGGL((sdpa_partial_many_kernel<256, 1>), grid, dim3(256), 0, ctx->stream, p);
-    } else {
-      if (four) hipLaunchKernelGGL((sdpa_partial_many_kernel<128, 4>), g4, dim3(256), 0, ctx->stream, p);
-      else hipLaunchKernelGGL((sdpa_partial_many_kernel<128, 1>), grid, dim3(256), 0, ctx->stream, p);
-    }
+    if (hd == 256)
+      hipLaunchKernelGGL(sdpa_partial_many_kernel<256>, dim3(sdpa_many_grid(p)), dim3(512), 0, ctx->stream, p);
+    else
+      hipLaunchKernelGGL(sdpa_partial_many_kernel<128>, dim3(sdpa_many_grid(p)), dim3(512), 0, ctx->stream, p);
   } else if (hd == 256) {
     // 150 KB of LDS a block (the whole key block staged at once): asked for once per kernel
     if (!(ctx->lds_attr_set & 1)) {

@@ -29,6 +29,16 @@ __device__ __forceinline__ T* dm_global_ptr(uint64_t bits) {
   return (T*)(__attribute__((address_space(1))) T*)bits;
 }
 
+// A range of device memory for the buffer loads: what lies past its end reads as zero, so ragged
+// blocks need no clamped addresses and no selects. The offset is 32 bits, from a wavefront-wide base; it
+// goes into the loads' vector and immediate offsets (the scalar one is not part of the comparison with
+// the end, it is taken off the end, which must not wrap).
+typedef unsigned int dm_u32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned int dm_u32x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t dm_buffer(const void* p, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)bytes, 0x00020000);
+}
+
 __device__ __forceinline__ float dm_fma(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 
 __device__ __forceinline__ float dm_bf2f(bf16_t b) { return __uint_as_float((uint32_t)b << 16); }
@@ -303,6 +313,44 @@ __device__ __forceinline__ int dm_multi_of(int c) {
 __device__ __forceinline__ float dm_lane_value(float v, int lane) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane));
 }
+
+// Fused multiply-adds whose first factor is one lane's value of a 16-lane row (DPP row_newbcast): a
+// factor that is the same for all lanes, a query's channels or a row of probabilities, stays one
+// value a lane, 16 to a register in every row, and is neither read from LDS nor moved to a scalar
+// register for each use (a 16-byte broadcast read is 16 clocks of the compute unit's LDS, a
+// v_readlane the price of the multiply-add). All 64 lanes must be active. The two wait states that a
+// DPP read needs after its register was written stand at the head of each group.
+#define DM_FMAC(A, X, Y, I) "v_fmac_f32_dpp %" #A ", %" #X ", %" #Y " row_newbcast:" #I " row_mask:0xf bank_mask:0xf\n\t"
+// acc[j] += q[j](lane B + e) * k[e], e = 0 .. 7 in order, B = 0 or 8
+template <int B>
+__device__ __forceinline__ void dm_dot8(float& a, float q, const float (&k)[8]) {
+  if constexpr (B == 0)
+    asm("s_nop 1\n\t" DM_FMAC(0, 1, 2, 0) DM_FMAC(0, 1, 3, 1) DM_FMAC(0, 1, 4, 2) DM_FMAC(0, 1, 5, 3) DM_FMAC(0, 1, 6, 4)
+            DM_FMAC(0, 1, 7, 5) DM_FMAC(0, 1, 8, 6) DM_FMAC(0, 1, 9, 7)
+        : "+&v"(a)
+        : "v"(q), "v"(k[0]), "v"(k[1]), "v"(k[2]), "v"(k[3]), "v"(k[4]), "v"(k[5]), "v"(k[6]), "v"(k[7]));
+  else
+    asm("s_nop 1\n\t" DM_FMAC(0, 1, 2, 8) DM_FMAC(0, 1, 3, 9) DM_FMAC(0, 1, 4, 10) DM_FMAC(0, 1, 5, 11) DM_FMAC(0, 1, 6, 12)
+            DM_FMAC(0, 1, 7, 13) DM_FMAC(0, 1, 8, 14) DM_FMAC(0, 1, 9, 15)
+        : "+&v"(a)
+        : "v"(q), "v"(k[0]), "v"(k[1]), "v"(k[2]), "v"(k[3]), "v"(k[4]), "v"(k[5]), "v"(k[6]), "v"(k[7]));
+}
+// o[e] += w(lane B + u) * v[u][e], u = 0 .. 3 in order: two channels, four keys; B = 0, 4, 8, 12
+#define DM_FMACW(V0, V1, I) DM_FMAC(0, 2, V0, I) DM_FMAC(1, 2, V1, I)
+#define DM_AXPY2(I0, I1, I2, I3)                                                                                          \
+  asm("s_nop 1\n\t" DM_FMACW(3, 4, I0) DM_FMACW(5, 6, I1) DM_FMACW(7, 8, I2) DM_FMACW(9, 10, I3)                           \
+      : "+&v"(o[0]), "+&v"(o[1])                                                                                            \
+      : "v"(w), "v"(v[0][0]), "v"(v[0][1]), "v"(v[1][0]), "v"(v[1][1]), "v"(v[2][0]), "v"(v[2][1]), "v"(v[3][0]), "v"(v[3][1]))
+template <int B>
+__device__ __forceinline__ void dm_axpy4(float (&o)[2], float w, const float (&v)[4][2]) {
+  if constexpr (B == 0) DM_AXPY2(0, 1, 2, 3);
+  else if constexpr (B == 4) DM_AXPY2(4, 5, 6, 7);
+  else if constexpr (B == 8) DM_AXPY2(8, 9, 10, 11);
+  else DM_AXPY2(12, 13, 14, 15);
+}
+#undef DM_FMACW
+#undef DM_AXPY2
+#undef DM_FMAC
 
 // byte k of a dword as a float, one instruction (the compiler's own pattern match gives
 // a bit-field extract plus a convert once the operand carries a nibble mask)
