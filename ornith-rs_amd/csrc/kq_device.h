@@ -251,6 +251,15 @@ __device__ __forceinline__ void q6_accumulate(const Q6Row& r, const Q6Lane<M>& L
   }
 }
 
+// A row's codes are not unpacked before `sum` is made: left alone, the compiler unpacks every row in
+// hand ahead, 32 registers a row.
+__device__ __forceinline__ void kq_after(Q4Row& r, float sum) {
+  asm volatile("" : "+v"(r.q.x), "+v"(r.q.y), "+v"(r.q.z), "+v"(r.q.w) : "v"(sum));
+}
+__device__ __forceinline__ void kq_after(Q6Row& r, float sum) {
+  asm volatile("" : "+v"(r.qa.x), "+v"(r.qa.y), "+v"(r.qa.z), "+v"(r.qa.w), "+v"(r.qb.x), "+v"(r.qb.y), "+v"(r.qb.z), "+v"(r.qb.w) : "v"(sum));
+}
+
 // format-generic front: lane registers, row load, accumulate
 template <int KIND, int M>
 struct KqLane;

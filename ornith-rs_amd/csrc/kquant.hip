@@ -215,7 +215,8 @@ __global__ __launch_bounds__(256) void kq_qmv_kernel(KqArgs a) {
 #pragma unroll
         for (int t = 0; t < M; ++t) one[t] = 0.f;
         if (u == 0 || it + u < a.iters) {
-          const typename KL::Row r = pf[i + u];
+          typename KL::Row r = pf[i + u];
+          if constexpr (FR > 1 && M == 1) kq_after(r, u > 0 ? acc[u - 1] : 0.f);
           if (it + u + PF < a.iters) pf[i + u] = KL::load(sg.qs, sg.scales, sg.dm, row_of(it + u + PF), nb, L);
           KL::accumulate(r, L, one);
         }

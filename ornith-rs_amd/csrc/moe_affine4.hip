@@ -210,35 +210,50 @@ __global__ __launch_bounds__(256) void moe_up_affine4_kernel(A4UpArgs<F> a) {
 // their gate and up rows asked for together and the four sums folded as one. What bounds it is the
 // chain gates -> top-k -> rows -> sums; the kernel above, which every other width takes, adds a trip
 // to memory for every 1024 columns of a row and unpacks with three instructions a code where this
-// one needs one and a half. us at T = 1 / 2, K = 2048, I = 512: 11.3 / 16.6 -> 7.3 / 10.2
-// grid (ceil(I / 8), T*k + T), 256 threads
-template <int NC, bool ROUTE>
+// one needs one and a half. LOOPS as in moe_up_kernel (moe_fused.hip): the next two rows asked for ahead
+// of the arithmetic of the present ones, once the grid is more than the chip holds. us at T = 1 / 2, K = 2048, I = 512: 11.3 / 16.6 -> 7.3 / 10.2
+// grid (ceil(I / (8 LOOPS)), T*k + T), 256 threads
+template <int NC, bool ROUTE, int LOOPS>
 __global__ __launch_bounds__(256) void moe_up_a4_kernel(A4UpArgs<FmtA4> a) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = blockIdx.y;
   const A4UpRow<FmtA4> u = a4_up_row<FmtA4, ROUTE>(a, lane, wave);
-  const int base = (blockIdx.x * 4 + wave) * 2;
-  AffRow<4, 64, NC> rg[2], ru[2];
+  const int base0 = (blockIdx.x * 4 + wave) * 2 * LOOPS;
+  constexpr int SETS = LOOPS > 1 ? 2 : 1;
+  AffRow<4, 64, NC> rows[SETS][4];  // gate 0, up 0, gate 1, up 1
+  auto fetch = [&](int l) {
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const size_t row = u.row0 + min(base + i, a.I - 1);
-    rg[i].load(u.wg.w, u.wg.scales, u.wg.biases, row, lane);
-    ru[i].load(u.wu.w, u.wu.scales, u.wu.biases, row, lane);
-  }
+    for (int i = 0; i < 2; ++i) {
+      const size_t row = u.row0 + min(base0 + 2 * l + i, a.I - 1);
+      rows[l % SETS][2 * i].load(u.wg.w, u.wg.scales, u.wg.biases, row, lane);
+      rows[l % SETS][2 * i + 1].load(u.wu.w, u.wu.scales, u.wu.biases, row, lane);
+    }
+  };
+  fetch(0);
   __builtin_amdgcn_sched_barrier(0);
   AffLane<4, 64, NC, 1> L;
   const bf16_t* xr[1] = {a.x + (size_t)u.token * a.K};
   L.load(xr, lane);
-  float g0[1] = {0.f}, u0[1] = {0.f}, g1[1] = {0.f}, u1[1] = {0.f};
-  rg[0].accumulate(L, g0);
-  ru[0].accumulate(L, u0);
-  rg[1].accumulate(L, g1);
-  ru[1].accumulate(L, u1);
-  // lanes [0,16): gate row 0, [32,48): up row 0, [16,32): gate row 1, [48,64): up row 1
-  const float red = dm_wave_sum4(g0[0], u0[0], g1[0], u1[0]);
-  float gs, us;
-  dm_row_swap<32>(red, gs, us);
-  const int o = base + ((lane >> 4) & 1);
-  if ((lane & 47) == 0 && o < a.I) a.act[(size_t)r * a.I + o] = swiglu_bf16(gs, us);
+#pragma unroll
+  for (int l = 0; l < LOOPS; ++l) {
+    if (l + 1 < LOOPS) {
+      fetch(l + 1);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    float v[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      float acc[1] = {0.f};
+      rows[l % SETS][i].accumulate(L, acc);
+      v[i] = acc[0];
+      if (LOOPS > 1 && i < 3) rows[l % SETS][i + 1].after(acc);
+    }
+    // lanes [0,16): gate row 0, [32,48): up row 0, [16,32): gate row 1, [48,64): up row 1
+    const float red = dm_wave_sum4(v[0], v[1], v[2], v[3]);
+    float gs, us;
+    dm_row_swap<32>(red, gs, us);
+    const int o = base0 + 2 * l + ((lane >> 4) & 1);
+    if ((lane & 47) == 0 && o < a.I) a.act[(size_t)r * a.I + o] = swiglu_bf16(gs, us);
+  }
 }
 
 template <class F>
@@ -325,6 +340,7 @@ __global__ __launch_bounds__(64 * (kA4MaxK + a4_shared_waves(64 / LPR * ITERS)))
   __shared__ float gsig;
   const bool shared = j >= k;
   const int it0 = shared ? (j - k) * SHARE : 0, its = shared ? SHARE : ITERS;
+  static_assert(SHARE <= 16, "a shared wavefront's passes fit its registers");
   const FmtA4::Mat w = shared ? a.sdown : a.down;
   const size_t row0 = shared ? 0 : (size_t)min(a.inds[t * k + j], (uint32_t)(a.E - 1)) * a.H;
   // what is small and cached first: loads return in issue order
@@ -334,19 +350,29 @@ __global__ __launch_bounds__(64 * (kA4MaxK + a4_shared_waves(64 / LPR * ITERS)))
   const uint16_t score_bits = a.scores[(size_t)t * k + (lane < k ? lane : 0)];
   const uint16_t egate_bits = a.egate[t];
   __builtin_amdgcn_sched_barrier(0);
-  AffRow<4, LPR, 1> rr[ITERS];
+  constexpr int PF = ITERS < 16 ? ITERS : 16;
+  AffRow<4, LPR, 1> rr[PF];
+  auto fetch = [&](int i) { rr[i % PF].load(w.w, w.scales, w.biases, row0 + min(c0 + (it0 + i) * RPW + slot, a.H - 1), c); };
 #pragma unroll
-  for (int i = 0; i < ITERS; ++i)
-    if (SW == 1 || i < its) rr[i].load(w.w, w.scales, w.biases, row0 + min(c0 + (it0 + i) * RPW + slot, a.H - 1), c);
+  for (int i = 0; i < PF; ++i)
+    if (SW == 1 || i < its) fetch(i);
   __builtin_amdgcn_sched_barrier(0);
   if (j == 0) a4_combine_weights(score_bits, egate_bits, k, a.normalize, lane, wj, &gsig);
-#pragma unroll
-  for (int i = 0; i < ITERS; ++i) {
-    if (SW > 1 && i >= its) continue;
+  auto pass = [&](int i) {
     float acc[1] = {0.f};
-    rr[i].accumulate(L, acc);
+    rr[i % PF].accumulate(L, acc);
     const float v = dm_wave_sum<LPR>(acc[0]);
     if (c == 0) yl[shared ? k : j][(it0 + i) * RPW + slot] = dm_rb(v);  // expert outputs are bf16 in the operator path
+  };
+  if (SW > 1 && shared) {
+#pragma unroll
+    for (int i = 0; i < SHARE; ++i) pass(i);
+  } else {
+#pragma unroll
+    for (int i = 0; i < ITERS; ++i) {
+      pass(i);
+      if (i + PF < ITERS) fetch(i + PF);
+    }
   }
   __syncthreads();
   const int col = threadIdx.x;
@@ -383,13 +409,21 @@ namespace {
 template <class F>
 bool launch_up_a4(ornith_ctx*, const A4UpArgs<F>&, bool) { return false; }
 bool launch_up_a4(ornith_ctx* ctx, const A4UpArgs<FmtA4>& u, bool route) {
-  const dim3 grid((u.I + 7) / 8, u.T * u.k + u.T);
-  const int nc = u.K % 1024 == 0 ? u.K / 1024 : 0;
-#define UP_NC(NC)                                                                                       \
-  if (route)                                                                                            \
-    hipLaunchKernelGGL((moe_up_a4_kernel<NC, true>), grid, dim3(256), 0, ctx->stream, u);               \
-  else                                                                                                  \
-    hipLaunchKernelGGL((moe_up_a4_kernel<NC, false>), grid, dim3(256), 0, ctx->stream, u);              \
+  const int rows_y = u.T * u.k + u.T, nc = u.K % 1024 == 0 ? u.K / 1024 : 0;
+  const long one = (long)((u.I + 7) / 8) * rows_y;
+  const int loops = one <= 5L * ctx->compute_units ? 1 : one <= 9L * ctx->compute_units ? 2 : 4;
+  const dim3 grid((u.I + 8 * loops - 1) / (8 * loops), rows_y);
+#define UP_GO(NC, ROUTE, LOOPS) hipLaunchKernelGGL((moe_up_a4_kernel<NC, ROUTE, LOOPS>), grid, dim3(256), 0, ctx->stream, u)
+#define UP_ROUTE(NC, ROUTE)                 \
+  if (loops == 1) UP_GO(NC, ROUTE, 1);      \
+  else if (loops == 2) UP_GO(NC, ROUTE, 2); \
+  else UP_GO(NC, ROUTE, 4)
+#define UP_NC(NC)         \
+  if (route) {            \
+    UP_ROUTE(NC, true);   \
+  } else {                \
+    UP_ROUTE(NC, false);  \
+  }                       \
   return true;
   switch (nc) {
     case 1: UP_NC(1)
@@ -397,6 +431,8 @@ bool launch_up_a4(ornith_ctx* ctx, const A4UpArgs<FmtA4>& u, bool route) {
     case 4: UP_NC(4)
     default: return false;
   }
+#undef UP_ROUTE
+#undef UP_GO
 #undef UP_NC
 }
 template <class F>
@@ -404,15 +440,18 @@ bool launch_down_a4(ornith_ctx*, const A4DownArgs<F>&) { return false; }
 bool launch_down_a4(ornith_ctx* ctx, const A4DownArgs<FmtA4>& d) {
   // columns a workgroup: 8 while that is no more than two workgroups a compute unit, then 16, then 32
   const int g8 = (d.H + 7) / 8 * d.T, cu = ctx->compute_units;
-  const int cols = g8 >= 3 * cu ? 32 : g8 >= 2 * cu ? 16 : 8;
+  // (and 64, half of them in registers at any time, once 32 are more workgroups than the chip holds)
+  const int cols = g8 > 4 * cu ? 64 : g8 >= 3 * cu ? 32 : g8 >= 2 * cu ? 16 : 8;
   const dim3 grid((d.H + cols - 1) / cols, d.T), block(64 * (d.k + a4_shared_waves(cols)));
 #define DOWN_LPR(LPR)                                                                                              \
   if (cols == 8)                                                                                                   \
     hipLaunchKernelGGL((moe_down_a4_kernel<LPR, 8 * LPR / 64>), grid, block, 0, ctx->stream, d);                   \
   else if (cols == 16)                                                                                             \
     hipLaunchKernelGGL((moe_down_a4_kernel<LPR, 16 * LPR / 64>), grid, block, 0, ctx->stream, d);                  \
-  else                                                                                                             \
+  else if (cols == 32) \
     hipLaunchKernelGGL((moe_down_a4_kernel<LPR, 32 * LPR / 64>), grid, block, 0, ctx->stream, d);                  \
+  else \
+    hipLaunchKernelGGL((moe_down_a4_kernel<LPR, 64 * LPR / 64>), grid, block, 0, ctx->stream, d);                  \
   return true;
   switch (d.I) {
     case 256: DOWN_LPR(16)

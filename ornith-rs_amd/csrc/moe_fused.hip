@@ -96,7 +96,15 @@ __device__ __forceinline__ float noacc_x(const Q6Lane<1>& L) { return L.x[0][0][
 // The leading flat arguments repeat what decides a workgroup's expert (the library is built with
 // kernel-argument preloading: they are in scalar registers when the wavefront starts, so the
 // gates / ids are asked for while the argument block is still being fetched).
-template <int KIND, int LPR, int ITERS, bool ROUTE>
+//
+// LOOPS: a wavefront takes its ITERS rows LOOPS times over, the next ones asked for ahead of the
+// arithmetic of the present ones. One time is the fastest while the whole grid is resident at once
+// (two tokens: 1152 workgroups); beyond that every further workgroup repeats the routing (1.2 us of
+// one wavefront, the others waiting) and the activations' conversion for two rows a wavefront, and a
+// new round of workgroups starts with an empty memory pipe. us, one / two / four times:
+// T = 2 7.9 / 8.8 / 10.7, T = 3 12.2 / 10.4 / 12.5, T = 4 14.5 / 13.5 / 13.3, T = 5 16.2 / 15.6 / 14.7, T = 8
+// 25.1 / 21.9 / 20.4, T = 16 47.1 / 39.3 / 34.1.
+template <int KIND, int LPR, int ITERS, bool ROUTE, int LOOPS = 1>
 __global__ __launch_bounds__(256) void moe_up_kernel(const bf16_t* h_gates, const uint32_t* h_inds, int h_T, int h_k,
                                                      int h_E, UpArgs a) {
   UP_MARK(0);
@@ -152,49 +160,69 @@ __global__ __launch_bounds__(256) void moe_up_kernel(const bf16_t* h_gates, cons
   const KqPtr wg = is_routed ? pin[0] : pin[2], wu = is_routed ? pin[1] : pin[3];
   typename KL::Lane L;
   L.set_chunk(c);
-  const int base = (blockIdx.x * 4 + wave) * (RPW * ITERS);
-  typename KL::Row rg[ITERS], ru[ITERS];
+  const int base0 = (blockIdx.x * 4 + wave) * (RPW * ITERS * LOOPS);
+  constexpr int SETS = LOOPS > 1 ? 2 : 1;
+  typename KL::Row rg[SETS][ITERS], ru[SETS][ITERS];
+  auto fetch = [&](int l) {
 #pragma unroll
-  for (int it = 0; it < ITERS; ++it) {
-    const int o = base + it * RPW + slot;
-    const int64_t row = row0 + (o < a.I ? o : a.I - 1);
-    rg[it] = KL::load(wg.qs, wg.scales, wg.dm, row, nb, L);
-    ru[it] = KL::load(wu.qs, wu.scales, wu.dm, row, nb, L);
-  }
+    for (int it = 0; it < ITERS; ++it) {
+      const int o = base0 + (l * ITERS + it) * RPW + slot;
+      const int64_t row = row0 + (o < a.I ? o : a.I - 1);
+      rg[l % SETS][it] = KL::load(wg.qs, wg.scales, wg.dm, row, nb, L);
+      ru[l % SETS][it] = KL::load(wu.qs, wu.scales, wu.dm, row, nb, L);
+    }
+  };
+  fetch(0);
   __builtin_amdgcn_sched_barrier(0);  // keep the weight loads ahead of the activation loads
   UP_MARK(1);
   const void* xrow[1] = {a.x + (size_t)token * a.K};
   L.template load_x<false>(xrow, c);
   UP_MARK(2);
-  if constexpr (LPR == 64 && ITERS % 2 == 0) {
-    // one row per wavefront pass: reduce two rows' gate and up sums together
 #pragma unroll
-    for (int it = 0; it < ITERS; it += 2) {
-      float g0[1] = {0.f}, u0[1] = {0.f}, g1[1] = {0.f}, u1[1] = {0.f};
-      ORN_KL_ACC(rg[it], L, g0);
-      ORN_KL_ACC(ru[it], L, u0);
-      ORN_KL_ACC(rg[it + 1], L, g1);
-      ORN_KL_ACC(ru[it + 1], L, u1);
-      const float red = dm_wave_sum4(g0[0], u0[0], g1[0], u1[0]);
-      // lanes [0,16): gate row it, [32,48): up row it, [16,32): gate row it+1, [48,64): up row it+1;
-      // after the halves trade places every lane holds a row's gate and up sums, and lanes 0
-      // and 16 finish the two rows in one pass over the swiglu code
-      float gsum, usum;
-      dm_row_swap<32>(red, gsum, usum);
-      const int o = base + it + ((lane >> 4) & 1);
-      if ((lane & 47) == 0 && o < a.I) a.act[(size_t)r * a.I + o] = swiglu_bf16(gsum, usum);
-      if (it == 0) UP_MARK(3);
+  for (int l = 0; l < LOOPS; ++l) {
+    if (l + 1 < LOOPS) {
+      fetch(l + 1);
+      __builtin_amdgcn_sched_barrier(0);
     }
-  } else {
+    auto& mg = rg[l % SETS];
+    auto& mu = ru[l % SETS];
+    float done = 0.f;  // (LOOPS > 1: a row's unpacking waits for the row before)
+    auto acc_row = [&](typename KL::Row& row, float (&acc)[1]) {
+      if constexpr (LOOPS > 1) kq_after(row, done);
+      ORN_KL_ACC(row, L, acc);
+      done = acc[0];
+    };
+    const int base = base0 + l * ITERS * RPW;
+    if constexpr (LPR == 64 && ITERS % 2 == 0) {
+      // one row per wavefront pass: reduce two rows' gate and up sums together
 #pragma unroll
-    for (int it = 0; it < ITERS; ++it) {
-      const int o = base + it * RPW + slot;
-      float ag[1] = {0.f}, au[1] = {0.f};
-      ORN_KL_ACC(rg[it], L, ag);
-      ORN_KL_ACC(ru[it], L, au);
-      const float g = dm_wave_sum<LPR>(ag[0]);
-      const float u = dm_wave_sum<LPR>(au[0]);
-      if (c == 0 && o < a.I) a.act[(size_t)r * a.I + o] = swiglu_bf16(g, u);
+      for (int it = 0; it < ITERS; it += 2) {
+        float g0[1] = {0.f}, u0[1] = {0.f}, g1[1] = {0.f}, u1[1] = {0.f};
+        acc_row(mg[it], g0);
+        acc_row(mu[it], u0);
+        acc_row(mg[it + 1], g1);
+        acc_row(mu[it + 1], u1);
+        const float red = dm_wave_sum4(g0[0], u0[0], g1[0], u1[0]);
+        // lanes [0,16): gate row it, [32,48): up row it, [16,32): gate row it+1, [48,64): up row it+1;
+        // after the halves trade places every lane holds a row's gate and up sums, and lanes 0
+        // and 16 finish the two rows in one pass over the swiglu code
+        float gsum, usum;
+        dm_row_swap<32>(red, gsum, usum);
+        const int o = base + it + ((lane >> 4) & 1);
+        if ((lane & 47) == 0 && o < a.I) a.act[(size_t)r * a.I + o] = swiglu_bf16(gsum, usum);
+        if (it == 0 && l == 0) UP_MARK(3);
+      }
+    } else {
+#pragma unroll
+      for (int it = 0; it < ITERS; ++it) {
+        const int o = base + it * RPW + slot;
+        float ag[1] = {0.f}, au[1] = {0.f};
+        acc_row(mg[it], ag);
+        acc_row(mu[it], au);
+        const float g = dm_wave_sum<LPR>(ag[0]);
+        const float u = dm_wave_sum<LPR>(au[0]);
+        if (c == 0 && o < a.I) a.act[(size_t)r * a.I + o] = swiglu_bf16(g, u);
+      }
     }
   }
   UP_MARK(4);
@@ -224,14 +252,20 @@ constexpr int kMaxK = 8;
 // 12 / 8 / 8 / 8 with a single shared wavefront (the passes are what is left to do when the rows
 // arrive: 1.1 us of a 29.5 us block at T = 4); at ITERS = 2 the same split (5 / 5 / 4 / 4 against
 // 6 / 4 / 4 / 4) measured no better, so there one wavefront k takes both groups.
+//
+// GROUPS > ITERS: the workgroup takes that many column groups, ITERS of them in registers at any time,
+// each slot asked for again as soon as its rows are worked off. Its twelve wavefronts fill the compute
+// unit, so more workgroups than compute units run one after another, each with the whole chain ids ->
+// rows -> arithmetic of its own. us, GROUPS 4 / 8: T = 5 15.0 / 11.1, T = 8
+// 16.1 / 12.5, T = 16 29.8 / 23.4
 template <int ITERS>
 constexpr int down_shared_waves() { return ITERS >= 4 ? ITERS : 1; }
-template <int KIND, int LPR, int ITERS>
+template <int KIND, int LPR, int ITERS, int GROUPS = ITERS>
 __global__ __launch_bounds__(64 * (kMaxK + down_shared_waves<ITERS>())) void moe_down_kernel(const uint8_t* h_qs, const uint8_t* h_scales,
                                                                         const uint16_t* h_dm, const uint32_t* h_inds,
                                                                         int h_k, int h_E, int h_H, int h_I, DownArgs a) {
   using KL = KqLane<KIND, 1>;
-  constexpr int RPW = 64 / LPR, COLS = RPW * ITERS;
+  constexpr int RPW = 64 / LPR, COLS = RPW * GROUPS;
   const int lane = threadIdx.x & 63, j = threadIdx.x >> 6;  // j < k: expert slot; j >= k: the shared expert's group j - k
   const int slot = lane / LPR, c = lane % LPR;
   const int nb = h_I >> 8;
@@ -245,7 +279,10 @@ __global__ __launch_bounds__(64 * (kMaxK + down_shared_waves<ITERS>())) void moe
 
   constexpr bool SPLIT = down_shared_waves<ITERS>() > 1;
   const bool shared = SPLIT ? j >= k : j == k;
-  const int only = j - k;  // SPLIT: the one column group a shared-expert wavefront takes
+  // SPLIT: a shared-expert wavefront takes SHARE column groups from `first` on
+  constexpr int SHARE = GROUPS / down_shared_waves<ITERS>();
+  static_assert(SHARE <= ITERS || !SPLIT, "a shared wavefront's groups fit its registers");
+  const int first = SPLIT && shared ? (j - k) * SHARE : 0;
   const int arow = shared ? a.T * k + t : t * k + j;
   const KqPtr w = shared ? a.sdown : KqPtr{h_qs, h_scales, h_dm};
   const int64_t row0 = shared ? 0 : (int64_t)min(h_inds[t * k + j], (uint32_t)(h_E - 1)) * h_H;
@@ -279,12 +316,13 @@ __global__ __launch_bounds__(64 * (kMaxK + down_shared_waves<ITERS>())) void moe
   const uint16_t egate_bits = a.egate[t];
   __builtin_amdgcn_sched_barrier(0);
   typename KL::Row rr[ITERS];
+  auto row_of = [&](int g) {
+    const int o = c0 + (first + g) * RPW + slot;
+    return row0 + (o < h_H ? o : h_H - 1);
+  };
 #pragma unroll
-  for (int it = 0; it < ITERS; ++it) {
-    if (SPLIT && shared && it != only) continue;
-    const int o = c0 + it * RPW + slot;
-    rr[it] = KL::load(w.qs, w.scales, w.dm, row0 + (o < h_H ? o : h_H - 1), nb, L);
-  }
+  for (int it = 0; it < ITERS; ++it)
+    if (!SPLIT || !shared || it < SHARE) rr[it] = KL::load(w.qs, w.scales, w.dm, row_of(it), nb, L);
   __builtin_amdgcn_sched_barrier(0);  // keep the weight loads ahead of everything that follows
   DOWN_MARK(1);
   if constexpr (X_VIA_LDS) {
@@ -312,13 +350,21 @@ __global__ __launch_bounds__(64 * (kMaxK + down_shared_waves<ITERS>())) void moe
   __builtin_amdgcn_s_waitcnt(0);  // vmcnt(0) with the other counters: the rows are here
   DOWN_WAVE_MARK(0);
 #endif
-#pragma unroll
-  for (int it = 0; it < ITERS; ++it) {
-    if (SPLIT && shared && it != only) continue;
+  auto group = [&](int g) {
     float acc[1] = {0.f};
-    ORN_KL_ACC(rr[it], L, acc);
+    ORN_KL_ACC(rr[g % ITERS], L, acc);
     const float v = dm_wave_sum<LPR>(acc[0]);
-    if (c == 0) yl[SPLIT && shared ? k : j][it * RPW + slot] = dm_rb(v);  // expert outputs are bf16 in the unfused path
+    if (c == 0) yl[SPLIT && shared ? k : j][(first + g) * RPW + slot] = dm_rb(v);  // expert outputs are bf16 in the unfused path
+  };
+  if (SPLIT && shared) {
+#pragma unroll
+    for (int g = 0; g < SHARE; ++g) group(g);
+  } else {
+#pragma unroll
+    for (int g = 0; g < GROUPS; ++g) {
+      group(g);
+      if (g + ITERS < GROUPS) rr[g % ITERS] = KL::load(w.qs, w.scales, w.dm, row_of(g + ITERS), nb, L);
+    }
   }
   DOWN_MARK(3);
   DOWN_WAVE_MARK(1);
@@ -350,7 +396,7 @@ struct RouterArgs {
   const bf16_t* eg_s;    // affine8 scales [K/64]
   const bf16_t* eg_b;    // affine8 biases [K/64]
   int eg_affine;
-  int E, K;
+  int E, K, M;
   PreNorm pre;           // pre.res != null: x is not read but made, x = rms_norm(res + y) (K == 2048),
                          // by every workgroup; workgroup 0 stores h and x
 };
@@ -435,7 +481,7 @@ __device__ __forceinline__ float egate_row_dot(const RouterArgs& a, const bf16_t
   return dm_wave_sum<64>(acc_lane);
 }
 
-// grid ceil(E / (RPW * 4)) + 1, 256 threads, M <= 4 tokens
+// grid (ceil(E / (RPW * 4)) + 1, groups of M <= 4 tokens), 256 threads
 // The leading flat arguments repeat what the first loads need (the norm's inputs and the router's
 // rows): preloaded into scalar registers, they let those loads leave while the argument block is
 // still being fetched.
@@ -447,6 +493,7 @@ __global__ __launch_bounds__(256) void moe_router_kernel(const bf16_t* h_res, co
   constexpr int RPW = 64 / LPR;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   __shared__ PreNormLds<M> pn;
+  const int m0 = blockIdx.y * M;  // this group's first token (of a.M; a norm in the head means a single group)
   const bool pre = h_res != nullptr;
   if (blockIdx.x == gridDim.x - 1) {
     const bool narrow = a.K / 8 <= 64 * kEgGroups;
@@ -456,10 +503,10 @@ __global__ __launch_bounds__(256) void moe_router_kernel(const bf16_t* h_res, co
     if (narrow && wave < M) egate_issue(a, lane, eg);
     __builtin_amdgcn_sched_barrier(0);
     if (pre) prenorm_finish<M>(a.pre, pg, false, pn);
-    if (wave < M) {
-      const bf16_t* xr = pre ? &pn.xn[wave][0] : a.x + (size_t)wave * a.K;
+    if (wave < M && m0 + wave < a.M) {
+      const bf16_t* xr = pre ? &pn.xn[wave][0] : a.x + (size_t)(m0 + wave) * a.K;
       const float e = narrow ? egate_finish(a, eg, xr, lane) : egate_row_dot(a, xr, lane);
-      if (lane == 0) a.egate[wave] = dm_f2bf(e);
+      if (lane == 0) a.egate[m0 + wave] = dm_f2bf(e);
     }
     return;
   }
@@ -484,16 +531,23 @@ __global__ __launch_bounds__(256) void moe_router_kernel(const bf16_t* h_res, co
   if (pre) prenorm_finish<M>(a.pre, pg, blockIdx.x == 0, pn);
   const void* xrow[M];
 #pragma unroll
-  for (int t = 0; t < M; ++t) xrow[t] = pre ? (const void*)&pn.xn[t][0] : (const void*)(a.x + (size_t)t * a.K);
+  for (int t = 0; t < M; ++t)
+    xrow[t] = pre ? (const void*)&pn.xn[t][0] : (const void*)(a.x + (size_t)min(m0 + t, a.M - 1) * a.K);
   L.template load_x<false>(xrow, c);
   float acc[M];
 #pragma unroll
   for (int t = 0; t < M; ++t) acc[t] = 0.f;
   KL::accumulate(row, L, acc);
+  if constexpr (LPR >= 32) {
+    const float v = dm_multi_sum<LPR, M>(acc);
+    const int t = dm_multi_of<LPR, M>(c);
+    if (dm_multi_leads<LPR, M>(c) && t < M && m0 + t < a.M && o < a.E) a.gates[(size_t)(m0 + t) * a.E + o] = dm_f2bf(v);
+  } else {
 #pragma unroll
-  for (int t = 0; t < M; ++t) {
-    const float v = dm_wave_sum<LPR>(acc[t]);
-    if (c == 0 && o < a.E) a.gates[(size_t)t * a.E + o] = dm_f2bf(v);
+    for (int t = 0; t < M; ++t) {
+      const float v = dm_wave_sum<LPR>(acc[t]);
+      if (c == 0 && m0 + t < a.M && o < a.E) a.gates[(size_t)(m0 + t) * a.E + o] = dm_f2bf(v);
+    }
   }
 }
 
@@ -501,8 +555,9 @@ __global__ __launch_bounds__(256) void moe_router_kernel(const bf16_t* h_res, co
 template <int KIND, int LPR>
 void launch_router_fused(ornith_ctx* ctx, const RouterArgs& a, int M) {
   constexpr int RPW = 64 / LPR;
-  dim3 grid((a.E + RPW * 4 - 1) / (RPW * 4) + 1);
-  switch (M) {
+  const int groups = (M + 3) / 4;
+  dim3 grid((a.E + RPW * 4 - 1) / (RPW * 4) + 1, groups);
+  switch ((M + groups - 1) / groups) {
     case 1: hipLaunchKernelGGL((moe_router_kernel<KIND, LPR, 1>), grid, dim3(256), 0, ctx->stream, ORN_ROUTER_HEAD(a), a); break;
     case 2: hipLaunchKernelGGL((moe_router_kernel<KIND, LPR, 2>), grid, dim3(256), 0, ctx->stream, ORN_ROUTER_HEAD(a), a); break;
     case 3: hipLaunchKernelGGL((moe_router_kernel<KIND, LPR, 3>), grid, dim3(256), 0, ctx->stream, ORN_ROUTER_HEAD(a), a); break;
@@ -835,15 +890,23 @@ void launch_up(ornith_ctx* ctx, const UpArgs& a, int rows_y) {
     else
       hipLaunchKernelGGL((moe_up_kernel<KIND, LPR, 4, false>), grid, dim3(256), 0, ctx->stream, a.gates, a.inds, a.T,
                          a.k, a.E, a);
-  } else {
-    dim3 grid((a.I + RPW * 4 * 2 - 1) / (RPW * 4 * 2), rows_y);
-    if (a.gates)
-      hipLaunchKernelGGL((moe_up_kernel<KIND, LPR, 2, true>), grid, dim3(256), 0, ctx->stream, a.gates, a.inds, a.T,
-                         a.k, a.E, a);
-    else
-      hipLaunchKernelGGL((moe_up_kernel<KIND, LPR, 2, false>), grid, dim3(256), 0, ctx->stream, a.gates, a.inds, a.T,
-                         a.k, a.E, a);
+    return;
   }
+  const long one = (long)((a.I + RPW * 8 - 1) / (RPW * 8)) * rows_y;
+  const int loops = one <= 5L * ctx->compute_units ? 1 : one <= 9L * ctx->compute_units ? 2 : 4;
+  const dim3 grid((a.I + RPW * 8 * loops - 1) / (RPW * 8 * loops), rows_y);
+#define UP_GO(ROUTE, LOOPS) \
+  hipLaunchKernelGGL((moe_up_kernel<KIND, LPR, 2, ROUTE, LOOPS>), grid, dim3(256), 0, ctx->stream, a.gates, a.inds, a.T, a.k, a.E, a)
+  if (a.gates) {
+    if (loops == 1) UP_GO(true, 1);
+    else if (loops == 2) UP_GO(true, 2);
+    else UP_GO(true, 4);
+  } else {
+    if (loops == 1) UP_GO(false, 1);
+    else if (loops == 2) UP_GO(false, 2);
+    else UP_GO(false, 4);
+  }
+#undef UP_GO
 }
 
 template <int KIND, int LPR>
@@ -858,8 +921,14 @@ void launch_down(ornith_ctx* ctx, const DownArgs& a) {
   const int iters = forced ? forced : groups1 >= 3 * cu ? 4 : groups1 >= 2 * cu ? 2 : 1;
   // k routed wavefronts and the shared expert's (one, or one a column group at four groups)
   const dim3 block(64 * (a.k + (iters >= 4 ? 4 : 1)));
-  if (iters >= 4) {
-    dim3 grid((a.H + RPW * 4 - 1) / (RPW * 4), a.T);
+  const dim3 grid4((a.H + RPW * 4 - 1) / (RPW * 4), a.T);
+  if (iters >= 4 && !forced && (long)grid4.x * a.T > cu) {
+    // more than the chip holds at once
+    const dim3 grid((a.H + RPW * 8 - 1) / (RPW * 8), a.T);
+    hipLaunchKernelGGL((moe_down_kernel<KIND, LPR, 4, 8>), grid, block, 0, ctx->stream, a.down.qs, a.down.scales,
+                       a.down.dm, a.inds, a.k, a.E, a.H, a.I, a);
+  } else if (iters >= 4) {
+    const dim3 grid = grid4;
     hipLaunchKernelGGL((moe_down_kernel<KIND, LPR, 4>), grid, block, 0, ctx->stream, a.down.qs, a.down.scales,
                        a.down.dm, a.inds, a.k, a.E, a.H, a.I, a);
   } else if (iters == 2) {
@@ -911,7 +980,7 @@ bool moe_fused_router(ornith_ctx* ctx, const ornith_moe_weights* w, const void* 
   *rc = ORNITH_OK;
   const ornith_linear& r = w->router;
   const ornith_linear& g = w->sh_egate;
-  if (T > 4 || r.mode != ORNITH_LIN_KQUANT) return false;
+  if ((T > 4 && pre) || r.mode != ORNITH_LIN_KQUANT) return false;
   if (g.mode != ORNITH_LIN_AFFINE8 && g.mode != ORNITH_LIN_DENSE) return false;
   if (g.K % 64 != 0) return false;
   const int E = r.O;
@@ -928,6 +997,7 @@ bool moe_fused_router(ornith_ctx* ctx, const ornith_moe_weights* w, const void* 
   a.eg_affine = g.mode == ORNITH_LIN_AFFINE8;
   a.E = E;
   a.K = r.K;
+  a.M = T;
   if (pre) {
     if (r.K != kPreN) return false;
     a.pre = *pre;
