@@ -117,19 +117,38 @@ __device__ __forceinline__ Q4Row q4_load(const uint8_t* qs, const uint8_t* scale
   return r;
 }
 
+// scales and minima of a chunk's two sub-blocks (64-group g of the block), d and dmin
+struct Q4Scales {
+  float s1, s2, m1, m2, d, dmin;
+  __device__ __forceinline__ Q4Scales(const Q4Row& r, int g) {
+    const int sh16 = (g & 1) * 16;
+    const uint32_t a = (r.s0 >> sh16) & 0xffffu, b = (r.s1 >> sh16) & 0xffffu, c = (r.s2 >> sh16) & 0xffffu;
+    // both field layouts evaluated, one selected: no branch in the row loop
+    const bool low = g < 2;
+    const uint32_t sc16 = low ? (a & 0x3f3fu) : ((c & 0x0f0fu) | ((a & 0xc0c0u) >> 2));
+    const uint32_t m16 = low ? (b & 0x3f3fu) : (((c >> 4) & 0x0f0fu) | ((b & 0xc0c0u) >> 2));
+    s1 = (float)(sc16 & 0xffu);
+    s2 = (float)(sc16 >> 8);
+    m1 = (float)(m16 & 0xffu);
+    m2 = (float)(m16 >> 8);
+    d = dm_h2f((f16_t)(r.dmw & 0xffffu));
+    dmin = dm_h2f((f16_t)(r.dmw >> 16));
+  }
+  // the chunk's contribution to an activation row: lo and 16 hi the sums over its low and high
+  // nibbles, sl and sh those of the activations
+  __device__ __forceinline__ float fold(float lo, float hi, float sl, float sh) const {
+    float t1 = lo * s1;
+    t1 = dm_fma(hi * 0.0625f, s2, t1);
+    float t2 = sl * m1;
+    t2 = dm_fma(sh, m2, t2);
+    const float p = d * t1;
+    return dm_fma(-dmin, t2, p);
+  }
+};
+
 template <int M>
 __device__ __forceinline__ void q4_accumulate(const Q4Row& r, const Q4Lane<M>& L, float (&acc)[M]) {
-  const int sh16 = (L.g & 1) * 16;
-  const uint32_t a = (r.s0 >> sh16) & 0xffffu, b = (r.s1 >> sh16) & 0xffffu,
-                 c = (r.s2 >> sh16) & 0xffffu;
-  // both field layouts evaluated, one selected: no branch in the row loop
-  const bool low = L.g < 2;
-  const uint32_t sc16 = low ? (a & 0x3f3fu) : ((c & 0x0f0fu) | ((a & 0xc0c0u) >> 2));
-  const uint32_t m16 = low ? (b & 0x3f3fu) : (((c >> 4) & 0x0f0fu) | ((b & 0xc0c0u) >> 2));
-  const float s1 = (float)(sc16 & 0xffu), s2 = (float)(sc16 >> 8);
-  const float m1 = (float)(m16 & 0xffu), m2 = (float)(m16 >> 8);
-  const float d = dm_h2f((f16_t)(r.dmw & 0xffffu)), dmin = dm_h2f((f16_t)(r.dmw >> 16));
-
+  const Q4Scales sc(r, L.g);
   const uint32_t w[4] = {r.q.x, r.q.y, r.q.z, r.q.w};
   float lo[M], hi[M];
 #pragma unroll
@@ -155,15 +174,7 @@ __device__ __forceinline__ void q4_accumulate(const Q4Row& r, const Q4Lane<M>& L
 #undef ORN_Q4_STEP
   }
 #pragma unroll
-  for (int t = 0; t < M; ++t) {
-    float t1 = lo[t] * s1;
-    t1 = dm_fma(hi[t] * 0.0625f, s2, t1);
-    float t2 = L.sl[t] * m1;
-    t2 = dm_fma(L.sh[t], m2, t2);
-    float p = d * t1;
-    p = dm_fma(-dmin, t2, p);
-    acc[t] = acc[t] + p;
-  }
+  for (int t = 0; t < M; ++t) acc[t] = acc[t] + sc.fold(lo[t], hi[t], L.sl[t], L.sh[t]);
 }
 
 // ---- Q6_K ---------------------------------------------------------------
@@ -208,6 +219,37 @@ __device__ __forceinline__ Q6Row q6_load(const uint8_t* qs, const uint8_t* scale
   return r;
 }
 
+// scales of a chunk's four quarters: bytes u, u+2, u+4, u+6 of the half's eight
+struct Q6Scales {
+  float c0, c1, c2, c3, d;
+  __device__ __forceinline__ Q6Scales(const Q6Row& r, int u) {
+    const uint32_t lo = r.sc.x >> (8 * u), hi = r.sc.y >> (8 * u);
+    c0 = kq_sb(lo, 0);
+    c1 = kq_sb(lo, 2);
+    c2 = kq_sb(hi, 0);
+    c3 = kq_sb(hi, 2);
+    d = dm_h2f(r.d);
+  }
+  __device__ __forceinline__ float fold(float s0, float s1, float s2, float s3) const {
+    float v = s0 * c0;
+    v = dm_fma(s1, c1, v);
+    v = dm_fma(s2, c2, v);
+    v = dm_fma(s3, c3, v);
+    return d * v;
+  }
+};
+// the codes of word k of a lane's rows, four a quarter
+template <int K>
+__device__ __forceinline__ void q6_codes(const Q6Row& r, uint32_t (&c)[4]) {
+  const uint32_t A = K == 0 ? r.qa.x : K == 1 ? r.qa.y : K == 2 ? r.qa.z : r.qa.w;
+  const uint32_t B = K == 0 ? r.qb.x : K == 1 ? r.qb.y : K == 2 ? r.qb.z : r.qb.w;
+  const uint32_t H = K == 0 ? r.qh.x : K == 1 ? r.qh.y : K == 2 ? r.qh.z : r.qh.w;
+  c[0] = (A & 0x0f0f0f0fu) | ((H << 4) & 0x30303030u);
+  c[1] = (B & 0x0f0f0f0fu) | ((H << 2) & 0x30303030u);
+  c[2] = ((A >> 4) & 0x0f0f0f0fu) | (H & 0x30303030u);
+  c[3] = ((B >> 4) & 0x0f0f0f0fu) | ((H >> 2) & 0x30303030u);
+}
+
 template <int M>
 __device__ __forceinline__ void q6_accumulate(const Q6Row& r, const Q6Lane<M>& L, float (&acc)[M]) {
   const uint32_t A[4] = {r.qa.x, r.qa.y, r.qa.z, r.qa.w};
@@ -237,18 +279,9 @@ __device__ __forceinline__ void q6_accumulate(const Q6Row& r, const Q6Lane<M>& L
     ORN_Q6_STEP(3)
 #undef ORN_Q6_STEP
   }
-  // scales: bytes u, u+2, u+4, u+6 of the half's eight
-  const uint32_t lo = r.sc.x >> (8 * L.u), hi = r.sc.y >> (8 * L.u);
-  const float c0 = kq_sb(lo, 0), c1 = kq_sb(lo, 2), c2 = kq_sb(hi, 0), c3 = kq_sb(hi, 2);
-  const float d = dm_h2f(r.d);
+  const Q6Scales sc(r, L.u);
 #pragma unroll
-  for (int t = 0; t < M; ++t) {
-    float v = s[t][0] * c0;
-    v = dm_fma(s[t][1], c1, v);
-    v = dm_fma(s[t][2], c2, v);
-    v = dm_fma(s[t][3], c3, v);
-    acc[t] = acc[t] + d * v;
-  }
+  for (int t = 0; t < M; ++t) acc[t] = acc[t] + sc.fold(s[t][0], s[t][1], s[t][2], s[t][3]);
 }
 
 // A row's codes are not unpacked before `sum` is made: left alone, the compiler unpacks every row in

@@ -232,3 +232,29 @@ def test_launch_sizing_never_changes_bits(orn, ctx):
                         assert np.array_equal(a, b), ("prenorm", kind, M, it)
     finally:
         orn.set_option("kq_iters", 0)
+
+
+@pytest.mark.parametrize("kind,K,Os,M", [(Q4K, 512, (44003,), 16), (Q4K, 1024, (29301,), 9), (Q4K, 2048, (14650, 7), 11),
+                                         (Q4K, 2048, (44001,), 3), (Q4K, 4096, (5503,), 13), (Q6K, 1024, (29298, 2), 10),
+                                         (Q6K, 2048, (22003,), 5), (Q6K, 4096, (5497,), 16), (Q4K, 256, (88001,), 15),
+                                         (Q6K, 512, (44001,), 14)])
+def test_qmv_large_launches_bit_exact(orn, ctx, kind, K, Os, M):
+    """Just beyond the size from which three and more activation rows take the matrix-core form, at each of its
+    widths (and two it does not cover): ragged weight rows, a part-filled last group, a second matrix of a few rows."""
+    rng = np.random.default_rng(K + M)
+    ts = [util.make_kq(kind, rng, 1, O, K) for O in Os]
+    lins = [orn.Linear.kquant(ctx, kind, *t, O, K) for t, O in zip(ts, Os)]
+    xb = util.bf16_normal(rng, (M, K))
+    dx, ys = ctx.to_device(xb), [ctx.alloc(M * O * 2) for O in Os]
+    ctx.linear_matmul_multi(lins, dx, M, ys)
+    for t, O, y in zip(ts, Os, ys):
+        want = util.f32_to_bf16(util.orc_qmv(kind, *t, O, K, util.bf16_to_f32(xb)))
+        assert np.array_equal(y.download(np.uint16, (M, O)), want)
+    w = _dev_matrix(orn, ctx, kind, ts[0], 1, Os[0], K)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    dxf, dyf = ctx.to_device(x), ctx.alloc(M * Os[0] * 4)
+    ctx.kq_qmv(w, dxf, orn.F32, M, dyf, orn.F32)
+    want = util.orc_qmv(kind, *ts[0], Os[0], K, x)
+    assert np.array_equal(dyf.download(np.float32, want.shape).view(np.uint32), want.view(np.uint32))
+    for b in (dx, dxf, dyf, *ys): b.free()
+    w.free()
