@@ -286,10 +286,8 @@ extern "C" int dense_gather_mv_multi(ornith_ctx* ctx, const void* const* d_ws, i
   return launch_dense<true>(ctx, s, d_x, K, E, x_rows, d_lhs, d_rhs, rows);
 }
 
-extern "C" {
-
-int ornith_linear_matmul(ornith_ctx* ctx, const ornith_linear* w, const void* d_x, int M,
-                         void* d_y) {
+// `wide`: prompt widths, matrix-core GEMMs where the shapes allow; otherwise every row as if alone.
+static int linear_matmul(ornith_ctx* ctx, const ornith_linear* w, const void* d_x, int M, void* d_y, bool wide) {
   ORN_REQUIRE(ctx && w && d_x && d_y, "linear_matmul: null argument");
   ORN_REQUIRE(M >= 1, "linear_matmul: M=%d", M);
   switch (w->mode) {
@@ -297,14 +295,14 @@ int ornith_linear_matmul(ornith_ctx* ctx, const ornith_linear* w, const void* d_
       ORN_REQUIRE(w->km.O == w->O && w->km.K == w->K, "linear_matmul: k-quant dims disagree");
       // kquant::matmul (src/ops/kquant.rs:783-800): rows within the exact window go through
       // the mat-vec (each row as if alone), prefill widths through the matrix cores
-      if (nmm::plain_ok(&w, 1, d_x, M, &d_y)) return nmm::plain(ctx, &w, 1, d_x, M, &d_y);
-      if (M >= kPrefillRows) return ornith_kq_matmul(ctx, &w->km, d_x, M, d_y);
+      if (wide && nmm::plain_ok(&w, 1, d_x, M, &d_y)) return nmm::plain(ctx, &w, 1, d_x, M, &d_y);
+      if (wide) return ornith_kq_matmul(ctx, &w->km, d_x, M, d_y);
       return ornith_kq_qmv(ctx, &w->km, d_x, ORNITH_BF16, M, d_y, ORNITH_BF16);
     case ORNITH_LIN_AFFINE8:
       ORN_REQUIRE(w->d_w && w->d_scales && w->d_biases, "linear_matmul: affine tensor missing");
       ORN_REQUIRE(w->K % 64 == 0 && w->O >= 1 && M <= 65535, "linear_matmul: affine O=%d K=%d",
                   w->O, w->K);
-      if (nmm::plain_ok(&w, 1, d_x, M, &d_y)) return nmm::plain(ctx, &w, 1, d_x, M, &d_y);
+      if (wide && nmm::plain_ok(&w, 1, d_x, M, &d_y)) return nmm::plain(ctx, &w, 1, d_x, M, &d_y);
       if (const int rc = affine_mv_multi(ctx, &w, 1, d_x, M, &d_y, nullptr); rc >= 0) return rc;
       hipLaunchKernelGGL(affine8_qmv_kernel, dim3(w->O, M), dim3(64), 0, ctx->stream,
                          (const uint8_t*)w->d_w, (const bf16_t*)w->d_scales,
@@ -314,7 +312,7 @@ int ornith_linear_matmul(ornith_ctx* ctx, const ornith_linear* w, const void* d_
     case ORNITH_LIN_AFFINE4:
       ORN_REQUIRE(w->d_w && w->d_scales && w->d_biases, "linear_matmul: affine tensor missing");
       ORN_REQUIRE(w->K % 32 == 0 && w->O >= 1 && M <= 65535, "linear_matmul: 4-bit affine O=%d K=%d", w->O, w->K);
-      if (nmm::plain_ok(&w, 1, d_x, M, &d_y)) return nmm::plain(ctx, &w, 1, d_x, M, &d_y);
+      if (wide && nmm::plain_ok(&w, 1, d_x, M, &d_y)) return nmm::plain(ctx, &w, 1, d_x, M, &d_y);
       if (const int rc = affine_mv_multi(ctx, &w, 1, d_x, M, &d_y, nullptr); rc >= 0) return rc;
       hipLaunchKernelGGL(affine4_qmv_kernel<false>, dim3((w->O + 3) / 4, M), dim3(256), 0, ctx->stream,
                          (const uint8_t*)w->d_w, (const bf16_t*)w->d_scales, (const bf16_t*)w->d_biases,
@@ -327,7 +325,7 @@ int ornith_linear_matmul(ornith_ctx* ctx, const ornith_linear* w, const void* d_
       ORN_REQUIRE(w->K % 8 == 0 && w->O >= 1 && M <= 65535, "linear_matmul: dense O=%d K=%d", w->O,
                   w->K);
       // prefill widths (outside the exact window, like the k-quant GEMM): on the matrix cores
-      if (M >= kPrefillRows && launch_dense_mm(ctx, &w, 1, d_x, M, &d_y)) {
+      if (wide && launch_dense_mm(ctx, &w, 1, d_x, M, &d_y)) {
         ORN_LAUNCH_CHECK("dense_mm_kernel");
         return ORNITH_OK;
       }
@@ -344,17 +342,17 @@ int ornith_linear_matmul(ornith_ctx* ctx, const ornith_linear* w, const void* d_
   }
 }
 
-int ornith_linear_matmul_multi(ornith_ctx* ctx, const ornith_linear* const* ws, int n,
-                               const void* d_x, int M, void* const* d_ys) {
+static int linear_matmul_multi(ornith_ctx* ctx, const ornith_linear* const* ws, int n, const void* d_x, int M,
+                               void* const* d_ys, bool wide) {
   ORN_REQUIRE(ctx && ws && d_x && d_ys && n >= 1, "linear_matmul_multi: bad argument");
-  bool fuse = ornith_option_fuse_proj() && n >= 2 && n <= 4 && M < kPrefillRows;
+  bool fuse = ornith_option_fuse_proj() && n >= 2 && n <= 4 && !wide;
   for (int i = 0; i < n; ++i) {
     ORN_REQUIRE(ws[i] && d_ys[i], "linear_matmul_multi: null entry %d", i);
     fuse = fuse && ws[i]->mode == ws[0]->mode && ws[i]->K == ws[0]->K;
     if (ws[i]->mode == ORNITH_LIN_KQUANT) fuse = fuse && ws[i]->km.kind == ws[0]->km.kind;
   }
   // affine matrices share a launch whatever their width in bits
-  if (ornith_option_fuse_proj() && n >= 2 && M < kPrefillRows)
+  if (ornith_option_fuse_proj() && n >= 2 && !wide)
     if (const int rc = affine_mv_multi(ctx, ws, n, d_x, M, d_ys, nullptr); rc >= 0) return rc;
   if (fuse && ws[0]->mode == ORNITH_LIN_KQUANT) {
     const ornith_kmatrix* kms[4];
@@ -374,7 +372,7 @@ int ornith_linear_matmul_multi(ornith_ctx* ctx, const ornith_linear* const* ws, 
   }
   // Prefill widths: the matrices that take the few-row GEMM share a launch of it (all of them, or the
   // ones with few columns of a wider call), the others go on below.
-  if (M >= kPrefillRows && ornith_option_fuse_proj() && n >= 2 && n <= 4) {
+  if (wide && ornith_option_fuse_proj() && n >= 2 && n <= 4) {
     const ornith_linear *few[4], *rest[4];
     void *yf[4], *yr[4];
     int nf = 0, nr = 0;
@@ -385,11 +383,11 @@ int ornith_linear_matmul_multi(ornith_ctx* ctx, const ornith_linear* const* ws, 
     }
     if (nf >= 2 && nmm::plain_ok(few, nf, d_x, M, yf)) {
       const int rc = nmm::plain(ctx, few, nf, d_x, M, yf);
-      return rc || nr == 0 ? rc : ornith_linear_matmul_multi(ctx, rest, nr, d_x, M, yr);
+      return rc || nr == 0 ? rc : linear_matmul_multi(ctx, rest, nr, d_x, M, yr, wide);
     }
   }
   // ... dense matrices of one K likewise
-  if (M >= kPrefillRows && ornith_option_fuse_proj() && n >= 2 && launch_dense_mm(ctx, ws, n, d_x, M, d_ys)) {
+  if (wide && ornith_option_fuse_proj() && n >= 2 && launch_dense_mm(ctx, ws, n, d_x, M, d_ys)) {
     ORN_LAUNCH_CHECK("dense_mm_kernel");
     return ORNITH_OK;
   }
@@ -398,7 +396,7 @@ int ornith_linear_matmul_multi(ornith_ctx* ctx, const ornith_linear* const* ws, 
   // run is narrow (a mixed launch takes 128-row tiles, which wide matrices should not pay for).
   for (int i = 0; i < n;) {
     int j = i + 1;
-    if (M >= kPrefillRows && ornith_option_fuse_proj() && ws[i]->mode == ORNITH_LIN_KQUANT) {
+    if (wide && ornith_option_fuse_proj() && ws[i]->mode == ORNITH_LIN_KQUANT) {
       int cols = ws[i]->O;
       bool mixed = false;
       while (j < n && j - i < 4 && ws[j]->mode == ORNITH_LIN_KQUANT && ws[j]->K == ws[i]->K) {
@@ -418,12 +416,28 @@ int ornith_linear_matmul_multi(ornith_ctx* ctx, const ornith_linear* const* ws, 
       }
       rc = ornith_kq_matmul_multi(ctx, kms, j - i, d_x, M, d_ys + i);
     } else {
-      rc = ornith_linear_matmul(ctx, ws[i], d_x, M, d_ys[i]);
+      rc = linear_matmul(ctx, ws[i], d_x, M, d_ys[i], wide);
     }
     if (rc) return rc;
     i = j;
   }
   return ORNITH_OK;
+}
+
+// The projections of a block whose sums are the exact path's at every width (moe.hip).
+int linear_exact_multi(ornith_ctx* ctx, const ornith_linear* const* ws, int n, const void* d_x, int M, void* const* d_ys) {
+  return linear_matmul_multi(ctx, ws, n, d_x, M, d_ys, false);
+}
+
+extern "C" {
+
+int ornith_linear_matmul(ornith_ctx* ctx, const ornith_linear* w, const void* d_x, int M, void* d_y) {
+  return linear_matmul(ctx, w, d_x, M, d_y, M >= kPrefillRows);
+}
+
+int ornith_linear_matmul_multi(ornith_ctx* ctx, const ornith_linear* const* ws, int n, const void* d_x, int M,
+                               void* const* d_ys) {
+  return linear_matmul_multi(ctx, ws, n, d_x, M, d_ys, M >= kPrefillRows);
 }
 
 int ornith_add_rms_linear_multi(ornith_ctx* ctx, const ornith_linear* const* ws, int n,

@@ -9,8 +9,6 @@
 //
 // Rounding points are the reference's: gates, probabilities, every expert output
 // and every step of the tail are bf16; sums inside a kernel are fp32.
-#include <algorithm>
-
 #include "linear_device.h"
 #include "mm_narrow_host.h"
 #include "moe_device.h"
@@ -21,6 +19,7 @@
 extern "C" int dense_gather_mv_multi(ornith_ctx* ctx, const void* const* d_ws, int n, int E, int O, int K,
                                      const void* d_x, int x_rows, const uint32_t* d_lhs,
                                      const uint32_t* d_rhs, int rows, void* const* d_ys);
+int linear_exact_multi(ornith_ctx* ctx, const ornith_linear* const* ws, int n, const void* d_x, int M, void* const* d_ys);
 // moe_fused.hip
 bool moe_fused_supported(const ornith_moe_weights* w);
 bool moe_fused_router(ornith_ctx* ctx, const ornith_moe_weights* w, const void* d_x, int T,
@@ -425,13 +424,11 @@ static int moe_block_impl(ornith_ctx* ctx, const ornith_moe_weights* w, const vo
     ORN_REQUIRE(!d_inds_out && !d_scores_out, "moe_block: index outputs are a decode-width feature");
     return moe_block_prefill(ctx, w, d_x, T, d_out);
   }
-  // dense experts have no prefill-width form, and the ids and scores are made by the exact path:
-  // the rows go in blocks (they are independent of each other, so the result is the same) of 64,
-  // of affine experts in blocks inside the exact window, so that every projection stays exact
-  const int block = ex_affine4 ? std::min(64, kPrefillRows - 1) : 64;
-  if (T > block) {
-    for (int t0 = 0; t0 < T; t0 += block) {
-      const int n = std::min(block, T - t0);
+  // dense experts have no prefill-width form, and the ids and scores are made by the exact path: the
+  // rows go in blocks of 64 (they are independent of each other, so the result is the same)
+  if (T > 64) {
+    for (int t0 = 0; t0 < T; t0 += 64) {
+      const int n = T - t0 < 64 ? T - t0 : 64;
       const int rcb = moe_block_impl(ctx, w, static_cast<const bf16_t*>(d_x) + (size_t)t0 * H, n,
                                      static_cast<bf16_t*>(d_out) + (size_t)t0 * H,
                                      d_inds_out ? d_inds_out + (size_t)t0 * k : nullptr,
@@ -469,6 +466,10 @@ static int moe_block_impl(ornith_ctx* ctx, const ornith_moe_weights* w, const vo
     rc = (e);           \
     if (rc) return rc;  \
   } while (0)
+  // what is over affine experts here is exact, whatever the width from which other calls run as GEMMs
+  auto linears = [&](const ornith_linear* const* ws, int n, const void* x, void* const* ys) {
+    return ex_affine4 ? linear_exact_multi(ctx, ws, n, x, T, ys) : ornith_linear_matmul_multi(ctx, ws, n, x, T, ys);
+  };
   if (ornith_option_fuse_moe() && moe_fused_supported(w)) {
     int rrc = ORNITH_OK;
     // router, up and down as one launch where the shapes are in its family
@@ -501,7 +502,7 @@ static int moe_block_impl(ornith_ctx* ctx, const ornith_moe_weights* w, const vo
     if (pre)  // (falls back to the separate norm where the launch does not cover the shapes)
       TRY(ornith_add_rms_linear_multi(ctx, in2, 2, pre->res, pre->y, pre->w, pre->eps, T, pre->h_out, pre->normed_out, out2));
     else
-      TRY(ornith_linear_matmul_multi(ctx, in2, 2, d_x, T, out2));
+      TRY(linears(in2, 2, d_x, out2));
     const bool topk_in_up = E % 64 == 0 && E <= 1024 && ((E / 64) & (E / 64 - 1)) == 0 && k <= 16;
     if (!topk_in_up) TRY(launch_router(ctx, gates, T, E, k, inds, scores, nullptr, nullptr, nullptr));
     if (pair_a4)
@@ -514,7 +515,7 @@ static int moe_block_impl(ornith_ctx* ctx, const ornith_moe_weights* w, const vo
     // the four projections of the block's input: one launch when their formats allow
     const ornith_linear* in4[4] = {&w->router, &w->sh_gate, &w->sh_up, &w->sh_egate};
     void* out4[4] = {gates, sg, su, eg};
-    TRY(ornith_linear_matmul_multi(ctx, in4, 4, d_x, T, out4));
+    TRY(linears(in4, 4, d_x, out4));
   }
   TRY(launch_router(ctx, gates, T, E, k, inds, scores, nullptr, lhs_tok, lhs_row));
   if (w->ex_dense) {
@@ -533,7 +534,9 @@ static int moe_block_impl(ornith_ctx* ctx, const ornith_moe_weights* w, const vo
     TRY(ornith_affine4_gather_qmv(ctx, w->ex_up.d_qs, w->ex_up.d_scales, w->ex_up.d_dm, E, I, H, d_x, T, lhs_tok,
                                   inds, T * k, xu));
     TRY(swiglu_pair(ctx, sg, su, (int64_t)T * SI, sact, xg, xu, (int64_t)T * k * I, act));
-    TRY(ornith_linear_matmul(ctx, &w->sh_down, sact, T, sy));
+    const ornith_linear* const shd = &w->sh_down;
+    void* const shy = sy;
+    TRY(linears(&shd, 1, sact, &shy));
     TRY(ornith_affine4_gather_qmv(ctx, w->ex_down.d_qs, w->ex_down.d_scales, w->ex_down.d_dm, E, H, I, act, T * k,
                                   lhs_row, inds, T * k, y));
   } else {
