@@ -267,7 +267,10 @@ typedef struct ornith_moe_weights {
 } ornith_moe_weights;
 
 /* moe::sparse_moe_block (src/ops/moe.rs:662-741): x bf16 [T,H] -> out bf16 [T,H].
- * d_inds_out (u32 [T,k]) and d_scores_out (bf16 [T,k]) may be null. T <= 64. */
+ * d_inds_out (u32 [T,k]) and d_scores_out (bf16 [T,k]) may be null; asking for them does not
+ * change the result. T <= 8192. Over k-quant experts, calls of "gemm_rows" rows and more run as
+ * matrix-core GEMMs and give no ids or scores (ORNITH_ERR_INVALID); over 4-bit affine and dense
+ * experts the expert sums are the exact path's at every width (blocks of 64 rows). */
 ORNITH_API int ornith_moe_block(ornith_ctx* ctx, const ornith_moe_weights* w, const void* d_x, int T,
                                 void* d_out, uint32_t* d_inds_out, void* d_scores_out);
 
@@ -275,7 +278,9 @@ ORNITH_API int ornith_moe_block(ornith_ctx* ctx, const ornith_moe_weights* w, co
  * the MLP of a decoder layer, src/model/qwen3_5.rs:384-392): h = res + y, normed =
  * rms_norm(h, w_norm), out = moe(normed). With the fused expert kernels, hidden size 2048 and
  * T <= 4 the norm is made inside the router's launch; otherwise add_rms_norm is issued first.
- * Bit-identical either way. */
+ * Bit-identical either way. This is the form a prompt takes through a layer, so from "gemm_rows"
+ * rows on blocks over 4-bit affine experts run as GEMMs here as well: the same arithmetic as
+ * ornith_moe_block's with its fp32 sums in another order (a router tie may fall the other way). */
 ORNITH_API int ornith_add_rms_moe_block(ornith_ctx* ctx, const ornith_moe_weights* w, const void* d_res,
                                         const void* d_y, const void* d_wnorm, float eps, int T,
                                         void* d_h_out, void* d_normed_out, void* d_out);

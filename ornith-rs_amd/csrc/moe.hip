@@ -222,7 +222,7 @@ int launch_router_egate(ornith_ctx* ctx, const bf16_t* gates, int T, int E, int 
   return ORNITH_OK;
 }
 
-// Prompts of few rows an expert (and any prompt over affine experts, which have no wide form): the
+// Prompts of few rows an expert (and a layer's prompt over affine experts, which have no wide form): the
 // shared expert is one more expert of the pair list, so the block is six launches: router, its
 // tail (shared gate, softmax + top-k), plan, gate + up + swiglu, down, combine.
 // false: the shapes are not covered.
@@ -384,8 +384,11 @@ int ornith_moe_combine(ornith_ctx* ctx, const void* d_scores, const void* d_y, c
 // The block. With `pre`, x is rms_norm(pre->res + pre->y): made inside the router launch when
 // the fused kernels cover the shapes (d_x then is where the normed rows get stored, and read
 // back by the expert kernels), by a separate add_rms_norm otherwise.
+// `gemm_affine`: a prompt's rows may run as GEMMs over affine experts too. It belongs to the entry
+// point, not to the outputs asked for: ornith_moe_block, which gives ids and scores on demand, keeps
+// these experts exact at every width, so that asking does not change the result.
 static int moe_block_impl(ornith_ctx* ctx, const ornith_moe_weights* w, const void* d_x, int T,
-                          void* d_out, uint32_t* d_inds_out, void* d_scores_out, const PreNorm* pre) {
+                          void* d_out, uint32_t* d_inds_out, void* d_scores_out, const PreNorm* pre, bool gemm_affine) {
   ORN_REQUIRE(ctx && w && d_x && d_out, "moe_block: null argument");
   const int E = w->router.O, H = w->router.K, I = w->ex_gate.O, k = w->top_k;
   ORN_REQUIRE(T >= 1 && T <= 8192, "moe_block: T=%d", T);
@@ -416,7 +419,7 @@ static int moe_block_impl(ornith_ctx* ctx, const ornith_moe_weights* w, const vo
   if (ex_affine4)
     ORN_REQUIRE(w->ex_up.kind == ORNITH_AFFINE4_G32 && w->ex_down.kind == ORNITH_AFFINE4_G32,
                 "moe_block: the three expert stacks must share the 4-bit affine format");
-  if (T >= kPrefillRows && !w->ex_dense && !d_inds_out && !d_scores_out) {
+  if (T >= kPrefillRows && !w->ex_dense && (ex_affine4 ? gemm_affine : !d_inds_out && !d_scores_out)) {
     int rcn = ORNITH_OK;
     if (moe_block_narrow(ctx, w, d_x, T, d_out, &rcn)) return rcn;
   }
@@ -424,15 +427,15 @@ static int moe_block_impl(ornith_ctx* ctx, const ornith_moe_weights* w, const vo
     ORN_REQUIRE(!d_inds_out && !d_scores_out, "moe_block: index outputs are a decode-width feature");
     return moe_block_prefill(ctx, w, d_x, T, d_out);
   }
-  // dense experts have no prefill-width form, and the ids and scores are made by the exact path: the
-  // rows go in blocks of 64 (they are independent of each other, so the result is the same)
+  // dense experts have no prefill-width form, affine ones none that is exact: the rows go in blocks
+  // of 64 (they are independent of each other, so the result is the same)
   if (T > 64) {
     for (int t0 = 0; t0 < T; t0 += 64) {
       const int n = T - t0 < 64 ? T - t0 : 64;
       const int rcb = moe_block_impl(ctx, w, static_cast<const bf16_t*>(d_x) + (size_t)t0 * H, n,
                                      static_cast<bf16_t*>(d_out) + (size_t)t0 * H,
                                      d_inds_out ? d_inds_out + (size_t)t0 * k : nullptr,
-                                     d_scores_out ? static_cast<bf16_t*>(d_scores_out) + (size_t)t0 * k : nullptr, nullptr);
+                                     d_scores_out ? static_cast<bf16_t*>(d_scores_out) + (size_t)t0 * k : nullptr, nullptr, false);
       if (rcb) return rcb;
     }
     return ORNITH_OK;
@@ -556,7 +559,7 @@ static int moe_block_impl(ornith_ctx* ctx, const ornith_moe_weights* w, const vo
 
 int ornith_moe_block(ornith_ctx* ctx, const ornith_moe_weights* w, const void* d_x, int T,
                      void* d_out, uint32_t* d_inds_out, void* d_scores_out) {
-  return moe_block_impl(ctx, w, d_x, T, d_out, d_inds_out, d_scores_out, nullptr);
+  return moe_block_impl(ctx, w, d_x, T, d_out, d_inds_out, d_scores_out, nullptr, false);
 }
 
 int ornith_add_rms_moe_block(ornith_ctx* ctx, const ornith_moe_weights* w, const void* d_res,
@@ -565,7 +568,7 @@ int ornith_add_rms_moe_block(ornith_ctx* ctx, const ornith_moe_weights* w, const
   ORN_REQUIRE(d_res && d_y && d_wnorm && d_h_out && d_normed_out, "add_rms_moe_block: null argument");
   const PreNorm pre{(const bf16_t*)d_res, (const bf16_t*)d_y, (const bf16_t*)d_wnorm, (bf16_t*)d_h_out,
                     (bf16_t*)d_normed_out, eps};
-  return moe_block_impl(ctx, w, d_normed_out, T, d_out, nullptr, nullptr, &pre);
+  return moe_block_impl(ctx, w, d_normed_out, T, d_out, nullptr, nullptr, &pre, true);
 }
 
 }  // extern "C"

@@ -132,7 +132,7 @@ def test_model_in_the_published_artifacts_format_matches_oracle(orn, ctx):
 @pytest.mark.parametrize("gemm_rows,T", [(32, 32), (32, 100), (1, 1), (1, 3), (2, 70), (5, 9)])
 def test_affine_block_with_index_outputs_at_every_gemm_rows(orn, ctx, gemm_rows, T):
     """Ids, scores and output of a block over affine experts are the oracle's bits at every setting of gemm_rows,
-    from one row on (70 and 100 rows: two blocks)."""
+    from one row on (70 and 100 rows: two blocks), and not asking for the ids changes nothing."""
     rng = np.random.default_rng(60 + T)
     moe = util.HostMoe(rng, H=512, E=64, I=512, top_k=8, gate_kind=util.AFFINE4)
     xb = util.bf16_normal(rng, (T, 512))
@@ -144,7 +144,7 @@ def test_affine_block_with_index_outputs_at_every_gemm_rows(orn, ctx, gemm_rows,
         orn.set_option("gemm_rows", gemm_rows)
         for fuse in (1, 0):
             orn.set_option("fuse_moe", fuse)
-            for outs in ((inds, scores), (inds, None), (None, scores)):
+            for outs in ((inds, scores), (None, None), (inds, None), (None, scores)):
                 for b in (out, inds, scores): b.zero()
                 ctx.moe_block(w, dx, T, out, *outs)
                 assert np.array_equal(out.download(np.uint16, (T, 512)), want), (fuse, outs)

@@ -50,7 +50,8 @@ def test_few_row_matmul_vs_float64(orn, ctx, fmt, O, K, M):
 def test_few_row_moe_block_vs_exact(orn, ctx, fmt, T):
     """16-, 32- and 64-row expert tiles (4 to 38 rows an expert on average), the shared expert among
     them. A router tie may fall the other way than in the oracle's exact block: such a row differs by an
-    expert, so the bound is on the rows' median and 93 % of them."""
+    expert, so the bound is on the rows' median and 93 % of them. (The operator keeps affine experts exact;
+    their GEMMs are a layer's, below.)"""
     rng = np.random.default_rng(T)
     moe = util.HostMoe(rng, H=1024, E=64, I=512, top_k=8, gate_kind=util.AFFINE4 if fmt == "affine4" else Q4K)
     xb = util.bf16_normal(rng, (T, 1024))
@@ -68,4 +69,36 @@ def test_few_row_moe_block_vs_exact(orn, ctx, fmt, T):
     bound = 0.004 if fmt == "affine4" else 0.01
     assert np.median(rel) < bound and (rel < 0.03).mean() >= 0.93, (float(np.median(rel)), float(np.sort(rel)[-5]))
     for b in (dx, out): b.free()
+    moe.free()
+
+
+@pytest.mark.parametrize("T", [32, 100, 150, 300])
+def test_few_row_moe_block_of_a_layer_over_affine_experts(orn, ctx, T):
+    """ornith_add_rms_moe_block from gemm_rows rows on: the affine experts as GEMMs behind the layer's norm,
+    against the oracle's exact block on the normed rows, with the bound of the test above; with GEMMs
+    switched off its bits."""
+    rng = np.random.default_rng(T)
+    H = 1024
+    moe = util.HostMoe(rng, H=H, E=64, I=512, top_k=8, gate_kind=util.AFFINE4)
+    res, y, wn = (util.bf16_normal(rng, s) for s in ((T, H), (T, H), (H,)))
+    wh, wnormed = util.orc_add_rms_norm(res, y, wn)
+    want16 = util.orc_moe_block(moe, wnormed, T)[0]
+    want = util.bf16_to_f32(want16).astype(np.float64)
+    w = moe.dev(orn, ctx)
+    bufs = [ctx.to_device(a) for a in (res, y, wn)] + [ctx.alloc(T * H * 2) for _ in range(3)]
+    dres, dy, dwn, dh, dn, out = bufs
+    try:
+        got = {}
+        for rows in (32, 0):
+            orn.set_option("gemm_rows", rows)
+            ctx.memset(out, 0xFF, T * H * 2)
+            orn.add_rms_moe_block(ctx, w, dres, dy, dwn, 1e-6, T, dh, dn, out)
+            assert np.array_equal(dh.download(np.uint16, (T, H)), wh) and np.array_equal(dn.download(np.uint16, (T, H)), wnormed)
+            got[rows] = out.download(np.uint16, (T, H))
+    finally:
+        orn.set_option("gemm_rows", 32)
+    assert np.array_equal(got[0], want16) and not np.array_equal(got[32], want16)
+    rel = np.linalg.norm(util.bf16_to_f32(got[32]).astype(np.float64) - want, axis=1) / np.linalg.norm(want, axis=1)
+    assert np.median(rel) < 0.004 and (rel < 0.03).mean() >= 0.93, (float(np.median(rel)), float(np.sort(rel)[-5]))
+    for b in bufs: b.free()
     moe.free()
