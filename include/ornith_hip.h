@@ -136,7 +136,7 @@ ORNITH_API int ornith_kq_dequantize(ornith_ctx* ctx, const ornith_kmatrix* w, vo
 
 /* kquant::qmv (src/ops/kquant.rs:539-595): y[M,O] = x[M,K] . W^T, fp32
  * accumulate, each row computed exactly as it would be alone. M <= 4 is the
- * decode/verify shape; larger M loops in groups of four. */
+ * decode/verify shape; larger M goes in groups of up to four, in one launch. x 16-byte aligned. */
 ORNITH_API int ornith_kq_qmv(ornith_ctx* ctx, const ornith_kmatrix* w, const void* d_x, int x_dtype, int M,
                   void* d_y, int y_dtype);
 

@@ -472,7 +472,7 @@ int ornith_kq_qmv_multi(ornith_ctx* ctx, const ornith_kmatrix* const* ws, int n,
                         int x_dtype, int M, void* const* d_ys, int y_dtype) {
   ORN_REQUIRE(ctx && ws && d_x && d_ys, "kq_qmv: null argument");
   ORN_REQUIRE(n >= 1 && n <= kMaxSeg, "kq_qmv: %d matrices in one launch (1..%d)", n, kMaxSeg);
-  ORN_REQUIRE(M >= 1 && M <= 4 * 65535, "kq_qmv: M=%d", M);
+  ORN_REQUIRE(M >= 1, "kq_qmv: M=%d", M);
   ORN_REQUIRE(((uintptr_t)d_x & 15) == 0, "kq_qmv: x must be 16-byte aligned");
   for (int s = 0; s < n; ++s) {
     int rc = check_matrix(ws[s], "kq_qmv");
@@ -483,22 +483,33 @@ int ornith_kq_qmv_multi(ornith_ctx* ctx, const ornith_kmatrix* const* ws, int n,
     ORN_REQUIRE(d_ys[s], "kq_qmv: null output");
   }
   const int kind = ws[0]->kind, K = ws[0]->K;
+  const size_t xs = ornith_dtype_size(x_dtype), ys = ornith_dtype_size(y_dtype);
   KqArgs a{};
   a.nseg = n;
   a.K = K;
   a.y_bf16 = y_dtype == ORNITH_BF16;
   a.iters = pick_iters();
-  a.x = d_x;
-  for (int s = 0; s < n; ++s) {
-    a.seg[s].qs = (const uint8_t*)ws[s]->d_qs;
-    a.seg[s].scales = (const uint8_t*)ws[s]->d_scales;
-    a.seg[s].dm = (const uint16_t*)ws[s]->d_dm;
-    a.seg[s].O = ws[s]->O;
-    a.seg[s].y = d_ys[s];
+  // one launch for as many rows as its second grid dimension can number in groups of two (launch_m)
+  constexpr int kLaunchRows = 2 * 65535;
+  for (int m0 = 0; m0 < M; m0 += kLaunchRows) {
+    const int mw = M - m0 < kLaunchRows ? M - m0 : kLaunchRows;
+    a.x = (const char*)d_x + (size_t)m0 * K * xs;
+    for (int s = 0; s < n; ++s) {
+      a.seg[s].qs = (const uint8_t*)ws[s]->d_qs;
+      a.seg[s].scales = (const uint8_t*)ws[s]->d_scales;
+      a.seg[s].dm = (const uint16_t*)ws[s]->d_dm;
+      a.seg[s].O = ws[s]->O;
+      a.seg[s].y = (char*)d_ys[s] + (size_t)m0 * ws[s]->O * ys;
+    }
+    int rc;
+    if (kind == ORNITH_Q4K)
+      rc = x_dtype == ORNITH_F32 ? launch_m<ORNITH_Q4K, true>(ctx, a, mw) : launch_m<ORNITH_Q4K, false>(ctx, a, mw);
+    else
+      rc = x_dtype == ORNITH_F32 ? launch_m<ORNITH_Q6K, true>(ctx, a, mw) : launch_m<ORNITH_Q6K, false>(ctx, a, mw);
+    if (rc) return rc;
+    if (M - m0 <= kLaunchRows) break;
   }
-  if (kind == ORNITH_Q4K)
-    return x_dtype == ORNITH_F32 ? launch_m<ORNITH_Q4K, true>(ctx, a, M) : launch_m<ORNITH_Q4K, false>(ctx, a, M);
-  return x_dtype == ORNITH_F32 ? launch_m<ORNITH_Q6K, true>(ctx, a, M) : launch_m<ORNITH_Q6K, false>(ctx, a, M);
+  return ORNITH_OK;
 }
 
 int ornith_kq_qmv(ornith_ctx* ctx, const ornith_kmatrix* w, const void* d_x, int x_dtype, int M,

@@ -258,3 +258,20 @@ def test_qmv_large_launches_bit_exact(orn, ctx, kind, K, Os, M):
     assert np.array_equal(dyf.download(np.float32, want.shape).view(np.uint32), want.view(np.uint32))
     for b in (dx, dxf, dyf, *ys): b.free()
     w.free()
+
+
+@pytest.mark.parametrize("kind", [Q4K, Q6K])
+def test_qmv_of_more_rows_than_a_launch_holds(orn, ctx, kind):
+    """262141 activation rows: one more than 65535 groups of four (and more than 65535 of two, Q6_K's), by bits."""
+    rng = np.random.default_rng(5)
+    K, O, M, P = 256, 4, 4 * 65535 + 1, 1021
+    t = util.make_kq(kind, rng, 1, O, K)
+    w = _dev_matrix(orn, ctx, kind, t, 1, O, K)
+    xb = np.tile(util.bf16_normal(rng, (P, K)), (M // P + 1, 1))[:M]
+    dx, dy = ctx.to_device(xb), ctx.alloc(M * O * 2)
+    ctx.memset(dy, 0xFF, M * O * 2)
+    ctx.kq_qmv(w, dx, orn.BF16, M, dy, orn.BF16)
+    want = util.f32_to_bf16(util.orc_qmv(kind, *t, O, K, util.bf16_to_f32(xb[:P])))
+    assert np.array_equal(dy.download(np.uint16, (M, O)), np.tile(want, (M // P + 1, 1))[:M])
+    for b in (dx, dy): b.free()
+    w.free()
