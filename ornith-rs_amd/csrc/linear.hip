@@ -445,7 +445,8 @@ int ornith_add_rms_linear_multi(ornith_ctx* ctx, const ornith_linear* const* ws,
                                 void* d_h_out, void* d_normed_out, void* const* d_ys) {
   ORN_REQUIRE(ctx && ws && d_res && d_y && d_wnorm && d_h_out && d_normed_out && d_ys && n >= 1,
               "add_rms_linear_multi: bad argument");
-  bool fuse = ornith_option_fuse_norm() && n <= 4 && M <= 4;
+  // (a call that runs as a GEMM has its norm in front)
+  bool fuse = ornith_option_fuse_norm() && n <= 4 && M <= 4 && M < kPrefillRows;
   const ornith_kmatrix* kms[4];
   for (int i = 0; i < n && fuse; ++i) {
     fuse = ws[i] && ws[i]->mode == ORNITH_LIN_KQUANT && ws[i]->K == 2048;

@@ -294,3 +294,44 @@ def test_expert_kernels_under_overlapping_routing(orn, ctx, H, E, I, gk, dk):
             assert np.array_equal(got_out, want_out)
     finally:
         moe.free()
+
+
+@pytest.mark.parametrize("fmt", ["kq", "affine4"])
+@pytest.mark.parametrize("gemm_rows,T", [(1, 1), (2, 3), (4, 4), (3, 2)])
+def test_norm_in_a_head_keeps_to_gemm_rows(orn, ctx, fmt, gemm_rows, T):
+    """With gemm_rows at four or below the calls that would take the norm in their head run as GEMMs instead:
+    the norm is a launch of its own then, and projections and block are those of add_rms_norm followed by
+    the operators (ornith_moe_block for k-quants; affine experts have GEMMs in the layer's form only)."""
+    rng = np.random.default_rng(10 * gemm_rows + T)
+    H, Os = 2048, (96, 520)
+    aff = fmt == "affine4"
+    moe = util.HostMoe(rng, H=H, E=64, I=512, top_k=8, gate_kind=util.AFFINE4 if aff else Q4K)
+    dw = moe.dev(orn, ctx)
+    lins = [(util.HostLinear.affine4(rng, O, H) if aff else util.HostLinear.kq(rng, Q4K, O, H)).dev(orn, ctx) for O in Os]
+    res, y = ctx.to_device(util.bf16_normal(rng, (T, H))), ctx.to_device(util.bf16_normal(rng, (T, H)))
+    wn = ctx.to_device(util.bf16_normal(rng, (H,)))
+    h1, n1, o1, h2, n2, o2 = (ctx.alloc(T * H * 2) for _ in range(6))
+    ys1, ys2 = ([ctx.alloc(T * O * 2) for O in Os] for _ in range(2))
+
+    def get(bufs):
+        return [b.download(np.uint16, (T, w)) for b, w in bufs]
+
+    try:
+        orn.set_option("gemm_rows", gemm_rows)
+        for b in (h1, n1, o1, h2, n2, o2, *ys1, *ys2): b.zero()
+        ctx.add_rms_norm(res, y, wn, T, H, 1e-6, h2, n2)
+        ctx.linear_matmul_multi(lins, n2, T, ys2)
+        orn.add_rms_linear_multi(ctx, lins, res, y, wn, 1e-6, T, h1, n1, ys1)
+        pairs = [(h1, H), (n1, H)] + list(zip(ys1, Os)), [(h2, H), (n2, H)] + list(zip(ys2, Os))
+        for a, b in zip(get(pairs[0]), get(pairs[1])): assert np.array_equal(a, b)
+        for b in (h1, n1): b.zero()
+        orn.add_rms_moe_block(ctx, dw, res, y, wn, 1e-6, T, h1, n1, o1)
+        for a, b in zip(get([(h1, H), (n1, H)]), get([(h2, H), (n2, H)])): assert np.array_equal(a, b)
+        if not aff:
+            ctx.moe_block(dw, n2, T, o2)
+            assert np.array_equal(*get([(o1, H), (o2, H)]))
+    finally:
+        orn.set_option("gemm_rows", 32)
+        for b in (res, y, wn, h1, n1, o1, h2, n2, o2, *ys1, *ys2): b.free()
+        for l in lins: l.free()
+        moe.free()
