@@ -187,6 +187,9 @@ int affine_mv_multi(ornith_ctx* ctx, const ornith_linear* const* ws, int n, cons
   const int K = ws[0]->K;
   if (K != 1024 && K != 2048 && K != 4096) return -1;
   if (pre && (M > 4 || K != kPreN)) return -1;
+  // (the norm's own launch, which takes the call then, refuses operands that are not 16-byte aligned)
+  if (pre && (((uintptr_t)pre->res | (uintptr_t)pre->y | (uintptr_t)pre->w | (uintptr_t)pre->h_out | (uintptr_t)pre->normed_out) & 15) != 0)
+    return -1;
   if (!pre && ((uintptr_t)d_x & 15) != 0) return -1;
   AffArgs a{};
   a.nseg = n;

@@ -155,3 +155,32 @@ def test_affine_block_with_index_outputs_at_every_gemm_rows(orn, ctx, gemm_rows,
         orn.set_option("fuse_moe", 1)
         for b in (dx, out, inds, scores): b.free()
         moe.free()
+
+
+def test_misaligned_norm_operands_are_refused(orn, ctx):
+    """Rows off a 16-byte boundary: an error from the host, with the norm in the head of the launch as with the
+    norm in front, for the projections and for the block."""
+    rng = np.random.default_rng(8)
+    H, T = 2048, 2
+    lin = util.HostLinear.affine4(rng, 40, H).dev(orn, ctx)
+    moe = util.HostMoe(rng, H=H, E=64, I=512, top_k=8, gate_kind=util.AFFINE4)
+    w = moe.dev(orn, ctx)
+    bufs = [ctx.alloc(T * H * 2 + 256) for _ in range(7)]
+    for b in bufs: b.zero()
+
+    class Off:
+        def __init__(self, b): self.ptr = type(b.ptr)(b.ptr.value + 2)
+
+    try:
+        for fuse in (1, 0):
+            orn.set_option("fuse_norm", fuse)
+            for i in range(5):
+                res, y, wn, h, nm = (Off(b) if j == i else b for j, b in enumerate(bufs[:5]))
+                with pytest.raises(orn.OrnithError, match="aligned"):
+                    orn.add_rms_linear_multi(ctx, [lin], res, y, wn, 1e-6, T, h, nm, [bufs[5]])
+                with pytest.raises(orn.OrnithError, match="aligned"):
+                    orn.add_rms_moe_block(ctx, w, res, y, wn, 1e-6, T, h, nm, bufs[6])
+    finally:
+        orn.set_option("fuse_norm", 1)
+        for b in bufs: b.free()
+        lin.free(); moe.free()
