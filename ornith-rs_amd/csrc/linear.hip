@@ -445,22 +445,23 @@ int ornith_add_rms_linear_multi(ornith_ctx* ctx, const ornith_linear* const* ws,
                                 void* d_h_out, void* d_normed_out, void* const* d_ys) {
   ORN_REQUIRE(ctx && ws && d_res && d_y && d_wnorm && d_h_out && d_normed_out && d_ys && n >= 1,
               "add_rms_linear_multi: bad argument");
-  // (a call that runs as a GEMM has its norm in front)
-  bool fuse = ornith_option_fuse_norm() && n <= 4 && M <= 4 && M < kPrefillRows;
-  const ornith_kmatrix* kms[4];
-  for (int i = 0; i < n && fuse; ++i) {
-    fuse = ws[i] && ws[i]->mode == ORNITH_LIN_KQUANT && ws[i]->K == 2048;
-    if (fuse) kms[i] = &ws[i]->km;
-  }
-  if (fuse) {
-    const int rc = kq_qmv_multi_prenorm(ctx, kms, n, d_res, d_y, d_wnorm, eps, M, d_h_out, d_normed_out, d_ys);
-    if (rc >= 0) return rc;
-  }
-  if (ornith_option_fuse_norm() && n <= 4 && M <= 4 && M < kPrefillRows) {
+  for (int i = 0; i < n; ++i) ORN_REQUIRE(ws[i] && d_ys[i], "add_rms_linear_multi: null entry %d", i);
+  // the norm in the head of the projections' launch (a call that runs as a GEMM has it in front)
+  bool head = ornith_option_fuse_norm() && n <= 4 && M >= 1 && M <= 4 && M < kPrefillRows;
+  for (int i = 0; i < n; ++i) head = head && ws[i]->K == kPreN;
+  if (head) {
     const PreNorm pre{(const bf16_t*)d_res, (const bf16_t*)d_y, (const bf16_t*)d_wnorm, (bf16_t*)d_h_out, (bf16_t*)d_normed_out, eps};
-    bool all = true;
-    for (int i = 0; i < n; ++i) all = all && ws[i];
-    const int rc = all ? affine_mv_multi(ctx, ws, n, nullptr, M, d_ys, &pre) : -1;
+    head = prenorm_apart(pre, M);
+    bool kq = true;
+    const ornith_kmatrix* kms[4];
+    for (int i = 0; i < n; ++i) {
+      head = head && prenorm_apart(pre, M, d_ys[i], (size_t)M * ws[i]->O * 2);
+      kq = kq && ws[i]->mode == ORNITH_LIN_KQUANT;
+      kms[i] = &ws[i]->km;
+    }
+    int rc = -1;
+    if (head) rc = kq ? kq_qmv_multi_prenorm(ctx, kms, n, d_res, d_y, d_wnorm, eps, M, d_h_out, d_normed_out, d_ys)
+                      : affine_mv_multi(ctx, ws, n, nullptr, M, d_ys, &pre);
     if (rc >= 0) return rc;
   }
   int rc = ornith_add_rms_norm(ctx, d_res, d_y, d_wnorm, M, ws[0]->K, eps, d_h_out, d_normed_out);

@@ -404,7 +404,7 @@ static int moe_block_impl(ornith_ctx* ctx, const ornith_moe_weights* w, const vo
                   w->sh_egate.O == 1,
               "moe_block: shared expert shapes do not chain");
   const int SI = w->sh_gate.O;
-  const bool pre_in_kernel = pre && T <= 4 && T < kPrefillRows && H == kPreN && ornith_option_fuse_norm() &&
+  const bool pre_in_kernel = pre && T <= 4 && T < kPrefillRows && H == kPreN && prenorm_apart(*pre, T) && ornith_option_fuse_norm() &&
                              ornith_option_fuse_moe() && moe_fused_supported(w) &&
                              w->router.mode == ORNITH_LIN_KQUANT;
   // (an affine block's router and shared-expert gate take it in the head of their launch, below)

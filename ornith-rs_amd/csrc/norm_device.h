@@ -116,6 +116,24 @@ struct PreNorm {
 
 constexpr int kPreN = 2048;
 
+// Host: whether n1 bytes at a and n2 bytes at b have one in common.
+static inline bool ranges_meet(const void* a, size_t n1, const void* b, size_t n2) {
+  const uintptr_t x = (uintptr_t)a, y = (uintptr_t)b;
+  return x < y + n2 && y < x + n1;
+}
+// Host: whether `bytes` at `out` lie apart from what the norm is made from. One workgroup of a launch
+// with the norm in its head stores h and the normed rows, and all of them their outputs, while others
+// still read these, so only outputs that lie apart may be written there; a norm in a launch of its own,
+// which has read a row before it writes one, works in place.
+static inline bool prenorm_apart(const PreNorm& p, int rows, const void* out, size_t bytes) {
+  const size_t n = (size_t)rows * kPreN * 2;
+  return !ranges_meet(out, bytes, p.res, n) && !ranges_meet(out, bytes, p.y, n) && !ranges_meet(out, bytes, p.w, (size_t)kPreN * 2);
+}
+static inline bool prenorm_apart(const PreNorm& p, int rows) {
+  const size_t n = (size_t)rows * kPreN * 2;
+  return prenorm_apart(p, rows, p.h_out, n) && prenorm_apart(p, rows, p.normed_out, n);
+}
+
 template <int T>
 struct PreNormLds {
   __attribute__((aligned(16))) bf16_t xn[T][kPreN];

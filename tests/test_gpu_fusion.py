@@ -335,3 +335,39 @@ def test_norm_in_a_head_keeps_to_gemm_rows(orn, ctx, fmt, gemm_rows, T):
         for b in (res, y, wn, h1, n1, o1, h2, n2, o2, *ys1, *ys2): b.free()
         for l in lins: l.free()
         moe.free()
+
+
+@pytest.mark.parametrize("fmt", ["q4k", "q6k", "affine4"])
+@pytest.mark.parametrize("T", [1, 2, 4])
+def test_norm_and_its_consumers_in_place(orn, ctx, fmt, T):
+    """h over the residual, the normed rows over the branch's output, and a projection over the branch's output:
+    the bits of the same call on buffers of their own (such calls have the norm in a launch of its own; with
+    the norm in a head one workgroup would store over what others still read)."""
+    rng = np.random.default_rng(90 + T)
+    H, Os = 2048, (2048, 40)
+    aff = fmt == "affine4"
+    kind = Q6K if fmt == "q6k" else Q4K
+    moe = util.HostMoe(rng, H=H, E=64, I=512, top_k=8, gate_kind=util.AFFINE4 if aff else kind)
+    dw = moe.dev(orn, ctx)
+    lins = [(util.HostLinear.affine4(rng, O, H) if aff else util.HostLinear.kq(rng, kind, O, H)).dev(orn, ctx) for O in Os]
+    rb, yb = util.bf16_normal(rng, (T, H)), util.bf16_normal(rng, (T, H))
+    wn = ctx.to_device(util.bf16_normal(rng, (H,)))
+    res, y, h, nm, out, y1 = bufs = [ctx.alloc(T * H * 2) for _ in range(6)]
+
+    def call(block, h, nm, y0):
+        res.upload(rb); y.upload(yb)
+        if block:
+            orn.add_rms_moe_block(ctx, dw, res, y, wn, 1e-6, T, h, nm, y0)
+        else:
+            orn.add_rms_linear_multi(ctx, lins, res, y, wn, 1e-6, T, h, nm, [y0, y1])
+        return [b.download(np.uint16, (T, H)) for b in (h, nm, y0)] + ([] if block else [y1.download(np.uint16, (T, Os[1]))])
+
+    for block in (False, True):
+        want = call(block, h, nm, out)
+        assert np.array_equal(want[1], util.orc_add_rms_norm(rb, yb, wn.download(np.uint16, (H,)))[1])
+        for args in ((res, nm, out), (h, y, out), (res, y, out), (h, nm, y), (h, nm, res)):
+            got = call(block, *args)
+            for i, (a, b) in enumerate(zip(got, want)): assert np.array_equal(a, b), (block, i)
+    for b in bufs + [wn]: b.free()
+    for l in lins: l.free()
+    moe.free()
