@@ -184,3 +184,109 @@ def test_misaligned_norm_operands_are_refused(orn, ctx):
         orn.set_option("fuse_norm", 1)
         for b in bufs: b.free()
         lin.free(); moe.free()
+
+
+def _lin(rng, bits, O, K):
+    return (util.HostLinear.affine4 if bits == 4 else util.HostLinear.affine8)(rng, O, K)
+
+
+def _orc_lin(lin, xb):
+    M = xb.shape[0]
+    want = np.empty((M, lin.O), np.uint16)
+    if lin.mode == "affine4":
+        oracle().orc_affine4_gather_qmv(p(lin.w), p(lin.scales), p(lin.biases), 1, lin.O, lin.K, p(xb), None, None, M, p(want))
+    else:
+        oracle().orc_affine8_qmv(p(lin.w), p(lin.scales), p(lin.biases), lin.O, lin.K, p(xb), M, p(want))
+    return want
+
+
+@pytest.mark.parametrize("K,mats", [
+    (1024, [(4, 257), (8, 33)]), (2048, [(4, 1000), (4, 36), (8, 256), (8, 1)]), (4096, [(4, 515), (8, 40)]),
+    # more rows than the chip holds at once: a wavefront walks several groups, the last ones ragged
+    (2048, [(4, 12289), (8, 9)]), (4096, [(4, 9001)]), (1024, [(4, 30011)]), (2048, [(8, 4099)])])
+def test_affine_projections_sharing_a_launch_bit_exact(orn, ctx, K, mats):
+    """Both bit widths in one launch, at each width of the kernel and every split of the activation rows over
+    it (1 to 9 rows), ragged matrices among them."""
+    rng = np.random.default_rng(K + len(mats))
+    lins = [_lin(rng, b, O, K) for b, O in mats]
+    dls = [l.dev(orn, ctx) for l in lins]
+    for M in (1, 2, 3, 4, 5, 9):
+        xb = util.bf16_normal(rng, (M, K))
+        dx, ys = ctx.to_device(xb), [ctx.alloc(M * l.O * 2) for l in lins]
+        ctx.linear_matmul_multi(dls, dx, M, ys)
+        for l, y in zip(lins, ys):
+            assert np.array_equal(y.download(np.uint16, (M, l.O)), _orc_lin(l, xb)), (M, l.mode, l.O)
+        for b in (dx, *ys): b.free()
+    for d in dls: d.free()
+
+
+@pytest.mark.parametrize("mats", [[(4, 40)], [(8, 256), (8, 1)], [(4, 8192), (4, 4096)], [(4, 8192), (4, 513), (4, 512)]])
+def test_affine_projections_with_the_norm_in_their_head_bit_exact(orn, ctx, mats):
+    """The residual add and the norm inside the projections' launch (width 2048, one to four rows; five take it in
+    front): h, the normed rows and every projection against the oracle's add_rms_norm and mat-vecs."""
+    rng = np.random.default_rng(len(mats))
+    H = 2048
+    lins = [_lin(rng, b, O, H) for b, O in mats]
+    dls = [l.dev(orn, ctx) for l in lins]
+    wn = util.bf16_normal(rng, (H,))
+    dwn = ctx.to_device(wn)
+    for M in (1, 2, 3, 4, 5):
+        res, y = util.bf16_normal(rng, (M, H)), util.bf16_normal(rng, (M, H))
+        wh, wnormed = util.orc_add_rms_norm(res, y, wn)
+        bufs = [ctx.to_device(res), ctx.to_device(y), ctx.alloc(M * H * 2), ctx.alloc(M * H * 2)]
+        ys = [ctx.alloc(M * l.O * 2) for l in lins]
+        orn.add_rms_linear_multi(ctx, dls, bufs[0], bufs[1], dwn, 1e-6, M, bufs[2], bufs[3], ys)
+        assert np.array_equal(bufs[2].download(np.uint16, (M, H)), wh) and np.array_equal(bufs[3].download(np.uint16, (M, H)), wnormed), M
+        for l, yy in zip(lins, ys):
+            assert np.array_equal(yy.download(np.uint16, (M, l.O)), _orc_lin(l, wnormed)), (M, l.mode, l.O)
+        for b in bufs + ys: b.free()
+    dwn.free()
+    for d in dls: d.free()
+
+
+# (2048, 512): the published artifact's block, the expert kernels of one column group a lane set each; 4096 and 256:
+# their other widths; 512 and 320: the kernels of any width
+@pytest.mark.parametrize("H,I", [(2048, 512), (4096, 256), (512, 320)])
+def test_affine_block_at_every_launch_size_bit_exact(orn, ctx, H, I):
+    """1 to 5, 9 and 16 tokens go through every row count a wavefront of the up launch takes (1, 2 and 4 times
+    two) and every column count of the down launch (8, 16, 32, 64): ids, scores and output of the operator, and
+    the layer's form with the norm in the router's head, by bits."""
+    rng = np.random.default_rng(H + I)
+    moe = util.HostMoe(rng, H=H, E=64, I=I, top_k=8, gate_kind=util.AFFINE4)
+    w = moe.dev(orn, ctx)
+    wn = util.bf16_normal(rng, (H,))
+    dwn = ctx.to_device(wn)
+    for T in (1, 2, 3, 4, 5, 9, 16):
+        res, y = util.bf16_normal(rng, (T, H)), util.bf16_normal(rng, (T, H))
+        wh, xb = util.orc_add_rms_norm(res, y, wn)
+        want, winds, wscores, _ = util.orc_moe_block(moe, xb, T)
+        bufs = [ctx.to_device(a) for a in (xb, res, y)] + [ctx.alloc(T * H * 2) for _ in range(3)] + [ctx.alloc(T * 32), ctx.alloc(T * 16)]
+        dx, dres, dy, dh, dn, out, inds, scores = bufs
+        ctx.moe_block(w, dx, T, out, inds, scores)
+        assert np.array_equal(inds.download(np.uint32, (T, 8)), winds) and np.array_equal(scores.download(np.uint16, (T, 8)), wscores), T
+        assert np.array_equal(out.download(np.uint16, (T, H)), want), T
+        out.zero()
+        orn.add_rms_moe_block(ctx, w, dres, dy, dwn, 1e-6, T, dh, dn, out)
+        assert np.array_equal(dh.download(np.uint16, (T, H)), wh) and np.array_equal(dn.download(np.uint16, (T, H)), xb), T
+        assert np.array_equal(out.download(np.uint16, (T, H)), want), T
+        for b in bufs: b.free()
+    dwn.free(); moe.free()
+
+
+@pytest.mark.parametrize("bits,O,K", [(4, 513, 2048), (8, 256, 2048), (4, 2048, 4096)])
+def test_affine_linear_is_exact_at_prompt_widths_without_gemms(orn, ctx, bits, O, K):
+    """gemm_rows = 0 brings the exact sums back at every width (from 32 rows on the default is a GEMM)."""
+    rng = np.random.default_rng(O)
+    lin = _lin(rng, bits, O, K)
+    dl = lin.dev(orn, ctx)
+    M = 70
+    xb = util.bf16_normal(rng, (M, K))
+    dx, dy = ctx.to_device(xb), ctx.alloc(M * O * 2)
+    try:
+        orn.set_option("gemm_rows", 0)
+        ctx.linear_matmul(dl, dx, M, dy)
+        assert np.array_equal(dy.download(np.uint16, (M, O)), _orc_lin(lin, xb))
+    finally:
+        orn.set_option("gemm_rows", 32)
+        for b in (dx, dy): b.free()
+        dl.free()

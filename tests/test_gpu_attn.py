@@ -66,3 +66,36 @@ def test_attention_bit_exact(orn, ctx, T, Hq, Hkv, hd, cap, offset):
         assert np.array_equal(dkc.download(np.uint16, kc.shape), wkc) and np.array_equal(dvc.download(np.uint16, vc.shape), wvc), fold
     orn.set_option("fuse_attn_prep", 1)
     for b in d + [dkc, dvc, dq, dout, dc, ds]: b.free()
+
+
+# the matrix-core form (four heads a workgroup; groups of eight and of three heads, head widths 256 and 128) and the
+# 1024-thread one, inside the first key block and past it
+@pytest.mark.parametrize("T,Hq,Hkv,hd,cap,offset", [(4, 16, 2, 256, 4096, 2500), (4, 16, 2, 128, 4096, 3000), (8, 6, 2, 256, 8192, 8000),
+                                                    (2, 16, 2, 256, 4096, 51), (2, 16, 2, 256, 4096, 600)])
+def test_attention_special_values(orn, ctx, T, Hq, Hkv, hd, cap, offset):
+    """Subnormal keys and values, score products below the normal range, infinities and NaNs in keys and values:
+    the oracle's values, NaN for NaN."""
+    rng = np.random.default_rng(offset)
+    q, gate = util.bf16_normal(rng, (T, Hq, hd)), util.bf16_normal(rng, (T, Hq, hd))
+    k0, v0 = (rng.standard_normal((Hkv, cap, hd)).astype(np.float32) for _ in range(2))
+    dq, dg, out = ctx.to_device(q), ctx.to_device(np.concatenate([np.zeros_like(gate), gate], -1)), ctx.alloc(T * Hq * hd * 2)
+    dk, dv = ctx.alloc(k0.size * 2), ctx.alloc(v0.size * 2)
+
+    def values(v): v[0, 3, 5], v[0, 4, 6], v[0, 9, 6], v[1, 7, 1] = np.inf, np.inf, -np.inf, np.nan
+    cases = {"subnormal values": lambda k, v: v.__imul__(np.float32(1e-39)),
+             "subnormal keys": lambda k, v: k.__imul__(np.float32(1e-39)),
+             "products below the normal range": lambda k, v: k.__imul__(np.float32(1e-37)),
+             "infinite and NaN values": lambda k, v: values(v),
+             "an infinite key": lambda k, v: k[0, 3].fill(np.inf),
+             "a key of minus infinity": lambda k, v: k[0, 7, :1].fill(-np.inf),
+             "a NaN key": lambda k, v: k[0, 3, :1].fill(np.nan)}
+    for name, change in cases.items():
+        k, v = k0.copy(), v0.copy()
+        change(k, v)
+        kb, vb = util.f32_to_bf16(k), util.f32_to_bf16(v)
+        dk.upload(kb); dv.upload(vb)
+        ctx.sdpa_decode_gated(dq, dk, dv, dg, T, Hq, Hkv, hd, offset, cap, hd ** -0.5, out)
+        want = util.orc_sdpa(q, kb, vb, gate, offset, hd ** -0.5)
+        assert util.same_values(out.download(np.uint16, want.shape), want), name
+        assert not np.isnan(util.bf16_to_f32(want)).all(), name
+    for b in (dq, dg, out, dk, dv): b.free()

@@ -43,6 +43,8 @@ def test_device_scalar_functions_bit_exact(orn, ctx):
     o.orc_sigmoid_bf16_n(util.p(bits), util.p(want), C.c_int64(65536))
     got = ctx.selftest_unary(orn.FN_SIGMOID_BF16, xb)
     assert np.array_equal(util.f32_to_bf16(got[fin]), want[fin])
+    # ... infinities and NaNs among them
+    assert util.same_values(util.f32_to_bf16(got), want) and np.isnan(got).sum() == np.isnan(xb).sum() == 254
     # rounding and the wavefront butterfly
     assert np.array_equal(util.f32_to_bf16(ctx.selftest_unary(orn.FN_ROUND_BF16, x)), util.f32_to_bf16(x))
     # ... over every exponent and upper mantissa, with the lower halves that decide rounding
@@ -274,4 +276,29 @@ def test_qmv_of_more_rows_than_a_launch_holds(orn, ctx, kind):
     want = util.f32_to_bf16(util.orc_qmv(kind, *t, O, K, util.bf16_to_f32(xb[:P])))
     assert np.array_equal(dy.download(np.uint16, (M, O)), np.tile(want, (M // P + 1, 1))[:M])
     for b in (dx, dy): b.free()
+    w.free()
+
+
+# the form on the matrix cores (three rows and more of large matrices) beside the vector one
+@pytest.mark.parametrize("kind,K,O,M", [(Q4K, 2048, 44001, 3), (Q4K, 4096, 5503, 13), (Q6K, 4096, 5497, 16), (Q4K, 2048, 512, 4),
+                                         (Q6K, 2048, 512, 3)])
+@pytest.mark.parametrize("what", ["subnormal", "products below the normal range", "infinities", "nan"])
+def test_qmv_special_activations(orn, ctx, kind, K, O, M, what):
+    """A chain of v_mfma_f32_4x4x1 is the chain of fused multiply-adds on every value there is: subnormal
+    activations and products are kept, an infinity or a NaN stays in its activation row."""
+    rng = np.random.default_rng(K + M)
+    t = util.make_kq(kind, rng, 1, O, K)
+    w = _dev_matrix(orn, ctx, kind, t, 1, O, K)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    if what == "subnormal": x *= np.float32(1e-39)
+    elif what == "nan": x[0, 5] = np.nan
+    elif what == "infinities": x[0, 5], x[1, 7], x[1, 9] = np.inf, -np.inf, np.inf
+    else: x *= np.float32(1e-36)
+    for dt, xb in ((orn.F32, x), (orn.BF16, util.f32_to_bf16(x))):
+        dx, dy = ctx.to_device(xb), ctx.alloc(M * O * 4)
+        ctx.kq_qmv(w, dx, dt, M, dy, orn.F32)
+        got, want = dy.download(np.float32, (M, O)), util.orc_qmv(kind, *t, O, K, xb if dt == orn.F32 else util.bf16_to_f32(xb))
+        assert util.same_values(got, want)
+        assert np.isfinite(got[2:]).all() and np.any(got[2:])
+        for b in (dx, dy): b.free()
     w.free()

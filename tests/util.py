@@ -158,6 +158,12 @@ def global_rel(got, want):
     return float(np.max(np.abs(got - want)) / max(np.max(np.abs(want)), 1e-300))
 
 
+def same_values(got, want):
+    """Equal bit for bit, NaNs (whose payload is the machine's own) wherever the other has one."""
+    got, want = (bf16_to_f32(a) if a.dtype == np.uint16 else a for a in (got, want))
+    return bool(np.all((got.view(np.uint32) == want.view(np.uint32)) | (np.isnan(got) & np.isnan(want))))
+
+
 # ---- host-side model pieces: numpy tensors that feed both the oracle and the device ----
 class OrcKmat(C.Structure):
     _fields_ = [("kind", C.c_int), ("E", C.c_int), ("O", C.c_int), ("K", C.c_int),
