@@ -10,7 +10,8 @@
 // and sigmoid_gate (kernels/ornith_elementwise.metal).
 //
 // Attention is split over keys in blocks of 256 by absolute position, one
-// workgroup per (block, query head, query row): a key's score is one fma chain per
+// workgroup per (block, query head, query row), or for four heads of a KV group where
+// there are many of them: a key's score is one fma chain per
 // 64 channels with the chains added pairwise, a channel's output one fma chain per
 // 64 keys of the block added the same way, so neither needs a cross-lane reduction
 // per key. The partial (max, sum, values) of each block go to scratch and a second
@@ -468,7 +469,8 @@ unsigned sdpa_many_grid(const SdpaArgs& p) {
 // four chains of a channel meet in LDS. Every sum of every head keeps its order.
 // us before (256 threads, vector fmas, queries read from LDS) -> now, two KV groups of eight heads of 256:
 // 4 rows at 6621 keys 23.7 -> 17.4, 2 at 9000 23.2 -> 17.0, 6 at 1445 19.3 -> 12.3, 9 at 16000 117 -> 62.
-// (A KV group that is no multiple of four heads repeats its last one; what that makes is not stored.)
+// (A KV group that is no multiple of four heads repeats its last one; what that makes is not stored. What
+// it costs stands at the choice of the form, sdpa_decode.)
 // grid sdpa_many_grid, 512 threads
 template <int HD>
 __global__ __launch_bounds__(512, 4) void sdpa_partial_many_kernel(SdpaArgs p) {
@@ -834,19 +836,22 @@ static int sdpa_decode(ornith_ctx* ctx, const void* d_q_rot, const void* d_k_cac
   p.cap = cap;
   p.nblk = nblk;
   p.scale = scale;
-  // one query head per workgroup: the arithmetic (256 keys x head_dim fmas per head) is what
-  // bounds a block, so spreading heads over workgroups beats sharing the key loads
+  // Which form. One 1024-thread workgroup a (key block, head, row) has the shorter chain, but 150 KB of LDS
+  // let a compute unit hold one of them: a round takes as long as the whole call of the many form (four
+  // heads of a KV group a workgroup, two workgroups a compute unit), so it is the faster one for as long as
+  // it is one round. Whole calls, us, 1024-thread form / many form, two KV groups of eight heads of 256:
+  // 256 workgroups of the first (one row at 4000 keys, four at 1000) 13.4 / 16.7, 288 (three rows at 1500)
+  // 20.1 / 16.8, 384 20.3 / 16.9, 768 27.4 / 17.0, 1536 47.8 / 22.2; head width 128, 256: 11.3 / 13.0, 384: 16.8 / 13.3.
+  // KV groups that are no multiple of four heads, whose last workgroup repeats heads, turn at the same
+  // place: groups of six 13.2 / 16.6 at 192 and 21.4 / 16.8 at 288, of three 13.0 / 16.7 and 20.0 / 16.8, of two
+  // 15.9 / 18.2 at 256 and 21.4 / 17.0 at 384, of one (four times the arithmetic) 13.4 / 16.8 at 256, level from 288
+  // to 512 (20.9 / 21.7, 22.9 / 22.7), 38.3 / 31.9 at 768.
+  // Inside the first key block the 1024-thread form finishes by itself, without the merge launch, and a second
+  // round is still ahead: 31 rows (496 workgroups) at 0 / 200 keys 12.0 / 22.5 and 17.1 / 22.8.
   const dim3 grid(nblk, Hq, T);
-  // few live blocks (short contexts): one 1024-thread block per (key block, head) finishes
-  // soonest; many: the 256-thread form keeps more blocks in flight. Same sums either way.
   const int last_max = (d_offset ? cap - 1 : (offset + T - 1 < cap - 1 ? offset + T - 1 : cap - 1));
   const long live = (long)(last_max / ATT_KB + 1) * Hq * T;
-  // four heads of a KV group a workgroup (the key / value block read once for the four) from a
-  // workgroup for every fourth compute unit on: 25.6 us against 35.4 for one row at a 6.6 k
-  // context (108 workgroups), 22.4 against 14.3 at 3 k (48)
-  // (inside the first key block the finishing form is one launch instead of two)
-  const bool four = (Hq / Hkv) % 4 == 0 && live / 4 >= ctx->compute_units / 4 && last_max >= ATT_KB;
-  const bool many = live > 2L * ctx->compute_units || four;
+  const bool many = live > (last_max < ATT_KB ? 2L : 1L) * ctx->compute_units;
   // one key block for every row, in the kernel form that knows how to finish: no merge launch
   p.finish = (last_max < ATT_KB && !many) ? 1 : 0;
   const bool fold = prep && !many && !d_offset && T <= 8 && ornith_option_fuse_attn_prep();

@@ -25,13 +25,17 @@ def _mk(rng, T, Hq, Hkv, hd, cap, offset):
     (1, 16, 2, 256, 4096, 0), (2, 16, 2, 256, 4096, 51), (4, 16, 2, 256, 4096, 254), (8, 16, 2, 256, 4096, 250),
     (8, 16, 2, 256, 4096, 100), (3, 8, 2, 128, 1024, 255), (5, 4, 4, 256, 512, 300),
     (3, 4, 1, 256, 512, 0), (2, 4, 2, 128, 768, 300), (1, 2, 2, 256, 256, 7),
-    # many live key blocks: the launch switches to its 256-thread form (same sums)
+    # many live key blocks: the launch switches to four heads of a KV group a workgroup (same sums)
     (4, 16, 2, 256, 4096, 4000), (4, 16, 2, 128, 4096, 3000),
-    # ... with one head a workgroup (KV groups of three heads) and four (groups of eight, ragged last block)
-    (8, 6, 2, 256, 8192, 8000), (3, 16, 2, 256, 8192, 7000),
-    # 16-row prompt chunks inside the first key block (one finishing launch) and across its end
-    # (enough rows for the four-head form, which leaves the finishing to the merge launch)
-    (16, 16, 2, 256, 4096, 35), (16, 16, 2, 128, 4096, 0), (16, 16, 2, 256, 4096, 250),
+    # ... with KV groups that are no multiple of four heads (three, one, two, six, five), and of eight (ragged last block)
+    (8, 6, 2, 256, 8192, 8000), (4, 16, 16, 256, 2048, 1500), (4, 16, 8, 256, 2048, 1500), (2, 24, 4, 256, 4096, 3000),
+    (7, 10, 2, 128, 4096, 3300), (3, 16, 2, 256, 8192, 7000),
+    # ... from one workgroup of the other form more than there are compute units: the last call before that, and the first
+    (4, 16, 2, 256, 4096, 1020), (4, 16, 1, 128, 4096, 1021),
+    # 16-row prompt chunks inside the first key block (one finishing launch, of two rounds from 17 rows on) and across
+    # its end (enough rows for the four-head form, which leaves the finishing to the merge launch)
+    (16, 16, 2, 256, 4096, 35), (16, 16, 2, 128, 4096, 0), (31, 16, 2, 256, 4096, 200), (31, 17, 1, 256, 4096, 0),
+    (16, 16, 2, 256, 4096, 250),
     # the long-context configuration: a depth-3 verify window at the end of a 16384-row cache
     (4, 16, 2, 256, 16384, 16380), (1, 16, 2, 256, 16384, 6621)])
 def test_attention_bit_exact(orn, ctx, T, Hq, Hkv, hd, cap, offset):
