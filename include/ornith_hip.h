@@ -66,7 +66,8 @@ ORNITH_API int ornith_device_info(ornith_ctx* ctx, char* name, size_t name_len, 
  * events; elapsed synchronises on the end event and returns milliseconds. */
 /* Behaviour switches (the reference's ORNITH_* flags with their runtime set_* twins,
  * src/ops/moe.rs:397-414, src/ops/gdn.rs:416-426). Each is also read once from the
- * environment variable named here; every value gives bit-identical results.
+ * environment variable named here; results are bit-identical for every value unless the
+ * switch says otherwise.
  *   "fuse_moe"  (ORNITH_FUSE_MOE, default 1): the two fused expert kernels vs. one
  *               launch per operator
  *   "fuse_proj" (ORNITH_FUSE_PROJ, default 1): projections sharing an input in one launch
@@ -74,12 +75,20 @@ ORNITH_API int ornith_device_info(ornith_ctx* ctx, char* name, size_t name_len, 
  *               rows per wavefront of the fused gate+up expert kernel, a tuning knob
  *   "fuse_gdn"  (ORNITH_FUSE_GDN, default 1): the gated-delta mixer core (a / b projections,
  *               front, recurrence, gated norm) in one launch at decode / verify widths
+ *   "moe_down_iters" (ORNITH_MOE_DOWN_ITERS, default 0 = chosen by shape; 1, 2 or 4): column
+ *               groups per workgroup of the fused expert down kernel, a tuning knob
  *   "fuse_norm" (ORNITH_FUSE_NORM, default 1): the residual add + RMS norm in front of a
- *               group of k-quant projections / the router is computed inside their launch
- *   "gemm_rows" (ORNITH_GEMM_ROWS, default 32; 0 = never): activation rows from which the
- *               k-quant projections and the MoE experts run as matrix-core GEMMs instead of
- *               exact mat-vecs. The one switch that changes results (to bf16 rounding of the
- *               weights): prefill is outside the exact window in the reference as well.
+ *               group of k-quant or affine projections / the router is computed inside their launch
+ *   "gemm_rows" (ORNITH_GEMM_ROWS, default 32; 0 = never): activation rows from which prompts
+ *               take the matrix cores instead of the exact path: every Linear (k-quant, affine and
+ *               dense), the MoE block over k-quant experts, a layer's MoE block over 4-bit affine ones
+ *               (ornith_add_rms_moe_block), attention, the gated-delta recurrence (its shorter
+ *               chain; chunks from 128 rows on whatever this switch is, see "gdn_chunked").
+ *               This switch changes results: sums run in another order, and k-quant weights (not
+ *               affine or dense ones) are rounded to bf16. So the rows of a call of gemm_rows or more
+ *               are not the bits of the same rows in shorter calls: through 40 bf16 layers the two
+ *               differ by 0.8 % (relative 2-norm; single rows by up to 1.2 %), in every weight
+ *               format. Prefill is outside the exact window in the reference as well.
  *   "kq_iters"  (ORNITH_KQ_ITERS, default 0 = chosen by the launch from its shape and from how
  *               many of its workgroups a compute unit holds; 1..8): output rows each
  *               wavefront of the k-quant mat-vec walks, a tuning knob
@@ -136,7 +145,8 @@ ORNITH_API int ornith_kq_dequantize(ornith_ctx* ctx, const ornith_kmatrix* w, vo
 
 /* kquant::qmv (src/ops/kquant.rs:539-595): y[M,O] = x[M,K] . W^T, fp32
  * accumulate, each row computed exactly as it would be alone. M <= 4 is the
- * decode/verify shape; larger M goes in groups of up to four, in one launch. x 16-byte aligned. */
+ * decode/verify shape; larger M goes in groups of up to four, 131070 rows a launch. x 16-byte
+ * aligned. */
 ORNITH_API int ornith_kq_qmv(ornith_ctx* ctx, const ornith_kmatrix* w, const void* d_x, int x_dtype, int M,
                   void* d_y, int y_dtype);
 
@@ -192,7 +202,11 @@ typedef struct ornith_linear {
   const void* d_biases; /* as d_scales */
 } ornith_linear;
 
-/* Linear::matmul (src/ops/linear.rs:60-110): y[M,O] = x[M,K] . W^T, bf16 in/out. */
+/* Linear::matmul (src/ops/linear.rs:60-110): y[M,O] = x[M,K] . W^T, bf16 in/out. Below "gemm_rows"
+ * rows every row is computed exactly as it would be alone, in every format; from there on as a
+ * matrix-core GEMM, in which a row's bits do not depend on what else shares the launch either but
+ * are not those of the exact path. Affine mat-vecs of K = 1024, 2048 and 4096 have kernels of their
+ * own, other widths take row-a-wavefront ones (same bits, 1.6 to 2.5 times as long at two rows). */
 ORNITH_API int ornith_linear_matmul(ornith_ctx* ctx, const ornith_linear* w, const void* d_x, int M,
                                     void* d_y);
 
@@ -206,10 +220,11 @@ ORNITH_API int ornith_linear_matmul_multi(ornith_ctx* ctx, const ornith_linear* 
 /* norm::add_rms_norm followed by the projections that read its output (the closing add of a
  * decoder layer, the next layer's input norm and its in_proj_qkv + in_proj_z or q/k/v
  * projections: src/model/qwen3_5.rs:374-396, 441-447, 493-499): h = res + y (bf16),
- * normed = rms_norm(h, w_norm), ys[i] = normed . W_i^T. For k-quant projections of width 2048
- * at M <= 4 the norm is made inside the projections' launch (every workgroup computes it while
- * its weight loads are in flight; one of them stores h and normed); otherwise add_rms_norm and
- * linear_matmul_multi are issued. Bit-identical either way. */
+ * normed = rms_norm(h, w_norm), ys[i] = normed . W_i^T. For k-quant or affine projections of width
+ * 2048 at M <= 4 the norm is made inside the projections' launch (every workgroup computes it while
+ * its weight loads are in flight; one of them stores h and normed), if the outputs lie apart from
+ * res, y and w_norm; otherwise add_rms_norm and linear_matmul_multi are issued, which work in place
+ * too. Bit-identical either way. */
 ORNITH_API int ornith_add_rms_linear_multi(ornith_ctx* ctx, const ornith_linear* const* ws, int n,
                                            const void* d_res, const void* d_y, const void* d_wnorm,
                                            float eps, int M, void* d_h_out, void* d_normed_out,
@@ -277,8 +292,8 @@ ORNITH_API int ornith_moe_block(ornith_ctx* ctx, const ornith_moe_weights* w, co
 /* norm::add_rms_norm followed by sparse_moe_block on its output (the post-attention norm and
  * the MLP of a decoder layer, src/model/qwen3_5.rs:384-392): h = res + y, normed =
  * rms_norm(h, w_norm), out = moe(normed). With the fused expert kernels, hidden size 2048 and
- * T <= 4 the norm is made inside the router's launch; otherwise add_rms_norm is issued first.
- * Bit-identical either way. This is the form a prompt takes through a layer, so from "gemm_rows"
+ * T <= 4 the norm is made inside the router's launch, if h_out and normed_out lie apart from its
+ * inputs; otherwise add_rms_norm is issued first. Bit-identical either way. This is the form a prompt takes through a layer, so from "gemm_rows"
  * rows on blocks over 4-bit affine experts run as GEMMs here as well: the same arithmetic as
  * ornith_moe_block's with its fp32 sums in another order (a router tie may fall the other way). */
 ORNITH_API int ornith_add_rms_moe_block(ornith_ctx* ctx, const ornith_moe_weights* w, const void* d_res,

@@ -6,7 +6,9 @@
 // /root/reference/kernels/q6k.metal:47-169,365-393). The storage format is the
 // reference's three tensors per matrix, untouched.
 //
-// Schedule (this build's own, for 64-lane wavefronts; bandwidth bound, no MFMA):
+// Schedule (this build's own, for 64-lane wavefronts; bound by the stream of weights and by vector
+// issue; large launches of three and more activation rows take the same chains to the matrix cores,
+// kquant_rows.hip):
 //   chunk j of a row belongs to lane j % 64 (see kq_device.h); rows narrower than
 //   64 chunks pack 64/LPR rows into one wavefront (LPR lanes per row); rows wider
 //   than 64 chunks are split over KS wavefronts whose lane partials are added

@@ -12,21 +12,24 @@
 // partial tiles meet in LDS once. No barrier inside the K loop, and narrow projections become O / 16
 // workgroups.
 //
-// What such a kernel then runs against is the L1's tag lookups: 64 lanes that each read their own row
-// are 64 lookups a load instruction, one a clock and compute unit, whatever a lane takes (with the
-// activation fragments read that way from memory and the codes in 8-byte pieces the counters showed
-// 61 lookups a load and the L1 busy 93 % of the time). So every lane takes 16 bytes of codes a load,
-// the activations come in as whole 64- or 128-byte pieces of a row straight into LDS
-// (global_load_lds: no registers; each wavefront its own K block, so nothing waits for another
+// What such a kernel can run against is the L1's tag lookups: 64 lanes that each read their own row
+// are 64 lookups a load instruction, one a clock and compute unit, whatever a lane takes. So every lane
+// takes 16 bytes of codes a load, the activations come in as whole 64- or 128-byte pieces of a row straight
+// into LDS (global_load_lds: no registers; each wavefront its own K block, so nothing waits for another
 // wavefront), and the scales of all the workgroup's rows, which lie side by side in memory, as one
 // block. The k order inside a block is free as long as both operands follow it, and is chosen so that
 // 16 bytes of codes make a lane's operands (piece()).
 //
+// Counters of the expert launches (profiles/few_row_gemm_pmc.md): 28 to 39 lookups a load instruction and the L1
+// busy 35 to 42 % of the time, the matrix cores 5 to 14 %, the vector units 48 to 66 % (the codes' way to
+// operands), 3.6 to 4.1 TB/s from memory: vector issue beside the stream is what bounds them. The
+// plain launches of a short prompt are one pass of a chain: load, unpack, multiply, meet (vector units 13 %).
+//
 // Measured (us, before -> now): 12288 x 2048 Q4_K at 64 rows 29.5 -> 15.8, 2048 x 4096 at 64 rows 52 -> 11.8,
-// 256 x 2048 Q6_K 28.6 -> 7.1; the experts of a 51-token prompt, gate + up + swiglu 104 -> 54.5 (243 MB:
-// 4.5 TB/s), down 49 -> 36.6 (4.8 TB/s), of a 700-token one 156 -> 125 and 76 -> 82 (the shared expert
-// included); a 600-token prompt over 4-bit affine weights 462 ms -> 17.7 ms (its experts and
-// projections were mat-vecs, row by row).
+// 256 x 2048 Q6_K 28.6 -> 7.1; the experts of a 51-token prompt, gate + up + swiglu 104 -> 54 (193 MB from memory),
+// down 49 -> 36.5 (142 MB), of a 700-token one 156 -> 122 and 76 -> 82 (the shared expert included); a
+// 600-token prompt over 4-bit affine weights 461 ms -> 15.9 ms (its experts and projections were mat-vecs,
+// row by row).
 //
 // The order of the sums depends on K alone (256-wide blocks: wavefront ks takes blocks ks, ks + KS,
 // ...; the partial sums are added in one order), never on M, O or the launch's other matrices.
@@ -70,7 +73,7 @@ struct Args {
   Mat m[4];  // plain: up to four matrices; gathered: [0] routed (or gate), [1] routed up, [2] shared (gate), [3] shared up
   int n;
   const bf16_t* x;
-  int M, K, ks;  // ks: wavefronts that split K (2, 4, 8)
+  int M, K, ks;  // ks: wavefronts that split K (2 or 4)
   // gathered forms: tiles over (expert, row range) of an expert-sorted pair list. Expert E is the
   // shared one: its "pairs" are pairs + token.
   const uint32_t* pair;

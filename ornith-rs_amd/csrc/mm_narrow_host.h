@@ -42,9 +42,10 @@ int launch_affine(ornith_ctx* ctx, const Args& a, int mode, int ct, int rows, di
 
 }  // namespace nmm
 
-// The kernels of a family. A plain workgroup is eight wavefronts, two a SIMD; a gathered one four,
-// and as many workgroups a compute unit as accumulators, codes and activation chunks leave room for
-// without spilling (W16, W32: wavefronts a SIMD at 16 and 32 rows).
+// The kernels of a family. A workgroup is four wavefronts, one a SIMD; a compute unit holds two plain
+// ones, and as many gathered ones as accumulators, codes and activation chunks leave room for (W16, W32:
+// wavefronts a SIMD at 16 and 32 rows) without spilling, but for the 32-row affine kernels, which spill four
+// (gathered) and two (gate + up) registers at three wavefronts a SIMD.
 #define NMM_KERNELS(NAME, AFF, W16, W32, LDS_BIT)                                                                   \
   template <int CT>                                                                                                 \
   __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void NAME##_plain_kernel(Args a) {   \

@@ -13,6 +13,9 @@
 //                   (the last the shared expert): eight row dots each, met in LDS, then the
 //                   block's tail (router weights, bf16 accumulation in slot order, sigmoid-gated
 //                   shared expert).
+// moe_up_a4, moe_down_a4: the same launches with the same sums for 4-bit rows of 1024, 2048 or 4096 columns
+//                   (up) and of 256 or 512 (down), the widths of this model family; other widths and the
+//                   dense format take the two above, which cost 1.5 to 4.4 times as much (figures at each).
 //
 // A 4-bit row dot is affine4_qmv_kernel's (linear.hip), operation for operation: lane l owns the
 // 16-code chunks l + 64c in ascending c, one fma chain a chunk in code order beside the plain
