@@ -180,7 +180,7 @@ int launch_router(ornith_ctx* ctx, const bf16_t* gates, int T, int E, int k, uin
     hipLaunchKernelGGL(router_topk_kernel<P>, dim3(T), dim3(64), 0, ctx->stream, gates, E, k, \
                        inds, scores, probs, lhs_tok, lhs_row);                               \
     break;
-  switch (E / 64) {
+  switch (E % 64 == 0 ? E / 64 : 0) {
     ROUTER_CASE(1)
     ROUTER_CASE(2)
     ROUTER_CASE(4)
@@ -208,7 +208,7 @@ int launch_router_egate(ornith_ctx* ctx, const bf16_t* gates, int T, int E, int 
   case P:                                                                                                      \
     hipLaunchKernelGGL(router_egate_kernel<P>, dim3(T), dim3(64), 0, ctx->stream, gates, E, k, inds, scores, g); \
     break;
-  switch (E / 64) {
+  switch (E % 64 == 0 ? E / 64 : 0) {
     ROUTER_CASE(1)
     ROUTER_CASE(2)
     ROUTER_CASE(4)

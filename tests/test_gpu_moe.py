@@ -170,3 +170,24 @@ def test_moe_block_small_all_q4k_and_all_q6k(orn, ctx):
         out, inds, sc = _run_block(orn, ctx, moe, dw, xb, 3)
         assert np.array_equal(inds, want_inds) and np.array_equal(sc, want_sc) and np.array_equal(out, want_out)
         moe.free()
+
+
+@pytest.mark.parametrize("E", [96, 192, 200])
+@pytest.mark.parametrize("T", [1, 40])
+def test_expert_counts_the_router_has_no_layout_for_are_refused(orn, ctx, E, T):
+    """A wavefront's top-k holds 64, 128, 256, 512 or 1024 gates: a block of another number of experts is an
+    error at decode and prompt widths, fused and not, never a choice among some of them."""
+    rng = np.random.default_rng(E)
+    for kind in (Q4K, util.AFFINE4):
+        moe = util.HostMoe(rng, H=512, E=E, I=256, top_k=8, gate_kind=kind)
+        w = moe.dev(orn, ctx)
+        dx, out = ctx.to_device(util.bf16_normal(rng, (T, 512))), ctx.alloc(T * 512 * 2)
+        try:
+            for fuse in (1, 0):
+                orn.set_option("fuse_moe", fuse)
+                with pytest.raises(orn.OrnithError, match="E=%d" % E):
+                    ctx.moe_block(w, dx, T, out)
+        finally:
+            orn.set_option("fuse_moe", 1)
+            for b in (dx, out): b.free()
+            moe.free()
