@@ -215,11 +215,12 @@ __global__ __launch_bounds__(256) void moe_up_affine4_kernel(A4UpArgs<F> a) {
 // to memory for every 1024 columns of a row and unpacks with three instructions a code where this
 // one needs one and a half. LOOPS as in moe_up_kernel (moe_fused.hip): the next two rows asked for ahead
 // of the arithmetic of the present ones, once the grid is more than the chip holds. us at T = 1 / 2, K = 2048, I = 512: 11.3 / 16.6 -> 7.3 / 10.2
+// The routing is always made in its head: the block has it nowhere else for the expert counts it takes.
 // grid (ceil(I / (8 LOOPS)), T*k + T), 256 threads
-template <int NC, bool ROUTE, int LOOPS>
+template <int NC, int LOOPS>
 __global__ __launch_bounds__(256) void moe_up_a4_kernel(A4UpArgs<FmtA4> a) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = blockIdx.y;
-  const A4UpRow<FmtA4> u = a4_up_row<FmtA4, ROUTE>(a, lane, wave);
+  const A4UpRow<FmtA4> u = a4_up_row<FmtA4, true>(a, lane, wave);
   const int base0 = (blockIdx.x * 4 + wave) * 2 * LOOPS;
   constexpr int SETS = LOOPS > 1 ? 2 : 1;
   AffRow<4, 64, NC> rows[SETS][4];  // gate 0, up 0, gate 1, up 1
@@ -410,23 +411,18 @@ namespace {
 
 // the 4-bit kernels of fixed width; false: another format or width
 template <class F>
-bool launch_up_a4(ornith_ctx*, const A4UpArgs<F>&, bool) { return false; }
-bool launch_up_a4(ornith_ctx* ctx, const A4UpArgs<FmtA4>& u, bool route) {
+bool launch_up_a4(ornith_ctx*, const A4UpArgs<F>&) { return false; }
+bool launch_up_a4(ornith_ctx* ctx, const A4UpArgs<FmtA4>& u) {
+  if (!u.gates) return false;
   const int rows_y = u.T * u.k + u.T, nc = u.K % 1024 == 0 ? u.K / 1024 : 0;
   const long one = (long)((u.I + 7) / 8) * rows_y;
   const int loops = one <= 5L * ctx->compute_units ? 1 : one <= 9L * ctx->compute_units ? 2 : 4;
   const dim3 grid((u.I + 8 * loops - 1) / (8 * loops), rows_y);
-#define UP_GO(NC, ROUTE, LOOPS) hipLaunchKernelGGL((moe_up_a4_kernel<NC, ROUTE, LOOPS>), grid, dim3(256), 0, ctx->stream, u)
-#define UP_ROUTE(NC, ROUTE)                 \
-  if (loops == 1) UP_GO(NC, ROUTE, 1);      \
-  else if (loops == 2) UP_GO(NC, ROUTE, 2); \
-  else UP_GO(NC, ROUTE, 4)
-#define UP_NC(NC)         \
-  if (route) {            \
-    UP_ROUTE(NC, true);   \
-  } else {                \
-    UP_ROUTE(NC, false);  \
-  }                       \
+#define UP_GO(NC, LOOPS) hipLaunchKernelGGL((moe_up_a4_kernel<NC, LOOPS>), grid, dim3(256), 0, ctx->stream, u)
+#define UP_NC(NC)                   \
+  if (loops == 1) UP_GO(NC, 1);      \
+  else if (loops == 2) UP_GO(NC, 2); \
+  else UP_GO(NC, 4);                 \
   return true;
   switch (nc) {
     case 1: UP_NC(1)
@@ -434,7 +430,6 @@ bool launch_up_a4(ornith_ctx* ctx, const A4UpArgs<FmtA4>& u, bool route) {
     case 4: UP_NC(4)
     default: return false;
   }
-#undef UP_ROUTE
 #undef UP_GO
 #undef UP_NC
 }
@@ -486,7 +481,7 @@ int launch_pair(ornith_ctx* ctx, const ornith_moe_weights* w, const typename F::
   u.inds_out = const_cast<uint32_t*>(d_inds);
   u.scores_out = (bf16_t*)const_cast<void*>(d_scores);
   const dim3 ugrid((I + 3) / 4, T * k + T);
-  if (launch_up_a4(ctx, u, d_gates != nullptr)) {
+  if (launch_up_a4(ctx, u)) {
   } else if (d_gates)
     hipLaunchKernelGGL((moe_up_affine4_kernel<F, true>), ugrid, dim3(256), 0, ctx->stream, u);
   else
