@@ -220,7 +220,8 @@ def test_affine_projections_sharing_a_launch_bit_exact(orn, ctx, K, mats):
     for d in dls: d.free()
 
 
-@pytest.mark.parametrize("mats", [[(4, 40)], [(8, 256), (8, 1)], [(4, 8192), (4, 4096)], [(4, 8192), (4, 513), (4, 512)]])
+@pytest.mark.parametrize("mats", [[(4, 40)], [(8, 256), (8, 1)], [(4, 8192), (4, 4096)], [(4, 8192), (4, 513), (4, 512)],
+                                  [(4, 12301)]])
 def test_affine_projections_with_the_norm_in_their_head_bit_exact(orn, ctx, mats):
     """The residual add and the norm inside the projections' launch (width 2048, one to four rows; five take it in
     front): h, the normed rows and every projection against the oracle's add_rms_norm and mat-vecs."""
@@ -244,9 +245,9 @@ def test_affine_projections_with_the_norm_in_their_head_bit_exact(orn, ctx, mats
     for d in dls: d.free()
 
 
-# (2048, 512): the published artifact's block, the expert kernels of one column group a lane set each; 4096 and 256:
-# their other widths; 512 and 320: the kernels of any width
-@pytest.mark.parametrize("H,I", [(2048, 512), (4096, 256), (512, 320)])
+# (2048, 512): the published artifact's block; 4096, 1024 and 256: the other widths of its kernels; 512 and 320: the
+# kernels of any width
+@pytest.mark.parametrize("H,I", [(2048, 512), (4096, 256), (1024, 256), (512, 320)])
 def test_affine_block_at_every_launch_size_bit_exact(orn, ctx, H, I):
     """1 to 5, 9 and 16 tokens go through every row count a wavefront of the up launch takes (1, 2 and 4 times
     two) and every column count of the down launch (8, 16, 32, 64): ids, scores and output of the operator, and

@@ -26,7 +26,9 @@ def _weights(lin):
 
 @pytest.mark.parametrize("fmt", ["q4k", "q6k", "affine4", "affine8"])
 @pytest.mark.parametrize("O,K,M", [(512, 2048, 32), (200, 512, 33), (264, 768, 48), (2048, 4096, 65), (40, 1024, 130),
-                                    (4096, 2048, 64), (64, 4096, 17 + 64), (8, 2048, 200)])
+                                    (4096, 2048, 64), (64, 4096, 17 + 64), (8, 2048, 200),
+                                    # two and four column tiles a wavefront; an odd number of columns
+                                    (4096, 512, 65), (4099, 2048, 130), (12288, 2048, 33)])
 def test_few_row_matmul_vs_float64(orn, ctx, fmt, O, K, M):
     rng = np.random.default_rng(O + K + M)
     lin = (util.HostLinear.kq(rng, Q4K if fmt == "q4k" else Q6K, O, K) if fmt[0] == "q" else
@@ -68,6 +70,23 @@ def test_few_row_moe_block_vs_exact(orn, ctx, fmt, T):
     rel = np.linalg.norm(got - want, axis=1) / np.linalg.norm(want, axis=1)
     bound = 0.004 if fmt == "affine4" else 0.01
     assert np.median(rel) < bound and (rel < 0.03).mean() >= 0.93, (float(np.median(rel)), float(np.sort(rel)[-5]))
+    for b in (dx, out): b.free()
+    moe.free()
+
+
+@pytest.mark.parametrize("E,T", [(128, 40), (512, 33), (1024, 32)])
+def test_few_row_moe_block_of_other_expert_counts(orn, ctx, E, T):
+    """The other layouts of the router's tail, against the oracle's exact block as above."""
+    rng = np.random.default_rng(E)
+    moe = util.HostMoe(rng, H=512, E=E, I=512, top_k=8)
+    xb = util.bf16_normal(rng, (T, 512))
+    want = util.bf16_to_f32(util.orc_moe_block(moe, xb, T)[0]).astype(np.float64)
+    w = moe.dev(orn, ctx)
+    dx, out = ctx.to_device(xb), ctx.alloc(T * 512 * 2)
+    ctx.moe_block(w, dx, T, out)
+    got = util.bf16_to_f32(out.download(np.uint16, (T, 512))).astype(np.float64)
+    rel = np.linalg.norm(got - want, axis=1) / np.linalg.norm(want, axis=1)
+    assert np.median(rel) < 0.01 and (rel < 0.03).mean() >= 0.93, np.sort(rel)[-5:]
     for b in (dx, out): b.free()
     moe.free()
 

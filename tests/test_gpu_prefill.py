@@ -370,7 +370,8 @@ def test_model_forward_of_a_whole_long_prompt_in_one_call(orn, ctx):
     for o in (a, b, model, ws): o.close()
 
 
-@pytest.mark.parametrize("O,K,M", [(32, 2048, 4096), (1, 2048, 300), (48, 256, 33), (130, 512, 77), (64, 128, 32)])
+@pytest.mark.parametrize("O,K,M", [(32, 2048, 4096), (1, 2048, 300), (48, 256, 33), (130, 512, 77), (64, 128, 32),
+                                    (40, 1024, 100), (17, 3072, 45)])
 def test_dense_matmul_vs_float64(orn, ctx, O, K, M):
     """narrow dense bf16 projections at prefill widths run as a small matrix-core GEMM (rows split
     over workgroups, K over a workgroup's wavefronts); reference: float64 over the same bf16 values"""
