@@ -20,7 +20,7 @@
 // block. The k order inside a block is free as long as both operands follow it, and is chosen so that
 // 16 bytes of codes make a lane's operands (piece()).
 //
-// Counters of the expert launches (profiles/few_row_gemm_pmc.md): 28 to 39 lookups a load instruction and the L1
+// Counters of the expert launches: 28 to 39 lookups a load instruction and the L1
 // busy 35 to 42 % of the time, the matrix cores 5 to 14 %, the vector units 48 to 66 % (the codes' way to
 // operands), 3.6 to 4.1 TB/s from memory: vector issue beside the stream is what bounds them. The
 // plain launches of a short prompt are one pass of a chain: load, unpack, multiply, meet (vector units 13 %).

@@ -28,7 +28,7 @@ def _weights(lin):
 @pytest.mark.parametrize("O,K,M", [(512, 2048, 32), (200, 512, 33), (264, 768, 48), (2048, 4096, 65), (40, 1024, 130),
                                     (4096, 2048, 64), (64, 4096, 17 + 64), (8, 2048, 200),
                                     # two and four column tiles a wavefront; an odd number of columns
-                                    (4096, 512, 65), (4099, 2048, 130), (12288, 2048, 33)])
+                                    (4096, 512, 65), (4096, 2048, 65), (4099, 2048, 130), (12288, 2048, 33)])
 def test_few_row_matmul_vs_float64(orn, ctx, fmt, O, K, M):
     rng = np.random.default_rng(O + K + M)
     lin = (util.HostLinear.kq(rng, Q4K if fmt == "q4k" else Q6K, O, K) if fmt[0] == "q" else
