@@ -88,7 +88,8 @@ ORNITH_API int ornith_device_info(ornith_ctx* ctx, char* name, size_t name_len, 
  *               affine or dense ones) are rounded to bf16. So the rows of a call of gemm_rows or more
  *               are not the bits of the same rows in shorter calls: through 40 bf16 layers the two
  *               differ by 0.8 % (relative 2-norm; single rows by up to 1.2 %), in every weight
- *               format. Prefill is outside the exact window in the reference as well.
+ *               format. Prefill is outside the exact window in the reference as well. (Exact
+ *               attention takes up to 64 rows a call, so a forward above gemm_rows' reach does too.)
  *   "kq_iters"  (ORNITH_KQ_ITERS, default 0 = chosen by the launch from its shape and from how
  *               many of its workgroups a compute unit holds; 1..8): output rows each
  *               wavefront of the k-quant mat-vec walks, a tuning knob
