@@ -850,7 +850,7 @@ static int sdpa_decode(ornith_ctx* ctx, const void* d_q_rot, const void* d_k_cac
   // fastest in the grid, over eight dies). With an odd number every head's workgroup fetches the block into
   // another die's L2 and the 1024-thread form takes longer the more there are of them: one row, 9 / 11 / 13 / 15
   // blocks 16.9 / 17.9 / 19.1 / 19.8 us, 8 / 10 / 12 / 14 / 16 blocks 12.4 / 14.3 / 13.3 / 15.2 / 13.3; at head width 128 12.0 to
-  // 13.5 and 10.6 to 11.5. That is the grid's numbering to mend, not this line's place.
+  // 13.5 and 10.7 to 11.5. That is the grid's numbering to mend, not this line's place.
   // Inside the first key block the 1024-thread form finishes by itself, without the merge launch, and a second
   // round is still ahead: 31 rows (496 workgroups) at 0 / 200 keys 12.0 / 22.5 and 17.1 / 22.8.
   const dim3 grid(nblk, Hq, T);
