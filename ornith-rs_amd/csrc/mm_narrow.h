@@ -20,19 +20,26 @@
 // block. The k order inside a block is free as long as both operands follow it, and is chosen so that
 // 16 bytes of codes make a lane's operands (piece()).
 //
-// Counters of the expert launches: 28 to 39 lookups a load instruction and the L1
-// busy 35 to 42 % of the time, the matrix cores 5 to 14 %, the vector units 48 to 66 % (the codes' way to
-// operands), 3.6 to 4.1 TB/s from memory: vector issue beside the stream is what bounds them. The
-// plain launches of a short prompt are one pass of a chain: load, unpack, multiply, meet (vector units 13 %).
+// The expert forms split columns, not K: an expert's tile takes thousands of workgroups whatever is split, and with K split
+// a wavefront worked through two blocks only, with nothing in flight behind them, and spent a fifth of its vector
+// instructions on partial sums. There a wavefront owns 32 columns over all of K (owned_tile()), its next block's codes in
+// flight, and four wavefronts share the activations a block at a time. Many small workgroups beat fewer that do more
+// (measured and not kept: eight wavefronts with K in halves, gate + up at 700 tokens 91 -> 123 us; four column groups a
+// workgroup over resident activations, down 70 -> 74).
 //
-// Measured (us, before -> now): 12288 x 2048 Q4_K at 64 rows 29.5 -> 15.8, 2048 x 4096 at 64 rows 52 -> 11.8,
-// 256 x 2048 Q6_K 28.6 -> 7.1; the experts of a 51-token prompt, gate + up + swiglu 104 -> 54 (193 MB from memory),
-// down 49 -> 36.5 (142 MB), of a 700-token one 156 -> 122 and 76 -> 82 (the shared expert included); a
-// 600-token prompt over 4-bit affine weights 461 ms -> 15.9 ms (its experts and projections were mat-vecs,
-// row by row).
+// What bounds the expert forms is vector issue beside the stream (700 tokens, gate + up: vector units 68 % of the time,
+// matrix cores 15 %, 4.5 TB/s; with every expert's weights in L2 the launch still takes 80 of its 90 us). The codes' way to
+// operands is 18 instructions for eight weights (scaled()). The plain launches of a short prompt are one pass of a
+// chain: load, unpack, multiply, meet (vector units 13 %).
 //
-// The order of the sums depends on K alone (256-wide blocks: wavefront ks takes blocks ks, ks + KS,
-// ...; the partial sums are added in one order), never on M, O or the launch's other matrices.
+// Measured (us, before -> now): 12288 x 2048 Q4_K at 64 rows 29.5 -> 15.8 -> 14.8, 2048 x 4096 at 64 rows 52 -> 11.8,
+// 256 x 2048 Q6_K 28.6 -> 7.1; the experts, gate + up + swiglu / down (the shared expert included): a 51-token prompt
+// 104 / 49 -> 53 / 36 with K split -> 47 / 38 with columns owned, a 700-token one 156 / 76 -> 122 / 81 -> 90 / 69, over 4-bit
+// affine weights at 600 tokens 109 / 62 -> 98 / 51; a 600-token prompt over 4-bit affine weights as a whole 461 ms
+// (mat-vecs, row by row) -> 15.9 -> 14.8 ms.
+//
+// The order of the sums depends on K alone, never on M, O or the launch's other matrices: plain, 256-wide blocks,
+// wavefront ks takes blocks ks, ks + KS, ... and the partial sums are added in one order; expert forms, all blocks in turn.
 //
 // Weight formats:
 //   Q4_K, Q6_K        dequantized with kquant::dequantize's arithmetic and rounded to bf16, as in
@@ -40,8 +47,8 @@
 //   affine 4 / 8 bit  the codes are exact bf16 numbers and go to the matrix cores as they are; the
 //                     sum over a group (32 / 64 k, one / two MFMAs) is multiplied by the group's
 //                     scale in fp32, and the bias meets the group's sum of activations, which the
-//                     same matrix core makes from a column of ones. No weight is rounded: the
-//                     arithmetic is that of the mat-vec (linear.hip), summed in another order.
+//                     matrix core makes from ones, four groups at a time in an fp32 product. No weight
+//                     is rounded: the arithmetic is that of the mat-vec (linear.hip), summed in another order.
 #pragma once
 
 #include <type_traits>
@@ -82,6 +89,8 @@ struct Args {
   const uint32_t* tile_count;
   const uint32_t* n_tiles;
   int up_div, pairs, E;
+  uint32_t up_magic;  // 2^32 / up_div rounded up: the upper half of its product with a pair is pair / up_div
+  int tiles_max, blocks;  // room in the tile list; column blocks a tile
 };
 
 // bytes of a 256-weight block in the three tensors
@@ -119,6 +128,13 @@ __device__ __forceinline__ void wait_loads() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
+// a barrier that leaves loads in flight
+__device__ __forceinline__ void barrier_only() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
 // ---- weight tiles: 16 weight rows x 256 k, lane (c = lane & 15, q = lane >> 4) ------------------
 // A block is eight k steps of 32, two to an activation chunk u. A chunk row has eight 16-byte slots of
 // eight k: lane q reads slot<H>(q) for step 2 u + H, and slot s of chunk u is piece(u, s) of the block's
@@ -131,12 +147,34 @@ __device__ __forceinline__ bf16x8_t as_frag(uint32_t a, uint32_t b, uint32_t c, 
   const u32x4_t v = {a, b, c, d};
   return __builtin_bit_cast(bf16x8_t, v);
 }
-// w = s * code + o of eight codes (bytes), rounded to bf16
-__device__ __forceinline__ bf16x8_t scaled(uint32_t c0, uint32_t c1, float s, float o) {
-  return as_frag(dm_f2bf2(dm_fma(s, dm_ubyte<0>(c0), o), dm_fma(s, dm_ubyte<1>(c0), o)),
-                 dm_f2bf2(dm_fma(s, dm_ubyte<2>(c0), o), dm_fma(s, dm_ubyte<3>(c0), o)),
-                 dm_f2bf2(dm_fma(s, dm_ubyte<0>(c1), o), dm_fma(s, dm_ubyte<1>(c1), o)),
-                 dm_f2bf2(dm_fma(s, dm_ubyte<2>(c1), o), dm_fma(s, dm_ubyte<3>(c1), o)));
+// s * h + o with h the lower (HI = 0) or upper 16 bits of w as an f16 number: one instruction, one rounding
+template <int HI>
+__device__ __forceinline__ float fma_half(float s, uint32_t w, float o) {
+  float r;
+  if constexpr (HI)
+    asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel:[0,1,0] op_sel_hi:[0,1,0]" : "=v"(r) : "v"(s), "v"(w), "v"(o));
+  else
+    asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel:[0,0,0] op_sel_hi:[0,1,0]" : "=v"(r) : "v"(s), "v"(w), "v"(o));
+  return r;
+}
+// w >> N (N < 0: w << -N). TAG makes it another instruction in every step that wants it: merged into one, the shifted words of a
+// block would be kept from step to step (a hundred registers spilled).
+template <int N, int TAG>
+__device__ __forceinline__ uint32_t shifted(uint32_t w) {
+  uint32_t r;
+  if constexpr (N >= 0)
+    asm("v_lshrrev_b32 %0, %1, %2 ; %3" : "=v"(r) : "n"(N), "v"(w), "n"(TAG));
+  else
+    asm("v_lshlrev_b32 %0, %1, %2 ; %3" : "=v"(r) : "n"(-N), "v"(w), "n"(TAG));
+  return r;
+}
+// w = s * code + o of eight codes, rounded to bf16. A code of up to ten bits at the bottom of a half is, read as a
+// (subnormal) f16 number, code * 2^-24, and four bits up code * 2^-20: no conversion, two codes a mask. s comes
+// multiplied by the 2^24 or 2^20, which loses nothing, so the fma's product is the code's times the scale's, bit for bit.
+// e0 / e1: codes 0, 2 and 4, 6; o0 / o1: codes 1, 3 and 5, 7.
+__device__ __forceinline__ bf16x8_t scaled(uint32_t e0, uint32_t o0, uint32_t e1, uint32_t o1, float s, float o) {
+  return as_frag(dm_f2bf2(fma_half<0>(s, e0, o), fma_half<0>(s, o0, o)), dm_f2bf2(fma_half<1>(s, e0, o), fma_half<1>(s, o0, o)),
+                 dm_f2bf2(fma_half<0>(s, e1, o), fma_half<0>(s, o1, o)), dm_f2bf2(fma_half<1>(s, e1, o), fma_half<1>(s, o1, o)));
 }
 
 // Q4_K: lane q takes pieces q (steps 0 - 3) and q + 4 of the block's eight 16-byte code pieces; piece
@@ -145,40 +183,46 @@ __device__ __forceinline__ bf16x8_t scaled(uint32_t c0, uint32_t c1, float s, fl
 template <>
 struct Tile<kQ4K> {
   static constexpr bool kAffine = false;
-  static constexpr int kSteps = 1;
-  u32x4_t w[2];
+  static constexpr int kSteps = 1, kLoads = 2;
+  struct Codes {
+    u32x4_t w[2];
+  } t;
+  float dd, nm;     // d * 2^24, -dmin
+  uint32_t sm;      // scales (low bytes) and minima of the half's two sub-blocks of this lane
   float s, o;
   static __device__ __forceinline__ int piece(int u, int slot) {
     return 16 * (u >> 1) + 4 * (u & 1) + 8 * (slot >> 2) + (slot & 3);
   }
+  static constexpr int half_bytes() { return 256; }  // from chunk u's pieces to chunk u + 2's
   template <int H>
   static __device__ __forceinline__ int slot(int q) { return 2 * q + H; }
-  __device__ __forceinline__ void load(const uint8_t* cq, uint32_t blk, int q) {
-    w[0] = ld_off<u32x4_t>(cq, blk * q_bytes(kQ4K) + 16 * q);
-    w[1] = ld_off<u32x4_t>(cq + 64, blk * q_bytes(kQ4K) + 16 * q);
+  static __device__ __forceinline__ void load(Codes& t, const uint8_t* cq, uint32_t blk, int q) {
+    t.w[0] = ld_off<u32x4_t>(cq, blk * q_bytes(kQ4K) + 16 * q);
+    t.w[1] = ld_off<u32x4_t>(cq + 64, blk * q_bytes(kQ4K) + 16 * q);
   }
   // sub-block 4 (u >> 1) + 2 (q >> 1) + (u & 1) of the block whose scales are at ls / ld in LDS
   template <int U>
   __device__ __forceinline__ void scales(const uint8_t* ls, const uint8_t* ld, int q) {
     const uint32_t* sc = reinterpret_cast<const uint32_t*>(ls);
-    const int sh = 16 * (q >> 1) + 8 * (U & 1);
-    uint32_t sb, mb;
-    if constexpr (U < 2) {
-      sb = (sc[0] >> sh) & 63u;
-      mb = (sc[1] >> sh) & 63u;
-    } else {
-      const uint32_t t = sc[2] >> sh;
-      sb = (t & 15u) | (((sc[0] >> sh) >> 2) & 0x30u);
-      mb = ((t >> 4) & 15u) | (((sc[1] >> sh) >> 2) & 0x30u);
+    const uint32_t pick = q >> 1 ? 0x07060302u : 0x05040100u;
+    if constexpr (U == 0) {
+      const uint32_t dmw = *reinterpret_cast<const uint32_t*>(ld);
+      dd = dm_h2f((f16_t)(dmw & 0xffffu)) * 16777216.f;
+      nm = -dm_h2f((f16_t)(dmw >> 16));
+      sm = __builtin_amdgcn_perm(sc[1], sc[0], pick) & 0x3f3f3f3fu;
     }
-    const uint32_t dmw = *reinterpret_cast<const uint32_t*>(ld);
-    s = dm_h2f((f16_t)(dmw & 0xffffu)) * (float)sb;
-    o = -(dm_h2f((f16_t)(dmw >> 16)) * (float)mb);
+    if constexpr (U == 2)
+      sm = __builtin_amdgcn_perm((sc[2] >> 4) & 0x0f0f0f0fu, sc[2] & 0x0f0f0f0fu, pick) |
+           ((__builtin_amdgcn_perm(sc[1], sc[0], pick) >> 2) & 0x30303030u);
+    // (the odd chunks hold the high nibbles, whose codes lie four bits up)
+    s = ((U & 1) ? dd * 0.0625f : dd) * dm_ubyte<(U & 1)>(sm);
+    o = nm * dm_ubyte<2 + (U & 1)>(sm);
   }
   template <int S>
   __device__ __forceinline__ bf16x8_t frag() const {
-    constexpr int NIB = (S >> 1) & 1, W = 2 * (S & 1);
-    return scaled((w[S >> 2][W] >> (4 * NIB)) & 0x0f0f0f0fu, (w[S >> 2][W + 1] >> (4 * NIB)) & 0x0f0f0f0fu, s, o);
+    constexpr uint32_t M = ((S >> 1) & 1) ? 0x00f000f0u : 0x000f000fu;
+    const uint32_t a = t.w[S >> 2][2 * (S & 1)], b = t.w[S >> 2][2 * (S & 1) + 1];
+    return scaled(a & M, shifted<8, S>(a) & M, b & M, shifted<8, S>(b) & M, s, o);
   }
 };
 
@@ -187,31 +231,38 @@ struct Tile<kQ4K> {
 template <>
 struct Tile<kQ6K> {
   static constexpr bool kAffine = false;
-  static constexpr int kSteps = 1;
-  u32x4_t la, lb, h;
+  static constexpr int kSteps = 1, kLoads = 3;
+  struct Codes {
+    u32x4_t la, lb, h;
+  } t;
   float s, o;
   static __device__ __forceinline__ int piece(int u, int slot) { return 16 * (slot >> 2) + 4 * u + (slot & 3); }
+  static constexpr int half_bytes() { return 128; }
   template <int H>
   static __device__ __forceinline__ int slot(int q) { return 2 * q + H; }
-  __device__ __forceinline__ void load(const uint8_t* cq, uint32_t blk, int q) {
+  static __device__ __forceinline__ void load(Codes& t, const uint8_t* cq, uint32_t blk, int q) {
     const uint32_t at = blk * q_bytes(kQ6K) + 64 * (q >> 1) + 16 * (q & 1);
-    la = ld_off<u32x4_t>(cq, at);
-    lb = ld_off<u32x4_t>(cq + 32, at);
-    h = ld_off<u32x4_t>(cq + 128, blk * q_bytes(kQ6K) + 16 * q);
+    t.la = ld_off<u32x4_t>(cq, at);
+    t.lb = ld_off<u32x4_t>(cq + 32, at);
+    t.h = ld_off<u32x4_t>(cq + 128, blk * q_bytes(kQ6K) + 16 * q);
   }
   // scale 8 (q >> 1) + 2 u + (q & 1) of the block's sixteen
   template <int U>
   __device__ __forceinline__ void scales(const uint8_t* ls, const uint8_t* ld, int q) {
     const int8_t sc = (int8_t)ls[8 * (q >> 1) + 2 * U + (q & 1)];
-    s = dm_h2f(*reinterpret_cast<const f16_t*>(ld)) * (float)(int)sc;
-    o = -32.f * s;
+    const float v = dm_h2f(*reinterpret_cast<const f16_t*>(ld)) * (float)(int)sc;
+    s = v * (U < 2 ? 16777216.f : 1048576.f);
+    o = -32.f * v;
   }
+  // quarters 0 and 1 are low nibbles (the codes lie at the bottom of their halves), 2 and 3 high ones (four bits up)
   template <int S>
   __device__ __forceinline__ bf16x8_t frag() const {
-    constexpr int QD = S >> 1, NIB = QD >> 1, W = 2 * (S & 1);
-    const u32x4_t& lo = (QD & 1) ? lb : la;
-    return scaled(((lo[W] >> (4 * NIB)) & 0x0f0f0f0fu) | (((h[W] >> (2 * QD)) & 0x03030303u) << 4),
-                  ((lo[W + 1] >> (4 * NIB)) & 0x0f0f0f0fu) | (((h[W + 1] >> (2 * QD)) & 0x03030303u) << 4), s, o);
+    constexpr int QD = S >> 1, NIB = QD >> 1, W = 2 * (S & 1), SH = 4 - 2 * (QD & 1);
+    constexpr uint32_t M = NIB ? 0x00f000f0u : 0x000f000fu, MH = NIB ? 0x03000300u : 0x00300030u;
+    const u32x4_t& lo = (QD & 1) ? t.lb : t.la;
+    const uint32_t a = lo[W], b = lo[W + 1], ha = t.h[W], hb = t.h[W + 1];
+    return scaled((a & M) | (shifted<-SH, S>(ha) & MH), (shifted<8, S>(a) & M) | (shifted<8 - SH, S>(ha) & MH), (b & M) | (shifted<-SH, S>(hb) & MH),
+                  (shifted<8, S>(b) & M) | (shifted<8 - SH, S>(hb) & MH), s, o);
   }
 };
 
@@ -238,43 +289,43 @@ __device__ __forceinline__ void swap_rows(uint32_t& a, uint32_t& b) {
 template <>
 struct Tile<kA4> {
   static constexpr bool kAffine = true;
-  static constexpr int kSteps = 1;  // k steps a group
-  u32x4_t t[2];                     // word q of groups 4 i + g
-  u32x4_t sc, bi;                   // the block's eight scales and biases, two to a word
+  static constexpr int kSteps = 1, kLoads = 2;  // k steps a group
+  struct Codes {
+    u32x4_t t[2];  // word q of groups 4 i + g
+  } t;
+  u32x4_t sc;  // the block's eight scales, two to a word
   static __device__ __forceinline__ int piece(int u, int slot) { return 8 * u + slot; }
+  static constexpr int half_bytes() { return 256; }
   template <int H>
   static __device__ __forceinline__ int slot(int q) { return 4 * H + q; }
-  __device__ __forceinline__ void load(const uint8_t* cq, uint32_t blk, int q) {
+  static __device__ __forceinline__ void load(Codes& t, const uint8_t* cq, uint32_t blk, int q) {
     // whole groups (16 bytes): lane q holds group 4 i + q
-    t[0] = ld_off<u32x4_t>(cq, blk * q_bytes(kA4) + 16 * q);
-    t[1] = ld_off<u32x4_t>(cq + 64, blk * q_bytes(kA4) + 16 * q);
+    t.t[0] = ld_off<u32x4_t>(cq, blk * q_bytes(kA4) + 16 * q);
+    t.t[1] = ld_off<u32x4_t>(cq + 64, blk * q_bytes(kA4) + 16 * q);
   }
   // word g of group q -> word q of group g: the 4 x 4 transpose over the lanes of a column
   template <int I>
   __device__ __forceinline__ void transpose() {
-    uint32_t a = t[I][0], b = t[I][1], c = t[I][2], d = t[I][3];
+    uint32_t a = t.t[I][0], b = t.t[I][1], c = t.t[I][2], d = t.t[I][3];
     swap_rows<32>(a, c);
     swap_rows<32>(b, d);
     swap_rows<16>(a, b);
     swap_rows<16>(c, d);
-    t[I] = u32x4_t{a, b, c, d};
+    t.t[I] = u32x4_t{a, b, c, d};
   }
   template <int U>
-  __device__ __forceinline__ void scales(const uint8_t* ls, const uint8_t* ld, int) {
+  __device__ __forceinline__ void scales(const uint8_t* ls, const uint8_t*, int) {
     if constexpr (U == 0) {
       transpose<0>();
       sc = *reinterpret_cast<const u32x4_t*>(ls);
-      bi = *reinterpret_cast<const u32x4_t*>(ld);
     }
     if constexpr (U == 2) transpose<1>();
   }
   template <int S>
   __device__ __forceinline__ float scale() const { return (S & 1) ? dm_bf2f_hi(sc[S >> 1]) : dm_bf2f_lo(sc[S >> 1]); }
   template <int S>
-  __device__ __forceinline__ float bias() const { return (S & 1) ? dm_bf2f_hi(bi[S >> 1]) : dm_bf2f_lo(bi[S >> 1]); }
-  template <int S>
   __device__ __forceinline__ bf16x8_t frag() const {
-    const uint32_t w = t[S >> 2][S & 3];
+    const uint32_t w = t.t[S >> 2][S & 3];
     const uint32_t even = w & 0x0f0f0f0fu, odd = (w >> 4) & 0x0f0f0f0fu;
     // codes 0 1 2 3 and 4 5 6 7 as bytes
     const uint32_t a = __builtin_amdgcn_perm(odd, even, 0x05010400u), b = __builtin_amdgcn_perm(odd, even, 0x07030602u);
@@ -286,30 +337,28 @@ struct Tile<kA4> {
 template <>
 struct Tile<kA8> {
   static constexpr bool kAffine = true;
-  static constexpr int kSteps = 2;
-  u32x2_t w[8];
-  u32x2_t sc, bi;  // the block's four scales and biases
+  static constexpr int kSteps = 2, kLoads = 8;
+  struct Codes {
+    u32x2_t w[8];
+  } t;
+  u32x2_t sc;  // the block's four scales
   static __device__ __forceinline__ int piece(int u, int slot) { return 8 * u + slot; }
+  static constexpr int half_bytes() { return 256; }
   template <int H>
   static __device__ __forceinline__ int slot(int q) { return 4 * H + q; }
-  __device__ __forceinline__ void load(const uint8_t* cq, uint32_t blk, int q) {
+  static __device__ __forceinline__ void load(Codes& t, const uint8_t* cq, uint32_t blk, int q) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) w[i] = ld_off<u32x2_t>(cq + 32 * i, blk * q_bytes(kA8) + 8 * q);
+    for (int i = 0; i < 8; ++i) t.w[i] = ld_off<u32x2_t>(cq + 32 * i, blk * q_bytes(kA8) + 8 * q);
   }
   template <int U>
-  __device__ __forceinline__ void scales(const uint8_t* ls, const uint8_t* ld, int) {
-    if constexpr (U == 0) {
-      sc = *reinterpret_cast<const u32x2_t*>(ls);
-      bi = *reinterpret_cast<const u32x2_t*>(ld);
-    }
+  __device__ __forceinline__ void scales(const uint8_t* ls, const uint8_t*, int) {
+    if constexpr (U == 0) sc = *reinterpret_cast<const u32x2_t*>(ls);
   }
   template <int S>
   __device__ __forceinline__ float scale() const { return (S & 2) ? dm_bf2f_hi(sc[S >> 2]) : dm_bf2f_lo(sc[S >> 2]); }
   template <int S>
-  __device__ __forceinline__ float bias() const { return (S & 2) ? dm_bf2f_hi(bi[S >> 2]) : dm_bf2f_lo(bi[S >> 2]); }
-  template <int S>
   __device__ __forceinline__ bf16x8_t frag() const {  // 0 .. 255 are bf16 numbers
-    const uint32_t a = w[S][0], b = w[S][1];
+    const uint32_t a = t.w[S][0], b = t.w[S][1];
     return as_frag(dm_f2bf2(dm_ubyte<0>(a), dm_ubyte<1>(a)), dm_f2bf2(dm_ubyte<2>(a), dm_ubyte<3>(a)),
                    dm_f2bf2(dm_ubyte<0>(b), dm_ubyte<1>(b)), dm_f2bf2(dm_ubyte<2>(b), dm_ubyte<3>(b)));
   }
@@ -317,11 +366,13 @@ struct Tile<kA8> {
 
 // ---- one wavefront's share: RT x CT tiles of 16 x 16 over its K blocks ----------------------------
 // NB: activation chunks (2 KB * RT each) its part of LDS holds
-template <int KIND, int RT, int CT, int NB>
+// PF: the codes of the wavefront's next block are asked for while it works on this one (plain form)
+template <int KIND, int RT, int CT, int NB, bool PF>
 struct Work {
   typedef Tile<KIND> T;
   f32x4_t acc[RT][CT];
   T t[CT];
+  float sx[RT];           // affine: the row's sum over group (its lane quarter) of the last four groups
   uint32_t ls0, ld0;      // LDS offsets of the scales of the lane's row of tile 0
   uint32_t ls_[CT], ld_[CT];  // ... of the other tiles from there (the same for every lane)
 
@@ -353,17 +404,22 @@ struct Work {
         for (int r = 0; r < RT; ++r) acc[r][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[r], b, acc[r][j], 0, 0, 0);
       }
     } else if constexpr (S % T::kSteps == 0) {
-      constexpr int N = T::kSteps;
+      constexpr int N = T::kSteps, G = S / N;  // group of the block
       const bf16x8_t ones = as_frag(0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u);
       const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
       bf16x8_t a1[RT];
-      f32x4_t sx[RT];  // the rows' sums over the group, in every column
       read(std::integral_constant<int, H>{}, a);
       if constexpr (N == 2) read(std::integral_constant<int, 1>{}, a1);
+      // the rows' sums over the group: ones times the activations' transpose puts row c's into lane c of every
+      // quarter, and quarter q keeps group q's, which is the operand layout of the fp32 product below
 #pragma unroll
       for (int r = 0; r < RT; ++r) {
-        sx[r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[r], ones, zero, 0, 0, 0);
-        if constexpr (N == 2) sx[r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1[r], ones, sx[r], 0, 0, 0);
+        f32x4_t v = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, a[r], zero, 0, 0, 0);
+        if constexpr (N == 2) v = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, a1[r], v, 0, 0, 0);
+        sx[r] = q == (G & 3) ? v[0] : sx[r];
+        // (v's other elements stay taken until its product has ended: their registers would go to the unpacking's inline
+        // assembly at once, which the compiler does not hold back for a matrix instruction in flight)
+        asm volatile("" : "+v"(sx[r]) : "v"(v));
       }
 #pragma unroll
       for (int j = 0; j < CT; ++j) {
@@ -380,54 +436,156 @@ struct Work {
 #pragma unroll
         for (int r = 0; r < RT; ++r)
 #pragma unroll
-          for (int e = 0; e < 4; ++e)
-            acc[r][j][e] = dm_fma(t[j].template scale<S>(), g[r][e], dm_fma(t[j].template bias<S>(), sx[r][e], acc[r][j][e]));
+          for (int e = 0; e < 4; ++e) acc[r][j][e] = dm_fma(t[j].template scale<S>(), g[r][e], acc[r][j][e]);
+      }
+      // the biases of four groups against the rows' sums over them, fp32 on the matrix cores (an fma an
+      // element and group beside the scale's was a third of the vector work)
+      if constexpr ((G & 3) == 3) {
+#pragma unroll
+        for (int j = 0; j < CT; ++j) {
+          const float bias = dm_bf2f(*reinterpret_cast<const bf16_t*>(smem + ld0 + ld_[j] + 2 * ((G & 4) + q)));
+#pragma unroll
+          for (int r = 0; r < RT; ++r) acc[r][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(sx[r], bias, acc[r][j], 0, 0, 0);
+        }
       }
     }
     // (or the scheduler dequantizes the whole block ahead, and spills)
     __builtin_amdgcn_sched_barrier(0);
   }
-  // x, xo: the activations and the byte offsets of the rows this lane fetches; code: the two halves'
-  // codes (GC column tiles each); row0: the lane's weight row of tile 0, O: their number; xs / lds:
-  // this wavefront's activation buffers; first(): what has to be done before the first block's arithmetic
-  template <int GC, class F>
-  __device__ __forceinline__ void run(const uint8_t* const (&code)[2], int row0, int O, const bf16_t* x,
-                                      const uint32_t (&xo)[2 * RT], int nb, int ks, int KS, int lane, const uint8_t* smem,
-                                      const uint8_t* xs, uint32_t lds, F first) {
+  // codes of block ib of weight row `row` of O
+  static __device__ __forceinline__ void load(typename T::Codes& d, const uint8_t* code, int row, int O, int ib, int nb, int q) {
+    T::load(d, code + (size_t)ib * q_bytes(KIND), (uint32_t)min(row, O - 1) * (uint32_t)nb, q);
+  }
+  // the first block's codes, ahead of what the activations' addresses wait for. code: of the two matrices (GC column
+  // tiles each); row0: the lane's weight row of tile 0
+  template <int GC>
+  __device__ __forceinline__ void start(const uint8_t* const (&code)[CT / GC], int row0, int O, int nb, int ks, int lane) {
+#pragma unroll
+    for (int j = 0; j < CT; ++j) load(t[j].t, code[j / GC], row0 + 16 * (j % GC), O, ks, nb, lane >> 4);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  // The plain form: one block, with two chunks and the codes of it asked for. MORE: the wavefront has another one, KS blocks
+  // on; its codes go out here behind this block's activations (which are waited for one by one), its activations as
+  // this block's buffers come free.
+  template <int GC, bool MORE, class F>
+  __device__ __forceinline__ void block(const uint8_t* code, int row0, int O, const uint8_t* xk, const uint32_t (&xo)[2 * RT], int ib,
+                                        int nb, int KS, int lane, const uint8_t* smem, const uint8_t* xs, uint32_t lds, F first) {
+    static_assert(NB == 2, "two chunks in flight");
     const int c = lane & 15, q = lane >> 4;
+    constexpr bool AHEAD = MORE && PF;
+    constexpr int NL = AHEAD ? CT * T::kLoads : 0;
+    const uint8_t* const xn = xk + (size_t)KS * 512;
+    typename T::Codes next[CT];
+    wait_loads<0>();
+    first();
+    step<0>(smem, xs, c, q);
+    step<1>(smem, xs, c, q);
+    fetch<2>(xk, xo, lds, lane);
+    step<2>(smem, xs, c, q);
+    step<3>(smem, xs, c, q);
+    fetch<3>(xk, xo, lds, lane);
+    if constexpr (AHEAD) {
 #pragma unroll
-    for (int r = 0; r < RT; ++r)
+      for (int j = 0; j < CT; ++j) load(next[j], code, row0 + 16 * j, O, ib + KS, nb, q);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    wait_loads<2 * RT + NL>();
+    step<4>(smem, xs, c, q);
+    step<5>(smem, xs, c, q);
+    if constexpr (MORE) fetch<0>(xn, xo, lds, lane);
+    wait_loads<NL + (MORE ? 2 * RT : 0)>();
+    step<6>(smem, xs, c, q);
+    step<7>(smem, xs, c, q);
+    if constexpr (MORE) {
+      fetch<1>(xn, xo, lds, lane);
 #pragma unroll
-      for (int j = 0; j < CT; ++j) acc[r][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    for (int ib = ks; ib < nb; ib += KS) {
-      const uint8_t* xk = reinterpret_cast<const uint8_t*>(x) + (size_t)ib * 512;
-      fetch<0>(xk, xo, lds, lane);
-      fetch<1>(xk, xo, lds, lane);
-      if constexpr (NB == 4) {
-        fetch<2>(xk, xo, lds, lane);
-        fetch<3>(xk, xo, lds, lane);
+      for (int j = 0; j < CT; ++j) {
+        if constexpr (PF) t[j].t = next[j];
+        else load(t[j].t, code, row0 + 16 * j, O, ib + KS, nb, q);
       }
-#pragma unroll
-      for (int j = 0; j < CT; ++j) t[j].load(code[j / GC] + (size_t)ib * q_bytes(KIND), (uint32_t)min(row0 + 16 * (j % GC), O - 1) * (uint32_t)nb, q);
-      wait_loads<0>();
-      if (ib == ks) first();
-      step<0>(smem, xs, c, q);
-      step<1>(smem, xs, c, q);
-      if constexpr (NB == 2) fetch<2>(xk, xo, lds, lane);
-      step<2>(smem, xs, c, q);
-      step<3>(smem, xs, c, q);
-      if constexpr (NB == 2) {
-        fetch<3>(xk, xo, lds, lane);
-        wait_loads<2 * RT>();
-      }
-      step<4>(smem, xs, c, q);
-      step<5>(smem, xs, c, q);
-      if constexpr (NB == 2) wait_loads<0>();
-      step<6>(smem, xs, c, q);
-      step<7>(smem, xs, c, q);
       ls0 += KS * s_bytes(KIND);
       ld0 += KS * d_bytes(KIND);
     }
+  }
+  // The form whose wavefronts own columns: every one works through all of K, a block at a time, and the workgroup's four
+  // share the block's activations, chunk U at xs + U * RT * 2 KB. They come in two chunks a piece (wavefront `wave` fetches
+  // half the rows of chunk `wave & 1` of a half block: xo, lds) or whole blocks (chunk `wave`):
+  //   whole blocks in two buffers, each asked for a block ahead;
+  //   HALF: half blocks in the halves of one buffer, each asked for half a block ahead.
+  // MORE: the next block's activations and codes go out here.
+  __device__ __forceinline__ static void ask_block(const uint8_t* x, const uint32_t (&xo)[2 * RT], uint32_t lds) {
+#pragma unroll
+    for (int i = 0; i < 2 * RT; ++i) dma16(x, xo[i], lds + i * 1024);
+  }
+  __device__ __forceinline__ static void ask_half(const uint8_t* x, const uint32_t (&xo)[2 * RT], int half, uint32_t lds) {
+#pragma unroll
+    for (int i = 0; i < RT; ++i) dma16(x + half * T::half_bytes(), xo[i], lds + half * (RT * 4096) + i * 1024);
+  }
+  template <int GC, bool HALF, bool FIRST, bool MORE>
+  __device__ __forceinline__ void owned_block(const uint8_t* const (&code)[CT / GC], int row0, int O, const uint8_t* x,
+                                              const uint32_t (&xo)[2 * RT], int ib, int nb, int lane, const uint8_t* smem,
+                                              const uint8_t* xs, uint32_t lds) {
+    const int c = lane & 15, q = lane >> 4;
+    typename T::Codes next[CT];
+    auto ask_codes = [&]() {
+#pragma unroll
+      for (int j = 0; j < CT; ++j) load(next[j], code[j / GC], row0 + 16 * (j % GC), O, ib + 1, nb, q);
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    const int buf = HALF ? 0 : (ib & 1) * (RT * 8192);
+    // this block's activations (their first half) were asked for ahead of its codes
+    wait_loads<FIRST ? 0 : CT * T::kLoads>();
+    barrier_only();
+    if constexpr (HALF) {
+      ask_half(x, xo, 1, lds);
+    } else if constexpr (MORE) {
+      ask_block(x + 512, xo, lds + ((ib + 1) & 1) * (RT * 8192));
+      ask_codes();
+    }
+    step<0>(smem, xs + buf, c, q);
+    step<1>(smem, xs + buf, c, q);
+    step<2>(smem, xs + buf, c, q);
+    step<3>(smem, xs + buf, c, q);
+    if constexpr (HALF) {
+      wait_loads<0>();
+      barrier_only();
+      if constexpr (MORE) {
+        ask_half(x + 512, xo, 0, lds);
+        ask_codes();
+      }
+    }
+    step<4>(smem, xs + buf, c, q);
+    step<5>(smem, xs + buf, c, q);
+    step<6>(smem, xs + buf, c, q);
+    step<7>(smem, xs + buf, c, q);
+    if constexpr (MORE) {
+#pragma unroll
+      for (int j = 0; j < CT; ++j) t[j].t = next[j];
+    }
+  }
+  __device__ __forceinline__ void clear() {
+#pragma unroll
+    for (int r = 0; r < RT; ++r) {
+      sx[r] = 0.f;
+#pragma unroll
+      for (int j = 0; j < CT; ++j) acc[r][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    }
+  }
+  // x, xo: the activations and the byte offsets of the rows this lane fetches; xs / lds: this wavefront's
+  // activation buffers; scales_here(): what has to be done before the first block's arithmetic. start() has been called.
+  template <class F>
+  __device__ __forceinline__ void run(const uint8_t* code, int row0, int O, const bf16_t* x, const uint32_t (&xo)[2 * RT], int nb, int ks,
+                                      int KS, int lane, const uint8_t* smem, const uint8_t* xs, uint32_t lds, F scales_here) {
+    clear();
+    const uint8_t* xk = reinterpret_cast<const uint8_t*>(x) + (size_t)ks * 512;
+    fetch<0>(xk, xo, lds, lane);
+    fetch<1>(xk, xo, lds, lane);
+    int ib = ks;
+    auto first = [&]() {
+      if (ib == ks) scales_here();
+    };
+    for (; ib + KS < nb; ib += KS, xk += (size_t)KS * 512) block<CT, true>(code, row0, O, xk, xo, ib, nb, KS, lane, smem, xs, lds, first);
+    block<CT, false>(code, row0, O, xk, xo, ib, nb, KS, lane, smem, xs, lds, first);
   }
 };
 
@@ -436,68 +594,53 @@ constexpr int kPad = 4;  // a row of a partial tile: 16 CT + 4 floats, so the fo
 
 // LDS of a workgroup: activation chunks of its NW wavefronts, then the scales of its rows; the
 // partial tiles go over both (host and device share the arithmetic)
-__host__ __device__ constexpr int chunks_held(int rows) { return rows <= 16 ? 4 : 2; }
-__host__ __device__ constexpr int x_bytes(int rows, int nw) { return nw * chunks_held(rows) * (rows / 16) * 2048; }
+__host__ __device__ constexpr int x_bytes(int rows, int nw) { return nw * 2 * (rows / 16) * 2048; }
 __host__ __device__ constexpr int red_bytes(int rows, int ct, int nw) { return nw / 2 * rows * (16 * ct + kPad) * 4; }
 
-// a workgroup's tile of up to 16 RT rows: partial products, their sums, the outputs
-template <int KIND, int RT, int CT, int MODE, int ROWS, int NW>
-__device__ __forceinline__ void tile_body(const Args& a, int mat0, int c0, int64_t row_base, int rows, int m0,
-                                          const uint32_t* my_pairs, uint8_t* smem) {
+// the plain form: a workgroup's tile of up to 16 RT rows (of ROWS): partial products, their sums, the outputs
+template <int KIND, int RT, int CT, int ROWS, int NW>
+__device__ __forceinline__ void tile_body(const Args& a, int mat, int c0, int rows, int m0, uint8_t* smem) {
   constexpr int SB = s_bytes(KIND), DB = d_bytes(KIND);
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), c = lane & 15, q = lane >> 4;
   const int KS = a.ks, nb = a.K >> 8;
   const int ks = wave & (KS - 1), cw = wave / KS;
-  constexpr int GC = MODE == kGateUp ? CT / 2 : CT;  // column tiles of one matrix a wavefront has
-  constexpr int LD = 16 * CT + kPad, HALVES = MODE == kGateUp ? 2 : 1, NB = chunks_held(ROWS);
-  const int O = a.m[mat0].O, cols = (NW / KS) * GC * 16;  // the workgroup's columns of one matrix
+  constexpr int LD = 16 * CT + kPad;
+  const Mat& m = a.m[mat];
+  const int O = m.O, cols = (NW / KS) * CT * 16;  // the workgroup's columns
   float* red = reinterpret_cast<float*>(smem);
 
-  // the scales of the workgroup's rows: one run of bytes in each tensor of each half (what would
-  // pass the matrix's end repeats its last 16 bytes: rows that are never stored)
+  // the scales of the workgroup's rows: one run of bytes in each tensor (what would pass the matrix's
+  // end repeats its last 16 bytes: rows that are never stored)
   const int s_len = cols * nb * SB, d_len = cols * nb * DB;
-  const uint8_t* code[2];
-#pragma unroll
-  for (int i = 0; i < HALVES; ++i) {
-    const Mat& m = a.m[mat0 + i];
-    code[i] = uniform(m.q + row_base * nb * q_bytes(KIND));
-    const uint8_t *gs = uniform(m.s + (row_base + c0) * nb * SB), *gd = uniform(m.d + (row_base + c0) * nb * DB);
+  const uint8_t* const code[1] = {uniform(m.q)};
+  {
+    const uint8_t *gs = uniform(m.s + (int64_t)c0 * nb * SB), *gd = uniform(m.d + (int64_t)c0 * nb * DB);
     const int s_end = (O - c0) * nb * SB - 16, d_end = (O - c0) * nb * DB - 16;
-    const uint32_t at = lds_address(smem + x_bytes(ROWS, NW)) + i * (s_len + d_len);
+    const uint32_t at = lds_address(smem + x_bytes(ROWS, NW));
     for (int p = wave * 1024; p < s_len; p += NW * 1024)
       if (p + 16 * lane < s_len) dma16(gs, (uint32_t)min(p + 16 * lane, s_end), at + p);
     for (int p = wave * 1024; p < d_len; p += NW * 1024)
       if (p + 16 * lane < d_len) dma16(gd, (uint32_t)min(p + 16 * lane, d_end), at + s_len + p);
   }
-  if constexpr (HALVES == 1) code[1] = code[0];
 
-  Work<KIND, RT, CT, NB> w;
-  const int lr = cw * GC * 16 + c;  // of tile 0, which of the workgroup's rows
+  // (the codes ahead where the registers hold two blocks of them)
+  Work<KIND, RT, CT, 2, (KIND == kQ4K || KIND == kA4) && RT <= 2> w;
+  const int lr = cw * CT * 16 + c;  // of tile 0, which of the workgroup's rows
+  w.template start<CT>(code, c0 + lr, O, nb, ks, lane);
   w.ls0 = x_bytes(ROWS, NW) + (lr * nb + ks) * SB;
   w.ld0 = x_bytes(ROWS, NW) + s_len + (lr * nb + ks) * DB;
 #pragma unroll
   for (int j = 0; j < CT; ++j) {
-    w.ls_[j] = (j / GC) * (s_len + d_len) + (j % GC) * 16 * nb * SB;
-    w.ld_[j] = (j / GC) * (s_len + d_len) + (j % GC) * 16 * nb * DB;
+    w.ls_[j] = j * 16 * nb * SB;
+    w.ld_[j] = j * 16 * nb * DB;
   }
-  // this lane fetches a piece of rows 8 i + (lane >> 3)
+  // this lane fetches a piece of rows 8 i + (lane >> 3); rows past the end read a valid row: what they produce is never stored
   uint32_t xo[2 * RT];
 #pragma unroll
-  for (int i = 0; i < 2 * RT; ++i) {
-    // rows past the end read a valid row: what they produce is never stored
-    const int r = 8 * i + (lane >> 3);
-    uint32_t src;
-    if constexpr (MODE == kPlain) {
-      src = (uint32_t)min(m0 + r, a.M - 1);
-    } else {
-      const uint32_t p = my_pairs[min(r, rows - 1)];
-      src = a.up_div == 1 ? p : (int)p < a.pairs ? p / (uint32_t)a.up_div : p - (uint32_t)a.pairs;
-    }
-    xo[i] = 2 * src * (uint32_t)a.K;
-  }
+  for (int i = 0; i < 2 * RT; ++i) xo[i] = 2 * (uint32_t)min(m0 + 8 * i + (lane >> 3), a.M - 1) * (uint32_t)a.K;
   const uint8_t* xs = smem + wave * (x_bytes(ROWS, NW) / NW);
-  w.template run<GC>(code, c0 + lr, O, a.x, xo, nb, ks, KS, lane, smem, xs, lds_address(xs),
-                     [&]() { __syncthreads(); });  // every wavefront's share of the scales has arrived
+  w.run(code[0], c0 + lr, O, a.x, xo, nb, ks, KS, lane, smem, xs, lds_address(xs),
+        [&]() { barrier_only(); });  // every wavefront's share of the scales has arrived (waited for by each)
   __syncthreads();
   // The partial tiles meet in LDS. First the upper half of the K split hands its registers to
   // the lower half as they are (16 bytes a lane), which halves what the second pass holds.
@@ -535,27 +678,14 @@ __device__ __forceinline__ void tile_body(const Args& a, int mat0, int c0, int64
   const int n = rows * quads;
   for (int i = tid; i < n; i += 64 * NW) {
     const int row = i / quads, c4 = i - row * quads;
-    const int w0 = (c4 / (4 * GC)) * HS, lc = 4 * (c4 % (4 * GC));
+    const int w0 = (c4 / (4 * CT)) * HS, lc = 4 * (c4 % (4 * CT));
     const float* p = red + (w0 * ROWS + row) * LD + lc;
-    f32x4_t v = *reinterpret_cast<const f32x4_t*>(p), u;
+    f32x4_t v = *reinterpret_cast<const f32x4_t*>(p);
     for (int k = 1; k < HS; ++k) v += *reinterpret_cast<const f32x4_t*>(p + k * ROWS * LD);
-    if constexpr (MODE == kGateUp) {
-      u = *reinterpret_cast<const f32x4_t*>(p + 16 * GC);
-      for (int k = 1; k < HS; ++k) u += *reinterpret_cast<const f32x4_t*>(p + 16 * GC + k * ROWS * LD);
-    }
     const int col = c0 + 4 * c4;
     if (col >= O) continue;
-    int64_t dst = m0 + row;
-    if constexpr (MODE != kPlain) dst = my_pairs[row];
-    bf16_t* y = a.m[mat0].y + dst * O + col;
-    u32x2_t o;
-    if constexpr (MODE == kGateUp) {
-      o[0] = (uint32_t)swiglu_bf16(v[0], u[0]) | ((uint32_t)swiglu_bf16(v[1], u[1]) << 16);
-      o[1] = (uint32_t)swiglu_bf16(v[2], u[2]) | ((uint32_t)swiglu_bf16(v[3], u[3]) << 16);
-    } else {
-      o[0] = dm_f2bf2(v[0], v[1]);
-      o[1] = dm_f2bf2(v[2], v[3]);
-    }
+    bf16_t* y = m.y + (int64_t)(m0 + row) * O + col;
+    const u32x2_t o = {dm_f2bf2(v[0], v[1]), dm_f2bf2(v[2], v[3])};
     if ((O & 3) == 0) {
       *reinterpret_cast<u32x2_t*>(y) = o;
     } else {  // (rows of y are not 8-byte aligned, and the last quad may be ragged)
@@ -567,13 +697,109 @@ __device__ __forceinline__ void tile_body(const Args& a, int mat0, int c0, int64
   }
 }
 
-// AFF: affine formats, else k-quants. NW wavefronts, grid (column blocks, row tiles), K >= 512.
-template <bool AFF, int CT, int MODE, int ROWS, int NW>
+// The gathered forms. A tile (an expert's up to 16 RT rows) takes four wavefronts a column block; each owns columns, 16 of gate
+// and of up or 32 of one matrix, over all of K, its codes a block ahead in registers, so nothing has to meet at the end.
+__host__ __device__ constexpr bool owned_half(int kind, int mode) { return kind == kA4 && mode == kGateUp; }
+__host__ __device__ constexpr int owned_x_bytes(int rows, int kind, int mode) { return rows * (owned_half(kind, mode) ? 512 : 1024); }
+template <int KIND, int RT, int MODE>
+__device__ __forceinline__ void owned_tile(const Args& a, int mat0, int c0, int64_t row_base, int rows, const uint32_t* my_pairs,
+                                           uint8_t* smem) {
+  constexpr int SB = s_bytes(KIND), DB = d_bytes(KIND), CT = 2, HALVES = MODE == kGateUp ? 2 : 1, GC = CT / HALVES;
+  // (8-bit and k-quant scales of a workgroup's rows take 16 KB at K = 2048, the 4-bit affine ones 32: there the
+  // activations make room for a third workgroup a compute unit)
+  constexpr bool HALF = owned_half(KIND, MODE);
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), c = lane & 15, q = lane >> 4;
+  const int nb = a.K >> 8, O = a.m[mat0].O;
+  constexpr int cols = 4 * GC * 16;  // the workgroup's columns of one matrix
+  typedef Work<KIND, RT, CT, 4, true> W;
+  // The activations' addresses take a trip to memory of their own (the pairs), the weights are the longest one:
+  // the pairs go out first, the scales and the first codes behind them, and the activations when the pairs are here.
+  uint32_t pr[2 * RT];
+  constexpr int NP = HALF ? RT : 2 * RT;
+#pragma unroll
+  for (int i = 0; i < NP; ++i) pr[i] = my_pairs[min(8 * ((HALF ? RT * (wave >> 1) : 0) + i) + (lane >> 3), rows - 1)];
+  __builtin_amdgcn_sched_barrier(0);
+  const int s_len = cols * nb * SB, d_len = cols * nb * DB, s_at = owned_x_bytes(16 * RT, KIND, MODE);
+  // 4-bit affine: a row's blocks (16 bytes of scales, 16 of biases each) lie at block ^ (row & 7), or the sixteen rows
+  // of a tile would be read from two places of the banks
+  const bool turned = KIND == kA4 && nb % 8 == 0;
+  auto from = [&](int p) { return turned ? p ^ (((p / (16 * nb)) & 7) << 4) : p; };
+  const uint8_t* code[HALVES];
+#pragma unroll
+  for (int i = 0; i < HALVES; ++i) {
+    const Mat& m = a.m[mat0 + i];
+    code[i] = uniform(m.q + row_base * nb * q_bytes(KIND));
+    const uint8_t *gs = uniform(m.s + (row_base + c0) * nb * SB), *gd = uniform(m.d + (row_base + c0) * nb * DB);
+    const int s_end = (O - c0) * nb * SB - 16, d_end = (O - c0) * nb * DB - 16;
+    const uint32_t at = lds_address(smem + s_at) + i * (s_len + d_len);
+    for (int p = wave * 1024; p < s_len; p += 4096)
+      if (p + 16 * lane < s_len) dma16(gs, (uint32_t)min(from(p + 16 * lane), s_end), at + p);
+    for (int p = wave * 1024; p < d_len; p += 4096)
+      if (p + 16 * lane < d_len) dma16(gd, (uint32_t)min(from(p + 16 * lane), d_end), at + s_len + p);
+  }
+  W w;
+  const int lr = wave * GC * 16 + c;
+  w.template start<GC>(code, c0 + lr, O, nb, 0, lane);
+#pragma unroll
+  for (int j = 0; j < CT; ++j) {
+    w.ls_[j] = (j / GC) * (s_len + d_len) + (j % GC) * 16 * nb * SB;
+    w.ld_[j] = (j / GC) * (s_len + d_len) + (j % GC) * 16 * nb * DB;
+  }
+  w.clear();
+  uint32_t xo[2 * RT];
+  const uint32_t piece = 16 * (uint32_t)Tile<KIND>::piece(HALF ? wave & 1 : wave, (lane & 7) ^ (lane >> 3));
+  const uint32_t lds = lds_address(smem) + (HALF ? (wave & 1) * (RT * 2048) + (wave >> 1) * (RT * 1024) : wave * (RT * 2048));
+  const uint8_t* x = reinterpret_cast<const uint8_t*>(a.x);
+#pragma unroll
+  for (int i = 0; i < NP; ++i) {
+    const uint32_t p = pr[i], src = a.up_div == 1 ? p : (int)p < a.pairs ? __umulhi(p, a.up_magic) : p - (uint32_t)a.pairs;
+    xo[i] = 2 * src * (uint32_t)a.K + piece;
+  }
+  if constexpr (HALF) W::ask_half(x, xo, 0, lds);
+  else W::ask_block(x, xo, lds);
+  auto scales_of = [&](int ib) {
+    const int s = turned ? ib ^ (c & 7) : ib;
+    w.ls0 = s_at + (lr * nb + s) * SB;
+    w.ld0 = s_at + s_len + (lr * nb + s) * DB;
+  };
+  scales_of(0);
+  w.template owned_block<GC, HALF, true, true>(code, c0 + lr, O, x, xo, 0, nb, lane, smem, smem, lds);
+  for (int ib = 1; ib + 1 < nb; ++ib) {
+    x += 512;
+    scales_of(ib);
+    w.template owned_block<GC, HALF, false, true>(code, c0 + lr, O, x, xo, ib, nb, lane, smem, smem, lds);
+  }
+  x += 512;
+  scales_of(nb - 1);
+  // D[row = 4 q + e][column = c]: where the lane's rows go
+  uint32_t dst[RT][4];
+#pragma unroll
+  for (int r = 0; r < RT; ++r)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) dst[r][e] = my_pairs[min(16 * r + 4 * q + e, rows - 1)];
+  w.template owned_block<GC, HALF, false, false>(code, c0 + lr, O, x, xo, nb - 1, nb, lane, smem, smem, lds);
+#pragma unroll
+  for (int j = 0; j < GC; ++j) {
+    const int col = c0 + lr + 16 * j;
+    if (col >= O) continue;
+    bf16_t* const y = a.m[mat0].y + col;
+#pragma unroll
+    for (int r = 0; r < RT; ++r)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (16 * r + 4 * q + e < rows) {
+          const float v = w.acc[r][j][e];
+          y[(size_t)dst[r][e] * O] = MODE == kGateUp ? swiglu_bf16(v, w.acc[r][CT - 1][e]) : dm_f2bf(v);
+        }
+  }
+}
+
+// AFF: affine formats, else k-quants; ONE: the kind of every matrix of the launch, or -1. NW wavefronts, K >= 512.
+// Plain: grid (column blocks, row tiles); gathered: a workgroup a column block of a tile.
+template <bool AFF, int CT, int MODE, int ROWS, int NW, int ONE = -1>
 __device__ __forceinline__ void body(const Args& a) {
   extern __shared__ __attribute__((aligned(1024))) uint8_t nmm_smem[];
-  constexpr int GC = MODE == kGateUp ? CT / 2 : CT;
-  const int cols = (NW / a.ks) * GC * 16;
-  int mat0 = 0, cb = blockIdx.x, rows, m0 = 0;
+  int mat0 = 0, cb = blockIdx.x, c0, rows, m0 = 0;
   int64_t row_base = 0;
   const uint32_t* my_pairs = nullptr;
   if constexpr (MODE == kPlain) {
@@ -585,36 +811,44 @@ __device__ __forceinline__ void body(const Args& a) {
       }
     m0 = blockIdx.y * ROWS;
     rows = min(ROWS, a.M - m0);
+    c0 = cb * (NW / a.ks) * CT * 16;
   } else {
-    const uint32_t tile = blockIdx.y;
-    if (tile >= *a.n_tiles) return;
-    const uint32_t e = __builtin_amdgcn_readfirstlane(a.tile_expert[tile]);
-    rows = __builtin_amdgcn_readfirstlane((int)a.tile_count[tile]);
-    my_pairs = a.pair + __builtin_amdgcn_readfirstlane(a.tile_start[tile]);
+    // Workgroups go round the eight dies: a tile's column blocks follow each other on one die, whose L2 then fetches
+    // the tile's activations once.
+    const uint32_t die = blockIdx.x % 8u, seq = blockIdx.x / 8u, tile = seq / (uint32_t)a.blocks * 8u + die;
+    c0 = (int)(seq % (uint32_t)a.blocks) * (MODE == kGateUp ? 64 : 128);
+    // (all four words in one trip; what lies past the list's end is not used)
+    const uint32_t at = min(tile, (uint32_t)a.tiles_max - 1u), n = *a.n_tiles;
+    const uint32_t e = __builtin_amdgcn_readfirstlane(a.tile_expert[at]);
+    rows = __builtin_amdgcn_readfirstlane((int)a.tile_count[at]);
+    my_pairs = a.pair + __builtin_amdgcn_readfirstlane(a.tile_start[at]);
+    if (tile >= n) return;
     if ((int)e >= a.E)
       mat0 = 2;
     else
       row_base = (int64_t)e * a.m[0].O;
   }
-  const int c0 = cb * cols;
   const int kind = a.m[mat0].kind;
-#define NMM_TILE(KIND, RT) tile_body<KIND, (RT <= ROWS / 16 ? RT : 1), CT, MODE, ROWS, NW>(a, mat0, c0, row_base, rows, m0, my_pairs, nmm_smem)
-#define NMM_KIND(KIND)                                     \
-  do {                                                     \
-    if (rows <= 16 || ROWS == 16) NMM_TILE(KIND, 1);       \
-    else if (rows <= 32 || ROWS <= 32) NMM_TILE(KIND, 2);  \
-    else if (rows <= 48) NMM_TILE(KIND, 3);                \
-    else NMM_TILE(KIND, 4);                                \
-  } while (0)
-  if constexpr (AFF) {
-    if (kind == kA4) NMM_KIND(kA4);
-    else NMM_KIND(kA8);
+  auto run = [&](auto kc, auto rc) {
+    constexpr int KIND = decltype(kc)::value, RT = decltype(rc)::value;
+    if constexpr (MODE == kPlain) tile_body<KIND, RT, CT, ROWS, NW>(a, mat0, c0, rows, m0, nmm_smem);
+    else owned_tile<KIND, RT, MODE>(a, mat0, c0, row_base, rows, my_pairs, nmm_smem);
+  };
+  auto of_kind = [&](auto kc) {
+    if (rows <= 16 || ROWS == 16) run(kc, std::integral_constant<int, 1>{});
+    else if (rows <= 32 || ROWS == 32) run(kc, std::integral_constant<int, (ROWS >= 32 ? 2 : 1)>{});
+    else if (rows <= 48) run(kc, std::integral_constant<int, (ROWS >= 48 ? 3 : 1)>{});
+    else run(kc, std::integral_constant<int, (ROWS >= 64 ? 4 : 1)>{});
+  };
+  if constexpr (ONE >= 0) {
+    of_kind(std::integral_constant<int, ONE>{});
+  } else if constexpr (AFF) {
+    if (kind == kA4) of_kind(std::integral_constant<int, kA4>{});
+    else of_kind(std::integral_constant<int, kA8>{});
   } else {
-    if (kind == kQ4K) NMM_KIND(kQ4K);
-    else NMM_KIND(kQ6K);
+    if (kind == kQ4K) of_kind(std::integral_constant<int, kQ4K>{});
+    else of_kind(std::integral_constant<int, kQ6K>{});
   }
-#undef NMM_KIND
-#undef NMM_TILE
 }
 
 }  // namespace nmm

@@ -2,5 +2,6 @@
 #include "mm_narrow_host.h"
 
 namespace nmm {
-NMM_KERNELS(affine, true, 3, 3, 8u)
+constexpr int affine_waves(int, int rows) { return rows == 16 ? 4 : rows == 32 ? 3 : 2; }
+NMM_KERNELS(affine, true, kA4, -1, affine_waves, 8u)
 }

@@ -37,38 +37,46 @@ int gate_up(ornith_ctx* ctx, const ornith_moe_weights* w, const void* d_x, int p
 bool moe_ok(const ornith_moe_weights* w, const void* d_x, int T, const void* d_act, const void* d_y);
 
 // the launches of a family; the first one on a context's device raises the kernels' LDS limits
-int launch_kq(ornith_ctx* ctx, const Args& a, int mode, int ct, int rows, dim3 grid, int lds);
-int launch_affine(ornith_ctx* ctx, const Args& a, int mode, int ct, int rows, dim3 grid, int lds);
+int launch_kq(ornith_ctx* ctx, const Args& a, int mode, int ct, int rows, int kind, dim3 grid, int lds);
+int launch_affine(ornith_ctx* ctx, const Args& a, int mode, int ct, int rows, int kind, dim3 grid, int lds);
 
 }  // namespace nmm
 
-// The kernels of a family. A workgroup is four wavefronts, one a SIMD; a compute unit holds two plain
-// ones, and as many gathered ones as accumulators, codes and activation chunks leave room for (W16, W32:
-// wavefronts a SIMD at 16 and 32 rows) without spilling, but for the 32-row affine kernels, which spill four
-// (gathered) and two (gate + up) registers at three wavefronts a SIMD.
-#define NMM_KERNELS(NAME, AFF, W16, W32, LDS_BIT)                                                                   \
+// The kernels of a family, gathered ones for launches of one kind (K1, K2) and of both (-1): a kernel has the registers of
+// its widest path. A workgroup is four wavefronts, one a SIMD; a compute unit holds two plain ones, and as many
+// gathered ones as registers and LDS allow (WAVES: asked for, a SIMD).
+#define NMM_KERNELS(NAME, AFF, K1, K2, WAVES, LDS_BIT)                                                              \
   template <int CT>                                                                                                 \
   __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void NAME##_plain_kernel(Args a) {   \
     body<AFF, CT, kPlain, 64, 4>(a);                                                                                \
   }                                                                                                                 \
-  template <int MODE, int ROWS>                                                                                     \
-  __global__ __launch_bounds__(256)                                                                                 \
-      __attribute__((amdgpu_waves_per_eu(ROWS == 16 ? W16 : ROWS == 32 ? W32 : 2))) void NAME##_gather_kernel(Args a) { \
-    body<AFF, 4, MODE, ROWS, 4>(a);                                                                                 \
+  template <int MODE, int ROWS, int KIND>                                                                           \
+  __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES(KIND, ROWS)))) void                    \
+      NAME##_gather_kernel(Args a) {                                                                                \
+    body<AFF, 2, MODE, ROWS, 4, KIND>(a);                                                                           \
   }                                                                                                                 \
-  int launch_##NAME(ornith_ctx* ctx, const Args& a, int mode, int ct, int rows, dim3 grid, int lds) {               \
+  int launch_##NAME(ornith_ctx* ctx, const Args& a, int mode, int ct, int rows, int kind, dim3 grid, int lds) {     \
     typedef void (*Kernel)(Args);                                                                                   \
-    static const Kernel kernels[9] = {                                                                              \
-        NAME##_plain_kernel<1>,           NAME##_plain_kernel<2>,           NAME##_plain_kernel<4>,                 \
-        NAME##_gather_kernel<kGather, 16>, NAME##_gather_kernel<kGather, 32>, NAME##_gather_kernel<kGather, 64>,    \
-        NAME##_gather_kernel<kGateUp, 16>, NAME##_gather_kernel<kGateUp, 32>, NAME##_gather_kernel<kGateUp, 64>};   \
+    static const Kernel plain[3] = {NAME##_plain_kernel<1>, NAME##_plain_kernel<2>, NAME##_plain_kernel<4>};        \
+    static const Kernel gather[3][2][3] = {                                                                         \
+        {{NAME##_gather_kernel<kGather, 16, K1>, NAME##_gather_kernel<kGather, 32, K1>, NAME##_gather_kernel<kGather, 64, K1>},     \
+         {NAME##_gather_kernel<kGateUp, 16, K1>, NAME##_gather_kernel<kGateUp, 32, K1>, NAME##_gather_kernel<kGateUp, 64, K1>}},    \
+        {{NAME##_gather_kernel<kGather, 16, K2>, NAME##_gather_kernel<kGather, 32, K2>, NAME##_gather_kernel<kGather, 64, K2>},     \
+         {NAME##_gather_kernel<kGateUp, 16, K2>, NAME##_gather_kernel<kGateUp, 32, K2>, NAME##_gather_kernel<kGateUp, 64, K2>}},    \
+        {{NAME##_gather_kernel<kGather, 16, -1>, NAME##_gather_kernel<kGather, 32, -1>, NAME##_gather_kernel<kGather, 64, -1>},     \
+         {NAME##_gather_kernel<kGateUp, 16, -1>, NAME##_gather_kernel<kGateUp, 32, -1>, NAME##_gather_kernel<kGateUp, 64, -1>}}};   \
     if (!(ctx->lds_attr_set & LDS_BIT)) {                                                                           \
-      for (const Kernel k : kernels)                                                                                \
+      for (const Kernel k : plain)                                                                                  \
         ORN_HIP(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes));        \
+      for (const auto& g : gather)                                                                                  \
+        for (const auto& m : g)                                                                                     \
+          for (const Kernel k : m)                                                                                  \
+            ORN_HIP(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes));    \
       ctx->lds_attr_set |= LDS_BIT;                                                                                 \
     }                                                                                                               \
-    const int i = mode == kPlain ? ct / 2 : (mode == kGather ? 3 : 6) + (rows == 16 ? 0 : rows == 32 ? 1 : 2);      \
-    hipLaunchKernelGGL(kernels[i], grid, dim3(256), lds, ctx->stream, a);                    \
+    const Kernel k = mode == kPlain ? plain[ct / 2]                                                                 \
+                                    : gather[kind == K1 ? 0 : kind == K2 ? 1 : 2][mode == kGateUp][rows / 32];      \
+    hipLaunchKernelGGL(k, grid, dim3(256), lds, ctx->stream, a);                                                    \
     ORN_LAUNCH_CHECK("nmm::" #NAME);                                                                                \
     return ORNITH_OK;                                                                                               \
   }

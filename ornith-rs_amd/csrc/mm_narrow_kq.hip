@@ -4,7 +4,8 @@
 #include "mm_narrow_host.h"
 
 namespace nmm {
-NMM_KERNELS(kq, false, 4, 3, 4u)
+constexpr int kq_waves(int kind, int rows) { return rows == 16 ? (kind == kQ4K ? 5 : 4) : rows == 32 ? (kind == kQ4K ? 4 : 3) : 2; }
+NMM_KERNELS(kq, false, kQ4K, kQ6K, kq_waves, 4u)
 
 namespace {
 
@@ -35,12 +36,11 @@ bool reachable(const Mat& m, int K) {
   return m.kind >= 0 && m.O >= 1 && m.q && m.s && m.d && (size_t)m.O * K < (size_t(1) << 32) && m.O * (size_t)(K / 256) % 8 == 0 &&
          (((uintptr_t)m.q | (uintptr_t)m.s | (uintptr_t)m.d) & 15) == 0 && ((uintptr_t)m.y & 7) == 0;
 }
-// LDS of a launch: activations and scales (of the widest format), or the partial tiles
-int lds_bytes(const Args& a, int mats, int halves, int cols, int rows, int ct, int nw) {
+// LDS of a plain launch: activations and scales (of the widest format), or the partial tiles
+int lds_bytes(const Args& a, int cols, int rows, int ct, int nw) {
   int per_block = 0;
-  for (int i = 0; i < mats; ++i)
-    if (a.m[i].q) per_block = std::max(per_block, s_bytes(a.m[i].kind) + d_bytes(a.m[i].kind));
-  return std::max(x_bytes(rows, nw) + halves * cols * (a.K / 256) * per_block, red_bytes(rows, ct, nw));
+  for (int i = 0; i < a.n; ++i) per_block = std::max(per_block, s_bytes(a.m[i].kind) + d_bytes(a.m[i].kind));
+  return std::max(x_bytes(rows, nw) + cols * (a.K / 256) * per_block, red_bytes(rows, ct, nw));
 }
 // wavefronts of NW that split K: as many as there are 256-wide blocks, a power of two
 int k_split(int K, int nw) {
@@ -93,8 +93,8 @@ int plain(ornith_ctx* ctx, const ornith_linear* const* ws, int n, const void* d_
     blocks += (ws[i]->O + cols - 1) / cols;
   }
   const dim3 grid(blocks, row_tiles);
-  const int lds = lds_bytes(a, n, 1, cols, 64, ct, 4);
-  return affine(a.m[0].kind) ? launch_affine(ctx, a, kPlain, ct, 64, grid, lds) : launch_kq(ctx, a, kPlain, ct, 64, grid, lds);
+  const int lds = lds_bytes(a, cols, 64, ct, 4);
+  return affine(a.m[0].kind) ? launch_affine(ctx, a, kPlain, ct, 64, -1, grid, lds) : launch_kq(ctx, a, kPlain, ct, 64, -1, grid, lds);
 }
 
 int tile_rows(int pairs, int E) {
@@ -115,16 +115,26 @@ bool experts_ok(const ornith_kmatrix* w, const void* d_x, size_t x_rows, const v
 
 namespace {
 int launch_gathered(ornith_ctx* ctx, Args& a, int mode, const Plan& p, int O) {
-  a.ks = k_split(a.K, 4);
   a.pair = p.pair;
   a.tile_expert = p.tile_expert;
   a.tile_start = p.tile_start;
   a.tile_count = p.tile_count;
   a.n_tiles = p.n_tiles;
-  const int cols = (4 / a.ks) * (mode == kGateUp ? 2 : 4) * 16;
-  const dim3 grid((O + cols - 1) / cols, (unsigned)p.tiles_max);
-  const int lds = lds_bytes(a, 4, mode == kGateUp ? 2 : 1, cols, p.rows, 4, 4);
-  return affine(a.m[0].kind) ? launch_affine(ctx, a, mode, 4, p.rows, grid, lds) : launch_kq(ctx, a, mode, 4, p.rows, grid, lds);
+  a.tiles_max = (int)p.tiles_max;
+  a.up_magic = (uint32_t)(((uint64_t(1) << 32) + a.up_div - 1) / a.up_div);
+  const int halves = mode == kGateUp ? 2 : 1, cols = 128 / halves;
+  a.blocks = (O + cols - 1) / cols;
+  // LDS: activations, and the scales of the workgroup's 128 rows
+  int kind = a.m[0].kind, lds = 0;
+  for (int i = 0; i < 4; ++i) {
+    if (!a.m[i].q) continue;
+    const int k = a.m[i].kind;
+    lds = std::max(lds, owned_x_bytes(p.rows, k, mode) + 128 * (a.K / 256) * (s_bytes(k) + d_bytes(k)));
+    if (k != kind) kind = -1;
+  }
+  const dim3 grid((unsigned)(a.blocks * ((p.tiles_max + 7) / 8 * 8)));
+  return affine(a.m[0].kind) ? launch_affine(ctx, a, mode, 0, p.rows, kind, grid, lds)
+                             : launch_kq(ctx, a, mode, 0, p.rows, kind, grid, lds);
 }
 }  // namespace
 

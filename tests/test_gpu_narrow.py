@@ -121,3 +121,68 @@ def test_few_row_moe_block_of_a_layer_over_affine_experts(orn, ctx, T):
     assert np.median(rel) < 0.004 and (rel < 0.03).mean() >= 0.93, (float(np.median(rel)), float(np.sort(rel)[-5]))
     for b in bufs: b.free()
     moe.free()
+
+
+def _deq(kind, t, E, O, K):
+    w = util.orc_dequant(kind, *t, E * O * K // 256)
+    return util.bf16_to_f32(util.f32_to_bf16(w)).astype(np.float64).reshape(E, O, K)
+
+
+@pytest.mark.parametrize("kind,E,O,K,T,k", [
+    # 16-, 32- and 64-row tiles; columns below, at and past a workgroup's 128; K of two, three, eight and sixteen blocks
+    (Q4K, 8, 200, 512, 20, 2), (Q6K, 8, 200, 512, 20, 2), (Q6K, 16, 8, 768, 90, 3), (Q4K, 16, 136, 768, 200, 2),
+    (Q4K, 8, 128, 2048, 60, 3), (Q6K, 8, 264, 2048, 90, 4), (Q4K, 4, 64, 4096, 33, 4), (Q6K, 4, 129, 4096, 33, 4)])
+@pytest.mark.parametrize("skew", [False, True])
+def test_few_row_gathered_matmul_vs_float64(orn, ctx, kind, E, O, K, T, k, skew):
+    """The expert form whose wavefronts own columns, over every pair of a token list: one rounding of the output, and
+    fp32 sums in another order (as above). skew: half of the picks fall on expert 1, which then has several tiles."""
+    rng = np.random.default_rng(E * O + K + T)
+    t = (util.make_q4k if kind == Q4K else util.make_q6k)(rng, E, O, K)
+    inds = np.stack([rng.permutation(E)[:k] for _ in range(T)]).astype(np.uint32)
+    if skew:
+        inds[: T // 2 * 2 : 2, 0] = 1
+    pairs = T * k
+    assert pairs < 48 * E
+    wt = _deq(kind, t, E, O, K)
+    w = orn.KMatrix(ctx, kind, *t, E, O, K)
+    plan = ctx.alloc(orn.kq_gather_plan_bytes(pairs, E))
+    di = ctx.to_device(inds.reshape(-1))
+    for is_up in (True, False):
+        rows = T if is_up else pairs
+        xb = util.bf16_normal(rng, (rows, K))
+        dx, dy = ctx.to_device(xb), ctx.alloc((pairs + 1) * O * 2)
+        ctx.memset(dy, 0xFF, (pairs + 1) * O * 2)
+        orn.kq_gather_matmul(ctx, w, dx, di, pairs, k, is_up, plan, is_up, dy)
+        out = dy.download(np.uint16, (pairs + 1, O))
+        assert np.all(out[pairs] == 0xFFFF)
+        got = util.bf16_to_f32(out[:pairs]).astype(np.float64)
+        x = util.bf16_to_f32(xb).astype(np.float64)
+        want = np.stack([wt[inds[p // k, p % k]] @ x[p // k if is_up else p] for p in range(pairs)])
+        scale = np.sqrt(np.mean(want ** 2))
+        assert np.all(np.abs(got - want) <= 2.0 ** -8 * np.abs(want) + 2e-5 * scale), float(np.abs(got - want).max() / scale)
+        for b in (dx, dy): b.free()
+    for b in (di, plan, w): b.free()
+
+
+@pytest.mark.parametrize("fmt,T", [("kq", 70), ("kq", 200), ("affine4", 40), ("affine4", 150)])
+def test_few_row_moe_block_whose_shared_expert_has_another_format(orn, ctx, fmt, T):
+    """Launches of two formats (Q4_K and Q6_K, 4-bit and 8-bit affine), at K = 2048 (where the 4-bit scales lie turned by
+    the row), against the oracle's exact block on the normed rows, with the bounds of the tests above."""
+    rng = np.random.default_rng(T)
+    H, I = 2048, 512
+    moe = util.HostMoe(rng, H=H, E=64, I=I, top_k=8, gate_kind=util.AFFINE4 if fmt == "affine4" else Q4K)
+    other = (lambda o, k, kind: util.HostLinear.kq(rng, kind, o, k)) if fmt == "kq" else (lambda o, k, _: util.HostLinear.affine8(rng, o, k))
+    moe.sh_gate, moe.sh_up, moe.sh_down = other(I, H, Q6K), other(I, H, Q6K), other(H, I, Q4K)
+    res, y, wn = (util.bf16_normal(rng, s) for s in ((T, H), (T, H), (H,)))
+    _, normed = util.orc_add_rms_norm(res, y, wn)
+    want = util.bf16_to_f32(util.orc_moe_block(moe, normed, T)[0]).astype(np.float64)
+    w = moe.dev(orn, ctx)
+    bufs = [ctx.to_device(a) for a in (res, y, wn)] + [ctx.alloc(T * H * 2) for _ in range(3)]
+    dres, dy, dwn, dh, dn, out = bufs
+    orn.add_rms_moe_block(ctx, w, dres, dy, dwn, 1e-6, T, dh, dn, out)
+    got = util.bf16_to_f32(out.download(np.uint16, (T, H))).astype(np.float64)
+    rel = np.linalg.norm(got - want, axis=1) / np.linalg.norm(want, axis=1)
+    bound = 0.004 if fmt == "affine4" else 0.01
+    assert np.median(rel) < bound and (rel < 0.03).mean() >= 0.93, (float(np.median(rel)), float(np.sort(rel)[-5]))
+    for b in bufs: b.free()
+    moe.free()
