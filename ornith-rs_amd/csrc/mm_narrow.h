@@ -65,7 +65,7 @@ typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x2_t __attribute__((ext_vector_type(2)));
 
 enum Kind { kQ4K = 0, kQ6K = 1, kA4 = 2, kA8 = 3 };
-enum Mode { kPlain = 0, kGather = 1, kGateUp = 2 };
+enum Mode { kPlain = 0, kGather = 1, kGateUp = 2, kTall = 3 };
 
 struct Mat {
   const uint8_t* q;  // codes
@@ -464,16 +464,17 @@ struct Work {
     for (int j = 0; j < CT; ++j) load(t[j].t, code[j / GC], row0 + 16 * (j % GC), O, ks, nb, lane >> 4);
     __builtin_amdgcn_sched_barrier(0);
   }
+  static constexpr int kScaleLoads = KIND == kA4 ? 2 : 0;
   // The plain form: one block, with two chunks and the codes of it asked for. MORE: the wavefront has another one, KS blocks
   // on; its codes go out here behind this block's activations (which are waited for one by one), its activations as
   // this block's buffers come free.
-  template <int GC, bool MORE, class F>
+  template <bool MORE, class F, class G>
   __device__ __forceinline__ void block(const uint8_t* code, int row0, int O, const uint8_t* xk, const uint32_t (&xo)[2 * RT], int ib,
-                                        int nb, int KS, int lane, const uint8_t* smem, const uint8_t* xs, uint32_t lds, F first) {
+                                        int nb, int KS, int lane, const uint8_t* smem, const uint8_t* xs, uint32_t lds, F first, G scales) {
     static_assert(NB == 2, "two chunks in flight");
     const int c = lane & 15, q = lane >> 4;
     constexpr bool AHEAD = MORE && PF;
-    constexpr int NL = AHEAD ? CT * T::kLoads : 0;
+    constexpr int NL = (AHEAD ? CT * T::kLoads : 0) + (MORE ? kScaleLoads : 0);
     const uint8_t* const xn = xk + (size_t)KS * 512;
     typename T::Codes next[CT];
     wait_loads<0>();
@@ -489,6 +490,7 @@ struct Work {
       for (int j = 0; j < CT; ++j) load(next[j], code, row0 + 16 * j, O, ib + KS, nb, q);
       __builtin_amdgcn_sched_barrier(0);
     }
+    if constexpr (MORE) scales(ib + KS);
     wait_loads<2 * RT + NL>();
     step<4>(smem, xs, c, q);
     step<5>(smem, xs, c, q);
@@ -503,8 +505,6 @@ struct Work {
         if constexpr (PF) t[j].t = next[j];
         else load(t[j].t, code, row0 + 16 * j, O, ib + KS, nb, q);
       }
-      ls0 += KS * s_bytes(KIND);
-      ld0 += KS * d_bytes(KIND);
     }
   }
   // The form whose wavefronts own columns: every one works through all of K, a block at a time, and the workgroup's four
@@ -521,10 +521,10 @@ struct Work {
 #pragma unroll
     for (int i = 0; i < RT; ++i) dma16(x + half * T::half_bytes(), xo[i], lds + half * (RT * 4096) + i * 1024);
   }
-  template <int GC, bool HALF, bool FIRST, bool MORE>
+  template <int GC, bool HALF, bool FIRST, bool MORE, class F>
   __device__ __forceinline__ void owned_block(const uint8_t* const (&code)[CT / GC], int row0, int O, const uint8_t* x,
                                               const uint32_t (&xo)[2 * RT], int ib, int nb, int lane, const uint8_t* smem,
-                                              const uint8_t* xs, uint32_t lds) {
+                                              const uint8_t* xs, uint32_t lds, F ask_scales) {
     const int c = lane & 15, q = lane >> 4;
     typename T::Codes next[CT];
     auto ask_codes = [&]() {
@@ -540,6 +540,7 @@ struct Work {
       ask_half(x, xo, 1, lds);
     } else if constexpr (MORE) {
       ask_block(x + 512, xo, lds + ((ib + 1) & 1) * (RT * 8192));
+      ask_scales(ib + 1);
       ask_codes();
     }
     step<0>(smem, xs + buf, c, q);
@@ -551,6 +552,7 @@ struct Work {
       barrier_only();
       if constexpr (MORE) {
         ask_half(x + 512, xo, 0, lds);
+        ask_scales(ib + 1);
         ask_codes();
       }
     }
@@ -573,9 +575,11 @@ struct Work {
   }
   // x, xo: the activations and the byte offsets of the rows this lane fetches; xs / lds: this wavefront's
   // activation buffers; scales_here(): what has to be done before the first block's arithmetic. start() has been called.
-  template <class F>
+  // scales(ib) as above, scales_of(ib): ls0 and ld0 of a block.
+  template <class F, class G, class S>
   __device__ __forceinline__ void run(const uint8_t* code, int row0, int O, const bf16_t* x, const uint32_t (&xo)[2 * RT], int nb, int ks,
-                                      int KS, int lane, const uint8_t* smem, const uint8_t* xs, uint32_t lds, F scales_here) {
+                                      int KS, int lane, const uint8_t* smem, const uint8_t* xs, uint32_t lds, F scales_here, G scales,
+                                      S scales_of) {
     clear();
     const uint8_t* xk = reinterpret_cast<const uint8_t*>(x) + (size_t)ks * 512;
     fetch<0>(xk, xo, lds, lane);
@@ -584,8 +588,12 @@ struct Work {
     auto first = [&]() {
       if (ib == ks) scales_here();
     };
-    for (; ib + KS < nb; ib += KS, xk += (size_t)KS * 512) block<CT, true>(code, row0, O, xk, xo, ib, nb, KS, lane, smem, xs, lds, first);
-    block<CT, false>(code, row0, O, xk, xo, ib, nb, KS, lane, smem, xs, lds, first);
+    for (; ib + KS < nb; ib += KS, xk += (size_t)KS * 512) {
+      scales_of(ib);
+      block<true>(code, row0, O, xk, xo, ib, nb, KS, lane, smem, xs, lds, first, scales);
+    }
+    scales_of(ib);
+    block<false>(code, row0, O, xk, xo, ib, nb, KS, lane, smem, xs, lds, first, scales);
   }
 };
 
@@ -609,12 +617,24 @@ __device__ __forceinline__ void tile_body(const Args& a, int mat, int c0, int ro
   const int O = m.O, cols = (NW / KS) * CT * 16;  // the workgroup's columns
   float* red = reinterpret_cast<float*>(smem);
 
-  // the scales of the workgroup's rows: one run of bytes in each tensor (what would pass the matrix's
-  // end repeats its last 16 bytes: rows that are never stored)
+  // The scales: of the workgroup's rows over all of K, one run of bytes in each tensor (what would pass the matrix's end
+  // repeats its last 16 bytes: rows that are never stored). 4-bit affine, whose 16-byte pieces can be fetched one
+  // by one: of the wavefront's columns, a block ahead in two buffers (all of K = 4096 would be 32 KB and leave a compute
+  // unit one workgroup: 2048 x 4096 at 600 rows 48 us).
+  constexpr bool RING = KIND == kA4;
   const int s_len = cols * nb * SB, d_len = cols * nb * DB;
   const uint8_t* const code[1] = {uniform(m.q)};
-  {
-    const uint8_t *gs = uniform(m.s + (int64_t)c0 * nb * SB), *gd = uniform(m.d + (int64_t)c0 * nb * DB);
+  const int lr = cw * CT * 16 + c;  // of tile 0, which of the workgroup's rows
+  const uint8_t *gs = uniform(m.s + (int64_t)c0 * nb * SB), *gd = uniform(m.d + (int64_t)c0 * nb * DB);
+  const uint32_t ring = x_bytes(ROWS, NW) + wave * 4096;
+  const uint32_t ring_at = lds_address(smem + ring), ring_off = (uint32_t)min(cw * CT * 16 + lane, O - c0 - 1) * (uint32_t)(nb * 16);
+  auto ask_scales = [&](int ib) {
+    if constexpr (RING) {
+      dma16(gs + ib * 16, ring_off, ring_at + (ib / KS & 1) * 2048);
+      dma16(gd + ib * 16, ring_off, ring_at + (ib / KS & 1) * 2048 + 1024);
+    }
+  };
+  if constexpr (!RING) {
     const int s_end = (O - c0) * nb * SB - 16, d_end = (O - c0) * nb * DB - 16;
     const uint32_t at = lds_address(smem + x_bytes(ROWS, NW));
     for (int p = wave * 1024; p < s_len; p += NW * 1024)
@@ -622,17 +642,19 @@ __device__ __forceinline__ void tile_body(const Args& a, int mat, int c0, int ro
     for (int p = wave * 1024; p < d_len; p += NW * 1024)
       if (p + 16 * lane < d_len) dma16(gd, (uint32_t)min(p + 16 * lane, d_end), at + s_len + p);
   }
+  ask_scales(ks);
 
   // (the codes ahead where the registers hold two blocks of them)
   Work<KIND, RT, CT, 2, (KIND == kQ4K || KIND == kA4) && RT <= 2> w;
-  const int lr = cw * CT * 16 + c;  // of tile 0, which of the workgroup's rows
   w.template start<CT>(code, c0 + lr, O, nb, ks, lane);
-  w.ls0 = x_bytes(ROWS, NW) + (lr * nb + ks) * SB;
-  w.ld0 = x_bytes(ROWS, NW) + s_len + (lr * nb + ks) * DB;
+  auto scales_of = [&](int ib) {
+    w.ls0 = RING ? ring + (ib / KS & 1) * 2048 + c * 16 : x_bytes(ROWS, NW) + (lr * nb + ib) * SB;
+    w.ld0 = RING ? w.ls0 + 1024 : x_bytes(ROWS, NW) + s_len + (lr * nb + ib) * DB;
+  };
 #pragma unroll
   for (int j = 0; j < CT; ++j) {
-    w.ls_[j] = j * 16 * nb * SB;
-    w.ld_[j] = j * 16 * nb * DB;
+    w.ls_[j] = RING ? j * 256 : j * 16 * nb * SB;
+    w.ld_[j] = RING ? j * 256 : j * 16 * nb * DB;
   }
   // this lane fetches a piece of rows 8 i + (lane >> 3); rows past the end read a valid row: what they produce is never stored
   uint32_t xo[2 * RT];
@@ -640,7 +662,8 @@ __device__ __forceinline__ void tile_body(const Args& a, int mat, int c0, int ro
   for (int i = 0; i < 2 * RT; ++i) xo[i] = 2 * (uint32_t)min(m0 + 8 * i + (lane >> 3), a.M - 1) * (uint32_t)a.K;
   const uint8_t* xs = smem + wave * (x_bytes(ROWS, NW) / NW);
   w.run(code[0], c0 + lr, O, a.x, xo, nb, ks, KS, lane, smem, xs, lds_address(xs),
-        [&]() { barrier_only(); });  // every wavefront's share of the scales has arrived (waited for by each)
+        [&]() { barrier_only(); },  // every wavefront's share of the scales has arrived (waited for by each)
+        ask_scales, scales_of);
   __syncthreads();
   // The partial tiles meet in LDS. First the upper half of the K split hands its registers to
   // the lower half as they are (16 bytes a lane), which halves what the second pass holds.
@@ -697,17 +720,25 @@ __device__ __forceinline__ void tile_body(const Args& a, int mat, int c0, int ro
   }
 }
 
-// The gathered forms. A tile (an expert's up to 16 RT rows) takes four wavefronts a column block; each owns columns, 16 of gate
-// and of up or 32 of one matrix, over all of K, its codes a block ahead in registers, so nothing has to meet at the end.
-__host__ __device__ constexpr bool owned_half(int kind, int mode) { return kind == kA4 && mode == kGateUp; }
+// The forms whose wavefronts own columns: an expert's tile, or (kTall) 64 rows of a plain product, takes four wavefronts a block
+// of 128 columns (64 of gate and of up); each owns 32 of them over all of K, its codes a block ahead in registers, so
+// nothing has to meet at the end.
+// LDS: activations, and the scales of 128 rows over all of K (4-bit affine: 32 KB at K = 2048, 16 KB the others). What
+// makes room for another workgroup a compute unit where those two are too much: HALF, the activations half a block at a time
+// (64-row tiles; 4-bit affine gate + up, 106 -> 98 us at 600 tokens; elsewhere the second barrier a block costs more), and RING,
+// the scales of two blocks (4-bit affine, 64-row tiles, 71 -> 61 us at 12288 x 2048 and 600 rows; it is 64 lookups a load, which
+// an expert's gate + up has no room for: 59 -> 73 us at 40 tokens).
+__host__ __device__ constexpr bool owned_half(int kind, int mode) { return mode == kTall || (kind == kA4 && mode == kGateUp); }
+__host__ __device__ constexpr bool owned_ring(int kind, int mode) { return mode == kTall && kind == kA4; }
 __host__ __device__ constexpr int owned_x_bytes(int rows, int kind, int mode) { return rows * (owned_half(kind, mode) ? 512 : 1024); }
+__host__ __device__ constexpr int owned_lds(int rows, int kind, int mode, int nb) {
+  return owned_x_bytes(rows, kind, mode) + 128 * (owned_ring(kind, mode) ? 2 : nb) * (s_bytes(kind) + d_bytes(kind));
+}
 template <int KIND, int RT, int MODE>
-__device__ __forceinline__ void owned_tile(const Args& a, int mat0, int c0, int64_t row_base, int rows, const uint32_t* my_pairs,
+__device__ __forceinline__ void owned_tile(const Args& a, int mat0, int c0, int64_t row_base, int rows, int m0, const uint32_t* my_pairs,
                                            uint8_t* smem) {
   constexpr int SB = s_bytes(KIND), DB = d_bytes(KIND), CT = 2, HALVES = MODE == kGateUp ? 2 : 1, GC = CT / HALVES;
-  // (8-bit and k-quant scales of a workgroup's rows take 16 KB at K = 2048, the 4-bit affine ones 32: there the
-  // activations make room for a third workgroup a compute unit)
-  constexpr bool HALF = owned_half(KIND, MODE);
+  constexpr bool HALF = owned_half(KIND, MODE), RING = owned_ring(KIND, MODE);
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), c = lane & 15, q = lane >> 4;
   const int nb = a.K >> 8, O = a.m[mat0].O;
   constexpr int cols = 4 * GC * 16;  // the workgroup's columns of one matrix
@@ -717,33 +748,52 @@ __device__ __forceinline__ void owned_tile(const Args& a, int mat0, int c0, int6
   uint32_t pr[2 * RT];
   constexpr int NP = HALF ? RT : 2 * RT;
 #pragma unroll
-  for (int i = 0; i < NP; ++i) pr[i] = my_pairs[min(8 * ((HALF ? RT * (wave >> 1) : 0) + i) + (lane >> 3), rows - 1)];
+  for (int i = 0; i < NP; ++i) {
+    const int r = min(8 * ((HALF ? RT * (wave >> 1) : 0) + i) + (lane >> 3), rows - 1);
+    if constexpr (MODE == kTall) pr[i] = m0 + r;
+    else pr[i] = my_pairs[r];
+  }
   __builtin_amdgcn_sched_barrier(0);
-  const int s_len = cols * nb * SB, d_len = cols * nb * DB, s_at = owned_x_bytes(16 * RT, KIND, MODE);
-  // 4-bit affine: a row's blocks (16 bytes of scales, 16 of biases each) lie at block ^ (row & 7), or the sixteen rows
-  // of a tile would be read from two places of the banks
-  const bool turned = KIND == kA4 && nb % 8 == 0;
+  const int s_len = RING ? cols * 16 : cols * nb * SB, d_len = cols * nb * DB, s_at = owned_x_bytes(16 * RT, KIND, MODE);
+  // 4-bit affine over all of K: a row's blocks (16 bytes of scales, 16 of biases each) lie at block ^ (row & 7), or the
+  // sixteen rows of a tile would be read from two places of the banks
+  const bool turned = KIND == kA4 && !RING && nb % 8 == 0;
   auto from = [&](int p) { return turned ? p ^ (((p / (16 * nb)) & 7) << 4) : p; };
   const uint8_t* code[HALVES];
 #pragma unroll
   for (int i = 0; i < HALVES; ++i) {
     const Mat& m = a.m[mat0 + i];
     code[i] = uniform(m.q + row_base * nb * q_bytes(KIND));
-    const uint8_t *gs = uniform(m.s + (row_base + c0) * nb * SB), *gd = uniform(m.d + (row_base + c0) * nb * DB);
-    const int s_end = (O - c0) * nb * SB - 16, d_end = (O - c0) * nb * DB - 16;
-    const uint32_t at = lds_address(smem + s_at) + i * (s_len + d_len);
-    for (int p = wave * 1024; p < s_len; p += 4096)
-      if (p + 16 * lane < s_len) dma16(gs, (uint32_t)min(from(p + 16 * lane), s_end), at + p);
-    for (int p = wave * 1024; p < d_len; p += 4096)
-      if (p + 16 * lane < d_len) dma16(gd, (uint32_t)min(from(p + 16 * lane), d_end), at + s_len + p);
+    if constexpr (!RING) {
+      const uint8_t *gs = uniform(m.s + (row_base + c0) * nb * SB), *gd = uniform(m.d + (row_base + c0) * nb * DB);
+      const int s_end = (O - c0) * nb * SB - 16, d_end = (O - c0) * nb * DB - 16;
+      const uint32_t at = lds_address(smem + s_at) + i * (s_len + d_len);
+      for (int p = wave * 1024; p < s_len; p += 4096)
+        if (p + 16 * lane < s_len) dma16(gs, (uint32_t)min(from(p + 16 * lane), s_end), at + p);
+      for (int p = wave * 1024; p < d_len; p += 4096)
+        if (p + 16 * lane < d_len) dma16(gd, (uint32_t)min(from(p + 16 * lane), d_end), at + s_len + p);
+    }
   }
+  // RING: wavefronts 0, 1 fetch the scales of 64 rows each (of a matrix each), 2, 3 the biases
+  const uint8_t* ring_from = nullptr;
+  uint32_t ring_off = 0;
+  const uint32_t ring_at = lds_address(smem + s_at) + wave * 1024;
+  if constexpr (RING) {
+    const Mat& m = a.m[mat0 + (HALVES == 2 ? wave & 1 : 0)];
+    ring_from = uniform((wave >> 1 ? m.d : m.s) + (row_base + c0) * nb * 16);
+    ring_off = (uint32_t)min((HALVES == 2 ? 0 : 64 * (wave & 1)) + lane, O - c0 - 1) * (uint32_t)(nb * 16);
+  }
+  auto ask_scales = [&](int ib) {
+    if constexpr (RING) dma16(ring_from + ib * 16, ring_off, ring_at + (ib & 1) * 4096);
+  };
+  ask_scales(0);
   W w;
   const int lr = wave * GC * 16 + c;
   w.template start<GC>(code, c0 + lr, O, nb, 0, lane);
 #pragma unroll
   for (int j = 0; j < CT; ++j) {
-    w.ls_[j] = (j / GC) * (s_len + d_len) + (j % GC) * 16 * nb * SB;
-    w.ld_[j] = (j / GC) * (s_len + d_len) + (j % GC) * 16 * nb * DB;
+    w.ls_[j] = RING ? (j / GC) * s_len + (j % GC) * 256 : (j / GC) * (s_len + d_len) + (j % GC) * 16 * nb * SB;
+    w.ld_[j] = RING ? (j / GC) * s_len + (j % GC) * 256 : (j / GC) * (s_len + d_len) + (j % GC) * 16 * nb * DB;
   }
   w.clear();
   uint32_t xo[2 * RT];
@@ -752,22 +802,22 @@ __device__ __forceinline__ void owned_tile(const Args& a, int mat0, int c0, int6
   const uint8_t* x = reinterpret_cast<const uint8_t*>(a.x);
 #pragma unroll
   for (int i = 0; i < NP; ++i) {
-    const uint32_t p = pr[i], src = a.up_div == 1 ? p : (int)p < a.pairs ? __umulhi(p, a.up_magic) : p - (uint32_t)a.pairs;
+    const uint32_t p = pr[i], src = MODE == kTall || a.up_div == 1 ? p : (int)p < a.pairs ? __umulhi(p, a.up_magic) : p - (uint32_t)a.pairs;
     xo[i] = 2 * src * (uint32_t)a.K + piece;
   }
   if constexpr (HALF) W::ask_half(x, xo, 0, lds);
   else W::ask_block(x, xo, lds);
   auto scales_of = [&](int ib) {
-    const int s = turned ? ib ^ (c & 7) : ib;
-    w.ls0 = s_at + (lr * nb + s) * SB;
-    w.ld0 = s_at + s_len + (lr * nb + s) * DB;
+    const int at = turned ? ib ^ (c & 7) : ib;
+    w.ls0 = RING ? s_at + (ib & 1) * 4096 + lr * 16 : s_at + (lr * nb + at) * SB;
+    w.ld0 = RING ? w.ls0 + 2048 : s_at + s_len + (lr * nb + at) * DB;
   };
   scales_of(0);
-  w.template owned_block<GC, HALF, true, true>(code, c0 + lr, O, x, xo, 0, nb, lane, smem, smem, lds);
+  w.template owned_block<GC, HALF, true, true>(code, c0 + lr, O, x, xo, 0, nb, lane, smem, smem, lds, ask_scales);
   for (int ib = 1; ib + 1 < nb; ++ib) {
     x += 512;
     scales_of(ib);
-    w.template owned_block<GC, HALF, false, true>(code, c0 + lr, O, x, xo, ib, nb, lane, smem, smem, lds);
+    w.template owned_block<GC, HALF, false, true>(code, c0 + lr, O, x, xo, ib, nb, lane, smem, smem, lds, ask_scales);
   }
   x += 512;
   scales_of(nb - 1);
@@ -776,8 +826,11 @@ __device__ __forceinline__ void owned_tile(const Args& a, int mat0, int c0, int6
 #pragma unroll
   for (int r = 0; r < RT; ++r)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) dst[r][e] = my_pairs[min(16 * r + 4 * q + e, rows - 1)];
-  w.template owned_block<GC, HALF, false, false>(code, c0 + lr, O, x, xo, nb - 1, nb, lane, smem, smem, lds);
+    for (int e = 0; e < 4; ++e) {
+      if constexpr (MODE == kTall) dst[r][e] = m0 + 16 * r + 4 * q + e;
+      else dst[r][e] = my_pairs[min(16 * r + 4 * q + e, rows - 1)];
+    }
+  w.template owned_block<GC, HALF, false, false>(code, c0 + lr, O, x, xo, nb - 1, nb, lane, smem, smem, lds, ask_scales);
 #pragma unroll
   for (int j = 0; j < GC; ++j) {
     const int col = c0 + lr + 16 * j;
@@ -812,6 +865,17 @@ __device__ __forceinline__ void body(const Args& a) {
     m0 = blockIdx.y * ROWS;
     rows = min(ROWS, a.M - m0);
     c0 = cb * (NW / a.ks) * CT * 16;
+  } else if constexpr (MODE == kTall) {
+    // (a die's workgroups: the row tiles of one column block after the other, so that its L2 fetches the weights once)
+    const uint32_t die = blockIdx.x % 8u, seq = blockIdx.x / 8u, rt = seq % (uint32_t)a.tiles_max;
+    cb = (int)(seq / (uint32_t)a.tiles_max * 8u + die);
+    if (cb >= a.blocks) return;
+#pragma unroll
+    for (int i = 1; i < 4; ++i)
+      if (i < a.n && cb >= a.m[i].cb0) mat0 = i;
+    c0 = (cb - a.m[mat0].cb0) * 128;
+    m0 = (int)rt * ROWS;
+    rows = min(ROWS, a.M - m0);
   } else {
     // Workgroups go round the eight dies: a tile's column blocks follow each other on one die, whose L2 then fetches
     // the tile's activations once.
@@ -832,7 +896,7 @@ __device__ __forceinline__ void body(const Args& a) {
   auto run = [&](auto kc, auto rc) {
     constexpr int KIND = decltype(kc)::value, RT = decltype(rc)::value;
     if constexpr (MODE == kPlain) tile_body<KIND, RT, CT, ROWS, NW>(a, mat0, c0, rows, m0, nmm_smem);
-    else owned_tile<KIND, RT, MODE>(a, mat0, c0, row_base, rows, my_pairs, nmm_smem);
+    else owned_tile<KIND, RT, MODE>(a, mat0, c0, row_base, rows, m0, my_pairs, nmm_smem);
   };
   auto of_kind = [&](auto kc) {
     if (rows <= 16 || ROWS == 16) run(kc, std::integral_constant<int, 1>{});

@@ -6,13 +6,19 @@
 
 namespace nmm {
 
-// Rows up to which a k-quant projection takes these kernels: the wide kernels' 256 x 128 tiles fill
-// the device from about 200 rows of 4096 columns and more on (12288 x 2048, us: 64 rows 15.8 here against
-// 29.5 there, 128 rows 21 / 29, 256 rows 33 / 31, 700 rows 79 / 68), for up to 2048 columns not before a
-// thousand rows (2048 x 4096: 64 rows 11.8 / 52, 256 rows 17 / 53, 700 rows 35 / 54, 1024 rows 38 / 55;
-// 256 x 2048: 7 / 29, 1024 rows 9 / 29). The rule looks at one matrix at a time, never at what shares
-// its launch: a matrix gives the same bits alone and in company.
-constexpr int kNarrowRows = 192, kNarrowRowsSlim = 1024;
+// Rows up to which a k-quant projection takes these kernels: the wide kernels' 256 x 128 tiles fill the device from about a
+// thousand rows of 12288 columns on, and for up to 2048 columns not before a thousand rows either (2048 x 4096, us here /
+// there: 64 rows 11.8 / 52, 256 rows 17 / 53, 700 rows 33 / 54, 1024 rows 38 / 55; 256 x 2048: 7 / 29, 1024 rows 9 / 29).
+// More columns than that go from K split over wavefronts to columns owned by them (kTall) at kNarrowRows rows, where the
+// former's activations, read by every 64 columns, start to weigh (12288 x 2048 Q4_K, us, split / owned / wide kernels:
+// 128 rows 20 / 20 / 29, 200 rows 30 / 26 / 42, 300 rows - / 26 / 41, 512 rows - / 35 / 42, 700 rows - / 53 / 66, 900 rows
+// - / 63 / 67, 1200 rows - / 82 / 71). Q6_K goes straight to the wide kernels: its one wide matrix, q_proj, shares their launch
+// with k and v (q, k, v: 300 rows 41 owned, k and v apart, 40 there; 700 rows 57 / 58). The rule looks at one matrix at a
+// time, never at what shares its launch: a matrix gives the same bits alone and in company.
+constexpr int kNarrowRows = 192, kNarrowRowsSlim = 1024, kTallRowsQ4K = 960;
+// The affine formats have no wide kernels: their projections own columns from here on (4-bit, 12288 x 2048, us, split /
+// owned: 300 rows 37 / 37, 400 rows 50 / 52, 512 rows 56 / 51, 600 rows 68 / 61, 2000 rows 207 / 187).
+constexpr int kTallFromAffine = 448;
 // pairs an expert below which the routed experts take them
 constexpr int kNarrowPairs = 48;
 
@@ -55,9 +61,14 @@ int launch_affine(ornith_ctx* ctx, const Args& a, int mode, int ct, int rows, in
       NAME##_gather_kernel(Args a) {                                                                                \
     body<AFF, 2, MODE, ROWS, 4, KIND>(a);                                                                           \
   }                                                                                                                 \
+  template <int KIND>                                                                                               \
+  __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KIND == kA4 ? 4 : 2))) void NAME##_tall_kernel(Args a) {       \
+    body<AFF, 2, kTall, 64, 4, KIND>(a);                                                                            \
+  }                                                                                                                 \
   int launch_##NAME(ornith_ctx* ctx, const Args& a, int mode, int ct, int rows, int kind, dim3 grid, int lds) {     \
     typedef void (*Kernel)(Args);                                                                                   \
     static const Kernel plain[3] = {NAME##_plain_kernel<1>, NAME##_plain_kernel<2>, NAME##_plain_kernel<4>};        \
+    static const Kernel tall[2] = {NAME##_tall_kernel<K1>, NAME##_tall_kernel<AFF ? -1 : K1>};                      \
     static const Kernel gather[3][2][3] = {                                                                         \
         {{NAME##_gather_kernel<kGather, 16, K1>, NAME##_gather_kernel<kGather, 32, K1>, NAME##_gather_kernel<kGather, 64, K1>},     \
          {NAME##_gather_kernel<kGateUp, 16, K1>, NAME##_gather_kernel<kGateUp, 32, K1>, NAME##_gather_kernel<kGateUp, 64, K1>}},    \
@@ -68,14 +79,16 @@ int launch_affine(ornith_ctx* ctx, const Args& a, int mode, int ct, int rows, in
     if (!(ctx->lds_attr_set & LDS_BIT)) {                                                                           \
       for (const Kernel k : plain)                                                                                  \
         ORN_HIP(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes));        \
+      for (const Kernel k : tall)                                                                                   \
+        ORN_HIP(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes));        \
       for (const auto& g : gather)                                                                                  \
         for (const auto& m : g)                                                                                     \
           for (const Kernel k : m)                                                                                  \
             ORN_HIP(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes));    \
       ctx->lds_attr_set |= LDS_BIT;                                                                                 \
     }                                                                                                               \
-    const Kernel k = mode == kPlain ? plain[ct / 2]                                                                 \
-                                    : gather[kind == K1 ? 0 : kind == K2 ? 1 : 2][mode == kGateUp][rows / 32];      \
+    const int of = kind == K1 ? 0 : kind == K2 ? 1 : 2;                                                             \
+    const Kernel k = mode == kPlain ? plain[ct / 2] : mode == kTall ? tall[of != 0] : gather[of][mode == kGateUp][rows / 32]; \
     hipLaunchKernelGGL(k, grid, dim3(256), lds, ctx->stream, a);                                                    \
     ORN_LAUNCH_CHECK("nmm::" #NAME);                                                                                \
     return ORNITH_OK;                                                                                               \

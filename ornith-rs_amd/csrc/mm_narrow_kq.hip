@@ -38,9 +38,12 @@ bool reachable(const Mat& m, int K) {
 }
 // LDS of a plain launch: activations and scales (of the widest format), or the partial tiles
 int lds_bytes(const Args& a, int cols, int rows, int ct, int nw) {
-  int per_block = 0;
-  for (int i = 0; i < a.n; ++i) per_block = std::max(per_block, s_bytes(a.m[i].kind) + d_bytes(a.m[i].kind));
-  return std::max(x_bytes(rows, nw) + cols * (a.K / 256) * per_block, red_bytes(rows, ct, nw));
+  int scales = 0;
+  for (int i = 0; i < a.n; ++i) {
+    const int k = a.m[i].kind;
+    scales = std::max(scales, k == kA4 ? nw * 4096 : cols * (a.K / 256) * (s_bytes(k) + d_bytes(k)));
+  }
+  return std::max(x_bytes(rows, nw) + scales, red_bytes(rows, ct, nw));
 }
 // wavefronts of NW that split K: as many as there are 256-wide blocks, a power of two
 int k_split(int K, int nw) {
@@ -61,40 +64,66 @@ bool plain_ok(const ornith_linear* const* ws, int n, const void* d_x, int M, voi
     if (ws[i]->mode == ORNITH_LIN_KQUANT && (ws[i]->km.E != 1 || ws[i]->km.O != ws[i]->O || ws[i]->km.K != K)) return false;
   }
   if (K > 4096) return false;  // (the scales of a workgroup's rows would not fit beside the activations)
-  // The k-quants have wide kernels of their own; the affine formats do not.
+  // (see kNarrowRows; the affine formats have no wider kernels)
   if (affine(kind_of(*ws[0]))) return true;
   for (int i = 0; i < n; ++i)
-    if (M > (ws[i]->O > 2048 ? kNarrowRows : kNarrowRowsSlim)) return false;
+    if (M > (ws[i]->O <= 2048 ? kNarrowRowsSlim : ws[i]->km.kind == ORNITH_Q4K ? kTallRowsQ4K : kNarrowRows)) return false;
   return true;
 }
 
-int plain(ornith_ctx* ctx, const ornith_linear* const* ws, int n, const void* d_x, int M, void* const* d_ys) {
-  Args a{};
-  a.n = n;
-  a.x = (const bf16_t*)d_x;
-  a.M = M;
-  a.K = ws[0]->K;
+namespace {
+// the form of one matrix, whatever shares its launch
+bool tall(const ornith_linear& w, int M) { return w.O > 2048 && M > (affine(kind_of(w)) ? kTallFromAffine : kNarrowRows); }
+
+int launch_tall(ornith_ctx* ctx, Args& a) {
+  int kind = a.m[0].kind, lds = 0;
+  a.blocks = 0;
+  for (int i = 0; i < a.n; ++i) {
+    a.m[i].cb0 = a.blocks;
+    a.blocks += (a.m[i].O + 127) / 128;
+    lds = std::max(lds, owned_lds(64, a.m[i].kind, kTall, a.K / 256));
+    if (a.m[i].kind != kind) kind = -1;
+  }
+  a.tiles_max = (a.M + 63) / 64;
+  const dim3 grid((unsigned)((a.blocks + 7) / 8 * 8 * a.tiles_max));
+  return affine(a.m[0].kind) ? launch_affine(ctx, a, kTall, 0, 64, kind, grid, lds) : launch_kq(ctx, a, kTall, 0, 64, kind, grid, lds);
+}
+
+int launch_split(ornith_ctx* ctx, Args& a) {
   a.ks = k_split(a.K, 4);
-  const int row_tiles = (M + 63) / 64;
+  const int row_tiles = (a.M + 63) / 64;
   // Columns a workgroup: 64 (four tiles a wavefront, each activation fragment used four times)
   // once that gives most compute units a workgroup, else 32 or 16.
   int ct = 4, blocks = 0;
   for (;; ct /= 2) {
     const int cols = (4 / a.ks) * ct * 16;
     blocks = 0;
-    for (int i = 0; i < n; ++i) blocks += (ws[i]->O + cols - 1) / cols;
+    for (int i = 0; i < a.n; ++i) {
+      a.m[i].cb0 = blocks;
+      blocks += (a.m[i].O + cols - 1) / cols;
+    }
     if (ct == 1 || blocks * row_tiles >= 3 * ctx->compute_units / 4) break;
   }
-  const int cols = (4 / a.ks) * ct * 16;
-  blocks = 0;
-  for (int i = 0; i < n; ++i) {
-    a.m[i] = mat_of(*ws[i], d_ys[i]);
-    a.m[i].cb0 = blocks;
-    blocks += (ws[i]->O + cols - 1) / cols;
-  }
   const dim3 grid(blocks, row_tiles);
-  const int lds = lds_bytes(a, cols, 64, ct, 4);
+  const int lds = lds_bytes(a, (4 / a.ks) * ct * 16, 64, ct, 4);
   return affine(a.m[0].kind) ? launch_affine(ctx, a, kPlain, ct, 64, -1, grid, lds) : launch_kq(ctx, a, kPlain, ct, 64, -1, grid, lds);
+}
+}  // namespace
+
+int plain(ornith_ctx* ctx, const ornith_linear* const* ws, int n, const void* d_x, int M, void* const* d_ys) {
+  // the matrices of one form share a launch
+  for (const bool form : {true, false}) {
+    Args a{};
+    a.x = (const bf16_t*)d_x;
+    a.M = M;
+    a.K = ws[0]->K;
+    for (int i = 0; i < n; ++i)
+      if (tall(*ws[i], M) == form) a.m[a.n++] = mat_of(*ws[i], d_ys[i]);
+    if (a.n == 0) continue;
+    const int rc = form ? launch_tall(ctx, a) : launch_split(ctx, a);
+    if (rc) return rc;
+  }
+  return ORNITH_OK;
 }
 
 int tile_rows(int pairs, int E) {
@@ -129,7 +158,7 @@ int launch_gathered(ornith_ctx* ctx, Args& a, int mode, const Plan& p, int O) {
   for (int i = 0; i < 4; ++i) {
     if (!a.m[i].q) continue;
     const int k = a.m[i].kind;
-    lds = std::max(lds, owned_x_bytes(p.rows, k, mode) + 128 * (a.K / 256) * (s_bytes(k) + d_bytes(k)));
+    lds = std::max(lds, owned_lds(p.rows, k, mode, a.K / 256));
     if (k != kind) kind = -1;
   }
   const dim3 grid((unsigned)(a.blocks * ((p.tiles_max + 7) / 8 * 8)));

@@ -28,7 +28,10 @@ def _weights(lin):
 @pytest.mark.parametrize("O,K,M", [(512, 2048, 32), (200, 512, 33), (264, 768, 48), (2048, 4096, 65), (40, 1024, 130),
                                     (4096, 2048, 64), (64, 4096, 17 + 64), (8, 2048, 200),
                                     # two and four column tiles a wavefront; an odd number of columns
-                                    (4096, 512, 65), (4096, 2048, 65), (4099, 2048, 130), (12288, 2048, 33)])
+                                    (4096, 512, 65), (4096, 2048, 65), (4099, 2048, 130), (12288, 2048, 33),
+                                    # columns owned by wavefronts: row tiles of 64 and remainders of 16, 32 and 48, two, three,
+                                    # eight and sixteen blocks of K, columns past the last workgroup's
+                                    (2056, 512, 193), (2184, 768, 481), (4099, 2048, 525), (2064, 4096, 449), (8192, 2048, 940)])
 def test_few_row_matmul_vs_float64(orn, ctx, fmt, O, K, M):
     rng = np.random.default_rng(O + K + M)
     lin = (util.HostLinear.kq(rng, Q4K if fmt == "q4k" else Q6K, O, K) if fmt[0] == "q" else
