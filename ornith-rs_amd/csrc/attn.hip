@@ -155,9 +155,38 @@ struct SdpaArgs {
   float scale;
   int finish;  // 1: every row has a single key block, the partial kernel applies the merge's
                //    arithmetic itself and writes `out` (no merge launch follows)
+  int by_die;  // the 1024-thread form's workgroups are numbered by die (sdpa_place)
 };
 
-// grid (nblk, Hq, T), 1024 threads: one query head against one block of ATT_KB keys.
+// Which (key block, first of N heads, row) a workgroup of a linear grid works on.
+// Workgroups go round the eight dies in order, and every die has an L2 of its own: with the block
+// index running fastest the heads and rows that read one key / value block sit on different dies, each
+// of which fetches it (nine rows at a 16 k context: 97 us against 82). So everything that reads one (block, KV head) is given to one die, next
+// to each other in its order. false: past the end (the last round of dies is padded).
+constexpr int kDies = 8, kManyHeads = 4;
+template <int N>
+__host__ __device__ __forceinline__ int sdpa_head_groups(const SdpaArgs& p) { return (p.Hq / p.Hkv + N - 1) / N; }
+// the (block, KV head, first head, how many of the N exist, row) of this workgroup
+template <int N>
+__device__ __forceinline__ bool sdpa_place(const SdpaArgs& p, int& b, int& hk, int& hq0, int& nh, int& t) {
+  const int group = p.Hq / p.Hkv, per = sdpa_head_groups<N>(p), sharers = per * p.T;
+  const int die = blockIdx.x % kDies, n = blockIdx.x / kDies, round = n / sharers, s = n - round * sharers;
+  const int pair = round * kDies + die;  // KV head fastest: the pairs of a short context on different dies
+  if (pair >= p.nblk * p.Hkv) return false;
+  b = pair / p.Hkv;
+  hk = pair - b * p.Hkv;
+  t = s / per;
+  const int h = (s - t * per) * N;
+  hq0 = hk * group + h;
+  nh = min(N, group - h);
+  return true;
+}
+template <int N>
+unsigned sdpa_die_grid(const SdpaArgs& p) {
+  return (unsigned)((p.nblk * p.Hkv + kDies - 1) / kDies * kDies * sdpa_head_groups<N>(p) * p.T);
+}
+
+// 1024 threads: one query head against one block of ATT_KB keys. Grid (nblk, Hq, T), with p.by_die sdpa_die_grid<1>.
 //
 // The sums: a key's score is one fma chain per 64 channels, the chains added pairwise
 // ((c0 + c1) + (c2 + c3)); a channel's output over the block is one chain per 64 keys, added
@@ -205,12 +234,16 @@ __device__ __forceinline__ float sdpa_pair_tree(const float* p, int stride) {
 template <int HD, bool PREP>
 __global__ __launch_bounds__(SDPA_NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void sdpa_partial_kernel(SdpaArgs p,
                                                                                                            PrepArgs q) {
-  const int b = blockIdx.x, hq = blockIdx.y, t = blockIdx.z, tid = threadIdx.x;
-  const int lane = tid & 63, wave = tid >> 6;
+  int b = blockIdx.x, hq = blockIdx.y, t = blockIdx.z, hk, one;
+  if (p.by_die) {
+    if (!sdpa_place<1>(p, b, hk, hq, one, t)) return;
+  } else {
+    hk = hq / (p.Hq / p.Hkv);
+  }
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int offset = PREP ? p.offset : (p.d_offset ? *p.d_offset : p.offset);
   const int last = min(offset + t, p.cap - 1);
   if (b * ATT_KB > last) return;
-  const int hk = hq / (p.Hq / p.Hkv);
 
   constexpr int PPR = HD / 8;                    // 16-byte pieces per row
   constexpr int RPU = SDPA_NT / PPR;             // value rows covered by one load per thread
@@ -426,31 +459,6 @@ __global__ __launch_bounds__(SDPA_NT) __attribute__((amdgpu_waves_per_eu(4, 4)))
   }
 }
 
-// Which (key block, first of four heads, row) a workgroup of a linear grid works on.
-// Workgroups go round the eight dies in order, and every die has an L2 of its own: with the block
-// index running fastest the heads and rows that read one key / value block sit on different dies, each
-// of which fetches it (nine rows at a 16 k context: 97 us against 82). So everything that reads one (block, KV head) is given to one die, next
-// to each other in its order. false: past the end (the last round of dies is padded).
-constexpr int kDies = 8, kManyHeads = 4;
-__host__ __device__ __forceinline__ int sdpa_head_groups(const SdpaArgs& p) { return (p.Hq / p.Hkv + kManyHeads - 1) / kManyHeads; }
-// the (KV head, first head, how many of the four exist, row) of this workgroup
-__device__ __forceinline__ bool sdpa_place(const SdpaArgs& p, int& b, int& hk, int& hq0, int& nh, int& t) {
-  const int group = p.Hq / p.Hkv, per = sdpa_head_groups(p), sharers = per * p.T;
-  const int die = blockIdx.x % kDies, n = blockIdx.x / kDies, round = n / sharers, s = n - round * sharers;
-  const int pair = round * kDies + die;  // KV head fastest: the pairs of a short context on different dies
-  if (pair >= p.nblk * p.Hkv) return false;
-  b = pair / p.Hkv;
-  hk = pair - b * p.Hkv;
-  t = s / per;
-  const int h = (s - t * per) * kManyHeads;
-  hq0 = hk * group + h;
-  nh = min(kManyHeads, group - h);
-  return true;
-}
-unsigned sdpa_many_grid(const SdpaArgs& p) {
-  return (unsigned)((p.nblk * p.Hkv + kDies - 1) / kDies * kDies * sdpa_head_groups(p) * p.T);
-}
-
 // The same partial sums when there are many blocks to work through (long contexts): several
 // workgroups resident per compute unit, and four query heads of a KV group in each, so that the key
 // and value block is read once for the four.
@@ -471,12 +479,12 @@ unsigned sdpa_many_grid(const SdpaArgs& p) {
 // 4 rows at 6621 keys 23.7 -> 17.4, 2 at 9000 23.2 -> 17.0, 6 at 1445 19.3 -> 12.3, 9 at 16000 117 -> 62.
 // (A KV group that is no multiple of four heads repeats its last one; what that makes is not stored. What
 // it costs stands at the choice of the form, sdpa_decode.)
-// grid sdpa_many_grid, 512 threads
+// grid sdpa_die_grid<kManyHeads>, 512 threads
 template <int HD>
 __global__ __launch_bounds__(512, 4) void sdpa_partial_many_kernel(SdpaArgs p) {
   constexpr int NH = kManyHeads, NT = 512;
   int b, hk, hq0, nh, t;
-  if (!sdpa_place(p, b, hk, hq0, nh, t)) return;
+  if (!sdpa_place<kManyHeads>(p, b, hk, hq0, nh, t)) return;
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int offset = p.d_offset ? *p.d_offset : p.offset;
@@ -846,17 +854,20 @@ static int sdpa_decode(ornith_ctx* ctx, const void* d_q_rot, const void* d_k_cac
   // place: groups of six 13.2 / 16.6 at 192 and 21.4 / 16.8 at 288, of three 13.0 / 16.7 and 20.0 / 16.8, of two
   // 15.9 / 18.2 at 256 and 21.4 / 17.0 at 384, of one (four times the arithmetic) 13.4 / 16.8 at 256, level from 288
   // to 512 (20.9 / 21.7, 22.9 / 22.7), 38.3 / 31.9 at 768.
-  // Those are numbers of key blocks that put the heads of one (block, KV head) on one die (the block runs
-  // fastest in the grid, over eight dies). With an odd number every head's workgroup fetches the block into
-  // another die's L2 and the 1024-thread form takes longer the more there are of them: one row, 9 / 11 / 13 / 15
-  // blocks 16.9 / 17.9 / 19.1 / 19.8 us, 8 / 10 / 12 / 14 / 16 blocks 12.4 / 14.3 / 13.3 / 15.2 / 13.3; at head width 128 12.0 to
-  // 13.5 and 10.7 to 11.5. That is the grid's numbering to mend, not this line's place.
   // Inside the first key block the 1024-thread form finishes by itself, without the merge launch, and a second
   // round is still ahead: 31 rows (496 workgroups) at 0 / 200 keys 12.0 / 22.5 and 17.1 / 22.8.
-  const dim3 grid(nblk, Hq, T);
   const int last_max = (d_offset ? cap - 1 : (offset + T - 1 < cap - 1 ? offset + T - 1 : cap - 1));
   const long live = (long)(last_max / ATT_KB + 1) * Hq * T;
   const bool many = live > (last_max < ATT_KB ? 2L : 1L) * ctx->compute_units;
+  // How the 1024-thread form's workgroups are numbered. With the block running fastest and an odd number of blocks, every
+  // head's workgroup fetches a (block, KV head) into another die's L2, the longer the more blocks there are; by die it
+  // is fetched once. One row of two KV groups of eight heads, us, block fastest / by die: 5 blocks 13.9 / 12.6, 7
+  // 14.8 / 12.6, 9 15.9 / 12.7, 13 18.0 / 12.8, 15 18.3 / 12.9; even numbers
+  // level (12.4 to 13.3 both). At head width 128 the odd numbers took 12.0 to 13.5 where the even ones took 10.7 to 11.5. One or two blocks are too few to matter (12.2 / 12.4), and where the pairs leave a die more workgroups than it has
+  // compute units (a workgroup has one to itself), its second round costs more than it saves (five rows, two blocks: 12.2 / 19.9).
+  const long a_die = (long)((nblk * Hkv + kDies - 1) / kDies) * (Hq / Hkv) * T;
+  p.by_die = nblk >= 3 && a_die * kDies <= ctx->compute_units;
+  const dim3 grid = p.by_die ? dim3(sdpa_die_grid<1>(p)) : dim3(nblk, Hq, T);
   // one key block for every row, in the kernel form that knows how to finish: no merge launch
   p.finish = (last_max < ATT_KB && !many) ? 1 : 0;
   const bool fold = prep && !many && !d_offset && T <= 8 && ornith_option_fuse_attn_prep();
@@ -870,9 +881,9 @@ static int sdpa_decode(ornith_ctx* ctx, const void* d_q_rot, const void* d_k_cac
   }
   if (many) {
     if (hd == 256)
-      hipLaunchKernelGGL(sdpa_partial_many_kernel<256>, dim3(sdpa_many_grid(p)), dim3(512), 0, ctx->stream, p);
+      hipLaunchKernelGGL(sdpa_partial_many_kernel<256>, dim3(sdpa_die_grid<kManyHeads>(p)), dim3(512), 0, ctx->stream, p);
     else
-      hipLaunchKernelGGL(sdpa_partial_many_kernel<128>, dim3(sdpa_many_grid(p)), dim3(512), 0, ctx->stream, p);
+      hipLaunchKernelGGL(sdpa_partial_many_kernel<128>, dim3(sdpa_die_grid<kManyHeads>(p)), dim3(512), 0, ctx->stream, p);
   } else if (hd == 256) {
     // 150 KB of LDS a block (the whole key block staged at once): asked for once per kernel
     if (!(ctx->lds_attr_set & 1)) {

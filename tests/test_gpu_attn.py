@@ -30,6 +30,10 @@ def _mk(rng, T, Hq, Hkv, hd, cap, offset):
     # ... with KV groups that are no multiple of four heads (three, one, two, six, five), and of eight (ragged last block)
     (8, 6, 2, 256, 8192, 8000), (4, 16, 16, 256, 2048, 1500), (4, 16, 8, 256, 2048, 1500), (2, 24, 4, 256, 4096, 3000),
     (7, 10, 2, 128, 4096, 3300), (3, 16, 2, 256, 8192, 7000),
+    # the 1024-thread form numbered by die: from three blocks on, odd numbers of them, ragged KV groups, new rows across a block's
+    # end, as many workgroups a die as it has compute units, and one row more (block fastest, or the other form)
+    (1, 16, 2, 256, 4096, 513), (1, 16, 2, 256, 4096, 2300), (2, 16, 2, 256, 4096, 1790), (1, 6, 2, 128, 4096, 3300),
+    (3, 5, 1, 256, 2048, 766), (4, 16, 2, 256, 4096, 800), (5, 16, 2, 256, 4096, 700), (1, 16, 16, 256, 2048, 600),
     # ... from one workgroup of the other form more than there are compute units: the last call before that, and the first
     (4, 16, 2, 256, 4096, 1020), (4, 16, 1, 128, 4096, 1021),
     # 16-row prompt chunks inside the first key block (one finishing launch, of two rounds from 17 rows on) and across
