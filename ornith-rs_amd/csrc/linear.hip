@@ -146,11 +146,12 @@ __global__ void embedding4_kernel(const uint8_t* w, const bf16_t* scales, const 
 // the shared expert's gate: O of 1 .. 64): as mat-vecs every activation row is read by O / 4
 // workgroups. One workgroup = 16 rows; its wavefronts split K and add up through LDS; a
 // wavefront feeds v_mfma_f32_16x16x32_bf16 straight from global memory (A: 16 rows x 32
-// channels, B: 16 outputs x 32 channels, 16 bytes a lane each). grid.y covers O in 64s.
+// channels, B: 16 outputs x 32 channels, 16 bytes a lane each). grid.y covers O in NT tiles of 16.
 // A launch is one latency chain of some workgroups, so K goes over as many wavefronts as it
-// divides into 128-channel pieces (up to 16) and a wavefront asks for a piece's operands at once:
-// 2 x 32 outputs of K = 2048, 51 / 700 / 6621 rows, with four wavefronts 24.4 / 24.5 / 25.5 us, with
-// sixteen 12.7 / 13.5 / 24.1.
+// divides into 128-channel pieces (up to 16) and a wavefront asks for a piece's operands at once: 2 x 32
+// outputs of K = 2048, 51 / 700 / 6621 rows, with four wavefronts 24.4 / 24.5 / 25.5 us, with sixteen (four tiles)
+// 11.6 / 11.8 / 22.0. What bounds it is the L1: sixteen lanes in a row ask for sixteen lines, 64 clocks a load, 320 loads a
+// workgroup with four tiles. One tile a workgroup asks 128 times: 5.9 / 6.0 us.
 typedef __bf16 dmm_bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float dmm_f32x4_t __attribute__((ext_vector_type(4)));
 
@@ -161,21 +162,21 @@ struct DenseMmSegs {
   int n;
 };
 
-template <int NW>
+template <int NW, int NT>
 __global__ __launch_bounds__(64 * NW) void dense_mm_kernel(DenseMmSegs s, const bf16_t* x, int M, int K) {
-  __shared__ __attribute__((aligned(16))) dmm_f32x4_t red[NW][4][64];
+  __shared__ __attribute__((aligned(16))) dmm_f32x4_t red[NW][NT][64];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l16 = lane & 15, lg = lane >> 4;
   const int row0 = blockIdx.x * 16;
   const int kw = K / NW, k0 = wave * kw;  // a multiple of 32
   const bf16_t* xp = x + (size_t)min(row0 + l16, M - 1) * K + k0 + 8 * lg;
-  // the four 16-output tiles of this workgroup: tile 4 * blockIdx.y + nt of the segments' tiles
-  // laid end to end (a segment's last tile may be ragged)
-  const bf16_t* wp[4];
-  bf16_t* yp[4];
-  int ocol[4], oend[4], ostride[4];
+  // the 16-output tiles of this workgroup: tile NT * blockIdx.y + nt of the segments' tiles laid end to end (a
+  // segment's last tile may be ragged)
+  const bf16_t* wp[NT];
+  bf16_t* yp[NT];
+  int ocol[NT], oend[NT], ostride[NT];
 #pragma unroll
-  for (int nt = 0; nt < 4; ++nt) {
-    int t = 4 * blockIdx.y + nt, seg = -1;
+  for (int nt = 0; nt < NT; ++nt) {
+    int t = NT * blockIdx.y + nt, seg = -1;
 #pragma unroll
     for (int i = 0; i < 4; ++i)
       if (seg < 0 && i < s.n) {
@@ -189,23 +190,23 @@ __global__ __launch_bounds__(64 * NW) void dense_mm_kernel(DenseMmSegs s, const 
     yp[nt] = s.y[sg];
     wp[nt] = s.w[sg] + (size_t)min(ocol[nt], s.O[sg] - 1) * K + k0 + 8 * lg;
   }
-  dmm_f32x4_t acc[4];
+  dmm_f32x4_t acc[NT];
 #pragma unroll
-  for (int nt = 0; nt < 4; ++nt) acc[nt] = dmm_f32x4_t{0.f, 0.f, 0.f, 0.f};
+  for (int nt = 0; nt < NT; ++nt) acc[nt] = dmm_f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll 4
   for (int k = 0; k < kw; k += 32) {
     const dmm_bf16x8_t a = *reinterpret_cast<const dmm_bf16x8_t*>(xp + k);
 #pragma unroll
-    for (int nt = 0; nt < 4; ++nt)
-      if (oend[nt] > 0) {  // (the same for every lane of the wavefront)
+    for (int nt = 0; nt < NT; ++nt)
+      if (NT == 1 || oend[nt] > 0) {  // (the same for every lane of the wavefront; a single tile is always one of the launch's)
         const dmm_bf16x8_t b = *reinterpret_cast<const dmm_bf16x8_t*>(wp[nt] + k);
         acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[nt], 0, 0, 0);
       }
   }
 #pragma unroll
-  for (int nt = 0; nt < 4; ++nt) red[wave][nt][lane] = acc[nt];
+  for (int nt = 0; nt < NT; ++nt) red[wave][nt][lane] = acc[nt];
   __syncthreads();
-  if (wave >= 4) return;
+  if (wave >= NT) return;
   // output tile nt = wave: D[m = 4 * lg + r][n = l16]
   dmm_f32x4_t v = red[0][wave][lane];
 #pragma unroll
@@ -213,7 +214,7 @@ __global__ __launch_bounds__(64 * NW) void dense_mm_kernel(DenseMmSegs s, const 
   int col = 0, end = 0, stride = 0;
   bf16_t* y = nullptr;
 #pragma unroll
-  for (int nt = 0; nt < 4; ++nt)
+  for (int nt = 0; nt < NT; ++nt)
     if (nt == wave) {
       col = ocol[nt];
       end = oend[nt];
@@ -244,14 +245,19 @@ static bool launch_dense_mm(ornith_ctx* ctx, const ornith_linear* const* ws, int
     s.O[i] = ws[i]->O;
     tiles += (ws[i]->O + 15) / 16;
   }
-  const dim3 grid((M + 15) / 16, (tiles + 3) / 4);
-  const int K = ws[0]->K;
-  if (K % 2048 == 0)
-    hipLaunchKernelGGL(dense_mm_kernel<16>, grid, dim3(1024), 0, ctx->stream, s, (const bf16_t*)d_x, M, K);
-  else if (K % 1024 == 0)
-    hipLaunchKernelGGL(dense_mm_kernel<8>, grid, dim3(512), 0, ctx->stream, s, (const bf16_t*)d_x, M, K);
-  else
-    hipLaunchKernelGGL(dense_mm_kernel<4>, grid, dim3(256), 0, ctx->stream, s, (const bf16_t*)d_x, M, K);
+  // One tile a workgroup while two workgroups a compute unit hold them all (a single tile always:
+  // 5.2 -> 4.9 us, at 6621 rows 8.8 -> 6.9); past that the rows read four times cost more than the loads' time divided by four
+  // saves. Four tiles, us, four a workgroup / one: 51 rows 11.6 / 5.9, 700 11.8 / 6.0, 1500 11.9 / 9.7, 2048 (two a unit) 11.9 / 9.5, 3000
+  // 12.0 / 12.9, 6621 22.0 / 28.5.
+  const int rt = (M + 15) / 16, K = ws[0]->K;
+  const bool one = tiles == 1 || (long)rt * tiles <= 2L * ctx->compute_units;
+  const dim3 grid(rt, one ? tiles : (tiles + 3) / 4);
+  typedef void (*Kernel)(DenseMmSegs, const bf16_t*, int, int);
+  static const Kernel kernels[3][2] = {{dense_mm_kernel<16, 4>, dense_mm_kernel<16, 1>},
+                                       {dense_mm_kernel<8, 4>, dense_mm_kernel<8, 1>},
+                                       {dense_mm_kernel<4, 4>, dense_mm_kernel<4, 1>}};
+  const int form = K % 2048 == 0 ? 0 : K % 1024 == 0 ? 1 : 2;
+  hipLaunchKernelGGL(kernels[form][one], grid, dim3(1024 >> form), 0, ctx->stream, s, (const bf16_t*)d_x, M, K);
   return true;
 }
 
