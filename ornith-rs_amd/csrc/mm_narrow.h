@@ -32,8 +32,8 @@
 // operands is 18 instructions for eight weights (scaled()). The plain launches of a short prompt are one pass of a
 // chain: load, unpack, multiply, meet (vector units 13 %).
 //
-// Measured (us, before -> now): 12288 x 2048 Q4_K at 64 rows 29.5 -> 15.8 -> 14.8, 2048 x 4096 at 64 rows 52 -> 11.8,
-// 256 x 2048 Q6_K 28.6 -> 7.1; the experts, gate + up + swiglu / down (the shared expert included): a 51-token prompt
+// Measured (us, before -> now): 12288 x 2048 Q4_K at 64 rows 29.5 -> 15.8 -> 14.8, 2048 x 4096 at 64 rows 52 -> 9.6 -> 7.2,
+// 256 x 2048 Q6_K 28.6 -> 6.6 -> 5.4; the experts, gate + up + swiglu / down (the shared expert included): a 51-token prompt
 // 104 / 49 -> 53 / 36 with K split -> 47 / 38 with columns owned, a 700-token one 156 / 76 -> 122 / 81 -> 90 / 69, over 4-bit
 // affine weights at 600 tokens 109 / 62 -> 98 / 51; a 600-token prompt over 4-bit affine weights as a whole 461 ms
 // (mat-vecs, row by row) -> 15.9 -> 14.8 ms.

@@ -8,7 +8,7 @@ namespace nmm {
 
 // Rows up to which a k-quant projection takes these kernels: the wide kernels' 256 x 128 tiles fill the device from about a
 // thousand rows of 12288 columns on, and for up to 2048 columns not before a thousand rows either (2048 x 4096, us here /
-// there: 64 rows 11.8 / 52, 256 rows 17 / 53, 700 rows 33 / 54, 1024 rows 38 / 55; 256 x 2048: 7 / 29, 1024 rows 9 / 29).
+// there: 64 rows 7.2 / 52, 256 rows 15 / 53, 700 rows 29 / 54, 1024 rows 38 / 55; 256 x 2048: 5 / 29, 1024 rows 9 / 29).
 // More columns than that go from K split over wavefronts to columns owned by them (kTall) at kNarrowRows rows, where the
 // former's activations, read by every 64 columns, start to weigh (12288 x 2048 Q4_K, us, split / owned / wide kernels:
 // 128 rows 20 / 20 / 29, 200 rows 30 / 26 / 42, 300 rows - / 26 / 41, 512 rows - / 35 / 42, 700 rows - / 53 / 66, 900 rows
@@ -52,9 +52,9 @@ int launch_affine(ornith_ctx* ctx, const Args& a, int mode, int ct, int rows, in
 // its widest path. A workgroup is four wavefronts, one a SIMD; a compute unit holds two plain ones, and as many
 // gathered ones as registers and LDS allow (WAVES: asked for, a SIMD).
 #define NMM_KERNELS(NAME, AFF, K1, K2, WAVES, LDS_BIT)                                                              \
-  template <int CT>                                                                                                 \
+  template <int CT, int ROWS>                                                                                       \
   __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void NAME##_plain_kernel(Args a) {   \
-    body<AFF, CT, kPlain, 64, 4>(a);                                                                                \
+    body<AFF, CT, kPlain, ROWS, 4>(a);                                                                              \
   }                                                                                                                 \
   template <int MODE, int ROWS, int KIND>                                                                           \
   __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES(KIND, ROWS)))) void                    \
@@ -67,7 +67,9 @@ int launch_affine(ornith_ctx* ctx, const Args& a, int mode, int ct, int rows, in
   }                                                                                                                 \
   int launch_##NAME(ornith_ctx* ctx, const Args& a, int mode, int ct, int rows, int kind, dim3 grid, int lds) {     \
     typedef void (*Kernel)(Args);                                                                                   \
-    static const Kernel plain[3] = {NAME##_plain_kernel<1>, NAME##_plain_kernel<2>, NAME##_plain_kernel<4>};        \
+    static const Kernel plain[3][2] = {{NAME##_plain_kernel<1, 32>, NAME##_plain_kernel<1, 64>},                    \
+                                       {NAME##_plain_kernel<2, 32>, NAME##_plain_kernel<2, 64>},                    \
+                                       {NAME##_plain_kernel<4, 64>, NAME##_plain_kernel<4, 64>}};                   \
     static const Kernel tall[2] = {NAME##_tall_kernel<K1>, NAME##_tall_kernel<AFF ? -1 : K1>};                      \
     static const Kernel gather[3][2][3] = {                                                                         \
         {{NAME##_gather_kernel<kGather, 16, K1>, NAME##_gather_kernel<kGather, 32, K1>, NAME##_gather_kernel<kGather, 64, K1>},     \
@@ -77,8 +79,9 @@ int launch_affine(ornith_ctx* ctx, const Args& a, int mode, int ct, int rows, in
         {{NAME##_gather_kernel<kGather, 16, -1>, NAME##_gather_kernel<kGather, 32, -1>, NAME##_gather_kernel<kGather, 64, -1>},     \
          {NAME##_gather_kernel<kGateUp, 16, -1>, NAME##_gather_kernel<kGateUp, 32, -1>, NAME##_gather_kernel<kGateUp, 64, -1>}}};   \
     if (!(ctx->lds_attr_set & LDS_BIT)) {                                                                           \
-      for (const Kernel k : plain)                                                                                  \
-        ORN_HIP(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes));        \
+      for (const auto& p : plain)                                                                                   \
+        for (const Kernel k : p)                                                                                    \
+          ORN_HIP(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes));      \
       for (const Kernel k : tall)                                                                                   \
         ORN_HIP(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes));        \
       for (const auto& g : gather)                                                                                  \
@@ -88,7 +91,7 @@ int launch_affine(ornith_ctx* ctx, const Args& a, int mode, int ct, int rows, in
       ctx->lds_attr_set |= LDS_BIT;                                                                                 \
     }                                                                                                               \
     const int of = kind == K1 ? 0 : kind == K2 ? 1 : 2;                                                             \
-    const Kernel k = mode == kPlain ? plain[ct / 2] : mode == kTall ? tall[of != 0] : gather[of][mode == kGateUp][rows / 32]; \
+    const Kernel k = mode == kPlain ? plain[ct / 2][rows / 64] : mode == kTall ? tall[of != 0] : gather[of][mode == kGateUp][rows / 32]; \
     hipLaunchKernelGGL(k, grid, dim3(256), lds, ctx->stream, a);                                                    \
     ORN_LAUNCH_CHECK("nmm::" #NAME);                                                                                \
     return ORNITH_OK;                                                                                               \

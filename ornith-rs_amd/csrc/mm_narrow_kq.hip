@@ -91,22 +91,48 @@ int launch_tall(ornith_ctx* ctx, Args& a) {
 
 int launch_split(ornith_ctx* ctx, Args& a) {
   a.ks = k_split(a.K, 4);
-  const int row_tiles = (a.M + 63) / 64;
-  // Columns a workgroup: 64 (four tiles a wavefront, each activation fragment used four times)
-  // once that gives most compute units a workgroup, else 32 or 16.
-  int ct = 4, blocks = 0;
-  for (;; ct /= 2) {
+  // The tile, columns x rows; sums and their order are the same in all of them.
+  // While one workgroup a compute unit covers the product with 32-row tiles, those: a workgroup asks for its rows'
+  // activations over all of K (64 rows of K = 4096: 512 KB, 4 us of the unit's address path), and half the
+  // rows are half of that. us, 64-row tiles / 32-row ones: 2048 x 4096 Q4_K 51 rows 9.4 / 7.2, Q6_K 11.0 / 8.8, 4-bit affine
+  // 12.6 / 9.5; 256 x 2048 Q6_K 51 .. 450 rows 6.6 .. 6.8 / 5.4 .. 5.7, 8-bit affine 7.6 / 6.4. One workgroup more and the second round
+  // costs what that gave (2048 x 4096 at 100 rows 10.3 / 10.3, at 150 14.3 / 14.7; 256 x 2048 8-bit affine at 600 7.8 / 10.5).
+  // With 32 columns the same holds from four blocks a wavefront on (2048 x 4096 at 100 rows: Q4_K 10.3 / 9.3, 4-bit affine 12.1 / 11.2;
+  // K = 2048 has two: 256 columns at 600 rows 7.2 / 7.6, 8-bit affine 7.9 / 9.0), but for Q6_K, whose unpacking is the longer
+  // part (80 / 100 / 128 rows 10.7 / 11.5 / 12.8, here 12.1 / 12.2 / 12.2).
+  // With 64-row tiles 64 columns (four tiles a wavefront, each activation fragment used four times) once that gives
+  // most compute units a workgroup, else 32 or 16. They have to share a compute unit once there is more than one for each: with
+  // Q6_K's 18 bytes of scales a block they don't at K = 4096 (82 KB of LDS), and take 32 columns (2048 columns, 600 / 700 / 900 rows
+  // 45.7 / 46.2 / 46.3 -> 35.4 / 36.0 / 45.1; at 450 rows, one each, 24.1 / 24.8).
+  auto blocks_of = [&](int ct) {
     const int cols = (4 / a.ks) * ct * 16;
-    blocks = 0;
+    a.blocks = 0;
     for (int i = 0; i < a.n; ++i) {
-      a.m[i].cb0 = blocks;
-      blocks += (a.m[i].O + cols - 1) / cols;
+      a.m[i].cb0 = a.blocks;
+      a.blocks += (a.m[i].O + cols - 1) / cols;
     }
-    if (ct == 1 || blocks * row_tiles >= 3 * ctx->compute_units / 4) break;
+    return a.blocks;
+  };
+  bool q6 = false;
+  for (int i = 0; i < a.n; ++i) q6 = q6 || a.m[i].kind == kQ6K;
+  const int units = ctx->compute_units, thirty = (a.M + 31) / 32, sixty = (a.M + 63) / 64;
+  int ct = 4, rows = 64;
+  if ((long)blocks_of(1) * thirty <= units) {
+    ct = 1;
+    rows = 32;
+  } else if (!q6 && a.K >= 4096 && (long)blocks_of(2) * thirty <= units) {
+    ct = 2;
+    rows = 32;
+  } else {
+    auto suits = [&]() {
+      const long n = (long)blocks_of(ct) * sixty;
+      return n >= 3 * units / 4 && (n <= units || lds_bytes(a, (4 / a.ks) * ct * 16, 64, ct, 4) <= kLdsBytes / 2);
+    };
+    while (ct > 1 && !suits()) ct /= 2;
   }
-  const dim3 grid(blocks, row_tiles);
-  const int lds = lds_bytes(a, (4 / a.ks) * ct * 16, 64, ct, 4);
-  return affine(a.m[0].kind) ? launch_affine(ctx, a, kPlain, ct, 64, -1, grid, lds) : launch_kq(ctx, a, kPlain, ct, 64, -1, grid, lds);
+  const dim3 grid(blocks_of(ct), rows == 32 ? thirty : sixty);
+  const int lds = lds_bytes(a, (4 / a.ks) * ct * 16, rows, ct, 4);
+  return affine(a.m[0].kind) ? launch_affine(ctx, a, kPlain, ct, rows, -1, grid, lds) : launch_kq(ctx, a, kPlain, ct, rows, -1, grid, lds);
 }
 }  // namespace
 

@@ -29,6 +29,11 @@ def _weights(lin):
                                     (4096, 2048, 64), (64, 4096, 17 + 64), (8, 2048, 200),
                                     # two and four column tiles a wavefront; an odd number of columns
                                     (4096, 512, 65), (4096, 2048, 65), (4099, 2048, 130), (12288, 2048, 33),
+                                    # 32-row tiles: the last product that one workgroup a compute unit covers with 16 columns
+                                    # each, with 32, and the first past both; remainders of 1 and 17 rows; 64-row tiles whose
+                                    # scales would leave a compute unit one workgroup
+                                    (2048, 4096, 64), (2040, 4096, 113), (2048, 4096, 129), (2048, 2048, 65), (256, 2048, 512),
+                                    (2048, 4096, 577),
                                     # columns owned by wavefronts: row tiles of 64 and remainders of 16, 32 and 48, two, three,
                                     # eight and sixteen blocks of K, columns past the last workgroup's
                                     (2056, 512, 193), (2184, 768, 481), (4099, 2048, 525), (2064, 4096, 449), (8192, 2048, 940)])
