@@ -654,59 +654,74 @@ __global__ __launch_bounds__(512, 4) void sdpa_partial_many_kernel(SdpaArgs p) {
   }
 }
 
-// grid (Hq, T), HD threads: merge blocks ascending, divide, gate.
-// Thread b fetches block b's maximum and sum (one load each for the whole row), every thread
-// asks for its channel's partial outputs of up to kMergeAhead blocks at once, and the block
-// weights exp(m_b - M) are made once (thread b) and shared through LDS; the sums over the blocks
-// stay one ascending fma chain per thread. (A loop that fetched the maxima one by one and then
-// eight blocks at a time was a dozen trips to memory for a 27-block row.)
+// Merge: blocks ascending, divide, gate. Grid (Hq, T), one wavefront a row, HD / 64 channels a lane.
+// A few trips to memory and little else: lane b fetches block b's maximum and sum, every lane asks for its
+// channels' partial outputs of up to kMergeAhead blocks in the same trip, and the block weights exp(m_b - M) are made once (lane b)
+// and read from its lane; the sums over the blocks stay one ascending fma chain a channel. A load
+// takes the address path 16 clocks whatever its width, so a lane takes all its channels in one. As HD / 64 wavefronts of
+// one channel a lane, which asked for the outputs behind the maxima and for 32 blocks whatever the row had, us a launch, before / now: one
+// row, 10 blocks 4.0 / 2.9, 63 blocks 5.6 / 4.8, two rows of 24 blocks 4.0 / 3.6, four rows of 27 4.0 / 3.9; whole calls, one row, 2 blocks
+// 12.2 / 10.8, 6 blocks 12.9 / 11.1, 36 blocks 19.0 / 17.3.
 constexpr int kMergeAhead = 32;
 template <int HD>
-__global__ __launch_bounds__(HD) void sdpa_merge_kernel(SdpaArgs p) {
-  const int h = blockIdx.x, t = blockIdx.y, d = threadIdx.x;
-  const int lane = d & 63, wave = d >> 6;
+__global__ __launch_bounds__(64) void sdpa_merge_kernel(SdpaArgs p) {
+  constexpr int PER = HD / 64, SET = 8;
+  typedef float chan_t __attribute__((ext_vector_type(PER)));
+  typedef uint32_t bits_t __attribute__((ext_vector_type(PER / 2)));
+  const int h = blockIdx.x, t = blockIdx.y, lane = threadIdx.x;
   const int offset = p.d_offset ? *p.d_offset : p.offset;
   const int last = min(offset + t, p.cap - 1);
   const int nb = last / ATT_KB + 1;
   const size_t pi = ((size_t)t * p.Hq + h) * p.nblk;
-  __shared__ float sw[kMergeAhead], sl[kMergeAhead];
-  __shared__ float red[HD / 64];
-  const bf16_t gate_bits = p.qg[((size_t)t * p.Hq + h) * 2 * HD + HD + d];
-  // the row's maximum: every thread over its blocks d, d + HD, ..., then over the workgroup
-  float M = -DM_INF;
-  for (int b = d; b < nb; b += HD) {
-    const float m = p.part_m[pi + b];
+  const float *pm = p.part_m + pi, *pl = p.part_l + pi, *po = p.part_o + pi * HD + PER * lane;
+  float mb = pm[min(lane, nb - 1)], lb = pl[min(lane, nb - 1)];
+  chan_t v[kMergeAhead];
+  auto fetch = [&](int b0) {  // sets of blocks that the row has (the last one repeats its last block)
+#pragma unroll
+    for (int s = 0; s < kMergeAhead; s += SET)
+      if (b0 + s < nb)
+#pragma unroll
+        for (int u = s; u < s + SET; ++u) v[u] = *reinterpret_cast<const chan_t*>(po + (size_t)min(b0 + u, nb - 1) * HD);
+  };
+  fetch(0);
+  bits_t gate;
+  __builtin_memcpy(&gate, p.qg + ((size_t)t * p.Hq + h) * 2 * HD + HD + PER * lane, sizeof gate);  // (as the caller has aligned it)
+  float M = mb > -DM_INF ? mb : -DM_INF;
+  for (int b = lane + 64; b < nb; b += 64) {
+    const float m = pm[b];
     M = m > M ? m : M;
   }
   M = dm_wave_max<64>(M);
-  if (lane == 0) red[wave] = M;
-  __syncthreads();
-  M = red[0];
+  float L = 0.f;
+  chan_t O = 0.f;
+  for (int b0 = 0;;) {
+    const float w = dm_exp(mb - M);
 #pragma unroll
-  for (int w = 1; w < HD / 64; ++w) M = red[w] > M ? red[w] : M;
-  float L = 0.f, O = 0.f;
-  for (int b0 = 0; b0 < nb; b0 += kMergeAhead) {
-    const int n = min(kMergeAhead, nb - b0);
-    float po[kMergeAhead];
+    for (int s = 0; s < kMergeAhead; s += SET)
+      if (b0 + s < nb)
 #pragma unroll
-    for (int u = 0; u < kMergeAhead; ++u) po[u] = p.part_o[(pi + b0 + min(u, n - 1)) * HD + d];
-    __syncthreads();  // the previous round's weights have been read
-    if (d < n) {
-      sw[d] = dm_exp(p.part_m[pi + b0 + d] - M);
-      sl[d] = p.part_l[pi + b0 + d];
-    }
-    __syncthreads();
+        for (int u = s; u < s + SET; ++u) {
+          const float wu = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, w), u));
+          const float lu = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, lb), u));
+          if (b0 + u < nb) {
+            L = dm_fma(lu, wu, L);
 #pragma unroll
-    for (int u = 0; u < kMergeAhead; ++u)
-      if (u < n) {
-        const float w = sw[u];
-        L = dm_fma(sl[u], w, L);
-        O = dm_fma(po[u], w, O);
-      }
+            for (int c = 0; c < PER; ++c) O[c] = dm_fma(v[u][c], wu, O[c]);
+          }
+        }
+    b0 += kMergeAhead;
+    if (b0 >= nb) break;
+    mb = pm[min(b0 + lane, nb - 1)];
+    lb = pl[min(b0 + lane, nb - 1)];
+    fetch(b0);
   }
-  const float att = dm_rb(O / L);
-  const float g = dm_sigmoid_bf16(dm_bf2f(gate_bits));
-  p.out[((size_t)t * p.Hq + h) * HD + d] = dm_f2bf(g * att);
+  bits_t out;
+#pragma unroll
+  for (int c = 0; c < PER; c += 2) {
+    const float g0 = dm_sigmoid_bf16(dm_bf2f_lo(gate[c / 2])), g1 = dm_sigmoid_bf16(dm_bf2f_hi(gate[c / 2]));
+    out[c / 2] = dm_f2bf2(g0 * dm_rb(O[c] / L), g1 * dm_rb(O[c + 1] / L));
+  }
+  __builtin_memcpy(p.out + ((size_t)t * p.Hq + h) * HD + PER * lane, &out, sizeof out);
 }
 
 }  // namespace
@@ -913,9 +928,9 @@ static int sdpa_decode(ornith_ctx* ctx, const void* d_q_rot, const void* d_k_cac
   ORN_LAUNCH_CHECK("sdpa_partial_kernel");
   if (p.finish) return ORNITH_OK;
   if (hd == 256)
-    hipLaunchKernelGGL(sdpa_merge_kernel<256>, dim3(Hq, T), dim3(256), 0, ctx->stream, p);
+    hipLaunchKernelGGL(sdpa_merge_kernel<256>, dim3(Hq, T), dim3(64), 0, ctx->stream, p);
   else
-    hipLaunchKernelGGL(sdpa_merge_kernel<128>, dim3(Hq, T), dim3(128), 0, ctx->stream, p);
+    hipLaunchKernelGGL(sdpa_merge_kernel<128>, dim3(Hq, T), dim3(64), 0, ctx->stream, p);
   ORN_LAUNCH_CHECK("sdpa_merge_kernel");
   return ORNITH_OK;
 }
