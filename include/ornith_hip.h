@@ -401,8 +401,8 @@ ORNITH_API int ornith_sdpa_decode_gated(ornith_ctx* ctx, const void* d_q_rot, co
                                         float scale, void* d_out);
 /* ornith_attn_prep followed by ornith_sdpa_decode_gated on the same rows, as Attention::forward
  * runs them (src/model/qwen3_5.rs:430-474), host-side offset: the same results and the same
- * cache contents; at decode widths (T <= 8, a context short enough for the one-workgroup-per-
- * block form) one launch does both -- every workgroup makes its query row and the call's new
+ * cache contents; at decode widths (T <= 8, in the forms with one workgroup a block and head and with
+ * one for eight heads) one launch does both -- every workgroup makes its query row and the call's new
  * key rows itself, and the caches are written as a side effect. d_q_rot is only written when
  * the prep runs as its own launch. */
 ORNITH_API int ornith_attn_decode(ornith_ctx* ctx, const void* d_qg, const void* d_kx, const void* d_vx,

@@ -10,8 +10,8 @@
 // and sigmoid_gate (kernels/ornith_elementwise.metal).
 //
 // Attention is split over keys in blocks of 256 by absolute position, one
-// workgroup per (block, query head, query row), or for four heads of a KV group where
-// there are many of them: a key's score is one fma chain per
+// workgroup per (block, query head, query row), or for four or eight heads of a KV group
+// where there are many of them: a key's score is one fma chain per
 // 64 channels with the chains added pairwise, a channel's output one fma chain per
 // 64 keys of the block added the same way, so neither needs a cross-lane reduction
 // per key. The partial (max, sum, values) of each block go to scratch and a second
@@ -51,26 +51,22 @@ struct PrepArgs {
 // returns the normed, rotated values (rounded to bf16 by whoever stores them).
 template <int PER>
 struct PrepRegs {
-  bf16_t x[PER], w[PER];
+  uint32_t x[PER / 2], w[PER / 2];  // pairs
   float c[PER], s[PER];
 };
 
-template <int PER>
+template <int PER, bool NORMED = false>
 __device__ __forceinline__ void prep_issue(const bf16_t* src, const bf16_t* w, const float* cos_t, const float* sin_t,
                                            int pos, int half, int lane, PrepRegs<PER>& g) {
-#pragma unroll
-  for (int i = 0; i < PER; ++i) g.x[i] = src[lane * PER + i];
-  if (w) {
-#pragma unroll
-    for (int i = 0; i < PER; ++i) g.w[i] = w[lane * PER + i];
+  __builtin_memcpy(g.x, src + lane * PER, sizeof g.x);
+  if (NORMED || w) {
+    __builtin_memcpy(g.w, w + lane * PER, sizeof g.w);
     const int hl = half / PER;
     const bool lowg = lane < hl, rot = lane < 2 * hl;
-#pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      const int e = (lowg ? lane : lane - hl) * PER + i;
-      g.c[i] = rot ? cos_t[(size_t)pos * half + e] : 0.f;
-      g.s[i] = rot ? sin_t[(size_t)pos * half + e] : 0.f;
-    }
+    // (a lane's entries lie side by side: one load each of the two tables; lanes that rotate nothing read the first ones)
+    const size_t e = (size_t)pos * half + (rot ? (lowg ? lane : lane - hl) * PER : 0);
+    __builtin_memcpy(g.c, cos_t + e, sizeof g.c);
+    __builtin_memcpy(g.s, sin_t + e, sizeof g.s);
   }
 }
 
@@ -79,14 +75,14 @@ __device__ __forceinline__ void prep_finish(const PrepRegs<PER>& g, bool normed,
                                             float (&x)[PER]) {
   constexpr int HD = 64 * PER;
 #pragma unroll
-  for (int i = 0; i < PER; ++i) x[i] = dm_bf2f(g.x[i]);
+  for (int i = 0; i < PER; ++i) x[i] = i & 1 ? dm_bf2f_hi(g.x[i >> 1]) : dm_bf2f_lo(g.x[i >> 1]);
   if (!normed) return;
   float a = 0.f;
 #pragma unroll
   for (int i = 0; i < PER; ++i) a = dm_fma(x[i], x[i], a);
   const float inv = dm_rsqrt(dm_wave_sum<64>(a) / (float)HD + eps);
 #pragma unroll
-  for (int i = 0; i < PER; ++i) x[i] = dm_rb(dm_bf2f(g.w[i]) * dm_rb(x[i] * inv));
+  for (int i = 0; i < PER; ++i) x[i] = dm_rb((i & 1 ? dm_bf2f_hi(g.w[i >> 1]) : dm_bf2f_lo(g.w[i >> 1])) * dm_rb(x[i] * inv));
   // rotate pairs (e, e + half), e < half; the partner channel lives hl lanes away
   const int hl = half / PER;
   const bool lowg = lane < hl, rot = lane < 2 * hl;
@@ -654,6 +650,333 @@ __global__ __launch_bounds__(512, 4) void sdpa_partial_many_kernel(SdpaArgs p) {
   }
 }
 
+// The same again for eight query heads of a KV group a workgroup and one workgroup a compute unit: half as many workgroups as the
+// four-head form has, for calls where those are more than the compute units and share them.
+//
+// What bounds a block here is issue. A load instruction takes the compute unit's address path 16 clocks whatever its width:
+// the block as 16 bytes a lane straight into LDS (keys) and 8 a lane into registers (values, four channels) is 384 of them,
+// 2.7 us. (The keys' requests are in the buffer form: behind one in the global form the compiler waits for every load in
+// flight where it means to wait for one.) The arithmetic is that of the four-head form, two quads of heads as independent
+// chains: 4096 instructions of eight clocks on four matrix cores, 4 us. The bf16 operands are unpacked 16 steps ahead,
+// between the products (right ahead of its own, each waits out the hazard between the two).
+//
+// Scores: lane = key; wavefronts 0 - 3 run the lower half of the 64-channel chains, 4 - 7 the upper half; a key's eight
+// pieces of a panel lie permuted in LDS (piece i at i ^ (key & 7)), so that eight keys' reads are on different banks.
+// Values: wavefront w of the first four has the 64-key chain w of all channels; the four chains of a channel
+// meet in LDS. Every sum of every head keeps its order. (A KV group that is no multiple of eight heads repeats its last one; what
+// that makes is not stored.)
+//
+// PREP: attn_prep's work too: wavefront w makes query head w and the key row of the call's w-th new position in the block, new value
+// rows are read from the raw projection, and the workgroup of a KV group's first heads appends its row. Static offset, T <= 8.
+// grid sdpa_die_grid<kEightHeads>, 512 threads
+constexpr int kEightHeads = 8;
+template <int HD>
+constexpr int sdpa_eight_bytes() { return (HD / 64) * ATT_KB * 128; }
+template <int HD, bool PREP>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void sdpa_partial_eight_kernel(SdpaArgs p, PrepArgs pq) {
+  constexpr int NH = kEightHeads, NQ = NH / 4, HPW = NH / 2;  // heads of the workgroup; of a half in the softmax
+  int b, hk, hq0, nh, t;
+  if (!sdpa_place<NH>(p, b, hk, hq0, nh, t)) return;
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int offset = PREP ? p.offset : (p.d_offset ? *p.d_offset : p.offset);
+  const int last = min(offset + t, p.cap - 1);
+  if (b * ATT_KB > last) return;
+  constexpr int NKC = HD / 64, NVB = ATT_KB / 64, STEPS = NKC / 2, PER = HD / 64, PANEL = ATT_KB * 128;
+  static_assert(ATT_KB == 256, "four wavefronts of keys");
+  static_assert(NKC == 2 || NKC == 4, "head widths of 128 and 256");
+  typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+  // the key panels; after them the halves' score sums and the value chains
+  extern __shared__ __align__(16) unsigned char stage[];
+  __shared__ float pr[NH][ATT_KB];                       // probabilities; before them the queries
+  __shared__ float red[NH][4], redm[NH][4];              // the key groups' sums and maxima
+  float* const part = reinterpret_cast<float*>(stage);   // [NH][NVB * HD]
+  static_assert(sdpa_eight_bytes<HD>() >= NH * NVB * HD * 4, "the value chains fit where the keys were");
+  float* const qsh = &pr[0][0];                          // PREP: [NH][HD]
+  static_assert(HD <= ATT_KB, "the queries fit where the probabilities will be");
+
+  const int half = wave >> 2, row = (wave & 3) * 64 + lane;  // of the scores: chains of this half, this key
+  const int j0 = HPW * half;                                 // of the softmax: heads j0 ..
+  const bool valid = b * ATT_KB + row <= last;
+  const int nvalid = min(ATT_KB, last - b * ATT_KB + 1);
+  // rows that the cache has; the others are this call's
+  const int nold = PREP ? min(nvalid, max(0, offset - b * ATT_KB)) : nvalid;
+  const size_t blk0 = ((size_t)hk * p.cap + (size_t)b * ATT_KB) * HD;
+  const __amdgpu_buffer_rsrc_t vbuf = dm_buffer(p.v_cache + blk0, nold * HD * 2);
+
+  // PREP: the few loads of this wavefront's rows go out ahead of the block's
+  PrepRegs<PER> pgq, pgk;
+  const int kpos = max(offset, b * ATT_KB) + wave;  // the call's position this wavefront makes the key row of
+  const bool has_k = PREP && kpos < b * ATT_KB + nvalid;
+  if constexpr (PREP) {
+    prep_issue<PER, true>(pq.qg + ((size_t)t * p.Hq + hq0 + min(wave, nh - 1)) * 2 * HD, pq.qw, pq.cos_t, pq.sin_t, offset + t, pq.half, lane, pgq);
+    const int kp = min(kpos, offset + p.T - 1);
+    prep_issue<PER, true>(pq.kx + ((size_t)(kp - offset) * p.Hkv + hk) * HD, pq.kw, pq.cos_t, pq.sin_t, kp, pq.half, lane, pgk);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  // this half's query channels: 16 g + a of head i of a quad in lane 4 a + i
+  constexpr int QG = HD / 32;
+  float q[NQ][QG];
+  bf16_t qraw[NQ][QG];
+  if constexpr (!PREP) {
+#pragma unroll
+    for (int n = 0; n < NQ; ++n) {
+      const bf16_t* qrow = p.q_rot + ((size_t)t * p.Hq + hq0 + min(4 * n + (lane & 3), nh - 1)) * HD + half * (HD / 2) + (lane >> 2);
+#pragma unroll
+      for (int g = 0; g < QG; ++g) qraw[n][g] = qrow[16 * g];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  // keys: 8 rows of a panel, 1 KB, a load; rows that the cache does not have repeat another (they are masked, or written
+  // below). (No load stands under a condition that others could be counted past.)
+  {
+    const __amdgpu_buffer_rsrc_t kbuf = dm_buffer(p.k_cache + blk0, max(nold, 1) * HD * 2);
+#pragma unroll
+    for (int i = 0; i < NKC * 4; ++i) {
+      const int c = wave + 8 * (i & 3), panel = i >> 2, r = min(8 * c + (lane >> 3), max(nold, 1) - 1);
+      typedef __attribute__((address_space(3))) void lds_t;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(kbuf, (lds_t*)(stage + panel * PANEL + c * 1024), 16,
+                                               r * (HD * 2) + panel * 128 + 16 * ((lane & 7) ^ (lane >> 3)), 0, 0, 0);
+    }
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  // values: PER channels a lane, the first half of the chain's keys right behind the block's keys
+  typedef uint32_t vrow_t __attribute__((ext_vector_type(PER / 2)));
+  const bool holds = wave < NVB;
+  vrow_t vreg[4][16];
+  auto load_row = [&](const __amdgpu_buffer_rsrc_t& buf, int at) {
+    vrow_t v;
+    if constexpr (PER == 4) {
+      v = __builtin_bit_cast(vrow_t, __builtin_amdgcn_raw_buffer_load_b64(buf, at + 8 * lane, 0, 0));
+    } else {
+      v[0] = __builtin_amdgcn_raw_buffer_load_b32(buf, at + 4 * lane, 0, 0);
+    }
+    return v;
+  };
+  auto fetch_values = [&](auto set) {
+    constexpr int S = decltype(set)::value;
+#pragma unroll
+    for (int u = 0; u < 16; ++u) vreg[S][u] = load_row(vbuf, (64 * wave + 16 * S + u) * (HD * 2));
+  };
+  using S0 = std::integral_constant<int, 0>;
+  using S1 = std::integral_constant<int, 1>;
+  using S2 = std::integral_constant<int, 2>;
+  using S3 = std::integral_constant<int, 3>;
+  uint32_t krow[PER / 2];
+  auto heads = [&](auto path) {  // (the paths' tags keep the compiler from doing it ahead of the requests, where the paths agree)
+    if constexpr (PREP) {
+      float x[PER];
+#pragma unroll
+      for (int i = 0; i < PER / 2; ++i) asm volatile("; rows on path %4" : "+v"(pgq.x[i]), "+v"(pgk.x[i]), "+v"(pgq.w[i]), "+v"(pgk.w[i]) : "n"(decltype(path)::value));
+      prep_finish<PER>(pgq, true, pq.half, pq.eps, lane, x);
+#pragma unroll
+      for (int i = 0; i < PER; ++i) qsh[wave * HD + lane * PER + i] = p.scale * dm_bf2f(dm_f2bf(x[i]));  // q_rot is bf16
+      if (has_k) {
+        prep_finish<PER>(pgk, true, pq.half, pq.eps, lane, x);
+#pragma unroll
+        for (int e = 0; e < PER; e += 2) krow[e / 2] = dm_f2bf2(x[e], x[e + 1]);
+      }
+    } else {
+#pragma unroll
+      for (int n = 0; n < NQ; ++n)
+#pragma unroll
+        for (int g = 0; g < QG; ++g) q[n][g] = p.scale * dm_bf2f(qraw[n][g]);
+    }
+  };
+  if (holds) {
+    fetch_values(S0{});
+    fetch_values(S1{});
+    __builtin_amdgcn_sched_barrier(0);
+    heads(S1{});
+  } else {
+    heads(S0{});
+  }
+  // this wavefront's part of the keys is here (the values behind it are not)
+  asm volatile("" ::: "memory");
+  if (holds) __builtin_amdgcn_s_waitcnt(0x0070 | (32 >> 4) << 14);  // at most 32 loads left, every LDS access done
+  else __builtin_amdgcn_s_waitcnt(0x0070);
+  __builtin_amdgcn_s_barrier();  // (__syncthreads would wait for the values too)
+  asm volatile("" ::: "memory");
+  if constexpr (PREP) {
+    if (nold < nvalid) {  // (of the whole workgroup)
+      if (has_k) {
+        const int r = kpos - b * ATT_KB, ch = lane * PER, at = ch % 64 * 2;
+#pragma unroll
+        for (int e = 0; e < PER / 2; ++e)
+          *reinterpret_cast<uint32_t*>(stage + ch / 64 * PANEL + r * 128 + ((at & ~15) ^ ((r & 7) << 4)) + (at & 15) + 4 * e) = krow[e];
+      }
+      __syncthreads();
+    }
+#pragma unroll
+    for (int n = 0; n < NQ; ++n)
+#pragma unroll
+      for (int g = 0; g < QG; ++g) q[n][g] = qsh[(4 * n + (lane & 3)) * HD + half * (HD / 2) + 16 * g + (lane >> 2)];
+  }
+  if (holds) {
+    fetch_values(S2{});
+    fetch_values(S3{});
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  f32x4 sum[NQ];
+#pragma unroll
+  for (int s = 0; s < STEPS; ++s) {
+    f32x4 chain[NQ];
+#pragma unroll
+    for (int n = 0; n < NQ; ++n) chain[n] = f32x4{0.f, 0.f, 0.f, 0.f};
+    uint4 kw[8];
+    const unsigned char* const kr = stage + (half * STEPS + s) * PANEL + row * 128;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) kw[i] = *reinterpret_cast<const uint4*>(kr + 16 * (i ^ (lane & 7)));
+    auto channel = [&](int i) {
+      const uint4& w = kw[i >> 3];
+      const uint32_t u[4] = {w.x, w.y, w.z, w.w};
+      return i & 1 ? dm_bf2f_hi(u[(i >> 1) & 3]) : dm_bf2f_lo(u[(i >> 1) & 3]);
+    };
+    float k[2][16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) k[0][i] = channel(i);
+    __builtin_amdgcn_sched_barrier(0);
+    auto sixteen = [&](auto gc) {
+      constexpr int G = decltype(gc)::value;
+#define ORN_STEP(A)                                                                                                  \
+  _Pragma("unroll") for (int n = 0; n < NQ; ++n)                                                                     \
+      chain[n] = __builtin_amdgcn_mfma_f32_4x4x1f32(q[n][4 * s + G], k[G & 1][A], chain[n], 4, A, 0);                \
+  if constexpr (G < 3) k[(G & 1) ^ 1][A] = channel((16 * G + 16 + A) & 63);
+      ORN_STEP(0) ORN_STEP(1) ORN_STEP(2) ORN_STEP(3) ORN_STEP(4) ORN_STEP(5) ORN_STEP(6) ORN_STEP(7)
+      ORN_STEP(8) ORN_STEP(9) ORN_STEP(10) ORN_STEP(11) ORN_STEP(12) ORN_STEP(13) ORN_STEP(14) ORN_STEP(15)
+#undef ORN_STEP
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, NQ, 0);
+        if constexpr (G < 3) __builtin_amdgcn_sched_group_barrier(0x002, 1, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    sixteen(S0{});
+    sixteen(S1{});
+    sixteen(S2{});
+    sixteen(S3{});
+#pragma unroll
+    for (int n = 0; n < NQ; ++n) sum[n] = s == 0 ? chain[n] : sum[n] + chain[n];
+  }
+  // PREP: the values of the call's own positions up to this row's come from the projection, and this row goes to the cache
+  if constexpr (PREP) {
+    if (holds && nold < nvalid) {
+      const __amdgpu_buffer_rsrc_t xbuf = dm_buffer(pq.vx + (size_t)hk * HD, (uint32_t)(t * p.Hkv + 1) * (HD * 2));
+      const int x0 = max(offset, b * ATT_KB) - offset - nold;
+#pragma unroll
+      for (int u = 0; u < 64; ++u) {
+        const int r = 64 * wave + u;
+        if (r >= nold && r < nvalid) vreg[u >> 4][u & 15] = load_row(xbuf, (x0 + r) * (p.Hkv * HD * 2));
+      }
+    }
+    if (hq0 == hk * (p.Hq / p.Hkv) && has_k && kpos == last) {
+#pragma unroll
+      for (int e = 0; e < PER / 2; ++e) {
+        const size_t at = ((size_t)hk * p.cap + last) * HD + lane * PER + 2 * e;
+        *reinterpret_cast<uint32_t*>(pq.k_cache + at) = krow[e];
+        *reinterpret_cast<uint32_t*>(pq.v_cache + at) =
+            *reinterpret_cast<const uint32_t*>(pq.vx + ((size_t)t * p.Hkv + hk) * HD + lane * PER + 2 * e);
+      }
+    }
+  }
+  __syncthreads();  // the keys have been read
+  // (c0 + c1) + (c2 + c3): each half hands the other the heads it does not go on with
+  auto head_sum = [&](int j) { return sum[j >> 2][j & 3]; };
+  float* const other = part + row;
+#pragma unroll
+  for (int j = 0; j < HPW; ++j) other[((half ^ 1) * HPW + j) * ATT_KB] = half ? head_sum(j) : head_sum(HPW + j);
+  __syncthreads();
+  float sc[HPW], mg[HPW];
+#pragma unroll
+  for (int j = 0; j < HPW; ++j) {
+    const float mine = half ? head_sum(HPW + j) : head_sum(j), theirs = other[(j0 + j) * ATT_KB];
+    sc[j] = mine + theirs;
+    const float m = dm_wave_max<64>(valid ? sc[j] : -DM_INF);  // block max
+    if (lane == 0) redm[j0 + j][wave & 3] = m;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < HPW; ++j) {
+    const float* r = redm[j0 + j];
+    float m = r[0];
+    m = r[1] > m ? r[1] : m;
+    m = r[2] > m ? r[2] : m;
+    m = r[3] > m ? r[3] : m;
+    mg[j] = m;
+    const float pv = valid ? dm_exp(sc[j] - m) : 0.f;
+    pr[j0 + j][row] = pv;
+    const float ws = dm_wave_sum<64>(pv);
+    if (lane == 0) red[j0 + j][wave & 3] = ws;
+    if (row == 0 && j0 + j < nh) p.part_m[((size_t)t * p.Hq + hq0 + j0 + j) * p.nblk + b] = m;
+  }
+  __syncthreads();
+  // values: chain `wave` = keys 64 * wave .. + 64, PER channels of the heads
+  if (holds) {
+    f32x4 o[PER][NQ];
+#pragma unroll
+    for (int c = 0; c < PER; ++c)
+#pragma unroll
+      for (int n = 0; n < NQ; ++n) o[c][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float w[NQ][4];  // key a of head i of sixteen in lane 4 a + i
+#pragma unroll
+    for (int n = 0; n < NQ; ++n)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) w[n][g] = pr[4 * n + (lane & 3)][64 * wave + 16 * g + (lane >> 2)];
+    constexpr int AHEAD = 4;  // keys unpacked ahead
+    float v[2][AHEAD][PER];
+    auto unpack = [&](int e, int i) {  // key i of the e-th four
+      const vrow_t u = vreg[e >> 2][4 * (e & 3) + i];
+#pragma unroll
+      for (int c = 0; c < PER; ++c) v[e & 1][i][c] = c & 1 ? dm_bf2f_hi(u[c >> 1]) : dm_bf2f_lo(u[c >> 1]);
+    };
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i) unpack(0, i);
+    __builtin_amdgcn_sched_barrier(0);
+    auto four = [&](auto ec) {
+      constexpr int E = decltype(ec)::value;
+#define ORN_KEY(A)                                                                                                         \
+  _Pragma("unroll") for (int c = 0; c < PER; ++c) _Pragma("unroll") for (int n = 0; n < NQ; ++n)                            \
+      o[c][n] = __builtin_amdgcn_mfma_f32_4x4x1f32(w[n][E >> 2], v[E & 1][A][c], o[c][n], 4, 4 * (E & 3) + A, 0);           \
+  if constexpr (E < 15) unpack((E + 1) & 15, A);
+      ORN_KEY(0) ORN_KEY(1) ORN_KEY(2) ORN_KEY(3)
+#undef ORN_KEY
+#pragma unroll
+      for (int i = 0; i < 4 * PER; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, NQ, 0);
+        if constexpr (E < 15) __builtin_amdgcn_sched_group_barrier(0x002, 1, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    };
+#define ORN_FOURS(E) four(std::integral_constant<int, E>{}); four(std::integral_constant<int, E + 1>{}); \
+                     four(std::integral_constant<int, E + 2>{}); four(std::integral_constant<int, E + 3>{});
+    ORN_FOURS(0) ORN_FOURS(4) ORN_FOURS(8) ORN_FOURS(12)
+#undef ORN_FOURS
+#pragma unroll
+    for (int n = 0; n < NQ; ++n)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        float* const to = &part[(4 * n + j) * (NVB * HD) + wave * HD + PER * lane];
+        if constexpr (PER == 4)
+          *reinterpret_cast<float4*>(to) = make_float4(o[0][n][j], o[1][n][j], o[PER - 2][n][j], o[PER - 1][n][j]);
+        else
+          *reinterpret_cast<float2*>(to) = make_float2(o[0][n][j], o[1][n][j]);
+      }
+  }
+  __syncthreads();
+  for (int i = tid; i < nh * HD; i += 512) {
+    const int j = i / HD, d = i - j * HD;
+    p.part_o[(((size_t)t * p.Hq + hq0 + j) * p.nblk + b) * HD + d] = sdpa_pair_tree<NVB>(part + j * (NVB * HD) + d, HD);
+  }
+  if (tid < nh) {
+    float l = red[tid][0] + red[tid][1];
+    l = l + red[tid][2];
+    l = l + red[tid][3];
+    p.part_l[((size_t)t * p.Hq + hq0 + tid) * p.nblk + b] = l;
+  }
+}
+
 // Merge: blocks ascending, divide, gate. Grid (Hq, T), one wavefront a row, HD / 64 channels a lane.
 // A few trips to memory and little else: lane b fetches block b's maximum and sum, every lane asks for its
 // channels' partial outputs of up to kMergeAhead blocks in the same trip, and the block weights exp(m_b - M) are made once (lane b)
@@ -815,7 +1138,7 @@ int ornith_attn_prep(ornith_ctx* ctx, const void* d_qg, const void* d_kx, const 
 }
 
 // prep != null: the prep of the same rows has not been launched yet; it is done inside the
-// attention launch where that launch's form can (the 1024-thread form, T <= 8, static offset), by
+// attention launch where that launch's form can (the 1024-thread and eight-head forms, T <= 8, static offset), by
 // its own launch first otherwise
 static int sdpa_decode(ornith_ctx* ctx, const void* d_q_rot, const void* d_k_cache, const void* d_v_cache,
                        const void* d_qg, int T, int Hq, int Hkv, int hd, int offset, const int* d_offset, int cap,
@@ -862,7 +1185,8 @@ static int sdpa_decode(ornith_ctx* ctx, const void* d_q_rot, const void* d_k_cac
   // Which form. One 1024-thread workgroup a (key block, head, row) has the shorter chain, but 150 KB of LDS
   // let a compute unit hold one of them: a round takes as long as the whole call of the many form (four
   // heads of a KV group a workgroup, two workgroups a compute unit), so it is the faster one for as long as
-  // it is one round. Whole calls, us, 1024-thread form / many form, two KV groups of eight heads of 256:
+  // it is one round. Whole calls, us, 1024-thread form / many form, two KV groups of eight heads of 256 (with an
+  // earlier merge launch, which took 1 to 1.5 more of both):
   // 256 workgroups of the first (one row at 4000 keys, four at 1000) 13.4 / 16.7, 288 (three rows at 1500)
   // 20.1 / 16.8, 384 20.3 / 16.9, 768 27.4 / 17.0, 1536 47.8 / 22.2; head width 128, 256: 11.3 / 13.0, 384: 16.8 / 13.3.
   // KV groups that are no multiple of four heads, whose last workgroup repeats heads, turn at the same
@@ -885,7 +1209,15 @@ static int sdpa_decode(ornith_ctx* ctx, const void* d_q_rot, const void* d_k_cac
   const dim3 grid = p.by_die ? dim3(sdpa_die_grid<1>(p)) : dim3(nblk, Hq, T);
   // one key block for every row, in the kernel form that knows how to finish: no merge launch
   p.finish = (last_max < ATT_KB && !many) ? 1 : 0;
-  const bool fold = prep && !many && !d_offset && T <= 8 && ornith_option_fuse_attn_prep();
+  // Eight heads a workgroup where four make more workgroups than there are compute units and eight don't: a block's way
+  // through a workgroup is longer (whole calls, us, two KV groups of eight heads of 256, four heads / eight: two rows at 6000 / 8100
+  // keys, 192 / 256 workgroups of four, 16.3 / 18.3 and 16.7 / 18.7), but two workgroups that share a unit are longer still (two rows
+  // at 9000 / 16000 keys, 288 / 504 workgroups of four, 22.2 / 19.3 and 23.9 / 21.0; four at 4200 / 6621 / 8100 20.9 / 18.3, 22.1 / 18.9 and
+  // 22.6 / 19.0; eight at 2100 20.6 / 18.0). A second round of eights costs what it saved (four rows at 9000 / 12000 keys
+  // 29.0 / 32.3 and 29.9 / 32.8, at 16000 35.0 / 33.4).
+  const long pairs = (long)(last_max / ATT_KB + 1) * Hkv * T, group = Hq / Hkv;
+  const bool eight = many && pairs * ((group + 3) / 4) > ctx->compute_units && pairs * ((group + 7) / 8) <= ctx->compute_units;
+  const bool fold = prep && (!many || eight) && !d_offset && T <= 8 && ornith_option_fuse_attn_prep();
   PrepArgs pq{};
   if (prep) {
     pq = *prep;
@@ -894,7 +1226,19 @@ static int sdpa_decode(ornith_ctx* ctx, const void* d_q_rot, const void* d_k_cac
       if (rcp) return rcp;
     }
   }
-  if (many) {
+  if (eight) {
+    typedef void (*Kernel)(SdpaArgs, PrepArgs);
+    static const Kernel kernels[2][2] = {{sdpa_partial_eight_kernel<128, false>, sdpa_partial_eight_kernel<128, true>},
+                                         {sdpa_partial_eight_kernel<256, false>, sdpa_partial_eight_kernel<256, true>}};
+    const int bytes[2] = {sdpa_eight_bytes<128>(), sdpa_eight_bytes<256>()};
+    if (!(ctx->lds_attr_set & 16)) {
+      for (int w = 0; w < 2; ++w)
+        for (const Kernel k : kernels[w])
+          ORN_HIP(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, bytes[w]));
+      ctx->lds_attr_set |= 16;
+    }
+    hipLaunchKernelGGL(kernels[hd == 256][fold], dim3(sdpa_die_grid<kEightHeads>(p)), dim3(512), bytes[hd == 256], ctx->stream, p, pq);
+  } else if (many) {
     if (hd == 256)
       hipLaunchKernelGGL(sdpa_partial_many_kernel<256>, dim3(sdpa_die_grid<kManyHeads>(p)), dim3(512), 0, ctx->stream, p);
     else

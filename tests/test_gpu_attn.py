@@ -34,6 +34,10 @@ def _mk(rng, T, Hq, Hkv, hd, cap, offset):
     # end, as many workgroups a die as it has compute units, and one row more (block fastest, or the other form)
     (1, 16, 2, 256, 4096, 513), (1, 16, 2, 256, 4096, 2300), (2, 16, 2, 256, 4096, 1790), (1, 6, 2, 128, 4096, 3300),
     (3, 5, 1, 256, 2048, 766), (4, 16, 2, 256, 4096, 800), (5, 16, 2, 256, 4096, 700), (1, 16, 16, 256, 2048, 600),
+    # eight heads a workgroup: new rows across a block's end, a last block of new rows alone, ragged KV groups (six, five, twelve
+    # heads), head width 128, more rows than the prep is done for
+    (8, 16, 2, 256, 4096, 2556), (4, 16, 2, 256, 8192, 5120), (8, 12, 2, 256, 4096, 2300), (7, 5, 1, 256, 8192, 6000),
+    (4, 24, 2, 128, 4096, 3500), (4, 16, 2, 128, 8192, 5000), (9, 16, 2, 256, 4096, 1900),
     # ... from one workgroup of the other form more than there are compute units: the last call before that, and the first
     (4, 16, 2, 256, 4096, 1020), (4, 16, 1, 128, 4096, 1021),
     # 16-row prompt chunks inside the first key block (one finishing launch, of two rounds from 17 rows on) and across
@@ -76,10 +80,10 @@ def test_attention_bit_exact(orn, ctx, T, Hq, Hkv, hd, cap, offset):
     for b in d + [dkc, dvc, dq, dout, dc, ds]: b.free()
 
 
-# the matrix-core form (four heads a workgroup; groups of eight and of three heads, head widths 256 and 128) and the
+# the matrix-core forms (four heads a workgroup, and eight; groups of eight and of three heads, head widths 256 and 128) and the
 # 1024-thread one, inside the first key block and past it
 @pytest.mark.parametrize("T,Hq,Hkv,hd,cap,offset", [(4, 16, 2, 256, 4096, 2500), (4, 16, 2, 128, 4096, 3000), (8, 6, 2, 256, 8192, 8000),
-                                                    (2, 16, 2, 256, 4096, 51), (2, 16, 2, 256, 4096, 600)])
+                                                    (2, 16, 2, 256, 4096, 51), (2, 16, 2, 256, 4096, 600), (8, 16, 2, 256, 4096, 2300)])
 def test_attention_special_values(orn, ctx, T, Hq, Hkv, hd, cap, offset):
     """Subnormal keys and values, score products below the normal range, infinities and NaNs in keys and values:
     the oracle's values, NaN for NaN."""
