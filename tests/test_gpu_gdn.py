@@ -28,6 +28,25 @@ def test_norms_bit_exact(orn, ctx):
         for d in (dx, db, dw, dz, dh, do): d.free()
 
 
+@pytest.mark.parametrize("rows", [1, 15, 16, 17, 200])
+def test_gated_norm_of_value_heads_bit_exact(orn, ctx, rows):
+    """128-wide rows, sixteen of them a workgroup: whole, ragged and single; huge and tiny rows (the sum of squares overflows, or is
+    below eps), zeros, infinities and NaN in the row and in the gate"""
+    rng = np.random.default_rng(rows)
+    x, w, z = util.bf16_normal(rng, (rows, 128), 3.0), util.bf16_normal(rng, (128,)), util.bf16_normal(rng, (rows, 128), 8.0)
+    x[0, :] = util.f32_to_bf16(np.float32(1e-20) * util.bf16_to_f32(x[0]))
+    x[rows // 2, 5] = 0x7F00; x[rows - 1, 7:9] = 0; z[rows - 1, 100] = 0x7F80; z[0, 127] = 0xFF80
+    if rows > 2: x[1, 64] = 0x7F80; z[1, 3] = 0x7FC0
+    dx, dw, dz, do = ctx.to_device(x), ctx.to_device(w), ctx.to_device(z), ctx.alloc(x.nbytes + 256)
+    ctx.memset(do, 0x5A, x.nbytes + 256)
+    ctx.rms_norm_gated(dx, dw, dz, rows, 128, 1e-6, do)
+    got, want = do.download(np.uint16, (rows + 1, 128)), util.orc_rms_norm_gated(x, w, z)
+    nan = np.isnan(util.bf16_to_f32(want))
+    assert np.array_equal(np.isnan(util.bf16_to_f32(got[:rows])), nan) and np.array_equal(got[:rows][~nan], want[~nan])
+    assert np.all(got[rows] == 0x5A5A)
+    for d in (dx, dw, dz, do): d.free()
+
+
 def _front(orn, ctx, i, T, Hk, Hv):
     D = 2 * Hk * 128 + Hv * 128
     names = ("conv_state", "qkv", "cw", "a", "b", "a_log", "dt_bias")
