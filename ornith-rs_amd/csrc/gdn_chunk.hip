@@ -90,110 +90,112 @@ extern "C" __attribute__((visibility("default"))) int ornith_debug_marks_prep(lo
 // pieces of the same token rows and write neighbouring operand blocks). Operand layout of v_mfma_f32_16x16x32_bf16: lane (l16, lg)
 // holds A[m = l16][k = 8 lg ..+8], B^T[n = l16][k = 8 lg ..+8] of a 32-wide k slab and
 // D[m = 4 lg + r][n = l16], r < 4.
+// A chain of phases with two workgroups a compute unit to overlap them: requests and transposes 1.6 to 3.3 us, K K^T and the diagonal
+// inverses 2.8, T 0.9, the two products with T 2.8. us a launch (32 heads), before (operands read in operand order, T a row at a time) /
+// now: 10 chunks 22.5 / 16, 11 23.1 / 16.4, 64 85.9 / 64.
 __global__ __launch_bounds__(256) void gdn_chunk_prep_kernel(ChunkArgs p) {
-  // A is kept as four planes, plane j % 4 holding A[i][j] at [i][j / 4] (rows of 16 + 4 pad, the
-  // planes 4 words apart in bank): the solve below reads a plane row by row, 16 bytes a read
-  constexpr int AROW = 20, APLANE = C * AROW + 4;
-  __shared__ float lg_s[C], ell_s[C], bet_s[C];
-  __shared__ __attribute__((aligned(16))) bf16_t Kt[DK][LDT];
-  __shared__ __attribute__((aligned(16))) bf16_t Vt[DK][LDT];  // Dv <= 128 rows used
-  __shared__ __attribute__((aligned(16))) float Ap[4 * APLANE];  // A, later T in two bf16 parts
-  bf16_t(*Th)[LDT] = reinterpret_cast<bf16_t(*)[LDT]>(&Ap[0]);
+  constexpr int LDK = DK + 8, LDA = C + 4, LDD = 20;
+  __shared__ float ell_s[C], bet_s[C];
+  // K^T and V^T: rows of 64 tokens whose 16-byte pieces lie permuted (row 8 a + e: piece i at i ^ ((a ^ e) & 7)), so that both
+  // the writes (one e, 16 a) and the operand reads (one a, 8 e) spread over the banks
+  __shared__ __attribute__((aligned(16))) bf16_t Kt[DK * C];
+  __shared__ __attribute__((aligned(16))) bf16_t Vt[DK * C];          // Dv <= 128 rows used
+  __shared__ __attribute__((aligned(16))) bf16_t Kr[2 * C * LDT];     // K by token, later T in two bf16 parts
+  __shared__ __attribute__((aligned(16))) float A[C * LDA];
+  __shared__ __attribute__((aligned(16))) float Dg[4][16 * LDD];      // the inverted diagonal blocks of I + A
+  bf16_t(*Th)[LDT] = reinterpret_cast<bf16_t(*)[LDT]>(&Kr[0]);
   bf16_t(*Tl)[LDT] = Th + C;
-  static_assert(sizeof(float) * 4 * APLANE >= sizeof(bf16_t) * 2 * C * LDT, "T fits where A was");
+  static_assert(2 * C * LDT >= C * LDK, "K by token fits where T will be");
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l16 = lane & 15, lg = lane >> 4;
   const int chunk = blockIdx.y, hv = blockIdx.x, hk = hv / (p.Hv / p.Hk);
   const int t0 = chunk * C, Dv = p.Dv;
   const size_t ch = (size_t)chunk * p.Hv + hv;
+  auto turned = [&](const bf16_t* m, int row, int piece) { return m + row * C + 8 * (piece ^ (((row >> 3) ^ row) & 7)); };
 
   PR_MARK(0);
-  // decay logs and beta of the chunk's tokens; tokens past the end leave the state alone
-  if (tid < C) {
-    const int t = t0 + tid;
-    const bool live = t < p.T;
-    const float gv = live ? p.g[(size_t)t * p.Hv + hv] : 1.f;
-    lg_s[tid] = live ? fmaxf(__logf(gv), -100.f) : 0.f;
-    bet_s[tid] = live ? dm_bf2f(p.beta[(size_t)t * p.Hv + hv]) : 0.f;
+  // Requests first, in whole rows (sixteen lanes a 256-byte row: in operand order sixteen lanes ask for sixteen lines, 64 clocks of
+  // the L1 a load): thread = (token pair, 8-wide piece) of K and V. This wavefront's tokens of Q are an operand as they are.
+  const int pc = tid & 15;
+  float gv = 1.f, bv = 0.f;  // decay and beta of the chunk's tokens; tokens past the end leave the state alone
+  if (wave == 0 && t0 + lane < p.T) {
+    gv = p.g[(size_t)(t0 + lane) * p.Hv + hv];
+    bv = dm_bf2f(p.beta[(size_t)(t0 + lane) * p.Hv + hv]);
   }
-  // Operand fragments of the K K^T / Q K^T products below, asked for now (they depend on
-  // nothing made here): tokens i = 16 wave + l16 as the n side, tokens j of the tiles nt < wave as
-  // the m side (tile nt = wave has the same rows as the n side).
-  bf16x8_t bki[4], bqi[4], akj[3][4];
+  uint4 kr[2][2], vr[2][2];
+#pragma unroll
+  for (int it = 0; it < 2; ++it) {
+    const int tp = (tid >> 4) + 16 * it;
+    const int ta = min(t0 + 2 * tp, p.T - 1), tb = min(t0 + 2 * tp + 1, p.T - 1);
+    kr[it][0] = *reinterpret_cast<const uint4*>(p.k + ((size_t)ta * p.Hk + hk) * DK + 8 * pc);
+    kr[it][1] = *reinterpret_cast<const uint4*>(p.k + ((size_t)tb * p.Hk + hk) * DK + 8 * pc);
+  }
+  bf16x8_t bqi[4];
   {
     const int ti = min(t0 + 16 * wave + l16, p.T - 1);
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      bki[ks] = ld8(p.k + ((size_t)ti * p.Hk + hk) * DK + 32 * ks + 8 * lg);
-      bqi[ks] = ld8(p.q + ((size_t)ti * p.Hk + hk) * DK + 32 * ks + 8 * lg);
-    }
+    for (int ks = 0; ks < 4; ++ks) bqi[ks] = ld8(p.q + ((size_t)ti * p.Hk + hk) * DK + 32 * ks + 8 * lg);
+  }
+  if (8 * pc < Dv) {
 #pragma unroll
-    for (int nt = 0; nt < 3; ++nt) {
-      if (nt < wave) {
-        const int tj = min(t0 + 16 * nt + l16, p.T - 1);
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks) akj[nt][ks] = ld8(p.k + ((size_t)tj * p.Hk + hk) * DK + 32 * ks + 8 * lg);
-      }
+    for (int it = 0; it < 2; ++it) {
+      const int tp = (tid >> 4) + 16 * it;
+      const int ta = min(t0 + 2 * tp, p.T - 1), tb = min(t0 + 2 * tp + 1, p.T - 1);
+      vr[it][0] = *reinterpret_cast<const uint4*>(p.v + ((size_t)ta * p.Hv + hv) * Dv + 8 * pc);
+      vr[it][1] = *reinterpret_cast<const uint4*>(p.v + ((size_t)tb * p.Hv + hv) * Dv + 8 * pc);
     }
   }
-  // K and V of the chunk, transposed into LDS: thread = (token pair, 8-wide piece); the two
-  // tokens' values of a channel are one 4-byte write, and a wavefront's 64 writes of a channel
-  // (32 pairs of two pieces) fall on 64 different banks. All loads first, then the writes.
-  {
-    uint4 kr[2][2], vr[2][2];
+  if (wave == 0) {
+    // l: running sum of the decays' logs, one after the other (a scan's two roundings a token would be in every difference of two)
+    const float own = t0 + lane < p.T ? fmaxf(__logf(gv), -100.f) : 0.f;
+    float sum = 0.f, l = 0.f;
 #pragma unroll
-    for (int it = 0; it < 2; ++it) {
-      const int idx = tid + 256 * it, tp = idx & 31, pc = idx >> 5;
-      const int ta = min(t0 + 2 * tp, p.T - 1), tb = min(t0 + 2 * tp + 1, p.T - 1);
-      kr[it][0] = *reinterpret_cast<const uint4*>(p.k + ((size_t)ta * p.Hk + hk) * DK + 8 * pc);
-      kr[it][1] = *reinterpret_cast<const uint4*>(p.k + ((size_t)tb * p.Hk + hk) * DK + 8 * pc);
-      if (8 * pc < Dv) {
-        vr[it][0] = *reinterpret_cast<const uint4*>(p.v + ((size_t)ta * p.Hv + hv) * Dv + 8 * pc);
-        vr[it][1] = *reinterpret_cast<const uint4*>(p.v + ((size_t)tb * p.Hv + hv) * Dv + 8 * pc);
-      }
+    for (int j = 0; j < C; ++j) {
+      sum += __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, own), j));
+      l = lane == j ? sum : l;
     }
-    auto put = [&](bf16_t(*dst)[LDT], const uint4& a, const uint4& b, int pc, int tp) {
-      const uint32_t aw[4] = {a.x, a.y, a.z, a.w}, bw[4] = {b.x, b.y, b.z, b.w};
+    ell_s[lane] = l;
+    bet_s[lane] = bv;
+    p.ell[ch * C + lane] = l;
+  }
+  // the two tokens' values of a channel are one 4-byte write
+  auto put = [&](bf16_t* dst, const uint4& a, const uint4& b, int tp) {
+    const uint32_t aw[4] = {a.x, a.y, a.z, a.w}, bw[4] = {b.x, b.y, b.z, b.w};
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const uint32_t w = (e & 1) ? ((aw[e >> 1] >> 16) | (bw[e >> 1] & 0xffff0000u))
-                                   : ((aw[e >> 1] & 0xffffu) | (bw[e >> 1] << 16));
-        *reinterpret_cast<uint32_t*>(&dst[8 * pc + e][2 * tp]) = w;
-      }
-    };
-#pragma unroll
-    for (int it = 0; it < 2; ++it) {
-      const int idx = tid + 256 * it, tp = idx & 31, pc = idx >> 5;
-      put(Kt, kr[it][0], kr[it][1], pc, tp);
-      if (8 * pc < Dv) put(Vt, vr[it][0], vr[it][1], pc, tp);
+    for (int e = 0; e < 8; ++e) {
+      const uint32_t w = (e & 1) ? ((aw[e >> 1] >> 16) | (bw[e >> 1] & 0xffff0000u))
+                                 : ((aw[e >> 1] & 0xffffu) | (bw[e >> 1] << 16));
+      *reinterpret_cast<uint32_t*>(const_cast<bf16_t*>(turned(dst, 8 * pc + e, tp >> 2)) + 2 * (tp & 3)) = w;
     }
+  };
+#pragma unroll
+  for (int it = 0; it < 2; ++it) {
+    const int tp = (tid >> 4) + 16 * it;
+    *reinterpret_cast<uint4*>(&Kr[(2 * tp) * LDK + 8 * pc]) = kr[it][0];
+    *reinterpret_cast<uint4*>(&Kr[(2 * tp + 1) * LDK + 8 * pc]) = kr[it][1];
+    put(Kt, kr[it][0], kr[it][1], tp);
+  }
+  const bool first = hv % (p.Hv / p.Hk) == 0;  // K^T and Q for the second kernel: once per key head
+  if (first) {
+    bf16_t* qdst = p.qf + ((size_t)chunk * p.Hk + hk) * C * DK;
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) *reinterpret_cast<bf16x8_t*>(qdst + ((size_t)(wave * 4 + ks) * 64 + lane) * 8) = bqi[ks];
   }
   __syncthreads();
   PR_MARK(1);
-  if (tid < C) {
-    float s = 0.f;
-    for (int j = 0; j <= tid; ++j) s += lg_s[j];
-    ell_s[tid] = s;
-    p.ell[ch * C + tid] = s;
+  if (8 * pc < Dv) {  // (read two barriers on)
+#pragma unroll
+    for (int it = 0; it < 2; ++it) put(Vt, vr[it][0], vr[it][1], (tid >> 4) + 16 * it);
   }
-  // K^T and Q for the second kernel, once per key head
-  if (hv % (p.Hv / p.Hk) == 0) {
+  if (first) {
     bf16_t* dst = p.kt + ((size_t)chunk * p.Hk + hk) * DK * C;
-    for (int idx = tid; idx < DK * (C / 8); idx += 256) {
-      const int r = idx / (C / 8), pc = idx % (C / 8);  // row dk = r, tokens 8 pc ..
-      *reinterpret_cast<bf16x8_t*>(dst + ((size_t)((r >> 4) * 2 + (pc >> 2)) * 64 + (pc & 3) * 16 + (r & 15)) * 8) =
-          ld8(&Kt[r][8 * pc]);
-    }
-    bf16_t* qdst = p.qf + ((size_t)chunk * p.Hk + hk) * C * DK;
-    for (int idx = tid; idx < C * (DK / 8); idx += 256) {
-      const int tok = idx / (DK / 8), pc = idx % (DK / 8);  // row token, channels 8 pc ..
-      const int t = min(t0 + tok, p.T - 1);
-      *reinterpret_cast<bf16x8_t*>(qdst + ((size_t)((tok >> 4) * 4 + (pc >> 2)) * 64 + (pc & 3) * 16 + (tok & 15)) * 8) =
-          ld8(p.q + ((size_t)t * p.Hk + hk) * DK + 8 * pc);
+#pragma unroll
+    for (int it = 0; it < DK * (C / 8) / 256; ++it) {
+      const int idx = tid + 256 * it, tile = idx >> 6;  // rows 16 (tile / 2) .., tokens 32 (tile % 2) ..: an operand
+      *reinterpret_cast<bf16x8_t*>(dst + (size_t)idx * 8) = ld8(turned(Kt, 16 * (tile >> 1) + l16, 4 * (tile & 1) + lg));
     }
   }
-  __syncthreads();
   PR_MARK(2);
 
   // ---- K K^T and Q K^T for the chunk's tokens i = 16 wave + l16 (the n side of the product, so
@@ -201,60 +203,85 @@ __global__ __launch_bounds__(256) void gdn_chunk_prep_kernel(ChunkArgs p) {
   {
     const int i = 16 * wave + l16;
     const float ell_i = ell_s[i], bet_i = bet_s[i];
+    bf16x8_t bki[4];
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) bki[ks] = ld8(&Kr[i * LDK + 32 * ks + 8 * lg]);
 #pragma unroll
     for (int nt = 0; nt < 4; ++nt) {
       f32x4_t kk = {0.f, 0.f, 0.f, 0.f}, qk = {0.f, 0.f, 0.f, 0.f};
       if (nt <= wave) {
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) {
-          const bf16x8_t a = nt < wave ? akj[nt < 3 ? nt : 0][ks] : bki[ks];
+          const bf16x8_t a = ld8(&Kr[(16 * nt + l16) * LDK + 32 * ks + 8 * lg]);
           kk = mfma(a, bki[ks], kk);  // [j][i]
           qk = mfma(a, bqi[ks], qk);
         }
       }
       bf16_t ph[4], pl[4];
+      f32x4_t ar;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int j = 16 * nt + 4 * lg + r;
         const float e = j <= i ? __expf(ell_i - ell_s[j]) : 0.f;
-        Ap[r * APLANE + i * AROW + 4 * nt + lg] = j < i ? bet_i * e * kk[r] : 0.f;
+        ar[r] = j < i ? bet_i * e * kk[r] : 0.f;
         split_bf16(e * qk[r], &ph[r], &pl[r]);
       }
+      if (nt <= wave) *reinterpret_cast<f32x4_t*>(&A[i * LDA + 16 * nt + 4 * lg]) = ar;
       // element (i, j = 16 nt + 4 lg + r): tile i / 16, slab j / 32, lane (j % 32 / 8) * 16 + i % 16
       const size_t po = ch * C * C + ((size_t)(wave * 2 + (nt >> 1)) * 64 + (2 * (nt & 1) + (lg >> 1)) * 16 + l16) * 8 + 4 * (lg & 1);
       *reinterpret_cast<uint2*>(p.pm + po) = make_uint2(ph[0] | ((uint32_t)ph[1] << 16), ph[2] | ((uint32_t)ph[3] << 16));
       *reinterpret_cast<uint2*>(p.pl + po) = make_uint2(pl[0] | ((uint32_t)pl[1] << 16), pl[2] | ((uint32_t)pl[3] << 16));
     }
   }
-  __syncthreads();
-  PR_MARK(3);
-
-  // ---- T = (I + A)^-1 by forward substitution. Thread (column c = tid / 4, part q4 = tid % 4)
-  // keeps T[j][c] for j = q4 mod 4; a row's sum over j is four partial sums met inside the quad.
-  const int col = tid >> 2, q4 = tid & 3;
-  float tq[C / 4];
-#pragma unroll
-  for (int m = 0; m < C / 4; ++m) tq[m] = 0.f;
+  // ---- T = (I + A)^-1 in blocks of 16, fp32 throughout (a row at a time over all 64 columns it was a chain of 64 steps, 4.3 of
+  // the workgroup's 12 us). Wavefront w owns the block column w. It inverts its diagonal block (16 steps; its rows of A are its own),
+  // and when all four are there, T_Iw = -D_I sum_K A_IK T_Kw downwards on the matrix cores. Lane (l16, lg) holds rows 4 lg + r of
+  // column l16 of a block, which is what a product leaves and, with the k of step s taken as 4 lg + s, what the next one takes.
+  f32x4_t tb[4];  // block rows
   {
-    const float* arow = &Ap[q4 * APLANE];
+    f32x4_t t = {0.f, 0.f, 0.f, 0.f};
+    f32x4_t arow[16];
 #pragma unroll
-    for (int i = 0; i < C; ++i) {
-      float acc = 0.f;
+    for (int i = 0; i < 16; ++i) arow[i] = *reinterpret_cast<const f32x4_t*>(&A[(16 * wave + i) * LDA + 16 * wave + 4 * lg]);
 #pragma unroll
-      for (int m4 = 0; m4 < (i + 3) / 4; m4 += 4) {
-        const float4 a4 = *reinterpret_cast<const float4*>(arow + i * AROW + m4);
-        acc = dm_fma(a4.x, tq[m4], acc);
-        if (m4 + 1 < (i + 3) / 4) acc = dm_fma(a4.y, tq[m4 + 1], acc);
-        if (m4 + 2 < (i + 3) / 4) acc = dm_fma(a4.z, tq[m4 + 2], acc);
-        if (m4 + 3 < (i + 3) / 4) acc = dm_fma(a4.w, tq[m4 + 3], acc);
+    for (int i = 0; i < 16; ++i) {
+      float acc = arow[i][0] * t[0];
+#pragma unroll
+      for (int r = 1; r < 4; ++r) acc = dm_fma(arow[i][r], t[r], acc);
+      float x, y;
+      dm_row_swap<16>(acc, x, y);
+      acc = x + y;
+      dm_row_swap<32>(acc, x, y);
+      acc = x + y;
+      const float ti = (i == l16 ? 1.f : 0.f) - acc;
+      t[i & 3] = lg == (i >> 2) ? ti : t[i & 3];
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) Dg[wave][(4 * lg + r) * LDD + l16] = t[r];
+#pragma unroll
+    for (int I = 0; I < 4; ++I) tb[I] = I == wave ? t : f32x4_t{0.f, 0.f, 0.f, 0.f};
+  }
+  __syncthreads();  // (K by token has been read, too: its memory becomes T)
+  PR_MARK(3);
+#pragma unroll
+  for (int I = 1; I < 4; ++I) {
+    if (I > wave) {
+      f32x4_t sum = {0.f, 0.f, 0.f, 0.f}, t = sum;
+#pragma unroll
+      for (int K = 0; K < I; ++K) {
+        if (K >= wave) {
+          const f32x4_t a = *reinterpret_cast<const f32x4_t*>(&A[(16 * I + l16) * LDA + 16 * K + 4 * lg]);
+#pragma unroll
+          for (int s = 0; s < 4; ++s) sum = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s], tb[K][s], sum, 0, 0, 0);
+        }
       }
-      acc = acc + dm_xor_lane<1>(acc);
-      acc = acc + dm_xor_lane<2>(acc);
-      const float ti = (i == col ? 1.f : 0.f) - acc;
-      tq[i >> 2] = q4 == (i & 3) ? ti : tq[i >> 2];
+      const f32x4_t d = *reinterpret_cast<const f32x4_t*>(&Dg[I][l16 * LDD + 4 * lg]);
+#pragma unroll
+      for (int s = 0; s < 4; ++s) t = __builtin_amdgcn_mfma_f32_16x16x4f32(d[s], sum[s], t, 0, 0, 0);
+      tb[I] = -t;
     }
   }
-  __syncthreads();  // A has been read; its memory becomes T
+  const int col = 16 * wave + l16;
   PR_MARK(4);
 
   // two passes over T with its columns scaled: by beta e_j0 against K (W), by beta against V (U).
@@ -264,7 +291,9 @@ __global__ __launch_bounds__(256) void gdn_chunk_prep_kernel(ChunkArgs p) {
     {
       const float sc = pass == 0 ? bet_s[col] * __expf(ell_s[col]) : bet_s[col];
 #pragma unroll
-      for (int m = 0; m < C / 4; ++m) split_bf16(tq[m] * sc, &Th[4 * m + q4][col], &Tl[4 * m + q4][col]);
+      for (int I = 0; I < 4; ++I)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) split_bf16(tb[I][r] * sc, &Th[16 * I + 4 * lg + r][col], &Tl[16 * I + 4 * lg + r][col]);
     }
     __syncthreads();
     const int i = 16 * wave + l16;
@@ -280,11 +309,11 @@ __global__ __launch_bounds__(256) void gdn_chunk_prep_kernel(ChunkArgs p) {
 #pragma unroll
       for (int ks = 0; ks < 2; ++ks) {
         if (pass == 0) {
-          const bf16x8_t a = ld8(&Kt[16 * nt + l16][32 * ks + 8 * lg]);
+          const bf16x8_t a = ld8(turned(Kt, 16 * nt + l16, 4 * ks + lg));
           acc = mfma(a, bh[ks], acc);  // [dk 16 nt + 4 lg + r][token i]
           acc = mfma(a, bl[ks], acc);
         } else {
-          const bf16x8_t b = ld8(&Vt[16 * nt + l16][32 * ks + 8 * lg]);
+          const bf16x8_t b = ld8(turned(Vt, 16 * nt + l16, 4 * ks + lg));
           acc = mfma(bh[ks], b, acc);  // [token 16 wave + 4 lg + r][dv 16 nt + l16]
           acc = mfma(bl[ks], b, acc);
         }
