@@ -379,19 +379,29 @@ static int linear_matmul_multi(ornith_ctx* ctx, const ornith_linear* const* ws, 
     return launch_dense<false>(ctx, s, d_x, ws[0]->K, 1, M, nullptr, nullptr, M);
   }
   // Prefill widths: the matrices that take the few-row GEMM share a launch of it (all of them, or the
-  // ones with few columns of a wider call), the others go on below.
+  // ones with few columns of a wider call), narrow dense ones ride along; the others go on below, the dense ones among themselves.
   if (wide && ornith_option_fuse_proj() && n >= 2 && n <= 4) {
-    const ornith_linear *few[4], *rest[4];
-    void *yf[4], *yr[4];
-    int nf = 0, nr = 0;
+    const ornith_linear *few[4], *dense[4], *rest[4];
+    void *yf[4], *yd[4], *yr[4];
+    int nf = 0, nd = 0, nr = 0;
     for (int i = 0; i < n; ++i) {
-      const bool ok = nmm::plain_ok(&ws[i], 1, d_x, M, &d_ys[i]);
-      (ok ? few[nf] : rest[nr]) = ws[i];
-      (ok ? yf[nf++] : yr[nr++]) = d_ys[i];
+      const bool ok = nmm::plain_ok(&ws[i], 1, d_x, M, &d_ys[i]), plain_dense = ws[i]->mode == ORNITH_LIN_DENSE;
+      (ok ? few[nf] : plain_dense ? dense[nd] : rest[nr]) = ws[i];
+      (ok ? yf[nf++] : plain_dense ? yd[nd++] : yr[nr++]) = d_ys[i];
     }
-    if (nf >= 2 && nmm::plain_ok(few, nf, d_x, M, yf)) {
-      const int rc = nmm::plain(ctx, few, nf, d_x, M, yf);
-      return rc || nr == 0 ? rc : linear_matmul_multi(ctx, rest, nr, d_x, M, yr, wide);
+    const bool shared = nf >= 2 && nmm::plain_ok(few, nf, d_x, M, yf);
+    if (shared || (nd && nd < n)) {
+      const bool riding = shared && nmm::riders_ok(dense, nd, few[0]->K);
+      int rc = ORNITH_OK;
+      if (shared) rc = nmm::plain(ctx, few, nf, d_x, M, yf, dense, riding ? nd : 0, yd);
+      else
+        for (int i = 0; i < nf; ++i) {
+          rest[nr] = few[i];
+          yr[nr++] = yf[i];
+        }
+      if (!rc && nr) rc = linear_matmul_multi(ctx, rest, nr, d_x, M, yr, wide);
+      if (!rc && nd && !riding) rc = linear_matmul_multi(ctx, dense, nd, d_x, M, yd, wide);
+      return rc;
     }
   }
   // ... dense matrices of one K likewise

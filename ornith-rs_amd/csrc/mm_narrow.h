@@ -76,6 +76,15 @@ struct Mat {
   int cb0;  // plain form: first column block of the launch that is this matrix's
 };
 
+// Dense bf16 matrices that ride along with a plain launch: 16 x 16 tiles, numbered row tile by row tile, the matrices' column
+// tiles laid end to end.
+struct Riders {
+  const bf16_t* w[2];
+  bf16_t* y[2];
+  int O[2];
+  int tiles, wgs;  // column tiles; workgroups
+};
+
 struct Args {
   Mat m[4];  // plain: up to four matrices; gathered: [0] routed (or gate), [1] routed up, [2] shared (gate), [3] shared up
   int n;
@@ -91,6 +100,7 @@ struct Args {
   int up_div, pairs, E;
   uint32_t up_magic;  // 2^32 / up_div rounded up: the upper half of its product with a pair is pair / up_div
   int tiles_max, blocks;  // room in the tile list; column blocks a tile
+  Riders d;
 };
 
 // bytes of a 256-weight block in the three tensors
@@ -858,6 +868,57 @@ __device__ __forceinline__ void owned_tile(const Args& a, int mat0, int c0, int6
   }
 }
 
+// One 16 x 16 tile of a riding dense matrix, K a multiple of 2048: sixteen parts of K, the partial tiles added in order, as
+// linear.hip's dense_mm_kernel<16, 1> does it (which has a wavefront a part; here it is four) and so with the same bits. As a launch of
+// its own that is a chain of 6 us in 16 workgroups (the a / b heads of a gated-delta layer, 51 rows); here it runs beside
+// the wide projections' 12288 columns: us, two launches / one, 51 rows 14.6 + 6.3 / 15.3, 600 rows over 4-bit affine weights 62.1 + 6.9 / 64.6.
+__device__ __forceinline__ void rider_tile(const Args& a, uint32_t id, uint8_t* smem) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l16 = lane & 15, lg = lane >> 4;
+  const int rt = (int)(id / (uint32_t)a.d.tiles);
+  int t = (int)id - rt * a.d.tiles;
+  const int first = (a.d.O[0] + 15) / 16, seg = t >= first;
+  t -= seg ? first : 0;
+  const bf16_t* w = seg ? a.d.w[1] : a.d.w[0];
+  bf16_t* y = seg ? a.d.y[1] : a.d.y[0];
+  const int O = seg ? a.d.O[1] : a.d.O[0], col = 16 * t + l16, kw = a.K / 16;
+  const bf16_t* xp = a.x + (size_t)min(16 * rt + l16, a.M - 1) * a.K + 8 * lg;
+  const bf16_t* wp = w + (size_t)min(col, O - 1) * a.K + 8 * lg;
+  f32x4_t acc[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) acc[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  for (int k0 = 0; k0 < kw; k0 += 128)
+#pragma unroll
+    for (int h = 0; h < 4; h += 2) {  // (two parts' operands at a time: all four are more registers than the smallest kernel has)
+      bf16x8_t xa[2][4], wb[2][4];
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+          const int at = (4 * wave + h + i) * kw + k0 + 32 * s;
+          xa[i][s] = *reinterpret_cast<const bf16x8_t*>(xp + at);
+          wb[i][s] = *reinterpret_cast<const bf16x8_t*>(wp + at);
+        }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int s = 0; s < 4; ++s) acc[h + i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa[i][s], wb[i][s], acc[h + i], 0, 0, 0);
+    }
+  f32x4_t* const red = reinterpret_cast<f32x4_t*>(smem) + lane;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) red[(4 * wave + i) * 64] = acc[i];
+  __syncthreads();
+  if (wave != 0) return;
+  f32x4_t v = red[0];
+#pragma unroll
+  for (int p = 1; p < 16; ++p) v += red[p * 64];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int row = 16 * rt + 4 * lg + r;
+    if (col < O && row < a.M) y[(size_t)row * O + col] = dm_f2bf(v[r]);
+  }
+}
+
 // AFF: affine formats, else k-quants; ONE: the kind of every matrix of the launch, or -1. NW wavefronts, K >= 512.
 // Plain: grid (column blocks, row tiles); gathered: a workgroup a column block of a tile.
 template <bool AFF, int CT, int MODE, int ROWS, int NW, int ONE = -1>
@@ -867,6 +928,11 @@ __device__ __forceinline__ void body(const Args& a) {
   int64_t row_base = 0;
   const uint32_t* my_pairs = nullptr;
   if constexpr (MODE == kPlain) {
+    if ((int)blockIdx.x >= a.blocks) {
+      const uint32_t id = (blockIdx.x - (uint32_t)a.blocks) * gridDim.y + blockIdx.y;
+      if (id < (uint32_t)a.d.wgs) rider_tile(a, id, nmm_smem);
+      return;
+    }
 #pragma unroll
     for (int i = 1; i < 4; ++i)
       if (i < a.n && (int)blockIdx.x >= a.m[i].cb0) {
@@ -878,7 +944,13 @@ __device__ __forceinline__ void body(const Args& a) {
     c0 = cb * (NW / a.ks) * CT * 16;
   } else if constexpr (MODE == kTall) {
     // (a die's workgroups: the row tiles of one column block after the other, so that its L2 fetches the weights once)
-    const uint32_t die = blockIdx.x % 8u, seq = blockIdx.x / 8u, rt = seq % (uint32_t)a.tiles_max;
+    // (the riders first, in whole rounds of dies)
+    const uint32_t ahead = ((uint32_t)a.d.wgs + 7u) / 8u * 8u;
+    if (blockIdx.x < ahead) {
+      if (blockIdx.x < (uint32_t)a.d.wgs) rider_tile(a, blockIdx.x, nmm_smem);
+      return;
+    }
+    const uint32_t id = blockIdx.x - ahead, die = id % 8u, seq = id / 8u, rt = seq % (uint32_t)a.tiles_max;
     cb = (int)(seq / (uint32_t)a.tiles_max * 8u + die);
     if (cb >= a.blocks) return;
 #pragma unroll

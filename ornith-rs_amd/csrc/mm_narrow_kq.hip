@@ -85,7 +85,7 @@ int launch_tall(ornith_ctx* ctx, Args& a) {
     if (a.m[i].kind != kind) kind = -1;
   }
   a.tiles_max = (a.M + 63) / 64;
-  const dim3 grid((unsigned)((a.blocks + 7) / 8 * 8 * a.tiles_max));
+  const dim3 grid((unsigned)((a.blocks + 7) / 8 * 8 * a.tiles_max + (a.d.wgs + 7) / 8 * 8));
   return affine(a.m[0].kind) ? launch_affine(ctx, a, kTall, 0, 64, kind, grid, lds) : launch_kq(ctx, a, kTall, 0, 64, kind, grid, lds);
 }
 
@@ -130,14 +130,30 @@ int launch_split(ornith_ctx* ctx, Args& a) {
     };
     while (ct > 1 && !suits()) ct /= 2;
   }
-  const dim3 grid(blocks_of(ct), rows == 32 ? thirty : sixty);
+  const int row_tiles = rows == 32 ? thirty : sixty;
+  const dim3 grid(blocks_of(ct) + (a.d.wgs + row_tiles - 1) / row_tiles, row_tiles);
   const int lds = lds_bytes(a, (4 / a.ks) * ct * 16, rows, ct, 4);
   return affine(a.m[0].kind) ? launch_affine(ctx, a, kPlain, ct, rows, -1, grid, lds) : launch_kq(ctx, a, kPlain, ct, rows, -1, grid, lds);
 }
 }  // namespace
 
-int plain(ornith_ctx* ctx, const ornith_linear* const* ws, int n, const void* d_x, int M, void* const* d_ys) {
-  // the matrices of one form share a launch
+bool riders_ok(const ornith_linear* const* ws, int n, int K) {
+  for (int i = 0; i < n; ++i)
+    if (ws[i]->mode != ORNITH_LIN_DENSE || !ws[i]->d_w || ws[i]->K != K || ws[i]->O < 1 || ((uintptr_t)ws[i]->d_w & 15) != 0) return false;
+  return n >= 1 && n <= 2 && K % 2048 == 0;
+}
+
+int plain(ornith_ctx* ctx, const ornith_linear* const* ws, int n, const void* d_x, int M, void* const* d_ys,
+          const ornith_linear* const* riders, int n_riders, void* const* d_yr) {
+  Riders d{};
+  for (int i = 0; i < n_riders; ++i) {
+    d.w[i] = (const bf16_t*)riders[i]->d_w;
+    d.y[i] = (bf16_t*)d_yr[i];
+    d.O[i] = riders[i]->O;
+    d.tiles += (riders[i]->O + 15) / 16;
+  }
+  d.wgs = (M + 15) / 16 * d.tiles;
+  // the matrices of one form share a launch; the riders go with the first
   for (const bool form : {true, false}) {
     Args a{};
     a.x = (const bf16_t*)d_x;
@@ -146,6 +162,8 @@ int plain(ornith_ctx* ctx, const ornith_linear* const* ws, int n, const void* d_
     for (int i = 0; i < n; ++i)
       if (tall(*ws[i], M) == form) a.m[a.n++] = mat_of(*ws[i], d_ys[i]);
     if (a.n == 0) continue;
+    a.d = d;
+    d = Riders{};
     const int rc = form ? launch_tall(ctx, a) : launch_split(ctx, a);
     if (rc) return rc;
   }

@@ -213,22 +213,20 @@ static int forward_rows(ornith_model* m, ornith_caches* cc, const uint32_t* d_to
     const PendingNorm* pp = i > 0 ? &pend : nullptr;
     if (L.linear) {
       const GdnLayer& g = L.gdn;
-      const ornith_linear* big[2] = {&g.in_proj_qkv, &g.in_proj_z};
-      void* ybig[2] = {s.qkv, s.z};
-      if (pp)
-        TRY(ornith_add_rms_linear_multi(ctx, big, 2, pp->res, pp->y, pp->w, c.rms_norm_eps, T, pp->h_out,
-                                        s.normed, ybig));
-      else
-        TRY(ornith_linear_matmul_multi(ctx, big, 2, s.normed, T, ybig));
-      const char* conv_state = (const char*)lc.conv[cc->conv_cur] + (size_t)cc->conv_off * D * 2;
-      const float* state_in = lc.state + (size_t)cc->state_cur * ssz;
       const bool dense_ab = g.in_proj_a.mode == ORNITH_LIN_DENSE && g.in_proj_b.mode == ORNITH_LIN_DENSE;
       const bool fused = T <= 16 && Dk == 128 && Dv == 128 && ornith_option_fuse_gdn();
-      if (!(fused && dense_ab)) {
-        const ornith_linear* ab[2] = {&g.in_proj_a, &g.in_proj_b};
-        void* yab[2] = {s.a, s.b};
-        TRY(ornith_linear_matmul_multi(ctx, ab, 2, s.normed, T, yab));
-      }
+      // the step makes dense a / b itself; at prompt widths they ride along with the wide projections
+      const bool ab_here = !(fused && dense_ab), together = ab_here && T >= kPrefillRows;
+      const ornith_linear* in[4] = {&g.in_proj_qkv, &g.in_proj_z, &g.in_proj_a, &g.in_proj_b};
+      void* out[4] = {s.qkv, s.z, s.a, s.b};
+      if (pp)
+        TRY(ornith_add_rms_linear_multi(ctx, in, together ? 4 : 2, pp->res, pp->y, pp->w, c.rms_norm_eps, T, pp->h_out,
+                                        s.normed, out));
+      else
+        TRY(ornith_linear_matmul_multi(ctx, in, together ? 4 : 2, s.normed, T, out));
+      const char* conv_state = (const char*)lc.conv[cc->conv_cur] + (size_t)cc->conv_off * D * 2;
+      const float* state_in = lc.state + (size_t)cc->state_cur * ssz;
+      if (ab_here && !together) TRY(ornith_linear_matmul_multi(ctx, in + 2, 2, s.normed, T, out + 2));
       if (fused) {
         TRY(ornith_gdn_step(ctx, conv_state, s.qkv, g.conv1d, dense_ab ? nullptr : s.a,
                             dense_ab ? nullptr : s.b, dense_ab ? g.in_proj_a.d_w : nullptr,

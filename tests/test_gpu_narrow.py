@@ -55,6 +55,34 @@ def test_few_row_matmul_vs_float64(orn, ctx, fmt, O, K, M):
     dl.free()
 
 
+@pytest.mark.parametrize("fmt", ["q4k", "affine4", "affine8"])
+@pytest.mark.parametrize("O,dense,K,M", [(512, (32, 32), 2048, 32), (4096, (1, 40), 2048, 51), (2056, (32,), 2048, 193),
+                                         (4096, (32, 17), 2048, 500), (264, (16, 1), 4096, 77), (512, (32, 32), 1024, 40),
+                                         (4096, (32, 32), 2048, 1300)])
+def test_dense_matrices_ride_along_with_a_few_row_gemm(orn, ctx, fmt, O, dense, K, M):
+    """linear_matmul_multi of two quantized matrices and one or two narrow dense ones at prompt widths: one launch where K
+    allows (in the form with K split over wavefronts and in the one with columns owned; rows and columns ragged), and
+    every output is the matrix's own launch bit for bit, past every output nothing is written"""
+    rng = np.random.default_rng(O + K + M)
+    make = {"q4k": lambda o: util.HostLinear.kq(rng, Q4K, o, K), "affine4": lambda o: util.HostLinear.affine4(rng, o, K),
+            "affine8": lambda o: util.HostLinear.affine8(rng, o, K)}[fmt]
+    hls = [make(O), make(256)] + [util.HostLinear.dense(rng, o, K) for o in dense]
+    Os = [O, 256] + list(dense)
+    lins = [h.dev(orn, ctx) for h in hls]
+    dx = ctx.to_device(util.bf16_normal(rng, (M, K)))
+    ys = [ctx.alloc((M + 1) * o * 2) for o in Os]
+    for y, o in zip(ys, Os): ctx.memset(y, 0x5A, (M + 1) * o * 2)
+    ctx.linear_matmul_multi(lins, dx, M, ys)
+    y1 = ctx.alloc(M * max(Os) * 2)
+    for lin, y, o in zip(lins, ys, Os):
+        ctx.linear_matmul(lin, dx, M, y1)
+        got = y.download(np.uint16, (M + 1, o))
+        assert np.array_equal(got[:M], y1.download(np.uint16, (M, o))), o
+        assert np.all(got[M] == 0x5A5A), o
+    for b in [dx, y1] + ys: b.free()
+    for l in lins: l.free()
+
+
 @pytest.mark.parametrize("fmt", ["kq", "affine4"])
 @pytest.mark.parametrize("T", [32, 100, 150, 300])
 def test_few_row_moe_block_vs_exact(orn, ctx, fmt, T):
