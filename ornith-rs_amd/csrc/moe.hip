@@ -128,42 +128,67 @@ __global__ void swiglu_kernel(const bf16_t* gate, const bf16_t* up, bf16_t* out,
   reinterpret_cast<P*>(out)[i] = o8;
 }
 
-// one thread per V output elements of a token; j ascends, every step rounds to bf16
+// One thread per V output elements of a token; j ascends, every step rounds to bf16. Bound by the stream at long prompts, by one trip
+// to memory at short ones: eight experts' rows, their scores and the rest are asked for at once (past k the last one again,
+// unused), and nothing is divided but by the workgroup. With the scores added up one load after the other ahead of the rows, us, 51 / 700 /
+// 6621 tokens: 5.3 / 10.3 / 62.4 -> 5.0 / 8.3 / 53.
 template <int V>
-__global__ void moe_combine_kernel(const bf16_t* scores, const bf16_t* y, const bf16_t* gate,
-                                   const bf16_t* shared, bf16_t* out, int T, int k, int dim,
-                                   int normalize) {
+__global__ __launch_bounds__(256) void moe_combine_kernel(const bf16_t* scores, const bf16_t* y, const bf16_t* gate,
+                                                          const bf16_t* shared, bf16_t* out, int T, int k, int dim, int normalize) {
   typedef typename BfPack<V>::type P;
-  const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int per_row = dim / V;
-  if (idx >= (int64_t)T * per_row) return;
-  const int t = (int)(idx / per_row), c = (int)(idx - (int64_t)t * per_row) * V;
+  // (a grid has fewer than 2^32 threads)
+  const uint32_t per_row = dim / V, base = blockIdx.x * 256u, t0 = base / per_row;
+  uint32_t r = base - t0 * per_row + threadIdx.x, t = t0;
+  if (per_row >= 256u) {
+    if (r >= per_row) {
+      r -= per_row;
+      ++t;
+    }
+  } else {
+    t += r / per_row;
+    r %= per_row;
+  }
+  if (t >= (uint32_t)T) return;
+  const uint32_t c = r * V;
   const bf16_t* s = scores + (size_t)t * k;
-  float denom = 0.f;
-  if (normalize)
-    for (int j = 0; j < k; ++j) denom = dm_rb(dm_bf2f(s[j]) + denom);
-  // eight experts' rows are asked for at once (in a loop over the experts every row waited for the
-  // arithmetic of the one before); past k the last row again, unused
+  P yj[8];
+  bf16_t sj[8];
+  auto fetch = [&](int j0) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      yj[j] = *reinterpret_cast<const P*>(y + ((size_t)t * k + min(j0 + j, k - 1)) * dim + c);
+      sj[j] = s[min(j0 + j, k - 1)];
+    }
+  };
+  fetch(0);
   const P sh = *reinterpret_cast<const P*>(shared + (size_t)t * dim + c);
+  const bf16_t gt = gate[t];
+  float denom = 0.f;
+  if (normalize) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      if (j < k) denom = dm_rb(dm_bf2f(sj[j]) + denom);
+    for (int j = 8; j < k; ++j) denom = dm_rb(dm_bf2f(s[j]) + denom);
+  }
   float acc[V];
 #pragma unroll
   for (int e = 0; e < V; ++e) acc[e] = 0.f;
-  for (int j0 = 0; j0 < k; j0 += 8) {
-    P yj[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) yj[j] = *reinterpret_cast<const P*>(y + ((size_t)t * k + min(j0 + j, k - 1)) * dim + c);
+  for (int j0 = 0;;) {
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       if (j0 + j >= k) break;
-      const float w = normalize ? dm_rb(dm_bf2f(s[j0 + j]) / denom) : dm_bf2f(s[j0 + j]);
+      const float w = normalize ? dm_rb(dm_bf2f(sj[j]) / denom) : dm_bf2f(sj[j]);
 #pragma unroll
       for (int e = 0; e < V; ++e) {
         const float weighted = dm_rb(bf_get<V>(yj[j], e) * w);
         acc[e] = dm_rb(weighted + acc[e]);
       }
     }
+    j0 += 8;
+    if (j0 >= k) break;
+    fetch(j0);
   }
-  const float g = dm_sigmoid_bf16(dm_bf2f(gate[t]));
+  const float g = dm_sigmoid_bf16(dm_bf2f(gt));
   P o;
 #pragma unroll
   for (int e = 0; e < V; ++e) {

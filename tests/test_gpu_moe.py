@@ -130,6 +130,28 @@ def test_swiglu_and_combine_bit_exact(orn, ctx):
     for b in (dg, du, do): b.free()
 
 
+@pytest.mark.parametrize("T,k,dim", [(7, 9, 24), (3, 16, 4104), (5, 1, 2056), (600, 8, 8), (33, 8, 2048), (300, 2, 3)])
+def test_combine_over_rows_and_workgroups(orn, ctx, T, k, dim):
+    """rows shorter and longer than a workgroup and no multiple of it, one expert and more than eight, one and eight elements
+    a thread; nothing past the last row is written"""
+    rng = np.random.default_rng(T + k + dim)
+    scores = util.f32_to_bf16(rng.random((T, k)).astype(np.float32) * 0.1)
+    y = util.f32_to_bf16(rng.standard_normal((T, k, dim)).astype(np.float32))
+    gate = util.f32_to_bf16(rng.standard_normal(T).astype(np.float32) * 3)
+    shared = util.f32_to_bf16(rng.standard_normal((T, dim)).astype(np.float32))
+    bufs = [ctx.to_device(a) for a in (scores, y, gate, shared)]
+    for norm in (1, 0):
+        want = np.empty((T, dim), np.uint16)
+        oracle().orc_moe_combine(p(scores), p(y), p(gate), p(shared), T, k, dim, norm, p(want))
+        out = ctx.alloc((T + 1) * dim * 2)
+        ctx.memset(out, 0x5A, (T + 1) * dim * 2)
+        ctx.moe_combine(*bufs, T, k, dim, norm, out)
+        got = out.download(np.uint16, (T + 1, dim))
+        assert np.array_equal(got[:T], want) and np.all(got[T] == 0x5A5A)
+        out.free()
+    for b in bufs: b.free()
+
+
 def _run_block(orn, ctx, moe, dw, xb, T):
     dx, dout = ctx.to_device(xb), ctx.alloc(T * moe.H * 2)
     di, ds = ctx.alloc(T * moe.top_k * 4), ctx.alloc(T * moe.top_k * 2)
