@@ -134,6 +134,12 @@ static inline bool prenorm_apart(const PreNorm& p, int rows) {
   return prenorm_apart(p, rows, p.h_out, n) && prenorm_apart(p, rows, p.normed_out, n);
 }
 
+// Rows from which a row's sum of squares is one wavefront's: its 64 canonical lanes are that wavefront's lanes, which read the
+// row back from LDS. Below, every thread runs its part of every row's chain, without the trip through LDS and its barrier. In front of
+// 12288 x 2048 of Q4_K, us, every thread / a wavefront a row: two rows 8.87 / 8.76 (a whole decode of two-row steps 82.2 / 82.8 ms), three
+// 11.0 / 10.7, four 13.0 / 12.8 (four-row steps 124.0 / 123.0 ms).
+constexpr int kPreSplit = 3;
+
 template <int T>
 struct PreNormLds {
   __attribute__((aligned(16))) bf16_t xn[T][kPreN];
@@ -199,6 +205,10 @@ __device__ __forceinline__ void prenorm_finish(const PreNorm& p, const PreNormRe
     }
     if (write_global)
       *reinterpret_cast<uint4*>(p.h_out + (size_t)t * kPreN + e0) = make_uint4(hp[0], hp[1], hp[2], hp[3]);
+    if constexpr (T >= kPreSplit) {
+      *reinterpret_cast<uint4*>(&s.xn[t][e0]) = make_uint4(hp[0], hp[1], hp[2], hp[3]);
+      continue;
+    }
     float acc = 0.f;
 #pragma unroll
     for (int step = 0; step < 4; ++step) {
@@ -214,9 +224,29 @@ __device__ __forceinline__ void prenorm_finish(const PreNorm& p, const PreNormRe
   }
   __syncthreads();
   float invs[T];
+  if constexpr (T >= kPreSplit) {
+    // wavefront t makes row t's sum, a canonical lane a lane: one chain of 32 where every thread ran T
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    if (wave < T) {
+      float acc = 0.f;
 #pragma unroll
-  for (int t = 0; t < T; ++t)
-    invs[t] = dm_rsqrt(dm_wave_sum<64>(s.part[t][lane]) / (float)kPreN + p.eps);
+      for (int c = 0; c < 4; ++c) {
+        float v[8];
+        unpack_bf16x8(*reinterpret_cast<const uint4*>(&s.xn[wave][32 * lane + 8 * c]), v);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) acc = dm_fma(v[i], v[i], acc);
+      }
+      const float inv = dm_rsqrt(dm_wave_sum<64>(acc) / (float)kPreN + p.eps);
+      if (lane == 0) s.part[wave][0] = inv;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < T; ++t) invs[t] = s.part[t][0];
+  } else {
+#pragma unroll
+    for (int t = 0; t < T; ++t)
+      invs[t] = dm_rsqrt(dm_wave_sum<64>(s.part[t][lane]) / (float)kPreN + p.eps);
+  }
 #pragma unroll
   for (int t = 0; t < T; ++t) {
     const float inv = invs[t];
