@@ -253,7 +253,11 @@ def test_model_prefill_in_wide_chunks_close_to_exact_chunks(orn, ctx, exact_weig
 
 
 @pytest.mark.parametrize("T,Hq,Hkv,cap,offset", [(64, 16, 2, 512, 0), (100, 4, 1, 1024, 37), (300, 16, 2, 2048, 1000),
-                                                 (33, 2, 2, 256, 200), (512, 8, 2, 1024, 512)])
+                                                 (33, 2, 2, 256, 200), (512, 8, 2, 1024, 512),
+                                                 # four key blocks (one set of wavefronts); five and seven, so that the second set
+                                                 # of two ends on a masked one, rows that it has no key of; 128-row workgroups, ragged
+                                                 (256, 2, 1, 512, 0), (320, 2, 1, 512, 0), (33, 4, 1, 512, 256), (130, 3, 3, 512, 300),
+                                                 (385, 64, 4, 512, 20)])
 def test_prefill_attention_close_to_exact_kernel(orn, ctx, T, Hq, Hkv, cap, offset):
     """Causal flash attention on the matrix cores vs the oracle's exact attention: every row
     within 1 % relative L2 (bf16 probabilities into the second GEMM, fp32 sums in block order).
