@@ -1367,19 +1367,17 @@ int ornith_kq_gather_matmul(ornith_ctx* ctx, const ornith_kmatrix* w, const void
   ORN_REQUIRE(pairs >= 1 && top_k >= 1 && pairs % top_k == 0 && w->E <= 1024,
               "kq_gather_matmul: pairs=%d top_k=%d E=%d", pairs, top_k, w->E);
   // Rows per plan tile: the choice depends only on pairs and E (and the option), so the calls
-  // sharing a plan agree on it. With 48 rows an expert or more: the smallest of 96 / 128 / 160 /
-  // 192 rows that holds an expert's share of the pairs with 2.5 standard deviations to spare, so
-  // that nearly every expert is one tile (the register form dequantizes its weights once).
-  // Otherwise the same rule over the few-row kernels' 16 / 32 / 64 rows.
+  // sharing a plan agree on it. With 48 rows an expert or more 192, the register form's most: nearly every expert
+  // is one tile there (its weights are dequantized once), one of fewer rows runs the loop for the rows it has, and the 64-row
+  // workgroups of the down projection come in threes, of which the empty ones end at once. (A height that just holds an expert's
+  // share brings those in twos, a full and a partial one, which fall on the same compute units over and over: us, gate / down,
+  // 1600 tokens with 96-row tiles 85 / 137, with 192 77 / 95; 2700 tokens, 128, 97 / 160, 192 94 / 128; 4096, 160, 115 / 181, 192 115 / 173;
+  // at 6621 tokens, 207 rows an expert, 160 162 / 266, 128 178 / 281, 192 164 / 250.)
+  // Otherwise the few-row kernels' 16 / 32 / 64 rows, the smallest that most experts' shares fit.
   const int avg = pairs / w->E;
-  int spare = 0;
-  while (4 * spare * spare < 25 * avg) ++spare;
-  const int need = avg + spare;
   const bool narrow = pairs < nmm::kNarrowPairs * w->E;
   const bool tall = ornith_option_gemm_reg() && !narrow;
-  const int tile_rows = narrow ? nmm::tile_rows(pairs, w->E)
-                        : tall ? (need <= 96 ? 96 : need <= 128 ? 128 : need <= 160 ? 160 : 192)
-                               : avg >= 96 ? 128 : 64;
+  const int tile_rows = narrow ? nmm::tile_rows(pairs, w->E) : tall ? RM : avg >= 96 ? 128 : 64;
   // The kernel for this matrix. Few rows an expert: the few-row kernels (mm_narrow.h). Tall plans
   // take the register form when its 32-bit offsets reach:
   // for K >= 1024 a workgroup a plan tile (one a compute unit), for fewer K slabs 64-row
