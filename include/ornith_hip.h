@@ -97,7 +97,7 @@ ORNITH_API int ornith_device_info(ornith_ctx* ctx, char* name, size_t name_len, 
  *               producer and consumer wavefronts (0: every wavefront dequantizes, then
  *               multiplies); same results either way
  *   "gemm_reg"  (ORNITH_GEMM_REG, default 1): the expert-gathered prefill GEMM dequantizes the
- *               weights into MFMA operand registers where the shape suits it (48 rows an expert
+ *               weights into MFMA operand registers where the shape suits it (80 rows an expert
  *               or more: a workgroup a tile for K >= 1024, 64-row workgroups for fewer K slabs;
  *               0: always through LDS); results agree to the order of the fp32 sums
  *   "gdn_chunked" (ORNITH_GDN_CHUNKED, default 1): the gated-delta recurrence of calls of 128

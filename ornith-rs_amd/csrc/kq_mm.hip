@@ -1367,7 +1367,7 @@ int ornith_kq_gather_matmul(ornith_ctx* ctx, const ornith_kmatrix* w, const void
   ORN_REQUIRE(pairs >= 1 && top_k >= 1 && pairs % top_k == 0 && w->E <= 1024,
               "kq_gather_matmul: pairs=%d top_k=%d E=%d", pairs, top_k, w->E);
   // Rows per plan tile: the choice depends only on pairs and E (and the option), so the calls
-  // sharing a plan agree on it. With 48 rows an expert or more 192, the register form's most: nearly every expert
+  // sharing a plan agree on it. With nmm::kNarrowPairs rows an expert or more 192, the register form's most: nearly every expert
   // is one tile there (its weights are dequantized once), one of fewer rows runs the loop for the rows it has, and the 64-row
   // workgroups of the down projection come in threes, of which the empty ones end at once. (A height that just holds an expert's
   // share brings those in twos, a full and a partial one, which fall on the same compute units over and over: us, gate / down,

@@ -19,8 +19,11 @@ constexpr int kNarrowRows = 192, kNarrowRowsSlim = 1024, kTallRowsQ4K = 960;
 // The affine formats have no wide kernels: their projections own columns from here on (4-bit, 12288 x 2048, us, split /
 // owned: 300 rows 37 / 37, 400 rows 50 / 52, 512 rows 56 / 51, 600 rows 68 / 61, 2000 rows 207 / 187).
 constexpr int kTallFromAffine = 448;
-// pairs an expert below which the routed experts take them
-constexpr int kNarrowPairs = 48;
+// Pairs an expert below which the routed experts take them: above that an expert is three tiles of 64 and more, and the wide kernels'
+// one unpacking for all its rows pays. Prompts through 256 experts of 8 a token, ms, here / there: 1600 tokens 24.9 / 26.8, 2000
+// 28.4 / 29.5, 2400 31.4 / 32.6, 2700 35.0 / 35.6, 3000 37.2 / 37.4, 3500 42.0 / 42.1, 4096 47.3 / 46.5, 5000 59.2 / 57.7 (80 is 2560 tokens: past
+// that the two are level).
+constexpr int kNarrowPairs = 80;
 
 // an expert-sorted pair list in device memory, tiles of up to `rows` pairs
 struct Plan {
