@@ -389,7 +389,8 @@ static int linear_matmul_multi(ornith_ctx* ctx, const ornith_linear* const* ws, 
       (ok ? few[nf] : plain_dense ? dense[nd] : rest[nr]) = ws[i];
       (ok ? yf[nf++] : plain_dense ? yd[nd++] : yr[nr++]) = d_ys[i];
     }
-    const bool shared = nf >= 2 && nmm::plain_ok(few, nf, d_x, M, yf);
+    // (a single one, too: in a launch of the wide kernels it would have other sums than alone)
+    const bool shared = nf >= 1 && nmm::plain_ok(few, nf, d_x, M, yf);
     if (shared || (nd && nd < n)) {
       const bool riding = shared && nmm::riders_ok(dense, nd, few[0]->K);
       int rc = ORNITH_OK;

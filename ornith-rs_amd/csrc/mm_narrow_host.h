@@ -15,7 +15,11 @@ namespace nmm {
 // - / 63 / 67, 1200 rows - / 82 / 71). Q6_K goes straight to the wide kernels: its one wide matrix, q_proj, shares their launch
 // with k and v (q, k, v: 300 rows 41 owned, k and v apart, 40 there; 700 rows 57 / 58). The rule looks at one matrix at a
 // time, never at what shares its launch: a matrix gives the same bits alone and in company.
-constexpr int kNarrowRows = 192, kNarrowRowsSlim = 1024, kTallRowsQ4K = 960;
+// The lines for up to 2048 columns, from K = 2048 on (below, the wide kernels' few slabs are over as soon: 2048 x 512 at 1024 rows 10.5 /
+// 9.9): Q4_K 1536 rows (2048 x 4096 at 1200 / 1500 / 2000 rows 44 / 54, 46 / 55, 58 / 57), Q6_K 1024 (2048 x 4096 at 1024 / 1200 / 1500 rows
+// 51 / 57, 56 / 57, 67 / 58), and up to 256 columns, which are 16 to 40 workgroups of the wide kernels, 2560 (the router at 1200 / 2000 / 2500
+// rows 13 / 29, 17 / 29, 21 / 29; level at 4096).
+constexpr int kNarrowRows = 192, kNarrowRowsSlim = 1024, kNarrowRowsSlimQ4K = 1536, kNarrowRowsSlimmest = 2560, kTallRowsQ4K = 960;
 // The affine formats have no wide kernels: their projections own columns from here on (4-bit, 12288 x 2048, us, split /
 // owned: 300 rows 37 / 37, 400 rows 50 / 52, 512 rows 56 / 51, 600 rows 68 / 61, 2000 rows 207 / 187).
 constexpr int kTallFromAffine = 448;

@@ -66,8 +66,11 @@ bool plain_ok(const ornith_linear* const* ws, int n, const void* d_x, int M, voi
   if (K > 4096) return false;  // (the scales of a workgroup's rows would not fit beside the activations)
   // (see kNarrowRows; the affine formats have no wider kernels)
   if (affine(kind_of(*ws[0]))) return true;
-  for (int i = 0; i < n; ++i)
-    if (M > (ws[i]->O <= 2048 ? kNarrowRowsSlim : ws[i]->km.kind == ORNITH_Q4K ? kTallRowsQ4K : kNarrowRows)) return false;
+  for (int i = 0; i < n; ++i) {
+    const bool q4 = ws[i]->km.kind == ORNITH_Q4K;
+    const int slim = K < 2048 ? kNarrowRowsSlim : ws[i]->O <= 256 ? kNarrowRowsSlimmest : q4 ? kNarrowRowsSlimQ4K : kNarrowRowsSlim;
+    if (M > (ws[i]->O <= 2048 ? slim : q4 ? kTallRowsQ4K : kNarrowRows)) return false;
+  }
   return true;
 }
 

@@ -34,6 +34,8 @@ def _weights(lin):
                                     # scales would leave a compute unit one workgroup
                                     (2048, 4096, 64), (2040, 4096, 113), (2048, 4096, 129), (2048, 2048, 65), (256, 2048, 512),
                                     (2048, 4096, 577),
+                                    # the last rows that narrow k-quant matrices take here, and the first past them
+                                    (264, 2048, 1536), (264, 2048, 1537), (256, 2048, 2560), (256, 2048, 2561),
                                     # columns owned by wavefronts: row tiles of 64 and remainders of 16, 32 and 48, two, three,
                                     # eight and sixteen blocks of K, columns past the last workgroup's
                                     (2056, 512, 193), (2184, 768, 481), (4099, 2048, 525), (2064, 4096, 449), (8192, 2048, 940)])
