@@ -37,6 +37,7 @@ struct FrontArgs {
   bf16_t* beta;              // [T, Hv]
   float* g;                  // [T, Hv]
   bf16_t* conv_input;        // [S + T, D]
+  int window_from;           // rows of conv_input before this one are not written
   int T, K, Hk, Hv, D;
   float q_scale, k_scale, eps;
 };
@@ -71,9 +72,9 @@ __global__ __launch_bounds__(64) void gdn_front_kernel(FrontArgs p) {
   // the concatenated window
   {
     uint32_t* ci = reinterpret_cast<uint32_t*>(p.conv_input + (size_t)(S + t) * D + c0);
-    *ci = *reinterpret_cast<const uint32_t*>(p.qkv + (size_t)t * D + c0);
+    if (S + t >= p.window_from) *ci = *reinterpret_cast<const uint32_t*>(p.qkv + (size_t)t * D + c0);
     if (t == 0) {
-      for (int j = 0; j < S; ++j)
+      for (int j = p.window_from; j < S; ++j)
         *reinterpret_cast<uint32_t*>(p.conv_input + (size_t)j * D + c0) =
             *reinterpret_cast<const uint32_t*>(p.conv_state + (size_t)j * D + c0);
     }
@@ -145,7 +146,8 @@ __global__ __launch_bounds__(64) void gdn_front_run_kernel(FrontArgs p) {
   for (int i = 0; i < S; ++i) win[i] = input(t0 + i);
   if (t0 == 0) {
 #pragma unroll
-    for (int j = 0; j < S; ++j) *reinterpret_cast<uint32_t*>(p.conv_input + (size_t)j * D + c0) = win[j];
+    for (int j = 0; j < S; ++j)
+      if (j >= p.window_from) *reinterpret_cast<uint32_t*>(p.conv_input + (size_t)j * D + c0) = win[j];
   }
   const bool is_qk = slot < 2 * p.Hk, is_q = slot < p.Hk;
   const float sc = is_q ? p.q_scale : p.k_scale;
@@ -165,7 +167,7 @@ __global__ __launch_bounds__(64) void gdn_front_run_kernel(FrontArgs p) {
       acc0 = dm_fma(dm_bf2f_lo(win[i]), w0[i], acc0);
       acc1 = dm_fma(dm_bf2f_hi(win[i]), w1[i], acc1);
     }
-    *reinterpret_cast<uint32_t*>(p.conv_input + (size_t)(S + t) * D + c0) = win[S];
+    if (S + t >= p.window_from) *reinterpret_cast<uint32_t*>(p.conv_input + (size_t)(S + t) * D + c0) = win[S];
 #pragma unroll
     for (int i = 0; i < S; ++i) win[i] = win[i + 1];
     const float cv0 = dm_rb(acc0), cv1 = dm_rb(acc1);
@@ -853,12 +855,26 @@ int ornith_gdn_front(ornith_ctx* ctx, const void* d_conv_state, const void* d_qk
                      const void* d_a, const void* d_b, const void* d_a_log, const void* d_dt_bias,
                      int T, int K, int Hk, int Dk, int Hv, int Dv, float eps, void* d_q, void* d_k,
                      void* d_v, void* d_beta, float* d_g, void* d_conv_input) {
+  return gdn_front_from(ctx, d_conv_state, d_qkv, d_cw, d_a, d_b, d_a_log, d_dt_bias, T, K, Hk, Dk, Hv, Dv, eps,
+                        d_q, d_k, d_v, d_beta, d_g, d_conv_input, 0);
+}
+
+}  // extern "C"
+
+// The window's rows before `window_from` are left as they were: a forward that cannot be rewound is
+// followed by one that reads the K - 1 rows from T on, and the other T were a third of the launch's bytes
+// (6621 tokens of 8192 channels 75.4 -> 69.9 us, 700 tokens 12.3 -> 11.9: vector issue is what is left).
+int gdn_front_from(ornith_ctx* ctx, const void* d_conv_state, const void* d_qkv, const void* d_cw,
+                   const void* d_a, const void* d_b, const void* d_a_log, const void* d_dt_bias, int T, int K,
+                   int Hk, int Dk, int Hv, int Dv, float eps, void* d_q, void* d_k, void* d_v, void* d_beta,
+                   float* d_g, void* d_conv_input, int window_from) {
   ORN_REQUIRE(ctx && d_conv_state && d_qkv && d_cw && d_a && d_b && d_a_log && d_dt_bias && d_q &&
                   d_k && d_v && d_beta && d_g && d_conv_input,
               "gdn_front: null argument");
   ORN_REQUIRE(Dk == 128 && Dv == 128, "gdn_front: head dims %d/%d (128 only)", Dk, Dv);
   ORN_REQUIRE(T >= 1 && T <= 65535 && K >= 2 && K <= 8 && Hk >= 1 && Hv >= Hk && Hv % Hk == 0,
               "gdn_front: T=%d K=%d Hk=%d Hv=%d", T, K, Hk, Hv);
+  ORN_REQUIRE(window_from >= 0 && window_from <= T, "gdn_front: window rows from %d of %d", window_from, T);
   ORN_REQUIRE(d_conv_input != d_conv_state, "gdn_front: conv_input must not alias conv_state");
   FrontArgs p{};
   p.conv_state = (const bf16_t*)d_conv_state;
@@ -874,6 +890,7 @@ int ornith_gdn_front(ornith_ctx* ctx, const void* d_conv_state, const void* d_qk
   p.beta = (bf16_t*)d_beta;
   p.g = d_g;
   p.conv_input = (bf16_t*)d_conv_input;
+  p.window_from = window_from;
   p.T = T;
   p.K = K;
   p.Hk = Hk;
@@ -903,6 +920,8 @@ int ornith_gdn_front(ornith_ctx* ctx, const void* d_conv_state, const void* d_qk
   ORN_LAUNCH_CHECK("gdn_front_kernel");
   return ORNITH_OK;
 }
+
+extern "C" {
 
 int ornith_gdn_recurrence(ornith_ctx* ctx, const void* d_q, const void* d_k, const void* d_v,
                           const float* d_g, const void* d_beta, const float* d_state_in, int T,

@@ -10,8 +10,9 @@
 // after a rejected draft moves integers, never bytes:
 //   KV        rows [0, offset) are live; a forward appends at `offset`.
 //   conv      two buffers of K-1+rows rows; a forward reads the live K-1 rows from
-//             one and writes the whole concatenated window into the other; the live
-//             rows afterwards are [keep, keep+K-1) of that window.
+//             one and writes the concatenated window into the other; the live rows
+//             afterwards are [keep, keep+K-1) of that window (past the decode widths a
+//             forward that does not capture writes the K-1 rows from T on only).
 //   state     `max_window` fp32 slots; a captured forward writes the state after
 //             token t into slot t; the live slot afterwards is keep-1.
 #include "model.h"
@@ -234,8 +235,9 @@ static int forward_rows(ornith_model* m, ornith_caches* cc, const uint32_t* d_to
                             g.dt_bias, T, K, Hk, Dk, Hv, Dv, 1e-6f, state_in, lc.state, capture ? 1 : 0,
                             g.norm, s.z, c.rms_norm_eps, lc.conv[1 - cc->conv_cur], s.gated));
       } else {
-        TRY(ornith_gdn_front(ctx, conv_state, s.qkv, g.conv1d, s.a, s.b, g.a_log, g.dt_bias, T, K, Hk,
-                             Dk, Hv, Dv, 1e-6f, s.q, s.k, s.v, s.beta, s.g, lc.conv[1 - cc->conv_cur]));
+        // only a captured forward can be rewound into its window; any other is followed from row T
+        TRY(gdn_front_from(ctx, conv_state, s.qkv, g.conv1d, s.a, s.b, g.a_log, g.dt_bias, T, K, Hk, Dk, Hv, Dv,
+                           1e-6f, s.q, s.k, s.v, s.beta, s.g, lc.conv[1 - cc->conv_cur], capture ? 0 : T));
         TRY(ornith_gdn_recurrence(ctx, s.q, s.k, s.v, s.g, s.beta, state_in, T, Hk, Hv, Dk, Dv, s.y,
                                   lc.state, capture ? 1 : 0));
         TRY(ornith_rms_norm_gated(ctx, s.y, g.norm, s.z, T * Hv, Dv, c.rms_norm_eps, s.gated));

@@ -127,6 +127,11 @@ int ornith_option_kq_iters();      // output rows per wavefront pass of the mat-
 int ornith_option_moe_up_iters();  // rows per wavefront of the fused gate+up kernel; 0 = by shape
 int ornith_option_moe_down_iters();  // column groups per workgroup of the expert down kernel; 0 = by shape
 int ornith_option_gdn_chunked();  // 1: the gated-delta recurrence of calls of 128 rows or more runs chunked on the matrix cores
+// ornith_gdn_front with the rows of d_conv_input before `window_from` (0..T) left unwritten (gdn.hip)
+int gdn_front_from(ornith_ctx* ctx, const void* d_conv_state, const void* d_qkv, const void* d_cw, const void* d_a,
+                   const void* d_b, const void* d_a_log, const void* d_dt_bias, int T, int K, int Hk, int Dk, int Hv,
+                   int Dv, float eps, void* d_q, void* d_k, void* d_v, void* d_beta, float* d_g, void* d_conv_input,
+                   int window_from);
 int ornith_option_fuse_moe_one();  // 1: the MoE block's router, up and down phases in one launch
 int ornith_option_ho_spins();      // polling rounds a hand-off wait inside a launch may take
 

@@ -184,6 +184,42 @@ def test_gdn_step_fused_equals_separate_launches(orn, ctx):
         model.close(); ws.close()
 
 
+@pytest.mark.parametrize("T", [1, 2, 3, 16, 17, 31, 32, 41])
+def test_conv_window_of_a_forward_that_does_not_capture(orn, ctx, T):
+    """Outside the fused step a forward without capture writes the window's last K - 1 rows only: what
+    follows it is the same with caches that held another prompt's rows there before, and (where a
+    capture of T rows is taken) the same as after a captured forward of the same tokens."""
+    import synth
+    s = synth.SynthModel(synth.TINY, seed=22, with_mtp=False)
+    ws = s.upload(orn, ctx)
+    model = orn.TextModel(ctx, ws, s.text_config(orn))
+    model.set_max_rows(64)
+    rng = np.random.default_rng(T)
+    toks = rng.integers(0, s.cfg["vocab_size"], T + 3).astype(np.uint32)
+    other = rng.integers(0, s.cfg["vocab_size"], 48).astype(np.uint32)
+
+    def run(stale, capture=False):
+        c = model.make_cache(128, 16)
+        if stale:
+            for n in (48, 45):  # both buffers
+                model.forward(c, other[:n])
+            c.reset()
+        model.forward(c, toks[:T], capture=capture)
+        out = [model.forward(c, toks[T:T + 1]), model.forward(c, toks[T + 1:])]
+        c.close()
+        return out
+
+    try:
+        orn.set_option("fuse_gdn", 0)
+        want = run(False)
+        for got in [run(True)] + ([run(True, True)] if T <= 16 else []):
+            for x, y in zip(got, want):
+                assert np.array_equal(x, y)
+    finally:
+        orn.set_option("fuse_gdn", 1)
+        model.close(); ws.close()
+
+
 @pytest.mark.parametrize("kind,Os", [(Q4K, (8192, 4096)), (Q6K, (8192, 512, 512)), (Q4K, (40,))])
 def test_norm_inside_projection_launch_equals_separate(orn, ctx, kind, Os):
     """add_rms_norm made inside the launch of the projections that read it (every workgroup
