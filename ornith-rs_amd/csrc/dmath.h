@@ -160,6 +160,34 @@ __device__ __forceinline__ float dm_sigmoid_bf16(float x) {
   const float y = dm_rb(__builtin_amdgcn_rcpf(s * 0x1p-32f) * 0x1p-32f);
   return (x < 0.0f) ? y : dm_rb(1.0f - y);
 }
+// Two at a time with the same bits: the roundings share their instruction.
+__device__ __forceinline__ void dm_rb2(float& a, float& b) {
+  const uint32_t w = dm_f2bf2(a, b);
+  a = dm_bf2f_lo(w);
+  b = dm_bf2f_hi(w);
+}
+__device__ __forceinline__ void dm_sigmoid_bf16x2(float x0, float x1, float& s0, float& s1) {
+  const float x[2] = {x0, x1};
+  float e[2], s[2], y[2], m[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const float a = __builtin_fabsf(x[i]);
+    const float t = a * 1.44269504088896341f;
+    const float lo = dm_fma(a, 1.925963033e-8f, dm_fma(a, 1.44269504088896341f, -t));
+    e[i] = __builtin_amdgcn_exp2f(t);
+    e[i] = dm_fma(e[i] * 0.693147180559945309f, lo, e[i]);
+    e[i] = a > 88.0f ? DM_INF : e[i];
+  }
+  dm_rb2(e[0], e[1]);
+  for (int i = 0; i < 2; ++i) s[i] = 1.0f + e[i];
+  dm_rb2(s[0], s[1]);
+  for (int i = 0; i < 2; ++i) y[i] = __builtin_amdgcn_rcpf(s[i] * 0x1p-32f) * 0x1p-32f;
+  dm_rb2(y[0], y[1]);
+  for (int i = 0; i < 2; ++i) m[i] = 1.0f - y[i];
+  dm_rb2(m[0], m[1]);
+  s0 = x0 < 0.0f ? y[0] : m[0];
+  s1 = x1 < 0.0f ? y[1] : m[1];
+}
 __device__ __forceinline__ float dm_sigmoid_f32(float x) {
   float y = 1.0f / (1.0f + dm_exp(__builtin_fabsf(x)));
   return (x < 0.0f) ? y : 1.0f - y;

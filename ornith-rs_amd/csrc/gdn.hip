@@ -110,9 +110,11 @@ __global__ __launch_bounds__(64) void gdn_front_kernel(FrontArgs p) {
 // one 64-thread workgroup per token and 128 channels. Per token the arithmetic and its order
 // are those of gdn_front_kernel; the decays and betas have grid column D / 128 to themselves (in
 // the wavefront of a conv column they were a second run of exponentials and logarithms behind its
-// own). What bounds it: vector instructions at long prompts (two exponentials, two reciprocals
-// and half a norm a channel pair), the run's serial chain at short ones. So the run is 16 tokens
-// where that still fills the chip and 4 below.
+// own). What bounds it: vector instructions at long prompts (two exponentials and two reciprocals a channel
+// pair), the run's serial chain at short ones. So the run is 16 tokens where that still fills the chip
+// and 4 below, and four tokens share what they can: the butterfly of their norms, one square root and
+// one division, and a pair of channels its roundings (6621 tokens of 8192 channels 73.0 -> 60.6 us, 700
+// tokens 11.9 -> 9.9).
 // grid (D / 128 + 1, ceil(T / RUN)), 64 threads.
 template <int RUN>
 __global__ __launch_bounds__(64) void gdn_front_run_kernel(FrontArgs p) {
@@ -136,10 +138,12 @@ __global__ __launch_bounds__(64) void gdn_front_run_kernel(FrontArgs p) {
     w0[0] = dm_bf2f_lo(a.x); w0[1] = dm_bf2f_hi(a.x); w0[2] = dm_bf2f_lo(a.y); w0[3] = dm_bf2f_hi(a.y);
     w1[0] = dm_bf2f_lo(a.z); w1[1] = dm_bf2f_hi(a.z); w1[2] = dm_bf2f_lo(a.w); w1[3] = dm_bf2f_hi(a.w);
   }
-  // window position j holds conv_state[j] for j < S, qkv[j - S] from there on
+  // window position j holds conv_state[j] for j < S, qkv[j - S] from there on (rows' addresses are the
+  // wavefront's, a lane adds its 32-bit offset)
+  const uint32_t lane4 = 4 * lane;
+  auto at = [&](const bf16_t* row) { return reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(const_cast<bf16_t*>(row)) + lane4); };
   auto input = [&](int j) {
-    const bf16_t* src = (j < S) ? (p.conv_state + (size_t)j * D) : (p.qkv + (size_t)(j - S) * D);
-    return *reinterpret_cast<const uint32_t*>(src + c0);
+    return *at(((j < S) ? (p.conv_state + (size_t)j * D) : (p.qkv + (size_t)(j - S) * D)) + slot * 128);
   };
   uint32_t win[K];
 #pragma unroll
@@ -147,41 +151,67 @@ __global__ __launch_bounds__(64) void gdn_front_run_kernel(FrontArgs p) {
   if (t0 == 0) {
 #pragma unroll
     for (int j = 0; j < S; ++j)
-      if (j >= p.window_from) *reinterpret_cast<uint32_t*>(p.conv_input + (size_t)j * D + c0) = win[j];
+      if (j >= p.window_from) *at(p.conv_input + (size_t)j * D + slot * 128) = win[j];
   }
   const bool is_qk = slot < 2 * p.Hk, is_q = slot < p.Hk;
   const float sc = is_q ? p.q_scale : p.k_scale;
+  const int ostride = is_qk ? key_dim : D - 2 * key_dim;
+  bf16_t* out = is_q ? p.q + slot * 128 : is_qk ? p.k + (slot - p.Hk) * 128 : p.v + (slot - 2 * p.Hk) * 128;
   // the run's inputs are asked for together (one after the other, every token would wait out a
   // memory latency of its own); rows past the end of the call read the last row, unused
   uint32_t in[RUN];
 #pragma unroll
   for (int u = 0; u < RUN; ++u) in[u] = input(min(t0 + u, p.T - 1) + S);
 #pragma unroll
-  for (int u = 0; u < RUN; ++u) {
-    const int t = t0 + u;
-    if (t >= t1) break;
-    win[S] = in[u];  // = qkv[t]
-    float acc0 = 0.f, acc1 = 0.f;
+  for (int u0 = 0; u0 < RUN; u0 += 4) {
+    if (t0 + u0 >= t1) break;
+    float y0[4], y1[4];
 #pragma unroll
-    for (int i = 0; i < K; ++i) {
-      acc0 = dm_fma(dm_bf2f_lo(win[i]), w0[i], acc0);
-      acc1 = dm_fma(dm_bf2f_hi(win[i]), w1[i], acc1);
+    for (int u = 0; u < 4; ++u) {
+      const int t = t0 + u0 + u;
+      win[S] = in[u0 + u];  // = qkv[t]
+      float acc0 = 0.f, acc1 = 0.f;
+#pragma unroll
+      for (int i = 0; i < K; ++i) {
+        acc0 = dm_fma(dm_bf2f_lo(win[i]), w0[i], acc0);
+        acc1 = dm_fma(dm_bf2f_hi(win[i]), w1[i], acc1);
+      }
+      if (t < t1 && S + t >= p.window_from)
+        *at(p.conv_input + (size_t)(S + t) * D + slot * 128) = win[S];
+#pragma unroll
+      for (int i = 0; i < S; ++i) win[i] = win[i + 1];
+      float s0, s1;
+      dm_rb2(acc0, acc1);
+      dm_sigmoid_bf16x2(acc0, acc1, s0, s1);
+      y0[u] = acc0 * s0;
+      y1[u] = acc1 * s1;
     }
-    if (S + t >= p.window_from) *reinterpret_cast<uint32_t*>(p.conv_input + (size_t)(S + t) * D + c0) = win[S];
-#pragma unroll
-    for (int i = 0; i < S; ++i) win[i] = win[i + 1];
-    const float cv0 = dm_rb(acc0), cv1 = dm_rb(acc1);
-    const float y0 = dm_rb(cv0 * dm_sigmoid_bf16(cv0)), y1 = dm_rb(cv1 * dm_sigmoid_bf16(cv1));
     if (is_qk) {
-      float ss = dm_fma(y0, y0, 0.f);
-      ss = dm_fma(y1, y1, ss);
-      const float inv = dm_rsqrt(dm_wave_sum<64>(ss) / 128.0f + p.eps);
-      bf16_t* dst = (is_q ? p.q : p.k) + (size_t)t * key_dim + (is_q ? c0 : c0 - key_dim);
-      const uint32_t n = dm_f2bf2(y0 * inv, y1 * inv);
-      *reinterpret_cast<uint32_t*>(dst) = dm_f2bf2(sc * dm_bf2f_lo(n), sc * dm_bf2f_hi(n));
+      // four tokens' sums share the butterfly and, a row of 16 lanes each, one root and one reciprocal
+      float ss[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        dm_rb2(y0[u], y1[u]);
+        ss[u] = dm_fma(y1[u], y1[u], dm_fma(y0[u], y0[u], 0.f));
+      }
+      const float inv4 = dm_rsqrt(dm_wave_sum4(ss[0], ss[1], ss[2], ss[3]) / 128.0f + p.eps);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int t = t0 + u0 + u;
+        if (t >= t1) break;
+        // dm_wave_sum4 leaves the second sum in the third row, the third in the second
+        const float inv = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(inv4), u == 1 ? 32 : u == 2 ? 16 : 16 * u));
+        float n0 = y0[u] * inv, n1 = y1[u] * inv;
+        dm_rb2(n0, n1);
+        *at(out + (size_t)t * ostride) = dm_f2bf2(sc * n0, sc * n1);
+      }
     } else {
-      bf16_t* dst = p.v + (size_t)t * (D - 2 * key_dim) + (c0 - 2 * key_dim);
-      *reinterpret_cast<uint32_t*>(dst) = dm_f2bf2(y0, y1);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int t = t0 + u0 + u;
+        if (t >= t1) break;
+        *at(out + (size_t)t * ostride) = dm_f2bf2(y0[u], y1[u]);
+      }
     }
   }
 }
@@ -863,7 +893,7 @@ int ornith_gdn_front(ornith_ctx* ctx, const void* d_conv_state, const void* d_qk
 
 // The window's rows before `window_from` are left as they were: a forward that cannot be rewound is
 // followed by one that reads the K - 1 rows from T on, and the other T were a third of the launch's bytes
-// (6621 tokens of 8192 channels 75.4 -> 69.9 us, 700 tokens 12.3 -> 11.9: vector issue is what is left).
+// (6621 tokens of 8192 channels 75.4 -> 69.9 us, 700 tokens 12.3 -> 11.9).
 int gdn_front_from(ornith_ctx* ctx, const void* d_conv_state, const void* d_qkv, const void* d_cw,
                    const void* d_a, const void* d_b, const void* d_a_log, const void* d_dt_bias, int T, int K,
                    int Hk, int Dk, int Hv, int Dv, float eps, void* d_q, void* d_k, void* d_v, void* d_beta,

@@ -13,7 +13,14 @@ __global__ void unary_kernel(int op, const float* in, float* out, int64_t n) {
     case ORNITH_FN_EXP: y = dm_exp(x); break;
     case ORNITH_FN_LOG: y = dm_log(x); break;
     case ORNITH_FN_LOG1P: y = dm_log1p(x); break;
-    case ORNITH_FN_SIGMOID_BF16: y = dm_sigmoid_bf16(dm_rb(x)); break;
+    case ORNITH_FN_SIGMOID_BF16: {  // and its two-at-a-time form: 2, which is no sigmoid, where they differ
+      const float xr = dm_rb(x), n = dm_sigmoid_bf16(-xr);
+      float u, v;
+      y = dm_sigmoid_bf16(xr);
+      dm_sigmoid_bf16x2(xr, -xr, u, v);
+      if (y == y && (u != y || v != n)) y = 2.0f;
+      break;
+    }
     case ORNITH_FN_SIGMOID_F32: y = dm_sigmoid_f32(x); break;
     case ORNITH_FN_RSQRT: y = dm_rsqrt(x); break;
     case ORNITH_FN_RECIP: y = 1.0f / x; break;

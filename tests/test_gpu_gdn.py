@@ -68,10 +68,10 @@ def _inputs(rng, T, Hk, Hv):
                 dt_bias=util.bf16_normal(rng, (Hv,), 0.5))
 
 
-# from 32 rows a call a wavefront takes a run of tokens (same arithmetic): four of them at 32, a ragged 45, 100
-# rows, sixteen where that still fills the chip (1021 rows of these heads, ragged)
-@pytest.mark.parametrize("T,Hk,Hv", [(1, 16, 32), (2, 16, 32), (4, 16, 32), (3, 2, 4), (7, 1, 1), (32, 2, 4), (45, 2, 4),
-                                     (100, 16, 32), (1021, 16, 32)])
+# from 32 rows a call a wavefront takes a run of tokens (same arithmetic): four of them at 32, a ragged 34, 45 and
+# 47, 100 rows, sixteen where that still fills the chip (1021 and 1042 rows of these heads, ragged)
+@pytest.mark.parametrize("T,Hk,Hv", [(1, 16, 32), (2, 16, 32), (4, 16, 32), (3, 2, 4), (7, 1, 1), (32, 2, 4), (34, 2, 4), (45, 2, 4),
+                                     (47, 2, 4), (100, 16, 32), (1021, 16, 32), (1042, 16, 32)])
 def test_gdn_front_bit_exact(orn, ctx, T, Hk, Hv):
     rng = np.random.default_rng(10 + T + Hv)
     i = _inputs(rng, T, Hk, Hv)
