@@ -67,7 +67,7 @@ __global__ __launch_bounds__(4 * ROWS * KSPLIT) __attribute__((amdgpu_waves_per_
   static_assert(KSPLIT == 1 || sizeof(tiles) >= ROWS * HD * 4 + ROWS * 8 * 4, "one set's outputs fit over the tiles");
 
   const int set = KSPLIT == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / NT);
-  const int tid = threadIdx.x - set * NT, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x - set * NT, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l16 = lane & 15, lg = lane >> 4;
   bf16_t(&Ks)[BKV][LDK] = tiles[set].k;
   bf16_t(&Vt)[HD][LDV] = tiles[set].v;
@@ -102,9 +102,10 @@ __global__ __launch_bounds__(4 * ROWS * KSPLIT) __attribute__((amdgpu_waves_per_
 #pragma unroll
   for (int t = 0; t < HD / 16; ++t) o[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   // base-2 exponentials: exp(scale * (s - m)) = exp2(s * c2 - m * c2) with c2 = scale * log2(e)
-  constexpr float kNone = -1e30f;
+  // (the reference point of a row that has seen nothing but masked keys is -inf, and its exponentials are taken from 0: all of them
+  // 0, so that a set's sums of masked keys are none, and a visible score that is no number stays one in the sums)
   const float c2 = p.scale * 1.44269504088896340736f;
-  float m_i = kNone, l_i = 0.f;  // l_i: this lane's share of the row sum
+  float m_i = -DM_INF, l_i = 0.f;  // l_i: this lane's share of the row sum
 
   const bf16_t* kbase = p.k_cache + (size_t)hk * p.cap * HD;
   const bf16_t* vbase = p.v_cache + (size_t)hk * p.cap * HD;
@@ -135,12 +136,8 @@ __global__ __launch_bounds__(4 * ROWS * KSPLIT) __attribute__((amdgpu_waves_per_
       vr[i] = *reinterpret_cast<const u32x4_t*>(vbase + (size_t)vkey * HD + 8 * vc8);
     }
   };
-  // (a set that has no block left takes one past the end, which is masked for every row)
-  fetch_k(set);
-  fetch_v(set);
-  for (int kb = set; kb - set < n_kb; kb += KSPLIT) {
-    FA_MARK(0);
-    // ---- K block as is, V block transposed
+  // K block as is, V block transposed
+  auto stage = [&]() {
 #pragma unroll
     for (int i = 0; i < NPC; ++i)
       *reinterpret_cast<u32x4_t*>(&Ks[(tid >> 5) + NT / 32 * i][8 * (tid & 31)]) = kr[i];
@@ -155,6 +152,19 @@ __global__ __launch_bounds__(4 * ROWS * KSPLIT) __attribute__((amdgpu_waves_per_
       *reinterpret_cast<u32x2_t*>(&Vt[8 * vc8 + ch][vcol]) = u32x2_t{col[0], col[1]};
       if constexpr (NPC == 8) *reinterpret_cast<u32x2_t*>(&Vt[8 * vc8 + ch][vcol + 8]) = u32x2_t{col[2], col[3]};
     }
+  };
+  // A block that lies past all of a wavefront's rows (a set's turn past the last one, the upper half of a 128-row workgroup's last two)
+  // is staged for the others and left out: its probabilities would be 0, but 0 times what a later token's value row holds need not be.
+  // (With one set of 64 rows such a block has some rows' keys, and asking costs what is there, us: 150 / 200 / 256 tokens 16.9 / 18.6 / 19.5
+  // without, 17.6 / 19.8 / 20.6 with; the other forms level.)
+  constexpr bool kLeaves = ROWS * KSPLIT > 64;
+  const int last_pos = p.offset + r0 + 15;
+  fetch_k(set);
+  fetch_v(set);
+  int kb = set;
+  for (; kb - set < n_kb && (!kLeaves || kb * BKV <= last_pos); kb += KSPLIT) {
+    FA_MARK(0);
+    stage();
     FA_MARK(1);
     __syncthreads();
     FA_MARK(2);
@@ -192,12 +202,12 @@ __global__ __launch_bounds__(4 * ROWS * KSPLIT) __attribute__((amdgpu_waves_per_
     {
       const int pos = p.offset + r0 + l16;
       const bool diag = kb * BKV + BKV - 1 > p.offset + r0;
-      float mx = kNone;
+      float mx = -DM_INF;
 #pragma unroll
       for (int nt = 0; nt < BKV / 16; ++nt)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          if (diag && kb * BKV + nt * 16 + 4 * lg + r > pos) st[nt][r] = kNone;
+          if (diag && kb * BKV + nt * 16 + 4 * lg + r > pos) st[nt][r] = -DM_INF;
           mx = fmaxf(mx, st[nt][r]);
         }
       mx = fmaxf(mx, dm_xor_lane<16>(mx));
@@ -212,7 +222,7 @@ __global__ __launch_bounds__(4 * ROWS * KSPLIT) __attribute__((amdgpu_waves_per_
       const float m_new = grow ? mx : m_i;
       const float alpha = grow ? __builtin_amdgcn_exp2f((m_i - m_new) * c2) : 1.f;
       m_i = m_new;
-      const float mc = -(m_new * c2);
+      const float mc = m_new > -DM_INF ? -(m_new * c2) : 0.f;
       float rs = 0.f;
 #pragma unroll
       for (int nt = 0; nt < BKV / 16; ++nt)
@@ -266,8 +276,15 @@ __global__ __launch_bounds__(4 * ROWS * KSPLIT) __attribute__((amdgpu_waves_per_
     __syncthreads();
     FA_MARK(7);
   }
+  for (; kLeaves && kb - set < n_kb; kb += KSPLIT) {
+    stage();
+    __syncthreads();
+    fetch_k(kb + KSPLIT);
+    fetch_v(kb + KSPLIT);
+    __syncthreads();
+  }
 
-  // ---- the second set's sums and outputs go to the first, both brought to the greater of the two reference points 
+  // ---- the second set's sums and outputs go to the first, both brought to the greater of the two reference points
   if constexpr (KSPLIT == 2) {
     f32x4_t* const there = reinterpret_cast<f32x4_t*>(&tiles[0]) + (wave * (HD / 16)) * 64 + lane;
     float2* const ml = reinterpret_cast<float2*>(reinterpret_cast<f32x4_t*>(&tiles[0]) + ROWS / 16 * (HD / 16) * 64) + wave * 64 + lane;
@@ -280,14 +297,13 @@ __global__ __launch_bounds__(4 * ROWS * KSPLIT) __attribute__((amdgpu_waves_per_
     if (set == 1) return;
     const float2 other = *ml;
     const float m = fmaxf(m_i, other.x);
-    const bool any = other.x > kNone;  // (the other set's sums of masked keys are no numbers to go on with)
     const float a = __builtin_amdgcn_exp2f((m_i - m) * c2), b = __builtin_amdgcn_exp2f((other.x - m) * c2);
-    l_i = l_i * a + (any ? other.y * b : 0.f);
+    l_i = l_i * a + other.y * b;
 #pragma unroll
     for (int t = 0; t < HD / 16; ++t) {
       const f32x4_t v = there[t * 64];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) o[t][r] = o[t][r] * a + (any ? v[r] * b : 0.f);
+      for (int r = 0; r < 4; ++r) o[t][r] = o[t][r] * a + v[r] * b;
     }
   }
   // ---- normalise, gate, store: the lane's row, channels 16*t + 4*lg .. + 4

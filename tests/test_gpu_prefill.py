@@ -282,6 +282,65 @@ def test_prefill_attention_close_to_exact_kernel(orn, ctx, T, Hq, Hkv, cap, offs
     for b in (dq, dk, dv, dg, dout): b.free()
 
 
+@pytest.mark.parametrize("what", ["nan key", "infinite key", "nan value"])
+@pytest.mark.parametrize("T,Hq,Hkv,offset,at", [
+    # two sets of wavefronts: the first key that a row's second set sees (64 of row 64), its last block's, an odd number of blocks
+    (300, 16, 2, 0, (64, 200)), (300, 16, 2, 0, (0, 255)), (130, 4, 2, 300, (350, 425)), (64, 4, 2, 325, (68, 384)),
+    # one set; 128-row workgroups
+    (200, 4, 2, 37, (63, 170)), (390, 64, 2, 20, (150, 340))])
+def test_prefill_attention_non_finite_operands(orn, ctx, T, Hq, Hkv, offset, at, what):
+    """A key or value row that holds NaN, or a key with one channel at -inf (scores of -inf and +inf, by the query's sign): the rows
+    that see it come out as float64 softmax attention over their visible keys says, NaN for NaN and the others within 1 % relative
+    L2 (the bound of finite operands); the rows before it keep the bits they have without it, as far as no row of their
+    sixteen (of their 64, up to four key blocks) sees any of its block of 64 keys (a masked value there meets a probability of 0 on
+    the matrix cores, and 0 times NaN is NaN)."""
+    hd, cap = 256, 512
+    rng = np.random.default_rng(T + Hq + offset)
+    q = util.bf16_normal(rng, (T, Hq, hd)); qg = util.bf16_normal(rng, (T, Hq, 2 * hd))
+    kc = np.full((Hkv, cap, hd), 0x7FC0, np.uint16); vc = kc.copy()
+    n = offset + T
+    kc[:, :n] = util.bf16_normal(rng, (Hkv, n, hd)); vc[:, :n] = util.bf16_normal(rng, (Hkv, n, hd))
+
+    def run():
+        bufs = [ctx.to_device(x) for x in (q, kc, vc, qg)] + [ctx.alloc(T * Hq * hd * 2)]
+        ctx.sdpa_decode_gated(*bufs[:4], T, Hq, Hkv, hd, offset, cap, hd ** -0.5, bufs[4])
+        got = bufs[4].download(np.uint16, (T, Hq, hd))
+        for b in bufs: b.free()
+        return got
+
+    clean = run()
+    for g, j in enumerate(at):
+        if what == "infinite key": kc[g, j, 7] = 0xFF80
+        else: (kc if what == "nan key" else vc)[g, j] = 0x7FC0
+    got = run()
+    pos = offset + np.arange(T)
+    gf = util.bf16_to_f32(got).astype(np.float64)
+    qf = util.bf16_to_f32(q).astype(np.float64)
+    gate = 1 / (1 + np.exp(-util.bf16_to_f32(qg[..., hd:]).astype(np.float64)))
+    per = Hq // Hkv
+    for g, j in enumerate(at):
+        heads = slice(g * per, (g + 1) * per)
+        share = 64 if n <= 256 else 16
+        last = pos - (pos - offset) % share + share - 1
+        apart = (pos < j) & (j // 64 * 64 > last) if what == "nan value" else pos < j
+        assert np.array_equal(got[apart, heads], clean[apart, heads]), (g, j)
+        K64, V64 = util.bf16_to_f32(kc[g, :n]).astype(np.float64), util.bf16_to_f32(vc[g, :n]).astype(np.float64)
+        rows = np.nonzero(pos >= j)[0]
+        with np.errstate(invalid="ignore"):
+            for h in range(heads.start, heads.stop):
+                sc = (qf[rows, h] @ K64.T) * hd ** -0.5
+                sc[np.arange(n)[None, :] > pos[rows, None]] = -np.inf
+                pr = np.exp(sc - sc.max(axis=1, keepdims=True))
+                v = V64.copy()
+                if what == "nan value": v[j] = 0
+                want = (pr @ v) / pr.sum(axis=1, keepdims=True) * gate[rows, h]
+                if what == "nan value": want[:] = np.nan
+                bad = np.isnan(want).any(axis=1)
+                assert np.isnan(gf[rows[bad], h]).all(), (g, j, h)
+                rel = np.linalg.norm(gf[rows[~bad], h] - want[~bad], axis=1) / np.linalg.norm(want[~bad], axis=1)
+                assert np.all(rel < 0.01), (g, j, h, float(rel.max()))
+
+
 @pytest.mark.parametrize("T,offset", [(4096, 4096), (6621, 0)])
 def test_prefill_attention_at_the_long_context_sizes(orn, ctx, T, offset):
     """The sampled configuration's sizes: a 4096-row prompt chunk behind 4096 cached rows, and
