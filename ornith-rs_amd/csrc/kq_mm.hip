@@ -52,6 +52,8 @@ struct MmArgs {
   const uint32_t* tile_count;  // [tiles] pairs in the tile (<= BM)
   const uint32_t* n_tiles;     // device scalar
   int sub;                     // workgroups a plan tile takes (plan tiles may be taller than the kernel's)
+  const uint32_t* expert_at;   // register form over a plan of lower tiles: [E] where an expert's pairs begin; else null
+  int E;
   int vec;                     // rows of y can be stored 16 bytes at a time
   // further matrices of the same kind and K over the same activations (plain form): the
   // workgroups from column block bx0 on belong to segment i
@@ -988,6 +990,14 @@ __device__ __forceinline__ void reg_body(const MmArgs& a) {
     const uint32_t e = a.tile_expert[tile], st = a.tile_start[tile] + part * ROWS;
     rows_here = min((int)a.tile_count[tile] - (int)(part * ROWS), ROWS);
     if (rows_here <= 0) return;
+    if constexpr (ROWS == RM) {
+      // a plan of lower tiles (16, 32 or 64 rows): the first of as many as ROWS holds works on the pairs of them all
+      if (a.expert_at) {
+        const uint32_t at = a.expert_at[e], end = (int)e + 1 < a.E ? a.expert_at[e + 1] : (uint32_t)a.M;
+        if ((st - at) % (uint32_t)ROWS != 0) return;
+        rows_here = min((int)(end - st), ROWS);
+      }
+    }
     wrow0 = (int64_t)e * a.O;
     for (int r = tid; r < ROWS; r += 256) {
       const uint32_t p = r < rows_here ? a.pair[st + r] : 0u;
@@ -1079,7 +1089,7 @@ __device__ __forceinline__ uint32_t shared_tiles(int shared_rows, int pairs, int
 __global__ __launch_bounds__(1024) void moe_sort_pairs_kernel(const uint32_t* inds, int pairs, int E,
                                                               int bm, int shared_rows, uint32_t* pair, uint32_t* tile_expert,
                                                               uint32_t* tile_start, uint32_t* tile_count,
-                                                              uint32_t* n_tiles) {
+                                                              uint32_t* n_tiles, uint32_t* expert_at) {
   __shared__ uint32_t cnt[1024], fill[1024];
   __shared__ unsigned long long scan[2][1024];  // pairs before an expert (low 40 bits) and tiles before it
   __shared__ uint32_t t_expert[kSortTilesMax], t_start[kSortTilesMax], t_count[kSortTilesMax];
@@ -1118,6 +1128,7 @@ __global__ __launch_bounds__(1024) void moe_sort_pairs_kernel(const uint32_t* in
   if (tid == 0) *n_tiles = total_tiles;
   __syncthreads();
   scan[0][tid] = start;  // (reused: where an expert's run of pairs begins)
+  if (tid < E) expert_at[tid] = start;
   __syncthreads();
   // placement: a pair takes the next free place of its expert. The order inside an expert's
   // run depends on the scheduling of the atomics, the results do not: every output row is one
@@ -1169,7 +1180,7 @@ __global__ __launch_bounds__(256) void moe_sort_count_kernel(const uint32_t* ind
   for (int e = threadIdx.x; e < E; e += 256) part_cnt[blockIdx.x * E + e] = cnt[e];
 }
 
-// part_cnt [parts, E] in: pairs of expert e in slice b; out: where slice b's pairs of expert e begin
+// part_cnt [parts, E] in: pairs of expert e in slice b; out: where slice b's pairs of expert e begin (slice 0: the expert's)
 __global__ __launch_bounds__(1024) void moe_sort_plan_kernel(int pairs, int E, int bm, int shared_rows, uint32_t* part_cnt,
                                                              uint32_t* pair, uint32_t* tile_expert,
                                                              uint32_t* tile_start, uint32_t* tile_count,
@@ -1263,6 +1274,7 @@ int moe_plan(ornith_ctx* ctx, const uint32_t* d_inds, int pairs, int E, int rows
   p.tile_count = pc.take<uint32_t>(p.tiles_max);
   p.n_tiles = pc.take<uint32_t>(1);
   uint32_t* parts = pc.take<uint32_t>((size_t)kSortParts * E);
+  p.expert_at = parts;
   if (build && pairs >= 8192) {
     hipLaunchKernelGGL(moe_sort_count_kernel, dim3(kSortParts), dim3(256), 0, ctx->stream, d_inds, pairs, E, parts);
     hipLaunchKernelGGL(moe_sort_plan_kernel, dim3(1), dim3(1024), 0, ctx->stream, pairs, E, rows, shared_rows, parts, p.pair,
@@ -1271,7 +1283,7 @@ int moe_plan(ornith_ctx* ctx, const uint32_t* d_inds, int pairs, int E, int rows
     ORN_LAUNCH_CHECK("moe_sort_*_kernel");
   } else if (build) {
     hipLaunchKernelGGL(moe_sort_pairs_kernel, dim3(1), dim3(1024), 0, ctx->stream, d_inds, pairs, E, rows, shared_rows,
-                       p.pair, p.tile_expert, p.tile_start, p.tile_count, p.n_tiles);
+                       p.pair, p.tile_expert, p.tile_start, p.tile_count, p.n_tiles, parts);
     ORN_LAUNCH_CHECK("moe_sort_pairs_kernel");
   }
   *out = p;
@@ -1354,6 +1366,12 @@ int ornith_kq_matmul(ornith_ctx* ctx, const ornith_kmatrix* w, const void* d_x, 
   return ornith_kq_matmul_multi(ctx, &w, 1, d_x, M, &d_y);
 }
 
+// Pairs an expert from which a matrix that the few-row kernels don't take is worked on in the register form. us, LDS form / register
+// form: 256 experts of 512 x 5120, Q4_K, 48 / 64 / 79 pairs an expert 243 / 190, 337 / 205, 431 / 223; 128 of 1024 x 4608, Q6_K, 250 / 190,
+// 341 / 206, 434 / 223; where the chip is filled once (64 of 1024 x 5120, Q4_K) 93 / 77, 128 / 86, 176 / 92. (64 of 512 x 7168, Q6_K, half
+// filled: 93 / 103, 117 / 109, 127 / 118. 64 of 514 x 1280: 25.8 / 26.2, 27.5 / 29.1, 35.2 / 32.1.)
+constexpr int kRegPairs = 48;
+
 // gather plan: expert-sorted pairs and the tile list, in caller-provided device memory
 // (ornith_kq_gather_plan_bytes(pairs, E) bytes)
 size_t ornith_kq_gather_plan_bytes(int pairs, int E) { return moe_plan_bytes(pairs, E, 16, 0); }
@@ -1378,8 +1396,9 @@ int ornith_kq_gather_matmul(ornith_ctx* ctx, const ornith_kmatrix* w, const void
   const bool narrow = pairs < nmm::kNarrowPairs * w->E;
   const bool tall = ornith_option_gemm_reg() && !narrow;
   const int tile_rows = narrow ? nmm::tile_rows(pairs, w->E) : tall ? RM : avg >= 96 ? 128 : 64;
-  // The kernel for this matrix. Few rows an expert: the few-row kernels (mm_narrow.h). Tall plans
-  // take the register form when its 32-bit offsets reach:
+  // The kernel for this matrix. Few rows an expert: the few-row kernels (mm_narrow.h). Tall plans, and from 48 rows an
+  // expert on the matrices that the few-row kernels don't take (K > 4096, rows whose scales are no whole 16-byte
+  // pieces; their 64-row tiles are worked on three at a time), take the register form when its 32-bit offsets reach:
   // for K >= 1024 a workgroup a plan tile (one a compute unit), for fewer K slabs 64-row
   // workgroups, two a compute unit (a workgroup's way in and out, which weighs more the fewer
   // slabs there are, then runs beside the other's main loop; the weights still bypass LDS, which
@@ -1388,12 +1407,14 @@ int ornith_kq_gather_matmul(ornith_ctx* ctx, const ornith_kmatrix* w, const void
   // split over several of them.
   const size_t x_rows = (size_t)(is_up ? pairs / top_k : pairs), x_bytes = x_rows * w->K * 2;
   const size_t q_bytes = (size_t)w->E * w->O * (w->K / 256) * (w->kind == ORNITH_Q4K ? 128 : 192);
-  const bool reg = tall && w->K >= 1024 && x_bytes < (size_t(1) << 32) && q_bytes < (size_t(1) << 32);
+  const bool few = narrow && nmm::experts_ok(w, d_x, x_rows, d_y);
+  const bool low = narrow && !few && pairs >= kRegPairs * w->E && ornith_option_gemm_reg();
+  const bool reg = (tall || low) && w->K >= 1024 && x_bytes < (size_t(1) << 32) && q_bytes < (size_t(1) << 32);
   const int lds_rows = (avg >= 96 && w->K >= 1024) ? 128 : 64;
   nmm::Plan pl;
   rc = moe_plan(ctx, d_inds, pairs, w->E, tile_rows, 0, d_plan, rebuild_plan != 0, &pl);
   if (rc) return rc;
-  if (narrow && nmm::experts_ok(w, d_x, x_rows, d_y)) return nmm::gathered(ctx, w, nullptr, d_x, pairs, is_up ? top_k : 1, pl, d_y);
+  if (few) return nmm::gathered(ctx, w, nullptr, d_x, pairs, is_up ? top_k : 1, pl, d_y);
   const size_t tiles_max = pl.tiles_max;
   MmArgs a{};
   a.qs = (const uint8_t*)w->d_qs;
@@ -1413,6 +1434,8 @@ int ornith_kq_gather_matmul(ornith_ctx* ctx, const ornith_kmatrix* w, const void
   a.n_tiles = pl.n_tiles;
   if (reg) {
     a.sub = 1;
+    if (low) a.expert_at = pl.expert_at;
+    a.E = w->E;
     const dim3 rgrid((w->O + RN - 1) / RN, (unsigned)tiles_max);
     if (w->kind == ORNITH_Q4K)
       hipLaunchKernelGGL((kq_mm_reg_kernel<ORNITH_Q4K, true>), rgrid, dim3(256), 0, ctx->stream, a);

@@ -32,6 +32,7 @@ constexpr int kNarrowPairs = 80;
 // an expert-sorted pair list in device memory, tiles of up to `rows` pairs
 struct Plan {
   uint32_t *pair, *tile_expert, *tile_start, *tile_count, *n_tiles;
+  uint32_t* expert_at;  // [E] where an expert's pairs begin
   size_t tiles_max;
   int rows;
 };

@@ -120,7 +120,11 @@ def ctx_off(buf, nbytes):
                                              # hundred rows an expert and one crowded expert: tall tiles, the
                                              # register form for K >= 1024 and its split over shorter workgroups
                                              (Q4K, 32, 512, 2048, 1100, 8), (Q6K, 32, 256, 1024, 1100, 8),
-                                             (Q6K, 32, 1024, 512, 1100, 8)])
+                                             (Q6K, 32, 1024, 512, 1100, 8),
+                                             # 75 to 79 rows an expert of matrices that the few-row kernels don't take (K > 4096; scales in
+                                             # no 16-byte pieces): low plan tiles, three a workgroup in the register form, and the LDS form
+                                             (Q4K, 8, 264, 4352, 316, 2), (Q6K, 8, 130, 4352, 316, 2), (Q4K, 128, 40, 4352, 1200, 8),
+                                             (Q6K, 16, 257, 1280, 300, 4), (Q6K, 16, 130, 768, 300, 4)])
 def test_kq_gather_matmul_vs_float64(orn, ctx, kind, E, O, K, T, k):
     rng = np.random.default_rng(E + O + K + T)
     t = util.make_kq(kind, rng, E, O, K)
