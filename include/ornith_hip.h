@@ -403,8 +403,8 @@ ORNITH_API int ornith_sdpa_decode_gated(ornith_ctx* ctx, const void* d_q_rot, co
  * runs them (src/model/qwen3_5.rs:430-474), host-side offset: the same results and the same
  * cache contents; at decode widths (T <= 8, in the forms with one workgroup a block and head and with
  * one for eight heads) one launch does both -- every workgroup makes its query row and the call's new
- * key rows itself, and the caches are written as a side effect. d_q_rot is only written when
- * the prep runs as its own launch. */
+ * key rows itself, and the caches are written as a side effect. d_q_rot is written by the form
+ * for eight heads and when the prep runs as its own launch, not by the form for one. */
 ORNITH_API int ornith_attn_decode(ornith_ctx* ctx, const void* d_qg, const void* d_kx, const void* d_vx,
                                   const void* d_q_norm_w, const void* d_k_norm_w, int T, int Hq, int Hkv,
                                   int hd, int rope_dims, float eps, const float* d_cos, const float* d_sin,

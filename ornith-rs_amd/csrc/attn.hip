@@ -667,7 +667,8 @@ __global__ __launch_bounds__(512, 4) void sdpa_partial_many_kernel(SdpaArgs p) {
 // that makes is not stored.)
 //
 // PREP: attn_prep's work too: wavefront w makes query head w and the key row of the call's w-th new position in the block, new value
-// rows are read from the raw projection, and the workgroup of a KV group's first heads appends its row. Static offset, T <= 8.
+// rows are read from the raw projection, and of the workgroups of a row's last block each stores its query heads, the one of a KV
+// group's first heads also the row's key and value. Static offset, T <= 8.
 // grid sdpa_die_grid<kEightHeads>, 512 threads
 constexpr int kEightHeads = 8;
 template <int HD>
@@ -763,7 +764,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   using S1 = std::integral_constant<int, 1>;
   using S2 = std::integral_constant<int, 2>;
   using S3 = std::integral_constant<int, 3>;
-  uint32_t krow[PER / 2];
+  uint32_t qrow[PER / 2], krow[PER / 2];
   auto heads = [&](auto path) {  // (the paths' tags keep the compiler from doing it ahead of the requests, where the paths agree)
     if constexpr (PREP) {
       float x[PER];
@@ -771,7 +772,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       for (int i = 0; i < PER / 2; ++i) asm volatile("; rows on path %4" : "+v"(pgq.x[i]), "+v"(pgk.x[i]), "+v"(pgq.w[i]), "+v"(pgk.w[i]) : "n"(decltype(path)::value));
       prep_finish<PER>(pgq, true, pq.half, pq.eps, lane, x);
 #pragma unroll
-      for (int i = 0; i < PER; ++i) qsh[wave * HD + lane * PER + i] = p.scale * dm_bf2f(dm_f2bf(x[i]));  // q_rot is bf16
+      for (int e = 0; e < PER; e += 2) {  // q_rot is bf16
+        qrow[e / 2] = dm_f2bf2(x[e], x[e + 1]);
+        qsh[wave * HD + lane * PER + e] = p.scale * dm_bf2f_lo(qrow[e / 2]);
+        qsh[wave * HD + lane * PER + e + 1] = p.scale * dm_bf2f_hi(qrow[e / 2]);
+      }
       if (has_k) {
         prep_finish<PER>(pgk, true, pq.half, pq.eps, lane, x);
 #pragma unroll
@@ -860,7 +865,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
     for (int n = 0; n < NQ; ++n) sum[n] = s == 0 ? chain[n] : sum[n] + chain[n];
   }
-  // PREP: the values of the call's own positions up to this row's come from the projection, and this row goes to the cache
+  // PREP: the values of the call's own positions up to this row's come from the projection; this row goes to the cache, its
+  // query heads to q_rot
   if constexpr (PREP) {
     if (holds && nold < nvalid) {
       const __amdgpu_buffer_rsrc_t xbuf = dm_buffer(pq.vx + (size_t)hk * HD, (uint32_t)(t * p.Hkv + 1) * (HD * 2));
@@ -871,6 +877,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         if (r >= nold && r < nvalid) vreg[u >> 4][u & 15] = load_row(xbuf, (x0 + r) * (p.Hkv * HD * 2));
       }
     }
+    if (b == last / ATT_KB && wave < nh)
+      __builtin_memcpy(pq.q_rot + ((size_t)t * p.Hq + hq0 + wave) * HD + lane * PER, qrow, sizeof qrow);  // (as the caller has aligned it)
     if (hq0 == hk * (p.Hq / p.Hkv) && has_k && kpos == last) {
 #pragma unroll
       for (int e = 0; e < PER / 2; ++e) {

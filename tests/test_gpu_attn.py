@@ -72,10 +72,14 @@ def test_attention_bit_exact(orn, ctx, T, Hq, Hkv, hd, cap, offset):
     # first otherwise; with the fold switched off it is always two): same output, same caches
     for fold in (1, 0):
         orn.set_option("fuse_attn_prep", fold)
-        dkc.upload(kc); dvc.upload(vc); dout.zero()
+        dkc.upload(kc); dvc.upload(vc); dout.zero(); dq.zero()
         ctx.attn_decode(*d, T, Hq, Hkv, hd, rd, 1e-6, dc, ds, cap, offset, cap, hd ** -0.5, dq, dkc, dvc, dout)
         assert np.array_equal(dout.download(np.uint16, want.shape), want), ("attn_decode", fold)
         assert np.array_equal(dkc.download(np.uint16, kc.shape), wkc) and np.array_equal(dvc.download(np.uint16, vc.shape), wvc), fold
+        # the rotated queries: of every form but the folded one of a head a workgroup (as many as are one round of a 256-unit device)
+        blocks = (offset + T - 1) // 256 + 1
+        if not fold or T > 8 or blocks * Hq * T > (512 if blocks == 1 else 256):
+            assert np.array_equal(dq.download(np.uint16, wq.shape), wq), ("rotated queries", fold)
     orn.set_option("fuse_attn_prep", 1)
     for b in d + [dkc, dvc, dq, dout, dc, ds]: b.free()
 
