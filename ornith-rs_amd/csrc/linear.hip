@@ -392,7 +392,7 @@ static int linear_matmul_multi(ornith_ctx* ctx, const ornith_linear* const* ws, 
     // (a single one, too: in a launch of the wide kernels it would have other sums than alone)
     const bool shared = nf >= 1 && nmm::plain_ok(few, nf, d_x, M, yf);
     if (shared || (nd && nd < n)) {
-      const bool riding = shared && nmm::riders_ok(dense, nd, few[0]->K);
+      const bool riding = shared && nmm::riders_ok(ctx, dense, nd, few[0]->K, M);
       int rc = ORNITH_OK;
       if (shared) rc = nmm::plain(ctx, few, nf, d_x, M, yf, dense, riding ? nd : 0, yd);
       else

@@ -39,8 +39,8 @@ struct Plan {
 
 // up to four matrices of one K over the same activations
 bool plain_ok(const ornith_linear* const* ws, int n, const void* d_x, int M, void* const* d_ys);
-// ... with up to two dense bf16 matrices over the same rows beside them (riders_ok: K too)
-bool riders_ok(const ornith_linear* const* ws, int n, int K);
+// ... with up to two dense bf16 matrices over the same rows beside them (riders_ok: K and the size too)
+bool riders_ok(ornith_ctx* ctx, const ornith_linear* const* ws, int n, int K, int M);
 int plain(ornith_ctx* ctx, const ornith_linear* const* ws, int n, const void* d_x, int M, void* const* d_ys,
           const ornith_linear* const* riders = nullptr, int n_riders = 0, void* const* d_yr = nullptr);
 // rows of a plan tile

@@ -140,10 +140,20 @@ int launch_split(ornith_ctx* ctx, Args& a) {
 }
 }  // namespace
 
-bool riders_ok(const ornith_linear* const* ws, int n, int K) {
-  for (int i = 0; i < n; ++i)
+// A riding tile is a workgroup of one 16 x 16 tile, which asks for 3.2 times what a tile of the dense launch's four-tile form does: riding
+// saves that launch (4 to 6 us) and loses on large products. us, beside 4096 x 2048 of Q4_K, a launch of its own / riding (tiles): up to
+// 192 rows, where the launch of its own is a chain whatever its width, 1024 columns, 128 rows 20.0 / 15.5 (512), 192 rows 25.4 / 21.4 (768); 2048
+// columns, 96 rows 23.5 / 21.2 (768), 192 36.2 / 31.8 (1536); 4096 columns, 128 rows 40.5 / 37.8 (2048), 192 48.6 / 54.1 (3072). More rows: 256
+// columns, 448 rows 28.2 / 24.9 (448), 600 36.8 / 31.3 (608), 900 38.1 / 42.4 (912); 512 columns, 320 rows 30.4 / 31.0 (640), 448 30.6 / 34.7 (896);
+// 2048 columns, 320 rows 50.4 / 52.6, 900 107 / 128 (7296). Over 4-bit affine weights alike; the a / b heads (64 columns) beside 12288 x 2048 of
+// them: 600 rows 68.5 / 65.4 (152), 2500 242 / 237 (628), 4096 382.1 / 382.2 (1024), 8192 755 / 757 (2048).
+bool riders_ok(ornith_ctx* ctx, const ornith_linear* const* ws, int n, int K, int M) {
+  long tiles = 0;
+  for (int i = 0; i < n; ++i) {
     if (ws[i]->mode != ORNITH_LIN_DENSE || !ws[i]->d_w || ws[i]->K != K || ws[i]->O < 1 || ((uintptr_t)ws[i]->d_w & 15) != 0) return false;
-  return n >= 1 && n <= 2 && K % 2048 == 0;
+    tiles += (ws[i]->O + 15) / 16;
+  }
+  return n >= 1 && n <= 2 && K % 2048 == 0 && 2 * tiles * ((M + 15) / 16) <= (M <= 192 ? 16L : 5L) * ctx->compute_units;
 }
 
 int plain(ornith_ctx* ctx, const ornith_linear* const* ws, int n, const void* d_x, int M, void* const* d_ys,

@@ -60,10 +60,12 @@ def test_few_row_matmul_vs_float64(orn, ctx, fmt, O, K, M):
 @pytest.mark.parametrize("fmt", ["q4k", "affine4", "affine8"])
 @pytest.mark.parametrize("O,dense,K,M", [(512, (32, 32), 2048, 32), (4096, (1, 40), 2048, 51), (2056, (32,), 2048, 193),
                                          (4096, (32, 17), 2048, 500), (264, (16, 1), 4096, 77), (512, (32, 32), 1024, 40),
-                                         (4096, (32, 32), 2048, 1300)])
+                                         (4096, (32, 32), 2048, 1300),
+                                         # a dense matrix beside them that does not ride: too large (192 rows and fewer, more, long prompts)
+                                         (512, (4096,), 2048, 192), (512, (512, 40), 2048, 300), (264, (48, 32), 2048, 2100)])
 def test_dense_matrices_ride_along_with_a_few_row_gemm(orn, ctx, fmt, O, dense, K, M):
-    """linear_matmul_multi of two quantized matrices and one or two narrow dense ones at prompt widths: one launch where K
-    allows (in the form with K split over wavefronts and in the one with columns owned; rows and columns ragged), and
+    """linear_matmul_multi of two quantized matrices and one or two dense ones at prompt widths: one launch where K and the dense ones'
+    size allow (in the form with K split over wavefronts and in the one with columns owned; rows and columns ragged), and
     every output is the matrix's own launch bit for bit, past every output nothing is written"""
     rng = np.random.default_rng(O + K + M)
     make = {"q4k": lambda o: util.HostLinear.kq(rng, Q4K, o, K), "affine4": lambda o: util.HostLinear.affine4(rng, o, K),
