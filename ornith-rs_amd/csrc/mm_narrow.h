@@ -36,10 +36,12 @@
 // 256 x 2048 Q6_K 28.6 -> 6.6 -> 5.4; the experts, gate + up + swiglu / down (the shared expert included): a 51-token prompt
 // 104 / 49 -> 53 / 36 with K split -> 47 / 38 with columns owned, a 700-token one 156 / 76 -> 122 / 81 -> 90 / 69, over 4-bit
 // affine weights at 600 tokens 109 / 62 -> 98 / 51; a 600-token prompt over 4-bit affine weights as a whole 461 ms
-// (mat-vecs, row by row) -> 15.9 -> 14.8 ms.
+// (mat-vecs, row by row) -> 15.9 -> 13.2 ms.
 //
-// The order of the sums depends on K alone, never on M, O or the launch's other matrices: plain, 256-wide blocks,
-// wavefront ks takes blocks ks, ks + KS, ... and the partial sums are added in one order; expert forms, all blocks in turn.
+// There are two orders of the sums, both by K alone: with K split over the wavefronts, 256-wide blocks, wavefront ks takes blocks ks,
+// ks + KS, ... and the partial sums are added in one order; with columns owned (expert forms and kTall), all blocks in turn.
+// Which one a plain matrix takes hangs on its own rows, columns and format (tall() in mm_narrow_kq.hip), never on the launch's
+// other matrices or its tile.
 //
 // Weight formats:
 //   Q4_K, Q6_K        dequantized with kquant::dequantize's arithmetic and rounded to bf16, as in
