@@ -1224,8 +1224,11 @@ static int sdpa_decode(ornith_ctx* ctx, const void* d_q_rot, const void* d_k_cac
   // 22.6 / 19.0; eight at 2100 20.6 / 18.0). A second round of eights costs what it saved (four rows at 9000 / 12000 keys
   // 29.0 / 32.3 and 29.9 / 32.8, at 16000 35.0 / 33.4).
   const long pairs = (long)(last_max / ATT_KB + 1) * Hkv * T, group = Hq / Hkv;
-  const bool eight = many && pairs * ((group + 3) / 4) > ctx->compute_units && pairs * ((group + 7) / 8) <= ctx->compute_units;
-  const bool fold = prep && (!many || eight) && !d_offset && T <= 8 && ornith_option_fuse_attn_prep();
+  // (its keys go from memory to LDS, 16 bytes a lane, and its new values come 8 bytes a lane in the buffer form: rows that are not
+  // aligned for that take the four-head form, and a prep launch)
+  const bool eight = many && pairs * ((group + 3) / 4) > ctx->compute_units && pairs * ((group + 7) / 8) <= ctx->compute_units &&
+                     (((uintptr_t)d_k_cache | (uintptr_t)d_v_cache) & 15) == 0;
+  const bool fold = prep && (!many || (eight && ((uintptr_t)prep->vx & 7) == 0)) && !d_offset && T <= 8 && ornith_option_fuse_attn_prep();
   PrepArgs pq{};
   if (prep) {
     pq = *prep;

@@ -84,6 +84,42 @@ def test_attention_bit_exact(orn, ctx, T, Hq, Hkv, hd, cap, offset):
     for b in d + [dkc, dvc, dq, dout, dc, ds]: b.free()
 
 
+@pytest.mark.parametrize("cache_off,vx_off", [(8, 0), (0, 4), (8, 4)])
+def test_attention_of_less_aligned_operands(orn, ctx, cache_off, vx_off):
+    """Caches that are aligned to 8 bytes only, raw value rows to 4, at a size of the eight-head form: the same bits as aligned ones
+    (without them the caches' rows could not go to LDS 16 bytes a lane)"""
+    import ctypes as C
+    T, Hq, Hkv, hd, cap, offset, rd = 4, 16, 2, 256, 4096, 2554, 64
+    rng = np.random.default_rng(5)
+    qg, kx, vx, qw, kw, kc, vc = _mk(rng, T, Hq, Hkv, hd, cap, offset)
+    c, s = util.orc_rope_table(cap, rd, 1e7)
+    dc, ds = ctx.rope_table(cap, rd, 1e7)
+    wkc, wvc = kc.copy(), vc.copy()
+    wq, wgate = util.orc_attn_prep(qg, kx, vx, qw, kw, rd, c, s, offset, wkc, wvc)
+    want = util.orc_sdpa(wq, wkc, wvc, wgate, offset, hd ** -0.5)
+
+    class At:                                         # a device address some bytes into a buffer
+        def __init__(self, a, off):
+            self.a, self.off = a, off
+            self.buf = ctx.alloc(a.nbytes + 16)
+            self.buf.upload(self.bytes(a))
+            self.ptr = C.c_void_p(self.buf.ptr.value + off)
+
+        def bytes(self, a):
+            return np.concatenate([np.zeros(self.off, np.uint8), a.reshape(-1).view(np.uint8), np.zeros(16 - self.off, np.uint8)])
+
+        def get(self):
+            return self.buf.download(np.uint8, self.a.nbytes + 16)[self.off:self.off + self.a.nbytes].view(np.uint16).reshape(self.a.shape)
+
+    d = [At(qg, 0), At(kx, 0), At(vx, vx_off), At(qw, 0), At(kw, 0)]
+    dk, dv, dq, dout = At(kc, cache_off), At(vc, cache_off), ctx.alloc(T * Hq * hd * 2), ctx.alloc(T * Hq * hd * 2)
+    ctx.attn_decode(*d, T, Hq, Hkv, hd, rd, 1e-6, dc, ds, cap, offset, cap, hd ** -0.5, dq, dk, dv, dout)
+    assert np.array_equal(dout.download(np.uint16, want.shape), want)
+    assert np.array_equal(dq.download(np.uint16, wq.shape), wq)
+    assert np.array_equal(dk.get(), wkc) and np.array_equal(dv.get(), wvc)
+    for b in [x.buf for x in d + [dk, dv]] + [dq, dout, dc, ds]: b.free()
+
+
 # the matrix-core forms (four heads a workgroup, and eight; groups of eight and of three heads, head widths 256 and 128) and the
 # 1024-thread one, inside the first key block and past it
 @pytest.mark.parametrize("T,Hq,Hkv,hd,cap,offset", [(4, 16, 2, 256, 4096, 2500), (4, 16, 2, 128, 4096, 3000), (8, 6, 2, 256, 8192, 8000),
