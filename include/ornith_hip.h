@@ -93,14 +93,13 @@ ORNITH_API int ornith_device_info(ornith_ctx* ctx, char* name, size_t name_len, 
  *   "kq_iters"  (ORNITH_KQ_ITERS, default 0 = chosen by the launch from its shape and from how
  *               many of its workgroups a compute unit holds; 1..8): output rows each
  *               wavefront of the k-quant mat-vec walks, a tuning knob
- *   "gemm_duo"  (ORNITH_GEMM_DUO, default 1): the 256-row tile of the prefill GEMM runs with
- *               producer and consumer wavefronts (0: every wavefront dequantizes, then
- *               multiplies); same results either way
- *   "gemm_reg"  (ORNITH_GEMM_REG, default 1): the expert-gathered prefill GEMM dequantizes the
- *               weights into MFMA operand registers where the shape suits it (80 rows an expert
- *               or more, 48 for matrices that the few-row kernels don't take, as K > 4096: up to
- *               192 rows a workgroup for K >= 1024; 64-row workgroups for fewer K slabs from 80;
- *               0: always through LDS); results agree to the order of the fp32 sums
+ *   "gemm_duo"  (ORNITH_GEMM_DUO, default 1): the prefill GEMM dequantizes the weights into MFMA
+ *               operand registers, beside the multiplication, where the shape suits it (from 193
+ *               rows on for more than 2048 columns; 0: always through LDS); results agree to the
+ *               order of the fp32 sums
+ *   "gemm_reg"  (ORNITH_GEMM_REG, default 1): the same of the expert-gathered prefill GEMM (80
+ *               rows an expert or more, 48 for matrices that the few-row kernels don't take, as
+ *               K > 4096; 0: always through LDS); results agree to the order of the fp32 sums
  *   "gdn_chunked" (ORNITH_GDN_CHUNKED, default 1): the gated-delta recurrence of calls of 128
  *               rows or more (without per-token snapshots) runs in 64-token chunks on the
  *               matrix cores (0: token by token); results agree to rounding

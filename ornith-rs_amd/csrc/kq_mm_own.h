@@ -1,0 +1,36 @@
+// The GEMM of long prompts over k-quants (kq_mm_own.hip): what the dispatch of kq_mm.hip fills in and calls.
+#pragma once
+
+#include "dmath.h"
+#include "rt.h"
+
+struct OwnMat {
+  const uint8_t *qs, *scales, *dm;
+  bf16_t* y;
+  int O, kind;
+  int vec;  // rows of y can be stored 16 bytes at a time
+  int t0;  // plain form: first column tile of the launch that is this matrix's
+};
+
+struct OwnArgs {
+  OwnMat m[4];  // plain: up to four matrices of one kind; gathered: the experts' stack
+  int n;
+  const bf16_t* x;
+  int M, K;
+  int tile_rows, row_tiles, col_tiles;  // set by kq_mm_own
+  // gathered form: tiles of up to kOwnRows pairs of an expert-sorted list
+  const uint32_t *pair, *tile_expert, *tile_start, *tile_count, *n_tiles;
+  int tiles_max, up_div;
+  const uint32_t* expert_at;  // over a plan of lower tiles: [E] where an expert's pairs begin; else null
+  int E;
+  uint32_t up_magic;  // 2^32 / up_div rounded up: the upper half of its product with a pair is pair / up_div
+};
+
+constexpr int kOwnRows = 256, kOwnCols = 256;  // a workgroup's tile
+
+// alignment and reach: x of `rows` rows, any K % 256 == 0
+bool kq_mm_own_ok(const ornith_kmatrix& w, const void* x, size_t rows);
+// ... and M rows are many enough for this matrix, whatever shares its launch
+bool kq_mm_own_suits(const ornith_kmatrix& w, const void* x, int M);
+OwnMat kq_mm_own_mat(const ornith_kmatrix& w, void* y);
+int kq_mm_own(ornith_ctx* ctx, OwnArgs& a, bool gather);

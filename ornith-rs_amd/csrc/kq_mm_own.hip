@@ -1,0 +1,576 @@
+// The k-quant GEMM of long prompts: Y[M, O] = X[M, K] . W^T, plain or over an expert-sorted pair list, with the
+// weights dequantized straight into matrix-core operands by the wavefront that owns their columns.
+//
+// Replaces, with kq_mm.hip's other forms, kquant::{qmm_t, gather_qmm_t} (/root/reference/src/ops/kquant.rs:783-1027;
+// kernels/kquant_mm.h).
+//
+// A workgroup is four wavefronts, one a SIMD, and a tile of 256 columns by up to 256 rows. A wavefront owns 64 columns over all the rows:
+// its weights are dequantized once a tile and never written anywhere, and its 16 x 16 accumulator registers (two column blocks
+// by eight row blocks of v_mfma_f32_32x32x16_bf16) are what one wavefront a SIMD leaves room for. The activations, which all
+// four wavefronts multiply by, come in slabs of 64 k straight into LDS (global_load_lds, whole 128-byte lines; no registers, no
+// writes), three slabs deep, with one barrier a slab that leaves requests in flight. The codes go to LDS the same way, into a
+// part that is the wavefront's own: 64 lanes that each read 16 bytes of their own row would look up 64 cache lines a load, whole
+// rows of a super-block 8. One super-block is unpacked while the next one's codes travel.
+//
+// A k step is 16 matrix instructions (at 256 rows), and between them, one piece after each, stands the work for the step
+// after: eight fragment reads, the unpacking of two fragments (36 vector instructions of Q4_K, 52 of Q6_K), a slab's
+// requests. The order is fixed in the source (sched_barrier after each piece) and every wait for memory is counted by hand: requests
+// are inline assembly, because waits that the compiler places at a loop's end are for everything in flight.
+//
+// What bounds it: at full size the matrix cores at the clock the card holds under them (12288 x 2048, 6621 rows: a step takes 0.39 us
+// with every compute unit at work and 0.29 with one; the same loop over weights that are bf16 already, no vector work at all,
+// reaches 1157 TFLOP/s there, this one 1130 to 1157); below about 128 rows a tile the unpacking (0.16 us a step however few the rows);
+// and 3 us of way in and 3.5 us of way out a tile, which nothing overlaps.
+//
+// Measured, us, against the producer / consumer form this replaces (256 x 128 tiles, weights through LDS): 12288 x 2048 Q4_K at 700 / 1500 /
+// 6621 rows 54 / 103 / 357 -> 41 / 77 / 278 (867 -> 1157 TFLOP/s), 2048 x 4096 at 6621 138 -> 96, q / k / v (9216 x 2048 Q6_K) at 700 / 6621 58 / 293 -> 38 /
+// 242, router + shared gate + up at 6621 83 -> 44; and against tiles of 192 rows with activations through registers, the experts of
+// 6621 tokens (207 rows each): gate or up 165 -> 121, down (K = 512) 274 -> 201.
+#include <type_traits>
+
+#include "kq_mm_own.h"
+
+namespace {
+
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef float f32x16_t __attribute__((ext_vector_type(16)));
+typedef unsigned int u32x2_t __attribute__((ext_vector_type(2)));
+typedef unsigned int u32x3_t __attribute__((ext_vector_type(3)));
+typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
+
+template <int N>
+using IC = std::integral_constant<int, N>;
+template <class F, int... I>
+__device__ __forceinline__ void each_of(F f, std::integer_sequence<int, I...>) {
+  (f(IC<I>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void each(F f) {
+  each_of(f, std::make_integer_sequence<int, N>{});
+}
+
+// ---- requests: a base the wavefront shares, a lane's offset. They are waited for by count (wait_loads), never by the
+// compiler; here() is where a request's registers may be used from
+template <int OFF>
+__device__ __forceinline__ void ask(u32x4_t& d, const uint8_t* base, uint32_t off) {
+  asm volatile("global_load_dwordx4 %0, %1, %2 offset:%3" : "=v"(d) : "v"(off), "s"(base), "n"(OFF));
+}
+__device__ __forceinline__ void ask(u32x3_t& d, const uint8_t* base, uint32_t off) {
+  asm volatile("global_load_dwordx3 %0, %1, %2" : "=v"(d) : "v"(off), "s"(base));
+}
+__device__ __forceinline__ void ask(u32x2_t& d, const uint8_t* base, uint32_t off) {
+  asm volatile("global_load_dwordx2 %0, %1, %2" : "=v"(d) : "v"(off), "s"(base));
+}
+__device__ __forceinline__ void ask(uint32_t& d, const uint8_t* base, uint32_t off) {
+  asm volatile("global_load_dword %0, %1, %2" : "=v"(d) : "v"(off), "s"(base));
+}
+__device__ __forceinline__ void ask16(uint32_t& d, const uint8_t* base, uint32_t off) {
+  asm volatile("global_load_ushort %0, %1, %2" : "=v"(d) : "v"(off), "s"(base));
+}
+template <int N>
+__device__ __forceinline__ void wait_loads() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+// BYTES (4 or 16) a lane from memory to LDS, the lanes' pieces side by side at `lds`
+template <int BYTES>
+__device__ __forceinline__ void dma(const uint8_t* base, uint32_t off, uint32_t lds) {
+  typedef const __attribute__((address_space(1))) void glb_t;
+  typedef __attribute__((address_space(3))) void lds_t;
+  if constexpr (BYTES == 16) __builtin_amdgcn_global_load_lds((glb_t*)(uint64_t)(base + off), (lds_t*)(uint64_t)lds, 16, 0, 0);
+  else __builtin_amdgcn_global_load_lds((glb_t*)(uint64_t)(base + off), (lds_t*)(uint64_t)lds, 4, 0, 0);
+}
+__device__ __forceinline__ uint32_t lds_address(const void* p) {
+  return (uint32_t)(uint64_t)(const __attribute__((address_space(3))) void*)p;
+}
+__device__ __forceinline__ const uint8_t* uniform(const uint8_t* p) {
+  const uint64_t v = (uint64_t)p;
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+  return dm_global_ptr<const uint8_t>(((uint64_t)hi << 32) | lo);
+}
+__device__ __forceinline__ void barrier_only() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+// ---- the weights of 32 rows (a wavefront's column block) and one super-block ---------------------
+// The codes go to LDS as whole rows of the super-block (kInstr requests of 64 16-byte pieces), piece `at(row, p)` of a row at a
+// place that keeps the rows of a fragment on different banks; a lane then takes the pieces of its row that are its own.
+template <int KIND>
+struct Fmt;
+template <>
+struct Fmt<ORNITH_Q4K> {
+  static constexpr int kQ = 128, kS = 12, kD = 4, kInstr = 4, kHalf = 2;
+  typedef u32x3_t Scales;
+  static __device__ __forceinline__ void source(int n, int& row, int& p) {  // what lies at 16-byte place n
+    row = n >> 3;
+    p = (n & 7) ^ ((row >> 1) & 7);
+  }
+  static __device__ __forceinline__ int at(int row, int p) { return 16 * (8 * row + (p ^ ((row >> 1) & 7))); }
+  // piece I of half HF that lane half h takes: bytes 16 h .. of 64-group 2 HF + I
+  static __device__ __forceinline__ int piece(int hf, int i, int h) { return 2 * (2 * hf + i) + h; }
+};
+template <>
+struct Fmt<ORNITH_Q6K> {
+  static constexpr int kQ = 192, kS = 16, kD = 2, kInstr = 6, kHalf = 3;
+  typedef u32x4_t Scales;
+  static __device__ __forceinline__ void source(int n, int& row, int& p) {
+    row = n / 12;
+    p = n - 12 * row - ((row >> 2) & 3);
+    p += p < 0 ? 12 : 0;
+  }
+  static __device__ __forceinline__ int at(int row, int p) {
+    int j = p + ((row >> 2) & 3);
+    j -= j >= 12 ? 12 : 0;
+    return 16 * (12 * row + j);
+  }
+  // low rows a and b (I = 0, 1) and high bits (2) of half HF
+  static __device__ __forceinline__ int piece(int hf, int i, int h) { return i < 2 ? 4 * hf + 2 * i + h : 8 + 2 * hf + h; }
+};
+template <int KIND>
+struct Sc {
+  typename Fmt<KIND>::Scales sc;
+  uint32_t dm;
+  template <int I>
+  __device__ __forceinline__ void load(const uint8_t* s0, const uint8_t* d0, uint32_t so, uint32_t dof) {
+    if constexpr (I == 0) {
+      if constexpr (KIND == ORNITH_Q4K) ask(sc, s0, so);
+      else ask<0>(sc, s0, so);
+    } else {
+      if constexpr (KIND == ORNITH_Q4K) ask(dm, d0, dof);
+      else ask16(dm, d0, dof);
+    }
+  }
+  __device__ __forceinline__ void here() { asm volatile("" : "+v"(sc), "+v"(dm)); }
+};
+
+// the upper half of a's lanes trades places with the lower half of b's (swap16: a's odd rows of sixteen with b's even ones)
+__device__ __forceinline__ u32x2_t swap32(uint32_t a, uint32_t b) {
+  const auto v = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+  return u32x2_t{v[0], v[1]};
+}
+__device__ __forceinline__ u32x2_t swap16(uint32_t a, uint32_t b) {
+  const auto v = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+  return u32x2_t{v[0], v[1]};
+}
+
+// s * h + o with h the lower (HI = 0) or upper 16 bits of w as an f16 number: one instruction, one rounding
+template <int HI>
+__device__ __forceinline__ float fma_half(float s, uint32_t w, float o) {
+  float r;
+  if constexpr (HI)
+    asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel:[0,1,0] op_sel_hi:[0,1,0]" : "=v"(r) : "v"(s), "v"(w), "v"(o));
+  else
+    asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel:[0,0,0] op_sel_hi:[0,1,0]" : "=v"(r) : "v"(s), "v"(w), "v"(o));
+  return r;
+}
+
+// w >> N (N < 0: w << -N), another instruction in every step TAG: merged into one, shifted words would be kept from step to step
+template <int N, int TAG>
+__device__ __forceinline__ uint32_t shifted(uint32_t w) {
+  uint32_t r;
+  if constexpr (N >= 0)
+    asm("v_lshrrev_b32 %0, %1, %2 ; %3" : "=v"(r) : "n"(N), "v"(w), "n"(TAG));
+  else
+    asm("v_lshlrev_b32 %0, %1, %2 ; %3" : "=v"(r) : "n"(-N), "v"(w), "n"(TAG));
+  return r;
+}
+
+// The operand of k step T (0 .. 15 of the super-block), made in seven pieces so that they can stand between matrix instructions.
+template <int KIND>
+struct Deq {
+  typedef Fmt<KIND> F;
+  u32x4_t q[2 * F::kHalf];  // the lane's codes, by half
+  float dl, dh, nm;         // d * 2^24, d * 2^20, -dmin
+  uint32_t sc4, m4;         // the half's four scales and minima
+  float s, o;
+  uint32_t e0, o0, e1, o1;
+  float x0, x1;
+  u32x4_t f;
+  template <int T, int P>
+  __device__ __forceinline__ void piece(const Sc<KIND>& z, int h) {
+    constexpr int HF = T >> 3, QD = (T >> 1) & 3, NIB = KIND == ORNITH_Q4K ? QD & 1 : QD >> 1;
+    if constexpr (P == 0) {
+      if constexpr (KIND == ORNITH_Q4K) {
+        if constexpr (T == 0) {
+          const float d = dm_h2f((f16_t)(z.dm & 0xffffu));
+          dl = d * 16777216.f;
+          dh = d * 1048576.f;
+          nm = -dm_h2f((f16_t)(z.dm >> 16));
+          sc4 = z.sc[0] & 0x3f3f3f3fu;
+          m4 = z.sc[1] & 0x3f3f3f3fu;
+        }
+        if constexpr (T == 8) {
+          sc4 = (z.sc[2] & 0x0f0f0f0fu) | ((z.sc[0] & 0xc0c0c0c0u) >> 2);
+          m4 = ((z.sc[2] >> 4) & 0x0f0f0f0fu) | ((z.sc[1] & 0xc0c0c0c0u) >> 2);
+        }
+        if constexpr (T % 2 == 0) {
+          s = (NIB ? dh : dl) * dm_ubyte<QD>(sc4);
+          o = nm * dm_ubyte<QD>(m4);
+        }
+      } else {
+        if constexpr (T == 0) dl = dm_h2f((f16_t)z.dm);
+        if constexpr (T % 2 == 0) {  // scale 8 HF + 2 QD + h of the sixteen
+          const float v = dl * (float)(int)(int8_t)(((z.sc[T >> 2] >> (8 * h)) >> (16 * (QD & 1))) & 0xffu);
+          s = v * (NIB ? 1048576.f : 16777216.f);
+          o = -32.f * v;
+        }
+      }
+    } else if constexpr (P == 1 || P == 2) {
+      constexpr int I = P - 1, W = 2 * (T & 1) + I;
+      constexpr uint32_t M = NIB ? 0x00f000f0u : 0x000f000fu;
+      uint32_t e, od;
+      if constexpr (KIND == ORNITH_Q4K) {
+        const uint32_t w = q[T >> 2][W];
+        e = w & M;
+        od = shifted<8, T>(w) & M;
+      } else {
+        constexpr int SH = 4 - 2 * (QD & 1);
+        constexpr uint32_t MH = NIB ? 0x03000300u : 0x00300030u;
+        const uint32_t w = q[3 * HF + (QD & 1)][W], hb = q[3 * HF + 2][W];
+        e = (w & M) | (shifted<-SH, T>(hb) & MH);
+        od = (shifted<8, T>(w) & M) | (shifted<8 - SH, T>(hb) & MH);
+      }
+      if constexpr (I == 0) e0 = e, o0 = od;
+      else e1 = e, o1 = od;
+    } else if constexpr (P == 3) {
+      x0 = fma_half<0>(s, e0, o), x1 = fma_half<0>(s, o0, o);
+    } else if constexpr (P == 4) {
+      const float y0 = fma_half<1>(s, e0, o), y1 = fma_half<1>(s, o0, o);
+      f[0] = dm_f2bf2(x0, x1);
+      x0 = y0, x1 = y1;
+    } else if constexpr (P == 5) {
+      const float y0 = fma_half<0>(s, e1, o), y1 = fma_half<0>(s, o1, o);
+      f[1] = dm_f2bf2(x0, x1);
+      x0 = y0, x1 = y1;
+    } else {
+      const float y0 = fma_half<1>(s, e1, o), y1 = fma_half<1>(s, o1, o);
+      f[2] = dm_f2bf2(x0, x1);
+      f[3] = dm_f2bf2(y0, y1);
+    }
+  }
+};
+
+constexpr int kStages = 3;                          // of 64 k: 128 bytes of a row
+constexpr int kActs = kStages * kOwnRows * 128;      // LDS: activations, then a part for each wavefront's codes
+constexpr int kLds = kActs + kOwnCols * 192;
+
+template <int KIND, int TM, bool GATHER>
+__device__ __forceinline__ void own_tile(const OwnArgs& a, const OwnMat& mt, uint8_t* smem, uint32_t* s_dst, int n0, int rows, int m0,
+                                         int64_t wrow0, const uint32_t* pairs) {
+  typedef Fmt<KIND> F;
+  constexpr int STAGE = TM * 4096, TN = 2, SL = TN * TM;
+  constexpr int NC = TN * (F::kInstr + 2);  // requests of a super-block's weights
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l32 = lane & 31, h = lane >> 5;
+  const int nb = a.K >> 8;
+  uint32_t qo[TN][F::kInstr], so[TN], dof[TN];
+#pragma unroll
+  for (int j = 0; j < TN; ++j) {
+    const int r0 = n0 + 64 * wave + 32 * j;
+#pragma unroll
+    for (int i = 0; i < F::kInstr; ++i) {
+      int row, p;
+      F::source(64 * i + lane, row, p);
+      qo[j][i] = (uint32_t)min(r0 + row, mt.O - 1) * (uint32_t)(nb * F::kQ) + 16 * p;
+    }
+    const uint32_t row = (uint32_t)min(r0 + l32, mt.O - 1) * (uint32_t)nb;
+    so[j] = row * F::kS;
+    dof[j] = row * F::kD;
+  }
+  const uint8_t *qb = uniform(mt.qs + wrow0 * nb * F::kQ), *sb = uniform(mt.scales + wrow0 * nb * F::kS), *db = uniform(mt.dm + wrow0 * nb * F::kD);
+  __builtin_amdgcn_sched_barrier(0);
+  // request i of a slab's activations: eight rows of row block i, 128 bytes each
+  uint32_t pr[TM];
+  if constexpr (GATHER) {
+    const uint8_t* pb = uniform((const uint8_t*)pairs);
+    dma<4>(pb, 4 * min(tid, rows - 1), lds_address(s_dst) + 256 * wave);
+#pragma unroll
+    for (int i = 0; i < TM; ++i) ask(pr[i], pb, 4 * min(32 * i + 8 * wave + (lane >> 3), rows - 1));
+  } else {
+#pragma unroll
+    for (int i = 0; i < TM; ++i) pr[i] = m0 + min(32 * i + 8 * wave + (lane >> 3), rows - 1);
+  }
+  uint8_t* const mine = smem + kActs + wave * (64 * F::kQ);
+  const uint32_t mine_at = lds_address(mine);
+  Sc<KIND> cur[TN], nxt[TN];
+  auto weights = [&](Sc<KIND> (&z)[TN], const uint8_t* q0, const uint8_t* s0, const uint8_t* d0, auto ic) {
+    constexpr int I = decltype(ic)::value;
+    if constexpr (I < TN * F::kInstr) dma<16>(q0, qo[I / F::kInstr][I % F::kInstr], mine_at + 1024 * I);
+    else z[(I - TN * F::kInstr) / 2].template load<I % 2>(s0, d0, so[(I - TN * F::kInstr) / 2], dof[(I - TN * F::kInstr) / 2]);
+  };
+  each<NC>([&](auto ic) { weights(cur, qb, sb, db, ic); });
+  __builtin_amdgcn_sched_barrier(0);
+  if constexpr (GATHER) {
+    wait_loads<NC>();
+#pragma unroll
+    for (int i = 0; i < TM; ++i) asm volatile("" : "+v"(pr[i]));
+  }
+  uint32_t xo[TM];
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {
+    const uint32_t src = GATHER && a.up_div > 1 ? __umulhi(pr[i], a.up_magic) : pr[i];
+    uint32_t at = src * (2u * (uint32_t)a.K);
+    asm volatile("" : "+v"(at));  // (or its sum becomes a 64-bit multiply-add that names registers still to be filled)
+    xo[i] = at + 16 * ((lane & 7) ^ ((4 * wave + (lane >> 4)) & 7));
+  }
+  const uint8_t* xg = reinterpret_cast<const uint8_t*>(a.x);
+  const uint32_t at = lds_address(smem) + wave * 1024;
+#pragma unroll
+  for (int s = 0; s < kStages; ++s)
+#pragma unroll
+    for (int i = 0; i < TM; ++i) dma<16>(xg + 128 * s, xo[i], at + s * STAGE + i * 4096);
+  __builtin_amdgcn_sched_barrier(0);
+  f32x16_t acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+  // step T's fragment of row block i: piece 4 ((T >> 1) & 1) + 2 h + (T & 1) of the slab's 128 bytes, which lie turned by the row
+  uint32_t rd[4];
+#pragma unroll
+  for (int t = 0; t < 4; ++t) rd[t] = l32 * 128 + 16 * ((4 * (t >> 1) + 2 * h + (t & 1)) ^ ((l32 >> 1) & 7));
+  uint32_t st = 0;  // stage of the slab
+  auto after = [](uint32_t s) { return s == 2 * STAGE ? 0u : s + STAGE; };
+  bf16x8_t af[TM], bf[2][TN];
+  auto read = [&](auto tc, uint32_t from, int i) {
+    af[i] = *reinterpret_cast<const bf16x8_t*>(smem + (rd[decltype(tc)::value & 3] + from) + i * 4096);
+  };
+  Deq<KIND> dq[TN];
+  auto codes = [&](auto hc, int j) {
+    constexpr int HF = decltype(hc)::value;
+#pragma unroll
+    for (int i = 0; i < F::kHalf; ++i)
+      dq[j].q[F::kHalf * HF + i] = *reinterpret_cast<const u32x4_t*>(mine + j * (32 * F::kQ) + F::at(l32, F::piece(HF, i, h)));
+  };
+  wait_loads<2 * TM>();  // the weights and stage 0
+#pragma unroll
+  for (int j = 0; j < TN; ++j) cur[j].here();
+  barrier_only();
+#pragma unroll
+  for (int j = 0; j < TN; ++j) codes(IC<0>{}, j), codes(IC<1>{}, j);
+#pragma unroll
+  for (int i = 0; i < TM; ++i) read(IC<0>{}, st, i);
+  each<TN * 7>([&](auto pc) {
+    constexpr int J = decltype(pc)::value / 7, P = decltype(pc)::value % 7;
+    dq[J].template piece<0, P>(cur[J], h);
+  });
+#pragma unroll
+  for (int j = 0; j < TN; ++j) bf[0][j] = __builtin_bit_cast(bf16x8_t, dq[j].f);
+  __builtin_amdgcn_sched_barrier(0);
+
+  for (int ib = 0; ib < nb; ++ib) {
+    // A slab's activations are asked for three slabs ahead (into the stage it leaves), the next block's weights in slab 0
+    // (the wavefront's own part of LDS has been read by then).
+    const bool last = ib + 1 == nb;
+    each<16>([&](auto tc) {
+      constexpr int T = decltype(tc)::value, S = T >> 2, U = T + 1;  // U: the step being made ready
+      const uint32_t st1 = after(st);
+      if constexpr ((T & 3) == 3) {
+        // Slab S + 1 has arrived (asked for two slabs ago: a slab's requests, in slab 1 the weights' too, may be out behind it),
+        // in slab 2 the weights; everyone has read what slab S holds
+        if constexpr (S == 0 || S == 3) wait_loads<TM>();
+        if constexpr (S == 1) {
+          if (last) wait_loads<TM>();
+          else wait_loads<TM + NC>();
+        }
+        if constexpr (S == 2) {
+          if (last) wait_loads<0>();
+          else wait_loads<TM>();
+#pragma unroll
+          for (int j = 0; j < TN; ++j) nxt[j].here();
+        }
+        if constexpr (S == 3) {
+#pragma unroll
+          for (int j = 0; j < TN; ++j) cur[j] = nxt[j];
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        barrier_only();
+      }
+      each<SL>([&](auto ic) {
+        constexpr int I = decltype(ic)::value, M = I / TN, N = I % TN;
+        acc[M][N] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bf[T & 1][N], af[M], acc[M][N], 0, 0, 0);
+        if constexpr (N == TN - 1) read(IC<U>{}, (T & 3) == 3 ? st1 : st, M);
+        if constexpr ((T == 12 || T == 15) && I < TN) codes(IC<(T == 12 ? 0 : 1)>{}, I);
+        constexpr int P0 = I * (TN * 7) / SL, P1 = (I + 1) * (TN * 7) / SL;
+        each<P1 - P0>([&](auto pc) {
+          constexpr int Q = P0 + decltype(pc)::value, J = Q % TN, P = Q / TN;
+          dq[J].template piece<(U & 15), P>(cur[J], h);
+          if constexpr (P == 6) bf[U & 1][J] = __builtin_bit_cast(bf16x8_t, dq[J].f);
+        });
+        if constexpr ((T & 3) == 3) {
+          constexpr int NR = TM + (S == 0 ? NC : 0);
+          if constexpr ((I * NR + SL - 1) / SL < ((I + 1) * NR + SL - 1) / SL)
+            each<NR>([&](auto nc) {
+              constexpr int Q = decltype(nc)::value;
+              if constexpr (Q * SL / NR == I) {
+                if constexpr (Q < TM) {
+                  if (S == 0 || !last) dma<16>(xg + 128 * (S + 3), xo[Q], at + st + Q * 4096);
+                } else {
+                  if (!last) weights(nxt, qb + F::kQ, sb + F::kS, db + F::kD, IC<Q - TM>{});
+                }
+              }
+            });
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      });
+      if constexpr ((T & 3) == 3) st = st1;
+    });
+    xg += 512;
+    qb += F::kQ;
+    sb += F::kS;
+    db += F::kD;
+  }
+  // D[n = 8 b + 4 h + r][m = l32]: two swaps of lanes bring 32 columns of a row into four lanes, 16 bytes each
+  const int half = 16 * ((lane >> 4) & 1) + 8 * h;
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {
+    bf16_t* y[2];
+    bool live[2];
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      const int r = 32 * i + 16 * b + (lane & 15);
+      live[b] = r < rows;
+      y[b] = mt.y + (size_t)(GATHER ? s_dst[r] : (uint32_t)(m0 + r)) * mt.O + n0 + 64 * wave + half;
+    }
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      const f32x16_t& c = acc[i][j];
+      u32x4_t v[2];
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {
+        const u32x2_t p = swap32(dm_f2bf2(c[8 * b], c[8 * b + 1]), dm_f2bf2(c[8 * b + 4], c[8 * b + 5]));
+        const u32x2_t q = swap32(dm_f2bf2(c[8 * b + 2], c[8 * b + 3]), dm_f2bf2(c[8 * b + 6], c[8 * b + 7]));
+        v[b] = u32x4_t{p[0], q[0], p[1], q[1]};  // columns 16 b + 8 h ..
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const u32x2_t p = swap16(v[0][e], v[1][e]);
+        v[0][e] = p[0];
+        v[1][e] = p[1];
+      }
+      const int left = mt.O - (n0 + 64 * wave + 32 * j + half);
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+        if (live[b] && left > 0) {
+          if (mt.vec) *reinterpret_cast<u32x4_t*>(y[b] + 32 * j) = v[b];
+          else {  // (rows of y that are not 16-byte aligned)
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+              if (e < left) y[b][32 * j + e] = (bf16_t)(v[b][e >> 1] >> (16 * (e & 1)));
+          }
+        }
+    }
+  }
+}
+
+constexpr int kMixed = 2;  // the matrices of the launch differ in kind
+template <int KIND, bool GATHER>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void kq_mm_own_kernel(OwnArgs a) {
+  __shared__ __attribute__((aligned(1024))) uint8_t smem[kLds];
+  __shared__ uint32_t s_dst[GATHER ? kOwnRows : 1];
+  int rows, m0 = 0, tc, mat = 0;
+  int64_t wrow0 = 0;
+  const uint32_t* pairs = nullptr;
+  const uint32_t die = blockIdx.x & 7, seq = blockIdx.x >> 3;
+  if constexpr (GATHER) {
+    const uint32_t tile = seq / (uint32_t)a.col_tiles * 8u + die, at = min(tile, (uint32_t)a.tiles_max - 1u), n = *a.n_tiles;
+    tc = (int)(seq % (uint32_t)a.col_tiles);
+    const uint32_t e = __builtin_amdgcn_readfirstlane(a.tile_expert[at]);
+    rows = __builtin_amdgcn_readfirstlane((int)a.tile_count[at]);
+    pairs = a.pair + __builtin_amdgcn_readfirstlane(a.tile_start[at]);
+    if (tile >= n) return;
+    if (a.expert_at) {
+      // a plan of lower tiles (16, 32 or 64 rows): the first of as many as a tile here holds works on the pairs of them all
+      const int first = (int)__builtin_amdgcn_readfirstlane(a.expert_at[e]), st = (int)(pairs - a.pair);
+      const int end = (int)e + 1 < a.E ? (int)__builtin_amdgcn_readfirstlane(a.expert_at[e + 1]) : a.M;
+      if ((st - first) % kOwnRows != 0) return;
+      rows = min(end - st, kOwnRows);
+    }
+    wrow0 = (int64_t)e * a.m[0].O;
+  } else {
+    const int total = a.row_tiles * a.col_tiles, per = (total + 7) / 8, id = (int)die * per + (int)seq;
+    if ((int)seq >= per || id >= total) return;
+    constexpr int GM = 8;
+    const int grp = id / (GM * a.col_tiles), in = id - grp * GM * a.col_tiles, gm = min(GM, a.row_tiles - grp * GM);
+    m0 = (grp * GM + in % gm) * a.tile_rows;
+    tc = in / gm;
+    rows = min(a.tile_rows, a.M - m0);
+#pragma unroll
+    for (int i = 1; i < 4; ++i)
+      if (i < a.n && tc >= a.m[i].t0) mat = i;
+  }
+  const OwnMat mt = a.m[mat];
+  const int n0 = (tc - mt.t0) * kOwnCols;
+  const int groups = (rows + 31) >> 5;
+  auto of_kind = [&](auto kc) {
+    constexpr int KD = decltype(kc)::value;
+#define OWN(N) own_tile<KD, N, GATHER>(a, mt, smem, s_dst, n0, rows, m0, wrow0, pairs)
+    if (groups >= 8) OWN(8);
+    else if (groups == 7) OWN(7);
+    else if (groups == 6) OWN(6);
+    else if (groups == 5) OWN(5);
+    else if (groups == 4) OWN(4);
+    else if (groups == 3) OWN(3);
+    else OWN(2);
+#undef OWN
+  };
+  if constexpr (KIND != kMixed) of_kind(IC<KIND>{});
+  else if (mt.kind == ORNITH_Q4K) of_kind(IC<ORNITH_Q4K>{});
+  else of_kind(IC<ORNITH_Q6K>{});
+}
+
+}  // namespace
+
+bool kq_mm_own_ok(const ornith_kmatrix& w, const void* x, size_t rows) {
+  return w.K >= 256 && w.K % 256 == 0 && rows * w.K * 2 < (size_t(1) << 32) && (size_t)w.O * (w.K / 256) * 192 < (size_t(1) << 32) &&
+         (((uintptr_t)x | (uintptr_t)w.d_qs) & 15) == 0 && (((uintptr_t)w.d_scales | (uintptr_t)w.d_dm) & 3) == 0;
+}
+
+// Rows from which a matrix runs here. Fewer take the few-row kernels (up to the lines of mm_narrow_host.h), whose splits suit
+// them: this form's step has a floor, so that a tile of any height takes 24 us at K = 2048 and 43 at 4096. us, there / here: 8192 + 4096
+// columns of K = 2048, Q4_K, 150 / 200 / 300 rows 24 / 25, 27 / 26, 30 / 27; 2048 x 4096 Q4_K at 1500 / 2000 45 / 45, 56 / 47, Q6_K at 1000 /
+// 1200 47 / 54, 57 / 55; 256 x 2048 Q6_K at 2000 / 3000 18 / 28, 29 / 28. Few slabs: 4096 x 1024 at 512 / 700 rows 12 / 15, 16 / 15; 2048 x 512 Q6_K at 2000 / 2500
+// rows 11 / 12, 15 / 14 (there: the 128-row tiles of kq_mm.hip).
+bool kq_mm_own_suits(const ornith_kmatrix& w, const void* x, int M) {
+  const int from = w.K < 2048 ? (w.O > 2048 ? 512 : 2048) : w.O > 2048 ? 192 : w.O > 256 ? 1024 : 2048;
+  return M > from && kq_mm_own_ok(w, x, M);
+}
+
+OwnMat kq_mm_own_mat(const ornith_kmatrix& w, void* y) {
+  return {(const uint8_t*)w.d_qs, (const uint8_t*)w.d_scales, (const uint8_t*)w.d_dm, (bf16_t*)y, w.O, w.kind, w.O % 8 == 0 && ((uintptr_t)y & 15) == 0, 0};
+}
+
+int kq_mm_own(ornith_ctx* ctx, OwnArgs& a, bool gather) {
+  int kind = a.m[0].kind, grid;
+  typedef void (*Kernel)(OwnArgs);
+  Kernel k;
+  if (gather) {
+    a.up_magic = (uint32_t)(((uint64_t(1) << 32) + a.up_div - 1) / a.up_div);
+    a.col_tiles = (a.m[0].O + kOwnCols - 1) / kOwnCols;
+    grid = a.col_tiles * ((a.tiles_max + 7) / 8 * 8);
+    k = kind == ORNITH_Q4K ? kq_mm_own_kernel<ORNITH_Q4K, true> : kq_mm_own_kernel<ORNITH_Q6K, true>;
+  } else {
+    a.col_tiles = 0;
+    for (int i = 0; i < a.n; ++i) {
+      a.m[i].t0 = a.col_tiles;
+      a.col_tiles += (a.m[i].O + kOwnCols - 1) / kOwnCols;
+      if (a.m[i].kind != kind) kind = kMixed;
+    }
+    // Tile height: a tile takes about as long as 6 + its row blocks (K = 2048, one tile a compute unit, us: 8 blocks 53, 7 49, 6 44, 5 42;
+    // K = 4096 8 82, 5 61, 2 45), and the rounds of tiles count.
+    long best = 0;
+    for (int tm = 8; tm >= 2; --tm) {
+      const long tiles = (long)((a.M + 32 * tm - 1) / (32 * tm)) * a.col_tiles, cost = (tiles + ctx->compute_units - 1) / ctx->compute_units * (tm + 6);
+      if (tm == 8 || cost < best) best = cost, a.tile_rows = 32 * tm;
+    }
+    a.row_tiles = (a.M + a.tile_rows - 1) / a.tile_rows;
+    grid = (a.row_tiles * a.col_tiles + 7) / 8 * 8;
+    k = kind == kMixed ? kq_mm_own_kernel<kMixed, false> : kind == ORNITH_Q4K ? kq_mm_own_kernel<ORNITH_Q4K, false> : kq_mm_own_kernel<ORNITH_Q6K, false>;
+  }
+  hipLaunchKernelGGL(k, dim3(grid), dim3(256), 0, ctx->stream, a);
+  ORN_LAUNCH_CHECK("kq_mm_own_kernel");
+  return ORNITH_OK;
+}

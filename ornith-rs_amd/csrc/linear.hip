@@ -13,6 +13,7 @@
 // a chunk: 12288 x 2048 in 4 bits at two rows 15.9 us here with the norm in front, 9.7 there), and prompts
 // of ornith_option_gemm_rows() rows and more the matrix cores (mm_narrow.h, kq_mm.hip, dense_mm_kernel below).
 #include "dmath.h"
+#include "kq_mm_own.h"
 #include "linear_device.h"
 #include "mm_narrow_host.h"
 #include "norm_device.h"
@@ -410,17 +411,18 @@ static int linear_matmul_multi(ornith_ctx* ctx, const ornith_linear* const* ws, 
     ORN_LAUNCH_CHECK("dense_mm_kernel");
     return ORNITH_OK;
   }
-  // prefill widths: runs of k-quant matrices of one K share a GEMM launch. A run of one kind may
-  // be large (it picks its tile by size); a matrix of the other kind joins a run only while the
-  // run is narrow (a mixed launch takes 128-row tiles, which wide matrices should not pay for).
+  // prefill widths: runs of k-quant matrices of one K share a GEMM launch. Those that suit the own-column form may always; of
+  // others a run of one kind may be large (it picks its tile by size), but a matrix of the other kind joins a run only
+  // while the run is narrow (a mixed launch takes 128-row tiles, which wide matrices should not pay for).
   for (int i = 0; i < n;) {
     int j = i + 1;
     if (wide && ornith_option_fuse_proj() && ws[i]->mode == ORNITH_LIN_KQUANT) {
       int cols = ws[i]->O;
-      bool mixed = false;
+      bool mixed = false, own = kq_mm_own_suits(ws[i]->km, d_x, M);
       while (j < n && j - i < 4 && ws[j]->mode == ORNITH_LIN_KQUANT && ws[j]->K == ws[i]->K) {
         const bool other = ws[j]->km.kind != ws[i]->km.kind;
-        if ((other || mixed) && cols + ws[j]->O > 2048) break;
+        own = own && kq_mm_own_suits(ws[j]->km, d_x, M);
+        if ((other || mixed) && !own && cols + ws[j]->O > 2048) break;
         mixed = mixed || other;
         cols += ws[j]->O;
         ++j;

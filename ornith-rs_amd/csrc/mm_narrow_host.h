@@ -9,17 +9,13 @@ namespace nmm {
 // Rows up to which a k-quant projection takes these kernels: the wide kernels' 256 x 128 tiles fill the device from about a
 // thousand rows of 12288 columns on, and for up to 2048 columns not before a thousand rows either (2048 x 4096, us here /
 // there: 64 rows 7.2 / 52, 256 rows 15 / 53, 700 rows 29 / 54, 1024 rows 38 / 55; 256 x 2048: 5 / 29, 1024 rows 9 / 29).
-// More columns than that go from K split over wavefronts to columns owned by them (kTall) at kNarrowRows rows, where the
-// former's activations, read by every 64 columns, start to weigh (12288 x 2048 Q4_K, us, split / owned / wide kernels:
-// 128 rows 20 / 20 / 29, 200 rows 30 / 26 / 42, 300 rows - / 26 / 41, 512 rows - / 35 / 42, 700 rows - / 53 / 66, 900 rows
-// - / 63 / 67, 1200 rows - / 82 / 71). Q6_K goes straight to the wide kernels: its one wide matrix, q_proj, shares their launch
-// with k and v (q, k, v: 300 rows 41 owned, k and v apart, 40 there; 700 rows 57 / 58). The rule looks at one matrix at a
-// time, never at what shares its launch: a matrix gives the same bits alone and in company.
+// More columns than that go to the own-column kernel of kq_mm_own.hip (12288 x 2048 Q4_K, us, here / there: 128 rows 20 / 25, 200 rows
+// 27 / 26; the rule there looks at one matrix at a time, never at what shares its launch: a matrix gives the same bits alone and in company).
 // The lines for up to 2048 columns, from K = 2048 on (below, the wide kernels' few slabs are over as soon: 2048 x 512 at 1024 rows 10.5 /
 // 9.9): Q4_K 1536 rows (2048 x 4096 at 1200 / 1500 / 2000 rows 44 / 54, 46 / 55, 58 / 57), Q6_K 1024 (2048 x 4096 at 1024 / 1200 / 1500 rows
 // 51 / 57, 56 / 57, 67 / 58), and up to 256 columns, which are 16 to 40 workgroups of the wide kernels, 2560 (the router at 1200 / 2000 / 2500
 // rows 13 / 29, 17 / 29, 21 / 29; level at 4096).
-constexpr int kNarrowRows = 192, kNarrowRowsSlim = 1024, kNarrowRowsSlimQ4K = 1536, kNarrowRowsSlimmest = 2560, kTallRowsQ4K = 960;
+constexpr int kNarrowRows = 192, kNarrowRowsSlim = 1024, kNarrowRowsSlimQ4K = 1536, kNarrowRowsSlimmest = 2560;
 // The affine formats have no wide kernels: their projections own columns from here on (4-bit, 12288 x 2048, us, split /
 // owned: 300 rows 37 / 37, 400 rows 50 / 52, 512 rows 56 / 51, 600 rows 68 / 61, 2000 rows 207 / 187).
 constexpr int kTallFromAffine = 448;
@@ -61,8 +57,8 @@ int launch_affine(ornith_ctx* ctx, const Args& a, int mode, int ct, int rows, in
 
 // The kernels of a family, gathered ones for launches of one kind (K1, K2) and of both (-1): a kernel has the registers of
 // its widest path. A workgroup is four wavefronts, one a SIMD; a compute unit holds two plain ones, and as many
-// gathered ones as registers and LDS allow (WAVES: asked for, a SIMD).
-#define NMM_KERNELS(NAME, AFF, K1, K2, WAVES, LDS_BIT)                                                              \
+// gathered ones as registers and LDS allow (WAVES: asked for, a SIMD). TALL1, TALL2: the kernels of kTall, if the family has them.
+#define NMM_KERNELS(NAME, AFF, K1, K2, WAVES, LDS_BIT, TALL1, TALL2)                                                \
   template <int CT, int ROWS>                                                                                       \
   __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void NAME##_plain_kernel(Args a) {   \
     body<AFF, CT, kPlain, ROWS, 4>(a);                                                                              \
@@ -72,16 +68,12 @@ int launch_affine(ornith_ctx* ctx, const Args& a, int mode, int ct, int rows, in
       NAME##_gather_kernel(Args a) {                                                                                \
     body<AFF, 2, MODE, ROWS, 4, KIND>(a);                                                                           \
   }                                                                                                                 \
-  template <int KIND>                                                                                               \
-  __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KIND == kA4 ? 4 : 2))) void NAME##_tall_kernel(Args a) {       \
-    body<AFF, 2, kTall, 64, 4, KIND>(a);                                                                            \
-  }                                                                                                                 \
   int launch_##NAME(ornith_ctx* ctx, const Args& a, int mode, int ct, int rows, int kind, dim3 grid, int lds) {     \
     typedef void (*Kernel)(Args);                                                                                   \
     static const Kernel plain[3][2] = {{NAME##_plain_kernel<1, 32>, NAME##_plain_kernel<1, 64>},                    \
                                        {NAME##_plain_kernel<2, 32>, NAME##_plain_kernel<2, 64>},                    \
                                        {NAME##_plain_kernel<4, 64>, NAME##_plain_kernel<4, 64>}};                   \
-    static const Kernel tall[2] = {NAME##_tall_kernel<K1>, NAME##_tall_kernel<AFF ? -1 : K1>};                      \
+    static const Kernel tall[2] = {TALL1, TALL2};                                                                   \
     static const Kernel gather[3][2][3] = {                                                                         \
         {{NAME##_gather_kernel<kGather, 16, K1>, NAME##_gather_kernel<kGather, 32, K1>, NAME##_gather_kernel<kGather, 64, K1>},     \
          {NAME##_gather_kernel<kGateUp, 16, K1>, NAME##_gather_kernel<kGateUp, 32, K1>, NAME##_gather_kernel<kGateUp, 64, K1>}},    \
@@ -94,7 +86,7 @@ int launch_affine(ornith_ctx* ctx, const Args& a, int mode, int ct, int rows, in
         for (const Kernel k : p)                                                                                    \
           ORN_HIP(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes));      \
       for (const Kernel k : tall)                                                                                   \
-        ORN_HIP(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes));        \
+        if (k) ORN_HIP(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes));        \
       for (const auto& g : gather)                                                                                  \
         for (const auto& m : g)                                                                                     \
           for (const Kernel k : m)                                                                                  \

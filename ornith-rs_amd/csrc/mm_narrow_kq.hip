@@ -5,7 +5,7 @@
 
 namespace nmm {
 constexpr int kq_waves(int kind, int rows) { return rows == 16 ? (kind == kQ4K ? 5 : 4) : rows == 32 ? (kind == kQ4K ? 4 : 3) : 2; }
-NMM_KERNELS(kq, false, kQ4K, kQ6K, kq_waves, 4u)
+NMM_KERNELS(kq, false, kQ4K, kQ6K, kq_waves, 4u, nullptr, nullptr)
 
 namespace {
 
@@ -69,14 +69,14 @@ bool plain_ok(const ornith_linear* const* ws, int n, const void* d_x, int M, voi
   for (int i = 0; i < n; ++i) {
     const bool q4 = ws[i]->km.kind == ORNITH_Q4K;
     const int slim = K < 2048 ? kNarrowRowsSlim : ws[i]->O <= 256 ? kNarrowRowsSlimmest : q4 ? kNarrowRowsSlimQ4K : kNarrowRowsSlim;
-    if (M > (ws[i]->O <= 2048 ? slim : q4 ? kTallRowsQ4K : kNarrowRows)) return false;
+    if (M > (ws[i]->O <= 2048 ? slim : kNarrowRows)) return false;
   }
   return true;
 }
 
 namespace {
 // the form of one matrix, whatever shares its launch
-bool tall(const ornith_linear& w, int M) { return w.O > 2048 && M > (affine(kind_of(w)) ? kTallFromAffine : kNarrowRows); }
+bool tall(const ornith_linear& w, int M) { return affine(kind_of(w)) && w.O > 2048 && M > kTallFromAffine; }
 
 int launch_tall(ornith_ctx* ctx, Args& a) {
   int kind = a.m[0].kind, lds = 0;
@@ -89,7 +89,7 @@ int launch_tall(ornith_ctx* ctx, Args& a) {
   }
   a.tiles_max = (a.M + 63) / 64;
   const dim3 grid((unsigned)((a.blocks + 7) / 8 * 8 * a.tiles_max + (a.d.wgs + 7) / 8 * 8));
-  return affine(a.m[0].kind) ? launch_affine(ctx, a, kTall, 0, 64, kind, grid, lds) : launch_kq(ctx, a, kTall, 0, 64, kind, grid, lds);
+  return launch_affine(ctx, a, kTall, 0, 64, kind, grid, lds);
 }
 
 int launch_split(ornith_ctx* ctx, Args& a) {

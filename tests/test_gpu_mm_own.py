@@ -1,0 +1,68 @@
+"""GPU: the long-prompt GEMM whose wavefronts own columns (csrc/kq_mm_own.hip), at the edges of its tiles: every
+tile height, rows and columns that end inside one, one super-block of K and an odd number of them, one
+row of an expert. Against a float64 product over the bf16-rounded dequantized weights, which is what the matrix cores
+are fed: an element may be off by the rounding of the bf16 result (half an ulp of 8 significant bits: 2^-8 of it at most) and by its fp32 sum, whose K additions
+err by at most 2^-24 each of what has been added up, sum |x w| at most; twice that for the matrix cores' own order."""
+import numpy as np
+import pytest
+
+import util
+from util import Q4K, Q6K
+
+pytestmark = pytest.mark.gpu
+
+
+def _deq(kind, t, E, O, K):
+    w = util.orc_dequant(kind, *t, E * O * K // 256).reshape(E, O, K)
+    return util.bf16_to_f32(util.f32_to_bf16(w)).astype(np.float64)
+
+
+def _check(got_bits, x, w, what):
+    want, mass = x @ w.T, np.abs(x) @ np.abs(w).T
+    err = np.abs(util.bf16_to_f32(got_bits).astype(np.float64) - want)
+    bound = 2.0 ** -8 * np.abs(want) + 2 * x.shape[1] * 2.0 ** -24 * mass
+    assert np.all(err <= bound), (what, float((err / bound).max()))
+
+
+@pytest.mark.parametrize("kind,O,K,M", [
+    # the lowest row counts of the rule: wide matrices of K >= 2048 and below, narrow ones
+    (Q4K, 2056, 2048, 193), (Q6K, 2056, 2304, 193), (Q4K, 2304, 256, 513), (Q6K, 2051, 768, 545), (Q6K, 72, 256, 2049),
+    (Q4K, 257, 2048, 1025 + 512),
+    # 64 column tiles: the tile height that fills 256 compute units, 8, 8, 7, 6 and 5 blocks of 32 rows, and what is left of it
+    (Q4K, 16384, 256, 1000), (Q6K, 16384, 256, 900), (Q4K, 16384, 256, 890), (Q6K, 16384, 256, 760), (Q4K, 16380, 512, 601),
+    # more than one round of tiles, in patches of eight row tiles and a rest
+    (Q6K, 4100, 256, 4129)])
+def test_own_columns_matmul(orn, ctx, kind, O, K, M):
+    rng = np.random.default_rng(O + K + M + kind)
+    t = util.make_kq(kind, rng, 1, O, K)
+    w = orn.KMatrix(ctx, kind, *t, 1, O, K)
+    xb = util.bf16_normal(rng, (M, K))
+    dx, dy = ctx.to_device(xb), ctx.alloc(M * O * 2)
+    ctx.memset(dy, 0xFF, M * O * 2)
+    orn.kq_matmul(ctx, w, dx, M, dy)
+    _check(dy.download(np.uint16, (M, O)), util.bf16_to_f32(xb).astype(np.float64), _deq(kind, t, 1, O, K)[0], (kind, O, K, M))
+    for b in (dx, dy): b.free()
+    w.free()
+
+
+@pytest.mark.parametrize("kind,O,K", [(Q4K, 264, 512), (Q6K, 131, 256), (Q6K, 512, 768), (Q4K, 1032, 2048)])
+def test_own_columns_experts_of_every_height(orn, ctx, kind, O, K):
+    """an expert of each number of 32-row blocks, one row to either side of a block's end, one without rows, one of several tiles"""
+    counts = [1, 31, 32, 33, 64, 65, 97, 128, 129, 161, 192, 193, 225, 256, 257, 0, 555]
+    E, pairs = len(counts), sum(counts)
+    assert pairs >= 80 * E
+    rng = np.random.default_rng(O + K)
+    t = util.make_kq(kind, rng, E, O, K)
+    w = orn.KMatrix(ctx, kind, *t, E, O, K)
+    inds = rng.permutation(np.repeat(np.arange(E), counts)).astype(np.uint32)
+    xb = util.bf16_normal(rng, (pairs, K))
+    plan = ctx.alloc(orn.kq_gather_plan_bytes(pairs, E))
+    di, dx, dy = ctx.to_device(inds), ctx.to_device(xb), ctx.alloc(pairs * O * 2)
+    ctx.memset(dy, 0xFF, pairs * O * 2)
+    orn.kq_gather_matmul(ctx, w, dx, di, pairs, 1, False, plan, True, dy)
+    got, x, deq = dy.download(np.uint16, (pairs, O)), util.bf16_to_f32(xb).astype(np.float64), _deq(kind, t, E, O, K)
+    for e in range(E):
+        sel = np.nonzero(inds == e)[0]
+        if len(sel): _check(got[sel], x[sel], deq[e], (kind, O, K, counts[e]))
+    for b in (plan, di, dx, dy): b.free()
+    w.free()
