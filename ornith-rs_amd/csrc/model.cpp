@@ -16,6 +16,7 @@
 //   state     `max_window` fp32 slots; a captured forward writes the state after
 //             token t into slot t; the live slot afterwards is keep-1.
 #include "model.h"
+#include "norm_device.h"
 
 #include <algorithm>
 #include <cmath>
@@ -27,6 +28,9 @@ static const int kMaxRows = 16;  // activation rows a single forward may carry
 
 // frspec_list.cpp: reads and validates an FR-Spec id file
 int frspec_read_file(const char* path, std::vector<uint32_t>& ids);
+
+// moe.hip
+int add_rms_moe_block_close(ornith_ctx* ctx, const ornith_moe_weights* w, const PreNorm& pre, int T, void* d_out, MoeClose* close);
 
 #define TRY(e)         \
   do {                 \
@@ -205,13 +209,14 @@ static int forward_rows(ornith_model* m, ornith_caches* cc, const uint32_t* d_to
   const int Hk = c.linear_num_key_heads, Hv = c.linear_num_value_heads;
   const int Dk = c.linear_key_head_dim, Dv = c.linear_value_head_dim, K = c.linear_conv_kernel_dim;
   const size_t D = m->conv_dim(), ssz = (size_t)Hv * Dv * Dk;
+  bool closed = true;  // s.x and s.normed are the layer's input
   for (size_t i = 0; i < m->layers.size(); ++i) {
     const Layer& L = m->layers[i];
     LayerCache& lc = cc->layers[i];
-    // From the second layer on the layer's input norm is still owed: x = h + mo of the layer
-    // before, normed = rms_norm(x, input_ln). The first projections of the mixer make it.
+    // Unless the last launch of the layer before has made it (prompts), the layer's input norm is still owed from the second layer
+    // on: x = h + mo of the layer before, normed = rms_norm(x, input_ln). The first projections of the mixer make it.
     const PendingNorm pend{s.h, s.mo, L.input_ln, s.x};
-    const PendingNorm* pp = i > 0 ? &pend : nullptr;
+    const PendingNorm* pp = closed ? nullptr : &pend;
     if (L.linear) {
       const GdnLayer& g = L.gdn;
       const bool dense_ab = g.in_proj_a.mode == ORNITH_LIN_DENSE && g.in_proj_b.mode == ORNITH_LIN_DENSE;
@@ -248,10 +253,15 @@ static int forward_rows(ornith_model* m, ornith_caches* cc, const uint32_t* d_to
                           s.vx, s.q_rot, s.att, pp));
       TRY(ornith_linear_matmul(ctx, &L.attn.o_proj, s.att, T, s.r));
     }
-    TRY(ornith_add_rms_moe_block(ctx, &L.moe, s.x, s.r, L.post_ln, c.rms_norm_eps, T, s.h, s.normed2, s.mo));
+    // the layer's closing add and the norm after it: the next layer's, or the model's final one
+    const bool last = i + 1 == m->layers.size();
+    MoeClose close{{(const bf16_t*)s.h, nullptr, (const bf16_t*)(last ? m->final_norm : m->layers[i + 1].input_ln), (bf16_t*)s.x,
+                    (bf16_t*)(last ? d_hidden_out : s.normed), c.rms_norm_eps}};
+    const PreNorm pre{(const bf16_t*)s.x, (const bf16_t*)s.r, (const bf16_t*)L.post_ln, (bf16_t*)s.h, (bf16_t*)s.normed2, c.rms_norm_eps};
+    TRY(add_rms_moe_block_close(ctx, &L.moe, pre, T, s.mo, ornith_option_fuse_norm() ? &close : nullptr));
+    closed = close.done;
   }
-  // the last layer's closing add and the model's final norm
-  TRY(ornith_add_rms_norm(ctx, s.h, s.mo, m->final_norm, T, H, c.rms_norm_eps, s.x, d_hidden_out));
+  if (!closed) TRY(ornith_add_rms_norm(ctx, s.h, s.mo, m->final_norm, T, H, c.rms_norm_eps, s.x, d_hidden_out));
   // every layer advanced together
   cc->conv_cur = 1 - cc->conv_cur;
   cc->conv_off = T;

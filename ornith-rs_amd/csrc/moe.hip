@@ -128,43 +128,34 @@ __global__ void swiglu_kernel(const bf16_t* gate, const bf16_t* up, bf16_t* out,
   reinterpret_cast<P*>(out)[i] = o8;
 }
 
-// One thread per V output elements of a token; j ascends, every step rounds to bf16. Bound by the stream at long prompts, by one trip
+// V output elements (from c on) of token t: j ascends, every step rounds to bf16. Bound by the stream at long prompts, by one trip
 // to memory at short ones: eight experts' rows, their scores and the rest are asked for at once (past k the last one again,
 // unused), and nothing is divided but by the workgroup. With the scores added up one load after the other ahead of the rows, us, 51 / 700 /
-// 6621 tokens: 5.3 / 10.3 / 62.4 -> 5.0 / 8.3 / 53.
-template <int V>
-__global__ __launch_bounds__(256) void moe_combine_kernel(const bf16_t* scores, const bf16_t* y, const bf16_t* gate,
-                                                          const bf16_t* shared, bf16_t* out, int T, int k, int dim, int normalize) {
+// 6621 tokens: 5.3 / 10.3 / 62.4 -> 5.0 / 8.3 / 53. `more` asks for what the caller needs besides.
+struct CombineArgs {
+  const bf16_t *scores, *y, *gate, *shared;
+  int T, k, dim, normalize;
+};
+template <int V, class F>
+__device__ __forceinline__ typename BfPack<V>::type combine_row(const CombineArgs& a, uint32_t t, uint32_t c, F more) {
   typedef typename BfPack<V>::type P;
-  // (a grid has fewer than 2^32 threads)
-  const uint32_t per_row = dim / V, base = blockIdx.x * 256u, t0 = base / per_row;
-  uint32_t r = base - t0 * per_row + threadIdx.x, t = t0;
-  if (per_row >= 256u) {
-    if (r >= per_row) {
-      r -= per_row;
-      ++t;
-    }
-  } else {
-    t += r / per_row;
-    r %= per_row;
-  }
-  if (t >= (uint32_t)T) return;
-  const uint32_t c = r * V;
-  const bf16_t* s = scores + (size_t)t * k;
+  const int k = a.k;
+  const bf16_t* s = a.scores + (size_t)t * k;
   P yj[8];
   bf16_t sj[8];
   auto fetch = [&](int j0) {
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      yj[j] = *reinterpret_cast<const P*>(y + ((size_t)t * k + min(j0 + j, k - 1)) * dim + c);
+      yj[j] = *reinterpret_cast<const P*>(a.y + ((size_t)t * k + min(j0 + j, k - 1)) * a.dim + c);
       sj[j] = s[min(j0 + j, k - 1)];
     }
   };
   fetch(0);
-  const P sh = *reinterpret_cast<const P*>(shared + (size_t)t * dim + c);
-  const bf16_t gt = gate[t];
+  const P sh = *reinterpret_cast<const P*>(a.shared + (size_t)t * a.dim + c);
+  const bf16_t gt = a.gate[t];
+  more();
   float denom = 0.f;
-  if (normalize) {
+  if (a.normalize) {
 #pragma unroll
     for (int j = 0; j < 8; ++j)
       if (j < k) denom = dm_rb(dm_bf2f(sj[j]) + denom);
@@ -177,7 +168,7 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(const bf16_t* scores, 
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       if (j0 + j >= k) break;
-      const float w = normalize ? dm_rb(dm_bf2f(sj[j]) / denom) : dm_bf2f(sj[j]);
+      const float w = a.normalize ? dm_rb(dm_bf2f(sj[j]) / denom) : dm_bf2f(sj[j]);
 #pragma unroll
       for (int e = 0; e < V; ++e) {
         const float weighted = dm_rb(bf_get<V>(yj[j], e) * w);
@@ -195,7 +186,45 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(const bf16_t* scores, 
     const float gated = dm_rb(g * bf_get<V>(sh, e));
     bf_put<V>(o, e, acc[e] + gated);
   }
-  *reinterpret_cast<P*>(out + (size_t)t * dim + c) = o;
+  return o;
+}
+template <int V>
+__global__ __launch_bounds__(256) void moe_combine_kernel(CombineArgs a, bf16_t* out) {
+  // (a grid has fewer than 2^32 threads)
+  const uint32_t per_row = a.dim / V, base = blockIdx.x * 256u, t0 = base / per_row;
+  uint32_t r = base - t0 * per_row + threadIdx.x, t = t0;
+  if (per_row >= 256u) {
+    if (r >= per_row) {
+      r -= per_row;
+      ++t;
+    }
+  } else {
+    t += r / per_row;
+    r %= per_row;
+  }
+  if (t >= (uint32_t)a.T) return;
+  *reinterpret_cast<typename BfPack<V>::type*>(out + (size_t)t * a.dim + r * V) = combine_row<V>(a, t, r * V, []() {});
+}
+// The same with what follows a block in the model, h = res + out and rms_norm(h): a workgroup of 8 * PER threads a token of 64 * PER values,
+// eight a thread, and the block's output goes nowhere. Bound as the combine is: the norm's streams hide in its wait. The two launches
+// and this one, us, 700 / 6621 tokens of 2048 values: 8.3 + 5.0 / 56 + 18.5 -> 10.4 / 65.7 (a layer; a prompt of 51: 6.37 -> 6.25 ms).
+template <int PER>
+__global__ __launch_bounds__(PER * 8) void moe_combine_norm_kernel(CombineArgs a, PreNorm n) {
+  __shared__ float sums[64];
+  const uint32_t t = blockIdx.x, c = 8 * threadIdx.x;
+  const size_t at = (size_t)t * a.dim + c;
+  float x[8], w[8];
+  const auto o = combine_row<8>(a, t, c, [&]() {
+    load_bf16<8>(n.res + at, x);
+    load_bf16<8>(n.w + c, w);
+  });
+#pragma unroll
+  for (int i = 0; i < 8; ++i) x[i] = dm_rb(x[i] + bf_get<8>(o, i));
+  store_bf16<8>(n.h_out + at, x);
+  const float inv = wide_row_inv<PER>(x, a.dim, n.eps, sums);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) x[i] = dm_rb(w[i] * dm_rb(x[i] * inv));
+  store_bf16<8>(n.normed_out + at, x);
 }
 
 int launch_router(ornith_ctx* ctx, const bf16_t* gates, int T, int E, int k, uint32_t* inds,
@@ -247,11 +276,31 @@ int launch_router_egate(ornith_ctx* ctx, const bf16_t* gates, int T, int E, int 
   return ORNITH_OK;
 }
 
+// The block's last launch: the combine, with `close` the sum and norm that follow it too where the shapes allow (*close->done says so; d_out is
+// not written then).
+int combine_and_close(ornith_ctx* ctx, const void* scores, const void* y, const void* gate, const void* shared, int T, int k, int dim,
+                      int normalize, void* d_out, MoeClose* close) {
+  if (close && (dim == 1024 || dim == 2048 || dim == 4096)) {
+    const PreNorm& n = close->norm;
+    const uintptr_t all = (uintptr_t)y | (uintptr_t)shared | (uintptr_t)n.res | (uintptr_t)n.w | (uintptr_t)n.h_out | (uintptr_t)n.normed_out;
+    if ((all & 15) == 0) {
+      const CombineArgs a{(const bf16_t*)scores, (const bf16_t*)y, (const bf16_t*)gate, (const bf16_t*)shared, T, k, dim, normalize};
+      if (dim == 1024) hipLaunchKernelGGL(moe_combine_norm_kernel<16>, dim3(T), dim3(128), 0, ctx->stream, a, n);
+      else if (dim == 2048) hipLaunchKernelGGL(moe_combine_norm_kernel<32>, dim3(T), dim3(256), 0, ctx->stream, a, n);
+      else hipLaunchKernelGGL(moe_combine_norm_kernel<64>, dim3(T), dim3(512), 0, ctx->stream, a, n);
+      ORN_LAUNCH_CHECK("moe_combine_norm_kernel");
+      close->done = true;
+      return ORNITH_OK;
+    }
+  }
+  return ornith_moe_combine(ctx, scores, y, gate, shared, T, k, dim, normalize, d_out);
+}
+
 // Prompts of few rows an expert (and a layer's prompt over affine experts, which have no wide form): the
 // shared expert is one more expert of the pair list, so the block is six launches: router, its
 // tail (shared gate, softmax + top-k), plan, gate + up + swiglu, down, combine.
 // false: the shapes are not covered.
-bool moe_block_narrow(ornith_ctx* ctx, const ornith_moe_weights* w, const void* d_x, int T, void* d_out, int* rc_out) {
+bool moe_block_narrow(ornith_ctx* ctx, const ornith_moe_weights* w, const void* d_x, int T, void* d_out, MoeClose* close, int* rc_out) {
   const int E = w->router.O, H = w->router.K, I = w->ex_gate.O, k = w->top_k, pairs = T * k;
   if (E % 64 != 0 || E > 1024) return false;
   const int rows = nmm::tile_rows(pairs, E);
@@ -281,7 +330,7 @@ bool moe_block_narrow(ornith_ctx* ctx, const ornith_moe_weights* w, const void* 
     TRY(moe_plan(ctx, inds, pairs, E, rows, T, plan, true, &pl));
     TRY(nmm::gate_up(ctx, w, d_x, pairs, pl, act));
     TRY(nmm::gathered(ctx, &w->ex_down, &w->sh_down, act, pairs, 1, pl, y));
-    TRY(ornith_moe_combine(ctx, scores, y, eg, y + (size_t)pairs * H, T, k, H, w->norm_topk_prob, d_out));
+    TRY(combine_and_close(ctx, scores, y, eg, y + (size_t)pairs * H, T, k, H, w->norm_topk_prob, d_out, close));
 #undef TRY
     return ORNITH_OK;
   };
@@ -292,7 +341,7 @@ bool moe_block_narrow(ornith_ctx* ctx, const ornith_moe_weights* w, const void* 
 // Prefill widths: the same block with every projection as a matrix-core GEMM and the routed
 // experts as three expert-grouped GEMMs over one sorted pair list
 // (/root/reference/src/ops/moe.rs:662-741 at T above the exact window; gather_qmm_t).
-int moe_block_prefill(ornith_ctx* ctx, const ornith_moe_weights* w, const void* d_x, int T, void* d_out) {
+int moe_block_prefill(ornith_ctx* ctx, const ornith_moe_weights* w, const void* d_x, int T, void* d_out, MoeClose* close) {
   const int E = w->router.O, H = w->router.K, I = w->ex_gate.O, k = w->top_k, SI = w->sh_gate.O;
   const int pairs = T * k;
   const size_t plan_bytes = ornith_kq_gather_plan_bytes(pairs, E);
@@ -335,7 +384,7 @@ int moe_block_prefill(ornith_ctx* ctx, const ornith_moe_weights* w, const void* 
   TRY(ornith_kq_gather_matmul(ctx, &w->ex_up, d_x, inds, pairs, k, 1, plan, 0, xu));
   TRY(ornith_swiglu(ctx, xg, xu, (int64_t)pairs * I, act));
   TRY(ornith_kq_gather_matmul(ctx, &w->ex_down, act, inds, pairs, k, 0, plan, 0, y));
-  TRY(ornith_moe_combine(ctx, scores, y, eg, sy, T, k, H, w->norm_topk_prob, d_out));
+  TRY(combine_and_close(ctx, scores, y, eg, sy, T, k, H, w->norm_topk_prob, d_out, close));
 #undef TRY
   return ORNITH_OK;
 }
@@ -394,14 +443,11 @@ int ornith_moe_combine(ornith_ctx* ctx, const void* d_scores, const void* d_y, c
   ORN_REQUIRE(ctx && d_scores && d_y && d_gate && d_shared && d_out, "moe_combine: null argument");
   ORN_REQUIRE(T >= 1 && k >= 1 && dim >= 1, "moe_combine: T=%d k=%d dim=%d", T, k, dim);
   const int64_t n = (int64_t)T * dim;
+  const CombineArgs a{(const bf16_t*)d_scores, (const bf16_t*)d_y, (const bf16_t*)d_gate, (const bf16_t*)d_shared, T, k, dim, normalize};
   if (dim % 8 == 0 && (((uintptr_t)d_y | (uintptr_t)d_shared | (uintptr_t)d_out) & 15) == 0)
-    hipLaunchKernelGGL(moe_combine_kernel<8>, dim3((unsigned)((n / 8 + 255) / 256)), dim3(256), 0,
-                       ctx->stream, (const bf16_t*)d_scores, (const bf16_t*)d_y, (const bf16_t*)d_gate,
-                       (const bf16_t*)d_shared, (bf16_t*)d_out, T, k, dim, normalize);
+    hipLaunchKernelGGL(moe_combine_kernel<8>, dim3((unsigned)((n / 8 + 255) / 256)), dim3(256), 0, ctx->stream, a, (bf16_t*)d_out);
   else
-    hipLaunchKernelGGL(moe_combine_kernel<1>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
-                       ctx->stream, (const bf16_t*)d_scores, (const bf16_t*)d_y, (const bf16_t*)d_gate,
-                       (const bf16_t*)d_shared, (bf16_t*)d_out, T, k, dim, normalize);
+    hipLaunchKernelGGL(moe_combine_kernel<1>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, ctx->stream, a, (bf16_t*)d_out);
   ORN_LAUNCH_CHECK("moe_combine_kernel");
   return ORNITH_OK;
 }
@@ -413,7 +459,8 @@ int ornith_moe_combine(ornith_ctx* ctx, const void* d_scores, const void* d_y, c
 // point, not to the outputs asked for: ornith_moe_block, which gives ids and scores on demand, keeps
 // these experts exact at every width, so that asking does not change the result.
 static int moe_block_impl(ornith_ctx* ctx, const ornith_moe_weights* w, const void* d_x, int T,
-                          void* d_out, uint32_t* d_inds_out, void* d_scores_out, const PreNorm* pre, bool gemm_affine) {
+                          void* d_out, uint32_t* d_inds_out, void* d_scores_out, const PreNorm* pre, bool gemm_affine,
+                          MoeClose* close = nullptr) {
   ORN_REQUIRE(ctx && w && d_x && d_out, "moe_block: null argument");
   const int E = w->router.O, H = w->router.K, I = w->ex_gate.O, k = w->top_k;
   ORN_REQUIRE(T >= 1 && T <= 8192, "moe_block: T=%d", T);
@@ -446,11 +493,11 @@ static int moe_block_impl(ornith_ctx* ctx, const ornith_moe_weights* w, const vo
                 "moe_block: the three expert stacks must share the 4-bit affine format");
   if (T >= kPrefillRows && !w->ex_dense && (ex_affine4 ? gemm_affine : !d_inds_out && !d_scores_out)) {
     int rcn = ORNITH_OK;
-    if (moe_block_narrow(ctx, w, d_x, T, d_out, &rcn)) return rcn;
+    if (moe_block_narrow(ctx, w, d_x, T, d_out, close, &rcn)) return rcn;
   }
   if (T >= kPrefillRows && !w->ex_dense && !ex_affine4) {
     ORN_REQUIRE(!d_inds_out && !d_scores_out, "moe_block: index outputs are a decode-width feature");
-    return moe_block_prefill(ctx, w, d_x, T, d_out);
+    return moe_block_prefill(ctx, w, d_x, T, d_out, close);
   }
   // dense experts have no prefill-width form, affine ones none that is exact: the rows go in blocks
   // of 64 (they are independent of each other, so the result is the same)
@@ -581,6 +628,15 @@ static int moe_block_impl(ornith_ctx* ctx, const ornith_moe_weights* w, const vo
 #undef TRY
   return ORNITH_OK;
 }
+
+}  // extern "C"
+
+// ornith_add_rms_moe_block with what follows it in the model, if that could ride along (close->done)
+int add_rms_moe_block_close(ornith_ctx* ctx, const ornith_moe_weights* w, const PreNorm& pre, int T, void* d_out, MoeClose* close) {
+  return moe_block_impl(ctx, w, pre.normed_out, T, d_out, nullptr, nullptr, &pre, true, close);
+}
+
+extern "C" {
 
 int ornith_moe_block(ornith_ctx* ctx, const ornith_moe_weights* w, const void* d_x, int T,
                      void* d_out, uint32_t* d_inds_out, void* d_scores_out) {

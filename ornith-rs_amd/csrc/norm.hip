@@ -10,9 +10,7 @@
 // per thread, because a single wavefront walking 32 or 64 values per lane through the
 // add / round / scale / round steps is a chain of thousands of dependent instructions.
 // The element-wise steps are spread over the workgroup; only the sum of squares keeps
-// its defined order (lane l of the first wavefront owns [l*PER, (l+1)*PER), one fma
-// chain, butterfly), reading the values from LDS laid out so that lane l's i-th value
-// sits at [i][l].
+// its defined order (lane l of a wavefront owns [l*PER, (l+1)*PER), one fma chain, butterfly), handed from thread to thread.
 #include "norm_device.h"
 #include "rt.h"
 
@@ -63,8 +61,7 @@ __global__ __launch_bounds__(PER * 8) void rms_wide_kernel(const bf16_t* a, cons
                                                            const bf16_t* w, bf16_t* h_out,
                                                            bf16_t* out, int n, float eps) {
   static_assert(PER % 8 == 0 && MODE != NORM_GATED, "wide rows: plain and add only");
-  __shared__ float xs[PER * 64];
-  __shared__ float s_inv;
+  __shared__ float sums[64];
   const size_t off = (size_t)blockIdx.x * n;
   const int tid = threadIdx.x, e0 = tid * 8;
   float x[8], wv[8];
@@ -77,23 +74,7 @@ __global__ __launch_bounds__(PER * 8) void rms_wide_kernel(const bf16_t* a, cons
     for (int i = 0; i < 8; ++i) x[i] = dm_rb(x[i] + y[i]);
     store_bf16<8>(h_out + off + e0, x);
   }
-  // value e belongs to lane e / PER, position e % PER
-  const int lane_of = e0 / PER, pos0 = e0 % PER;
-#pragma unroll
-  for (int i = 0; i < 8; ++i) xs[(pos0 + i) * 64 + lane_of] = x[i];
-  __syncthreads();
-  if (tid < 64) {
-    float acc = 0.f;
-#pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      const float v = xs[i * 64 + tid];
-      acc = dm_fma(v, v, acc);
-    }
-    const float inv = dm_rsqrt(dm_wave_sum<64>(acc) / (float)n + eps);
-    if (tid == 0) s_inv = inv;
-  }
-  __syncthreads();
-  const float inv = s_inv;
+  const float inv = wide_row_inv<PER>(x, n, eps, sums);
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
     x[i] = dm_rb(x[i] * inv);

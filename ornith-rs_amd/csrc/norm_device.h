@@ -114,6 +114,13 @@ struct PreNorm {
   float eps;
 };
 
+// What follows a MoE block in the model, h_out = res + the block's output and normed_out = rms_norm(h_out) (y is not used), for the
+// block's last launch to make where it can: then `done`, and the block's output is not written.
+struct MoeClose {
+  PreNorm norm;
+  bool done = false;
+};
+
 constexpr int kPreN = 2048;
 
 // Host: whether n1 bytes at a and n2 bytes at b have one in common.
@@ -275,4 +282,25 @@ __device__ __forceinline__ void prenorm_rows(const PreNorm& p, bool write_global
   PreNormRegs<T> g;
   prenorm_issue<T>(p, g);
   prenorm_finish<T, COH>(p, g, write_global, s);
+}
+
+// 1 / sqrt(mean square + eps) of a row of 64 * PER values that a workgroup of 8 * PER threads holds, eight each: the sum in rms_row's
+// order. The PER / 8 threads that hold a lane's piece hand its chain of fmas on from one to the next (row_shr:1; a thread's
+// result counts in the step in which it is the next one), and every wavefront makes the butterfly over the 64 sums: one barrier, and
+// no value goes through LDS.
+template <int PER>
+__device__ __forceinline__ float wide_row_inv(const float (&x)[8], int n, float eps, float* sums) {
+  constexpr int G = PER / 8;
+  static_assert(G >= 1 && G <= 16, "a piece's threads stand in one row of sixteen lanes");
+  float acc = 0.f;
+#pragma unroll
+  for (int s = 0; s < G; ++s) {
+    if (s) acc = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, acc), 0x111, 0xF, 0xF, false));
+#pragma unroll
+    for (int i = 0; i < 8; ++i) acc = dm_fma(x[i], x[i], acc);
+  }
+  const int tid = threadIdx.x;
+  if ((tid & (G - 1)) == G - 1) sums[tid / G] = acc;
+  __syncthreads();
+  return dm_rsqrt(dm_wave_sum<64>(sums[tid & 63]) / (float)n + eps);
 }

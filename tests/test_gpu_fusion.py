@@ -407,3 +407,29 @@ def test_norm_and_its_consumers_in_place(orn, ctx, fmt, T):
     for b in bufs + [wn]: b.free()
     for l in lins: l.free()
     moe.free()
+
+
+@pytest.mark.parametrize("H,k,T", [(1024, 8, 33), (2048, 10, 90), (4096, 8, 40), (2048, 8, 700)])
+def test_norm_inside_combine_launch_equals_separate(orn, ctx, H, k, T):
+    """The residual add and the norm after a prompt's MoE block, made by its combine launch, == the launches of
+    their own: the same bits of every row and of the decode step that follows (caches), through both forms of the
+    block (T = 700: tall expert groups)."""
+    import synth
+    cfg = dict(synth.TINY, hidden_size=H, num_experts_per_tok=k, num_hidden_layers=2, full_attention_interval=2)
+    s = synth.SynthModel(cfg, seed=H + T, with_mtp=False, with_oracle=False)
+    ws = s.upload(orn, ctx)
+    model = orn.TextModel(ctx, ws, s.text_config(orn))
+    model.set_max_rows(T)
+    toks = np.random.default_rng(T).integers(0, cfg["vocab_size"], T).astype(np.uint32)
+    got = []
+    try:
+        for fuse in (1, 0):
+            orn.set_option("fuse_norm", fuse)
+            cache = model.make_cache(T + 8, 2)
+            got.append((model.forward(cache, toks), model.forward(cache, toks[:1])))
+            cache.close()
+        for a, b in zip(*got):
+            assert np.array_equal(a, b)
+    finally:
+        orn.set_option("fuse_norm", 1)
+        for o in (model, ws): o.close()
