@@ -617,7 +617,7 @@ int ornith_kq_matmul_multi(ornith_ctx* ctx, const ornith_kmatrix* const* ws, int
   ORN_REQUIRE(M >= 1, "kq_matmul: M=%d", M);
   ORN_REQUIRE(((uintptr_t)d_x & 15) == 0, "kq_matmul: x must be 16-byte aligned");
   MmArgs a{};
-  OwnArgs own{};
+  OwnArgs own[2] = {};  // those that take halves of K go by themselves
   int nx = 0, rest = 0;
   bool mixed = false;
   a.vec = 1;
@@ -630,7 +630,8 @@ int ornith_kq_matmul_multi(ornith_ctx* ctx, const ornith_kmatrix* const* ws, int
   }
   for (int i = 0; i < n; ++i) {
     if (ornith_option_gemm_duo() && kq_mm_own_suits(*ws[i], d_x, M)) {
-      own.m[own.n++] = kq_mm_own_mat(*ws[i], d_ys[i]);
+      OwnArgs& o = own[kq_mm_own_halves(*ws[i], M)];
+      o.m[o.n++] = kq_mm_own_mat(*ws[i], d_ys[i]);
       continue;
     }
     a.vec = a.vec && ws[i]->O % 8 == 0 && ((uintptr_t)d_ys[i] & 15) == 0;
@@ -649,13 +650,16 @@ int ornith_kq_matmul_multi(ornith_ctx* ctx, const ornith_kmatrix* const* ws, int
     nx += (ws[i]->O + BN - 1) / BN;
     ++rest;
   }
-  if (own.n) {
-    own.x = (const bf16_t*)d_x;
-    own.M = M;
-    own.K = ws[0]->K;
-    const int rc = kq_mm_own(ctx, own, false);
-    if (rc || !rest) return rc;
+  for (const bool halves : {false, true}) {
+    OwnArgs& o = own[halves];
+    if (!o.n) continue;
+    o.x = (const bf16_t*)d_x;
+    o.M = M;
+    o.K = ws[0]->K;
+    o.halves = halves;
+    if (const int rc = kq_mm_own(ctx, o, false)) return rc;
   }
+  if (!rest) return ORNITH_OK;
   a.nseg = rest - 1;
   a.x = (const bf16_t*)d_x;
   a.M = M;

@@ -17,6 +17,7 @@ struct OwnArgs {
   int n;
   const bf16_t* x;
   int M, K;
+  bool halves;  // plain form: the matrices are of kq_mm_own_halves
   int tile_rows, row_tiles, col_tiles;  // set by kq_mm_own
   // gathered form: tiles of up to kOwnRows pairs of an expert-sorted list
   const uint32_t *pair, *tile_expert, *tile_start, *tile_count, *n_tiles;
@@ -32,5 +33,7 @@ constexpr int kOwnRows = 256, kOwnCols = 256;  // a workgroup's tile
 bool kq_mm_own_ok(const ornith_kmatrix& w, const void* x, size_t rows);
 // ... and M rows are many enough for this matrix, whatever shares its launch
 bool kq_mm_own_suits(const ornith_kmatrix& w, const void* x, int M);
+// ... and then whether its sums are taken in two halves of K
+bool kq_mm_own_halves(const ornith_kmatrix& w, int M);
 OwnMat kq_mm_own_mat(const ornith_kmatrix& w, void* y);
 int kq_mm_own(ornith_ctx* ctx, OwnArgs& a, bool gather);

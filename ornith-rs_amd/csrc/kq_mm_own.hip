@@ -17,15 +17,23 @@
 // requests. The order is fixed in the source (sched_barrier after each piece) and every wait for memory is counted by hand: requests
 // are inline assembly, because waits that the compiler places at a loop's end are for everything in flight.
 //
+// Shorter prompts (kHalves): tiles of 128 columns by up to 128 rows and two such sets of wavefronts, each over half of K, whose sums meet
+// in LDS at the end. With few rows a tile the unpacking is the work, and a wavefront alone on its SIMD issues one instruction every 5
+// to 8 clocks (two share 4), so a step of 64 columns costs as much as 8 row blocks' matrix instructions whether there are 2 or 5: half
+// the columns a wavefront and twice the wavefronts are 2.2 times as fast a tile (K = 2048, 2 / 4 row blocks 25 / 32 -> 15 / 20 us, K = 4096 42 / 56 -> 23 /
+// 30). Four stages of activations with two super-blocks of codes in flight gave nothing, nor did eight wavefronts of 32 columns over
+// all of K (K = 4096, 2 row blocks 38).
+//
 // What bounds it: at full size the matrix cores at the clock the card holds under them (12288 x 2048, 6621 rows: a step takes 0.39 us
 // with every compute unit at work and 0.29 with one; the same loop over weights that are bf16 already, no vector work at all,
-// reaches 1157 TFLOP/s there, this one 1130 to 1157); below about 128 rows a tile the unpacking (0.16 us a step however few the rows);
+// reaches 1157 TFLOP/s there, this one 1130 to 1157); below about 160 rows a tile the unpacking (0.14 us a step however few the rows);
 // and 3 us of way in and 3.5 us of way out a tile, which nothing overlaps.
 //
 // Measured, us, against the producer / consumer form this replaces (256 x 128 tiles, weights through LDS): 12288 x 2048 Q4_K at 700 / 1500 /
 // 6621 rows 54 / 103 / 357 -> 41 / 77 / 278 (867 -> 1157 TFLOP/s), 2048 x 4096 at 6621 138 -> 96, q / k / v (9216 x 2048 Q6_K) at 700 / 6621 58 / 293 -> 38 /
 // 242, router + shared gate + up at 6621 83 -> 44; and against tiles of 192 rows with activations through registers, the experts of
-// 6621 tokens (207 rows each): gate or up 165 -> 121, down (K = 512) 274 -> 201.
+// 6621 tokens (207 rows each): gate or up 165 -> 121, down (K = 512) 274 -> 201. With kHalves, against the few-row kernels and kFour: 12288 x 2048
+// Q4_K at 129 / 200 rows 25 / 25 -> 18 / 20, 2048 x 4096 Q4_K at 600 / 1200 / 2000 30 / 44 / 46 -> 25 / 29 / 39, Q6_K 36 / 53 / 55 -> 28 / 33 / 42.
 #include <type_traits>
 
 #include "kq_mm_own.h"
@@ -33,6 +41,7 @@
 namespace {
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 typedef unsigned int u32x2_t __attribute__((ext_vector_type(2)));
 typedef unsigned int u32x3_t __attribute__((ext_vector_type(3)));
@@ -252,33 +261,41 @@ struct Deq {
   }
 };
 
+// How a workgroup's wavefronts divide its tile: four of 64 columns, or two sets of four of 32 columns that have half of K each
+enum { kFour, kHalves };
+constexpr int tn_of(int form) { return form == kFour ? 2 : 1; }
+constexpr int threads_of(int form) { return form == kFour ? 256 : 512; }
+constexpr int cols_of(int form) { return form == kHalves ? 128 : kOwnCols; }
+constexpr int rows_of(int form) { return form == kHalves ? 128 : kOwnRows; }
+
 constexpr int kStages = 3;                          // of 64 k: 128 bytes of a row
-constexpr int kActs = kStages * kOwnRows * 128;      // LDS: activations, then a part for each wavefront's codes
+constexpr int kActs = kStages * kOwnRows * 128;      // LDS: activations (kHalves: a half for each set), then a part for each wavefront's codes
 constexpr int kLds = kActs + kOwnCols * 192;
 
-template <int KIND, int TM, bool GATHER>
+template <int KIND, int TM, int FORM, bool GATHER>
 __device__ __forceinline__ void own_tile(const OwnArgs& a, const OwnMat& mt, uint8_t* smem, uint32_t* s_dst, int n0, int rows, int m0,
                                          int64_t wrow0, const uint32_t* pairs) {
   typedef Fmt<KIND> F;
-  constexpr int STAGE = TM * 4096, TN = 2, SL = TN * TM;
+  constexpr int TN = tn_of(FORM), STAGE = TM * 4096, SL = TN * TM;
   constexpr int NC = TN * (F::kInstr + 2);  // requests of a super-block's weights
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l32 = lane & 31, h = lane >> 5;
-  const int nb = a.K >> 8;
+  const int tid = threadIdx.x, lane = tid & 63, wave_of = __builtin_amdgcn_readfirstlane(tid >> 6), l32 = lane & 31, h = lane >> 5;
+  const int wave = wave_of & 3, set = wave_of >> 2, row_blocks = a.K >> 8, nb = FORM == kHalves ? row_blocks / 2 : row_blocks, b0 = set * nb;
   uint32_t qo[TN][F::kInstr], so[TN], dof[TN];
 #pragma unroll
   for (int j = 0; j < TN; ++j) {
-    const int r0 = n0 + 64 * wave + 32 * j;
+    const int r0 = n0 + 32 * TN * wave + 32 * j;
 #pragma unroll
     for (int i = 0; i < F::kInstr; ++i) {
       int row, p;
       F::source(64 * i + lane, row, p);
-      qo[j][i] = (uint32_t)min(r0 + row, mt.O - 1) * (uint32_t)(nb * F::kQ) + 16 * p;
+      qo[j][i] = (uint32_t)min(r0 + row, mt.O - 1) * (uint32_t)(row_blocks * F::kQ) + 16 * p;
     }
-    const uint32_t row = (uint32_t)min(r0 + l32, mt.O - 1) * (uint32_t)nb;
+    const uint32_t row = (uint32_t)min(r0 + l32, mt.O - 1) * (uint32_t)row_blocks;
     so[j] = row * F::kS;
     dof[j] = row * F::kD;
   }
-  const uint8_t *qb = uniform(mt.qs + wrow0 * nb * F::kQ), *sb = uniform(mt.scales + wrow0 * nb * F::kS), *db = uniform(mt.dm + wrow0 * nb * F::kD);
+  const uint8_t *qb = uniform(mt.qs + (wrow0 * row_blocks + b0) * F::kQ), *sb = uniform(mt.scales + (wrow0 * row_blocks + b0) * F::kS),
+                *db = uniform(mt.dm + (wrow0 * row_blocks + b0) * F::kD);
   __builtin_amdgcn_sched_barrier(0);
   // request i of a slab's activations: eight rows of row block i, 128 bytes each
   uint32_t pr[TM];
@@ -291,7 +308,7 @@ __device__ __forceinline__ void own_tile(const OwnArgs& a, const OwnMat& mt, uin
 #pragma unroll
     for (int i = 0; i < TM; ++i) pr[i] = m0 + min(32 * i + 8 * wave + (lane >> 3), rows - 1);
   }
-  uint8_t* const mine = smem + kActs + wave * (64 * F::kQ);
+  uint8_t* const mine = smem + kActs + wave_of * (32 * TN * F::kQ);
   const uint32_t mine_at = lds_address(mine);
   Sc<KIND> cur[TN], nxt[TN];
   auto weights = [&](Sc<KIND> (&z)[TN], const uint8_t* q0, const uint8_t* s0, const uint8_t* d0, auto ic) {
@@ -314,8 +331,8 @@ __device__ __forceinline__ void own_tile(const OwnArgs& a, const OwnMat& mt, uin
     asm volatile("" : "+v"(at));  // (or its sum becomes a 64-bit multiply-add that names registers still to be filled)
     xo[i] = at + 16 * ((lane & 7) ^ ((4 * wave + (lane >> 4)) & 7));
   }
-  const uint8_t* xg = reinterpret_cast<const uint8_t*>(a.x);
-  const uint32_t at = lds_address(smem) + wave * 1024;
+  const uint8_t* xg = reinterpret_cast<const uint8_t*>(a.x) + 512 * b0;
+  const uint32_t mem = set * (kActs / 2), at = lds_address(smem) + mem + wave * 1024;
 #pragma unroll
   for (int s = 0; s < kStages; ++s)
 #pragma unroll
@@ -331,7 +348,7 @@ __device__ __forceinline__ void own_tile(const OwnArgs& a, const OwnMat& mt, uin
   // step T's fragment of row block i: piece 4 ((T >> 1) & 1) + 2 h + (T & 1) of the slab's 128 bytes, which lie turned by the row
   uint32_t rd[4];
 #pragma unroll
-  for (int t = 0; t < 4; ++t) rd[t] = l32 * 128 + 16 * ((4 * (t >> 1) + 2 * h + (t & 1)) ^ ((l32 >> 1) & 7));
+  for (int t = 0; t < 4; ++t) rd[t] = mem + l32 * 128 + 16 * ((4 * (t >> 1) + 2 * h + (t & 1)) ^ ((l32 >> 1) & 7));
   uint32_t st = 0;  // stage of the slab
   auto after = [](uint32_t s) { return s == 2 * STAGE ? 0u : s + STAGE; };
   bf16x8_t af[TM], bf[2][TN];
@@ -423,17 +440,39 @@ __device__ __forceinline__ void own_tile(const OwnArgs& a, const OwnMat& mt, uin
     sb += F::kS;
     db += F::kD;
   }
+  if constexpr (FORM == kHalves) {
+    // each set finishes every other row block, and hands the other its part of the rest
+    barrier_only();
+    f32x4_t* const part = reinterpret_cast<f32x4_t*>(smem) + (size_t)wave * TM * 256 + lane;
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+      if ((i & 1) != set)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) part[i * 256 + e * 64] = f32x4_t{acc[i][0][4 * e], acc[i][0][4 * e + 1], acc[i][0][4 * e + 2], acc[i][0][4 * e + 3]};
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    barrier_only();
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+      if ((i & 1) == set)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const f32x4_t v = part[i * 256 + e * 64];
+#pragma unroll
+          for (int f = 0; f < 4; ++f) acc[i][0][4 * e + f] += v[f];
+        }
+  }
   // D[n = 8 b + 4 h + r][m = l32]: two swaps of lanes bring 32 columns of a row into four lanes, 16 bytes each
   const int half = 16 * ((lane >> 4) & 1) + 8 * h;
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
+    if (FORM == kHalves && (i & 1) != set) continue;
     bf16_t* y[2];
     bool live[2];
 #pragma unroll
     for (int b = 0; b < 2; ++b) {
       const int r = 32 * i + 16 * b + (lane & 15);
       live[b] = r < rows;
-      y[b] = mt.y + (size_t)(GATHER ? s_dst[r] : (uint32_t)(m0 + r)) * mt.O + n0 + 64 * wave + half;
+      y[b] = mt.y + (size_t)(GATHER ? s_dst[r] : (uint32_t)(m0 + r)) * mt.O + n0 + 32 * TN * wave + half;
     }
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
@@ -451,7 +490,7 @@ __device__ __forceinline__ void own_tile(const OwnArgs& a, const OwnMat& mt, uin
         v[0][e] = p[0];
         v[1][e] = p[1];
       }
-      const int left = mt.O - (n0 + 64 * wave + 32 * j + half);
+      const int left = mt.O - (n0 + 32 * TN * wave + 32 * j + half);
 #pragma unroll
       for (int b = 0; b < 2; ++b)
         if (live[b] && left > 0) {
@@ -467,8 +506,8 @@ __device__ __forceinline__ void own_tile(const OwnArgs& a, const OwnMat& mt, uin
 }
 
 constexpr int kMixed = 2;  // the matrices of the launch differ in kind
-template <int KIND, bool GATHER>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void kq_mm_own_kernel(OwnArgs a) {
+template <int KIND, int FORM, bool GATHER>
+__global__ __launch_bounds__(threads_of(FORM)) __attribute__((amdgpu_waves_per_eu(threads_of(FORM) / 256, threads_of(FORM) / 256))) void kq_mm_own_kernel(OwnArgs a) {
   __shared__ __attribute__((aligned(1024))) uint8_t smem[kLds];
   __shared__ uint32_t s_dst[GATHER ? kOwnRows : 1];
   int rows, m0 = 0, tc, mat = 0;
@@ -503,16 +542,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
       if (i < a.n && tc >= a.m[i].t0) mat = i;
   }
   const OwnMat mt = a.m[mat];
-  const int n0 = (tc - mt.t0) * kOwnCols;
+  const int n0 = (tc - mt.t0) * cols_of(FORM);
   const int groups = (rows + 31) >> 5;
   auto of_kind = [&](auto kc) {
     constexpr int KD = decltype(kc)::value;
-#define OWN(N) own_tile<KD, N, GATHER>(a, mt, smem, s_dst, n0, rows, m0, wrow0, pairs)
-    if (groups >= 8) OWN(8);
-    else if (groups == 7) OWN(7);
-    else if (groups == 6) OWN(6);
-    else if (groups == 5) OWN(5);
-    else if (groups == 4) OWN(4);
+#define OWN(N) own_tile<KD, N, FORM, GATHER>(a, mt, smem, s_dst, n0, rows, m0, wrow0, pairs)
+    if constexpr (FORM == kFour) {
+      if (groups >= 8) return OWN(8);
+      if (groups == 7) return OWN(7);
+      if (groups == 6) return OWN(6);
+      if (groups == 5) return OWN(5);
+    }
+    if (groups >= 4) OWN(4);
     else if (groups == 3) OWN(3);
     else OWN(2);
 #undef OWN
@@ -530,13 +571,20 @@ bool kq_mm_own_ok(const ornith_kmatrix& w, const void* x, size_t rows) {
 }
 
 // Rows from which a matrix runs here. Fewer take the few-row kernels (up to the lines of mm_narrow_host.h), whose splits suit
-// them: this form's step has a floor, so that a tile of any height takes 24 us at K = 2048 and 43 at 4096. us, there / here: 8192 + 4096
-// columns of K = 2048, Q4_K, 150 / 200 / 300 rows 24 / 25, 27 / 26, 30 / 27; 2048 x 4096 Q4_K at 1500 / 2000 45 / 45, 56 / 47, Q6_K at 1000 /
-// 1200 47 / 54, 57 / 55; 256 x 2048 Q6_K at 2000 / 3000 18 / 28, 29 / 28. Few slabs: 4096 x 1024 at 512 / 700 rows 12 / 15, 16 / 15; 2048 x 512 Q6_K at 2000 / 2500
-// rows 11 / 12, 15 / 14 (there: the 128-row tiles of kq_mm.hip).
+// them, or kq_mm.hip's 128-row tiles. us, there / here: 8192 + 4096 columns of K = 2048, Q4_K, 100 / 129 rows 18 / 18, 25 / 18; 8192 + 512 + 512 Q6_K, where
+// the narrow two then want a launch of their own, 192 / 200 rows 23 / 24, 35 / 25; 2048 x 4096 Q4_K at 512 / 513 21 / 24, 30 / 24, Q6_K 25 / 28,
+// 36 / 28; 256 x 2048 Q6_K at 2000 / 3000 18 / 28, 29 / 28. Few slabs: 4096 x 1024 at 100 / 200 rows 7 / 9, 16 / 9; 2048 x 512 Q6_K at 2000 / 2500 rows 11 / 12,
+// 15 / 14.
 bool kq_mm_own_suits(const ornith_kmatrix& w, const void* x, int M) {
-  const int from = w.K < 2048 ? (w.O > 2048 ? 512 : 2048) : w.O > 2048 ? 192 : w.O > 256 ? 1024 : 2048;
+  const int from = w.O > 2048 ? (w.kind == ORNITH_Q4K ? 128 : 192) : w.K < 2048 ? 2048 : w.O > 512 ? 512 : w.O > 256 ? 1024 : 2048;
   return M > from && kq_mm_own_ok(w, x, M);
+}
+
+// ... and those that do it in kHalves, one matrix at a time whatever shares the launch, for the sums' order: while its tiles of 128
+// rows are one round of workgroups. us, kFour / kHalves: 8192 + 4096 columns of K = 2048, Q4_K, 200 / 256 / 300 rows 25 / 20, 27 / 21, 27 / 32;
+// 2048 x 4096 Q4_K at 1500 / 2000 / 2400 rows 43 / 32, 46 / 39, 47 / 53. Up to 512 columns are left to the launch of the wide matrices beside them.
+bool kq_mm_own_halves(const ornith_kmatrix& w, int M) {
+  return w.K % 512 == 0 && (w.O > 2048 ? M <= 256 : w.O > 512 && M <= 2048);
 }
 
 OwnMat kq_mm_own_mat(const ornith_kmatrix& w, void* y) {
@@ -544,33 +592,39 @@ OwnMat kq_mm_own_mat(const ornith_kmatrix& w, void* y) {
 }
 
 int kq_mm_own(ornith_ctx* ctx, OwnArgs& a, bool gather) {
-  int kind = a.m[0].kind, grid;
+  int kind = a.m[0].kind, grid, threads = 256;
   typedef void (*Kernel)(OwnArgs);
   Kernel k;
   if (gather) {
     a.up_magic = (uint32_t)(((uint64_t(1) << 32) + a.up_div - 1) / a.up_div);
     a.col_tiles = (a.m[0].O + kOwnCols - 1) / kOwnCols;
     grid = a.col_tiles * ((a.tiles_max + 7) / 8 * 8);
-    k = kind == ORNITH_Q4K ? kq_mm_own_kernel<ORNITH_Q4K, true> : kq_mm_own_kernel<ORNITH_Q6K, true>;
+    k = kind == ORNITH_Q4K ? kq_mm_own_kernel<ORNITH_Q4K, kFour, true> : kq_mm_own_kernel<ORNITH_Q6K, kFour, true>;
   } else {
+    // Tile height: a tile takes about as long as 6 + its row blocks (kFour; K = 2048, one tile a compute unit, us: 8 blocks 53, 7 49, 6 44,
+    // 5 42; K = 4096 8 82, 5 61, 2 42), in the same measure 2.7 + 0.675 of them (kHalves; K = 2048 2 blocks 15, 3 18, 4 20; K = 4096 23, 27, 30),
+    // and the rounds of tiles count.
+    const int form = a.halves ? kHalves : kFour;
+    threads = threads_of(form);
     a.col_tiles = 0;
     for (int i = 0; i < a.n; ++i) {
       a.m[i].t0 = a.col_tiles;
-      a.col_tiles += (a.m[i].O + kOwnCols - 1) / kOwnCols;
+      a.col_tiles += (a.m[i].O + cols_of(form) - 1) / cols_of(form);
       if (a.m[i].kind != kind) kind = kMixed;
     }
-    // Tile height: a tile takes about as long as 6 + its row blocks (K = 2048, one tile a compute unit, us: 8 blocks 53, 7 49, 6 44, 5 42;
-    // K = 4096 8 82, 5 61, 2 45), and the rounds of tiles count.
     long best = 0;
-    for (int tm = 8; tm >= 2; --tm) {
-      const long tiles = (long)((a.M + 32 * tm - 1) / (32 * tm)) * a.col_tiles, cost = (tiles + ctx->compute_units - 1) / ctx->compute_units * (tm + 6);
-      if (tm == 8 || cost < best) best = cost, a.tile_rows = 32 * tm;
+    for (int tm = rows_of(form) / 32; tm >= 2; --tm) {
+      const long tiles = (long)((a.M + 32 * tm - 1) / (32 * tm)) * a.col_tiles, rounds = (tiles + ctx->compute_units - 1) / ctx->compute_units;
+      const long cost = rounds * (a.halves ? 4 + tm : 6 + tm);
+      if (best == 0 || cost < best) best = cost, a.tile_rows = 32 * tm;
     }
     a.row_tiles = (a.M + a.tile_rows - 1) / a.tile_rows;
     grid = (a.row_tiles * a.col_tiles + 7) / 8 * 8;
-    k = kind == kMixed ? kq_mm_own_kernel<kMixed, false> : kind == ORNITH_Q4K ? kq_mm_own_kernel<ORNITH_Q4K, false> : kq_mm_own_kernel<ORNITH_Q6K, false>;
+#define OWN(F) (kind == kMixed ? kq_mm_own_kernel<kMixed, F, false> : kind == ORNITH_Q4K ? kq_mm_own_kernel<ORNITH_Q4K, F, false> : kq_mm_own_kernel<ORNITH_Q6K, F, false>)
+    k = form == kFour ? OWN(kFour) : OWN(kHalves);
+#undef OWN
   }
-  hipLaunchKernelGGL(k, dim3(grid), dim3(256), 0, ctx->stream, a);
+  hipLaunchKernelGGL(k, dim3(grid), dim3(threads), 0, ctx->stream, a);
   ORN_LAUNCH_CHECK("kq_mm_own_kernel");
   return ORNITH_OK;
 }

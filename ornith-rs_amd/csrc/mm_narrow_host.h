@@ -6,23 +6,18 @@
 
 namespace nmm {
 
-// Rows up to which a k-quant projection takes these kernels: the wide kernels' 256 x 128 tiles fill the device from about a
-// thousand rows of 12288 columns on, and for up to 2048 columns not before a thousand rows either (2048 x 4096, us here /
-// there: 64 rows 7.2 / 52, 256 rows 15 / 53, 700 rows 29 / 54, 1024 rows 38 / 55; 256 x 2048: 5 / 29, 1024 rows 9 / 29).
-// More columns than that go to the own-column kernel of kq_mm_own.hip (12288 x 2048 Q4_K, us, here / there: 128 rows 20 / 25, 200 rows
-// 27 / 26; the rule there looks at one matrix at a time, never at what shares its launch: a matrix gives the same bits alone and in company).
-// The lines for up to 2048 columns, from K = 2048 on (below, the wide kernels' few slabs are over as soon: 2048 x 512 at 1024 rows 10.5 /
-// 9.9): Q4_K 1536 rows (2048 x 4096 at 1200 / 1500 / 2000 rows 44 / 54, 46 / 55, 58 / 57), Q6_K 1024 (2048 x 4096 at 1024 / 1200 / 1500 rows
-// 51 / 57, 56 / 57, 67 / 58), and up to 256 columns, which are 16 to 40 workgroups of the wide kernels, 2560 (the router at 1200 / 2000 / 2500
-// rows 13 / 29, 17 / 29, 21 / 29; level at 4096).
-constexpr int kNarrowRows = 192, kNarrowRowsSlim = 1024, kNarrowRowsSlimQ4K = 1536, kNarrowRowsSlimmest = 2560;
+// Rows up to which a k-quant projection takes these kernels; more go to the own-column kernel (kq_mm_own.hip, us, here / there).
+// More than 2048 columns: Q4_K 128 rows (8192 + 4096 x 2048 at 100 / 129 rows 18 / 18, 25 / 18), Q6_K 192 (8192 + 512 + 512 x 2048, of which the narrow ones
+// then run by themselves, at 192 / 200 23 / 24, 35 / 25). Up to 2048 columns, from K = 2048 on: 512 rows (2048 x 4096 Q4_K at 512 / 513 21 / 24, 30 / 24, Q6_K 25 / 28,
+// 36 / 28); up to 512 columns, which rarely come alone, 1024 and of Q4_K 1536; up to 256, a handful of workgroups there, 2560 (256 x 2048 at 1200 /
+// 2000 / 2500 rows 13 / 28, 18 / 28, 21 / 28). Below K = 2048 1024 rows (2048 x 512 at 1024 10.9 / 10.6).
+constexpr int kNarrowRows = 192, kNarrowRowsQ4K = 128, kNarrowRowsMid = 512, kNarrowRowsSlim = 1024, kNarrowRowsSlimQ4K = 1536, kNarrowRowsSlimmest = 2560;
 // The affine formats have no wide kernels: their projections own columns from here on (4-bit, 12288 x 2048, us, split /
 // owned: 300 rows 37 / 37, 400 rows 50 / 52, 512 rows 56 / 51, 600 rows 68 / 61, 2000 rows 207 / 187).
 constexpr int kTallFromAffine = 448;
-// Pairs an expert below which the routed experts take them: above that an expert is three tiles of 64 and more, and the wide kernels'
-// one unpacking for all its rows pays. Prompts through 256 experts of 8 a token, ms, here / there: 1600 tokens 24.9 / 26.8, 2000
-// 28.4 / 29.5, 2400 31.4 / 32.6, 2700 35.0 / 35.6, 3000 37.2 / 37.4, 3500 42.0 / 42.1, 4096 47.3 / 46.5, 5000 59.2 / 57.7 (80 is 2560 tokens: past
-// that the two are level).
+// Pairs an expert below which the routed experts take them: above that an expert is three tiles of 64 and more, and one unpacking for
+// all its rows pays. Prompts through 256 experts of 8 a token, ms, here / there: 1600 tokens 21.7 / 24.4, 2000 24.8 / 27.0, 2400 28.2 / 29.8, 2600
+// 31.6 / 31.4, 3000 35.3 / 34.3, 4096 44.7 / 42.2 (80 is 2560 tokens).
 constexpr int kNarrowPairs = 80;
 
 // an expert-sorted pair list in device memory, tiles of up to `rows` pairs

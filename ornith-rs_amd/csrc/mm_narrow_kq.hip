@@ -68,8 +68,8 @@ bool plain_ok(const ornith_linear* const* ws, int n, const void* d_x, int M, voi
   if (affine(kind_of(*ws[0]))) return true;
   for (int i = 0; i < n; ++i) {
     const bool q4 = ws[i]->km.kind == ORNITH_Q4K;
-    const int slim = K < 2048 ? kNarrowRowsSlim : ws[i]->O <= 256 ? kNarrowRowsSlimmest : q4 ? kNarrowRowsSlimQ4K : kNarrowRowsSlim;
-    if (M > (ws[i]->O <= 2048 ? slim : kNarrowRows)) return false;
+    const int slim = K < 2048 ? kNarrowRowsSlim : ws[i]->O <= 256 ? kNarrowRowsSlimmest : ws[i]->O > 512 ? kNarrowRowsMid : q4 ? kNarrowRowsSlimQ4K : kNarrowRowsSlim;
+    if (M > (ws[i]->O <= 2048 ? slim : q4 ? kNarrowRowsQ4K : kNarrowRows)) return false;
   }
   return true;
 }

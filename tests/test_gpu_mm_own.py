@@ -28,6 +28,10 @@ def _check(got_bits, x, w, what):
     # the lowest row counts of the rule: wide matrices of K >= 2048 and below, narrow ones
     (Q4K, 2056, 2048, 193), (Q6K, 2056, 2304, 193), (Q4K, 2304, 256, 513), (Q6K, 2051, 768, 545), (Q6K, 72, 256, 2049),
     (Q4K, 257, 2048, 1025 + 512),
+    # two sets of wavefronts with half of K each: one super-block a set and an odd number, the ends of the rule, columns and rows that
+    # end inside a tile, tiles of 2, 3 and 4 row blocks
+    (Q4K, 2056, 512, 129), (Q6K, 2049, 1536, 193), (Q4K, 2056, 2048, 256), (Q4K, 2056, 2048, 257), (Q4K, 600, 2048, 513), (Q6K, 2043, 2048, 545),
+    (Q6K, 1032, 2048, 2048), (Q6K, 1032, 2048, 2049), (Q4K, 10880, 512, 200), (Q4K, 16384, 512, 225), (Q6K, 2304, 768, 200),
     # 64 column tiles: the tile height that fills 256 compute units, 8, 8, 7, 6 and 5 blocks of 32 rows, and what is left of it
     (Q4K, 16384, 256, 1000), (Q6K, 16384, 256, 900), (Q4K, 16384, 256, 890), (Q6K, 16384, 256, 760), (Q4K, 16380, 512, 601),
     # more than one round of tiles, in patches of eight row tiles and a rest
@@ -66,3 +70,19 @@ def test_own_columns_experts_of_every_height(orn, ctx, kind, O, K):
         if len(sel): _check(got[sel], x[sel], deq[e], (kind, O, K, counts[e]))
     for b in (plan, di, dx, dy): b.free()
     w.free()
+
+
+def test_own_columns_forms_in_one_call(orn, ctx):
+    """matrices of one call whose sums are taken over K as a whole and in halves, and one that neither form takes: each the same bits as alone"""
+    K, M, Os = 2048, 1100, (2304, 600, 264, 64)
+    rng = np.random.default_rng(3)
+    ws = [orn.Linear.kquant(ctx, kind, *util.make_kq(kind, rng, 1, O, K), O, K) for kind, O in zip((Q4K, Q6K, Q6K, Q6K), Os)]
+    dx, ys = ctx.to_device(util.bf16_normal(rng, (M, K))), [ctx.alloc(M * O * 2) for O in Os]
+    ctx.linear_matmul_multi(ws, dx, M, ys)
+    for w, O, y in zip(ws, Os, ys):
+        alone = ctx.alloc(M * O * 2)
+        ctx.linear_matmul(w, dx, M, alone)
+        assert np.array_equal(y.download(np.uint16, (M, O)), alone.download(np.uint16, (M, O))), O
+        for b in (y, alone): b.free()
+        w.free()
+    dx.free()
