@@ -13,7 +13,7 @@ struct OwnMat {
 };
 
 struct OwnArgs {
-  OwnMat m[4];  // plain: up to four matrices of one kind; gathered: the experts' stack
+  OwnMat m[4];  // plain: up to four matrices of one K, of either kind; gathered: the experts' stack
   int n;
   const bf16_t* x;
   int M, K;
@@ -27,7 +27,7 @@ struct OwnArgs {
   uint32_t up_magic;  // 2^32 / up_div rounded up: the upper half of its product with a pair is pair / up_div
 };
 
-constexpr int kOwnRows = 256, kOwnCols = 256;  // a workgroup's tile
+constexpr int kOwnRows = 256, kOwnCols = 256;  // a workgroup's tile (in halves of K 128 x 128)
 
 // alignment and reach: x of `rows` rows, any K % 256 == 0
 bool kq_mm_own_ok(const ornith_kmatrix& w, const void* x, size_t rows);
