@@ -10,12 +10,13 @@
 // four wavefronts multiply by, come in slabs of 64 k straight into LDS (global_load_lds, whole 128-byte lines; no registers, no
 // writes), three slabs deep, with one barrier a slab that leaves requests in flight. The codes go to LDS the same way, into a
 // part that is the wavefront's own: 64 lanes that each read 16 bytes of their own row would look up 64 cache lines a load, whole
-// rows of a super-block 8. One super-block is unpacked while the next one's codes travel.
+// rows of a super-block 8. So do the scales. One super-block is unpacked while the next one's weights travel.
 //
 // A k step is 16 matrix instructions (at 256 rows), and between them, one piece after each, stands the work for the step
 // after: eight fragment reads, the unpacking of two fragments (36 vector instructions of Q4_K, 52 of Q6_K), a slab's
-// requests. The order is fixed in the source (sched_barrier after each piece) and every wait for memory is counted by hand: requests
-// are inline assembly, because waits that the compiler places at a loop's end are for everything in flight.
+// requests. The order is fixed in the source (sched_barrier after each piece) and every wait for memory is counted by hand. That is
+// sound because nothing of it goes to registers: a load to a register in inline assembly is, to the compiler, done there and then, so
+// that it may copy or spill what is still to come; and one that it knows of it waits for with everything else in flight.
 //
 // Shorter prompts (kHalves): tiles of 128 columns by up to 128 rows and two such sets of wavefronts, each over half of K, whose sums meet
 // in LDS at the end. With few rows a tile the unpacking is the work, and a wavefront alone on its SIMD issues one instruction every 5
@@ -44,7 +45,6 @@ typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 typedef unsigned int u32x2_t __attribute__((ext_vector_type(2)));
-typedef unsigned int u32x3_t __attribute__((ext_vector_type(3)));
 typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
 
 template <int N>
@@ -58,35 +58,21 @@ __device__ __forceinline__ void each(F f) {
   each_of(f, std::make_integer_sequence<int, N>{});
 }
 
-// ---- requests: a base the wavefront shares, a lane's offset. They are waited for by count (wait_loads), never by the
-// compiler; here() is where a request's registers may be used from
-template <int OFF>
-__device__ __forceinline__ void ask(u32x4_t& d, const uint8_t* base, uint32_t off) {
-  asm volatile("global_load_dwordx4 %0, %1, %2 offset:%3" : "=v"(d) : "v"(off), "s"(base), "n"(OFF));
-}
-__device__ __forceinline__ void ask(u32x3_t& d, const uint8_t* base, uint32_t off) {
-  asm volatile("global_load_dwordx3 %0, %1, %2" : "=v"(d) : "v"(off), "s"(base));
-}
-__device__ __forceinline__ void ask(u32x2_t& d, const uint8_t* base, uint32_t off) {
-  asm volatile("global_load_dwordx2 %0, %1, %2" : "=v"(d) : "v"(off), "s"(base));
-}
-__device__ __forceinline__ void ask(uint32_t& d, const uint8_t* base, uint32_t off) {
-  asm volatile("global_load_dword %0, %1, %2" : "=v"(d) : "v"(off), "s"(base));
-}
-__device__ __forceinline__ void ask16(uint32_t& d, const uint8_t* base, uint32_t off) {
-  asm volatile("global_load_ushort %0, %1, %2" : "=v"(d) : "v"(off), "s"(base));
-}
+// ---- requests, all of them to LDS: waited for by count (the compiler does not connect them with the reads of what they bring)
 template <int N>
 __device__ __forceinline__ void wait_loads() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
-// BYTES (4 or 16) a lane from memory to LDS, the lanes' pieces side by side at `lds`
+// BYTES (2, 4 or 16) a lane from a base the wavefront shares and the lane's offset to LDS, the lanes' pieces side by side at `lds` (two bytes
+// in places of four)
 template <int BYTES>
 __device__ __forceinline__ void dma(const uint8_t* base, uint32_t off, uint32_t lds) {
   typedef const __attribute__((address_space(1))) void glb_t;
   typedef __attribute__((address_space(3))) void lds_t;
+  static_assert(BYTES == 2 || BYTES == 4 || BYTES == 16, "");
   if constexpr (BYTES == 16) __builtin_amdgcn_global_load_lds((glb_t*)(uint64_t)(base + off), (lds_t*)(uint64_t)lds, 16, 0, 0);
-  else __builtin_amdgcn_global_load_lds((glb_t*)(uint64_t)(base + off), (lds_t*)(uint64_t)lds, 4, 0, 0);
+  else if constexpr (BYTES == 4) __builtin_amdgcn_global_load_lds((glb_t*)(uint64_t)(base + off), (lds_t*)(uint64_t)lds, 4, 0, 0);
+  else __builtin_amdgcn_global_load_lds((glb_t*)(uint64_t)(base + off), (lds_t*)(uint64_t)lds, 2, 0, 0);
 }
 __device__ __forceinline__ uint32_t lds_address(const void* p) {
   return (uint32_t)(uint64_t)(const __attribute__((address_space(3))) void*)p;
@@ -111,7 +97,6 @@ struct Fmt;
 template <>
 struct Fmt<ORNITH_Q4K> {
   static constexpr int kQ = 128, kS = 12, kD = 4, kInstr = 4, kHalf = 2;
-  typedef u32x3_t Scales;
   static __device__ __forceinline__ void source(int n, int& row, int& p) {  // what lies at 16-byte place n
     row = n >> 3;
     p = (n & 7) ^ ((row >> 1) & 7);
@@ -123,7 +108,6 @@ struct Fmt<ORNITH_Q4K> {
 template <>
 struct Fmt<ORNITH_Q6K> {
   static constexpr int kQ = 192, kS = 16, kD = 2, kInstr = 6, kHalf = 3;
-  typedef u32x4_t Scales;
   static __device__ __forceinline__ void source(int n, int& row, int& p) {
     row = n / 12;
     p = n - 12 * row - ((row >> 2) & 3);
@@ -137,21 +121,23 @@ struct Fmt<ORNITH_Q6K> {
   // low rows a and b (I = 0, 1) and high bits (2) of half HF
   static __device__ __forceinline__ int piece(int hf, int i, int h) { return i < 2 ? 4 * hf + 2 * i + h : 8 + 2 * hf + h; }
 };
-template <int KIND>
+// The scales of a super-block, four words a column: of Q4_K its 12 bytes of scales and, fourth, d and dmin; of Q6_K its 16 bytes of
+// scales, and d in a request by itself. A request brings them of 16 columns, a word a lane.
+template <int KIND, int TN>
 struct Sc {
-  typename Fmt<KIND>::Scales sc;
-  uint32_t dm;
-  template <int I>
-  __device__ __forceinline__ void load(const uint8_t* s0, const uint8_t* d0, uint32_t so, uint32_t dof) {
-    if constexpr (I == 0) {
-      if constexpr (KIND == ORNITH_Q4K) ask(sc, s0, so);
-      else ask<0>(sc, s0, so);
-    } else {
-      if constexpr (KIND == ORNITH_Q4K) ask(dm, d0, dof);
-      else ask16(dm, d0, dof);
-    }
+  typedef Fmt<KIND> F;
+  static constexpr int kReq = 2 * TN + (KIND == ORNITH_Q6K);
+  u32x4_t sc;
+  uint32_t d;  // Q6_K
+  // of column l32 of block j
+  __device__ __forceinline__ void read(const uint8_t* lds, int j, int l32) {
+    sc = *reinterpret_cast<const u32x4_t*>(lds + 16 * (32 * j + l32));
+    if constexpr (KIND == ORNITH_Q6K) d = *reinterpret_cast<const uint16_t*>(lds + 512 * TN + 4 * (32 * j + l32));
   }
-  __device__ __forceinline__ void here() { asm volatile("" : "+v"(sc), "+v"(dm)); }
+  __device__ __forceinline__ uint32_t dm() const {
+    if constexpr (KIND == ORNITH_Q4K) return sc[3];
+    else return d;
+  }
 };
 
 // the upper half of a's lanes trades places with the lower half of b's (swap16: a's odd rows of sixteen with b's even ones)
@@ -197,16 +183,16 @@ struct Deq {
   uint32_t e0, o0, e1, o1;
   float x0, x1;
   u32x4_t f;
-  template <int T, int P>
-  __device__ __forceinline__ void piece(const Sc<KIND>& z, int h) {
+  template <int T, int P, class Z>
+  __device__ __forceinline__ void piece(const Z& z, int h) {
     constexpr int HF = T >> 3, QD = (T >> 1) & 3, NIB = KIND == ORNITH_Q4K ? QD & 1 : QD >> 1;
     if constexpr (P == 0) {
       if constexpr (KIND == ORNITH_Q4K) {
         if constexpr (T == 0) {
-          const float d = dm_h2f((f16_t)(z.dm & 0xffffu));
+          const float d = dm_h2f((f16_t)(z.dm() & 0xffffu));
           dl = d * 16777216.f;
           dh = d * 1048576.f;
-          nm = -dm_h2f((f16_t)(z.dm >> 16));
+          nm = -dm_h2f((f16_t)(z.dm() >> 16));
           sc4 = z.sc[0] & 0x3f3f3f3fu;
           m4 = z.sc[1] & 0x3f3f3f3fu;
         }
@@ -219,7 +205,7 @@ struct Deq {
           o = nm * dm_ubyte<QD>(m4);
         }
       } else {
-        if constexpr (T == 0) dl = dm_h2f((f16_t)z.dm);
+        if constexpr (T == 0) dl = dm_h2f((f16_t)z.dm());
         if constexpr (T % 2 == 0) {  // scale 8 HF + 2 QD + h of the sixteen
           const float v = dl * (float)(int)(int8_t)(((z.sc[T >> 2] >> (8 * h)) >> (16 * (QD & 1))) & 0xffu);
           s = v * (NIB ? 1048576.f : 16777216.f);
@@ -270,17 +256,20 @@ constexpr int rows_of(int form) { return form == kHalves ? 128 : kOwnRows; }
 
 constexpr int kStages = 3;                          // of 64 k: 128 bytes of a row
 constexpr int kActs = kStages * kOwnRows * 128;      // LDS: activations (kHalves: a half for each set), then a part for each wavefront's codes
-constexpr int kLds = kActs + kOwnCols * 192;
+constexpr int kCodes = kOwnCols * 192;               // ... and its scales
+constexpr int kScales = kOwnCols * 20 + 8 * 128;     // (kHalves: 128 bytes of each request for Q6_K's d are there twice)
+constexpr int kLds = kActs + kCodes + kScales;
 
 template <int KIND, int TM, int FORM, bool GATHER>
-__device__ __forceinline__ void own_tile(const OwnArgs& a, const OwnMat& mt, uint8_t* smem, uint32_t* s_dst, int n0, int rows, int m0,
+__device__ __forceinline__ void own_tile(const OwnArgs& a, const OwnMat& mt, uint8_t* smem, int n0, int rows, int m0,
                                          int64_t wrow0, const uint32_t* pairs) {
   typedef Fmt<KIND> F;
   constexpr int TN = tn_of(FORM), STAGE = TM * 4096, SL = TN * TM;
-  constexpr int NC = TN * (F::kInstr + 2);  // requests of a super-block's weights
+  typedef Sc<KIND, TN> Z;
+  constexpr int NC = TN * F::kInstr + Z::kReq;  // requests of a super-block's weights
   const int tid = threadIdx.x, lane = tid & 63, wave_of = __builtin_amdgcn_readfirstlane(tid >> 6), l32 = lane & 31, h = lane >> 5;
   const int wave = wave_of & 3, set = wave_of >> 2, row_blocks = a.K >> 8, nb = FORM == kHalves ? row_blocks / 2 : row_blocks, b0 = set * nb;
-  uint32_t qo[TN][F::kInstr], so[TN], dof[TN];
+  uint32_t qo[TN][F::kInstr];
 #pragma unroll
   for (int j = 0; j < TN; ++j) {
     const int r0 = n0 + 32 * TN * wave + 32 * j;
@@ -290,46 +279,57 @@ __device__ __forceinline__ void own_tile(const OwnArgs& a, const OwnMat& mt, uin
       F::source(64 * i + lane, row, p);
       qo[j][i] = (uint32_t)min(r0 + row, mt.O - 1) * (uint32_t)(row_blocks * F::kQ) + 16 * p;
     }
-    const uint32_t row = (uint32_t)min(r0 + l32, mt.O - 1) * (uint32_t)row_blocks;
-    so[j] = row * F::kS;
-    dof[j] = row * F::kD;
   }
   const uint8_t *qb = uniform(mt.qs + (wrow0 * row_blocks + b0) * F::kQ), *sb = uniform(mt.scales + (wrow0 * row_blocks + b0) * F::kS),
                 *db = uniform(mt.dm + (wrow0 * row_blocks + b0) * F::kD);
+  const int word = lane & 3;
+  const bool of_d = KIND == ORNITH_Q4K && word == 3;
+  const uint8_t* sp[2 * TN];  // what the lane takes of 16 columns' scales
+#pragma unroll
+  for (int i = 0; i < 2 * TN; ++i) {
+    const uint32_t row = (uint32_t)min(n0 + 32 * TN * wave + 16 * i + (lane >> 2), mt.O - 1) * (uint32_t)row_blocks;
+    sp[i] = of_d ? db + row * F::kD : sb + (row * F::kS + 4 * word);
+  }
+  const uint32_t sp_step = of_d ? F::kD : F::kS;
+  const uint32_t dof = (uint32_t)min(n0 + 32 * TN * wave + (TN == 2 ? lane : l32), mt.O - 1) * (uint32_t)row_blocks * F::kD;  // Q6_K
   __builtin_amdgcn_sched_barrier(0);
   // request i of a slab's activations: eight rows of row block i, 128 bytes each
+  uint32_t* const s_dst = reinterpret_cast<uint32_t*>(smem + kLds);  // (gathered form)
+  uint32_t* const s_src = s_dst + kOwnRows;
   uint32_t pr[TM];
-  if constexpr (GATHER) {
+  if constexpr (GATHER) {  // (the rows a wavefront asks for, eight of each block, go to a part of its own)
     const uint8_t* pb = uniform((const uint8_t*)pairs);
     dma<4>(pb, 4 * min(tid, rows - 1), lds_address(s_dst) + 256 * wave);
-#pragma unroll
-    for (int i = 0; i < TM; ++i) ask(pr[i], pb, 4 * min(32 * i + 8 * wave + (lane >> 3), rows - 1));
+    dma<4>(pb, 4 * min(32 * (lane >> 3) + 8 * wave + (lane & 7), rows - 1), lds_address(s_src) + 256 * wave);
   } else {
 #pragma unroll
     for (int i = 0; i < TM; ++i) pr[i] = m0 + min(32 * i + 8 * wave + (lane >> 3), rows - 1);
   }
   uint8_t* const mine = smem + kActs + wave_of * (32 * TN * F::kQ);
-  const uint32_t mine_at = lds_address(mine);
-  Sc<KIND> cur[TN], nxt[TN];
-  auto weights = [&](Sc<KIND> (&z)[TN], const uint8_t* q0, const uint8_t* s0, const uint8_t* d0, auto ic) {
-    constexpr int I = decltype(ic)::value;
-    if constexpr (I < TN * F::kInstr) dma<16>(q0, qo[I / F::kInstr][I % F::kInstr], mine_at + 1024 * I);
-    else z[(I - TN * F::kInstr) / 2].template load<I % 2>(s0, d0, so[(I - TN * F::kInstr) / 2], dof[(I - TN * F::kInstr) / 2]);
+  const uint8_t* const my_scales = smem + kActs + kCodes + wave_of * (kScales / (FORM == kHalves ? 8 : 4));
+  const uint32_t mine_at = lds_address(mine), scales_at = lds_address(my_scales);
+  Z z[TN];
+  // request I of a super-block's weights: the first (NEXT = 0), or the one after what was asked for before
+  auto weights = [&](auto next, auto ic) {
+    constexpr int NEXT = decltype(next)::value, I = decltype(ic)::value, J = I - TN * F::kInstr;
+    if constexpr (I < TN * F::kInstr) dma<16>(qb + NEXT * F::kQ, qo[I / F::kInstr][I % F::kInstr], mine_at + 1024 * I);
+    else if constexpr (J < 2 * TN) {
+      sp[J] += NEXT * sp_step;
+      dma<4>(sp[J], 0, scales_at + 256 * J);
+    } else dma<2>(db + NEXT * F::kD, dof, scales_at + 512 * TN);
   };
-  each<NC>([&](auto ic) { weights(cur, qb, sb, db, ic); });
+  each<NC>([&](auto ic) { weights(IC<0>{}, ic); });
   __builtin_amdgcn_sched_barrier(0);
   if constexpr (GATHER) {
     wait_loads<NC>();
 #pragma unroll
-    for (int i = 0; i < TM; ++i) asm volatile("" : "+v"(pr[i]));
+    for (int i = 0; i < TM; ++i) pr[i] = s_src[64 * wave + 8 * i + (lane >> 3)];
   }
   uint32_t xo[TM];
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
     const uint32_t src = GATHER && a.up_div > 1 ? __umulhi(pr[i], a.up_magic) : pr[i];
-    uint32_t at = src * (2u * (uint32_t)a.K);
-    asm volatile("" : "+v"(at));  // (or its sum becomes a 64-bit multiply-add that names registers still to be filled)
-    xo[i] = at + 16 * ((lane & 7) ^ ((4 * wave + (lane >> 4)) & 7));
+    xo[i] = src * (2u * (uint32_t)a.K) + 16 * ((lane & 7) ^ ((4 * wave + (lane >> 4)) & 7));
   }
   const uint8_t* xg = reinterpret_cast<const uint8_t*>(a.x) + 512 * b0;
   const uint32_t mem = set * (kActs / 2), at = lds_address(smem) + mem + wave * 1024;
@@ -363,16 +363,14 @@ __device__ __forceinline__ void own_tile(const OwnArgs& a, const OwnMat& mt, uin
       dq[j].q[F::kHalf * HF + i] = *reinterpret_cast<const u32x4_t*>(mine + j * (32 * F::kQ) + F::at(l32, F::piece(HF, i, h)));
   };
   wait_loads<2 * TM>();  // the weights and stage 0
-#pragma unroll
-  for (int j = 0; j < TN; ++j) cur[j].here();
   barrier_only();
 #pragma unroll
-  for (int j = 0; j < TN; ++j) codes(IC<0>{}, j), codes(IC<1>{}, j);
+  for (int j = 0; j < TN; ++j) z[j].read(my_scales, j, l32), codes(IC<0>{}, j), codes(IC<1>{}, j);
 #pragma unroll
   for (int i = 0; i < TM; ++i) read(IC<0>{}, st, i);
   each<TN * 7>([&](auto pc) {
     constexpr int J = decltype(pc)::value / 7, P = decltype(pc)::value % 7;
-    dq[J].template piece<0, P>(cur[J], h);
+    dq[J].template piece<0, P>(z[J], h);
   });
 #pragma unroll
   for (int j = 0; j < TN; ++j) bf[0][j] = __builtin_bit_cast(bf16x8_t, dq[j].f);
@@ -396,12 +394,6 @@ __device__ __forceinline__ void own_tile(const OwnArgs& a, const OwnMat& mt, uin
         if constexpr (S == 2) {
           if (last) wait_loads<0>();
           else wait_loads<TM>();
-#pragma unroll
-          for (int j = 0; j < TN; ++j) nxt[j].here();
-        }
-        if constexpr (S == 3) {
-#pragma unroll
-          for (int j = 0; j < TN; ++j) cur[j] = nxt[j];
         }
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         barrier_only();
@@ -411,10 +403,11 @@ __device__ __forceinline__ void own_tile(const OwnArgs& a, const OwnMat& mt, uin
         acc[M][N] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bf[T & 1][N], af[M], acc[M][N], 0, 0, 0);
         if constexpr (N == TN - 1) read(IC<U>{}, (T & 3) == 3 ? st1 : st, M);
         if constexpr ((T == 12 || T == 15) && I < TN) codes(IC<(T == 12 ? 0 : 1)>{}, I);
+        if constexpr (T == 14 && I < TN) z[I].read(my_scales, I, l32);  // (the last that step 13 needed)
         constexpr int P0 = I * (TN * 7) / SL, P1 = (I + 1) * (TN * 7) / SL;
         each<P1 - P0>([&](auto pc) {
           constexpr int Q = P0 + decltype(pc)::value, J = Q % TN, P = Q / TN;
-          dq[J].template piece<(U & 15), P>(cur[J], h);
+          dq[J].template piece<(U & 15), P>(z[J], h);
           if constexpr (P == 6) bf[U & 1][J] = __builtin_bit_cast(bf16x8_t, dq[J].f);
         });
         if constexpr ((T & 3) == 3) {
@@ -426,7 +419,7 @@ __device__ __forceinline__ void own_tile(const OwnArgs& a, const OwnMat& mt, uin
                 if constexpr (Q < TM) {
                   if (S == 0 || !last) dma<16>(xg + 128 * (S + 3), xo[Q], at + st + Q * 4096);
                 } else {
-                  if (!last) weights(nxt, qb + F::kQ, sb + F::kS, db + F::kD, IC<Q - TM>{});
+                  if (!last) weights(IC<1>{}, IC<Q - TM>{});
                 }
               }
             });
@@ -437,7 +430,6 @@ __device__ __forceinline__ void own_tile(const OwnArgs& a, const OwnMat& mt, uin
     });
     xg += 512;
     qb += F::kQ;
-    sb += F::kS;
     db += F::kD;
   }
   if constexpr (FORM == kHalves) {
@@ -508,8 +500,8 @@ __device__ __forceinline__ void own_tile(const OwnArgs& a, const OwnMat& mt, uin
 constexpr int kMixed = 2;  // the matrices of the launch differ in kind
 template <int KIND, int FORM, bool GATHER>
 __global__ __launch_bounds__(threads_of(FORM)) __attribute__((amdgpu_waves_per_eu(threads_of(FORM) / 256, threads_of(FORM) / 256))) void kq_mm_own_kernel(OwnArgs a) {
-  __shared__ __attribute__((aligned(1024))) uint8_t smem[kLds];
-  __shared__ uint32_t s_dst[GATHER ? kOwnRows : 1];
+  // (one array: with more than one, the compiler does connect some reads with requests, and waits for everything in flight ahead of them)
+  __shared__ __attribute__((aligned(1024))) uint8_t smem[kLds + (GATHER ? 4 * (kOwnRows + 256) : 0)];
   int rows, m0 = 0, tc, mat = 0;
   int64_t wrow0 = 0;
   const uint32_t* pairs = nullptr;
@@ -546,7 +538,7 @@ __global__ __launch_bounds__(threads_of(FORM)) __attribute__((amdgpu_waves_per_e
   const int groups = (rows + 31) >> 5;
   auto of_kind = [&](auto kc) {
     constexpr int KD = decltype(kc)::value;
-#define OWN(N) own_tile<KD, N, FORM, GATHER>(a, mt, smem, s_dst, n0, rows, m0, wrow0, pairs)
+#define OWN(N) own_tile<KD, N, FORM, GATHER>(a, mt, smem, n0, rows, m0, wrow0, pairs)
     if constexpr (FORM == kFour) {
       if (groups >= 8) return OWN(8);
       if (groups == 7) return OWN(7);
