@@ -39,6 +39,14 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t dm_buffer(const void* p, uint3
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)bytes, 0x00020000);
 }
 
+// p / d for p, d < 2^31, d > 1, with magic = dm_div_magic(d), 2^32 / d rounded up: the upper half of p * magic is the quotient or, from where p times
+// what the rounding added passes 2^32, one more.
+inline uint32_t dm_div_magic(int d) { return (uint32_t)(((uint64_t(1) << 32) + (uint32_t)d - 1) / (uint32_t)d); }
+__device__ __forceinline__ uint32_t dm_div(uint32_t p, uint32_t d, uint32_t magic) {
+  const uint32_t q = __umulhi(p, magic);
+  return q - (q * d > p ? 1u : 0u);
+}
+
 __device__ __forceinline__ float dm_fma(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 
 __device__ __forceinline__ float dm_bf2f(bf16_t b) { return __uint_as_float((uint32_t)b << 16); }

@@ -24,7 +24,7 @@ struct OwnArgs {
   int tiles_max, up_div;
   const uint32_t* expert_at;  // over a plan of lower tiles: [E] where an expert's pairs begin; else null
   int E;
-  uint32_t up_magic;  // 2^32 / up_div rounded up: the upper half of its product with a pair is pair / up_div
+  uint32_t up_magic;  // dm_div_magic(up_div)
 };
 
 constexpr int kOwnRows = 256, kOwnCols = 256;  // a workgroup's tile (in halves of K 128 x 128)

@@ -328,7 +328,7 @@ __device__ __forceinline__ void own_tile(const OwnArgs& a, const OwnMat& mt, uin
   uint32_t xo[TM];
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
-    const uint32_t src = GATHER && a.up_div > 1 ? __umulhi(pr[i], a.up_magic) : pr[i];
+    const uint32_t src = GATHER && a.up_div > 1 ? dm_div(pr[i], (uint32_t)a.up_div, a.up_magic) : pr[i];
     xo[i] = src * (2u * (uint32_t)a.K) + 16 * ((lane & 7) ^ ((4 * wave + (lane >> 4)) & 7));
   }
   const uint8_t* xg = reinterpret_cast<const uint8_t*>(a.x) + 512 * b0;
@@ -588,7 +588,7 @@ int kq_mm_own(ornith_ctx* ctx, OwnArgs& a, bool gather) {
   typedef void (*Kernel)(OwnArgs);
   Kernel k;
   if (gather) {
-    a.up_magic = (uint32_t)(((uint64_t(1) << 32) + a.up_div - 1) / a.up_div);
+    a.up_magic = dm_div_magic(a.up_div);
     a.col_tiles = (a.m[0].O + kOwnCols - 1) / kOwnCols;
     grid = a.col_tiles * ((a.tiles_max + 7) / 8 * 8);
     k = kind == ORNITH_Q4K ? kq_mm_own_kernel<ORNITH_Q4K, kFour, true> : kq_mm_own_kernel<ORNITH_Q6K, kFour, true>;

@@ -100,7 +100,7 @@ struct Args {
   const uint32_t* tile_count;
   const uint32_t* n_tiles;
   int up_div, pairs, E;
-  uint32_t up_magic;  // 2^32 / up_div rounded up: the upper half of its product with a pair is pair / up_div
+  uint32_t up_magic;  // dm_div_magic(up_div)
   int tiles_max, blocks;  // room in the tile list; column blocks a tile
   Riders d;
 };
@@ -825,7 +825,7 @@ __device__ __forceinline__ void owned_tile(const Args& a, int mat0, int c0, int6
   const uint8_t* x = reinterpret_cast<const uint8_t*>(a.x);
 #pragma unroll
   for (int i = 0; i < NP; ++i) {
-    const uint32_t p = pr[i], src = MODE == kTall || a.up_div == 1 ? p : (int)p < a.pairs ? __umulhi(p, a.up_magic) : p - (uint32_t)a.pairs;
+    const uint32_t p = pr[i], src = MODE == kTall || a.up_div == 1 ? p : (int)p < a.pairs ? dm_div(p, (uint32_t)a.up_div, a.up_magic) : p - (uint32_t)a.pairs;
     xo[i] = 2 * src * (uint32_t)a.K + piece;
   }
   if constexpr (HALF) W::ask_half(x, xo, 0, lds);

@@ -207,7 +207,7 @@ int launch_gathered(ornith_ctx* ctx, Args& a, int mode, const Plan& p, int O) {
   a.tile_count = p.tile_count;
   a.n_tiles = p.n_tiles;
   a.tiles_max = (int)p.tiles_max;
-  a.up_magic = (uint32_t)(((uint64_t(1) << 32) + a.up_div - 1) / a.up_div);
+  a.up_magic = dm_div_magic(a.up_div);
   const int halves = mode == kGateUp ? 2 : 1, cols = 128 / halves;
   a.blocks = (O + cols - 1) / cols;
   // LDS: activations, and the scales of the workgroup's 128 rows

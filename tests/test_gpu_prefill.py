@@ -166,6 +166,28 @@ def test_kq_gather_matmul_vs_float64(orn, ctx, kind, E, O, K, T, k):
     w.free()
 
 
+@pytest.mark.parametrize("E,k,T", [(1024, 81915, 1), (4, 100099, 2)])
+def test_a_pair_reads_its_own_token_however_many_pairs_a_token_has(orn, ctx, E, k, T):
+    """pair p reads row p / k of x where the quotient's reciprocal, rounded up to 32 bits, times p is off by one (the last pairs of
+    a token: the row after the last one), in the few-row kernels (fewer than 80 pairs an expert) and in those whose wavefronts own columns"""
+    magic = (2 ** 32 + k - 1) // k
+    assert ((k * T - 1) * magic) >> 32 == T  # T - 1 is right
+    O, K, pairs = 8, 512, T * k
+    rng = np.random.default_rng(E)
+    t = util.make_kq(Q4K, rng, E, O, K)
+    w = orn.KMatrix(ctx, Q4K, *t, E, O, K)
+    inds = rng.integers(0, E, pairs).astype(np.uint32)
+    xb = util.bf16_normal(rng, (T, K))
+    plan = ctx.alloc(orn.kq_gather_plan_bytes(pairs, E))
+    di, dx, dy = ctx.to_device(inds), ctx.to_device(xb), ctx.alloc(pairs * O * 2)
+    ctx.memset(dy, 0xFF, pairs * O * 2)
+    orn.kq_gather_matmul(ctx, w, dx, di, pairs, k, True, plan, True, dy)
+    want = np.einsum("tk,eok->teo", util.bf16_to_f32(xb).astype(np.float64), _deq_bf16(Q4K, t, E, O, K))
+    _check(dy.download(np.uint16, (pairs, O)), want[np.arange(pairs) // k, inds], K, (E, k, T))
+    for b in (plan, di, dx, dy): b.free()
+    w.free()
+
+
 def _rows_close(got_bits, want_bits, tol):
     """per-row relative L2 error of two bf16 [T, n] arrays"""
     g = util.bf16_to_f32(got_bits).astype(np.float64)
