@@ -195,6 +195,12 @@ class LinearStruct(C.Structure):
                 ("d_w", C.c_void_p), ("d_scales", C.c_void_p), ("d_biases", C.c_void_p)]
 
 
+def gemm_form(kind, O, K, M, x=4096, qs=4096, scales=4096, dm=4096, y=4096):
+    """The form of the prompt GEMM for a k-quant matrix at those addresses (ornith_selftest_gemm_form; no GPU needed)."""
+    s = LinearStruct(LIN_KQUANT, O, K, KMatrixStruct(kind, 1, O, K, qs, scales, dm), None, None, None)
+    return lib().ornith_selftest_gemm_form(C.byref(s), C.c_void_p(x), M, C.c_void_p(y))
+
+
 class MoeWeightsStruct(C.Structure):
     _fields_ = [("router", LinearStruct), ("ex_gate", KMatrixStruct), ("ex_up", KMatrixStruct),
                 ("ex_down", KMatrixStruct), ("sh_gate", LinearStruct), ("sh_up", LinearStruct),

@@ -629,7 +629,7 @@ int ornith_kq_matmul_multi(ornith_ctx* ctx, const ornith_kmatrix* const* ws, int
     ORN_REQUIRE(ws[i]->K == ws[0]->K, "kq_matmul: matrices of one launch differ in K");
   }
   for (int i = 0; i < n; ++i) {
-    if (ornith_option_gemm_duo() && kq_mm_own_suits(*ws[i], d_x, M)) {
+    if (kq_mm_own_suits(*ws[i], d_x, M)) {
       OwnArgs& o = own[kq_mm_own_halves(*ws[i], M)];
       o.m[o.n++] = kq_mm_own_mat(*ws[i], d_ys[i]);
       continue;

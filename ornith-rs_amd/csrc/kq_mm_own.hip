@@ -569,7 +569,7 @@ bool kq_mm_own_ok(const ornith_kmatrix& w, const void* x, size_t rows) {
 // 15 / 14.
 bool kq_mm_own_suits(const ornith_kmatrix& w, const void* x, int M) {
   const int from = w.O > 2048 ? (w.kind == ORNITH_Q4K ? 128 : 192) : w.K < 2048 ? 2048 : w.O > 512 ? 512 : w.O > 256 ? 1024 : 2048;
-  return M > from && kq_mm_own_ok(w, x, M);
+  return ornith_option_gemm_duo() && M > from && kq_mm_own_ok(w, x, M);
 }
 
 // ... and those that do it in kHalves, one matrix at a time whatever shares the launch, for the sums' order: while its tiles of 128

@@ -1,6 +1,8 @@
 // Element-wise evaluation of the device scalar functions, so a caller can check
 // them bit for bit against a CPU evaluation of the same formulae.
 #include "dmath.h"
+#include "kq_mm_own.h"
+#include "mm_narrow_host.h"
 #include "rt.h"
 
 namespace {
@@ -49,4 +51,11 @@ extern "C" int ornith_selftest_unary(ornith_ctx* ctx, int fn, const float* d_in,
                      d_in, d_out, n);
   ORN_LAUNCH_CHECK("unary_kernel");
   return ORNITH_OK;
+}
+
+extern "C" int ornith_selftest_gemm_form(const ornith_linear* w, const void* d_x, int M, const void* d_y) {
+  if (!w || w->mode != ORNITH_LIN_KQUANT) return -1;
+  void* const y = const_cast<void*>(d_y);
+  if (nmm::plain_ok(&w, 1, d_x, M, &y)) return 3;
+  return !kq_mm_own_suits(w->km, d_x, M) ? 0 : kq_mm_own_halves(w->km, M) ? 2 : 1;
 }

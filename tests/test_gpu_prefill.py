@@ -57,6 +57,64 @@ def test_kq_matmul_vs_float64(orn, ctx, kind, O, K, M):
     w.free()
 
 
+@pytest.mark.parametrize("mats,K,M", [
+    # 256-row tiles, ragged and whole (enough of them to fill the device), 128-row ones, wide matrices of both kinds, narrow ones that share a launch
+    ([(Q4K, 8192)], 512, 1061), ([(Q6K, 8192)], 512, 1024), ([(Q4K, 2056)], 512, 300), ([(Q4K, 4096), (Q6K, 4096)], 512, 1061),
+    ([(Q4K, 600), (Q6K, 264)], 256, 300)])
+def test_kq_matmul_weights_through_lds(orn, ctx, mats, K, M):
+    """gemm_duo = 0: every matrix through the tiles that unpack into LDS, the same bits in company as alone"""
+    rng = np.random.default_rng(M + K)
+    ts = [util.make_kq(kind, rng, 1, O, K) for kind, O in mats]
+    ws = [orn.Linear.kquant(ctx, kind, *t, O, K) for (kind, O), t in zip(mats, ts)]
+    xb = util.bf16_normal(rng, (M, K))
+    dx, ys = ctx.to_device(xb), [ctx.alloc((M + 1) * O * 2) for _, O in mats]
+    x = util.bf16_to_f32(xb).astype(np.float64)
+    try:
+        orn.set_option("gemm_duo", 0)
+        for (_, O), y in zip(mats, ys): ctx.memset(y, 0xFF, (M + 1) * O * 2)
+        ctx.linear_matmul_multi(ws, dx, M, ys)
+        for (kind, O), t, w, y in zip(mats, ts, ws, ys):
+            got = y.download(np.uint16, (M + 1, O))
+            assert np.all(got[M] == 0xFFFF)
+            assert orn.gemm_form(kind, O, K, M) == 0
+            _check(got[:M], x @ _deq_bf16(kind, t, 1, O, K)[0].T, K, (kind, O, K, M))
+            alone = ctx.alloc(M * O * 2)
+            orn.kq_matmul(ctx, w.keep[0], dx, M, alone)
+            assert np.array_equal(alone.download(np.uint16, (M, O)), got[:M])
+            alone.free()
+    finally:
+        orn.set_option("gemm_duo", 1)
+        for b in [dx] + ys + ws: b.free()
+
+
+@pytest.mark.parametrize("kind,E,O,K,T,k", [(Q4K, 8, 256, 512, 400, 2), (Q6K, 16, 131, 256, 500, 4), (Q4K, 8, 264, 1024, 700, 2),
+                                             (Q6K, 4, 130, 4352, 140, 2)])
+def test_kq_gather_matmul_weights_through_lds(orn, ctx, kind, E, O, K, T, k):
+    """gemm_reg = 0: the experts' GEMM in 64- and 128-row workgroups that unpack into LDS, a 48-row average among them"""
+    rng = np.random.default_rng(E + O + K)
+    t = util.make_kq(kind, rng, E, O, K)
+    w = orn.KMatrix(ctx, kind, *t, E, O, K)
+    pairs = T * k
+    inds = np.stack([rng.permutation(E)[:k] for _ in range(T)]).astype(np.uint32)
+    xb = util.bf16_normal(rng, (T, K))
+    plan = ctx.alloc(orn.kq_gather_plan_bytes(pairs, E))
+    di, dx, dy = ctx.to_device(inds.reshape(-1)), ctx.to_device(xb), ctx.alloc((pairs + 1) * O * 2)
+    ctx.memset(dy, 0xFF, (pairs + 1) * O * 2)
+    try:
+        orn.set_option("gemm_reg", 0)
+        orn.kq_gather_matmul(ctx, w, dx, di, pairs, k, True, plan, True, dy)
+        got = dy.download(np.uint16, (pairs + 1, O))
+        assert np.all(got[pairs] == 0xFFFF)
+        x, deq, flat = util.bf16_to_f32(xb).astype(np.float64), _deq_bf16(kind, t, E, O, K), inds.reshape(-1)
+        for e in range(E):
+            sel = np.nonzero(flat == e)[0]
+            _check(got[sel], x[sel // k] @ deq[e].T, K, (kind, E, O, K, e))
+    finally:
+        orn.set_option("gemm_reg", 1)
+        for b in (plan, di, dx, dy): b.free()
+        w.free()
+
+
 @pytest.mark.parametrize("kind,O,K,M", [(Q4K, 512, 2048, 256), (Q6K, 2048, 512, 256), (Q4K, 8192, 2048, 512),
                                          (Q6K, 2048, 4096, 300)])
 def test_kq_matmul_error_against_the_true_weights(orn, ctx, kind, O, K, M):
