@@ -850,7 +850,8 @@ ORNITH_API int ornith_json_dumps(const char* json, size_t len, char* out, size_t
 ORNITH_API int ornith_selftest_unary(ornith_ctx* ctx, int fn, const float* d_in, float* d_out, int64_t n);
 
 /* The form of the prompt GEMM that M rows take this k-quant matrix to, by itself or in company (host only; x and y: where they would lie):
- * 0 weights through LDS, 1 wavefronts own columns, 2 ... of two halves of K, 3 the few-row kernels. -1: not a k-quant matrix. */
+ * 0 weights through LDS, 1 wavefronts own columns, 2 ... of two halves of K, 3 the few-row kernels, 4 as 1 (with the same sums) in smaller tiles, as
+ * it does by itself on 256 compute units. -1: not a k-quant matrix. */
 ORNITH_API int ornith_selftest_gemm_form(const ornith_linear* w, const void* d_x, int M, const void* d_y);
 
 /* ---- machine probes (`bench.py --ceiling`) ------------------------------------------

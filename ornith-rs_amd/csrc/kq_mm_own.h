@@ -27,7 +27,7 @@ struct OwnArgs {
   uint32_t up_magic;  // dm_div_magic(up_div)
 };
 
-constexpr int kOwnRows = 256, kOwnCols = 256;  // a workgroup's tile (in halves of K 128 x 128)
+constexpr int kOwnRows = 256, kOwnCols = 256;  // a workgroup's tile (in halves of K, and of a thin launch, 128 x 128)
 
 // alignment and reach: x of `rows` rows, any K % 256 == 0
 bool kq_mm_own_ok(const ornith_kmatrix& w, const void* x, size_t rows);
@@ -35,5 +35,7 @@ bool kq_mm_own_ok(const ornith_kmatrix& w, const void* x, size_t rows);
 bool kq_mm_own_suits(const ornith_kmatrix& w, const void* x, int M);
 // ... and then whether its sums are taken in two halves of K
 bool kq_mm_own_halves(const ornith_kmatrix& w, int M);
+// whether a plain launch of whole sums over K takes tiles of 128 x 128 (a.m[].O, n, M, K), on a device of that many compute units: the sums are the same
+bool kq_mm_own_thin(const OwnArgs& a, int units);
 OwnMat kq_mm_own_mat(const ornith_kmatrix& w, void* y);
 int kq_mm_own(ornith_ctx* ctx, OwnArgs& a, bool gather);

@@ -25,6 +25,9 @@
 // 30). Four stages of activations with two super-blocks of codes in flight gave nothing, nor did eight wavefronts of 32 columns over
 // all of K (K = 4096, 2 row blocks 38).
 //
+// kThin is one such set, over all of K and two workgroups a compute unit: the sums of the full tile in a fourth of it, for a launch
+// that full tiles leave most compute units idle in.
+//
 // What bounds it: at full size the matrix cores at the clock the card holds under them (12288 x 2048, 6621 rows: a step takes 0.39 us
 // with every compute unit at work and 0.29 with one; the same loop over weights that are bf16 already, no vector work at all,
 // reaches 1157 TFLOP/s there, this one 1130 to 1157); below about 160 rows a tile the unpacking (0.14 us a step however few the rows);
@@ -247,24 +250,28 @@ struct Deq {
   }
 };
 
-// How a workgroup's wavefronts divide its tile: four of 64 columns, or two sets of four of 32 columns that have half of K each
-enum { kFour, kHalves };
+// How a workgroup's wavefronts divide its tile: four of 64 columns, four of 32, or two sets of four of 32 columns that have half of K each
+enum { kFour, kThin, kHalves };
 constexpr int tn_of(int form) { return form == kFour ? 2 : 1; }
-constexpr int threads_of(int form) { return form == kFour ? 256 : 512; }
-constexpr int cols_of(int form) { return form == kHalves ? 128 : kOwnCols; }
-constexpr int rows_of(int form) { return form == kHalves ? 128 : kOwnRows; }
+constexpr int sets_of(int form) { return form == kHalves ? 2 : 1; }
+constexpr int threads_of(int form) { return 256 * sets_of(form); }
+constexpr int cols_of(int form) { return form == kFour ? kOwnCols : 128; }
+constexpr int rows_of(int form) { return form == kFour ? kOwnRows : 128; }
 
-constexpr int kStages = 3;                          // of 64 k: 128 bytes of a row
-constexpr int kActs = kStages * kOwnRows * 128;      // LDS: activations (kHalves: a half for each set), then a part for each wavefront's codes
-constexpr int kCodes = kOwnCols * 192;               // ... and its scales
-constexpr int kScales = kOwnCols * 20 + 8 * 128;     // (kHalves: 128 bytes of each request for Q6_K's d are there twice)
-constexpr int kLds = kActs + kCodes + kScales;
+constexpr int kStages = 3;  // of 64 k: 128 bytes of a row
+// LDS: a set's activations, then a part for each wavefront's codes and one for its scales (Q6_K's d in a request of 64 words, half of them unused with
+// 32 columns). kThin has 77 KB, so that a compute unit holds two workgroups.
+constexpr int acts_of(int form) { return kStages * rows_of(form) * 128; }
+constexpr int codes_of(int form) { return 32 * tn_of(form) * 192; }
+constexpr int scales_of(int form) { return 512 * tn_of(form) + 256; }
+constexpr int lds_of(int form) { return sets_of(form) * (acts_of(form) + 4 * (codes_of(form) + scales_of(form))); }
 
 template <int KIND, int TM, int FORM, bool GATHER>
 __device__ __forceinline__ void own_tile(const OwnArgs& a, const OwnMat& mt, uint8_t* smem, int n0, int rows, int m0,
                                          int64_t wrow0, const uint32_t* pairs) {
   typedef Fmt<KIND> F;
   constexpr int TN = tn_of(FORM), STAGE = TM * 4096, SL = TN * TM;
+  constexpr int CODES = sets_of(FORM) * acts_of(FORM), SCALES = CODES + 4 * sets_of(FORM) * codes_of(FORM);  // where in LDS
   typedef Sc<KIND, TN> Z;
   constexpr int NC = TN * F::kInstr + Z::kReq;  // requests of a super-block's weights
   const int tid = threadIdx.x, lane = tid & 63, wave_of = __builtin_amdgcn_readfirstlane(tid >> 6), l32 = lane & 31, h = lane >> 5;
@@ -294,7 +301,7 @@ __device__ __forceinline__ void own_tile(const OwnArgs& a, const OwnMat& mt, uin
   const uint32_t dof = (uint32_t)min(n0 + 32 * TN * wave + (TN == 2 ? lane : l32), mt.O - 1) * (uint32_t)row_blocks * F::kD;  // Q6_K
   __builtin_amdgcn_sched_barrier(0);
   // request i of a slab's activations: eight rows of row block i, 128 bytes each
-  uint32_t* const s_dst = reinterpret_cast<uint32_t*>(smem + kLds);  // (gathered form)
+  uint32_t* const s_dst = reinterpret_cast<uint32_t*>(smem + lds_of(FORM));  // (gathered form)
   uint32_t* const s_src = s_dst + kOwnRows;
   uint32_t pr[TM];
   if constexpr (GATHER) {  // (the rows a wavefront asks for, eight of each block, go to a part of its own)
@@ -305,8 +312,8 @@ __device__ __forceinline__ void own_tile(const OwnArgs& a, const OwnMat& mt, uin
 #pragma unroll
     for (int i = 0; i < TM; ++i) pr[i] = m0 + min(32 * i + 8 * wave + (lane >> 3), rows - 1);
   }
-  uint8_t* const mine = smem + kActs + wave_of * (32 * TN * F::kQ);
-  const uint8_t* const my_scales = smem + kActs + kCodes + wave_of * (kScales / (FORM == kHalves ? 8 : 4));
+  uint8_t* const mine = smem + CODES + wave_of * (32 * TN * F::kQ);
+  const uint8_t* const my_scales = smem + SCALES + wave_of * scales_of(FORM);
   const uint32_t mine_at = lds_address(mine), scales_at = lds_address(my_scales);
   Z z[TN];
   // request I of a super-block's weights: the first (NEXT = 0), or the one after what was asked for before
@@ -332,7 +339,7 @@ __device__ __forceinline__ void own_tile(const OwnArgs& a, const OwnMat& mt, uin
     xo[i] = src * (2u * (uint32_t)a.K) + 16 * ((lane & 7) ^ ((4 * wave + (lane >> 4)) & 7));
   }
   const uint8_t* xg = reinterpret_cast<const uint8_t*>(a.x) + 512 * b0;
-  const uint32_t mem = set * (kActs / 2), at = lds_address(smem) + mem + wave * 1024;
+  const uint32_t mem = set * acts_of(FORM), at = lds_address(smem) + mem + wave * 1024;
 #pragma unroll
   for (int s = 0; s < kStages; ++s)
 #pragma unroll
@@ -499,9 +506,9 @@ __device__ __forceinline__ void own_tile(const OwnArgs& a, const OwnMat& mt, uin
 
 constexpr int kMixed = 2;  // the matrices of the launch differ in kind
 template <int KIND, int FORM, bool GATHER>
-__global__ __launch_bounds__(threads_of(FORM)) __attribute__((amdgpu_waves_per_eu(threads_of(FORM) / 256, threads_of(FORM) / 256))) void kq_mm_own_kernel(OwnArgs a) {
+__global__ __launch_bounds__(threads_of(FORM)) __attribute__((amdgpu_waves_per_eu(FORM == kFour ? 1 : 2, FORM == kFour ? 1 : 2))) void kq_mm_own_kernel(OwnArgs a) {
   // (one array: with more than one, the compiler does connect some reads with requests, and waits for everything in flight ahead of them)
-  __shared__ __attribute__((aligned(1024))) uint8_t smem[kLds + (GATHER ? 4 * (kOwnRows + 256) : 0)];
+  __shared__ __attribute__((aligned(1024))) uint8_t smem[lds_of(FORM) + (GATHER ? 4 * (kOwnRows + 256) : 0)];
   int rows, m0 = 0, tc, mat = 0;
   int64_t wrow0 = 0;
   const uint32_t* pairs = nullptr;
@@ -583,6 +590,16 @@ OwnMat kq_mm_own_mat(const ornith_kmatrix& w, void* y) {
   return {(const uint8_t*)w.d_qs, (const uint8_t*)w.d_scales, (const uint8_t*)w.d_dm, (bf16_t*)y, w.O, w.kind, w.O % 8 == 0 && ((uintptr_t)y & 15) == 0, 0};
 }
 
+// A plain launch's form. kFour and kThin give the same sums, so what shares a launch may decide between them: kThin while its tiles are
+// one a compute unit, as kFour leaves three of four idle then and its tile takes half as long again. us, kFour / kThin, Q4_K: 2560 x 2048 at 300 / 600 / 1200
+// rows 23 / 16, 23 / 16, 24 / 21, 3072 x 4096 at 600 43 / 28; past that (320 tiles) level: 2048 x 2600 x 2048 28 / 28, 8192 x 600 x 4096 52 / 56. Of few slabs
+// the ways in and out weigh most, and two workgroups a compute unit hide one another's: K = 512, 320 / 512 tiles, Q4_K 12 / 11, 14 / 13, Q6_K 13 / 12, 15 / 14.
+bool kq_mm_own_thin(const OwnArgs& a, int units) {
+  long tiles = 0;
+  for (int i = 0; i < a.n; ++i) tiles += (long)((a.m[i].O + 127) / 128) * ((a.M + 127) / 128);
+  return tiles <= (a.K <= 512 ? 2L : 1L) * units;
+}
+
 int kq_mm_own(ornith_ctx* ctx, OwnArgs& a, bool gather) {
   int kind = a.m[0].kind, grid, threads = 256;
   typedef void (*Kernel)(OwnArgs);
@@ -594,9 +611,9 @@ int kq_mm_own(ornith_ctx* ctx, OwnArgs& a, bool gather) {
     k = kind == ORNITH_Q4K ? kq_mm_own_kernel<ORNITH_Q4K, kFour, true> : kq_mm_own_kernel<ORNITH_Q6K, kFour, true>;
   } else {
     // Tile height: a tile takes about as long as 6 + its row blocks (kFour; K = 2048, one tile a compute unit, us: 8 blocks 53, 7 49, 6 44,
-    // 5 42; K = 4096 8 82, 5 61, 2 42), in the same measure 2.7 + 0.675 of them (kHalves; K = 2048 2 blocks 15, 3 18, 4 20; K = 4096 23, 27, 30),
-    // and the rounds of tiles count.
-    const int form = a.halves ? kHalves : kFour;
+    // 5 42; K = 4096 8 82, 5 61, 2 42), in the same measure 2.7 + 0.675 of them (kHalves; K = 2048 2 blocks 15, 3 18, 4 20; K = 4096 23, 27, 30; kThin 15, 19, 22;
+    // 27, 33, 37), and the rounds of tiles count.
+    const int form = a.halves ? kHalves : kq_mm_own_thin(a, ctx->compute_units) ? kThin : kFour;
     threads = threads_of(form);
     a.col_tiles = 0;
     for (int i = 0; i < a.n; ++i) {
@@ -607,13 +624,13 @@ int kq_mm_own(ornith_ctx* ctx, OwnArgs& a, bool gather) {
     long best = 0;
     for (int tm = rows_of(form) / 32; tm >= 2; --tm) {
       const long tiles = (long)((a.M + 32 * tm - 1) / (32 * tm)) * a.col_tiles, rounds = (tiles + ctx->compute_units - 1) / ctx->compute_units;
-      const long cost = rounds * (a.halves ? 4 + tm : 6 + tm);
+      const long cost = rounds * (form == kFour ? 6 + tm : 4 + tm);
       if (best == 0 || cost < best) best = cost, a.tile_rows = 32 * tm;
     }
     a.row_tiles = (a.M + a.tile_rows - 1) / a.tile_rows;
     grid = (a.row_tiles * a.col_tiles + 7) / 8 * 8;
 #define OWN(F) (kind == kMixed ? kq_mm_own_kernel<kMixed, F, false> : kind == ORNITH_Q4K ? kq_mm_own_kernel<ORNITH_Q4K, F, false> : kq_mm_own_kernel<ORNITH_Q6K, F, false>)
-    k = form == kFour ? OWN(kFour) : OWN(kHalves);
+    k = form == kFour ? OWN(kFour) : form == kThin ? OWN(kThin) : OWN(kHalves);
 #undef OWN
   }
   hipLaunchKernelGGL(k, dim3(grid), dim3(threads), 0, ctx->stream, a);

@@ -57,5 +57,11 @@ extern "C" int ornith_selftest_gemm_form(const ornith_linear* w, const void* d_x
   if (!w || w->mode != ORNITH_LIN_KQUANT) return -1;
   void* const y = const_cast<void*>(d_y);
   if (nmm::plain_ok(&w, 1, d_x, M, &y)) return 3;
-  return !kq_mm_own_suits(w->km, d_x, M) ? 0 : kq_mm_own_halves(w->km, M) ? 2 : 1;
+  if (!kq_mm_own_suits(w->km, d_x, M)) return 0;
+  OwnArgs a{};
+  a.m[0].O = w->km.O;
+  a.n = 1;
+  a.M = M;
+  a.K = w->km.K;
+  return kq_mm_own_halves(w->km, M) ? 2 : kq_mm_own_thin(a, 256) ? 4 : 1;
 }

@@ -72,6 +72,28 @@ def test_own_columns_experts_of_every_height(orn, ctx, kind, O, K):
     w.free()
 
 
+@pytest.mark.parametrize("kind", [Q4K, Q6K])
+@pytest.mark.parametrize("O,K,M", [(2056, 256, 300), (2051, 768, 257), (2056, 2048, 385), (2304, 512, 1400), (4104, 2048, 260)])
+def test_small_tiles_give_the_full_ones_sums(orn, ctx, kind, O, K, M):
+    """a matrix that by itself runs in 128 x 128 tiles, every number of row blocks and an end inside one: the same bits beside a matrix that fills
+    the device, where it runs in 256 x 256 ones, no store past the last row, and float64's numbers"""
+    rng = np.random.default_rng(O + K + M)
+    t, big = util.make_kq(kind, rng, 1, O, K), 32768
+    w = orn.Linear.kquant(ctx, kind, *t, O, K)
+    wide = orn.Linear.kquant(ctx, kind, *util.make_kq(kind, rng, 1, big, K), big, K)
+    assert orn.gemm_form(kind, O, K, M) == 4 and orn.gemm_form(kind, big, K, M) == 1
+    xb = util.bf16_normal(rng, (M, K))
+    dx, alone, beside, ybig = ctx.to_device(xb), ctx.alloc((M + 1) * O * 2), ctx.alloc((M + 1) * O * 2), ctx.alloc(M * big * 2)
+    for y in (alone, beside): ctx.memset(y, 0xFF, (M + 1) * O * 2)
+    ctx.linear_matmul(w, dx, M, alone)
+    ctx.linear_matmul_multi([wide, w], dx, M, [ybig, beside])
+    got = alone.download(np.uint16, (M + 1, O))
+    assert np.array_equal(got, beside.download(np.uint16, (M + 1, O)))
+    assert np.all(got[M] == 0xFFFF)
+    _check(got[:M], util.bf16_to_f32(xb).astype(np.float64), _deq(kind, t, 1, O, K)[0], (kind, O, K, M))
+    for b in (dx, alone, beside, ybig, w, wide): b.free()
+
+
 def test_own_columns_forms_in_one_call(orn, ctx):
     """matrices of one call whose sums are taken over K as a whole and in halves, and one that neither form takes: each the same bits as alone"""
     K, M, Os = 2048, 1100, (2304, 600, 264, 64)
