@@ -31,7 +31,7 @@ constexpr int kOwnRows = 256, kOwnCols = 256;  // a workgroup's tile (in halves 
 
 // alignment and reach: x of `rows` rows, any K % 256 == 0
 bool kq_mm_own_ok(const ornith_kmatrix& w, const void* x, size_t rows);
-// ... and M rows are many enough for this matrix, whatever shares its launch (and the option gemm_duo is on)
+// ... and M rows are many enough, whatever shares the launch (and the option gemm_duo is on); the few-row kernels come first
 bool kq_mm_own_suits(const ornith_kmatrix& w, const void* x, int M);
 // ... and then whether its sums are taken in two halves of K
 bool kq_mm_own_halves(const ornith_kmatrix& w, int M);

@@ -569,21 +569,17 @@ bool kq_mm_own_ok(const ornith_kmatrix& w, const void* x, size_t rows) {
          (((uintptr_t)x | (uintptr_t)w.d_qs) & 15) == 0 && (((uintptr_t)w.d_scales | (uintptr_t)w.d_dm) & 3) == 0;
 }
 
-// Rows from which a matrix runs here. Fewer take the few-row kernels (up to the lines of mm_narrow_host.h), whose splits suit
-// them, or kq_mm.hip's 128-row tiles. us, there / here: 8192 + 4096 columns of K = 2048, Q4_K, 100 / 129 rows 18 / 18, 25 / 18; 8192 + 512 + 512 Q6_K, where
-// the narrow two then want a launch of their own, 192 / 200 rows 23 / 24, 35 / 25; 2048 x 4096 Q4_K at 512 / 513 21 / 24, 30 / 24, Q6_K 25 / 28,
-// 36 / 28; 256 x 2048 Q6_K at 2000 / 3000 18 / 28, 29 / 28. Few slabs: 4096 x 1024 at 100 / 200 rows 7 / 9, 16 / 9; 2048 x 512 Q6_K at 2000 / 2500 rows 11 / 12,
-// 15 / 14.
-bool kq_mm_own_suits(const ornith_kmatrix& w, const void* x, int M) {
-  const int from = w.O > 2048 ? (w.kind == ORNITH_Q4K ? 128 : 192) : w.K < 2048 ? 2048 : w.O > 512 ? 512 : w.O > 256 ? 1024 : 2048;
-  return ornith_option_gemm_duo() && M > from && kq_mm_own_ok(w, x, M);
-}
+// What the few-row kernels don't take (up to the lines of mm_narrow_host.h, where their splits suit better) runs here from 129 rows on. us, kq_mm.hip's
+// 128-row tiles / here, Q4_K at 129 rows: 264 x 512 9.2 / 6.2, 264 x 2048 28 / 15, 2560 x 2048 28 / 13, 8192 x 4096 53 / 24.
+bool kq_mm_own_suits(const ornith_kmatrix& w, const void* x, int M) { return ornith_option_gemm_duo() && M > 128 && kq_mm_own_ok(w, x, M); }
 
-// ... and those that do it in kHalves, one matrix at a time whatever shares the launch, for the sums' order: while its tiles of 128
-// rows are one round of workgroups. us, kFour / kHalves: 8192 + 4096 columns of K = 2048, Q4_K, 200 / 256 / 300 rows 25 / 20, 27 / 21, 27 / 32;
-// 2048 x 4096 Q4_K at 1500 / 2000 / 2400 rows 43 / 32, 46 / 39, 47 / 53. Up to 512 columns are left to the launch of the wide matrices beside them.
+// ... and those that do it in kHalves, one matrix at a time whatever shares the launch, for the sums' order: up to the rows at which the widest launches that
+// bring it (12288 columns, 2048 with a few more) are one round of its tiles, so that none of them is split in two. us, kFour / kHalves: 8192 + 4096 columns of K = 2048, Q4_K,
+// 200 / 256 / 300 rows 25 / 20, 27 / 21, 27 / 32; 2048 x 4096 Q4_K at 1500 / 2000 / 2400 rows 43 / 32, 46 / 39, 47 / 53. A matrix in between, whose own tiles would be one round for
+// longer, has kThin past that (4096 x 2048 at 300 rows 14 here, 16 there). Up to 512 columns are left to the launch of the wide matrices beside them;
+// up to 2048 of K < 2048 are as fast in kThin and faster together in kFour (four of 2048 x 512 at 1025 / 2000 rows 20 / 30 here, 15 / 22 there).
 bool kq_mm_own_halves(const ornith_kmatrix& w, int M) {
-  return w.K % 512 == 0 && (w.O > 2048 ? M <= 256 : w.O > 512 && M <= 2048);
+  return w.K % 512 == 0 && (w.O > 2048 ? M <= 256 : w.O > 512 && w.K >= 2048 && M <= 2048);
 }
 
 OwnMat kq_mm_own_mat(const ornith_kmatrix& w, void* y) {

@@ -2,16 +2,30 @@
 // call, and the kernels of one weight family.
 #pragma once
 
+#include <algorithm>
+
 #include "mm_narrow.h"
 
 namespace nmm {
 
-// Rows up to which a k-quant projection takes these kernels; more go to the own-column kernel (kq_mm_own.hip, us, here / there).
-// More than 2048 columns: Q4_K 128 rows (8192 + 4096 x 2048 at 100 / 129 rows 18 / 18, 25 / 18), Q6_K 192 (8192 + 512 + 512 x 2048, of which the narrow ones
-// then run by themselves, at 192 / 200 23 / 24, 35 / 25). Up to 2048 columns, from K = 2048 on: 512 rows (2048 x 4096 Q4_K at 512 / 513 21 / 24, 30 / 24, Q6_K 25 / 28,
-// 36 / 28); up to 512 columns, which rarely come alone, 1024 and of Q4_K 1536; up to 256, a handful of workgroups there, 2560 (256 x 2048 at 1200 /
-// 2000 / 2500 rows 13 / 28, 18 / 28, 21 / 28). Below K = 2048 1024 rows (2048 x 512 at 1024 10.9 / 10.6).
-constexpr int kNarrowRows = 192, kNarrowRowsQ4K = 128, kNarrowRowsMid = 512, kNarrowRowsSlim = 1024, kNarrowRowsSlimQ4K = 1536, kNarrowRowsSlimmest = 2560;
+// Rows up to which a k-quant projection takes these kernels; more go to the own-column kernel (kq_mm_own.hip, us, here / there). One matrix at a time,
+// never by what shares its launch: a matrix gives the same bits alone and in company.
+// More than 512 columns: up to 2^20 outputs, about where these kernels' 64-row tiles no longer are one a compute unit (Q4_K x 2048: 1536 columns at 600 / 800 rows
+// 13 / 14, 18 / 14, 2048 at 400 / 513 12 / 13, 15 / 14, 3072 at 300 / 400 13 / 16, 18 / 16; x 4096: 2048 at 513 / 600 24 / 24, 30 / 25; Q6_K x 4096: 2048 at 400 /
+// 600 25 / 28, 37 / 30), of fewer than 1820 columns 576 rows, of fewer than 910 2^19 outputs: one of those alone is no faster there up to 2^20 either, two
+// together are (Q4_K x 4096: 768 at 600 / 800 16 / 24, 24 / 24, 1024 at 513 / 600 / 800 17 / 24, 23 / 24, 22 / 24, two of them at 513 / 700 24 / 24, 30 / 24).
+// From 4096 columns on, which come with others as wide, Q4_K 128 rows (8192 + 4096 x 2048 at 100 / 129 rows 18 / 18, 25 / 18), Q6_K 192 (8192 + 512 + 512
+// x 2048, of which the narrow ones then run by themselves, at 192 / 200 23 / 24, 35 / 25).
+// Up to 512 columns, which rarely come alone, 1024 and of Q4_K 1536; up to 256, a handful of workgroups there, 2560 (256 x 2048 at 1200 / 2000 rows 13 / 15,
+// 18 / 15). Below K = 2048 1024 rows up to 2048 columns (264 x 512 at 1025 / 2000 5 / 6, 7 / 6; 2048 x 1024 at 400 / 600 9 / 10, 12 / 10, with two of 512 columns, which
+// then run by themselves, at 513 12 / 16).
+constexpr int kNarrowOutputs = 1 << 20, kNarrowRows = 192, kNarrowRowsQ4K = 128, kNarrowRowsMid = 576, kNarrowRowsSlim = 1024, kNarrowRowsSlimQ4K = 1536,
+              kNarrowRowsSlimmest = 2560;
+inline int kq_rows(bool q4, int O, int K) {
+  if (O >= 4096) return q4 ? kNarrowRowsQ4K : kNarrowRows;
+  if (O > 2048 || (O > 512 && K >= 2048)) return std::min(kNarrowOutputs / O, std::max(kNarrowOutputs / 2 / O, kNarrowRowsMid));
+  return K < 2048 ? kNarrowRowsSlim : O <= 256 ? kNarrowRowsSlimmest : q4 && O <= 512 ? kNarrowRowsSlimQ4K : kNarrowRowsSlim;
+}
 // The affine formats have no wide kernels: their projections own columns from here on (4-bit, 12288 x 2048, us, split /
 // owned: 300 rows 37 / 37, 400 rows 50 / 52, 512 rows 56 / 51, 600 rows 68 / 61, 2000 rows 207 / 187).
 constexpr int kTallFromAffine = 448;

@@ -64,13 +64,9 @@ bool plain_ok(const ornith_linear* const* ws, int n, const void* d_x, int M, voi
     if (ws[i]->mode == ORNITH_LIN_KQUANT && (ws[i]->km.E != 1 || ws[i]->km.O != ws[i]->O || ws[i]->km.K != K)) return false;
   }
   if (K > 4096) return false;  // (the scales of a workgroup's rows would not fit beside the activations)
-  // (see kNarrowRows; the affine formats have no wider kernels)
-  if (affine(kind_of(*ws[0]))) return true;
-  for (int i = 0; i < n; ++i) {
-    const bool q4 = ws[i]->km.kind == ORNITH_Q4K;
-    const int slim = K < 2048 ? kNarrowRowsSlim : ws[i]->O <= 256 ? kNarrowRowsSlimmest : ws[i]->O > 512 ? kNarrowRowsMid : q4 ? kNarrowRowsSlimQ4K : kNarrowRowsSlim;
-    if (M > (ws[i]->O <= 2048 ? slim : q4 ? kNarrowRowsQ4K : kNarrowRows)) return false;
-  }
+  if (affine(kind_of(*ws[0]))) return true;  // (no wider kernels)
+  for (int i = 0; i < n; ++i)
+    if (M > kq_rows(ws[i]->km.kind == ORNITH_Q4K, ws[i]->O, K)) return false;
   return true;
 }
 

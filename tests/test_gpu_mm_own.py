@@ -73,7 +73,7 @@ def test_own_columns_experts_of_every_height(orn, ctx, kind, O, K):
 
 
 @pytest.mark.parametrize("kind", [Q4K, Q6K])
-@pytest.mark.parametrize("O,K,M", [(2056, 256, 300), (2051, 768, 257), (2056, 2048, 385), (2304, 512, 1400), (4104, 2048, 260)])
+@pytest.mark.parametrize("O,K,M", [(2056, 256, 300), (2051, 768, 257), (2056, 2048, 609), (2304, 512, 1400), (4104, 2048, 260)])
 def test_small_tiles_give_the_full_ones_sums(orn, ctx, kind, O, K, M):
     """a matrix that by itself runs in 128 x 128 tiles, every number of row blocks and an end inside one: the same bits beside a matrix that fills
     the device, where it runs in 256 x 256 ones, no store past the last row, and float64's numbers"""

@@ -59,7 +59,7 @@ def test_kq_matmul_vs_float64(orn, ctx, kind, O, K, M):
 
 @pytest.mark.parametrize("mats,K,M", [
     # 256-row tiles, ragged and whole (enough of them to fill the device), 128-row ones, wide matrices of both kinds, narrow ones that share a launch
-    ([(Q4K, 8192)], 512, 1061), ([(Q6K, 8192)], 512, 1024), ([(Q4K, 2056)], 512, 300), ([(Q4K, 4096), (Q6K, 4096)], 512, 1061),
+    ([(Q4K, 8192)], 512, 1061), ([(Q6K, 8192)], 512, 1024), ([(Q4K, 2056)], 256, 300), ([(Q4K, 4096), (Q6K, 4096)], 512, 1061),
     ([(Q4K, 600), (Q6K, 264)], 256, 300)])
 def test_kq_matmul_weights_through_lds(orn, ctx, mats, K, M):
     """gemm_duo = 0: every matrix through the tiles that unpack into LDS, the same bits in company as alone"""
