@@ -853,6 +853,8 @@ ORNITH_API int ornith_selftest_unary(ornith_ctx* ctx, int fn, const float* d_in,
  * 0 weights through LDS, 1 wavefronts own columns, 2 ... of two halves of K, 3 the few-row kernels, 4 as 1 (with the same sums) in smaller tiles, as
  * it does by itself on 256 compute units. -1: not a k-quant matrix. */
 ORNITH_API int ornith_selftest_gemm_form(const ornith_linear* w, const void* d_x, int M, const void* d_y);
+/* ... and that ornith_kq_gather_matmul takes (0, 1, 3 or 4; -1: no such call). */
+ORNITH_API int ornith_selftest_gather_form(const ornith_kmatrix* w, const void* d_x, int pairs, int top_k, int is_up, const void* d_y);
 
 /* ---- machine probes (`bench.py --ceiling`) ------------------------------------------
  * No reference counterpart (the reference times its own dispatches from the host,

@@ -201,6 +201,12 @@ def gemm_form(kind, O, K, M, x=4096, qs=4096, scales=4096, dm=4096, y=4096):
     return lib().ornith_selftest_gemm_form(C.byref(s), C.c_void_p(x), M, C.c_void_p(y))
 
 
+def gather_form(kind, E, O, K, pairs, top_k=1, is_up=False, x=4096, qs=4096, scales=4096, dm=4096, y=4096):
+    """The form of the experts' GEMM for a k-quant stack at those addresses (ornith_selftest_gather_form; no GPU needed)."""
+    s = KMatrixStruct(kind, E, O, K, qs, scales, dm)
+    return lib().ornith_selftest_gather_form(C.byref(s), C.c_void_p(x), pairs, top_k, int(is_up), C.c_void_p(y))
+
+
 class MoeWeightsStruct(C.Structure):
     _fields_ = [("router", LinearStruct), ("ex_gate", KMatrixStruct), ("ex_up", KMatrixStruct),
                 ("ex_down", KMatrixStruct), ("sh_gate", LinearStruct), ("sh_up", LinearStruct),

@@ -682,8 +682,50 @@ int ornith_kq_matmul(ornith_ctx* ctx, const ornith_kmatrix* w, const void* d_x, 
   return ornith_kq_matmul_multi(ctx, &w, 1, d_x, M, &d_y);
 }
 
-// Pairs an expert from which a matrix that the few-row kernels don't take runs in the form whose wavefronts own columns.
+}  // extern "C"
+
+namespace {
+
+// Pairs an expert from which a matrix that the few-row kernels don't take runs in the form whose wavefronts own columns, for K >= 1024 (us, LDS form / there, Q4_K, 48 rows an
+// expert: 512 x 4352, 4 / 64 / 128 experts 42 / 29, 67 / 48, 108 / 97, 2048 x 8192, 8 experts 93 / 61; fewer slabs, 2048 x 256 at 16 / 256
+// experts 6.6 / 7.6, 50 / 56, 131 x 512 at 16 / 256 8.9 / 10, 17 / 19).
 constexpr int kOwnPairs = 48;
+
+struct GatherRoute {
+  int tile_rows;  // of the plan: depends only on pairs and E (and the option), so the calls sharing a plan agree on it
+  int lds_rows;   // a workgroup's in the LDS form
+  bool few, own, low;
+};
+
+// Rows per plan tile: with nmm::kNarrowPairs rows an expert or more 256, the own-column form's most: nearly every expert
+// is one tile there (its weights are dequantized once), and one of fewer rows runs the loop for the rows it has.
+// Otherwise the few-row kernels' 16 / 32 / 64 rows, the smallest that most experts' shares fit.
+// The kernel for this matrix: with few rows an expert the few-row kernels (mm_narrow.h). Tall plans, and from kOwnPairs rows an
+// expert on the matrices that the few-row kernels don't take (K > 4096, rows whose scales are no whole 16-byte
+// pieces; their 64-row tiles are worked on four at a time), take the own-column form where its alignment holds.
+// Otherwise the LDS form: 128 rows a workgroup from 96 rows an expert on and K >= 1024, else 64. A plan tile
+// taller than its kernel's workgroups is split over several of them.
+GatherRoute gather_route(const ornith_kmatrix& w, const void* d_x, int pairs, int top_k, bool is_up, const void* d_y) {
+  const int avg = pairs / w.E;
+  const bool narrow = pairs < nmm::kNarrowPairs * w.E, reg = ornith_option_gemm_reg();
+  const size_t x_rows = (size_t)(is_up ? pairs / top_k : pairs);
+  GatherRoute r;
+  r.tile_rows = narrow ? nmm::tile_rows(pairs, w.E) : reg ? kOwnRows : avg >= 96 ? 128 : 64;
+  r.lds_rows = avg >= 96 && w.K >= 1024 ? 128 : 64;
+  r.few = narrow && nmm::experts_ok(&w, d_x, x_rows, d_y);
+  r.low = narrow && !r.few && pairs >= kOwnPairs * w.E && w.K >= 1024 && reg;
+  r.own = ((reg && !narrow) || r.low) && kq_mm_own_ok(w, d_x, x_rows);
+  return r;
+}
+
+}  // namespace
+
+int kq_gather_form(const ornith_kmatrix& w, const void* d_x, int pairs, int top_k, bool is_up, const void* d_y, int units) {
+  const GatherRoute r = gather_route(w, d_x, pairs, top_k, is_up, d_y);
+  return r.few ? 3 : !r.own ? 0 : kq_mm_own_thin_experts(w.O, w.E, pairs, units) ? 4 : 1;
+}
+
+extern "C" {
 
 // gather plan: expert-sorted pairs and the tile list, in caller-provided device memory
 // (ornith_kq_gather_plan_bytes(pairs, E) bytes)
@@ -697,29 +739,12 @@ int ornith_kq_gather_matmul(ornith_ctx* ctx, const ornith_kmatrix* w, const void
   if (rc) return rc;
   ORN_REQUIRE(pairs >= 1 && top_k >= 1 && pairs % top_k == 0 && w->E <= 1024,
               "kq_gather_matmul: pairs=%d top_k=%d E=%d", pairs, top_k, w->E);
-  // Rows per plan tile: the choice depends only on pairs and E (and the option), so the calls
-  // sharing a plan agree on it. With nmm::kNarrowPairs rows an expert or more 256, the own-column form's most: nearly every expert
-  // is one tile there (its weights are dequantized once), and one of fewer rows runs the loop for the rows it has.
-  // Otherwise the few-row kernels' 16 / 32 / 64 rows, the smallest that most experts' shares fit.
-  const int avg = pairs / w->E;
-  const bool narrow = pairs < nmm::kNarrowPairs * w->E;
-  const bool tall = ornith_option_gemm_reg() && !narrow;
-  const int tile_rows = narrow ? nmm::tile_rows(pairs, w->E) : tall ? kOwnRows : avg >= 96 ? 128 : 64;
-  // The kernel for this matrix. Few rows an expert: the few-row kernels (mm_narrow.h). Tall plans, and from 48 rows an
-  // expert on the matrices that the few-row kernels don't take (K > 4096, rows whose scales are no whole 16-byte
-  // pieces; their 64-row tiles are worked on four at a time), take the own-column form where its alignment holds.
-  // Otherwise the LDS form: 128 rows a workgroup from 96
-  // rows an expert on and K >= 1024, else 64. A plan tile taller than its kernel's workgroups is
-  // split over several of them.
-  const size_t x_rows = (size_t)(is_up ? pairs / top_k : pairs);
-  const bool few = narrow && nmm::experts_ok(w, d_x, x_rows, d_y);
-  const bool low = narrow && !few && pairs >= kOwnPairs * w->E && ornith_option_gemm_reg();
-  const int lds_rows = (avg >= 96 && w->K >= 1024) ? 128 : 64;
+  const GatherRoute r = gather_route(*w, d_x, pairs, top_k, is_up != 0, d_y);
   nmm::Plan pl;
-  rc = moe_plan(ctx, d_inds, pairs, w->E, tile_rows, 0, d_plan, rebuild_plan != 0, &pl);
+  rc = moe_plan(ctx, d_inds, pairs, w->E, r.tile_rows, 0, d_plan, rebuild_plan != 0, &pl);
   if (rc) return rc;
-  if (few) return nmm::gathered(ctx, w, nullptr, d_x, pairs, is_up ? top_k : 1, pl, d_y);
-  if ((tall || low) && kq_mm_own_ok(*w, d_x, x_rows)) {
+  if (r.few) return nmm::gathered(ctx, w, nullptr, d_x, pairs, is_up ? top_k : 1, pl, d_y);
+  if (r.own) {
     OwnArgs o{};
     o.m[0] = kq_mm_own_mat(*w, d_y);
     o.n = 1;
@@ -733,7 +758,7 @@ int ornith_kq_gather_matmul(ornith_ctx* ctx, const ornith_kmatrix* w, const void
     o.n_tiles = pl.n_tiles;
     o.tiles_max = (int)pl.tiles_max;
     o.up_div = is_up ? top_k : 1;
-    o.expert_at = low ? pl.expert_at : nullptr;
+    o.expert_at = r.low ? pl.expert_at : nullptr;
     o.E = w->E;
     return kq_mm_own(ctx, o, true);
   }
@@ -753,9 +778,9 @@ int ornith_kq_gather_matmul(ornith_ctx* ctx, const ornith_kmatrix* w, const void
   a.tile_start = pl.tile_start;
   a.tile_count = pl.tile_count;
   a.n_tiles = pl.n_tiles;
-  a.sub = (tile_rows + lds_rows - 1) / lds_rows;
+  a.sub = (r.tile_rows + r.lds_rows - 1) / r.lds_rows;
   const dim3 grid((w->O + BN - 1) / BN, (unsigned)(pl.tiles_max * a.sub));
-  if (lds_rows == 128) {
+  if (r.lds_rows == 128) {
     if (w->kind == ORNITH_Q4K)
       hipLaunchKernelGGL((kq_mm_kernel<ORNITH_Q4K, 128, true>), grid, dim3(256), 0, ctx->stream, a);
     else

@@ -37,5 +37,9 @@ bool kq_mm_own_suits(const ornith_kmatrix& w, const void* x, int M);
 bool kq_mm_own_halves(const ornith_kmatrix& w, int M);
 // whether a plain launch of whole sums over K takes tiles of 128 x 128 (a.m[].O, n, M, K), on a device of that many compute units: the sums are the same
 bool kq_mm_own_thin(const OwnArgs& a, int units);
+// ... and a gathered one, by its experts' columns and the pairs of them all
+bool kq_mm_own_thin_experts(int O, int E, int pairs, int units);
+// kq_mm.hip: the form that kq_gather_matmul takes, as ornith_selftest_gather_form gives it
+int kq_gather_form(const ornith_kmatrix& w, const void* d_x, int pairs, int top_k, bool is_up, const void* d_y, int units);
 OwnMat kq_mm_own_mat(const ornith_kmatrix& w, void* y);
 int kq_mm_own(ornith_ctx* ctx, OwnArgs& a, bool gather);

@@ -514,7 +514,12 @@ __global__ __launch_bounds__(threads_of(FORM)) __attribute__((amdgpu_waves_per_e
   const uint32_t* pairs = nullptr;
   const uint32_t die = blockIdx.x & 7, seq = blockIdx.x >> 3;
   if constexpr (GATHER) {
-    const uint32_t tile = seq / (uint32_t)a.col_tiles * 8u + die, at = min(tile, (uint32_t)a.tiles_max - 1u), n = *a.n_tiles;
+    // The columns over a plan's tile stay on one die, whose cache its rows then stay in. kThin: first all tiles' upper 128 rows, then the lower ones, which
+    // not every tile has (taken in turn they fall on every other die, and half the dies idle: 512 x 4352, 64 experts of 207 rows 96 us, round the dies
+    // column by column 145)
+    const uint32_t unit = seq / (uint32_t)a.col_tiles * 8u + die, tiles = ((uint32_t)a.tiles_max + 7u) / 8u * 8u;
+    const uint32_t sub = FORM == kThin && unit >= tiles ? 1u : 0u, tile = unit - sub * tiles;
+    const uint32_t at = min(tile, (uint32_t)a.tiles_max - 1u), n = *a.n_tiles;
     tc = (int)(seq % (uint32_t)a.col_tiles);
     const uint32_t e = __builtin_amdgcn_readfirstlane(a.tile_expert[at]);
     rows = __builtin_amdgcn_readfirstlane((int)a.tile_count[at]);
@@ -526,6 +531,11 @@ __global__ __launch_bounds__(threads_of(FORM)) __attribute__((amdgpu_waves_per_e
       const int end = (int)e + 1 < a.E ? (int)__builtin_amdgcn_readfirstlane(a.expert_at[e + 1]) : a.M;
       if ((st - first) % kOwnRows != 0) return;
       rows = min(end - st, kOwnRows);
+    }
+    if constexpr (FORM == kThin) {
+      rows = min(rows - (int)(sub * 128), 128);
+      if (rows <= 0) return;
+      pairs += sub * 128;
     }
     wrow0 = (int64_t)e * a.m[0].O;
   } else {
@@ -596,15 +606,25 @@ bool kq_mm_own_thin(const OwnArgs& a, int units) {
   return tiles <= (a.K <= 512 ? 2L : 1L) * units;
 }
 
+// ... and a gathered one's (the tiles are in the device's hands: what the host knows of them is the experts' mean), while kFour would leave half the compute units
+// idle and more. us, Q4_K, kFour / kThin, rows an expert: 2048 x 512, 8 experts of 128 / 300 13 / 9.1, 19 / 11, 16 of 207 19 / 19, 32 of 128 19 / 22;
+// 512 x 2048, 16 experts of 128 45 / 21, 64 of 80 / 207 34 / 28, 49 / 51, 128 of 80 42 / 49; 512 x 4352, 16 of 207 87 / 42, 64 of 128 91 / 76.
+bool kq_mm_own_thin_experts(int O, int E, int pairs, int units) {
+  return 2L * E * ((pairs / E + kOwnRows - 1) / kOwnRows) * ((O + kOwnCols - 1) / kOwnCols) <= units;
+}
+
 int kq_mm_own(ornith_ctx* ctx, OwnArgs& a, bool gather) {
   int kind = a.m[0].kind, grid, threads = 256;
   typedef void (*Kernel)(OwnArgs);
   Kernel k;
   if (gather) {
     a.up_magic = dm_div_magic(a.up_div);
-    a.col_tiles = (a.m[0].O + kOwnCols - 1) / kOwnCols;
-    grid = a.col_tiles * ((a.tiles_max + 7) / 8 * 8);
-    k = kind == ORNITH_Q4K ? kq_mm_own_kernel<ORNITH_Q4K, kFour, true> : kq_mm_own_kernel<ORNITH_Q6K, kFour, true>;
+    const bool thin = kq_mm_own_thin_experts(a.m[0].O, a.E, a.M, ctx->compute_units);
+    const int cols = cols_of(thin ? kThin : kFour);
+    a.col_tiles = (a.m[0].O + cols - 1) / cols;
+    grid = a.col_tiles * ((a.tiles_max + 7) / 8 * 8) * (thin ? 2 : 1);
+    k = kind == ORNITH_Q4K ? (thin ? kq_mm_own_kernel<ORNITH_Q4K, kThin, true> : kq_mm_own_kernel<ORNITH_Q4K, kFour, true>)
+                           : (thin ? kq_mm_own_kernel<ORNITH_Q6K, kThin, true> : kq_mm_own_kernel<ORNITH_Q6K, kFour, true>);
   } else {
     // Tile height: a tile takes about as long as 6 + its row blocks (kFour; K = 2048, one tile a compute unit, us: 8 blocks 53, 7 49, 6 44,
     // 5 42; K = 4096 8 82, 5 61, 2 42), in the same measure 2.7 + 0.675 of them (kHalves; K = 2048 2 blocks 15, 3 18, 4 20; K = 4096 23, 27, 30; kThin 15, 19, 22;

@@ -53,6 +53,11 @@ extern "C" int ornith_selftest_unary(ornith_ctx* ctx, int fn, const float* d_in,
   return ORNITH_OK;
 }
 
+extern "C" int ornith_selftest_gather_form(const ornith_kmatrix* w, const void* d_x, int pairs, int top_k, int is_up, const void* d_y) {
+  if (!w || w->E < 1 || pairs < 1 || top_k < 1) return -1;
+  return kq_gather_form(*w, d_x, pairs, top_k, is_up != 0, d_y, 256);
+}
+
 extern "C" int ornith_selftest_gemm_form(const ornith_linear* w, const void* d_x, int M, const void* d_y) {
   if (!w || w->mode != ORNITH_LIN_KQUANT) return -1;
   void* const y = const_cast<void*>(d_y);

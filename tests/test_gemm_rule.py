@@ -38,3 +38,14 @@ def test_rows_at_which_the_forms_change(orn, kind, O, K, M, form):
     (12288, 2048, 257, OWN)])
 def test_a_launch_of_few_full_tiles_takes_small_ones(orn, kind, O, K, M, form):
     assert orn.gemm_form(kind, O, K, M) == form
+
+
+@pytest.mark.parametrize("kind", [Q4K, Q6K])
+@pytest.mark.parametrize("E,O,K,avg,form", [
+    # what the few-row kernels don't take, from 48 pairs an expert: not of few slabs
+    (16, 131, 512, 48, LDS), (256, 2048, 256, 79, LDS), (256, 512, 4352, 47, LDS), (256, 512, 4352, 48, OWN), (16, 512, 4352, 48, THIN),
+    # 80 pairs an expert and more: small tiles while large ones are half the compute units or fewer
+    (256, 2048, 512, 79, FEW), (256, 2048, 512, 80, OWN), (16, 2048, 512, 256, THIN), (16, 2048, 512, 257, OWN), (17, 2048, 512, 80, OWN),
+    (64, 512, 2048, 207, THIN), (65, 512, 2048, 207, OWN), (16, 131, 512, 600, THIN)])
+def test_experts_of_few_full_tiles_take_small_ones(orn, kind, E, O, K, avg, form):
+    assert orn.gather_form(kind, E, O, K, E * avg) == form

@@ -49,22 +49,30 @@ def test_own_columns_matmul(orn, ctx, kind, O, K, M):
     w.free()
 
 
-@pytest.mark.parametrize("kind,O,K", [(Q4K, 264, 512), (Q6K, 131, 256), (Q6K, 512, 768), (Q4K, 1032, 2048)])
-def test_own_columns_experts_of_every_height(orn, ctx, kind, O, K):
+TALL = (1, 31, 32, 33, 64, 65, 97, 128, 129, 161, 192, 193, 225, 256, 257, 0, 555)
+LOW = (1, 31, 32, 33, 64, 65, 0, 97, 48, 20, 129, 7, 12, 260, 3)  # 53 an expert: a plan of tiles lower than the kernel's
+
+
+@pytest.mark.parametrize("counts,kind,O,K", [
+    # tiles of 128 x 128, while larger ones are half the compute units or fewer
+    (TALL, Q4K, 264, 512), (TALL, Q6K, 131, 256), (TALL, Q6K, 512, 768), (TALL, Q4K, 1032, 2048), (LOW, Q4K, 264, 4352), (LOW, Q6K, 131, 1280),
+    # ... of 256 x 256
+    (TALL, Q4K, 2056, 512), (TALL, Q6K, 2051, 256), (TALL, Q6K, 2304, 768), (LOW, Q4K, 2312, 4352), (LOW, Q6K, 2307, 1280)])
+def test_own_columns_experts_of_every_height(orn, ctx, counts, kind, O, K):
     """an expert of each number of 32-row blocks, one row to either side of a block's end, one without rows, one of several tiles"""
-    counts = [1, 31, 32, 33, 64, 65, 97, 128, 129, 161, 192, 193, 225, 256, 257, 0, 555]
     E, pairs = len(counts), sum(counts)
-    assert pairs >= 80 * E
+    assert pairs >= (80 if counts is TALL else 48) * E and orn.gather_form(kind, E, O, K, pairs) == (1 if O > 2048 else 4)
     rng = np.random.default_rng(O + K)
     t = util.make_kq(kind, rng, E, O, K)
     w = orn.KMatrix(ctx, kind, *t, E, O, K)
     inds = rng.permutation(np.repeat(np.arange(E), counts)).astype(np.uint32)
     xb = util.bf16_normal(rng, (pairs, K))
     plan = ctx.alloc(orn.kq_gather_plan_bytes(pairs, E))
-    di, dx, dy = ctx.to_device(inds), ctx.to_device(xb), ctx.alloc(pairs * O * 2)
-    ctx.memset(dy, 0xFF, pairs * O * 2)
+    di, dx, dy = ctx.to_device(inds), ctx.to_device(xb), ctx.alloc((pairs + 1) * O * 2)
+    ctx.memset(dy, 0xFF, (pairs + 1) * O * 2)
     orn.kq_gather_matmul(ctx, w, dx, di, pairs, 1, False, plan, True, dy)
-    got, x, deq = dy.download(np.uint16, (pairs, O)), util.bf16_to_f32(xb).astype(np.float64), _deq(kind, t, E, O, K)
+    got, x, deq = dy.download(np.uint16, (pairs + 1, O)), util.bf16_to_f32(xb).astype(np.float64), _deq(kind, t, E, O, K)
+    assert np.all(got[pairs] == 0xFFFF)
     for e in range(E):
         sel = np.nonzero(inds == e)[0]
         if len(sel): _check(got[sel], x[sel], deq[e], (kind, O, K, counts[e]))
