@@ -8,7 +8,6 @@ struct OwnMat {
   const uint8_t *qs, *scales, *dm;
   bf16_t* y;
   int O, kind;
-  int vec;  // rows of y can be stored 16 bytes at a time
   int t0;  // plain form: first column tile of the launch that is this matrix's
 };
 
