@@ -517,10 +517,10 @@ __global__ __launch_bounds__(threads_of(FORM)) __attribute__((amdgpu_waves_per_e
   const uint32_t die = blockIdx.x & 7, seq = blockIdx.x >> 3;
   if constexpr (GATHER) {
     // The columns over a plan's tile stay on one die, whose cache its rows then stay in. kThin: first all tiles' upper 128 rows, then the lower ones, which
-    // not every tile has (taken in turn they fall on every other die, and half the dies idle: 512 x 4352, 64 experts of 207 rows 96 us, round the dies
-    // column by column 145)
-    const uint32_t unit = seq / (uint32_t)a.col_tiles * 8u + die, tiles = ((uint32_t)a.tiles_max + 7u) / 8u * 8u;
-    const uint32_t sub = FORM == kThin && unit >= tiles ? 1u : 0u, tile = unit - sub * tiles;
+    // not every tile has, four dies on (taken in turn they fall on every other die, and half the dies idle: 512 x 4352, 64 experts of 207 rows, round
+    // the dies column by column 145 us, in turn 96)
+    const uint32_t eights = ((uint32_t)a.tiles_max + 7u) / 8u, at8 = seq / (uint32_t)a.col_tiles;
+    const uint32_t sub = FORM == kThin && at8 >= eights ? 1u : 0u, tile = (at8 - sub * eights) * 8u + ((die + 4u * sub) & 7u);
     const uint32_t at = min(tile, (uint32_t)a.tiles_max - 1u), n = *a.n_tiles;
     tc = (int)(seq % (uint32_t)a.col_tiles);
     const uint32_t e = __builtin_amdgcn_readfirstlane(a.tile_expert[at]);
