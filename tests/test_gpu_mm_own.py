@@ -25,7 +25,8 @@ def _check(got_bits, x, w, what):
 
 
 @pytest.mark.parametrize("kind,O,K,M", [
-    # the lowest row counts of the rule: wide matrices of K >= 2048 and below, narrow ones
+    # the lowest row counts of the rule; columns that end inside a tile
+    (Q4K, 40, 256, 129), (Q6K, 264, 768, 129), (Q4K, 2304, 768, 129),
     (Q4K, 2056, 2048, 193), (Q6K, 2056, 2304, 193), (Q4K, 2304, 256, 513), (Q6K, 2051, 768, 545), (Q6K, 72, 256, 2049),
     (Q4K, 257, 2048, 1025 + 512),
     # two sets of wavefronts with half of K each: one super-block a set and an odd number, the ends of the rule, columns and rows that
@@ -41,10 +42,12 @@ def test_own_columns_matmul(orn, ctx, kind, O, K, M):
     t = util.make_kq(kind, rng, 1, O, K)
     w = orn.KMatrix(ctx, kind, *t, 1, O, K)
     xb = util.bf16_normal(rng, (M, K))
-    dx, dy = ctx.to_device(xb), ctx.alloc(M * O * 2)
-    ctx.memset(dy, 0xFF, M * O * 2)
+    dx, dy = ctx.to_device(xb), ctx.alloc((M + 1) * O * 2)
+    ctx.memset(dy, 0xFF, (M + 1) * O * 2)
     orn.kq_matmul(ctx, w, dx, M, dy)
-    _check(dy.download(np.uint16, (M, O)), util.bf16_to_f32(xb).astype(np.float64), _deq(kind, t, 1, O, K)[0], (kind, O, K, M))
+    got = dy.download(np.uint16, (M + 1, O))
+    assert np.all(got[M] == 0xFFFF)
+    _check(got[:M], util.bf16_to_f32(xb).astype(np.float64), _deq(kind, t, 1, O, K)[0], (kind, O, K, M))
     for b in (dx, dy): b.free()
     w.free()
 
@@ -100,6 +103,32 @@ def test_small_tiles_give_the_full_ones_sums(orn, ctx, kind, O, K, M):
     assert np.all(got[M] == 0xFFFF)
     _check(got[:M], util.bf16_to_f32(xb).astype(np.float64), _deq(kind, t, 1, O, K)[0], (kind, O, K, M))
     for b in (dx, alone, beside, ybig, w, wide): b.free()
+
+
+@pytest.mark.parametrize("mats,K,M,form", [
+    # a gated-delta layer's two wide projections; both kinds, columns that end inside a tile, more than one round of tiles; the ends of the rule
+    ([(Q4K, 8192), (Q4K, 4096)], 2048, 200, 2), ([(Q4K, 1032), (Q6K, 2043)], 2048, 700, 2), ([(Q6K, 2048), (Q4K, 1800), (Q6K, 2041)], 2048, 2048, 2),
+    ([(Q6K, 4104), (Q4K, 4100), (Q6K, 4097), (Q4K, 4096)], 512, 256, 2),
+    # small tiles over all of K: both kinds, three and four matrices
+    ([(Q4K, 2060), (Q6K, 2051), (Q6K, 300)], 768, 1025, 4)])
+def test_matrices_of_one_form_share_a_launch(orn, ctx, mats, K, M, form):
+    """each the same bits as alone, and float64's numbers; no store past the last row"""
+    rng = np.random.default_rng(M + K)
+    ts = [util.make_kq(kind, rng, 1, O, K) for kind, O in mats]
+    ws = [orn.Linear.kquant(ctx, kind, *t, O, K) for (kind, O), t in zip(mats, ts)]
+    xb = util.bf16_normal(rng, (M, K))
+    dx, ys, alone = ctx.to_device(xb), [ctx.alloc((M + 1) * O * 2) for _, O in mats], ctx.alloc(M * max(O for _, O in mats) * 2)
+    for (_, O), y in zip(mats, ys): ctx.memset(y, 0xFF, (M + 1) * O * 2)
+    ctx.linear_matmul_multi(ws, dx, M, ys)
+    x = util.bf16_to_f32(xb).astype(np.float64)
+    for (kind, O), t, w, y in zip(mats, ts, ws, ys):
+        assert orn.gemm_form(kind, O, K, M) == form, (kind, O)
+        got = y.download(np.uint16, (M + 1, O))
+        assert np.all(got[M] == 0xFFFF)
+        ctx.linear_matmul(w, dx, M, alone)
+        assert np.array_equal(got[:M], alone.download(np.uint16, (M, O))), (kind, O)
+        _check(got[:M], x, _deq(kind, t, 1, O, K)[0], (kind, O, K, M))
+    for b in [dx, alone] + ys + ws: b.free()
 
 
 def test_own_columns_forms_in_one_call(orn, ctx):
