@@ -856,6 +856,12 @@ ORNITH_API int ornith_selftest_gemm_form(const ornith_linear* w, const void* d_x
 /* ... and that ornith_kq_gather_matmul takes (0, 1, 3 or 4; -1: no such call). */
 ORNITH_API int ornith_selftest_gather_form(const ornith_kmatrix* w, const void* d_x, int pairs, int top_k, int is_up, const void* d_y);
 
+/* ornith_add_rms_moe_block as a model's forward calls it: where *done comes back 1 its last launch has made x_out = h + the block's output and
+ * next_out = rms_norm(x_out, wnext) as well, and d_out is not written; else the block is all that was done. */
+ORNITH_API int ornith_selftest_moe_close(ornith_ctx* ctx, const ornith_moe_weights* w, const void* d_res, const void* d_y, const void* d_wnorm,
+                                         const void* d_wnext, float eps, int T, void* d_h, void* d_normed, void* d_out, void* d_x_out,
+                                         void* d_next_out, int* done);
+
 /* ---- machine probes (`bench.py --ceiling`) ------------------------------------------
  * No reference counterpart (the reference times its own dispatches from the host,
  * src/bin/dispatch.rs, Q4K.md:479-484); nothing on the decode path calls these. They price a

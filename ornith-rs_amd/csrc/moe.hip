@@ -652,4 +652,15 @@ int ornith_add_rms_moe_block(ornith_ctx* ctx, const ornith_moe_weights* w, const
   return moe_block_impl(ctx, w, d_normed_out, T, d_out, nullptr, nullptr, &pre, true);
 }
 
+int ornith_selftest_moe_close(ornith_ctx* ctx, const ornith_moe_weights* w, const void* d_res, const void* d_y, const void* d_wnorm,
+                              const void* d_wnext, float eps, int T, void* d_h, void* d_normed, void* d_out, void* d_x_out,
+                              void* d_next_out, int* done) {
+  ORN_REQUIRE(d_res && d_y && d_wnorm && d_wnext && d_h && d_normed && d_x_out && d_next_out && done, "moe_close: null argument");
+  const PreNorm pre{(const bf16_t*)d_res, (const bf16_t*)d_y, (const bf16_t*)d_wnorm, (bf16_t*)d_h, (bf16_t*)d_normed, eps};
+  MoeClose close{{(const bf16_t*)d_h, nullptr, (const bf16_t*)d_wnext, (bf16_t*)d_x_out, (bf16_t*)d_next_out, eps}};
+  const int rc = add_rms_moe_block_close(ctx, w, pre, T, d_out, &close);
+  *done = close.done;
+  return rc;
+}
+
 }  // extern "C"

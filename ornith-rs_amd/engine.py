@@ -615,6 +615,14 @@ def add_rms_linear_multi(ctx, lins, res, y, wnorm, eps, M, h_out, normed_out, ys
                                              h_out.ptr, normed_out.ptr, yp), "add_rms_linear_multi")
 
 
+def moe_close(ctx, w, res, y, wnorm, wnext, eps, T, h, normed, out, x_out, next_out):
+    """ornith_selftest_moe_close: whether the block's last launch made the closing add and the next norm"""
+    done = C.c_int()
+    _check(lib().ornith_selftest_moe_close(ctx.h, C.byref(w), res.ptr, y.ptr, wnorm.ptr, wnext.ptr, C.c_float(eps), T, h.ptr, normed.ptr,
+                                           out.ptr, x_out.ptr, next_out.ptr, C.byref(done)), "moe_close")
+    return bool(done.value)
+
+
 def add_rms_moe_block(ctx, w, res, y, wnorm, eps, T, h_out, normed_out, out):
     _check(lib().ornith_add_rms_moe_block(ctx.h, C.byref(w), res.ptr, y.ptr, wnorm.ptr, C.c_float(eps), T,
                                           h_out.ptr, normed_out.ptr, out.ptr), "add_rms_moe_block")

@@ -1,6 +1,8 @@
 """GPU: every fused launch structure gives the same bits as the one-launch-per-operator
 path (the reference holds its own fusions to the same standard, e.g. tests/gdn.rs:176-230,
 tests/q4k.rs:778-822), and as the oracle."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -409,14 +411,16 @@ def test_norm_and_its_consumers_in_place(orn, ctx, fmt, T):
     moe.free()
 
 
-@pytest.mark.parametrize("H,k,T", [(1024, 8, 33), (2048, 10, 90), (4096, 8, 40), (2048, 8, 700)])
-def test_norm_inside_combine_launch_equals_separate(orn, ctx, H, k, T):
+@pytest.mark.parametrize("H,k,T,I,trunk", [(1024, 8, 33, 256, "kq"), (2048, 10, 90, 256, "kq"), (4096, 8, 40, 256, "kq"), (2048, 8, 700, 256, "kq"),
+                                           (2048, 8, 51, 512, "kq"), (2048, 8, 700, 512, "kq"), (2048, 8, 600, 512, "affine4"), (4096, 8, 35, 512, "affine4")])
+def test_norm_inside_combine_launch_equals_separate(orn, ctx, H, k, T, I, trunk):
     """The residual add and the norm after a prompt's MoE block, made by its combine launch, == the launches of
-    their own: the same bits of every row and of the decode step that follows (caches), through both forms of the
-    block (T = 700: tall expert groups)."""
+    their own: the same bits of every row and of the decode step that follows (caches). 256-wide experts are not the few-row
+    kernels': the block in separate launches (of tall expert groups at T = 700); 512-wide ones and the 4-bit ones are."""
     import synth
-    cfg = dict(synth.TINY, hidden_size=H, num_experts_per_tok=k, num_hidden_layers=2, full_attention_interval=2)
-    s = synth.SynthModel(cfg, seed=H + T, with_mtp=False, with_oracle=False)
+    cfg = dict(synth.TINY, hidden_size=H, num_experts_per_tok=k, num_hidden_layers=2, full_attention_interval=2,
+               moe_intermediate_size=I, shared_expert_intermediate_size=I)
+    s = synth.SynthModel(cfg, seed=H + T, with_mtp=False, with_oracle=False, trunk=trunk, affine="affine4" if trunk == "affine4" else "affine8")
     ws = s.upload(orn, ctx)
     model = orn.TextModel(ctx, ws, s.text_config(orn))
     model.set_max_rows(T)
@@ -433,3 +437,39 @@ def test_norm_inside_combine_launch_equals_separate(orn, ctx, H, k, T):
     finally:
         orn.set_option("fuse_norm", 1)
         for o in (model, ws): o.close()
+
+
+@pytest.mark.parametrize("fmt,H,I,T,shift", [
+    # few rows an expert: the block whose shared expert is one of the list; 640 tokens: tall expert groups; 256-wide experts: neither
+    ("kq", 1024, 512, 51, 0), ("kq", 2048, 512, 51, 0), ("kq", 4096, 512, 37, 0), ("kq", 2048, 512, 640, 0), ("kq", 2048, 256, 90, 0),
+    ("affine4", 2048, 512, 51, 0), ("affine4", 2048, 512, 640, 0),
+    # widths, an alignment and a row count at which the close stays with its own launch
+    ("kq", 512, 512, 51, 0), ("kq", 2048, 512, 51, 8), ("affine4", 2048, 512, 51, 2), ("kq", 2048, 512, 4, 0)])
+def test_combine_launch_makes_the_closing_add_and_norm(orn, ctx, fmt, H, I, T, shift):
+    """that it does where it can, into poisoned buffers, with the bits of the block, the add and the norm by themselves, and stores nothing past the last row;
+    where it cannot, nothing but the block has run. `shift`: bytes by which the next norm's output misses 16-byte alignment"""
+    rng = np.random.default_rng(H + I + T)
+    moe = util.HostMoe(rng, H=H, E=64, I=I, top_k=8, gate_kind=util.AFFINE4 if fmt == "affine4" else Q4K)
+    dw, n = moe.dev(orn, ctx), T * H * 2
+    res, y = ctx.to_device(util.bf16_normal(rng, (T, H))), ctx.to_device(util.bf16_normal(rng, (T, H)))
+    wn, wx = ctx.to_device(util.bf16_normal(rng, (H,))), ctx.to_device(util.bf16_normal(rng, (H,)))
+    h, nm, out, x, nx, out1, x1, nx1 = bufs = [ctx.alloc(n + H * 2) for _ in range(8)]
+    for b in bufs: ctx.memset(b, 0xFF, n + H * 2)
+
+    class At:
+        ptr = C.c_void_p(nx.ptr.value + shift)
+    done = orn.moe_close(ctx, dw, res, y, wn, wx, 1e-6, T, h, nm, out, x, At)
+    assert done == (H in (1024, 2048, 4096) and shift == 0 and T > 16)
+    if done:
+        assert np.all(out.download(np.uint16, (T, H)) == 0xFFFF)
+        orn.add_rms_moe_block(ctx, dw, res, y, wn, 1e-6, T, h, nm, out1)
+        ctx.add_rms_norm(h, out1, wx, T, H, 1e-6, x1, nx1)
+        for got, want in ((x, x1), (nx, nx1)):
+            got, want = got.download(np.uint16, (T + 1, H)), want.download(np.uint16, (T + 1, H))
+            assert np.array_equal(got, want) and np.all(got[T] == 0xFFFF) and not np.any(got[:T] == 0xFFFF)
+    else:
+        assert np.all(x.download(np.uint16, (T, H)) == 0xFFFF) and np.all(nx.download(np.uint16, (T, H)) == 0xFFFF)
+        orn.add_rms_moe_block(ctx, dw, res, y, wn, 1e-6, T, h, nm, out1)
+        assert np.array_equal(out.download(np.uint16, (T, H)), out1.download(np.uint16, (T, H)))
+    for b in bufs + [res, y, wn, wx]: b.free()
+    moe.free()
