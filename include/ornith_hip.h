@@ -93,13 +93,15 @@ ORNITH_API int ornith_device_info(ornith_ctx* ctx, char* name, size_t name_len, 
  *   "kq_iters"  (ORNITH_KQ_ITERS, default 0 = chosen by the launch from its shape and from how
  *               many of its workgroups a compute unit holds; 1..8): output rows each
  *               wavefront of the k-quant mat-vec walks, a tuning knob
- *   "gemm_duo"  (ORNITH_GEMM_DUO, default 1): the prefill GEMM dequantizes the weights into MFMA
- *               operand registers, beside the multiplication, where the shape suits it (from 193
- *               rows on for more than 2048 columns; 0: always through LDS); results agree to the
- *               order of the fp32 sums
- *   "gemm_reg"  (ORNITH_GEMM_REG, default 1): the same of the expert-gathered prefill GEMM (80
- *               rows an expert or more, 48 for matrices that the few-row kernels don't take, as
- *               K > 4096; 0: always through LDS); results agree to the order of the fp32 sums
+ *   "gemm_duo"  (ORNITH_GEMM_DUO, default 1; the name is older than what it switches): the prefill
+ *               GEMM dequantizes the weights into MFMA operand registers, beside the multiplication,
+ *               where M > 128 rows and the few-row kernels do not take the matrix. Those stop at:
+ *               4096 columns and more Q4_K 128 rows, Q6_K 192; 2049 .. 4095, and 513 .. 2048 of
+ *               K >= 2048, 2^20 outputs and 576 rows or 2^19 outputs; of narrower ones and K < 2048
+ *               1024 to 2560 rows. 0: through LDS; results agree to the order of the fp32 sums
+ *   "gemm_reg"  (ORNITH_GEMM_REG, default 1; likewise): the same of the expert-gathered prefill GEMM
+ *               (80 rows an expert or more, 48 for matrices of K >= 1024 that the few-row kernels
+ *               don't take, as K > 4096; 0: through LDS); results agree to the order of the fp32 sums
  *   "gdn_chunked" (ORNITH_GDN_CHUNKED, default 1): the gated-delta recurrence of calls of 128
  *               rows or more (without per-token snapshots) runs in 64-token chunks on the
  *               matrix cores (0: token by token); results agree to rounding

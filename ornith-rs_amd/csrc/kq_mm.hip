@@ -10,7 +10,7 @@
 // (v_mfma_f32_32x32x16_bf16), the weights read as k-quant codes (the 144 / 210 bytes per 256
 // weights that HBM holds) and dequantized with the arithmetic of kquant::dequantize
 // (d*sc*q - dmin*m, resp. d*sc*q), rounded to bf16. Here are the dispatch, the expert-sorted pair list and the
-// form for any shape and alignment: a workgroup tile of BM x 128 outputs over K slabs of 128; activations go
+// form for any shape and alignment, and for what the options take off the others: a workgroup tile of BM x 128 outputs over K slabs of 128; activations go
 // global -> LDS as they are, weights are dequantized on the way into LDS; LDS rows padded by
 // 8 elements so the 16-byte fragment reads of 32 consecutive rows spread over the banks;
 // four wavefronts: 2 x 2 of 64 x 64 outputs each for BM = 128, 1 x 4 of 64 x 32 for BM = 64.
@@ -235,7 +235,8 @@ __device__ __forceinline__ void store_tile(const MmArgs& a, const f32x16_t (&acc
   }
 }
 
-// BM = 256: 2 x 2 wavefronts of 128 x 64; BM = 128: 2 x 2 of 64 x 64; BM = 64: 1 x 4 of 64 x 32.
+// BM = 128: 2 x 2 wavefronts of 64 x 64; BM = 64: 1 x 4 of 64 x 32; BM = 256: 2 x 2 of 128 x 64 (plain, enough tiles to fill the device: matrices
+// or activations that are not 16-byte aligned or past 32-bit offsets, and gemm_duo = 0).
 // KIND = kMixed: the matrices of the launch differ in kind (a workgroup asks its own).
 constexpr int kMixed = 2;
 template <int KIND, int BM, bool GATHER>

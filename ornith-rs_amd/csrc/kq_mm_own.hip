@@ -28,15 +28,16 @@
 // kThin is one such set, over all of K and two workgroups a compute unit: the sums of the full tile in a fourth of it, for a launch
 // that full tiles leave most compute units idle in.
 //
-// What bounds it: at full size the matrix cores at the clock the card holds under them (12288 x 2048, 6621 rows: a step takes 0.39 us
-// with every compute unit at work and 0.29 with one; the same loop over weights that are bf16 already, no vector work at all,
-// reaches 1157 TFLOP/s there, this one 1130 to 1157); below about 160 rows a tile the unpacking (0.14 us a step however few the rows);
-// and 3 us of way in and 3.5 us of way out a tile, which nothing overlaps.
+// What bounds it: at full size (12288 x 2048, 6621 rows) the matrix cores are busy for 55 % of the launch's clocks. What is left of them are the ways in and
+// out of a tile, 3 and 3.5 us of 56 that nothing overlaps, the last of five rounds of tiles (0.88 full), and the step: 0.39 us
+// with every compute unit at work where one alone takes 0.29, by the clock, which falls under load; the same loop over weights that are bf16
+// already, no vector work at all, is no faster. Below about 160 rows a tile the unpacking (0.14 us a step however few the rows).
 //
-// Measured, us, against the producer / consumer form this replaces (256 x 128 tiles, weights through LDS): 12288 x 2048 Q4_K at 700 / 1500 /
-// 6621 rows 54 / 103 / 357 -> 41 / 77 / 278 (867 -> 1157 TFLOP/s), 2048 x 4096 at 6621 138 -> 96, q / k / v (9216 x 2048 Q6_K) at 700 / 6621 58 / 293 -> 38 /
-// 242, router + shared gate + up at 6621 83 -> 44; and against tiles of 192 rows with activations through registers, the experts of
-// 6621 tokens (207 rows each): gate or up 165 -> 121, down (K = 512) 274 -> 201. With kHalves, against the few-row kernels and kFour: 12288 x 2048
+// Measured on one card, us, launches by themselves, against what this replaces (256 x 128 tiles with weights through LDS): 12288 x 2048 Q4_K at 700 / 1500 /
+// 6621 rows 52 / 100 / 342 -> 37 / 74 / 268 (975 -> 1244 TFLOP/s; in a prompt's trace 1135 to 1198), 2048 x 4096 at 6621 132 -> 92, q / k / v (9216 x 2048 Q6_K) at
+// 700 / 6621 44 / 292 -> 37 / 229; the experts of 6621 tokens, 256 of them, against tiles of 192 and 64 rows with activations through registers: gate or up 151 -> 107
+// with 207 rows each, 148 -> 120 with a spread as a router's, down (K = 512) 272 -> 186 and 256 -> 219. In a trace of that prompt: gate or up 131, down 227, router +
+// shared gate + up 46. With kHalves, against the few-row kernels and kFour: 12288 x 2048
 // Q4_K at 129 / 200 rows 25 / 25 -> 18 / 20, 2048 x 4096 Q4_K at 600 / 1200 / 2000 30 / 44 / 46 -> 25 / 29 / 39, Q6_K 36 / 53 / 55 -> 28 / 33 / 42.
 #include <type_traits>
 

@@ -31,8 +31,8 @@ def _check(got_bits, want64, K, what):
 @pytest.mark.parametrize("kind,O,K,M", [(Q4K, 256, 512, 128), (Q4K, 512, 2048, 300), (Q6K, 256, 512, 128),
                                          (Q6K, 384, 2048, 77), (Q4K, 8192, 2048, 256), (Q6K, 2048, 4096, 129),
                                          (Q4K, 200, 256, 16),
-                                         # enough 256-row tiles to fill the device: the producer / consumer kernel,
-                                         # ragged in rows (1061 = 4 tiles + 37) and a whole number of tiles
+                                         # enough tiles of 256 rows to fill the device, ragged in rows
+                                         # (1061 = 4 tiles + 37) and a whole number of them
                                          (Q4K, 8192, 512, 1061), (Q6K, 8192, 1024, 1024),
                                          # a 4096-row prompt chunk through the widest projection of a gated-delta
                                          # layer and through q_proj: the sampled configuration's prefill call
@@ -87,7 +87,7 @@ def test_kq_matmul_weights_through_lds(orn, ctx, mats, K, M):
         for b in [dx] + ys + ws: b.free()
 
 
-@pytest.mark.parametrize("kind,E,O,K,T,k", [(Q4K, 8, 256, 512, 400, 2), (Q6K, 16, 131, 256, 500, 4), (Q4K, 8, 264, 1024, 700, 2),
+@pytest.mark.parametrize("kind,E,O,K,T,k", [(Q4K, 8, 256, 512, 400, 2), (Q6K, 16, 131, 256, 500, 4), (Q4K, 8, 264, 1024, 700, 2), (Q6K, 8, 131, 1024, 700, 2),
                                              (Q6K, 4, 130, 4352, 140, 2)])
 def test_kq_gather_matmul_weights_through_lds(orn, ctx, kind, E, O, K, T, k):
     """gemm_reg = 0: the experts' GEMM in 64- and 128-row workgroups that unpack into LDS, a 48-row average among them"""
@@ -175,12 +175,11 @@ def ctx_off(buf, nbytes):
                                              # about 100 rows an expert and more: 128-row tiles
                                              (Q4K, 8, 256, 512, 400, 2), (Q6K, 16, 128, 256, 500, 4),
                                              # more than 8192 pairs (the plan made by three launches), a few
-                                             # hundred rows an expert and one crowded expert: tall tiles, the
-                                             # register form for K >= 1024 and its split over shorter workgroups
+                                             # hundred rows an expert and one crowded expert: tall plan tiles
                                              (Q4K, 32, 512, 2048, 1100, 8), (Q6K, 32, 256, 1024, 1100, 8),
                                              (Q6K, 32, 1024, 512, 1100, 8),
                                              # 75 to 79 rows an expert of matrices that the few-row kernels don't take (K > 4096; scales in
-                                             # no 16-byte pieces): low plan tiles, three a workgroup in the register form, and the LDS form
+                                             # no 16-byte pieces): low plan tiles, four a workgroup where K >= 1024, and the LDS form
                                              (Q4K, 8, 264, 4352, 316, 2), (Q6K, 8, 130, 4352, 316, 2), (Q4K, 128, 40, 4352, 1200, 8),
                                              (Q6K, 16, 257, 1280, 300, 4), (Q6K, 16, 130, 768, 300, 4)])
 def test_kq_gather_matmul_vs_float64(orn, ctx, kind, E, O, K, T, k):
@@ -254,9 +253,9 @@ def _rows_close(got_bits, want_bits, tol):
 
 
 @pytest.mark.parametrize("H,E,I,T", [(512, 64, 256, 48), (2048, 256, 512, 160),
-                                     # 64 rows an expert: the few-row kernels; 80, 82 and 150: tall plan tiles, split over 64-row workgroups
+                                     # 64 rows an expert; 80, 82 and 150: tall plan tiles
                                      (512, 64, 256, 512), (512, 64, 256, 640), (512, 64, 256, 1200),
-                                     # gate / up in the register form (K = 1024), down on the same plan in 64-row workgroups
+                                     # gate / up of K = 1024, down of K = 256 on the same plan
                                      (1024, 64, 256, 512), (1024, 64, 256, 656), (1024, 64, 256, 1300)])
 def test_moe_block_prefill_width_close_to_exact_path(orn, ctx, H, E, I, T):
     """At prefill width the block runs as GEMMs. Against the oracle's exact path the rows agree
@@ -617,8 +616,8 @@ def test_dense_projections_sharing_an_input_share_a_launch(orn, ctx, Os, K, M):
 
 
 def test_gathered_matmuls_of_different_depth_share_a_plan(orn, ctx):
-    """The MoE block builds the pair plan with its gate projection (K = 1024 here: tall tiles,
-    register form) and runs the down projection (K = 256: 64-row workgroups) on the same plan
+    """The MoE block builds the pair plan with its gate projection (K = 1024 here: tall tiles) and
+    runs the down projection (K = 256) on the same plan
     without rebuilding it: every pair's row must be computed, whatever the kernel's own tile
     height (outputs poisoned beforehand)."""
     rng = np.random.default_rng(12)
